@@ -223,15 +223,6 @@ def prefill_attention(
     if q.is_cuda:
         ext = _require_ext("prefill_attention")
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        ql = query_lens.cpu().tolist()
-        cu = [0]
-        tile_req, tile_row0 = [], []
-        for i, l in enumerate(ql):
-            cu.append(cu[-1] + int(l))
-            for r0 in range(0, int(l), 32):
-                tile_req.append(i)
-                tile_row0.append(r0)
-        dev = q.device
         ext.prefill_attention(
             out,
             q,
@@ -239,9 +230,7 @@ def prefill_attention(
             v_cache,
             block_tables.to(torch.int32),
             seq_lens.to(torch.int32),
-            torch.tensor(cu, dtype=torch.int32, device=dev),
-            torch.tensor(tile_req, dtype=torch.int32, device=dev),
-            torch.tensor(tile_row0, dtype=torch.int32, device=dev),
+            query_lens.to(device=q.device, dtype=torch.int32).contiguous(),
             scale,
             sliding_window,
             softcap,

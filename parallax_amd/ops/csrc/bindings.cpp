@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 
 #define CHECK_GPU(x) TORCH_CHECK(x.is_cuda(), #x " must be on GPU")
@@ -82,11 +83,12 @@ void launch_sample_gumbel(int64_t*, const float*, const float*,
                           const uint8_t*, uint64_t, int, int, hipStream_t);
 void launch_skinny_gemm(void*, const void*, const void*, const void*, int,
                         int, int, int64_t, int64_t, hipStream_t, bool*);
-void launch_prefill_attention(void*, const void*, const void*, const void*,
-                              const int*, const int*, const int*, const int*,
-                              const int*, int, int, int, int, int, int, int64_t,
-                              float, int, float, const float*, bool, float,
-                              float, hipStream_t, bool*);
+int prefill_attention_tiles(int, int, int, int);
+void launch_prefill_attention(void*, float*, float*, const void*, const void*,
+                              const void*, const int*, const int*, const int*,
+                              int, int, int, int, int, int, int, int64_t, float,
+                              int, float, const float*, int, bool, float, float,
+                              hipStream_t, bool*);
 }
 
 static hipStream_t cur_stream() {
@@ -312,8 +314,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
 void prefill_attention(torch::Tensor out, torch::Tensor q,
                        torch::Tensor k_cache, torch::Tensor v_cache,
                        torch::Tensor block_tables, torch::Tensor seq_lens,
-                       torch::Tensor cu_q, torch::Tensor tile_req,
-                       torch::Tensor tile_row0, double scale,
+                       torch::Tensor query_lens, double scale,
                        int64_t sliding_window, double softcap,
                        torch::Tensor sinks, double k_scale, double v_scale) {
   CHECK_GPU(q);
@@ -323,14 +324,17 @@ void prefill_attention(torch::Tensor out, torch::Tensor q,
               "k_cache must be bf16 or fp8_e4m3fn");
   TORCH_CHECK(block_tables.scalar_type() == at::kInt);
   TORCH_CHECK(seq_lens.scalar_type() == at::kInt);
-  TORCH_CHECK(cu_q.scalar_type() == at::kInt);
+  TORCH_CHECK(query_lens.scalar_type() == at::kInt &&
+              query_lens.is_contiguous());
+  const int T = q.size(0);
+  const int B = query_lens.size(0);
   const int Hq = q.size(1);
   const int D = q.size(2);
   const int Hk = k_cache.size(1);
   const int BS = k_cache.size(2);
   const int max_blocks = block_tables.size(1);
-  const int n_tiles = tile_req.size(0);
   TORCH_CHECK(D == 128 || D == 64, "head_dim must be 64 or 128");
+  if (T == 0 || B == 0) return;
 
   const float* sinks_ptr = nullptr;
   torch::Tensor sinks_f;
@@ -338,15 +342,34 @@ void prefill_attention(torch::Tensor out, torch::Tensor q,
     sinks_f = sinks.to(at::kFloat).contiguous();
     sinks_ptr = sinks_f.data_ptr<float>();
   }
+  // Short portions on long contexts leave most of the 256 CUs idle: their keys
+  // are split over workgroups until two a CU are there, at least 512 keys each
+  // (a split writes and reads its fp32 sums once more).
+  const int64_t blocks = (int64_t)prefill_attention_tiles(T, B, Hq, Hk) * Hk;
+  const int64_t keys = (int64_t)max_blocks * BS;
+  int splits = (int)std::max<int64_t>(
+      1, std::min<int64_t>({512 / blocks, keys / 512, 64}));
+  torch::Tensor tmp_acc, tmp_ml;
+  float *acc_ptr = nullptr, *ml_ptr = nullptr;
+  if (splits > 1) {
+    auto opts = q.options().dtype(at::kFloat);
+    tmp_acc = torch::empty({T, Hq, splits, D}, opts);
+    tmp_ml = torch::empty({T, Hq, splits, 2}, opts);
+    acc_ptr = tmp_acc.data_ptr<float>();
+    ml_ptr = tmp_ml.data_ptr<float>();
+  }
   bool launched = false;
   launch_prefill_attention(
-      out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-      block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(),
-      cu_q.data_ptr<int>(), tile_req.data_ptr<int>(), tile_row0.data_ptr<int>(),
-      n_tiles, Hq, Hk, D, BS, max_blocks, row_stride(q, "q"), (float)scale,
-      (int)sliding_window, (float)softcap, sinks_ptr, kv_fp8, (float)k_scale,
+      out.data_ptr(), acc_ptr, ml_ptr, q.data_ptr(), k_cache.data_ptr(),
+      v_cache.data_ptr(), block_tables.data_ptr<int>(),
+      seq_lens.data_ptr<int>(), query_lens.data_ptr<int>(), T, B, Hq, Hk, D,
+      BS, max_blocks, row_stride(q, "q"), (float)scale, (int)sliding_window,
+      (float)softcap, sinks_ptr, splits, kv_fp8, (float)k_scale,
       (float)v_scale, cur_stream(), &launched);
   TORCH_CHECK(launched, "no prefill kernel instantiation for D=", D);
+  if (splits > 1)
+    launch_paged_attention_reduce(out.data_ptr(), acc_ptr, ml_ptr, T, Hq, D,
+                                  splits, sinks_ptr, cur_stream());
 }
 
 void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,

@@ -109,3 +109,36 @@ def test_prefill_engine_parity_gpu_vs_cpu():
     out_cpu = list(eng_cpu.generate(prompts, sp).values())
     # random init + bf16-vs-fp32: expect identical argmax on a tiny model
     assert out_gpu == out_cpu
+
+
+@pytest.mark.parametrize("Hq,Hk,D,BS,fp8,kw", [
+    (4, 4, 128, 16, False, {}),                       # one row an item
+    (14, 2, 64, 32, False, {}),                       # rows cut by a tile's edge
+    (16, 1, 128, 64, False, {"sliding_window": 70}),
+    (8, 2, 128, 8, False, {"softcap": 30.0}),         # general page sizes
+    (8, 2, 64, 24, False, {}),
+    (8, 1, 128, 16, True, {}),
+    (8, 2, 64, 40, True, {"sliding_window": 33}),
+])
+def test_prefill_items_pages_and_splits(Hq, Hk, D, BS, fp8, kw):
+    """Portions around the 128-item and 64-key tiles, requests of one row, and
+    (few items, long prefix) keys split over workgroups. Slots past the end of
+    a sequence hold NaN. Weights and results are rounded to bf16 once each:
+    an error of at most 2 * 2^-9 * max |v|, max |v| < 5.2 here."""
+    per = max(1, 128 // (Hq // Hk))
+    for ql, pre in (([per, 1, per + 1], [0, 63, 64]), ([3], [2100])):
+        sl = [a + b for a, b in zip(ql, pre)]
+        q, kc, vc, bt, slt, qlt = _setup(ql, sl, Hq, Hk, D, BS=BS, seed=len(ql))
+        if fp8:
+            kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+        ref_k, ref_v = kc.float(), vc.float()
+        for i, n in enumerate(sl):
+            if n % BS and not fp8:
+                page = int(bt[i, n // BS])
+                kc[page, :, n % BS:] = float("nan")
+                vc[page, :, :, n % BS:] = float("nan")
+        out = ops.prefill_attention(q, kc, vc, bt, slt, qlt, D ** -0.5, **kw)
+        want = ref.prefill_attention(
+            q.float().cpu(), ref_k.cpu(), ref_v.cpu(), bt.cpu(), slt.cpu(),
+            qlt.cpu(), D ** -0.5, **kw)
+        torch.testing.assert_close(out.float().cpu(), want, atol=2.1e-2, rtol=0)
