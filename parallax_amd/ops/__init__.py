@@ -503,21 +503,11 @@ def fused_moe_forward(
     its output."""
     assert x.is_cuda
     ext = _require_ext("moe_forward")
-    T, H = x.shape
-    E = w_gate_up.shape[0]
-    k = topk_ids.shape[1]
-    flat = topk_ids.reshape(-1)
-    sorted_ids, perm = torch.sort(flat)
-    seg = torch.searchsorted(
-        sorted_ids, torch.arange(E + 1, device=x.device, dtype=sorted_ids.dtype)
-    ).to(torch.int32)
-    route_w = topk_weights.reshape(-1).float()[perm].contiguous()
-    out = torch.zeros(T, H, dtype=torch.float32, device=x.device)
-    ext.moe_forward(out, x.contiguous(), w_gate_up, w_down, perm.contiguous(),
-                    seg.contiguous(), route_w, k, activation == "gelu", limit,
-                    bias_gate_up if bias_gate_up is not None
-                    else x.new_empty(0), bool(weight_on_input))
-    return out
+    return ext.moe_forward(
+        x.contiguous(), w_gate_up, w_down, topk_ids.long().contiguous(),
+        topk_weights.float().contiguous(), activation == "gelu", limit,
+        bias_gate_up if bias_gate_up is not None else x.new_empty(0),
+        bool(weight_on_input))
 
 
 _FP8_LIN_BUFS = {}
@@ -576,20 +566,10 @@ def fused_moe_forward_fp8(
     per-token on device). Returns fp32 [T, H]."""
     assert x.is_cuda
     ext = _require_ext("moe_forward_fp8")
-    T, H = x.shape
-    E = w_gate_up.shape[0]
-    k = topk_ids.shape[1]
-    flat = topk_ids.reshape(-1)
-    sorted_ids, perm = torch.sort(flat)
-    seg = torch.searchsorted(
-        sorted_ids, torch.arange(E + 1, device=x.device, dtype=sorted_ids.dtype)
-    ).to(torch.int32)
-    route_w = topk_weights.reshape(-1).float()[perm].contiguous()
-    out = torch.zeros(T, H, dtype=torch.float32, device=x.device)
-    ext.moe_forward_fp8(out, x.contiguous(), w_gate_up, w_gu_scale, w_down,
-                        w_down_scale, perm.contiguous(), seg.contiguous(),
-                        route_w, k, activation == "gelu", limit)
-    return out
+    return ext.moe_forward_fp8(
+        x.contiguous(), w_gate_up, w_gu_scale, w_down, w_down_scale,
+        topk_ids.long().contiguous(), topk_weights.float().contiguous(),
+        activation == "gelu", limit)
 
 
 # -- sampling (torch ops; GPU path uses torch's ROCm kernels — not a hot spot

@@ -51,14 +51,21 @@ void launch_msa_paged_attention_decode(void*, const void*, const void*,
                                        const int*, int, int, int, int, int,
                                        int, int, int, int64_t, float,
                                        hipStream_t, bool*);
-void launch_build_moe_tiles(int*, int*, const int*, int, int, hipStream_t);
-void launch_moe_gate_up(void*, const void*, const void*, const int*,
-                        const int*, const int64_t*, const int*, int, int, int,
-                        int, int, bool, float, const void*, const float*,
-                        hipStream_t);
-void launch_moe_down(void*, const void*, const void*, const float*, const int*,
-                     const int*, const int64_t*, const int*, int, int, int,
-                     int, int, hipStream_t);
+int moe_tile_rows(int, int, int, bool);
+int64_t moe_route_scratch(int, int);
+int moe_max_tiles(int, int, int);
+void launch_moe_route(int*, void*, int*, int*, const int64_t*, int, int, int,
+                      hipStream_t);
+void launch_moe_gate_up(void*, const void*, const float*, const void*,
+                        const float*, const int*, const void*, const int*,
+                        const float*, const void*, int, int, int, int, int,
+                        bool, bool, bool, float, hipStream_t);
+void launch_moe_down(float*, const void*, const float*, const void*,
+                     const float*, const int*, const void*, const int*,
+                     const float*, int, int, int, int, int, bool, bool,
+                     hipStream_t);
+void launch_moe_combine(float*, const float*, const int64_t*, int, int, int,
+                        int, hipStream_t);
 void launch_dsa_indexer_scores(float*, const void*, const void*, const float*,
                                const int*, const int*, int, int, int, int,
                                int, int, hipStream_t, bool*);
@@ -71,14 +78,6 @@ void launch_msa_topk_tokens(int64_t*, const float*, const int*, int, int, int,
                             int, int, int, int, hipStream_t);
 void launch_quantize_fp8_rows(void*, float*, const void*, int, int,
                               hipStream_t);
-void launch_moe_gate_up_fp8(void*, const void*, const float*, const void*,
-                            const float*, const int*, const int*,
-                            const int64_t*, const int*, int, int, int, int,
-                            int, bool, float, hipStream_t);
-void launch_moe_down_fp8(void*, const void*, const float*, const void*,
-                         const float*, const float*, const int*, const int*,
-                         const int64_t*, const int*, int, int, int, int, int,
-                         hipStream_t);
 void launch_sample_gumbel(int64_t*, const float*, const float*,
                           const uint8_t*, uint64_t, int, int, hipStream_t);
 void launch_skinny_gemm(void*, const void*, const void*, const void*, int,
@@ -434,51 +433,116 @@ void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,
                                   num_parts, nullptr, cur_stream());
 }
 
-void moe_forward(torch::Tensor out, torch::Tensor x, torch::Tensor w_gu,
-                 torch::Tensor w_down, torch::Tensor perm,
-                 torch::Tensor seg_offsets, torch::Tensor route_w,
-                 int64_t topk, bool gelu, double limit,
-                 torch::Tensor bias_gu, bool weight_on_input) {
+// Routed experts of x [T, H]: bf16, or fp8 (W8A8) with w_gu_scale / w_down_scale
+// given. Returns fp32 [T, H].
+static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
+                               torch::Tensor w_gu_scale, torch::Tensor w_down,
+                               torch::Tensor w_down_scale,
+                               torch::Tensor topk_ids, torch::Tensor topk_w,
+                               bool gelu, double limit, torch::Tensor bias_gu,
+                               bool weight_on_input, bool fp8) {
   CHECK_GPU(x);
   CHECK_CONTIG(x);
   CHECK_BF16(x);
-  CHECK_BF16(w_gu);
-  CHECK_BF16(w_down);
-  TORCH_CHECK(out.scalar_type() == at::kFloat && out.is_contiguous());
-  TORCH_CHECK(perm.scalar_type() == at::kLong);
-  TORCH_CHECK(seg_offsets.scalar_type() == at::kInt);
-  TORCH_CHECK(route_w.scalar_type() == at::kFloat);
+  CHECK_CONTIG(w_gu);
+  CHECK_CONTIG(w_down);
+  TORCH_CHECK(topk_ids.dim() == 2 && topk_ids.is_contiguous() &&
+              topk_ids.scalar_type() == at::kLong);
+  TORCH_CHECK(topk_w.is_contiguous() && topk_w.scalar_type() == at::kFloat &&
+              topk_w.numel() == topk_ids.numel());
+  const int T = x.size(0);
+  const int k = topk_ids.size(1);
   const int E = w_gu.size(0);
   const int I = w_gu.size(1) / 2;
   const int H = w_gu.size(2);
-  const int n_assign = perm.size(0);
-  TORCH_CHECK(H % 32 == 0 && I % 32 == 0,
-              "MoE dims must be multiples of 32 (H=", H, " I=", I, ")");
-  const int max_tiles = (n_assign + 15) / 16 + E;
-  auto iopts = x.options().dtype(at::kInt);
-  torch::Tensor tile_expert = torch::empty({max_tiles}, iopts);
-  torch::Tensor tile_row0 = torch::empty({max_tiles}, iopts);
-  torch::Tensor h_buf =
-      torch::empty({n_assign, I}, x.options().dtype(at::kBFloat16));
-  auto stream = cur_stream();
-  launch_build_moe_tiles(tile_expert.data_ptr<int>(), tile_row0.data_ptr<int>(),
-                         seg_offsets.data_ptr<int>(), E, max_tiles, stream);
+  const int n = T * k;
+  TORCH_CHECK(topk_ids.size(0) == T && x.size(1) == H &&
+              w_down.size(0) == E && w_down.size(1) == H &&
+              w_down.size(2) == I, "MoE operand shapes do not match");
+  TORCH_CHECK(H % 32 == 0 && I % (fp8 ? 64 : 32) == 0,
+              "MoE dims must be multiples of 32, fp8 I of 64 (H=", H, " I=", I,
+              ")");
+  TORCH_CHECK(E <= 16384, "more than 16384 experts");
   TORCH_CHECK(bias_gu.numel() == 0 ||
               (bias_gu.scalar_type() == at::kBFloat16 &&
-               bias_gu.is_contiguous() && bias_gu.numel() == (int64_t)E * 2 * I));
-  launch_moe_gate_up(h_buf.data_ptr(), x.data_ptr(), w_gu.data_ptr(),
-                     tile_expert.data_ptr<int>(), tile_row0.data_ptr<int>(),
-                     perm.data_ptr<int64_t>(), seg_offsets.data_ptr<int>(), E,
-                     (int)topk, H, I, max_tiles, gelu, (float)limit,
-                     bias_gu.numel() ? bias_gu.data_ptr() : nullptr,
-                     weight_on_input ? route_w.data_ptr<float>() : nullptr,
+               bias_gu.is_contiguous() &&
+               bias_gu.numel() == (int64_t)E * 2 * I));
+  auto fopts = x.options().dtype(at::kFloat);
+  auto bopts = x.options().dtype(at::kByte);
+  if (n == 0) return torch::zeros({T, H}, fopts);
+  auto stream = cur_stream();
+
+  const int tm = moe_tile_rows(n, E, I, fp8);
+  const int max_tiles = moe_max_tiles(n, E, tm);
+  // tiles (16 bytes each) first, then their number, the order, the counts
+  torch::Tensor ws = torch::empty(
+      {4 * (int64_t)max_tiles + 4 + n + moe_route_scratch(n, E)},
+      x.options().dtype(at::kInt));
+  int* tiles = ws.data_ptr<int>();
+  int* n_tiles = tiles + 4 * (int64_t)max_tiles;
+  int* perm = n_tiles + 4;
+  const int64_t* ids = topk_ids.data_ptr<int64_t>();
+  const float* wts = topk_w.data_ptr<float>();
+  launch_moe_route(perm, tiles, n_tiles, perm + n, ids, n, E, tm, stream);
+
+  torch::Tensor xq, xs, hq, hs;
+  const void* xp = x.data_ptr();
+  if (fp8) {
+    xq = torch::empty({T, H}, bopts);
+    xs = torch::empty({T}, fopts);
+    launch_quantize_fp8_rows(xq.data_ptr(), xs.data_ptr<float>(), xp, T, H,
+                             stream);
+    xp = xq.data_ptr();
+  }
+  torch::Tensor h = torch::empty({n, I}, x.options());
+  launch_moe_gate_up(h.data_ptr(), xp, fp8 ? xs.data_ptr<float>() : nullptr,
+                     w_gu.data_ptr(),
+                     fp8 ? w_gu_scale.data_ptr<float>() : nullptr, perm, tiles,
+                     n_tiles, wts,
+                     bias_gu.numel() ? bias_gu.data_ptr() : nullptr, k, H, I,
+                     max_tiles, tm, fp8, weight_on_input, gelu, (float)limit,
                      stream);
-  launch_moe_down(out.data_ptr(), h_buf.data_ptr(), w_down.data_ptr(),
-                  weight_on_input ? nullptr : route_w.data_ptr<float>(),
-                  tile_expert.data_ptr<int>(),
-                  tile_row0.data_ptr<int>(), perm.data_ptr<int64_t>(),
-                  seg_offsets.data_ptr<int>(), E, (int)topk, H, I, max_tiles,
+  const void* hp = h.data_ptr();
+  if (fp8) {
+    hq = torch::empty({n, I}, bopts);
+    hs = torch::empty({n}, fopts);
+    launch_quantize_fp8_rows(hq.data_ptr(), hs.data_ptr<float>(), hp, n, I,
+                             stream);
+    hp = hq.data_ptr();
+  }
+  torch::Tensor y = torch::empty({n, H}, fopts);
+  torch::Tensor out = torch::empty({T, H}, fopts);
+  launch_moe_down(y.data_ptr<float>(), hp,
+                  fp8 ? hs.data_ptr<float>() : nullptr, w_down.data_ptr(),
+                  fp8 ? w_down_scale.data_ptr<float>() : nullptr, perm, tiles,
+                  n_tiles, wts, k, H, I, max_tiles, tm, fp8, weight_on_input,
                   stream);
+  launch_moe_combine(out.data_ptr<float>(), y.data_ptr<float>(), ids, T, k, E,
+                     H, stream);
+  return out;
+}
+
+torch::Tensor moe_forward(torch::Tensor x, torch::Tensor w_gu,
+                          torch::Tensor w_down, torch::Tensor topk_ids,
+                          torch::Tensor topk_w, bool gelu, double limit,
+                          torch::Tensor bias_gu, bool weight_on_input) {
+  CHECK_BF16(w_gu);
+  CHECK_BF16(w_down);
+  return moe_layer(x, w_gu, {}, w_down, {}, topk_ids, topk_w, gelu, limit,
+                   bias_gu, weight_on_input, false);
+}
+
+torch::Tensor moe_forward_fp8(torch::Tensor x, torch::Tensor w_gu,
+                              torch::Tensor w_gu_scale, torch::Tensor w_down,
+                              torch::Tensor w_down_scale,
+                              torch::Tensor topk_ids, torch::Tensor topk_w,
+                              bool gelu, double limit) {
+  TORCH_CHECK(is_fp8(w_gu) && is_fp8(w_down));
+  TORCH_CHECK(w_gu_scale.scalar_type() == at::kFloat &&
+              w_down_scale.scalar_type() == at::kFloat &&
+              w_gu_scale.is_contiguous() && w_down_scale.is_contiguous());
+  return moe_layer(x, w_gu, w_gu_scale, w_down, w_down_scale, topk_ids, topk_w,
+                   gelu, limit, x.new_empty({0}), false, true);
 }
 
 torch::Tensor dsa_indexer_scores(torch::Tensor q_index,
@@ -562,64 +626,6 @@ torch::Tensor msa_topk_tokens(torch::Tensor block_scores,
                          (int)init_blocks, (int)local_blocks,
                          (int)max_positions, cur_stream());
   return out;
-}
-
-void moe_forward_fp8(torch::Tensor out, torch::Tensor x, torch::Tensor w_gu,
-                     torch::Tensor w_gu_scale, torch::Tensor w_down,
-                     torch::Tensor w_down_scale, torch::Tensor perm,
-                     torch::Tensor seg_offsets, torch::Tensor route_w,
-                     int64_t topk, bool gelu, double limit) {
-  CHECK_GPU(x);
-  CHECK_CONTIG(x);
-  CHECK_BF16(x);
-  TORCH_CHECK(w_gu.scalar_type() == at::kFloat8_e4m3fn && w_gu.is_contiguous());
-  TORCH_CHECK(w_down.scalar_type() == at::kFloat8_e4m3fn &&
-              w_down.is_contiguous());
-  TORCH_CHECK(w_gu_scale.scalar_type() == at::kFloat &&
-              w_down_scale.scalar_type() == at::kFloat);
-  TORCH_CHECK(out.scalar_type() == at::kFloat && out.is_contiguous());
-  TORCH_CHECK(perm.scalar_type() == at::kLong);
-  TORCH_CHECK(seg_offsets.scalar_type() == at::kInt);
-  TORCH_CHECK(route_w.scalar_type() == at::kFloat);
-  const int T = x.size(0);
-  const int E = w_gu.size(0);
-  const int I = w_gu.size(1) / 2;
-  const int H = w_gu.size(2);
-  const int n_assign = perm.size(0);
-  TORCH_CHECK(H % 32 == 0 && I % 64 == 0,
-              "MoE dims must be multiples of 32/64 (H=", H, " I=", I, ")");
-  const int max_tiles = (n_assign + 15) / 16 + E;
-  auto iopts = x.options().dtype(at::kInt);
-  auto fopts = x.options().dtype(at::kFloat);
-  auto bopts = x.options().dtype(at::kByte);
-  torch::Tensor tile_expert = torch::empty({max_tiles}, iopts);
-  torch::Tensor tile_row0 = torch::empty({max_tiles}, iopts);
-  torch::Tensor x_fp8 = torch::empty({T, H}, bopts);
-  torch::Tensor x_scale = torch::empty({T}, fopts);
-  torch::Tensor h_buf =
-      torch::empty({n_assign, I}, x.options().dtype(at::kBFloat16));
-  torch::Tensor h_fp8 = torch::empty({n_assign, I}, bopts);
-  torch::Tensor h_scale = torch::empty({std::max(n_assign, 1)}, fopts);
-  auto stream = cur_stream();
-  launch_quantize_fp8_rows(x_fp8.data_ptr(), x_scale.data_ptr<float>(),
-                           x.data_ptr(), T, H, stream);
-  launch_build_moe_tiles(tile_expert.data_ptr<int>(), tile_row0.data_ptr<int>(),
-                         seg_offsets.data_ptr<int>(), E, max_tiles, stream);
-  launch_moe_gate_up_fp8(
-      h_buf.data_ptr(), x_fp8.data_ptr(), x_scale.data_ptr<float>(),
-      w_gu.data_ptr(), w_gu_scale.data_ptr<float>(),
-      tile_expert.data_ptr<int>(), tile_row0.data_ptr<int>(),
-      perm.data_ptr<int64_t>(), seg_offsets.data_ptr<int>(), E, (int)topk, H,
-      I, max_tiles, gelu, (float)limit, stream);
-  if (n_assign > 0)
-    launch_quantize_fp8_rows(h_fp8.data_ptr(), h_scale.data_ptr<float>(),
-                             h_buf.data_ptr(), n_assign, I, stream);
-  launch_moe_down_fp8(
-      out.data_ptr(), h_fp8.data_ptr(), h_scale.data_ptr<float>(),
-      w_down.data_ptr(), w_down_scale.data_ptr<float>(),
-      route_w.data_ptr<float>(), tile_expert.data_ptr<int>(),
-      tile_row0.data_ptr<int>(), perm.data_ptr<int64_t>(),
-      seg_offsets.data_ptr<int>(), E, (int)topk, H, I, max_tiles, stream);
 }
 
 torch::Tensor sample_gumbel(torch::Tensor logits, torch::Tensor inv_temp,

@@ -1,226 +1,491 @@
-// Grouped MoE GEMMs for gfx950 — device-side routing, graph-capture safe.
+// Routed experts for gfx950: device-side routing, two grouped GEMMs, a combine.
 //
-// Pipeline (host side in ops/__init__.py, all capturable torch ops):
-//   topk -> sort assignments by expert -> searchsorted segment offsets
-// then three kernels here:
-//   build_moe_tiles:  segment offsets -> (expert, row0) per 16-row tile
-//   moe_gate_up:      h = act(x[gather] @ W_gu[e]^T)   (gate/up column pairs
-//                     land in the same lane -> activation fused in-register)
-//   moe_down:         out[t] += route_w * (h @ W_down[e]^T)  (fp32 atomics)
+//   moe_route      counts the choices of every expert, sorts them (perm: sorted
+//                  place -> flat choice t * k + j) and lists the tiles of TM
+//                  rows; one workgroup, no host involvement
+//   moe_gemm<GATE> h = act(x[gather] . W_gu[e]^T): gate and up columns meet in
+//                  the same lane, the activation is applied in registers
+//   moe_gemm       y[choice] = w * (h . W_down[e]^T), fp32
+//   moe_combine    out[t] = sum of its choices' y, in the order of the choices
 // With in_w the routing weight multiplies the expert's INPUT instead: the
-// gate/up accumulators are scaled by it (both projections are linear) and
-// moe_down adds the result unweighted.
+// gate/up accumulators are scaled by it (both projections are linear).
+// fp8: W8A8, weights e4m3 with a scale per output row, activations quantised a
+// row (x before the first product, h before the second).
 //
-// Shapes: W_gu [E, 2I, H], W_down [E, H, I] (row-major, out-major) — B operand
-// fragments read rows k-consecutive, so no transposition anywhere. Fixed
-// MAX_TILES grid (tiles past the live count exit) keeps kernel launches
-// hipGraph-stable. Reference analogue: the reference delegates MoE to
-// SGLang/vLLM fused kernels; this is the MI355X-native equivalent.
+// W_gu is [E, 2I, H], W_down [E, H, I]. Choices of an expert outside [0, E) (the
+// experts of another rank) are left out. Grids are upper bounds (blocks past
+// the live tiles exit), so a captured step replays with any routing.
 
 #include "common.h"
 
-#define MOE_THREADS 256
-#define MOE_TM 64  // assignment rows per tile (4 MFMA M-tiles; big tiles
-                   // amortize the expert-weight stream across more tokens)
+#include <type_traits>
 
-__global__ void build_moe_tiles_kernel(
-    int* __restrict__ tile_expert,   // [max_tiles]
-    int* __restrict__ tile_row0,     // [max_tiles]
-    const int* __restrict__ seg_offsets,  // [E+1]
-    const int E, const int max_tiles) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int t = 0;
-  for (int e = 0; e < E && t < max_tiles; ++e) {
-    const int begin = seg_offsets[e], end = seg_offsets[e + 1];
-    for (int r = begin; r < end && t < max_tiles; r += MOE_TM) {
-      tile_expert[t] = e;
-      tile_row0[t] = r;
-      ++t;
-    }
-  }
-  for (; t < max_tiles; ++t) tile_expert[t] = -1;
+#define MOE_BKB 128    // bytes of the contraction a stage
+
+typedef float f32x16v __attribute__((ext_vector_type(16)));
+typedef int i32x4v __attribute__((ext_vector_type(4)));
+typedef int i32x8v __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2n __attribute__((ext_vector_type(2)));
+
+namespace {
+
+DEVINL uint32_t pack_bf16(float a, float b) {
+  bf16x2n p;
+  p[0] = (__bf16)a;
+  p[1] = (__bf16)b;
+  return __builtin_bit_cast(uint32_t, p);
 }
 
-// ---- grouped gate_up + activation --------------------------------------------
-// grid: (max_tiles, I/64). Wave w handles N-tile w of a 64-col slab; each lane
-// accumulates the gate tile and the matching up tile (same columns of I).
+DEVINL void copy16_to_lds(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)src,
+      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
 
-template <bool GELU>
-__global__ __launch_bounds__(MOE_THREADS) void moe_gate_up_kernel(
-    uint16_t* __restrict__ h_buf,          // [rows_padded, I] bf16
-    const uint16_t* __restrict__ x,        // [T, H]
-    const uint16_t* __restrict__ w_gu,     // [E, 2I, H]
-    const int* __restrict__ tile_expert,
-    const int* __restrict__ tile_row0,
-    const int64_t* __restrict__ perm,      // [T*k] sorted-assignment -> flat idx
-    const int* __restrict__ seg_offsets,   // [E+1]
-    const int E, const int topk, const int H, const int I,
-    const float limit,                     // >0: gpt-oss clamped act
-    const uint16_t* __restrict__ bias_gu = nullptr,  // [E, 2I] or null
-    const float* __restrict__ in_w = nullptr) {  // [T*k] sorted, or null
-  const int tile = blockIdx.x;
-  const int e = tile_expert[tile];
-  if (e < 0) return;
-  const int row0 = tile_row0[tile];
-  const int rows_end = seg_offsets[e + 1];
+}  // namespace
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int l15 = lane & 15;
-  const int l4 = lane >> 4;
+// ---- routing ------------------------------------------------------------------
+// perm [n], tiles [max_tiles] as (expert, first row, end of the expert's rows,
+// -), n_tiles [1]. A decode step has a few hundred choices: one workgroup and
+// one launch do it in 5 us. LDS counters bound it, 60 cycles an atomic of a
+// wave: 65,536 choices took one workgroup 52 us, so parts of ROUTE_PART choices
+// are counted first (moe_count), and each then places its own behind the
+// parts before it.
 
-  const int n0 = blockIdx.y * 64 + wid * 16;  // column tile within I
-  if (n0 >= I) return;  // I is a multiple of 16, not necessarily of 64
-  // gate row n0+l15 of W_gu; up row I+n0+l15
-  const uint16_t* wg_row = w_gu + ((size_t)e * 2 * I + (n0 + l15)) * H;
-  const uint16_t* wu_row = w_gu + ((size_t)e * 2 * I + (I + n0 + l15)) * H;
+#define ROUTE_THREADS 1024
+#define ROUTE_PART 4096
 
-  // 4 token M-tiles share each streamed W fragment
-  const uint16_t* xrow[4];
-  bool arow_ok[4];
+// cnt[e] += this part's choices of expert e; cnt is in LDS
+DEVINL void count_choices(int* cnt, const int64_t* ids, int begin, int end,
+                          int E) {
+  // ids are fetched four ahead of the counters, which would wait for each
+  constexpr int AHEAD = ROUTE_PART / ROUTE_THREADS;
+  for (int i0 = begin + threadIdx.x; i0 < end; i0 += ROUTE_PART) {
+    int64_t e[AHEAD];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int arow = row0 + mt * 16 + l15;
-    arow_ok[mt] = arow < rows_end;
-    xrow[mt] = arow_ok[mt] ? x + (size_t)(perm[arow] / topk) * H : x;
-  }
-
-  f32x4v acc_g[4] = {}, acc_u[4] = {};
-  for (int k = 0; k < H; k += 32) {
-    const bf16x8v bg = *reinterpret_cast<const bf16x8v*>(wg_row + k + l4 * 8);
-    const bf16x8v bu = *reinterpret_cast<const bf16x8v*>(wu_row + k + l4 * 8);
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (row0 + mt * 16 >= rows_end) break;
-      bf16x8v afrag = {};
-      if (arow_ok[mt])
-        afrag = *reinterpret_cast<const bf16x8v*>(xrow[mt] + k + l4 * 8);
-      acc_g[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, bg, acc_g[mt], 0, 0, 0);
-      acc_u[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, bu, acc_u[mt], 0, 0, 0);
+    for (int u = 0; u < AHEAD; ++u) {
+      const int i = i0 + u * ROUTE_THREADS;
+      e[u] = i < end ? ids[i] : -1;
     }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (e[u] >= 0 && e[u] < E) atomicAdd(&cnt[e[u]], 1);
   }
+}
 
-  // D layout (verified by the numerics tests): element (lane, reg) is
-  // row m = (lane>>4)*4 + reg (token), col n = lane&15 (output feature).
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = mt * 16 + l4 * 4 + r;  // token row within tile
-      const int grow = row0 + m;
-      if (grow >= rows_end) continue;
-      const int n = n0 + l15;              // column within I
-      float g = acc_g[mt][r], u = acc_u[mt][r];
-      if (in_w != nullptr) {
-        const float w = in_w[grow];
-        g *= w;
-        u *= w;
-      }
-      if (bias_gu != nullptr) {
-        g += bf16_bits_to_f32(bias_gu[(size_t)e * 2 * I + n]);
-        u += bf16_bits_to_f32(bias_gu[(size_t)e * 2 * I + I + n]);
-      }
-      float a;
-      if (limit > 0.f) {                   // gpt-oss clamped act
-        g = fminf(g, limit);
-        u = fminf(fmaxf(u, -limit), limit);
-        a = (u + 1.f) * (g / (1.f + __expf(-g * 1.702f)));
-      } else if (GELU) {
-        const float c = 0.7978845608028654f;
-        a = 0.5f * g * (1.f + tanhf(c * (g + 0.044715f * g * g * g))) * u;
+__global__ __launch_bounds__(ROUTE_THREADS) void moe_count_kernel(
+    int* __restrict__ counts,  // [parts, E]
+    const int64_t* __restrict__ ids, const int n, const int E) {
+  extern __shared__ int lds[];
+  for (int e = threadIdx.x; e < E; e += ROUTE_THREADS) lds[e] = 0;
+  __syncthreads();
+  const int begin = blockIdx.x * ROUTE_PART;
+  count_choices(lds, ids, begin, min(n, begin + ROUTE_PART), E);
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += ROUTE_THREADS)
+    counts[(size_t)blockIdx.x * E + e] = lds[e];
+}
+
+__global__ __launch_bounds__(ROUTE_THREADS) void moe_route_kernel(
+    int* __restrict__ perm, int4* __restrict__ tiles, int* __restrict__ n_tiles,
+    const int* __restrict__ counts, const int64_t* __restrict__ ids,
+    const int n, const int E, const int tm) {
+  extern __shared__ int lds[];
+  int* cur = lds;  // counters, then the next place of every expert
+  __shared__ int wave_rows[16], wave_tiles[16];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wid = tid >> 6;
+  const int parts = gridDim.x;
+  const int begin = parts > 1 ? blockIdx.x * ROUTE_PART : 0;
+  const int end = parts > 1 ? min(n, begin + ROUTE_PART) : n;
+  if (parts == 1) {
+    for (int e = tid; e < E; e += ROUTE_THREADS) cur[e] = 0;
+    __syncthreads();
+    count_choices(cur, ids, begin, end, E);
+    __syncthreads();
+  }
+  // exclusive sums of rows and tiles over the experts, 1024 at a time
+  int rows0 = 0, tiles0 = 0;
+  for (int e0 = 0; e0 < E; e0 += ROUTE_THREADS) {
+    const int e = e0 + tid;
+    int c = 0, before = 0;
+    if (e < E) {
+      if (parts == 1) {
+        c = cur[e];
       } else {
-        a = g / (1.f + __expf(-g)) * u;
+        for (int q = 0; q < parts; ++q) {
+          const int v = counts[(size_t)q * E + e];
+          c += v;
+          before += q < (int)blockIdx.x ? v : 0;
+        }
       }
-      h_buf[(size_t)grow * I + n] = f32_to_bf16_bits(a);
     }
+    const int t = (c + tm - 1) / tm;
+    int rs = c, ts = t;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int r2 = __shfl_up(rs, o, WAVE_SIZE);
+      const int t2 = __shfl_up(ts, o, WAVE_SIZE);
+      if (lane >= o) {
+        rs += r2;
+        ts += t2;
+      }
+    }
+    if (lane == 63) {
+      wave_rows[wid] = rs;
+      wave_tiles[wid] = ts;
+    }
+    __syncthreads();
+    int rb = rows0, tb = tiles0, rsum = 0, tsum = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      if (w < wid) {
+        rb += wave_rows[w];
+        tb += wave_tiles[w];
+      }
+      rsum += wave_rows[w];
+      tsum += wave_tiles[w];
+    }
+    if (e < E) {
+      const int r0 = rb + rs - c;
+      int at = tb + ts - t;
+      cur[e] = r0 + before;
+      if (blockIdx.x == 0)
+        for (int r = r0; r < r0 + c; r += tm)
+          tiles[at++] = make_int4(e, r, r0 + c, 0);
+    }
+    rows0 += rsum;
+    tiles0 += tsum;
+    __syncthreads();
+  }
+  if (tid == 0 && blockIdx.x == 0) *n_tiles = tiles0;
+  constexpr int AHEAD = ROUTE_PART / ROUTE_THREADS;
+  for (int i0 = begin + tid; i0 < end; i0 += ROUTE_PART) {
+    int64_t e[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int i = i0 + u * ROUTE_THREADS;
+      e[u] = i < end ? ids[i] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (e[u] >= 0 && e[u] < E)
+        perm[atomicAdd(&cur[e[u]], 1)] = i0 + u * ROUTE_THREADS;
   }
 }
 
-// ---- grouped down projection + weighted scatter -------------------------------
-// grid: (max_tiles, H/64). out is fp32 [T, H]; routing weight applied here.
+// ---- grouped GEMM ----------------------------------------------------------------
+// A workgroup takes one tile of TM rows of one expert and TN of its weight
+// rows: D[feature x row] = W . A^T on 32x32 matrix instructions, so that a lane
+// ends with four neighbouring features of one row. Both operands go global ->
+// LDS directly (16 bytes a lane, STAGES - 1 stages of 128 bytes of every row in
+// flight), 16-byte chunks XOR-swizzled by row so that 16 rows of one chunk
+// column lie in 16 bank groups.
+//   TM 32, 64: the weights' stream is the work. 4 waves x 32 weight rows.
+//   TM 128:    matrix products, 256 weight rows: 4 x 2 waves of 64 x 64.
+// GATE: of 32 weight rows of a wave 16 are gate and 16 the up rows of the same
+// columns; the accumulator's upper registers are the lower ones' partners.
+// What bounds it: few rows, the weights' stream: 256 fp8 experts of 7168 x 2048,
+// 200 tokens x 8 choices, gate/up 0.99 ms and down 0.55 ms = 6.2 TB/s of the
+// experts touched (2.44 and 1.06 ms with fragments loaded straight to
+// registers). Many rows, the address unit: it moves 64 bytes a cycle and CU, so
+// a 128 x 256 tile takes 768 of its cycles for 1024 of the matrix cores (128 x
+// 128: 512 for 512), and copies asked for in one burst hold their wave up: they
+// are spread over the products. 128 bf16 experts of 2048 x 768, 8192 tokens x 8:
+// gate/up 583 us = 707 TFLOP/s, down 429 us (2247 and 1530 us before).
 
-__global__ __launch_bounds__(MOE_THREADS) void moe_down_kernel(
-    float* __restrict__ out,               // [T, H] fp32 (pre-zeroed)
-    const uint16_t* __restrict__ h_buf,    // [rows_padded, I]
-    const uint16_t* __restrict__ w_down,   // [E, H, I]
-    const float* __restrict__ route_w,     // [T*k] flat routing weights
-    const int* __restrict__ tile_expert,
-    const int* __restrict__ tile_row0,
-    const int64_t* __restrict__ perm,
-    const int* __restrict__ seg_offsets,
-    const int E, const int topk, const int H, const int I) {
-  const int tile = blockIdx.x;
-  const int e = tile_expert[tile];
-  if (e < 0) return;
-  const int row0 = tile_row0[tile];
-  const int rows_end = seg_offsets[e + 1];
+struct MoeArgs {
+  const uint8_t* w;        // [E, w_rows, kb] bytes
+  const float* w_scale;    // [E, w_rows] (fp8)
+  const uint8_t* a;        // rows of kb bytes: x [T] or h [n]
+  const float* a_scale;    // per row of a (fp8)
+  const int* perm;
+  const int4* tiles;
+  const int* n_tiles;
+  const float* choice_w;   // [T, k] routing weights
+  const uint16_t* bias;    // [E, 2I] or null (GATE)
+  void* out;               // GATE: h [n, N] bf16; else y [T * k, N] fp32
+  int topk, N, kb, nb;     // N output features, kb bytes a row, nb column blocks
+  int in_w, gelu;
+  float limit;             // > 0: clamped activation
+};
+
+template <bool FP8, int TN, int TM, bool GATE, int STAGES>
+__global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
+  constexpr int WN = TM == 128 ? 2 : 1;  // 32-row weight tiles a wave
+  constexpr int WM = TM == 32 ? 1 : 2;   // 32-row activation tiles a wave
+  constexpr int PASS = TN / 4;            // rows the threads copy at once
+  constexpr int APASS = TM / PASS;
+  constexpr int LOADS = 4 + APASS;        // copies a thread and stage
+  constexpr int BUF = (TN + TM) * MOE_BKB;
+  __shared__ __attribute__((aligned(16))) uint8_t S0[BUF];
+  __shared__ __attribute__((aligned(16))) uint8_t S1[BUF];
+  __shared__ __attribute__((aligned(16))) uint8_t S2[BUF];
+  __shared__ __attribute__((aligned(16))) uint8_t S3[STAGES > 3 ? BUF : 16];
+
+  // Blocks go round-robin to the 8 XCDs. Each XCD takes a contiguous eighth of
+  // the (tile, column block) list, so that the blocks of an expert share one
+  // L2: its weights and rows are read from memory once.
+  const int total = *p.n_tiles * p.nb;
+  const int chunk = (total + 7) >> 3;
+  const int slot = blockIdx.x >> 3;
+  const int idx = (blockIdx.x & 7) * chunk + slot;
+  if (slot >= chunk || idx >= total) return;
+  const int4 tile = p.tiles[idx / p.nb];
+  const int e = __builtin_amdgcn_readfirstlane(tile.x);
+  const int row0 = __builtin_amdgcn_readfirstlane(tile.y);
+  const int rows_end = __builtin_amdgcn_readfirstlane(tile.z);
+  const int n0 = (idx % p.nb) * (GATE ? TN / 2 : TN);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int l15 = lane & 15;
-  const int l4 = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5;
+  const int l31 = lane & 31;
 
-  const int n0 = blockIdx.y * 256 + wid * 64;  // 4 waves x 4 n-tiles = 256 cols
-  const uint16_t* hrow[4];
-  bool arow_ok[4];
+  // ---- what a thread copies: one chunk of rows tid / 8 + PASS i --------------------
+  const int src = (tid & 7) ^ ((tid >> 4) & 7);
+  const uint8_t* wp[4];
+  const uint8_t* ap[APASS];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int arow = row0 + mt * 16 + l15;
-    arow_ok[mt] = arow < rows_end;
-    hrow[mt] = arow_ok[mt] ? h_buf + (size_t)arow * I : h_buf;
-  }
-
-  f32x4v acc[4][4] = {};
-  for (int k = 0; k < I; k += 32) {
-    bf16x8v bfr[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int n = n0 + nt * 16 + l15;
-      bfr[nt] = {};
-      if (n < H)
-        bfr[nt] = *reinterpret_cast<const bf16x8v*>(
-            w_down + ((size_t)e * H + n) * I + k + l4 * 8);
-    }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (row0 + mt * 16 >= rows_end) break;
-      bf16x8v afrag = {};
-      if (arow_ok[mt])
-        afrag = *reinterpret_cast<const bf16x8v*>(hrow[mt] + k + l4 * 8);
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            afrag, bfr[nt], acc[mt][nt], 0, 0, 0);
-    }
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * PASS + (tid >> 3);
+    int row;  // rows past the last feature are read twice and never stored
+    if (GATE)
+      row = ((r >> 4) & 1) * p.N + min(n0 + (r >> 5) * 16 + (r & 15), p.N - 1);
+    else
+      row = min(n0 + r, p.N - 1);
+    wp[i] = p.w + ((size_t)e * (GATE ? 2 * p.N : p.N) + row) * p.kb;
   }
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
+  for (int i = 0; i < APASS; ++i) {
+    const int r = min(row0 + i * PASS + (tid >> 3), rows_end - 1);
+    ap[i] = p.a + (size_t)(GATE ? p.perm[r] / p.topk : r) * p.kb;
+  }
+  // copy i of a stage: 4 passes over the weight rows, then the activation rows
+  auto copy = [&](int i, int off, uint8_t* S) {
+    if (i < 4)
+      copy16_to_lds(wp[i] + off, S + (i * PASS + wid * 8) * MOE_BKB);
+    else
+      copy16_to_lds(ap[i - 4] + off,
+                    S + (TN + (i - 4) * PASS + wid * 8) * MOE_BKB);
+  };
+  auto offset = [&](int kt) {
+    return min(kt * MOE_BKB + src * 16, p.kb - 16);
+  };
+  auto issue = [&](int kt, uint8_t* S) {
+    const int off = offset(kt);
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int n = n0 + nt * 16 + l15;
-      if (n >= H) break;
+    for (int i = 0; i < LOADS; ++i) copy(i, off, S);
+  };
+
+  // waves: TM 128: TN / 64 x 2 of 64 x 64; else TN / 32 x 1 of 32 x TM
+  const int wb = TM == 128 ? (wid & (TN / 64 - 1)) * 64 : wid * 32;
+  const int ab = TM == 128 ? wid / (TN / 64) * 64 : 0;
+  const int swz_l = (l31 >> 1) & 7;
+  using frag_t = std::conditional_t<FP8, i32x8v, bf16x8v>;
+  f32x16v acc[WN][WM] = {};
+
+  // FULL: 128 bytes of the contraction; else what is left of it (32 k bytes).
+  auto stage = [&](const uint8_t* S, int left, auto full, auto&& between) {
+    constexpr bool FULL = decltype(full)::value;
+    constexpr int KS = FP8 ? 2 : 4;
+    const uint8_t* Wl = S + (wb + l31) * MOE_BKB;
+    const uint8_t* Al = S + (TN + ab + l31) * MOE_BKB;
+    frag_t a[2][WN], b[2][WM];
+    auto fetch = [&](int ks) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int grow = row0 + mt * 16 + l4 * 4 + r;
-        if (grow >= rows_end) continue;
-        const float w = route_w != nullptr ? route_w[grow] : 1.f;
-        const int64_t token = perm[grow] / topk;
-        atomicAdd(out + (size_t)token * H + n, acc[mt][nt][r] * w);
+      for (int i = 0; i < WN + WM; ++i) {
+        const uint8_t* r = i < WN ? Wl + i * 32 * MOE_BKB
+                                  : Al + (i - WN) * 32 * MOE_BKB;
+        frag_t& f = i < WN ? a[ks & 1][i] : b[ks & 1][i - WN];
+        if constexpr (FP8) {
+          const int c0 = ((4 * ks + 2 * half) ^ swz_l) * 16;
+          const int c1 = ((4 * ks + 2 * half + 1) ^ swz_l) * 16;
+          f = __builtin_shufflevector(*(const i32x4v*)(r + c0),
+                                      *(const i32x4v*)(r + c1), 0, 1, 2, 3, 4,
+                                      5, 6, 7);
+          // of a last step of 32 the upper half of the lanes has nothing, and
+          // of a step behind the end no lane has
+          if (!FULL && left - ks * 64 < (half ? 64 : 1)) f = 0;
+        } else {
+          f = *(const bf16x8v*)(r + ((2 * ks + half) ^ swz_l) * 16);
+          if (!FULL && ks * 32 >= left) f = 0;
+        }
+      }
+    };
+    // lgkmcnt(0) before the next step's operands are asked for: this step's
+    // products need no further wait and run while those are under way
+    auto landed = [] {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    fetch(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      landed();
+      if (ks + 1 < KS) fetch(ks + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < WN; ++i)
+#pragma unroll
+        for (int j = 0; j < WM; ++j) {
+          if constexpr (FP8)
+            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                a[ks & 1][i], b[ks & 1][j], acc[i][j], 0, 0, 0, 0x7f7f7f7f, 0,
+                0x7f7f7f7f);
+          else
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                a[ks & 1][i], b[ks & 1][j], acc[i][j], 0, 0, 0);
+          between((ks * WN + i) * WM + j);
+        }
+    }
+  };
+
+  // One barrier a stage: behind it stage kt is in LDS for every wave, and the
+  // buffer that stage kt + STAGES - 1 goes to has been left by every wave. Past
+  // the end the copies go on, of one cached chunk a row, so that the number of
+  // copies in flight is the same for every stage and the wait a constant.
+  auto turn = [&](int kt, uint8_t* S, uint8_t* Sn) {
+    constexpr int V = (STAGES - 2) * LOADS;  // copies of the later stages
+    // a fence would wait for every copy: vmcnt(V), lgkmcnt(0) by hand, and no
+    // LDS access moves over the barrier
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (V & 15) | ((V >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    // the copies are spread over the products: a wave that asks for all of
+    // them at once waits for the address unit, which takes 64 bytes a cycle
+    const int off = offset(kt + STAGES - 1);
+    constexpr int PRODUCTS = (FP8 ? 2 : 4) * WN * WM;
+    stage(S, MOE_BKB, std::true_type{}, [&](int m) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+        if (m == i * PRODUCTS / LOADS) {
+          __builtin_amdgcn_sched_barrier(0);
+          copy(i, off, Sn);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    });
+  };
+  const int nk = p.kb / MOE_BKB;  // full stages
+  issue(0, S0);
+  issue(1, S1);
+  if constexpr (STAGES > 3) issue(2, S2);
+  for (int kt = 0; kt < nk;) {
+    turn(kt, S0, STAGES == 3 ? S2 : S3);
+    if (++kt >= nk) break;
+    turn(kt, S1, S0);
+    if (++kt >= nk) break;
+    turn(kt, S2, S1);
+    if (++kt >= nk) break;
+    if constexpr (STAGES > 3) {
+      turn(kt, S3, S2);
+      if (++kt >= nk) break;
+    }
+  }
+  // the last copies: no more may land in LDS once the workgroup has ended
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  if (p.kb % MOE_BKB) {
+    __syncthreads();
+    const int at = nk % STAGES;
+    stage(at == 0 ? S0 : at == 1 ? S1 : at == 2 ? S2 : S3, p.kb % MOE_BKB,
+          std::false_type{}, [](int) {});
+  }
+
+  // ---- results: column = row of the tile, registers = features --------------------
+#pragma unroll
+  for (int j = 0; j < WM; ++j) {
+    const int r = row0 + ab + j * 32 + l31;
+    if (r >= rows_end) continue;
+    const int choice = p.perm[r];
+    const float w = p.choice_w[choice];
+    const float sa = FP8 ? p.a_scale[GATE ? choice / p.topk : r] : 1.f;
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+      if (GATE) {
+        uint16_t* h = (uint16_t*)p.out + (size_t)r * p.N;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int f = n0 + (wb >> 1) + i * 16 + 8 * q + 4 * half;
+          if (f >= p.N) continue;
+          float v[4];
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            float g = acc[i][j][4 * q + s], u = acc[i][j][8 + 4 * q + s];
+            if (FP8) {
+              const float* ws = p.w_scale + (size_t)e * 2 * p.N + f + s;
+              g *= sa * ws[0];
+              u *= sa * ws[p.N];
+            }
+            if (p.in_w) {
+              g *= w;
+              u *= w;
+            }
+            if (p.bias != nullptr) {
+              const uint16_t* b = p.bias + (size_t)e * 2 * p.N + f + s;
+              g += bf16_bits_to_f32(b[0]);
+              u += bf16_bits_to_f32(b[p.N]);
+            }
+            if (p.limit > 0.f) {  // gpt-oss clamped act
+              g = fminf(g, p.limit);
+              u = fminf(fmaxf(u, -p.limit), p.limit);
+              v[s] = (u + 1.f) * (g / (1.f + __expf(-g * 1.702f)));
+            } else if (p.gelu) {
+              const float c = 0.7978845608028654f;
+              v[s] =
+                  0.5f * g * (1.f + tanhf(c * (g + 0.044715f * g * g * g))) * u;
+            } else {
+              v[s] = g / (1.f + __expf(-g)) * u;
+            }
+          }
+          uint2 o;
+          o.x = pack_bf16(v[0], v[1]);
+          o.y = pack_bf16(v[2], v[3]);
+          *reinterpret_cast<uint2*>(h + f) = o;
+        }
+      } else {
+        float* y = (float*)p.out + (size_t)choice * p.N;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int f = n0 + wb + i * 32 + 8 * q + 4 * half;
+          if (f >= p.N) continue;
+          f32x4v o;
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            float c = p.in_w ? 1.f : w;
+            if (FP8) c *= sa * p.w_scale[(size_t)e * p.N + f + s];
+            o[s] = acc[i][j][4 * q + s] * c;
+          }
+          *reinterpret_cast<f32x4v*>(y + f) = o;
+        }
       }
     }
   }
 }
 
-// ---- fp8 (OCP e4m3) grouped path ---------------------------------------------
-// W8A8: weights pre-quantized per output channel (w_scale[n] = amax_row/448,
-// host side); activations quantized per token row on the fly. Non-scaled fp8
-// MFMA runs at the bf16 rate on gfx950 (guide §3: only MX-block-scaled K=128
-// reaches the 2x fp8 peak), so the win here is the HALVED weight stream —
-// which is exactly what bounds grouped MoE: each expert's weights are read
-// once per activated tile while tokens/expert stay small. Matches the
-// BASELINE DeepSeek-V3 "fp8 MFMA" config.
+// ---- combine --------------------------------------------------------------------
+// out[t] = sum over its choices; four features a thread.
+
+__global__ __launch_bounds__(256) void moe_combine_kernel(
+    float* __restrict__ out, const float* __restrict__ y,
+    const int64_t* __restrict__ ids, const int T, const int k, const int E,
+    const int H) {
+  const int t = blockIdx.x;
+  for (int c = (blockIdx.y * 256 + threadIdx.x) * 4; c < H;
+       c += gridDim.y * 1024) {
+    f32x4v s = {0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < k; ++j) {
+      const int64_t e = ids[(size_t)t * k + j];
+      if (e >= 0 && e < E)
+        s += *reinterpret_cast<const f32x4v*>(y + ((size_t)t * k + j) * H + c);
+    }
+    *reinterpret_cast<f32x4v*>(out + (size_t)t * H + c) = s;
+  }
+}
+
+// ---- activations to fp8 (OCP e4m3), one scale a row --------------------------------
 
 #define FP8_MAX 448.f
 
@@ -256,165 +521,6 @@ __global__ __launch_bounds__(256) void quantize_fp8_rows_kernel(
   }
 }
 
-// grid: (max_tiles, I/64); acc dequant = x_scale[token] * w_scale[n].
-template <bool GELU>
-__global__ __launch_bounds__(MOE_THREADS) void moe_gate_up_fp8_kernel(
-    uint16_t* __restrict__ h_buf,          // [rows_padded, I] bf16
-    const uint8_t* __restrict__ x,         // [T, H] fp8
-    const float* __restrict__ x_scale,     // [T]
-    const uint8_t* __restrict__ w_gu,      // [E, 2I, H] fp8
-    const float* __restrict__ w_scale,     // [E, 2I]
-    const int* __restrict__ tile_expert,
-    const int* __restrict__ tile_row0,
-    const int64_t* __restrict__ perm,
-    const int* __restrict__ seg_offsets,
-    const int E, const int topk, const int H, const int I,
-    const float limit) {
-  const int tile = blockIdx.x;
-  const int e = tile_expert[tile];
-  if (e < 0) return;
-  const int row0 = tile_row0[tile];
-  const int rows_end = seg_offsets[e + 1];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int l15 = lane & 15;
-  const int l4 = lane >> 4;
-
-  const int n0 = blockIdx.y * 64 + wid * 16;
-  const uint8_t* wg_row = w_gu + ((size_t)e * 2 * I + (n0 + l15)) * H;
-  const uint8_t* wu_row = w_gu + ((size_t)e * 2 * I + (I + n0 + l15)) * H;
-  const float sg = w_scale[(size_t)e * 2 * I + n0 + l15];
-  const float su = w_scale[(size_t)e * 2 * I + I + n0 + l15];
-
-  const uint8_t* xrow[4];
-  bool arow_ok[4];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int arow = row0 + mt * 16 + l15;
-    arow_ok[mt] = arow < rows_end;
-    xrow[mt] = arow_ok[mt] ? x + (size_t)(perm[arow] / topk) * H : x;
-  }
-
-  f32x4v acc_g[4] = {}, acc_u[4] = {};
-  for (int k = 0; k < H; k += 32) {
-    const long bg = *reinterpret_cast<const long*>(wg_row + k + l4 * 8);
-    const long bu = *reinterpret_cast<const long*>(wu_row + k + l4 * 8);
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (row0 + mt * 16 >= rows_end) break;
-      long afrag = 0;
-      if (arow_ok[mt])
-        afrag = *reinterpret_cast<const long*>(xrow[mt] + k + l4 * 8);
-      acc_g[mt] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(afrag, bg, acc_g[mt], 0, 0, 0);
-      acc_u[mt] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(afrag, bu, acc_u[mt], 0, 0, 0);
-    }
-  }
-
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = mt * 16 + l4 * 4 + r;
-      const int grow = row0 + m;
-      if (grow >= rows_end) continue;
-      const int n = n0 + l15;
-      const float sx = x_scale[perm[grow] / topk];
-      float g = acc_g[mt][r] * sx * sg, u = acc_u[mt][r] * sx * su;
-      float a;
-      if (limit > 0.f) {
-        g = fminf(g, limit);
-        u = fminf(fmaxf(u, -limit), limit);
-        a = (u + 1.f) * (g / (1.f + __expf(-g * 1.702f)));
-      } else if (GELU) {
-        const float c = 0.7978845608028654f;
-        a = 0.5f * g * (1.f + tanhf(c * (g + 0.044715f * g * g * g))) * u;
-      } else {
-        a = g / (1.f + __expf(-g)) * u;
-      }
-      h_buf[(size_t)grow * I + n] = f32_to_bf16_bits(a);
-    }
-  }
-}
-
-// grid: (max_tiles, H/256); h rows quantized by a quantize_fp8_rows pass.
-__global__ __launch_bounds__(MOE_THREADS) void moe_down_fp8_kernel(
-    float* __restrict__ out,               // [T, H] fp32 (pre-zeroed)
-    const uint8_t* __restrict__ h_fp8,     // [rows_padded, I]
-    const float* __restrict__ h_scale,     // [rows_padded]
-    const uint8_t* __restrict__ w_down,    // [E, H, I] fp8
-    const float* __restrict__ w_scale,     // [E, H]
-    const float* __restrict__ route_w,
-    const int* __restrict__ tile_expert,
-    const int* __restrict__ tile_row0,
-    const int64_t* __restrict__ perm,
-    const int* __restrict__ seg_offsets,
-    const int E, const int topk, const int H, const int I) {
-  const int tile = blockIdx.x;
-  const int e = tile_expert[tile];
-  if (e < 0) return;
-  const int row0 = tile_row0[tile];
-  const int rows_end = seg_offsets[e + 1];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int l15 = lane & 15;
-  const int l4 = lane >> 4;
-
-  const int n0 = blockIdx.y * 256 + wid * 64;
-  const uint8_t* hrow[4];
-  bool arow_ok[4];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int arow = row0 + mt * 16 + l15;
-    arow_ok[mt] = arow < rows_end;
-    hrow[mt] = arow_ok[mt] ? h_fp8 + (size_t)arow * I : h_fp8;
-  }
-
-  f32x4v acc[4][4] = {};
-  for (int k = 0; k < I; k += 32) {
-    long bfr[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int n = n0 + nt * 16 + l15;
-      bfr[nt] = 0;
-      if (n < H)
-        bfr[nt] = *reinterpret_cast<const long*>(
-            w_down + ((size_t)e * H + n) * I + k + l4 * 8);
-    }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (row0 + mt * 16 >= rows_end) break;
-      long afrag = 0;
-      if (arow_ok[mt])
-        afrag = *reinterpret_cast<const long*>(hrow[mt] + k + l4 * 8);
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-            afrag, bfr[nt], acc[mt][nt], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int n = n0 + nt * 16 + l15;
-      if (n >= H) break;
-      const float sw = w_scale[(size_t)e * H + n];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int grow = row0 + mt * 16 + l4 * 4 + r;
-        if (grow >= rows_end) continue;
-        const float w = route_w[grow] * h_scale[grow] * sw;
-        const int64_t token = perm[grow] / topk;
-        atomicAdd(out + (size_t)token * H + n, acc[mt][nt][r] * w);
-      }
-    }
-  }
-}
-
 extern "C" void launch_quantize_fp8_rows(
     void* out, float* scales, const void* x, int R, int C,
     hipStream_t stream) {
@@ -422,68 +528,100 @@ extern "C" void launch_quantize_fp8_rows(
       (uint8_t*)out, scales, (const uint16_t*)x, C);
 }
 
-extern "C" void launch_moe_gate_up_fp8(
-    void* h_buf, const void* x, const float* x_scale, const void* w_gu,
-    const float* w_scale, const int* tile_expert, const int* tile_row0,
-    const int64_t* perm, const int* seg_offsets, int E, int topk, int H, int I,
-    int max_tiles, bool gelu, float limit, hipStream_t stream) {
-  dim3 grid(max_tiles, ceil_div(I, 64), 1);
-  if (gelu)
-    moe_gate_up_fp8_kernel<true><<<grid, MOE_THREADS, 0, stream>>>(
-        (uint16_t*)h_buf, (const uint8_t*)x, x_scale, (const uint8_t*)w_gu,
-        w_scale, tile_expert, tile_row0, perm, seg_offsets, E, topk, H, I,
-        limit);
+// ---- the two products of a layer -----------------------------------------------
+
+template <bool FP8, int TN, int TM, int STAGES>
+static void launch_gemm(bool gate, MoeArgs& p, int max_tiles,
+                        hipStream_t stream) {
+  p.nb = ceil_div(p.N, gate ? TN / 2 : TN);
+  const int blocks = (max_tiles * p.nb + 7) / 8 * 8;
+  if (gate)
+    moe_gemm_kernel<FP8, TN, TM, true, STAGES>
+        <<<blocks, 2 * TN, 0, stream>>>(p);
   else
-    moe_gate_up_fp8_kernel<false><<<grid, MOE_THREADS, 0, stream>>>(
-        (uint16_t*)h_buf, (const uint8_t*)x, x_scale, (const uint8_t*)w_gu,
-        w_scale, tile_expert, tile_row0, perm, seg_offsets, E, topk, H, I,
-        limit);
+    moe_gemm_kernel<FP8, TN, TM, false, STAGES>
+        <<<blocks, 2 * TN, 0, stream>>>(p);
 }
 
-extern "C" void launch_moe_down_fp8(
-    void* out, const void* h_fp8, const float* h_scale, const void* w_down,
-    const float* w_scale, const float* route_w, const int* tile_expert,
-    const int* tile_row0, const int64_t* perm, const int* seg_offsets, int E,
-    int topk, int H, int I, int max_tiles, hipStream_t stream) {
-  dim3 grid(max_tiles, ceil_div(H, 256), 1);
-  moe_down_fp8_kernel<<<grid, MOE_THREADS, 0, stream>>>(
-      (float*)out, (const uint8_t*)h_fp8, h_scale, (const uint8_t*)w_down,
-      w_scale, route_w, tile_expert, tile_row0, perm, seg_offsets, E, topk, H,
-      I);
+template <bool FP8>
+static void launch_gemm_tm(int tm, bool gate, MoeArgs& p, int max_tiles,
+                           hipStream_t stream) {
+  if (tm == 32)
+    launch_gemm<FP8, 128, 32, 4>(gate, p, max_tiles, stream);
+  else if (tm == 64)
+    launch_gemm<FP8, 128, 64, 3>(gate, p, max_tiles, stream);
+  else
+    launch_gemm<FP8, 256, 128, 3>(gate, p, max_tiles, stream);
 }
 
-extern "C" void launch_build_moe_tiles(
-    int* tile_expert, int* tile_row0, const int* seg_offsets, int E,
-    int max_tiles, hipStream_t stream) {
-  build_moe_tiles_kernel<<<1, 64, 0, stream>>>(tile_expert, tile_row0,
-                                               seg_offsets, E, max_tiles);
+// Rows a tile, by the mean number of choices an expert. Measured (us, tiles of
+// 32 / 64 / 128 rows): bf16 128 experts of 2048 x 768, mean 6: 182 / 189 / 230,
+// 25: 251 / 246 / 247, 43: 326 / 284 / 311, 62: 390 / 338 / 319, 512: 1855 /
+// 1378 / 1089; 32 experts of 2048 x 1024, mean 25: 106 / 122 / 151, 62: 148 /
+// 123 / 156, 250: 353 / 252 / 223; fp8 256 experts of 7168 x 2048, mean 6: 1334 /
+// 1296 / 1360, 21: 2167 / 1926 / 1989, 46: 3178 / 2503 / 2306. Below, the
+// weights' stream is the work and few rows cost nothing; 128 rows pay earlier
+// where there are blocks enough for the chip (8 a CU).
+extern "C" int moe_tile_rows(int n, int E, int I, bool fp8) {
+  const int mean = n / (E > 0 ? E : 1);
+  if (mean <= (fp8 ? 12 : 24)) return 32;
+  const int64_t blocks = ((int64_t)n / 128 + E / 2) * ceil_div(I, 128);
+  return mean > 96 || (mean > 40 && blocks >= 2048) ? 128 : 64;
+}
+
+extern "C" int moe_max_tiles(int n, int E, int tm) {
+  return n / tm + (n < E ? n : E);
+}
+
+// ints of scratch that routing n choices takes besides perm and tiles
+extern "C" int64_t moe_route_scratch(int n, int E) {
+  return n > 2 * ROUTE_PART ? (int64_t)ceil_div(n, ROUTE_PART) * E : 0;
+}
+
+extern "C" void launch_moe_route(int* perm, void* tiles, int* n_tiles,
+                                 int* counts, const int64_t* ids, int n, int E,
+                                 int tm, hipStream_t stream) {
+  const int parts = n > 2 * ROUTE_PART ? ceil_div(n, ROUTE_PART) : 1;
+  if (parts > 1)
+    moe_count_kernel<<<parts, ROUTE_THREADS, E * sizeof(int), stream>>>(
+        counts, ids, n, E);
+  moe_route_kernel<<<parts, ROUTE_THREADS, E * sizeof(int), stream>>>(
+      perm, (int4*)tiles, n_tiles, counts, ids, n, E, tm);
 }
 
 extern "C" void launch_moe_gate_up(
-    void* h_buf, const void* x, const void* w_gu, const int* tile_expert,
-    const int* tile_row0, const int64_t* perm, const int* seg_offsets, int E,
-    int topk, int H, int I, int max_tiles, bool gelu, float limit,
-    const void* bias_gu, const float* in_w, hipStream_t stream) {
-  dim3 grid(max_tiles, ceil_div(I, 64), 1);
-  if (gelu)
-    moe_gate_up_kernel<true><<<grid, MOE_THREADS, 0, stream>>>(
-        (uint16_t*)h_buf, (const uint16_t*)x, (const uint16_t*)w_gu,
-        tile_expert, tile_row0, perm, seg_offsets, E, topk, H, I, limit,
-        (const uint16_t*)bias_gu, in_w);
+    void* h, const void* x, const float* x_scale, const void* w_gu,
+    const float* w_scale, const int* perm, const void* tiles,
+    const int* n_tiles, const float* choice_w, const void* bias, int topk,
+    int H, int I, int max_tiles, int tm, bool fp8, bool in_w, bool gelu,
+    float limit, hipStream_t stream) {
+  MoeArgs p{(const uint8_t*)w_gu, w_scale, (const uint8_t*)x, x_scale, perm,
+            (const int4*)tiles, n_tiles, choice_w, (const uint16_t*)bias, h,
+            topk, I, fp8 ? H : 2 * H, 0, in_w, gelu,
+            limit};
+  if (fp8)
+    launch_gemm_tm<true>(tm, true, p, max_tiles, stream);
   else
-    moe_gate_up_kernel<false><<<grid, MOE_THREADS, 0, stream>>>(
-        (uint16_t*)h_buf, (const uint16_t*)x, (const uint16_t*)w_gu,
-        tile_expert, tile_row0, perm, seg_offsets, E, topk, H, I, limit,
-        (const uint16_t*)bias_gu, in_w);
+    launch_gemm_tm<false>(tm, true, p, max_tiles, stream);
 }
 
 extern "C" void launch_moe_down(
-    void* out, const void* h_buf, const void* w_down, const float* route_w,
-    const int* tile_expert, const int* tile_row0, const int64_t* perm,
-    const int* seg_offsets, int E, int topk, int H, int I, int max_tiles,
-    hipStream_t stream) {
-  dim3 grid(max_tiles, ceil_div(H, 256), 1);
-  moe_down_kernel<<<grid, MOE_THREADS, 0, stream>>>(
-      (float*)out, (const uint16_t*)h_buf, (const uint16_t*)w_down, route_w,
-      tile_expert, tile_row0, perm, seg_offsets, E, topk, H, I);
+    float* y, const void* h, const float* h_scale, const void* w_down,
+    const float* w_scale, const int* perm, const void* tiles,
+    const int* n_tiles, const float* choice_w, int topk, int H, int I,
+    int max_tiles, int tm, bool fp8, bool in_w, hipStream_t stream) {
+  MoeArgs p{(const uint8_t*)w_down, w_scale, (const uint8_t*)h, h_scale, perm,
+            (const int4*)tiles, n_tiles, choice_w, nullptr, y, topk, H,
+            fp8 ? I : 2 * I, 0, in_w, 0, 0.f};
+  if (fp8)
+    launch_gemm_tm<true>(tm, false, p, max_tiles, stream);
+  else
+    launch_gemm_tm<false>(tm, false, p, max_tiles, stream);
+}
+
+extern "C" void launch_moe_combine(float* out, const float* y,
+                                   const int64_t* ids, int T, int k, int E,
+                                   int H, hipStream_t stream) {
+  dim3 grid(T, T < 256 ? ceil_div(H, 1024) : 1, 1);
+  moe_combine_kernel<<<grid, 256, 0, stream>>>(out, y, ids, T, k, E, H);
 }

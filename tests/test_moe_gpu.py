@@ -149,3 +149,79 @@ def test_moe_engine_graph_capture():
     )
     assert eng.graph_runner is not None and len(eng.graph_runner._graphs) > 0
     assert all(len(v) == 6 for v in out.values())
+
+
+def _experts64(x, gu, dn, ids, w, fp8=False, on_input=False, bias=None,
+               limit=0.0, gelu=False):
+    """The experts in float64 on the device, one at a time; fp8: operands
+    quantised a row before both products."""
+    def q8(t):
+        s = t.abs().amax(-1, keepdim=True).clamp_min(1e-8) / 448.0
+        return (t / s).float().to(torch.float8_e4m3fn).double() * s
+
+    inter = dn.shape[2]
+    xd = q8(x.double()) if fp8 else x.double()
+    out = torch.zeros(x.shape, dtype=torch.float64, device=x.device)
+    for e in range(gu.shape[0]):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        wt = w[t, j].double()[:, None]
+        h = xd[t] @ gu[e].double().T
+        if on_input:
+            h = h * wt
+        if bias is not None:
+            h = h + bias[e].double()
+        g, u = h[:, :inter], h[:, inter:]
+        if limit:
+            g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+            a = (u + 1) * g * torch.sigmoid(1.702 * g)
+        elif gelu:
+            a = torch.nn.functional.gelu(g, approximate="tanh") * u
+        else:
+            a = torch.nn.functional.silu(g) * u
+        a = q8(a.bfloat16().double()) if fp8 else a
+        y = a @ dn[e].double().T
+        out.index_add_(0, t, y if on_input else y * wt)
+    return out
+
+
+@pytest.mark.parametrize("T,E,k,H,I,fp8", [
+    (1, 3, 1, 32, 32, False),       # less than a stage of the contraction
+    (40, 5, 2, 96, 96, False),      # its last stage partly filled
+    (300, 2, 1, 160, 352, False),   # several tiles an expert, odd features
+    (450, 3, 2, 320, 288, False),   # 128-row tiles
+    (5000, 9, 2, 64, 32, False),    # choices counted in parts
+    (40, 5, 2, 96, 64, True),
+    (700, 6, 2, 224, 192, True),
+])
+def test_moe_tiles(T, E, k, H, I, fp8):
+    """Tile heights, remainders of rows, features and contraction, experts
+    without a token and choices of another rank's expert (id E). bf16: h is
+    rounded once, 2^-9 relative, so the error's norm stays below 2^-8 of the
+    result's; fp8: h values next to a rounding edge move by one e4m3 step
+    (2^-3) where the fp32 sums differ in their last bits: below 2 %."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
+    ids = torch.rand(T, E + 1, generator=g, device="cuda")
+    ids[:, E // 2] = -1                       # an expert that nobody chooses
+    ids = ids.topk(k, dim=-1).indices
+    w = torch.rand(T, k, generator=g, device="cuda")
+    if fp8:
+        qg, sg = ops.quantize_fp8_weight(gu)
+        qd, sd = ops.quantize_fp8_weight(dn)
+        got = ops.fused_moe_forward_fp8(x, qg, sg, qd, sd, ids, w)
+        want = _experts64(x, qg.double() * sg[..., None], qd.double() * sd[..., None],
+                          ids, w, fp8=True)
+        assert (got - want).norm() < 2e-2 * want.norm()
+        return
+    for kw in ({}, {"on_input": True}, {"limit": 7.0}, {"gelu": True}):
+        bias = (torch.randn(E, 2 * I, generator=g, device="cuda").bfloat16()
+                if "limit" in kw else None)
+        got = ops.fused_moe_forward(
+            x, gu, dn, ids, w, activation="gelu" if kw.get("gelu") else "silu",
+            limit=kw.get("limit", 0.0), bias_gate_up=bias,
+            weight_on_input=kw.get("on_input", False))
+        want = _experts64(x, gu, dn, ids, w, bias=bias, **kw)
+        assert (got - want).norm() < 2 ** -8 * want.norm()
+    assert ops.fused_moe_forward(x[:0], gu, dn, ids[:0], w[:0]).shape == (0, H)
