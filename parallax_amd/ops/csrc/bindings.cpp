@@ -44,8 +44,9 @@ void launch_paged_attention_reduce(void*, const float*, const float*, int, int,
 void launch_mla_paged_attention_decode(void*, const void*, const void*,
                                        const void*, const int*, const int*,
                                        int, int, int, int, int, int, float,
-                                       int, int, float*, float*, const int*,
-                                       int, bool, float, hipStream_t, bool*);
+                                       int, float*, float*, const int*, int,
+                                       bool, float, hipStream_t, bool*);
+int mla_decode_runs(int, int, int);
 void launch_msa_paged_attention_decode(void*, const void*, const void*,
                                        const void*, const int*, const int*,
                                        const int*, int, int, int, int, int,
@@ -392,27 +393,6 @@ void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,
   const int max_blocks = block_tables.size(1);
   TORCH_CHECK(cache.size(2) == R + DR, "cache entry dim mismatch");
 
-  // same grid-fill-aware partition sizing as the GQA decode path
-  const int mla_wg_base = B * ((H + 31) / 32);  // MLA_HBLOCK = 32
-  int part_tokens = 256;
-  if (mla_wg_base >= 4096) part_tokens = 2048;
-  else if (mla_wg_base >= 1024) part_tokens = 1024;
-  else if (mla_wg_base >= 512) part_tokens = 512;
-  int num_parts = (int)((max_seq_len + part_tokens - 1) / part_tokens);
-  if (num_parts > 128) {
-    part_tokens = (int)((max_seq_len + 127) / 128);
-    part_tokens = (part_tokens + 127) / 128 * 128;
-    num_parts = (int)((max_seq_len + part_tokens - 1) / part_tokens);
-  }
-  torch::Tensor tmp_acc, tmp_ml;
-  float *acc_ptr = nullptr, *ml_ptr = nullptr;
-  if (num_parts > 1) {
-    auto opts = q_latent.options().dtype(at::kFloat);
-    tmp_acc = torch::empty({B, H, num_parts, R}, opts);
-    tmp_ml = torch::empty({B, H, num_parts, 2}, opts);
-    acc_ptr = tmp_acc.data_ptr<float>();
-    ml_ptr = tmp_ml.data_ptr<float>();
-  }
   const int* idx_ptr = nullptr;
   int max_topk = 0;
   if (topk_indices.numel() > 0) {
@@ -421,16 +401,26 @@ void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,
     idx_ptr = topk_indices.data_ptr<int>();
     max_topk = topk_indices.size(1);
   }
+  // Every part of a sequence is named by (run + sequence); see the kernel.
+  const int runs = mla_decode_runs(
+      B, H, (int)std::max<int64_t>(max_seq_len, max_topk));
+  torch::Tensor tmp_acc, tmp_ml;
+  float *acc_ptr = nullptr, *ml_ptr = nullptr;
+  if (runs > 0) {
+    auto opts = q_latent.options().dtype(at::kFloat);
+    tmp_acc = torch::empty({(int64_t)runs + B, H, R}, opts);
+    tmp_ml = torch::empty({(int64_t)runs + B, H, 2}, opts);
+    acc_ptr = tmp_acc.data_ptr<float>();
+    ml_ptr = tmp_ml.data_ptr<float>();
+  }
+  if (B == 0) return;
   bool launched = false;
   launch_mla_paged_attention_decode(
       out.data_ptr(), q_latent.data_ptr(), q_pe.data_ptr(), cache.data_ptr(),
       block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, H, R, DR, BS,
-      max_blocks, (float)scale, num_parts, part_tokens, acc_ptr, ml_ptr,
-      idx_ptr, max_topk, is_fp8(cache), 1.0f, cur_stream(), &launched);
+      max_blocks, (float)scale, runs, acc_ptr, ml_ptr, idx_ptr, max_topk,
+      is_fp8(cache), 1.0f, cur_stream(), &launched);
   TORCH_CHECK(launched, "no MLA kernel for R=", R, " DR=", DR, " BS=", BS);
-  if (num_parts > 1)
-    launch_paged_attention_reduce(out.data_ptr(), acc_ptr, ml_ptr, B, H, R,
-                                  num_parts, nullptr, cur_stream());
 }
 
 // Routed experts of x [T, H]: bf16, or fp8 (W8A8) with w_gu_scale / w_down_scale

@@ -1,326 +1,630 @@
-// DeepSeek MLA decode attention over the compressed latent cache — MFMA/CDNA4.
+// MLA decode attention over the compressed latent cache for gfx950.
 //
-//   S^T[32tok x 32heads] = C_tile · Q^T   (C = [latent | rope] rows, 576 dims;
-//                                          Q fragments read straight from
-//                                          q_latent/q_pe global — L1-resident)
-//   O^T[512 x 32heads]  += C_v^T · P      (latent transposed during staging)
+//   S^T[64 tok x 16 heads] = C . Q^T     C = [latent | rope] rows, 576 values
+//   O^T[512 x 16 heads]   += C_v^T . P   C_v = the latent part of the same rows
+// All query heads share ONE cache row a token; a workgroup takes 64 heads (16 a
+// wave, Q and O^T in registers). With 128 heads two workgroups read a row, at
+// the same time and through one XCD's L2: 128 heads a workgroup need 512
+// registers a wave, which the compiler spilled.
+// Tiles of 64 tokens are copied global -> LDS directly, the next one while this
+// one is computed. Both products read the one copy: S^T's operand rows are token rows; O^T's operand
+// is transposed on the way out of LDS (ds_read_b64_tr_b16), and in the order in
+// which the accumulators of S^T hold their tokens, so P stays in registers.
+// 16-byte chunks are XOR-swizzled so that both kinds of read spread over the
+// banks. An fp8 cache is widened on its way through registers.
 //
-// All query heads share ONE latent cache (MQA-like), so arithmetic intensity is
-// ~240 flop/byte — compute-bound, hence matrix cores. A workgroup covers a
-// 32-head block; the cache tile re-read across the H/32 head-block workgroups
-// of a sequence is L2/L3-absorbed. Fixed-size context partitions (graph-stable)
-// combine through the shared reduce kernel.
+// Work is split by tiles, not by sequences: the tiles of all sequences form one
+// list, of which every workgroup takes an equal run. Lengths are read on the
+// device, so a captured step balances for any lengths. A sequence that lies in
+// one run is finished there; the others leave fp32 parts that a second kernel
+// adds up. Short sequences (256 tokens at most) take a workgroup each and need
+// no second kernel.
+//
+// What bounds it: the waves of a workgroup go through a tile in step (operands out
+// of LDS, products, softmax), 37% of the matrix cores' time at 64 heads; with 16
+// heads the latent rows, 4.2 TB/s. Measured (before: single-buffered tiles
+// transposed value by value into LDS, fixed partitions of the context): 64 heads,
+// 4 x 100,000 tokens 111 us (613); 128 heads, 40 x 4,000 78 us (351); 16 heads, 64
+// x 6,000 69 us (230); 128 heads, one sequence of 1,000 22 us (57).
 //
 // Reference analogue: parallax_extensions/kernels/mla/ (Metal, VALU); fresh
 // MFMA design. Layout: cache [NB, BS, R+DR], q_latent [B, H, R], q_pe [B, H, DR].
 
 #include "common.h"
 
-#define MLA_THREADS 256
-#define MLA_KTILE 32
-#define MLA_HBLOCK 32
+#define MLA_R 512
+#define MLA_DR 64
+#define MLA_DK 576          // values a cache row
+#define MLA_CH 72           // 16-byte chunks a row
+#define MLA_KT 64           // tokens a tile
+#define MLA_DT 16           // 16-value tiles of O^T a wave
+#define MLA_MIN_TILES 2     // a run is at least this long
+#define MLA_MAX_RUNS 256    // one a CU
 
-template <int R, int DR, int BLOCK_SIZE, bool PARTITIONED, bool SPARSE,
-          bool KV_FP8 = false>
-__global__ __launch_bounds__(MLA_THREADS) void mla_decode_kernel(
-    uint16_t* __restrict__ out,       // [B, H, R]
-    float* __restrict__ tmp_acc,      // [B, H, P, R]
-    float* __restrict__ tmp_ml,      // [B, H, P, 2]
+// the lambdas below are called once a buffer: left out of line, their captures
+// would live in scratch
+#define INL __attribute__((always_inline))
+
+typedef short s16x4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2n __attribute__((ext_vector_type(2)));
+
+namespace {
+
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kHidden = -1e30f;
+
+DEVINL uint32_t pack_bf16(float a, float b) {
+  bf16x2n p;
+  p[0] = (__bf16)a;
+  p[1] = (__bf16)b;
+  return __builtin_bit_cast(uint32_t, p);
+}
+
+DEVINL void copy16_to_lds(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)src,
+      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// over the four lanes that hold one head (l, l + 16, l + 32, l + 48)
+template <class F>
+DEVINL float over_head(float v, F f) {
+  const auto a = __builtin_amdgcn_permlane16_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// Chunk c of row r lies at chunk_at(r, c). A row of 72 chunks is 8 modulo a turn
+// of 16 over the banks, so row bit 0 does its part; the other bits move pairs of
+// chunks, which spreads both kinds of read: transposing ones, where half a wave
+// takes two chunks of 8 rows, and 16-byte ones, which go by lanes {0-3, 12-15,
+// 20-23, 24-27} and so on: 8 rows of one chunk and 8 others of the next.
+DEVINL int row_xor(int r) { return ((r >> 1) & 3) << 1; }
+DEVINL int chunk_at(int r, int c) { return (c & ~7) | ((c & 7) ^ row_xor(r)); }
+
+// tiles of sequence b: its tokens, or its list of token positions
+template <bool SPARSE>
+DEVINL int domain_of(const int* seq_lens, const int* topk, int max_topk,
+                     int b) {
+  if (SPARSE && topk[(size_t)b * max_topk] >= 0) return max_topk;
+  return max(seq_lens[b], 0);
+}
+
+// A sequence and its place in the list of all tiles, found by one wave: the
+// sequence with first <= tile < first + tiles. Returns the total of tiles.
+template <bool SPARSE>
+DEVINL int find_tile(const int* seq_lens, const int* topk, int max_topk, int B,
+                     int tile, int* seq, int* first) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  *seq = -1;
+  *first = 0;
+  for (int b0 = 0; b0 < B; b0 += 64) {
+    const int b = b0 + lane;
+    const int n =
+        b < B ? (domain_of<SPARSE>(seq_lens, topk, max_topk, b) + MLA_KT - 1) /
+                    MLA_KT
+              : 0;
+    int sum = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(sum, o, WAVE_SIZE);
+      if (lane >= o) sum += t;
+    }
+    const int t = tile - before;
+    const unsigned long long hit = __ballot(t >= sum - n && t < sum);
+    if (hit) {
+      const int src = __ffsll(hit) - 1;
+      *seq = b0 + src;
+      *first = before + __shfl(sum, src, WAVE_SIZE) -
+               __shfl(n, src, WAVE_SIZE);
+    }
+    before += __shfl(sum, 63, WAVE_SIZE);
+  }
+  return before;
+}
+
+DEVINL int run_length(int total, int runs) {
+  return max((total + runs - 1) / runs, MLA_MIN_TILES);
+}
+
+}  // namespace
+
+template <int W, bool KV_FP8, bool SPARSE>
+__global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
+    uint16_t* __restrict__ out,             // [B, H, R]
+    float* __restrict__ tmp_acc,            // [parts, H, R]; null: a workgroup
+    float* __restrict__ tmp_ml,             // [parts, H, 2]      a sequence
     const uint16_t* __restrict__ q_latent,  // [B, H, R]
     const uint16_t* __restrict__ q_pe,      // [B, H, DR]
-    const void* __restrict__ cache_v,       // [NB, BS, R+DR] bf16 | fp8(e4m3)
-    const int* __restrict__ block_tables,
+    const void* __restrict__ cache,         // [NB, BS, R+DR] bf16 | fp8(e4m3)
+    const int* __restrict__ block_tables,   // [B, max_blocks]
     const int* __restrict__ seq_lens,
-    const int max_blocks, const int H, const float scale,
-    const int part_tokens,
-    const int* __restrict__ topk_indices,  // [B, max_topk] (SPARSE only)
-    const int max_topk, const float c_scale = 1.f) {
-  constexpr int DK = R + DR;            // 576
-  constexpr int KSTEPS = DK / 32;       // 18
-  constexpr int PROW = 40;              // padded row length (bank spread)
-  const int hb = blockIdx.x;            // head block (32 heads)
-  const int seq = blockIdx.y;
-  const int L = seq_lens[seq];
-  // DSA sparse mode: iterate the top-k index list; a row starting with -1
-  // falls back to dense (reference dsa_paged_attention semantics)
-  const int* idx_row = SPARSE ? topk_indices + (size_t)seq * max_topk : nullptr;
-  const bool sparse_row = SPARSE && idx_row[0] >= 0;
-  const int domain = sparse_row ? max_topk : L;
-
-  int tok_begin = 0, tok_end = domain;
-  if (PARTITIONED) {
-    const int p = blockIdx.z;
-    tok_begin = max(tok_begin, p * part_tokens);
-    tok_end = min(tok_end, (p + 1) * part_tokens);
-  }
+    const int* __restrict__ topk,           // [B, max_topk] (SPARSE)
+    const int max_topk, const int B, const int max_blocks, const int H,
+    const int bs_shift, const float scale, const float c_scale) {
+  constexpr int COPIES = MLA_KT * MLA_CH / 64;   // 72 of 64 chunks each
+  constexpr int CPW = COPIES / W;                // a wave
+  constexpr int BUF = MLA_KT * MLA_DK;
+  __shared__ __attribute__((aligned(16))) uint16_t S0[BUF];
+  __shared__ __attribute__((aligned(16))) uint16_t S1[BUF];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wid = tid >> 6;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15;
   const int l4 = lane >> 4;
+  const int BS = 1 << bs_shift;
 
-  if (tok_begin >= tok_end) {
-    if (PARTITIONED) {
-      const int p = blockIdx.z;
-      for (int i = tid; i < MLA_HBLOCK; i += MLA_THREADS) {
-        const int h = hb * MLA_HBLOCK + i;
-        if (h < H) {
-          float* ml = tmp_ml + (((size_t)seq * H + h) * gridDim.z + p) * 2;
-          ml[0] = -1e30f;
-          ml[1] = 0.f;
-        }
+  // ---- this workgroup's run of tiles --------------------------------------------
+  int seq, at, todo;  // sequence, tile of it, tiles left
+  if (tmp_acc == nullptr) {
+    seq = blockIdx.x;
+    at = 0;
+    todo = (domain_of<SPARSE>(seq_lens, topk, max_topk, seq) + MLA_KT - 1) /
+           MLA_KT;
+  } else {
+    int first;
+    const int total = find_tile<SPARSE>(seq_lens, topk, max_topk, B, 0, &seq,
+                                        &first);
+    const int per = run_length(total, gridDim.x);
+    const int begin = blockIdx.x * per;
+    todo = min(per, total - begin);
+    if (todo > 0)
+      find_tile<SPARSE>(seq_lens, topk, max_topk, B, begin, &seq, &first);
+    at = begin - first;
+  }
+  seq = __builtin_amdgcn_readfirstlane(seq);
+  at = __builtin_amdgcn_readfirstlane(at);
+  todo = __builtin_amdgcn_readfirstlane(todo);
+
+  // two waves share 16 heads: both compute S^T, each half of the latent values
+  const int head0 = (blockIdx.y * (W / 2) + (wid >> 1)) * 16;
+  const int head = head0 + l15;
+  const int d0 = (wid & 1) * (MLA_R / 2);
+
+  // what a lane reads of a tile: S^T's operand has two places in a group of
+  // eight chunks, O^T's has four; the groups follow at 64 values
+  int qk_at[2], tr_at[4];
+  {
+    const int r = 4 * l4 + (l15 >> 2);  // token row of a transposing read
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      qk_at[i] = l15 * MLA_DK + chunk_at(l15, i * 4 + l4) * 8;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      tr_at[i] = r * MLA_DK + d0 + chunk_at(r, i * 2 + ((l15 & 3) >> 1)) * 8 +
+                 (l15 & 1) * 4;
+  }
+
+  while (todo > 0) {
+    const int* btab = block_tables + (size_t)seq * max_blocks;
+    const int L = seq_lens[seq];
+    const int dom = domain_of<SPARSE>(seq_lens, topk, max_topk, seq);
+    const bool listed = SPARSE && dom == max_topk &&
+                        topk[(size_t)seq * max_topk] >= 0;
+    const int* list = SPARSE ? topk + (size_t)seq * max_topk : nullptr;
+    const int tiles = (dom + MLA_KT - 1) / MLA_KT;
+    if (at >= tiles) {  // a sequence without tokens
+      ++seq;
+      at = 0;
+      continue;
+    }
+    const int t0 = at;
+    const int t1 = min(tiles, at + todo);
+
+    // ---- Q: B operands, head l15, values 32 ks + 8 l4 + (0..7) -------------------
+    bf16x8v qf[MLA_DK / 32];
+    {
+      const size_t row = (size_t)seq * H + min(head, H - 1);
+#pragma unroll
+      for (int ks = 0; ks < MLA_DK / 32; ++ks) {
+        const int k = ks * 32 + l4 * 8;
+        qf[ks] = ks < MLA_R / 32
+                     ? *(const bf16x8v*)(q_latent + row * MLA_R + k)
+                     : *(const bf16x8v*)(q_pe + row * MLA_DR + k - MLA_R);
       }
     }
-    return;
-  }
+    f32x4v acc[MLA_DT] = {};
+    float m = kHidden, l = 0.f;
+    const float c = scale * kLog2e;
 
-  __shared__ uint16_t Cl[MLA_KTILE * DK];        // row = token (1152 B), swz
-  __shared__ uint16_t VTl[R * PROW];             // row = latent dim, 80 B pad
-  __shared__ uint16_t Pl[MLA_HBLOCK * PROW];     // row = head, 80 B pad
-  __shared__ float m_s[MLA_HBLOCK], l_s[MLA_HBLOCK], resc[MLA_HBLOCK];
-  __shared__ float wred[4][MLA_HBLOCK];
-
-  if (tid < MLA_HBLOCK) {
-    m_s[tid] = -3.0e4f;
-    l_s[tid] = 0.f;
-  }
-
-  // O^T acc: wave w owns latent rows [128w, 128w+128) = 8 M-tiles x 2 N-tiles
-  constexpr int MT = R / 16 / 4;  // 8
-  f32x4v acc_o[MT][2] = {};
-
-  const int* btab = block_tables + (size_t)seq * max_blocks;
-  const int kt_begin = tok_begin / MLA_KTILE;
-  const int kt_end = (tok_end + MLA_KTILE - 1) / MLA_KTILE;
-
-  for (int kt = kt_begin; kt < kt_end; ++kt) {
-    const int kbase = kt * MLA_KTILE;
-    __syncthreads();
-
-    // ---- stage C rows (swz) + transposed latent (padded rows) ------------------
-    {
-      const int tok = tid & 31;
-      const int dv = tid >> 5;  // 8 slices of 72 dims (9 int4 each)
-      const int j = kbase + tok;
-      int gtok = j;
-      bool ok = j >= tok_begin && j < tok_end;
-      if (sparse_row && ok) {
-        gtok = idx_row[j];
-        ok = gtok >= 0 && gtok < L;
-      }
-      size_t crow_tok = 0;
-      if (ok) {
-        const int blk = btab[gtok / BLOCK_SIZE];
-        const int off = gtok % BLOCK_SIZE;
-        crow_tok = (size_t)blk * BLOCK_SIZE + off;
-      }
+    // ---- copies --------------------------------------------------------------------
+    // a list entry outside [0, L) stands for no token; its row reads token 0
+    auto entry = [&](int j) INL { return j < dom ? list[j] : -1; };
+    auto slot_of = [&](int tok) INL -> int {
+      return (btab[tok >> bs_shift] << bs_shift) + (tok & (BS - 1));
+    };
+    // cache row (token slot) of tile row `lane`, listed
+    auto listed_slot = [&](int t) INL {
+      const int e = entry(t * MLA_KT + lane);
+      return slot_of(e >= 0 && e < L ? e : 0);
+    };
+    constexpr int ESZ = KV_FP8 ? 1 : 2;
+    // where the copies of tile t read: a base that all lanes share, and 32 bits.
+    // 16 rows lie in one page and are 18 copies; rows past the end read a page
+    // that is there.
+    auto each_copy = [&](int t, auto&& use) INL {
+      // worked out anew for every tile: nine more registers would spill
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      int base[MLA_KT / 16], mine = 0;
+      if (listed) mine = listed_slot(t);
 #pragma unroll
-      for (int c = 0; c < 9; ++c) {
-        const int d = (dv * 9 + c) * 8;
-        int4 val = make_int4(0, 0, 0, 0);
-        if (ok) {
-          if (KV_FP8) {
-            // 8 fp8 bytes -> 8 bf16 (one cache-wide scale), packed converts
-            const uint64_t raw = *reinterpret_cast<const uint64_t*>(
-                (const uint8_t*)cache_v + crow_tok * DK + d);
-            fp8x8_to_bf16x8(raw, c_scale, reinterpret_cast<uint16_t*>(&val));
-          } else {
-            val = *reinterpret_cast<const int4*>(
-                (const uint16_t*)cache_v + crow_tok * DK + d);
-          }
+      for (int g = 0; g < MLA_KT / 16; ++g)
+        base[g] = listed ? 0
+                         : slot_of(min(t * MLA_KT + 16 * g, (L - 1) & ~15)) -
+                               16 * g;
+#pragma unroll
+      for (int i = 0; i < CPW; ++i) {
+        const int k = wid + W * i;
+        const int ch = k * 64 + ln;
+        const int row = ch / MLA_CH;
+        const int at = row * MLA_DK + chunk_at(row, ch % MLA_CH) * 8;
+        const uint8_t* src = (const uint8_t*)cache;
+        if (SPARSE && listed) {
+          const int slot = __shfl(mine, row, WAVE_SIZE) - row;
+          src += ((int64_t)slot * MLA_DK + at) * ESZ;
+        } else {
+          const int b = k < 36 ? (k < 18 ? base[0] : base[1])
+                               : (k < 54 ? base[2] : base[3]);
+          src += (int64_t)b * (MLA_DK * ESZ);
+          src += (uint32_t)(at * ESZ);
         }
-        const int byte = swz(tok * DK * 2 + d * 2, tok);
-        *reinterpret_cast<int4*>(reinterpret_cast<char*>(Cl) + byte) = val;
-        const uint16_t* vs = reinterpret_cast<const uint16_t*>(&val);
+        use(i, k, src);
+      }
+    };
+    auto issue = [&](int t, uint16_t* S) INL {
+      each_copy(t, [&](int, int k, const uint8_t* src) INL {
+        copy16_to_lds(src, S + k * 512);
+      });
+    };
+    uint64_t raw[KV_FP8 ? CPW : 1];
+    auto fetch8 = [&](int t) INL {
+      each_copy(t, [&](int i, int, const uint8_t* src) INL {
+        raw[KV_FP8 ? i : 0] = *(const uint64_t*)src;
+      });
+    };
+    auto widen8 = [&](uint16_t* S) INL {
+      int at = lane * 8;
+      asm volatile("" : "+v"(at));
+#pragma unroll
+      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i) {
+        int4 v;
+        fp8x8_to_bf16x8(raw[i], c_scale, reinterpret_cast<uint16_t*>(&v));
+        *reinterpret_cast<int4*>(S + (wid + W * i) * 512 + at) = v;
+      }
+    };
+
+    // ---- one tile --------------------------------------------------------------------
+    auto compute = [&](int t, uint16_t* S) INL {
+      // rows that stand for a token, one bit each
+      uint64_t alive = ~0ull;
+      if (listed) {
+        const int e = entry(t * MLA_KT + lane);
+        alive = __ballot(e >= 0 && e < L);
+      } else if (dom - t * MLA_KT < MLA_KT) {
+        alive = (1ull << (dom - t * MLA_KT)) - 1;
+      }
+      if (alive != ~0ull) {  // the others may hold anything: weight 0 times it
+        int i0 = tid;
+        asm volatile("" : "+v"(i0));
+        for (int i = i0; i < MLA_KT * MLA_CH; i += W * 64)
+          if (!((alive >> (i / MLA_CH)) & 1))
+            *reinterpret_cast<int4*>(S + i * 8) = make_int4(0, 0, 0, 0);
+        __syncthreads();
+      }
+      if (head0 >= H) return;  // copies only
+
+      // opaque, or the addresses of every buffer are kept in registers
+      int qk[2] = {qk_at[0], qk_at[1]};
+      int tr[4] = {tr_at[0], tr_at[1], tr_at[2], tr_at[3]};
+      asm volatile("" : "+v"(qk[0]), "+v"(qk[1]), "+v"(tr[0]), "+v"(tr[1]),
+                   "+v"(tr[2]), "+v"(tr[3]));
+      // Operands come in batches, the next one under way while this one's
+      // products run: one read at a time would wait out the LDS each time.
+      auto landed = [] INL {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      constexpr int KB = KV_FP8 ? 1 : 2;  // of the 18 steps of S^T
+      constexpr int TU = MLA_KT / 16;
+      f32x4v s[TU] = {};
+      {
+        bf16x8v a[2][KB][TU];
+        auto fetch = [&](int n) INL {
+#pragma unroll
+          for (int i = 0; i < KB; ++i)
+#pragma unroll
+            for (int u = 0; u < TU; ++u) {
+              const int ks = n * KB + i;
+              a[n & 1][i][u] = *reinterpret_cast<const bf16x8v*>(
+                  S + qk[ks & 1] + (ks >> 1) * 64 + u * 16 * MLA_DK);
+            }
+        };
+        fetch(0);
+#pragma unroll
+        for (int n = 0; n < MLA_DK / 32 / KB; ++n) {
+          landed();
+          if (n + 1 < MLA_DK / 32 / KB) fetch(n + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < KB; ++i)
+#pragma unroll
+            for (int u = 0; u < TU; ++u)
+              s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  a[n & 1][i][u], qf[n * KB + i], s[u], 0, 0, 0);
+        }
+      }
+      float mx = kHidden;
+      if (alive == ~0ull) {
+#pragma unroll
+        for (int u = 0; u < TU; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            s[u][r] *= c;
+            mx = fmaxf(mx, s[u][r]);
+          }
+      } else {
+        const uint64_t mine = alive >> (l4 * 4);
+#pragma unroll
+        for (int u = 0; u < TU; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            s[u][r] = (mine >> (u * 16 + r)) & 1 ? s[u][r] * c : kHidden;
+            mx = fmaxf(mx, s[u][r]);
+          }
+      }
+      mx = over_head(mx, [](float x, float y) { return fmaxf(x, y); });
+      // rescaled only when a maximum moved by more than 2^8
+      if (__any(mx > m + 8.f)) {
+        const float m2 = fmaxf(m, mx);
+        const float f = __builtin_amdgcn_exp2f(m - m2);
+        m = m2;
+        l *= f;
+#pragma unroll
+        for (int d = 0; d < MLA_DT; ++d) acc[d] *= f;
+      }
+      bf16x8v b[TU / 2];
+#pragma unroll
+      for (int n = 0; n < TU / 2; ++n) {
+        float p[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const int dd = d + j;
-          if (dd < R)
-            VTl[dd * PROW + tok] = vs[j];
+          p[j] = __builtin_amdgcn_exp2f(s[2 * n + (j >> 2)][j & 3] - m);
+          l += p[j];
+        }
+        uint32_t pk[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) pk[j] = pack_bf16(p[2 * j], p[2 * j + 1]);
+        b[n] = *reinterpret_cast<const bf16x8v*>(pk);
+      }
+
+      // O^T: rows = 16 latent values, contraction over tokens 4 l4 + (0..3) and
+      // 16 more: what lane group l4 of S^T holds
+      constexpr int DB = 2;  // of a wave's latent tiles
+      {
+        bf16x8v a[2][DB][TU / 2];
+        auto fetch = [&](int n) INL {
+#pragma unroll
+          for (int i = 0; i < DB; ++i)
+#pragma unroll
+            for (int u = 0; u < TU / 2; ++u) {
+              const int d = n * DB + i;
+              uint16_t* src =
+                  S + tr[d & 3] + (d >> 2) * 64 + u * 32 * MLA_DK;
+              const s16x4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                  (__attribute__((address_space(3))) s16x4v*)src);
+              const s16x4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                  (__attribute__((address_space(3))) s16x4v*)(src +
+                                                              16 * MLA_DK));
+              a[n & 1][i][u] =
+                  __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+        };
+        fetch(0);
+#pragma unroll
+        for (int n = 0; n < MLA_DT / DB; ++n) {
+          landed();
+          if (n + 1 < MLA_DT / DB) fetch(n + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int u = 0; u < TU / 2; ++u)
+#pragma unroll
+            for (int i = 0; i < DB; ++i)
+              acc[n * DB + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  a[n & 1][i][u], b[u], acc[n * DB + i], 0, 0, 0);
+        }
+      }
+    };
+
+    // ---- the run, one barrier a tile -----------------------------------------------
+    // Behind it this tile is in LDS, and every wave has left the buffer that the
+    // next one goes to.
+    __syncthreads();  // the buffers may still be read for the last sequence
+    auto turn = [&](int t, uint16_t* S, uint16_t* Sn) INL {
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's copies
+      __syncthreads();
+      const bool more = t + 1 < t1;
+      if (more) {
+        if constexpr (KV_FP8) fetch8(t + 1);
+        else issue(t + 1, Sn);
+      }
+      compute(t, S);
+      if constexpr (KV_FP8)
+        if (more) widen8(Sn);
+    };
+    if constexpr (KV_FP8) {
+      fetch8(t0);
+      widen8(S0);
+    } else {
+      issue(t0, S0);
+    }
+    for (int t = t0; t < t1;) {
+      turn(t, S0, S1);
+      if (++t >= t1) break;
+      turn(t, S1, S0);
+      ++t;
+    }
+
+    // ---- results: column = head, rows = latent values --------------------------------
+    l = over_head(l, [](float x, float y) { return x + y; });
+    if (head < H) {
+      if (t0 == 0 && t1 == tiles) {
+        const float inv = 1.f / l;
+        uint16_t* o = out + ((size_t)seq * H + head) * MLA_R + d0 + l4 * 4;
+#pragma unroll
+        for (int d = 0; d < MLA_DT; ++d) {
+          uint2 v;
+          v.x = pack_bf16(acc[d][0] * inv, acc[d][1] * inv);
+          v.y = pack_bf16(acc[d][2] * inv, acc[d][3] * inv);
+          *reinterpret_cast<uint2*>(o + d * 16) = v;
+        }
+      } else {
+        // runs and sequences both advance: their sum names a part
+        const size_t part = ((size_t)blockIdx.x + seq) * H + head;
+        float* o = tmp_acc + part * MLA_R + d0 + l4 * 4;
+#pragma unroll
+        for (int d = 0; d < MLA_DT; ++d)
+          *reinterpret_cast<f32x4v*>(o + d * 16) = acc[d];
+        if (l4 == 0 && d0 == 0) {
+          tmp_ml[part * 2] = m;  // in units of log2
+          tmp_ml[part * 2 + 1] = l;
         }
       }
     }
-    __syncthreads();
-
-    // ---- S^T[32tok x 32h] = C . Q^T ---------------------------------------------
-    // waves: w>>1 selects the 16-token M strip, w&1 selects the 16-head N strip
-    const int mw = wid >> 1;  // 0..1
-    const int nw = wid & 1;   // 0..1
-    f32x4v acc_s = {};
-    const int head = hb * MLA_HBLOCK + nw * 16 + l15;
-    const bool head_ok = head < H;
-#pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) {
-      const int trow = mw * 16 + l15;
-      const int ca = swz(trow * DK * 2 + s * 64 + l4 * 16, trow);
-      const bf16x8v afrag = *reinterpret_cast<const bf16x8v*>(
-          reinterpret_cast<const char*>(Cl) + ca);
-      bf16x8v bfrag = {};
-      if (head_ok) {
-        const int k = s * 32 + l4 * 8;
-        if (k < R)
-          bfrag = *reinterpret_cast<const bf16x8v*>(
-              q_latent + ((size_t)seq * H + head) * R + k);
-        else
-          bfrag = *reinterpret_cast<const bf16x8v*>(
-              q_pe + ((size_t)seq * H + head) * DR + (k - R));
-      }
-      acc_s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, bfrag, acc_s, 0, 0, 0);
-    }
-
-    // ---- mask + softmax (per head column, online) ------------------------------
-    float mx = -3.0e4f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int j = kbase + mw * 16 + l4 * 4 + r;
-      float s = acc_s[r] * scale;
-      bool vis = j >= tok_begin && j < tok_end && head_ok;
-      if (sparse_row && vis) {
-        const int gt = idx_row[j];
-        vis = gt >= 0 && gt < L;
-      }
-      s = vis ? s : -3.0e4f;
-      acc_s[r] = s;
-      mx = fmaxf(mx, s);
-    }
-    // same head column lives in lanes {c, c+16, c+32, c+48} of this wave
-    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
-    if (lane < 16) wred[wid][nw * 16 + lane] = mx;
-    __syncthreads();
-    if (tid < MLA_HBLOCK) {
-      // waves (0,2) cover N strip 0; (1,3) N strip 1 — combine the two M strips
-      const int nwi = tid >> 4;
-      const float m_chunk = fmaxf(wred[nwi][tid], wred[nwi + 2][tid]);
-      const float m_new = fmaxf(m_s[tid], m_chunk);
-      resc[tid] = __expf(m_s[tid] - m_new);
-      m_s[tid] = m_new;
-    }
-    __syncthreads();
-
-    float sm = 0.f;
-    {
-      const float m = m_s[nw * 16 + l15];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = __expf(acc_s[r] - m);
-        sm += p;
-        const int kk = mw * 16 + l4 * 4 + r;
-        Pl[(nw * 16 + l15) * PROW + kk] = f32_to_bf16_bits(p);
-      }
-      sm += __shfl_xor(sm, 16, WAVE_SIZE);
-      sm += __shfl_xor(sm, 32, WAVE_SIZE);
-    }
-    if (lane < 16) wred[wid][nw * 16 + lane] = sm;
-    __syncthreads();
-    if (tid < MLA_HBLOCK) {
-      const int nwi = tid >> 4;
-      l_s[tid] = l_s[tid] * resc[tid] + wred[nwi][tid] + wred[nwi + 2][tid];
-    }
-    __syncthreads();
-
-    // ---- O^T += C_v^T . P --------------------------------------------------------
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const float rsc = resc[nt * 16 + l15];
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) acc_o[mt][nt][rr] *= rsc;
-      }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int rrow = wid * (R / 4) + mt * 16 + l15;
-      const bf16x8v afrag = *reinterpret_cast<const bf16x8v*>(
-          VTl + rrow * PROW + l4 * 8);
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const bf16x8v bfrag = *reinterpret_cast<const bf16x8v*>(
-            Pl + (nt * 16 + l15) * PROW + l4 * 8);
-        acc_o[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            afrag, bfrag, acc_o[mt][nt], 0, 0, 0);
-      }
-    }
+    todo -= t1 - t0;
+    ++seq;
+    at = 0;
   }
+}
 
-  // ---- write out (O^T: col = head, row = latent dim) ------------------------------
+// Adds up the parts of the sequences that several runs share: four groups of 128
+// threads, a thread four values. Few sequences (BY_HEAD false) have many parts:
+// a workgroup a head, the groups share its parts. Many have few: a group a head.
+// Measured, 64 heads x 4 sequences x 64 parts: 8.5 us (54 us as a serial loop
+// over the parts); 128 heads x 256 sequences of two parts: 28 us.
+template <bool SPARSE, bool BY_HEAD>
+__global__ __launch_bounds__(512) void mla_reduce_kernel(
+    uint16_t* __restrict__ out, const float* __restrict__ tmp_acc,
+    const float* __restrict__ tmp_ml, const int* __restrict__ seq_lens,
+    const int* __restrict__ topk, const int max_topk, const int B, const int H,
+    const int runs) {
+  const int seq = blockIdx.y;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, grp = tid >> 7;
+  const int head = BY_HEAD ? blockIdx.x * 4 + grp : blockIdx.x;
+  int total = 0, first = 0;  // tiles of all sequences, of those before this one
+  for (int b = lane; b < B; b += 64) {
+    const int n =
+        (domain_of<SPARSE>(seq_lens, topk, max_topk, b) + MLA_KT - 1) / MLA_KT;
+    total += n;
+    first += b < seq ? n : 0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    total += __shfl_xor(total, o, WAVE_SIZE);
+    first += __shfl_xor(first, o, WAVE_SIZE);
+  }
+  const int tiles =
+      (domain_of<SPARSE>(seq_lens, topk, max_topk, seq) + MLA_KT - 1) / MLA_KT;
+  if (tiles == 0) return;
+  const int per = run_length(total, runs);
+  const int r0 = first / per, r1 = (first + tiles - 1) / per;
+  if (r0 == r1) return;  // finished by its run
+
+  __shared__ f32x4v sums[4][128];
+  __shared__ float wt[BY_HEAD ? 4 : 1][MLA_MAX_RUNS];
+  const int parts = r1 - r0 + 1;
+  const bool on = head < H;
+  const size_t first_part = ((size_t)r0 + seq) * H + (on ? head : 0);
+  // the weights, worked out by each wave for itself, written by one of them
+  float M = kHidden, l = 0.f;
+  for (int r = lane; r < parts; r += 64)
+    M = fmaxf(M, tmp_ml[(first_part + (size_t)r * H) * 2]);
+  M = wave_reduce_max(M);
+  for (int r = lane; r < parts; r += 64) {
+    const float* ml = tmp_ml + (first_part + (size_t)r * H) * 2;
+    const float w = __builtin_amdgcn_exp2f(ml[0] - M);
+    l += ml[1] * w;
+    if ((BY_HEAD ? tid & 127 : tid) < 64) wt[BY_HEAD ? grp : 0][r] = w;
+  }
+  l = wave_reduce_sum(l);
   __syncthreads();
+  const int d = (tid & 127) * 4;
+  f32x4v s = {0.f, 0.f, 0.f, 0.f};
+  const float* src = tmp_acc + first_part * MLA_R + d;
+  constexpr int STEP = BY_HEAD ? 1 : 4;
+#pragma unroll 8
+  for (int r = BY_HEAD ? 0 : grp; r < parts; r += STEP) {
+    const f32x4v v =
+        *reinterpret_cast<const f32x4v*>(src + (size_t)r * H * MLA_R);
+    const float w = wt[BY_HEAD ? grp : 0][r];
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
-    const int h = hb * MLA_HBLOCK + nt * 16 + l15;
-    if (h >= H) continue;
-    if (PARTITIONED) {
-      const int p = blockIdx.z;
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int r0 = wid * (R / 4) + mt * 16 + l4 * 4;
-        float* dst = tmp_acc + (((size_t)seq * H + h) * gridDim.z + p) * R + r0;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) dst[rr] = acc_o[mt][nt][rr];
-      }
-      if (wid == 0 && l4 == 0) {
-        float* ml = tmp_ml + (((size_t)seq * H + h) * gridDim.z + blockIdx.z) * 2;
-        ml[0] = m_s[nt * 16 + l15];
-        ml[1] = l_s[nt * 16 + l15];
-      }
-    } else {
-      const float inv = 1.f / l_s[nt * 16 + l15];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int r0 = wid * (R / 4) + mt * 16 + l4 * 4;
-        uint16_t vals[4];
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr)
-          vals[rr] = f32_to_bf16_bits(acc_o[mt][nt][rr] * inv);
-        *reinterpret_cast<uint2*>(out + ((size_t)seq * H + h) * R + r0) =
-            *reinterpret_cast<const uint2*>(vals);
-      }
-    }
+    for (int i = 0; i < 4; ++i) s[i] = fmaf(v[i], w, s[i]);
   }
+  if (!BY_HEAD) {
+    sums[grp][tid & 127] = s;
+    __syncthreads();
+    if (grp > 0) return;
+    s = sums[0][tid] + sums[1][tid] + sums[2][tid] + sums[3][tid];
+  }
+  if (!on) return;
+  const float inv = 1.f / l;
+  uint2 v;
+  v.x = pack_bf16(s[0] * inv, s[1] * inv);
+  v.y = pack_bf16(s[2] * inv, s[3] * inv);
+  *reinterpret_cast<uint2*>(out + ((size_t)seq * H + head) * MLA_R + d) = v;
+}
+
+// Runs the tiles are dealt to; 0: every sequence has a workgroup of its own.
+// One workgroup a CU: its two tiles (144 KB) fill the LDS.
+extern "C" int mla_decode_runs(int B, int H, int max_domain) {
+  const int blocks = ceil_div(H, 64);
+  if (max_domain <= 256) return 0;
+  return MLA_MAX_RUNS / blocks > 1 ? MLA_MAX_RUNS / blocks : 1;
 }
 
 extern "C" void launch_mla_paged_attention_decode(
     void* out, const void* q_latent, const void* q_pe, const void* cache,
     const int* block_tables, const int* seq_lens, int B, int H, int R, int DR,
-    int BS, int max_blocks, float scale, int num_parts, int part_tokens,
-    float* tmp_acc, float* tmp_ml, const int* topk_indices, int max_topk,
-    bool kv_fp8, float c_scale, hipStream_t stream, bool* launched) {
+    int BS, int max_blocks, float scale, int runs, float* tmp_acc,
+    float* tmp_ml, const int* topk_indices, int max_topk, bool kv_fp8,
+    float c_scale, hipStream_t stream, bool* launched) {
   *launched = false;
-  if (R != 512 || DR != 64) return;  // DeepSeek V2/V3/R1/K2 geometry
-  const int head_blocks = (H + MLA_HBLOCK - 1) / MLA_HBLOCK;
+  if (R != MLA_R || DR != MLA_DR) return;  // DeepSeek V2/V3/R1/K2 geometry
+  if (BS != 16 && BS != 32 && BS != 64) return;
+  const int shift = __builtin_ctz(BS);
+  const int waves = H > 32 ? 8 : 4;
+  dim3 grid(runs > 0 ? runs : B, ceil_div(H, waves * 8), 1);
 
-#define MLA_LAUNCH3(BSZ, SP, FP8)                                             \
-  if (num_parts <= 1) {                                                       \
-    dim3 grid(head_blocks, B, 1);                                             \
-    mla_decode_kernel<512, 64, BSZ, false, SP, FP8>                           \
-        <<<grid, MLA_THREADS, 0, stream>>>(                                   \
-        (uint16_t*)out, nullptr, nullptr, (const uint16_t*)q_latent,          \
-        (const uint16_t*)q_pe, cache, block_tables,                           \
-        seq_lens, max_blocks, H, scale, 0, topk_indices, max_topk, c_scale);  \
-  } else {                                                                    \
-    dim3 grid(head_blocks, B, num_parts);                                     \
-    mla_decode_kernel<512, 64, BSZ, true, SP, FP8>                            \
-        <<<grid, MLA_THREADS, 0, stream>>>(                                   \
-        nullptr, tmp_acc, tmp_ml, (const uint16_t*)q_latent,                  \
-        (const uint16_t*)q_pe, cache, block_tables,                           \
-        seq_lens, max_blocks, H, scale, part_tokens, topk_indices, max_topk,  \
-        c_scale);                                                             \
-  }                                                                           \
-  *launched = true;
+#define MLA_LAUNCH(WV, FP8, SP)                                               \
+  mla_decode_kernel<WV, FP8, SP><<<grid, WV * 64, 0, stream>>>(               \
+      (uint16_t*)out, tmp_acc, tmp_ml, (const uint16_t*)q_latent,             \
+      (const uint16_t*)q_pe, cache, block_tables, seq_lens, topk_indices,     \
+      max_topk, B, max_blocks, H, shift, scale, c_scale);
+#define MLA_LAUNCH2(FP8, SP)                 \
+  if (waves == 8) { MLA_LAUNCH(8, FP8, SP) } \
+  else { MLA_LAUNCH(4, FP8, SP) }
+#define MLA_REDUCE(SP, BY_HEAD, GRID)                                         \
+  mla_reduce_kernel<SP, BY_HEAD><<<dim3(GRID, B, 1), 512, 0, stream>>>(       \
+      (uint16_t*)out, tmp_acc, tmp_ml, seq_lens, topk_indices, max_topk, B, H, \
+      runs);
+#define MLA_LAUNCH3(SP)                                       \
+  if (kv_fp8) { MLA_LAUNCH2(true, SP) }                       \
+  else { MLA_LAUNCH2(false, SP) }                             \
+  if (runs > 0 && runs >= 16 * B) { MLA_REDUCE(SP, false, H) } \
+  else if (runs > 0) { MLA_REDUCE(SP, true, ceil_div(H, 4)) }
 
-#define MLA_LAUNCH2(BSZ, SP)                                                  \
-  if (kv_fp8) { MLA_LAUNCH3(BSZ, SP, true) }                                  \
-  else { MLA_LAUNCH3(BSZ, SP, false) }
-
-#define MLA_LAUNCH(BSZ)                                                       \
-  if (topk_indices != nullptr) { MLA_LAUNCH2(BSZ, true) }                     \
-  else { MLA_LAUNCH2(BSZ, false) }
-
-  if (BS == 32) { MLA_LAUNCH(32) }
-  else if (BS == 16) { MLA_LAUNCH(16) }
-  else if (BS == 64) { MLA_LAUNCH(64) }
+  if (topk_indices != nullptr) { MLA_LAUNCH3(true) }
+  else { MLA_LAUNCH3(false) }
 #undef MLA_LAUNCH
 #undef MLA_LAUNCH2
 #undef MLA_LAUNCH3
+#undef MLA_REDUCE
+  *launched = true;
 }

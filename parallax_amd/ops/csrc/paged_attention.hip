@@ -368,9 +368,6 @@ extern "C" void launch_paged_attention_reduce(
   else if (D == 64)
     paged_attention_reduce_kernel<64><<<rgrid, 64, 0, stream>>>(
         (uint16_t*)out, tmp_acc, tmp_ml, num_parts, sinks, Hq);
-  else if (D == 512)  // MLA latent dim
-    paged_attention_reduce_kernel<512><<<rgrid, 64, 0, stream>>>(
-        (uint16_t*)out, tmp_acc, tmp_ml, num_parts, sinks, Hq);
 }
 
 extern "C" void launch_paged_attention_decode(

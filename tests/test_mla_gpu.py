@@ -108,3 +108,53 @@ def test_mla_decode_fp8_cache():
     torch.testing.assert_close(out8.float(), out16.float(), atol=0.12, rtol=0.12)
     # and the fp8 store actually quantized (bytes differ from bf16 view)
     assert cache8.dtype == torch.float8_e4m3fn
+
+
+@pytest.mark.parametrize("H,BS,ctxs,fp8", [
+    (16, 16, [1, 31, 33, 700], False),     # runs that cross sequences
+    (40, 32, [5000, 64, 3], False),        # one sequence over many runs
+    (128, 64, [600, 90, 1500], False),
+    (200, 32, [300, 257], False),          # more heads than a workgroup takes
+    (24, 32, [250] * 3, False),            # a workgroup a sequence
+    (64, 16, [47, 900], True),
+    (128, 32, [333, 70], True),
+])
+def test_mla_decode_runs(H, BS, ctxs, fp8):
+    """Tiles dealt over sequences, every page size and head count per wave,
+    cache slots behind a sequence's end holding NaN. Weights and results are
+    rounded to bf16 once each: at most 2 * 2^-9 * max |cache| (5.5)."""
+    ql, qp, cache, bt, sl = _setup(len(ctxs), H, ctxs, BS=BS, seed=H)
+    ql, qp = ql * 10, qp * 10
+    if fp8:
+        cache = cache.to(torch.float8_e4m3fn)
+    plain = cache.float()
+    for i, n in enumerate(ctxs):
+        if n % BS and not fp8:
+            cache[int(bt[i, n // BS]), n % BS:] = float("nan")
+    scale = 192 ** -0.5
+    out = ops.mla_paged_attention_decode(ql, qp, cache, bt, sl, scale)
+    want = ref.mla_paged_attention_decode(
+        ql.float().cpu(), qp.float().cpu(), plain.cpu(), bt.cpu(), sl.cpu(), scale)
+    torch.testing.assert_close(out.float().cpu(), want, atol=2.2e-2, rtol=0)
+
+
+@pytest.mark.parametrize("H,topk", [(16, 40), (128, 512)])
+def test_mla_decode_listed_tokens(H, topk):
+    """Rows restricted to listed positions (some entries stand for none), beside
+    a row without a list."""
+    ctxs = [700, 90, 1300]
+    ql, qp, cache, bt, sl = _setup(3, H, ctxs, seed=topk)
+    ql = ql * 10
+    idx = torch.full((3, topk), -1, dtype=torch.int32)
+    g = torch.Generator().manual_seed(1)
+    for i, n in enumerate(ctxs):
+        k = min(topk, n) - 7
+        idx[i, :k] = torch.randperm(n, generator=g)[:k].int()
+    idx[0, 11] = -1
+    idx[1, 0] = -1                          # attends to everything
+    scale = 192 ** -0.5
+    out = ops.dsa_paged_attention_decode(ql, qp, cache, bt, sl, idx.cuda(), scale)
+    want = ref.dsa_paged_attention_decode(
+        ql.float().cpu(), qp.float().cpu(), cache.float().cpu(), bt.cpu(),
+        sl.cpu(), idx, scale)
+    torch.testing.assert_close(out.float().cpu(), want, atol=2.2e-2, rtol=0)
