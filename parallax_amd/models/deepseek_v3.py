@@ -125,11 +125,12 @@ class MLAAttention(nn.Module):
         return None
 
     def _prefill_attention(self, q_nope, q_pe, meta: ForwardMeta, cache):
-        """Absorbed, L-chunked online-softmax prefill over the COMPRESSED
-        cache: q_nope folds through w_uk so QK^T and PV both contract against
-        the latent directly (same math as the absorbed decode kernel) —
-        no [L, H, dn+dv] expansion and no [QL, L] full-logits buffer, which
-        is what makes 256k-context prefill (BASELINE Kimi-K2 config) fit.
+        """Prefill over the COMPRESSED cache, a request at a time: the flash
+        kernel (keys and values expanded a run of rows at a time) where there
+        is one. Elsewhere absorbed, L-chunked online softmax: q_nope folds
+        through w_uk so QK^T and PV both contract against the latent directly
+        (same math as the absorbed decode kernel). Neither holds [QL, L]
+        logits, which is what makes 256k-context prefill fit.
         Sparse subclasses (DSA) still take the dense masked path below."""
         H, dn, dv, r = self.num_heads, self.dn, self.dv, self.r
         bs = cache.shape[1]
@@ -137,15 +138,20 @@ class MLAAttention(nn.Module):
             q_nope.shape[0], H, dv, dtype=q_nope.dtype, device=q_nope.device
         )
         t0 = 0
-        for i in range(meta.batch_size):
-            QL = int(meta.query_lens[i])
-            L = int(meta.seq_lens[i])
+        lens = zip(meta.query_lens.tolist(), meta.seq_lens.tolist())
+        for i, (QL, L) in enumerate(lens):
             nb = (L + bs - 1) // bs
             entries = cache[meta.block_tables[i, :nb].long()].reshape(nb * bs, -1)[:L]
+            extra = self._prefill_sparse_mask(i, t0, QL, L, meta)
+            if extra is None and ops.mla_prefill_attention(
+                out[t0 : t0 + QL], q_nope[t0 : t0 + QL], q_pe[t0 : t0 + QL],
+                entries, self.w_uk, self.w_uv, self.scale,
+            ):
+                t0 += QL
+                continue
             lat, kpe_ctx = entries[:, :r], entries[:, r:]        # [L, r], [L, dr]
             qi_n = q_nope[t0 : t0 + QL].float()                  # [QL, H, dn]
             qi_p = q_pe[t0 : t0 + QL].float()                    # [QL, H, dr]
-            extra = self._prefill_sparse_mask(i, t0, QL, L, meta)
             if extra is not None:  # DSA (deepseek_v32) top-k restriction
                 kv = torch.einsum("lr,hdr->lhd", lat.float(),
                                   torch.cat([self.w_uk, self.w_uv], dim=1).float())

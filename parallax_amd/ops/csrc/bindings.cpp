@@ -47,6 +47,10 @@ void launch_mla_paged_attention_decode(void*, const void*, const void*,
                                        int, float*, float*, const int*, int,
                                        bool, float, hipStream_t, bool*);
 int mla_decode_runs(int, int, int);
+void launch_mla_prefill_run(void*, float*, const void*, const void*, void*, void*,
+                            void*, void*, const void*, const void*, const void*,
+                            int, int, int, int, int, int, int64_t, int64_t, float,
+                            bool, bool, hipStream_t);
 void launch_msa_paged_attention_decode(void*, const void*, const void*,
                                        const void*, const int*, const int*,
                                        const int*, int, int, int, int, int,
@@ -423,6 +427,53 @@ void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,
   TORCH_CHECK(launched, "no MLA kernel for R=", R, " DR=", DR, " BS=", BS);
 }
 
+// One request's prompt portion [T, H] over its context rows [L, 512 + 64], the
+// portion's own rows last. Returns false where there is no kernel.
+bool mla_prefill_attention(torch::Tensor out, torch::Tensor q_nope,
+                           torch::Tensor q_pe, torch::Tensor rows,
+                           torch::Tensor w_uk, torch::Tensor w_uv, double scale) {
+  CHECK_GPU(q_nope);
+  const int64_t T = q_nope.size(0), H = q_nope.size(1), L = rows.size(0);
+  for (const auto& t : {out, q_nope, q_pe, rows, w_uk, w_uv}) {
+    if (t.scalar_type() != at::kBFloat16 || (uintptr_t)t.data_ptr() % 16)
+      return false;
+  }
+  if (q_nope.size(2) != 128 || q_pe.size(2) != 64 || w_uk.size(1) != 128 ||
+      w_uv.size(1) != 128 || w_uk.size(2) != 512 || rows.size(1) != 576)
+    return false;
+  if (q_nope.stride(2) != 1 || q_nope.stride(1) % 8 || q_nope.stride(0) % 8)
+    return false;
+  CHECK_CONTIG(out);
+  CHECK_CONTIG(q_pe);
+  CHECK_CONTIG(rows);
+  CHECK_CONTIG(w_uk);
+  CHECK_CONTIG(w_uv);
+  TORCH_CHECK(q_pe.size(0) == T && q_pe.size(1) == H && out.size(0) == T &&
+              out.size(1) == H && out.size(2) == 128 && w_uk.size(0) == H &&
+              w_uv.size(0) == H && w_uv.size(2) == 512 && L >= T);
+  if (T == 0 || H == 0) return true;
+  // 1 GB of expanded keys and values a run
+  const int64_t run = std::max<int64_t>(128, ((1 << 20) / H) & ~127);
+  const int64_t cap = (std::min(L, run) + 127) & ~127;
+  auto kv = torch::empty({4, H * cap * 128}, q_nope.options());
+  torch::Tensor state;
+  if (L > run)
+    state = torch::empty({T, H, 130}, q_nope.options().dtype(at::kFloat));
+  uint16_t* p = (uint16_t*)kv.data_ptr();
+  const size_t part = (size_t)H * cap * 128;
+  for (int64_t k0 = 0; k0 < L; k0 += run) {
+    const int64_t n = std::min(run, L - k0);
+    launch_mla_prefill_run(
+        out.data_ptr(), L > run ? state.data_ptr<float>() : nullptr,
+        q_nope.data_ptr(), q_pe.data_ptr(), p, p + part, p + 2 * part,
+        p + 3 * part, (const uint16_t*)rows.data_ptr() + k0 * 576,
+        w_uk.data_ptr(), w_uv.data_ptr(), T, H, n, cap, L - T, k0,
+        q_nope.stride(0), q_nope.stride(1), (float)scale, k0 == 0, k0 + n == L,
+        cur_stream());
+  }
+  return true;
+}
+
 // Routed experts of x [T, H]: bf16, or fp8 (W8A8) with w_gu_scale / w_down_scale
 // given. Returns fp32 [T, H].
 static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
@@ -701,6 +752,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("msa_block_scores", &msa_block_scores);
   m.def("msa_topk_tokens", &msa_topk_tokens);
   m.def("mla_paged_attention_decode", &mla_paged_attention_decode);
+  m.def("mla_prefill_attention", &mla_prefill_attention);
   m.def("prefill_attention", &prefill_attention);
   m.def("rmsnorm", &rmsnorm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);

@@ -1,0 +1,417 @@
+// MLA prefill for gfx950: a request's prompt portion against its context.
+//
+//   mla_expand   keys k = latent . W_uk[h]^T and values v = latent . W_uv[h]^T of
+//                a run of context rows, for every head, to bf16 pairs (below)
+//   mla_prefill  flash attention of the portion's rows over those keys and the
+//                rotated key parts, which are read from the context rows
+//
+// Everything between the bf16 inputs (queries, rotated parts, latents, weights)
+// and the bf16 result was computed in fp32 and stays that accurate: a value that
+// is not a bf16 number (k, v, the softmax weights p) enters the matrix
+// instructions as hi + lo, hi = bf16(x), lo = bf16(x - hi), 16 bits of mantissa
+// and more; q . k takes two products, p . v three (lo . lo is 2^-18 of it). The
+// sums are fp32. Measured against 64 bits (8 to 128 heads, 40 to 2,500 rows,
+// contexts to 9,000) the result is as far off as with fp32 products, 0.00165792
+// of it at 2,500 rows either way: the rounding of the result itself.
+//
+// Why keys are expanded: per pair of row and key a head then takes 320 + 384
+// multiply-adds (the parts counted); in latent space 1,088 + 1,024. The expanded
+// run is at most MLA_RUN context rows (1 GB at 128 heads); longer contexts go
+// run by run, the fp32 state of the rows in memory between.
+//
+// What bounds it: matrix cores, 44 instructions of 32x32x16 per wave and 32 keys
+// beside about 900 VALU cycles; two workgroups a CU overlap them. A prompt of
+// 2,500 rows at 128 heads: expansion 230 us, attention 500 us; the fp32 torch
+// operations in latent space that this replaced 25 ms. 512 rows on a context of
+// 40,000: 8.2 ms, before 71 ms.
+
+#include "common.h"
+
+#define MP_R 512    // latent rank
+#define MP_DR 64    // rotated part
+#define MP_DK 576   // values a context row
+#define MP_D 128    // key and value width a head
+#define MP_ROWS 128 // query rows a workgroup
+#define MP_KT 32    // keys a tile
+
+typedef float f32x16v __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2n __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
+
+namespace {
+
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kHidden = -1e30f;
+
+DEVINL uint32_t pack_bf16(float a, float b) {
+  bf16x2n p;
+  p[0] = (__bf16)a;
+  p[1] = (__bf16)b;
+  return __builtin_bit_cast(uint32_t, p);
+}
+
+// two fp32 values to their hi and lo parts
+DEVINL void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  hi = pack_bf16(a, b);
+  lo = pack_bf16(a - __uint_as_float(hi << 16),
+                 b - __uint_as_float(hi & 0xffff0000u));
+}
+
+DEVINL void copy16_to_lds(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)src,
+      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+DEVINL float max_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+DEVINL float sum_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+}  // namespace
+
+// ---- keys and values of a run ------------------------------------------------------
+// 128 context rows x 128 features a workgroup, 4 waves of 64 x 64, both operands
+// global -> LDS directly, 128 bytes of every row a stage. Keys come out as
+// [head, row, feature] and values as [head, feature, row]: the operand order is
+// swapped between the two, so that a lane's four neighbouring registers are
+// neighbours in memory either way. Rows past the run are written as zeros.
+
+__global__ __launch_bounds__(256, 2) void mla_expand_kernel(
+    uint16_t* __restrict__ k_hi, uint16_t* __restrict__ k_lo,  // [H, cap, 128]
+    uint16_t* __restrict__ v_hi, uint16_t* __restrict__ v_lo,  // [H, 128, cap]
+    const uint16_t* __restrict__ rows,  // [n, 576]
+    const uint16_t* __restrict__ w_uk,  // [H, 128, 512]
+    const uint16_t* __restrict__ w_uv, const int n, const int cap) {
+  constexpr int BKB = 128;
+  __shared__ __attribute__((aligned(16))) uint8_t S0[256 * BKB];
+  __shared__ __attribute__((aligned(16))) uint8_t S1[256 * BKB];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, l31 = lane & 31;
+  const int r0 = blockIdx.y * 128;
+  const int h = blockIdx.x >> 1;
+  const bool val = blockIdx.x & 1;
+  const uint8_t* w =
+      (const uint8_t*)((val ? w_uv : w_uk) + (size_t)h * MP_D * MP_R);
+
+  // a thread's chunk of rows tid / 8 + 32 i: weights are LDS rows 0..127
+  const int src = ((tid & 7) ^ ((tid >> 4) & 7)) * 16;
+  const uint8_t *wp[4], *rp[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 32 + (tid >> 3);
+    wp[i] = w + (size_t)r * (MP_R * 2) + src;
+    rp[i] = (const uint8_t*)(rows + (size_t)min(r0 + r, n - 1) * MP_DK) + src;
+  }
+  auto issue = [&](int kt, uint8_t* S) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      copy16_to_lds(wp[i] + kt * BKB, S + (i * 32 + wid * 8) * BKB);
+      copy16_to_lds(rp[i] + kt * BKB, S + (128 + i * 32 + wid * 8) * BKB);
+    }
+  };
+  // registers run over the features of a key, over the rows of a value
+  const int ra = (val ? 128 : 0) + (wid & 1) * 64;
+  const int rb = (val ? 0 : 128) + (wid >> 1) * 64;
+  const int swz_l = (l31 >> 1) & 7;
+  f32x16v acc[2][2] = {};
+  auto stage = [&](const uint8_t* S) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int c = ((2 * ks + half) ^ swz_l) * 16;
+      bf16x8v a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[i] = *(const bf16x8v*)(S + (ra + i * 32 + l31) * BKB + c);
+        b[i] = *(const bf16x8v*)(S + (rb + i * 32 + l31) * BKB + c);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j],
+                                                              acc[i][j], 0, 0, 0);
+    }
+  };
+  constexpr int NK = MP_R * 2 / BKB;
+  issue(0, S0);
+#pragma unroll
+  for (int kt = 0; kt < NK; kt += 2) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    __syncthreads();
+    issue(kt + 1, S1);
+    stage(S0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    __syncthreads();
+    if (kt + 2 < NK) issue(kt + 2, S0);
+    stage(S1);
+  }
+
+  uint16_t* hi = (val ? v_hi : k_hi) + (size_t)h * cap * MP_D;
+  uint16_t* lo = (val ? v_lo : k_lo) + (size_t)h * cap * MP_D;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int col = (rb & 127) + j * 32 + l31;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = (ra & 127) + i * 32 + 8 * q + 4 * half;
+        uint2 a, b;
+        float x[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int tok = r0 + (val ? row + s : col);
+          x[s] = tok < n ? acc[i][j][4 * q + s] : 0.f;
+        }
+        split2(x[0], x[1], a.x, b.x);
+        split2(x[2], x[3], a.y, b.y);
+        const size_t at = val ? (size_t)col * cap + r0 + row
+                              : (size_t)(r0 + col) * MP_D + row;
+        *reinterpret_cast<uint2*>(hi + at) = a;
+        *reinterpret_cast<uint2*>(lo + at) = b;
+      }
+  }
+}
+
+// ---- attention ------------------------------------------------------------------------
+// 128 query rows of one head a workgroup, 32 a wave; see prefill_attention for
+// the operand orders (S^T = K Q^T, O^T = V^T P, P from the accumulators).
+
+__global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
+    uint16_t* __restrict__ out,           // [T, H, 128]
+    float* __restrict__ state,            // [T, H, 130] or null
+    const uint16_t* __restrict__ q_nope,  // [T, H, 128] by strides
+    const uint16_t* __restrict__ q_pe,    // [T, H, 64]
+    const uint16_t* __restrict__ k_hi, const uint16_t* __restrict__ k_lo,
+    const uint16_t* __restrict__ v_hi, const uint16_t* __restrict__ v_lo,
+    const uint16_t* __restrict__ rows,    // [n, 576]
+    const int T, const int H, const int n, const int cap, const int prefix,
+    const int first_key, const int64_t q_row, const int64_t q_head,
+    const float scale, const int first, const int last) {
+  __shared__ __attribute__((aligned(16))) uint16_t Kh0[MP_KT * 128], Kl0[MP_KT * 128];
+  __shared__ __attribute__((aligned(16))) uint16_t Kh1[MP_KT * 128], Kl1[MP_KT * 128];
+  __shared__ __attribute__((aligned(16))) uint16_t R0[MP_KT * 64], R1[MP_KT * 64];
+  __shared__ __attribute__((aligned(16))) uint16_t Vh0[MP_KT * 128], Vl0[MP_KT * 128];
+  __shared__ __attribute__((aligned(16))) uint16_t Vh1[MP_KT * 128], Vl1[MP_KT * 128];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, l31 = lane & 31;
+  // heads fastest: with 8 | H a head's blocks share an XCD's L2; the last rows
+  // see the most keys and come first
+  const int h = blockIdx.x % H;
+  const int tile = gridDim.x / H - 1 - blockIdx.x / H;
+  const int w0 = tile * MP_ROWS + wid * 32;
+  const int row = w0 + l31;
+  const bool row_ok = row < T;
+  const int row_c = min(row, T - 1);
+  // positions within this run of keys
+  const int qpos = prefix + row - first_key;
+  const int wpos_lo = prefix + w0 - first_key;
+  const bool wave_on = w0 < T;
+  const int wpos_hi = prefix + min(w0 + 31, T - 1) - first_key;
+  const int pos_hi =
+      prefix + min(tile * MP_ROWS + MP_ROWS - 1, T - 1) - first_key;
+  const int kt_end = max(0, (min(n, pos_hi + 1) + MP_KT - 1) / MP_KT);
+
+  bf16x8v qf[12];
+  {
+    const uint16_t* a =
+        q_nope + (size_t)row_c * q_row + (size_t)h * q_head + half * 8;
+    const uint16_t* b = q_pe + ((size_t)row_c * H + h) * MP_DR + half * 8;
+#pragma unroll
+    for (int s = 0; s < 12; ++s)
+      qf[s] = s < 8 ? *(const bf16x8v*)(a + s * 16)
+                    : *(const bf16x8v*)(b + (s - 8) * 16);
+  }
+  f32x16v o[4] = {};
+  float m = kHidden, l = 0.f;  // l: this half's keys only
+  float* st = state + ((size_t)row_c * H + h) * 130;
+  if (!first) {
+    m = st[128];
+    l = half == 0 ? st[129] : 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          o[t][4 * i + r] = st[t * 32 + 8 * i + 4 * half + r];
+  }
+  const float c = scale * kLog2e;
+
+  // ---- copies: chunk numbers within a tile, LDS places XOR-swizzled by row ---------
+  const uint16_t* kh = k_hi + (size_t)h * cap * MP_D;
+  const uint16_t* kl = k_lo + (size_t)h * cap * MP_D;
+  const uint16_t* vh = v_hi + (size_t)h * cap * MP_D;
+  const uint16_t* vl = v_lo + (size_t)h * cap * MP_D;
+  int k_at[2], v_at[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int ch = (wid * 2 + i) * 64 + lane;
+    const int kr = ch >> 4, vr = ch >> 2;
+    k_at[i] = kr * MP_D + ((ch & 15) ^ (kr & 15)) * 8;
+    v_at[i] = vr * cap + ((ch & 3) ^ ((vr >> 2) & 3)) * 8;
+  }
+  const int pe_row = tid >> 3;
+  const int pe_at = MP_R + ((tid & 7) ^ ((pe_row >> 1) & 7)) * 8;
+  auto issue = [&](int kt, uint16_t* Kh, uint16_t* Kl, uint16_t* R,
+                   uint16_t* Vh, uint16_t* Vl) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int dst = (wid * 2 + i) * 512;
+      copy16_to_lds(kh + (size_t)kt * (MP_KT * MP_D) + k_at[i], Kh + dst);
+      copy16_to_lds(kl + (size_t)kt * (MP_KT * MP_D) + k_at[i], Kl + dst);
+      copy16_to_lds(vh + (size_t)kt * MP_KT + v_at[i], Vh + dst);
+      copy16_to_lds(vl + (size_t)kt * MP_KT + v_at[i], Vl + dst);
+    }
+    copy16_to_lds(
+        rows + (size_t)min(kt * MP_KT + pe_row, n - 1) * MP_DK + pe_at,
+        R + wid * 512);
+  };
+
+  // K row with bits 2 and 3 swapped: a lane half's weights are 8 neighbouring keys
+  const int krow = (l31 & 0x13) | ((l31 & 4) << 1) | ((l31 & 8) >> 1);
+  auto compute = [&](int kt, const uint16_t* Kh, const uint16_t* Kl,
+                     const uint16_t* R, const uint16_t* Vh, const uint16_t* Vl)
+      __attribute__((always_inline)) {
+    const int kbase = kt * MP_KT;
+    if (!wave_on || kbase > wpos_hi) return;
+    f32x16v s = {}, s2 = {};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      const int at = krow * 128 + ((2 * ks + half) ^ (krow & 15)) * 8;
+      const bf16x8v a = *(const bf16x8v*)(Kh + at);
+      const bf16x8v b = *(const bf16x8v*)(Kl + at);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], s, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, qf[ks], s2, 0, 0, 0);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const bf16x8v a = *(const bf16x8v*)(
+          R + krow * 64 + ((2 * ks + half) ^ ((krow >> 1) & 7)) * 8);
+      f32x16v& d = ks & 1 ? s2 : s;
+      d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[8 + ks], d, 0, 0, 0);
+    }
+    s += s2;
+
+    if (kbase + MP_KT - 1 > wpos_lo || kbase + MP_KT > n) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = kbase + 16 * (r >> 3) + 8 * half + (r & 7);
+        s[r] = key <= qpos && key < n ? s[r] : kHidden;
+      }
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = max_halves(mx) * c;
+    // rescaled only when a maximum moved by more than 2^8
+    if (__any(mx > m + 8.f)) {
+      const float m2 = fmaxf(m, mx);
+      const float f = __builtin_amdgcn_exp2f(m - m2);
+      m = m2;
+      l *= f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) o[t] *= f;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      float p[8];
+      u32x4v ph, pl;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        p[j] = __builtin_amdgcn_exp2f(fmaf(s[ks * 8 + j], c, -m));
+        l += p[j];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t hi, lo;
+        split2(p[2 * j], p[2 * j + 1], hi, lo);
+        ph[j] = hi;
+        pl[j] = lo;
+      }
+      const bf16x8v bh = __builtin_bit_cast(bf16x8v, ph);
+      const bf16x8v bl = __builtin_bit_cast(bf16x8v, pl);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int d = t * 32 + l31;
+        const int at = d * MP_KT + ((2 * ks + half) ^ ((d >> 2) & 3)) * 8;
+        const bf16x8v ah = *(const bf16x8v*)(Vh + at);
+        const bf16x8v al = *(const bf16x8v*)(Vl + at);
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, o[t], 0, 0, 0);
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, o[t], 0, 0, 0);
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, o[t], 0, 0, 0);
+      }
+    }
+  };
+
+  if (kt_end > 0) issue(0, Kh0, Kl0, R0, Vh0, Vl0);
+  for (int kt = 0; kt < kt_end; kt += 2) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    __syncthreads();
+    if (kt + 1 < kt_end) issue(kt + 1, Kh1, Kl1, R1, Vh1, Vl1);
+    compute(kt, Kh0, Kl0, R0, Vh0, Vl0);
+    if (kt + 1 >= kt_end) break;
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    __syncthreads();
+    if (kt + 2 < kt_end) issue(kt + 2, Kh0, Kl0, R0, Vh0, Vl0);
+    compute(kt + 1, Kh1, Kl1, R1, Vh1, Vl1);
+  }
+
+  if (!row_ok) return;
+  l = sum_halves(l);
+  if (!last) {
+    if (half == 0) {
+      st[128] = m;
+      st[129] = l;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          st[t * 32 + 8 * i + 4 * half + r] = o[t][4 * i + r];
+    return;
+  }
+  const float inv = 1.f / l;
+  uint16_t* dst = out + ((size_t)row * H + h) * MP_D + 4 * half;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint2 v;
+      v.x = pack_bf16(o[t][4 * i] * inv, o[t][4 * i + 1] * inv);
+      v.y = pack_bf16(o[t][4 * i + 2] * inv, o[t][4 * i + 3] * inv);
+      *reinterpret_cast<uint2*>(dst + t * 32 + 8 * i) = v;
+    }
+}
+
+extern "C" void launch_mla_prefill_run(
+    void* out, float* state, const void* q_nope, const void* q_pe, void* k_hi,
+    void* k_lo, void* v_hi, void* v_lo, const void* rows, const void* w_uk,
+    const void* w_uv, int T, int H, int n, int cap, int prefix, int first_key,
+    int64_t q_row, int64_t q_head, float scale, bool first, bool last,
+    hipStream_t stream) {
+  mla_expand_kernel<<<dim3(2 * H, ceil_div(n, 128), 1), 256, 0, stream>>>(
+      (uint16_t*)k_hi, (uint16_t*)k_lo, (uint16_t*)v_hi, (uint16_t*)v_lo,
+      (const uint16_t*)rows, (const uint16_t*)w_uk, (const uint16_t*)w_uv, n,
+      cap);
+  mla_prefill_kernel<<<ceil_div(T, MP_ROWS) * H, 256, 0, stream>>>(
+      (uint16_t*)out, state, (const uint16_t*)q_nope, (const uint16_t*)q_pe,
+      (const uint16_t*)k_hi, (const uint16_t*)k_lo, (const uint16_t*)v_hi,
+      (const uint16_t*)v_lo, (const uint16_t*)rows, T, H, n, cap, prefix,
+      first_key, q_row, q_head, scale, first, last);
+}

@@ -158,3 +158,50 @@ def test_mla_decode_listed_tokens(H, topk):
         ql.float().cpu(), qp.float().cpu(), cache.float().cpu(), bt.cpu(),
         sl.cpu(), idx, scale)
     torch.testing.assert_close(out.float().cpu(), want, atol=2.2e-2, rtol=0)
+
+
+@pytest.mark.parametrize("H,T,L,fp8", [
+    (128, 1, 1, False),
+    (8, 33, 33, False),           # past a wave's 32 rows and a tile's 32 keys
+    (16, 127, 160, True),
+    (16, 129, 1000, False),       # past a workgroup's 128 rows
+    (128, 130, 8192 + 40, False), # a second run of expanded rows, the
+                                  # portion's first rows before it
+])
+def test_mla_prefill(H, T, L, fp8):
+    """Against fp32 products. The result's rounding is 2^-9 of it; a logit is
+    off by at most the lo parts' rounding, sum |q k| * scale * 2^-17 < 2e-4,
+    a result by twice that of max |v| < 6."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    q = r(T, H, 192).bfloat16()
+    q_nope, q_pe = q[..., :128], q[..., 128:].contiguous()
+    rows = r(L, 576).to(torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    uk, uv = ((r(H, 128, 512) * 512 ** -0.5).bfloat16() for _ in range(2))
+    out = torch.empty(T, H, 128, dtype=torch.bfloat16, device="cuda")
+    scale = 192 ** -0.5
+    assert ops.mla_prefill_attention(out, q_nope, q_pe, rows, uk, uv, scale)
+    e = rows.float()
+    hidden = torch.arange(L, device="cuda")[None] > torch.arange(
+        L - T, L, device="cuda")[:, None]
+    for h in {0, H // 2, H - 1}:
+        k, v = e[:, :512] @ uk[h].float().t(), e[:, :512] @ uv[h].float().t()
+        s = q_nope[:, h].float() @ k.t() + q_pe[:, h].float() @ e[:, 512:].t()
+        p = (s * scale).masked_fill(hidden, float("-inf")).softmax(-1)
+        torch.testing.assert_close(
+            out[:, h].float(), p @ v, atol=2.4e-3, rtol=2 ** -8)
+
+
+def test_mla_prefill_left_to_the_caller():
+    """Types, widths and few rows on a long context have no kernel."""
+    def call(T, L, H=16, dtype=torch.bfloat16, dn=128, dr=64, dev="cuda"):
+        z = lambda *s: torch.zeros(*s, dtype=dtype, device=dev)
+        return ops.mla_prefill_attention(
+            z(T, H, 128), z(T, H, dn), z(T, H, dr), z(L, 512 + dr),
+            z(H, dn, 512), z(H, 128, 512), 1.0)
+    assert call(40, 40)
+    assert not call(4, 30000)
+    assert not call(40, 40, dtype=torch.float32)
+    assert not call(40, 40, dn=64)
+    assert not call(40, 40, dr=32)
+    assert not call(40, 40, dev="cpu")
