@@ -74,6 +74,14 @@ struct Descs {
   }
 };
 
+// per-tensor scales on the device (A = w, B = x in our TN formulation)
+void set_scales(Descs& d, const void* w_scale, const void* x_scale) {
+  LT_CHECK(hipblasLtMatmulDescSetAttribute(
+      d.op, HIPBLASLT_MATMUL_DESC_A_SCALE_POINTER, &w_scale, sizeof(w_scale)));
+  LT_CHECK(hipblasLtMatmulDescSetAttribute(
+      d.op, HIPBLASLT_MATMUL_DESC_B_SCALE_POINTER, &x_scale, sizeof(x_scale)));
+}
+
 void make_descs(Descs& d, int64_t M, int64_t N, int64_t K,
                 hipDataType in_type = HIP_R_16BF) {
   LT_CHECK(hipblasLtMatmulDescCreate(&d.op, HIPBLAS_COMPUTE_32F, HIP_R_32F));
@@ -98,10 +106,15 @@ struct CachedShape {
 hipblasLtMatmulAlgo_t tune_shape(int64_t M, int64_t N, int64_t K,
                                  const void* wp, const void* xp, void* yp,
                                  hipStream_t stream,
-                                 hipDataType in_type = HIP_R_16BF) {
+                                 hipDataType in_type = HIP_R_16BF,
+                                 const void* w_scale = nullptr,
+                                 const void* x_scale = nullptr) {
   LtState& s = state();
   Descs d;
   make_descs(d, M, N, K, in_type);
+  // before any candidate is asked for: one picked without the scales may have
+  // no code for them and returns unscaled sums
+  if (w_scale) set_scales(d, w_scale, x_scale);
 
   hipblasLtMatmulPreference_t pref;
   LT_CHECK(hipblasLtMatmulPreferenceCreate(&pref));
@@ -305,18 +318,13 @@ torch::Tensor lt_linear_fp8(torch::Tensor x_q, torch::Tensor w_q,
       auto entry = std::make_unique<CachedShape>();
       make_descs(entry->descs, M, N, K, HIP_R_8F_E4M3);
       entry->algo = tune_shape(M, N, K, w_q.data_ptr(), x_q.data_ptr(),
-                               y.data_ptr(), stream, HIP_R_8F_E4M3);
+                               y.data_ptr(), stream, HIP_R_8F_E4M3,
+                               w_scale.data_ptr(), x_scale.data_ptr());
       it = s.shapes.emplace(key, std::move(entry)).first;
     }
     cs = it->second.get();
   }
-  // per-call device scale pointers (A = w, B = x in our TN formulation)
-  const void* sa = w_scale.data_ptr();
-  const void* sb = x_scale.data_ptr();
-  LT_CHECK(hipblasLtMatmulDescSetAttribute(
-      cs->descs.op, HIPBLASLT_MATMUL_DESC_A_SCALE_POINTER, &sa, sizeof(sa)));
-  LT_CHECK(hipblasLtMatmulDescSetAttribute(
-      cs->descs.op, HIPBLASLT_MATMUL_DESC_B_SCALE_POINTER, &sb, sizeof(sb)));
+  set_scales(cs->descs, w_scale.data_ptr(), x_scale.data_ptr());
   const float alpha = 1.f, beta = 0.f;
   LT_CHECK(hipblasLtMatmul(s.handle, cs->descs.op, &alpha, w_q.data_ptr(),
                            cs->descs.a, x_q.data_ptr(), cs->descs.b, &beta,
