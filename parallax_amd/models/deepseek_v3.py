@@ -106,17 +106,13 @@ class MLAAttention(nn.Module):
             attn = self._prefill_attention(q_nope, q_pe, meta, cache)
         else:
             # absorbed: q_latent[b,h] = q_nope[b,h] @ W_UK[h]^T... (dn x r)
-            q_latent = torch.einsum(
-                "bhd,hdr->bhr", q_nope.float(), self.w_uk.float()
-            ).to(q_nope.dtype)
+            q_latent = ops.mla_absorb(q_nope, self.w_uk)
             out_latent = ops.mla_paged_attention_decode(
                 q_latent.contiguous(), q_pe.contiguous(), cache,
                 meta.block_tables, meta.seq_lens, self.scale,
                 max_seq_len=meta.max_seq_len or None,
             )
-            attn = torch.einsum(
-                "bhr,hvr->bhv", out_latent.float(), self.w_uv.float()
-            ).to(x.dtype)
+            attn = ops.mla_project_out(out_latent, self.w_uv)
         return self.o_proj(attn.reshape(T, H * self.dv))
 
     def _prefill_sparse_mask(self, i, t0, QL, L, meta):

@@ -118,17 +118,13 @@ class DSAMLAAttention(MLAAttention):
         else:
             scores = self._decode_scores(q_idx, w_idx, idx_cache, meta)
             topk_indices = self._decode_topk(scores, meta.seq_lens)
-            q_latent = torch.einsum(
-                "bhd,hdr->bhr", q_nope.float(), self.w_uk.float()
-            ).to(q_nope.dtype)
+            q_latent = ops.mla_absorb(q_nope, self.w_uk)
             out_latent = ops.dsa_paged_attention_decode(
                 q_latent.contiguous(), q_pe.contiguous(), cache,
                 meta.block_tables, meta.seq_lens, topk_indices, self.scale,
                 max_seq_len=meta.max_seq_len or None,
             )
-            attn = torch.einsum(
-                "bhr,hvr->bhv", out_latent.float(), self.w_uv.float()
-            ).to(x.dtype)
+            attn = ops.mla_project_out(out_latent, self.w_uv)
         return self.o_proj(attn.reshape(T, H * self.dv))
 
     def _decode_scores(self, q_idx, w_idx, idx_cache, meta) -> torch.Tensor:

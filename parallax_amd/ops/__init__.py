@@ -455,10 +455,9 @@ def gelu_and_mul(x: torch.Tensor) -> torch.Tensor:
 
 # -- dense linear (skinny-M fast path) ------------------------------------------
 
-# Disabled by default: hipBLASLt reaches 3.4-5.8 TB/s of weight streaming at
-# decode shapes when measured in isolation (scripts/bench_gemm.py) and beats
-# this kernel's simple 2-barrier structure; opt in for experiments.
-SKINNY_GEMM_MAX_M = int(os.environ.get("PARALLAX_SKINNY_GEMM_MAX_M", "0"))
+# Rows of x up to which linear() and linear_fp8() try the weight-streaming kernel
+# (it has none above 32); 0 leaves every product to the library.
+SKINNY_GEMM_MAX_M = int(os.environ.get("PARALLAX_SKINNY_GEMM_MAX_M", "32"))
 LT_GEMM = os.environ.get("PARALLAX_LT_GEMM", "1") != "0"
 _LT_REFUSED = set()  # (N, K) shapes hipBLASLt had no algorithm for
 
@@ -466,23 +465,25 @@ _LT_REFUSED = set()  # (N, K) shapes hipBLASLt had no algorithm for
 def linear(
     x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None
 ) -> torch.Tensor:
-    """F.linear with a custom streaming kernel for decode-sized M (hipBLASLt
-    tile picks are 2-5x off the weight-streaming roofline at M <= 256)."""
+    """F.linear: a weight-streaming kernel for few rows (skinny_gemm.hip has the
+    sizes, with both sides measured), tuned hipBLASLt for the rest."""
     if (
         x.is_cuda
         and x.dim() == 2
         and x.dtype == torch.bfloat16
         and 0 < x.shape[0] <= SKINNY_GEMM_MAX_M
-        and weight.shape[0] % 64 == 0
-        and weight.shape[1] % 32 == 0
+        and weight.dtype == torch.bfloat16
+        and weight.is_contiguous()
         and x.stride(1) == 1
+        and (bias is None or bias.dtype == torch.bfloat16)
     ):
         ext = _require_ext("skinny_gemm")
         out = torch.empty(
             x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device
         )
-        if ext.skinny_gemm(out, x, weight,
-                           bias if bias is not None else x.new_empty(0)):
+        none = x.new_empty(0)
+        if ext.skinny_gemm(out, x, weight, none if bias is None else bias,
+                           none, none):
             return out
     if (
         LT_GEMM
@@ -541,35 +542,54 @@ def fused_moe_forward(
         bool(weight_on_input))
 
 
-_FP8_LIN_BUFS = {}
-
-
 def linear_fp8(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor,
                bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """W8A8 dense GEMM through hipBLASLt fp8: x quantized per-tensor on the
-    fly into persistent per-shape buffers (graph-capture safe: the scale and
-    xq pointers baked into a captured graph never move). CPU fallback
-    dequantizes (plumbing tests)."""
+    """W8A8 dense GEMM: x quantized per-tensor on the fly (two launches, the
+    scale stays on the device), then the weight-streaming kernel for few rows
+    or hipBLASLt fp8. CPU fallback dequantizes (plumbing tests)."""
     if not x.is_cuda:
         w = (w_q.float() * w_scale.float()).to(torch.float32)
         y = torch.nn.functional.linear(x.float(), w).to(x.dtype)
         return y if bias is None else y + bias
     ext = _require_ext("lt_linear_fp8")
-    M, K = x.shape
-    key = (M, K, x.device.index)
-    bufs = _FP8_LIN_BUFS.get(key)
-    if bufs is None:
-        bufs = (
-            torch.empty(M, K, dtype=torch.float8_e4m3fn, device=x.device),
-            torch.ones(1, dtype=torch.float32, device=x.device),
+    M, _ = x.shape
+    xq, xs = ext.quantize_fp8_tensor(
+        (x if x.dtype == torch.bfloat16 else x.float()).contiguous())
+    if 0 < M <= SKINNY_GEMM_MAX_M and (
+        bias is None or bias.dtype == torch.bfloat16
+    ):
+        out = torch.empty(
+            M, w_q.shape[0], dtype=torch.bfloat16, device=x.device
         )
-        _FP8_LIN_BUFS[key] = bufs
-    xq, xs = bufs
-    xf = x.float()
-    xs.copy_((xf.abs().amax() / 448.0).clamp_min(1e-8).reshape(1))
-    xq.copy_((xf / xs).clamp(-448.0, 448.0))
+        if ext.skinny_gemm(out, xq, w_q, xs.new_empty(0, dtype=torch.bfloat16)
+                           if bias is None else bias, xs, w_scale):
+            return out
     y = ext.lt_linear_fp8(xq, w_q, xs, w_scale)
     return y if bias is None else y + bias
+
+
+def mla_absorb(q_nope: torch.Tensor, w_uk: torch.Tensor) -> torch.Tensor:
+    """Queries [B, H, dn] into latent space [B, H, r] through w_uk [H, dn, r],
+    fp32 sums."""
+    if q_nope.is_cuda and q_nope.dtype == w_uk.dtype == torch.bfloat16:
+        ext = _require_ext("mla_absorb")
+        out = q_nope.new_empty(*q_nope.shape[:2], w_uk.shape[2])
+        if ext.mla_absorb(out, q_nope, w_uk):
+            return out
+    return torch.einsum(
+        "bhd,hdr->bhr", q_nope.float(), w_uk.float()).to(q_nope.dtype)
+
+
+def mla_project_out(out_latent: torch.Tensor, w_uv: torch.Tensor) -> torch.Tensor:
+    """Latent results [B, H, r] to heads [B, H, dv] through w_uv [H, dv, r],
+    fp32 sums."""
+    if out_latent.is_cuda and out_latent.dtype == w_uv.dtype == torch.bfloat16:
+        ext = _require_ext("mla_project")
+        out = out_latent.new_empty(*out_latent.shape[:2], w_uv.shape[1])
+        if ext.mla_project(out, out_latent, w_uv):
+            return out
+    return torch.einsum(
+        "bhr,hvr->bhv", out_latent.float(), w_uv.float()).to(out_latent.dtype)
 
 
 def quantize_fp8_weight(w: torch.Tensor):

@@ -85,8 +85,14 @@ void launch_quantize_fp8_rows(void*, float*, const void*, int, int,
                               hipStream_t);
 void launch_sample_gumbel(int64_t*, const float*, const float*,
                           const uint8_t*, uint64_t, int, int, hipStream_t);
-void launch_skinny_gemm(void*, const void*, const void*, const void*, int,
-                        int, int, int64_t, int64_t, hipStream_t, bool*);
+void launch_skinny_gemm(void*, const void*, const void*, const void*,
+                        const float*, const float*, bool, int, int, int, int64_t,
+                        int64_t, int, int64_t, int64_t, hipStream_t, bool*);
+void launch_mla_absorb(void*, const void*, const void*, int, int, int, int64_t,
+                       int64_t, hipStream_t);
+int quantize_fp8_tensor_parts(int64_t);
+void launch_quantize_fp8_tensor(void*, float*, uint32_t*, const void*, int64_t,
+                                bool, hipStream_t);
 int prefill_attention_tiles(int, int, int, int);
 void launch_prefill_attention(void*, float*, float*, const void*, const void*,
                               const void*, const int*, const int*, const int*,
@@ -686,21 +692,98 @@ torch::Tensor sample_gumbel(torch::Tensor logits, torch::Tensor inv_temp,
   return out;
 }
 
+// c = x . w^T (+ bias): bf16, or fp8 with the two scales given. False where there
+// is no kernel.
 bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
-                 torch::Tensor bias) {
+                 torch::Tensor bias, torch::Tensor x_scale,
+                 torch::Tensor w_scale) {
   CHECK_GPU(x);
-  CHECK_BF16(x);
-  CHECK_BF16(w);
-  TORCH_CHECK(w.is_contiguous());
-  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1);
-  TORCH_CHECK(c.dim() == 2 && c.stride(1) == 1);
-  const int M = x.size(0);
-  const int K = x.size(1);
-  const int N = w.size(0);
+  const bool fp8 = x_scale.numel() > 0;
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) &&
+              x.stride(1) == 1 && c.dim() == 2 && c.stride(1) == 1 &&
+              c.size(0) == x.size(0) && c.size(1) == w.size(0));
+  CHECK_CONTIG(w);
+  CHECK_BF16(c);
+  if (fp8) {
+    TORCH_CHECK(is_fp8(x) && is_fp8(w) &&
+                x_scale.scalar_type() == at::kFloat &&
+                w_scale.scalar_type() == at::kFloat);
+    if (w_scale.numel() != 1) return false;
+  } else {
+    CHECK_BF16(x);
+    CHECK_BF16(w);
+  }
+  CHECK_BF16(bias);
+  if (bias.numel() && (bias.dim() != 1 || bias.numel() != w.size(0) ||
+                       !bias.is_contiguous()))
+    return false;
+  const int64_t es = x.element_size();
+  if ((uintptr_t)x.data_ptr() % 16 || (uintptr_t)w.data_ptr() % 16 ||
+      x.stride(0) * es % 16 || (uintptr_t)c.data_ptr() % 8 || c.stride(0) % 4)
+    return false;
   bool launched = false;
   launch_skinny_gemm(c.data_ptr(), x.data_ptr(), w.data_ptr(),
-                     bias.numel() ? bias.data_ptr() : nullptr, M, N, K,
-                     x.stride(0), c.stride(0), cur_stream(), &launched);
+                     bias.numel() ? bias.data_ptr() : nullptr,
+                     fp8 ? x_scale.data_ptr<float>() : nullptr,
+                     fp8 ? w_scale.data_ptr<float>() : nullptr, fp8, x.size(0),
+                     w.size(0), x.size(1) * es, x.stride(0) * es, c.stride(0), 1,
+                     0, 0, cur_stream(), &launched);
+  return launched;
+}
+
+// x quantised per tensor: (fp8 values, scale [1])
+std::tuple<torch::Tensor, torch::Tensor> quantize_fp8_tensor(torch::Tensor x) {
+  CHECK_GPU(x);
+  CHECK_CONTIG(x);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat);
+  TORCH_CHECK(x.numel() > 0, "quantize_fp8_tensor: empty input");
+  auto q = torch::empty(x.sizes(), x.options().dtype(at::kFloat8_e4m3fn));
+  const int64_t n = x.numel();
+  auto scale = torch::empty({1}, x.options().dtype(at::kFloat));
+  auto part = torch::empty({quantize_fp8_tensor_parts(n)},
+                           x.options().dtype(at::kInt));
+  launch_quantize_fp8_tensor(q.data_ptr(), scale.data_ptr<float>(),
+                             (uint32_t*)part.data_ptr(), x.data_ptr(), n,
+                             x.scalar_type() == at::kBFloat16, cur_stream());
+  return {q, scale};
+}
+
+static bool rows16(const torch::Tensor& t) {
+  return t.scalar_type() == at::kBFloat16 && (uintptr_t)t.data_ptr() % 16 == 0 &&
+         t.stride(2) == 1 && t.stride(1) % 8 == 0 && t.stride(0) % 8 == 0;
+}
+
+// MLA's per-head products with bf16 results [B, H, R] and [B, H, dv]; false where
+// there is no kernel.
+bool mla_absorb(torch::Tensor out, torch::Tensor q, torch::Tensor w) {
+  CHECK_GPU(q);
+  const int64_t B = q.size(0), H = q.size(1), R = w.size(2);
+  if (!rows16(q) || !rows16(w) || q.size(2) != 128 || R % 128) return false;
+  CHECK_CONTIG(w);
+  CHECK_CONTIG(out);
+  CHECK_BF16(out);
+  TORCH_CHECK(w.size(0) == H && w.size(1) == 128 && out.size(0) == B &&
+              out.size(1) == H && out.size(2) == R);
+  if (B == 0) return true;
+  launch_mla_absorb(out.data_ptr(), q.data_ptr(), w.data_ptr(), B, H, R,
+                    q.stride(0), q.stride(1), cur_stream());
+  return true;
+}
+
+bool mla_project(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
+  CHECK_GPU(x);
+  const int64_t B = x.size(0), H = x.size(1), N = w.size(1), K = w.size(2);
+  if (!rows16(x) || !rows16(w) || K % 64 || N % 64) return false;
+  CHECK_CONTIG(w);
+  CHECK_CONTIG(out);
+  CHECK_BF16(out);
+  TORCH_CHECK(w.size(0) == H && x.size(2) == K && out.size(0) == B &&
+              out.size(1) == H && out.size(2) == N);
+  if (B == 0) return true;
+  bool launched = false;
+  launch_skinny_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), nullptr, nullptr,
+                     nullptr, false, B, N, K * 2, x.stride(0) * 2, out.stride(0),
+                     H, x.stride(1) * 2, out.stride(1), cur_stream(), &launched);
   return launched;
 }
 
@@ -744,6 +827,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "tuned hipBLASLt y = x @ w^T (bf16, fp32 accum)");
   m.def("msa_paged_attention_decode", &msa_paged_attention_decode);
   m.def("skinny_gemm", &skinny_gemm);
+  m.def("quantize_fp8_tensor", &quantize_fp8_tensor);
+  m.def("mla_absorb", &mla_absorb);
+  m.def("mla_project", &mla_project);
   m.def("sample_gumbel", &sample_gumbel);
   m.def("moe_forward", &moe_forward);
   m.def("moe_forward_fp8", &moe_forward_fp8);

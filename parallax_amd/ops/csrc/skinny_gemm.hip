@@ -1,100 +1,446 @@
-// Skinny-M dense GEMM: C[M,N] = X[M,K] . W[N,K]^T (+bias), M <= 256.
+// Products of few rows with a large weight: C[M, N] = X[M, K] . W[N, K]^T (+ bias),
+// bf16 or (scaled per tensor) fp8.
 //
-// Decode-step GEMMs are M = batch (1-256) against multi-hundred-MB weight
-// matrices — pure weight streaming. hipBLASLt's tile picks run 2-5x off the
-// HBM roofline at these shapes (measured, profiles/README.md). Structure:
-// one workgroup per 64-column W slab; the X K-slab (M x 128) is staged in LDS
-// once per iteration (cooperative coalesced loads, padded rows against bank
-// conflicts) and every wave's MFMA A-fragments come from LDS; each W row is
-// streamed exactly once per slab by the lane that owns that output column.
+// A decode step's projections: the weight's stream is the bound. A workgroup
+// takes NT rows of W; its waves deal the 128-byte columns of those rows among
+// them (wave w the columns w, w + WAVES, ..), so that it reads long runs of
+// each row, and every wave is on its own: W and X go global -> LDS directly
+// into its own ring of STAGES, and it waits for its own copies only. No barrier
+// until the sums of the waves are added at the end. A head start of its own
+// rotates every workgroup's columns: rows lie a power of two apart, and all
+// workgroups at one column would wait for the same L2 channels (28672 x 4096, 8
+// rows: 44 to 40 us).
+//
+// What bounds it: up to 8 rows the stream from memory (28672 x 4096 in 39 us, 6.0
+// TB/s; 4096 x 14336 in 22 us; the library 52 and 25), for small weights one round
+// trip and the launch (896 x 896 in 3.3 us, before 5.5); with more rows what L2
+// delivers, W and X together 8.8 TB/s.
+
+#include <type_traits>
 
 #include "common.h"
 
-#define SG_THREADS 256
-#define SG_BK 128           // K elements staged per iteration
-#define SG_PROW (SG_BK + 8) // padded LDS row (elements)
+typedef float f32x16v __attribute__((ext_vector_type(16)));
+typedef short s16x4v __attribute__((ext_vector_type(4)));
+typedef long longx2n __attribute__((ext_vector_type(2)));
 
-template <int MTILES>
-__global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
-    uint16_t* __restrict__ c,        // [M, N] bf16 rows at c_stride
-    const uint16_t* __restrict__ x,  // [M, K] rows at x_stride
-    const uint16_t* __restrict__ w,  // [N, K]
-    const uint16_t* __restrict__ bias,  // [N] or nullptr
-    const int M, const int N, const int K, const int64_t x_stride,
-    const int64_t c_stride) {
+namespace {
+
+DEVINL void copy16_to_lds(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)src,
+      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+template <int N>
+DEVINL void wait_copies() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N & 48) << 10));
+  asm volatile("" ::: "memory");
+}
+
+// Two to six operands of 16 bytes a lane, at at + 2048 t and x_at + 2048 u. Not
+// plain loads: before those the compiler waits for every copy in flight.
+template <int A, int B>
+DEVINL void read_operands(const uint32_t at, const uint32_t x_at, bf16x8v (&a)[A],
+                          bf16x8v (&b)[B]) {
+  static_assert((A == 1 || A == 2 || A == 4) && (B == 1 || B == 2 || B == 4), "");
+  if constexpr (A == 4) {
+    asm volatile(
+        "ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\t"
+        "ds_read_b128 %2, %4 offset:4096\n\tds_read_b128 %3, %4 offset:6144\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3])
+        : "v"(at) : "memory");
+  }
+  if constexpr (B == 4) {
+    asm volatile(
+        "ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\t"
+        "ds_read_b128 %2, %4 offset:4096\n\tds_read_b128 %3, %4 offset:6144\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
+        : "v"(x_at) : "memory");
+  }
+  if constexpr (A == 1 && B == 1)
+    asm volatile(
+        "ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(b[0]) : "v"(at), "v"(x_at) : "memory");
+  if constexpr (A == 2 && B == 1)
+    asm volatile(
+        "ds_read_b128 %0, %3\n\tds_read_b128 %1, %3 offset:2048\n\t"
+        "ds_read_b128 %2, %4\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(a[1]), "=&v"(b[0])
+        : "v"(at), "v"(x_at) : "memory");
+  if constexpr (A == 1 && B == 2)
+    asm volatile(
+        "ds_read_b128 %0, %3\n\tds_read_b128 %1, %4\n\t"
+        "ds_read_b128 %2, %4 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(b[0]), "=&v"(b[1])
+        : "v"(at), "v"(x_at) : "memory");
+  if constexpr (A == 2 && B == 2)
+    asm volatile(
+        "ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\t"
+        "ds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:2048\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(a[1]), "=&v"(b[0]), "=&v"(b[1])
+        : "v"(at), "v"(x_at) : "memory");
+  if constexpr (A == 2 && B == 4)
+    asm volatile(
+        "ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:2048\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(a[1]) : "v"(at) : "memory");
+  if constexpr (A == 4 && B == 2)
+    asm volatile(
+        "ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:2048\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(b[0]), "=&v"(b[1]) : "v"(x_at) : "memory");
+  if constexpr (A == 1 && B == 4)
+    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0]) : "v"(at) : "memory");
+  if constexpr (A == 4 && B == 1)
+    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(b[0]) : "v"(x_at) : "memory");
+}
+
+}  // namespace
+
+// XR: rows of X staged, a multiple of 8 that holds M.
+template <bool FP8, int NT, int XR, int WAVES, int STAGES>
+__global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
+    uint16_t* __restrict__ c,          // [M, N] bf16 rows at c_stride
+    const uint8_t* __restrict__ x,     // [M, K] rows at x_stride bytes
+    const uint8_t* __restrict__ w,     // [N, K]
+    const uint16_t* __restrict__ bias, // [N] or null
+    const float* __restrict__ x_scale, const float* __restrict__ w_scale,
+    const int M_all, const int N, const int row_bytes, const int64_t x_stride,
+    const int64_t c_stride, const int64_t x_batch, const int64_t c_batch) {
+  constexpr int ROWS = NT + XR;
+  constexpr int NI = ROWS / 8;  // copies a stage: 8 rows of 128 bytes each
+  constexpr int MT = (XR + 15) / 16;
+  constexpr int MP = MT * 16;
+  constexpr int RING = ROWS * 128;  // a wave's stage
+  __shared__ __attribute__((aligned(128))) uint8_t S[WAVES * STAGES * RING];
+
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int l15 = lane & 15;
-  const int l4 = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, l4 = lane >> 4;
+  const int n0 = blockIdx.x * NT;
+  const int M = min(XR, M_all - (int)blockIdx.z * XR);
+  x += blockIdx.y * x_batch + blockIdx.z * XR * x_stride;
+  c += blockIdx.y * c_batch + blockIdx.z * XR * c_stride;
+  const uint8_t* wb = w + ((size_t)blockIdx.y * N + n0) * row_bytes;
 
-  const int n = blockIdx.x * 64 + wid * 16 + l15;  // this lane's W row / C col
-  const uint16_t* wrow = w + (size_t)n * K;
-
-  __shared__ uint16_t Xl[MTILES * 16 * SG_PROW];
-
-  f32x4v acc[MTILES] = {};
-  for (int k0 = 0; k0 < K; k0 += SG_BK) {
-    __syncthreads();
-    // stage X[:, k0:k0+128]: (row, 16B chunk) pairs over all threads so small
-    // M still engages the whole workgroup, chunks coalesce within a row.
-    // Rows past M are zero-filled (read by padded MFMA rows).
-    for (int idx = tid; idx < MTILES * 16 * (SG_BK / 8); idx += SG_THREADS) {
-      const int row = idx / (SG_BK / 8);
-      const int cc = idx % (SG_BK / 8);
-      int4 val = make_int4(0, 0, 0, 0);
-      if (row < M)
-        val = *reinterpret_cast<const int4*>(
-            x + (size_t)row * x_stride + k0 + cc * 8);
-      *reinterpret_cast<int4*>(Xl + row * SG_PROW + cc * 8) = val;
-    }
-    __syncthreads();
-
+  // chunk (row, j) of a stage lies at j ^ (row / 2 & 7) in the row's 128 bytes
+  uint32_t at[NI];
 #pragma unroll
-    for (int ks = 0; ks < SG_BK / 32; ++ks) {
-      const bf16x8v bfrag = *reinterpret_cast<const bf16x8v*>(
-          wrow + k0 + ks * 32 + l4 * 8);
-#pragma unroll
-      for (int mt = 0; mt < MTILES; ++mt) {
-        const int row = mt * 16 + l15;
-        // stale LDS rows past M contribute to padded acc rows only, which are
-        // never stored — but keep them zeroed for NaN safety
-        const bf16x8v afrag = *reinterpret_cast<const bf16x8v*>(
-            Xl + row * SG_PROW + ks * 32 + l4 * 8);
-        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, bfrag,
-                                                          acc[mt], 0, 0, 0);
-      }
-    }
+  for (int i = 0; i < NI; ++i) {
+    const int r = i * 8 + (lane >> 3);
+    const int j = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    at[i] = r < NT ? (uint32_t)min(r, N - 1 - n0) * row_bytes + j
+                   : (uint32_t)min(r - NT, M - 1) * (uint32_t)x_stride + j;
   }
+  const int cols = row_bytes / 128;
+  const int mine = (cols - wid + WAVES - 1) / WAVES;
 
-  const float b = bias != nullptr ? bf16_bits_to_f32(bias[n]) : 0.f;
+  const int rot0 = mine > 0 ? (int)((blockIdx.x >> 3) * 3 % mine) : 0;
+  uint8_t* ring = S + wid * (STAGES * RING);
+  auto issue = [&](int i, int place) __attribute__((always_inline)) {
+    int t = min(i, mine - 1) + rot0;
+    if (t >= mine) t -= mine;
+    const int k = (t * WAVES + wid) * 128;
+    uint8_t* dst = ring + place * RING;
 #pragma unroll
-  for (int mt = 0; mt < MTILES; ++mt) {
+    for (int q = 0; q < NI; ++q)
+      copy16_to_lds((q * 8 < NT ? wb : x) + k + at[q], dst + q * 1024);
+  };
+
+  f32x4v acc[NT / 16][MT] = {};
+  const uint32_t ring_at =
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring;
+  const int j0 = (l4 ^ ((l15 >> 1) & 7)) * 16;
+  const int xr = l15 & (XR < 16 ? XR - 1 : 15);
+  const uint32_t a_at = ring_at + l15 * 128 + j0;
+  const uint32_t b_at =
+      ring_at + (NT + xr) * 128 + (l4 ^ ((xr >> 1) & 7)) * 16;
+  int place = 0, next = STAGES - 1;
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i)
+    if (mine > 0) issue(i, i);
+  for (int i = 0; i < mine; ++i) {
+    wait_copies<(STAGES - 2) * NI>();
+    // into the place read in the turn before: its operands are in registers
+    issue(i + STAGES - 1, next);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8v a[NT / 16], b[MT];
+      read_operands((a_at + place * RING) ^ (ks * 64), (b_at + place * RING) ^ (ks * 64),
+                    a, b);
+#pragma unroll
+      for (int t = 0; t < NT / 16; ++t)
+#pragma unroll
+        for (int u = 0; u < MT; ++u) {
+          if constexpr (FP8) {
+            const auto p = __builtin_bit_cast(longx2n, a[t]);
+            const auto q = __builtin_bit_cast(longx2n, b[u]);
+            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                p[0], q[0], acc[t][u], 0, 0, 0);
+            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                p[1], q[1], acc[t][u], 0, 0, 0);
+          } else {
+            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a[t], b[u], acc[t][u], 0, 0, 0);
+          }
+        }
+    }
+    place = place + 1 == STAGES ? 0 : place + 1;
+    next = next + 1 == STAGES ? 0 : next + 1;
+  }
+  wait_copies<0>();
+  __syncthreads();
+  float* part = reinterpret_cast<float*>(S);
+  static_assert(MP * NT * 4 <= STAGES * RING, "");
+#pragma unroll
+  for (int t = 0; t < NT / 16; ++t)
+#pragma unroll
+    for (int u = 0; u < MT; ++u)
+      *reinterpret_cast<f32x4v*>(
+          part + ((wid * MP + u * 16 + l15) * NT + t * 16 + l4 * 4)) = acc[t][u];
+  __syncthreads();
+  const float scale = FP8 ? x_scale[0] * w_scale[0] : 1.f;
+  for (int e = tid; e < M * (NT / 4); e += WAVES * 64) {
+    const int m = e / (NT / 4), n = e % (NT / 4) * 4;
+    if (n0 + n >= N) continue;
+    f32x4v s = {};
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v)
+      s += *reinterpret_cast<const f32x4v*>(part + ((v * MP + m) * NT + n));
+    uint16_t o[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = mt * 16 + l4 * 4 + r;
-      if (row < M)
-        c[(size_t)row * c_stride + n] = f32_to_bf16_bits(acc[mt][r] + b);
+      float f = FP8 ? s[r] * scale : s[r];
+      if (bias != nullptr) f += bf16_bits_to_f32(bias[n0 + n + r]);
+      o[r] = f32_to_bf16_bits(f);
     }
+    *reinterpret_cast<uint2*>(c + (size_t)m * c_stride + n0 + n) =
+        make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
   }
 }
 
+// Tiles, by rows of X and by how many tiles W gives. us of bf16 products, W from
+// memory (N x K; the library's tuned pick last):
+//   up to 8 rows, NT 16 of 4 waves, 5 stages / 3 stages (four workgroups a CU
+//   instead of two): 28672 x 4096 40 / 41 (50), 4096 x 14336 22 / 25 (25), 9728 x
+//   896 8.6 / 6.6 (12), 24576 x 1536 17 / 16 (21), 896 x 896 3.3 (5.5)
+//   9 to 16, NT 16 / 32 / 64: X comes from L2 once a tile, so the widest tile
+//   that still gives 150 workgroups: 6144 x 4096 14.5 / 12.1 / 16.6 (15.7),
+//   28672 x 4096 48 / 45 / 42 (54), 4096 x 14336 26 / 32 / 49 (26)
+//   17 to 32, the same: 28672 x 4096 60 / 47 / 43 (56), 6144 x 4096 18 / 13.9 /
+//   19.5 (15.2), 4096 x 4096 10.7 / 13.4 / 19 (11.8); below 4800 rows of W and
+//   above 10 KB a row the library's split of K is better: 1536 x 7168 15 (12)
+// More rows of X than 32 need W's tiles shared: the library.
+static int skinny_tile(int M, int64_t N, int row_bytes) {
+  if (M <= 8) return 16;
+  if (N >= 9600) return 64;
+  if (N >= 4800) return 32;
+  return M <= 16 || row_bytes <= 10240 ? 16 : 0;
+}
+
+// batch products of the same shape: x, w and c advance by x_batch bytes, N rows
+// and c_batch elements. A batch takes any number of rows of X, 32 at a time.
 extern "C" void launch_skinny_gemm(
-    void* c, const void* x, const void* w, const void* bias, int M, int N,
-    int K, int64_t x_stride, int64_t c_stride, hipStream_t stream,
-    bool* launched) {
+    void* c, const void* x, const void* w, const void* bias,
+    const float* x_scale, const float* w_scale, bool fp8, int M, int N,
+    int row_bytes, int64_t x_stride, int64_t c_stride, int batch,
+    int64_t x_batch, int64_t c_batch, hipStream_t stream, bool* launched) {
   *launched = false;
-  if (M > 256 || N % 64 != 0 || K % SG_BK != 0) return;
-  dim3 grid(N / 64, 1, 1);
-#define SG_LAUNCH(MT)                                                      \
-  skinny_gemm_kernel<MT><<<grid, SG_THREADS, 0, stream>>>(                 \
-      (uint16_t*)c, (const uint16_t*)x, (const uint16_t*)w,                \
-      (const uint16_t*)bias, M, N, K, x_stride, c_stride);                 \
+  const int nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes);
+  if (nt == 0 || (M > 32 && batch == 1) || row_bytes % 128 || N % 4) return;
   *launched = true;
-  if (M <= 16) { SG_LAUNCH(1) }
-  else if (M <= 32) { SG_LAUNCH(2) }
-  else if (M <= 64) { SG_LAUNCH(4) }
-  else if (M <= 128) { SG_LAUNCH(8) }
-  else { SG_LAUNCH(16) }
-#undef SG_LAUNCH
+  auto run = [&](auto kernel, int xr, int waves) {
+    kernel<<<dim3(ceil_div(N, nt), batch, ceil_div(M, xr)), waves * 64, 0,
+             stream>>>(
+        (uint16_t*)c, (const uint8_t*)x, (const uint8_t*)w,
+        (const uint16_t*)bias, x_scale, w_scale, M, N, row_bytes, x_stride,
+        c_stride, x_batch, c_batch);
+  };
+  auto pick = [&](auto f) {
+    constexpr bool F = decltype(f)::value;
+    if (M <= 8) {
+      if (row_bytes <= 4096) run(skinny_gemm_kernel<F, 16, 8, 4, 3>, 8, 4);
+      else run(skinny_gemm_kernel<F, 16, 8, 4, 5>, 8, 4);
+    } else if (M <= 16) {
+      if (nt == 64) run(skinny_gemm_kernel<F, 64, 16, 2, 4>, 16, 2);
+      else if (nt == 32) run(skinny_gemm_kernel<F, 32, 16, 4, 3>, 16, 4);
+      else run(skinny_gemm_kernel<F, 16, 16, 4, 4>, 16, 4);
+    } else {
+      if (nt == 64) run(skinny_gemm_kernel<F, 64, 32, 2, 3>, 32, 2);
+      else if (nt == 32) run(skinny_gemm_kernel<F, 32, 32, 2, 4>, 32, 2);
+      else run(skinny_gemm_kernel<F, 16, 32, 4, 3>, 32, 4);
+    }
+  };
+  if (fp8) pick(std::true_type{});
+  else pick(std::false_type{});
+}
+
+// ---- MLA queries into latent space ----------------------------------------------------
+// out[b, h] = q[b, h] . W[h] of [128, R]: rows of W run along the result, so its
+// operand is read transposed from LDS. A workgroup takes 128 of the R columns of
+// one head and 32 rows of q, one pass. W's stream bounds it: 40 rows at 128
+// heads 9 us, fp32 copies and an fp32
+// product before 45 us.
+
+__global__ __launch_bounds__(256) void mla_absorb_kernel(
+    uint16_t* __restrict__ out,      // [B, H, R]
+    const uint16_t* __restrict__ q,  // [B, H, 128] by strides
+    const uint16_t* __restrict__ w,  // [H, 128, R]
+    const int B, const int H, const int R, const int64_t q_row,
+    const int64_t q_head) {
+  __shared__ __attribute__((aligned(128))) uint16_t W[128 * 128];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, l31 = lane & 31;
+  const int h = blockIdx.y;
+  const int b = blockIdx.z * 32 + l31;
+  const uint16_t* src = w + (size_t)h * 128 * R + blockIdx.x * 128;
+  // 16-byte chunk j of row k lies at j ^ 4 (k & 3)
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int k = i * 16 + (tid >> 4);
+    copy16_to_lds(src + (size_t)k * R + ((tid & 15) ^ ((k & 3) * 4)) * 8,
+                  W + (i * 16 + wid * 4) * 128);
+  }
+  bf16x8v x[8];
+  const uint16_t* qr =
+      q + (size_t)min(b, B - 1) * q_row + (size_t)h * q_head + half * 8;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) x[s] = *(const bf16x8v*)(qr + s * 16);
+  wait_copies<0>();
+  __syncthreads();
+  const int i15 = lane & 15;
+  const int chunk = (wid * 4 + ((lane >> 4) & 1) * 2 + ((i15 & 3) >> 1)) ^
+                    ((i15 >> 2) * 4);
+  uint16_t* at = W + (half * 8 + (i15 >> 2)) * 128 + chunk * 8 + (i15 & 1) * 4;
+  f32x16v acc = {};
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const s16x4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4v*)(at + s * 16 * 128));
+    const s16x4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4v*)(at + s * 16 * 128 + 4 * 128));
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+        __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), x[s], acc, 0, 0,
+        0);
+  }
+  if (b >= B) return;
+  uint16_t* dst = out + ((size_t)b * H + h) * R + blockIdx.x * 128 + wid * 32 +
+                  4 * half;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint16_t o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = f32_to_bf16_bits(acc[4 * i + r]);
+    *reinterpret_cast<uint2*>(dst + 8 * i) =
+        make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
+  }
+}
+
+extern "C" void launch_mla_absorb(void* out, const void* q, const void* w, int B,
+                                  int H, int R, int64_t q_row, int64_t q_head,
+                                  hipStream_t stream) {
+  mla_absorb_kernel<<<dim3(R / 128, H, ceil_div(B, 32)), 256, 0, stream>>>(
+      (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)w, B, H, R, q_row,
+      q_head);
+}
+
+// ---- activations to fp8 (OCP e4m3), one scale a tensor -------------------------------
+// scale = max(amax * (1 / 448), 1e-8), values x / scale clamped to +-448. Two passes:
+// the largest magnitude a workgroup (as bits, so that NaN is the largest), then
+// every workgroup reduces those and converts its part. Launches bound it at
+// decode sizes: 2 instead of 7 operations of torch and a copy.
+
+#define Q8_MAX_BLOCKS 256
+
+template <typename T>
+DEVINL uint32_t magnitude(T v) {
+  if constexpr (sizeof(T) == 2) return (uint32_t)(v & 0x7fff) << 16;
+  else return v & 0x7fffffffu;
+}
+
+DEVINL uint32_t block_max(uint32_t m, uint32_t* lds) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = m;
+  __syncthreads();
+  return max(max(lds[0], lds[1]), max(lds[2], lds[3]));
+}
+
+// T: the bits of a bf16 or fp32 value; whole vectors of 8 first, then the rest
+template <typename T, typename F>
+DEVINL void for_each8(const T* x, int64_t n, bool aligned, F f) {
+  struct __attribute__((aligned(16))) V { T v[8]; };
+  const int64_t step = (int64_t)gridDim.x * 256;
+  const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t nv = aligned ? n / 8 : 0;
+  for (int64_t i = first; i < nv; i += step) {
+    const V v = reinterpret_cast<const V*>(x)[i];
+    f(i * 8, v.v, 8);
+  }
+  for (int64_t i = nv * 8 + first; i < n; i += step) f(i, x + i, 1);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void fp8_amax_kernel(
+    uint32_t* __restrict__ part, const T* __restrict__ x, const int64_t n,
+    const bool aligned) {
+  __shared__ uint32_t lds[4];
+  uint32_t m = 0;
+  for_each8(x, n, aligned, [&](int64_t, const T* v, int c) {
+    for (int j = 0; j < c; ++j) m = max(m, magnitude(v[j]));
+  });
+  m = block_max(m, lds);
+  if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void fp8_convert_kernel(
+    uint8_t* __restrict__ out, float* __restrict__ scale_out,
+    const uint32_t* __restrict__ part, const T* __restrict__ x, const int64_t n,
+    const bool aligned) {
+  __shared__ uint32_t lds[4];
+  const uint32_t m = threadIdx.x < gridDim.x ? part[threadIdx.x] : 0;
+  float scale = __uint_as_float(block_max(m, lds)) * (1.f / 448.f);
+  if (scale < 1e-8f) scale = 1e-8f;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
+  for_each8(x, n, aligned, [&](int64_t i, const T* v, int c) {
+    uint64_t q = 0;
+    for (int j = 0; j < c; ++j) {
+      float f = (sizeof(T) == 2 ? __uint_as_float((uint32_t)v[j] << 16)
+                                : __uint_as_float((uint32_t)v[j])) / scale;
+      f = f > 448.f ? 448.f : f < -448.f ? -448.f : f;
+      q |= (uint64_t)f32_to_fp8_e4m3(f) << (8 * j);
+    }
+    if (c == 8) *reinterpret_cast<uint64_t*>(out + i) = q;
+    else out[i] = (uint8_t)q;
+  });
+}
+
+extern "C" int quantize_fp8_tensor_parts(int64_t n) {
+  return clamp_int((n + 2047) / 2048, 1, Q8_MAX_BLOCKS);
+}
+
+extern "C" void launch_quantize_fp8_tensor(void* out, float* scale,
+                                           uint32_t* part, const void* x,
+                                           int64_t n, bool is_bf16,
+                                           hipStream_t stream) {
+  const int blocks = quantize_fp8_tensor_parts(n);
+  const bool aligned = (uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0;
+  auto run = [&](auto* p) {
+    fp8_amax_kernel<<<blocks, 256, 0, stream>>>(part, p, n, aligned);
+    fp8_convert_kernel<<<blocks, 256, 0, stream>>>((uint8_t*)out, scale, part, p,
+                                                   n, aligned);
+  };
+  if (is_bf16) run((const uint16_t*)x);
+  else run((const uint32_t*)x);
 }

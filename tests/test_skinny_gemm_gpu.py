@@ -1,0 +1,111 @@
+"""Few rows against a large weight, its fp8 form and MLA's per-head products,
+against fp32."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from parallax_amd import ops
+
+
+def _rand(g, *s):
+    return torch.randn(*s, generator=g, device="cuda")
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [
+    (4, 64),        # one column of 128 bytes: waves without one
+    (900, 896),     # a tile cut by the last row
+    (4804, 2176),   # 32 rows a tile, deep rings
+    (9604, 320),    # 64 rows a tile
+])
+def test_linear_few_rows(M, N, K):
+    """fp32 sums of exact products: 2^-9 of the result for its rounding, and
+    K 2^-24 of the sum of magnitudes (< K here) for the sums."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = _rand(g, M, 2 * K).bfloat16()[:, K:]
+    w = _rand(g, N, K).bfloat16()
+    b = _rand(g, N).bfloat16()
+    ext = ops._require_ext("skinny_gemm")
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    none = x.new_empty(0)
+    assert ext.skinny_gemm(out, x, w, none, none, none)
+    want = x.float() @ w.float().t()
+    tol = dict(rtol=2 ** -8, atol=K * K * 2 ** -24)
+    torch.testing.assert_close(out.float(), want, **tol)
+    torch.testing.assert_close(ops.linear(x, w, b).float(), want + b.float(), **tol)
+
+
+def test_linear_without_a_kernel():
+    """Odd widths and misaligned rows take the library and agree."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    for M, N, K in ((5, 8, 72), (3, 6, 64), (33, 64, 64), (20, 576, 7168)):
+        x, w = _rand(g, M, K).bfloat16(), _rand(g, N, K).bfloat16()
+        torch.testing.assert_close(
+            ops.linear(x, w).float(), x.float() @ w.float().t(), rtol=2 ** -8,
+            atol=K * K * 2 ** -24)
+    x = _rand(g, 4, 65).bfloat16()[:, 1:]
+    w = _rand(g, 64, 64).bfloat16()
+    torch.testing.assert_close(
+        ops.linear(x, w).float(), x.float() @ w.float().t(), rtol=2 ** -8, atol=1e-3)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 128), (7, 4800, 5120), (16, 64, 256),
+                                   (30, 9600, 384), (40, 256, 512)])
+def test_linear_fp8_rows(M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = _rand(g, M, K).bfloat16()
+    w = _rand(g, N, K).to(torch.float8_e4m3fn)
+    ws = torch.tensor([0.37], device="cuda")
+    xs = (x.float().abs().amax() / 448.0).clamp_min(1e-8).reshape(1)
+    xq = (x.float() / xs).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+    want = (xq.float() @ w.float().t()) * (xs * ws)
+    torch.testing.assert_close(
+        ops.linear_fp8(x, w, ws).float(), want, rtol=2 ** -8,
+        atol=K * K * 2 ** -24)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 7, 2048, 2057, 700001])
+def test_quantize_fp8_tensor(dtype, n):
+    """Bytes and scale as the torch operations give them, also with zeros,
+    infinities and NaN."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    ext = ops._require_ext("quantize_fp8_tensor")
+    base = (_rand(g, n + 1) * 100).to(dtype)
+    for x in (base[1:].clone(), base[1:], torch.zeros_like(base[1:])):
+        for special in (None, float("inf"), float("nan")):
+            x = x.clone() if special is not None else x
+            if special is not None:
+                x[n // 2] = special
+            q, s = ext.quantize_fp8_tensor(x)
+            xf = x.float()
+            want_s = (xf.abs().amax() / 448.0).clamp_min(1e-8).reshape(1)
+            want = (xf / want_s).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+            assert torch.equal(s.view(torch.int32), want_s.view(torch.int32)) or (
+                s.isnan().item() and want_s.isnan().item())
+            a, b = q.float(), want.float()
+            assert torch.equal(a.isnan(), b.isnan())
+            assert torch.equal(a.nan_to_num(), b.nan_to_num())
+
+
+@pytest.mark.parametrize("B,H", [(1, 16), (8, 3), (16, 128), (33, 16), (70, 2)])
+def test_mla_products(B, H):
+    g = torch.Generator(device="cuda").manual_seed(B)
+    q = _rand(g, B, H, 192).bfloat16()[..., :128]
+    uk, uv = (_rand(g, H, 128, 512).bfloat16() for _ in range(2))
+    lat = _rand(g, B, H, 512).bfloat16()
+    torch.testing.assert_close(
+        ops.mla_absorb(q, uk).float(),
+        torch.einsum("bhd,hdr->bhr", q.float(), uk.float()), rtol=2 ** -8,
+        atol=128 ** 2 * 2 ** -24)
+    torch.testing.assert_close(
+        ops.mla_project_out(lat, uv).float(),
+        torch.einsum("bhr,hvr->bhv", lat.float(), uv.float()), rtol=2 ** -8,
+        atol=512 ** 2 * 2 ** -24)
+    # other widths: the torch products
+    torch.testing.assert_close(
+        ops.mla_absorb(q[..., :96], uk[:, :96]).float(),
+        torch.einsum("bhd,hdr->bhr", q[..., :96].float(), uk[:, :96].float()),
+        rtol=2 ** -8, atol=1e-2)
