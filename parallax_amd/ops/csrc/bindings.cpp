@@ -34,11 +34,11 @@ void launch_paged_attention_decode(void*, const void*, const void*, const void*,
                                    int, int, int64_t, float, int, float,
                                    const float*, int, int, float*, float*,
                                    hipStream_t, bool*);
-void launch_paged_decode_mfma(void*, const void*, const void*, const void*,
-                              const int*, const int*, int, int, int, int, int,
-                              int, int64_t, float, int, float, const float*,
-                              int, int, float*, float*, bool, float, float,
-                              hipStream_t, bool*);
+int paged_decode_runs(int, int, int, int, int);
+void launch_paged_decode(void*, const void*, const void*, const void*, const int*,
+                         const int*, int, int, int, int, int, int, int64_t, float,
+                         int, float, const float*, int, float*, float*, bool,
+                         float, float, hipStream_t, bool*);
 void launch_paged_attention_reduce(void*, const float*, const float*, int, int,
                                    int, int, const float*, hipStream_t);
 void launch_mla_paged_attention_decode(void*, const void*, const void*,
@@ -270,12 +270,33 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     sinks_ptr = sinks_f.data_ptr<float>();
   }
 
-  // Flash-decoding split, graph-capture friendly (num_parts depends only on
-  // max_seq_len and the batch bucket; partitions past a sequence's actual
-  // length exit immediately / are skipped by the reduce kernel). Partition
-  // size grows with B*Hk: when the batch alone fills the chip, bigger
-  // partitions cut empty-partition sweep + reduce cost and pick the KT=128
-  // tile path (A/B'd: profiles/README.md round 2).
+  static const bool use_valu = std::getenv("PARALLAX_ATTN_VALU") != nullptr;
+  auto opts = q.options().dtype(at::kFloat);
+  torch::Tensor tmp_acc, tmp_ml;
+  float *acc_ptr = nullptr, *ml_ptr = nullptr;
+  bool launched = false;
+  if (!use_valu || kv_fp8) {
+    if (B == 0) return;
+    // every part of a sequence is named by (run + sequence); see the kernel
+    const int runs = paged_decode_runs(B, Hk, D, (int)max_seq_len,
+                                       (int)sliding_window);
+    if (runs > 0) {
+      tmp_acc = torch::empty({(int64_t)runs + B, Hq, D}, opts);
+      tmp_ml = torch::empty({(int64_t)runs + B, Hq, 2}, opts);
+      acc_ptr = tmp_acc.data_ptr<float>();
+      ml_ptr = tmp_ml.data_ptr<float>();
+    }
+    launch_paged_decode(
+        out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+        block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, Hq, Hk, D,
+        BS, max_blocks, row_stride(q, "q"), (float)scale, (int)sliding_window,
+        (float)softcap, sinks_ptr, runs, acc_ptr, ml_ptr, kv_fp8, (float)k_scale,
+        (float)v_scale, cur_stream(), &launched);
+    TORCH_CHECK(launched, "no kernel instantiation for D=", D, " BS=", BS,
+                " G=", G);
+    return;
+  }
+  // fixed partitions of the context and a reduce kernel
   const int wg_base = B * Hk;
   int part_tokens = 256;
   if (wg_base >= 4096) part_tokens = 2048;
@@ -287,36 +308,21 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     part_tokens = (part_tokens + 127) / 128 * 128;  // chunk-aligned
     num_parts = (int)((max_seq_len + part_tokens - 1) / part_tokens);
   }
-  torch::Tensor tmp_acc, tmp_ml;
-  float *acc_ptr = nullptr, *ml_ptr = nullptr;
   if (num_parts > 1) {
-    auto opts = q.options().dtype(at::kFloat);
     tmp_acc = torch::empty({B, Hq, num_parts, D}, opts);
     tmp_ml = torch::empty({B, Hq, num_parts, 2}, opts);
     acc_ptr = tmp_acc.data_ptr<float>();
     ml_ptr = tmp_ml.data_ptr<float>();
   }
-  bool launched = false;
-  static const bool use_valu = std::getenv("PARALLAX_ATTN_VALU") != nullptr;
-  if (!use_valu || kv_fp8) {
-    launch_paged_decode_mfma(
-        out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-        block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, Hq, Hk, D,
-        BS, max_blocks, row_stride(q, "q"), (float)scale, (int)sliding_window,
-        (float)softcap, sinks_ptr, num_parts, part_tokens, acc_ptr, ml_ptr,
-        kv_fp8, (float)k_scale, (float)v_scale, cur_stream(), &launched);
-  }
-  if (!launched) {
-    launch_paged_attention_decode(
-        out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-        block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, Hq, Hk, D,
-        BS, max_blocks, row_stride(q, "q"), (float)scale, (int)sliding_window,
-        (float)softcap, sinks_ptr, num_parts, part_tokens, acc_ptr, ml_ptr,
-        cur_stream(), &launched);
-  }
+  launch_paged_attention_decode(
+      out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+      block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, Hq, Hk, D,
+      BS, max_blocks, row_stride(q, "q"), (float)scale, (int)sliding_window,
+      (float)softcap, sinks_ptr, num_parts, part_tokens, acc_ptr, ml_ptr,
+      cur_stream(), &launched);
   TORCH_CHECK(launched, "no kernel instantiation for D=", D, " BS=", BS,
               " G=", G);
-  if (num_parts > 1 && launched)
+  if (num_parts > 1)
     launch_paged_attention_reduce(out.data_ptr(), acc_ptr, ml_ptr, B, Hq, D,
                                   num_parts, sinks_ptr, cur_stream());
 }

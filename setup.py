@@ -28,6 +28,7 @@ sources = [
     os.path.join(CSRC, "elementwise.hip"),
     os.path.join(CSRC, "paged_attention.hip"),
     os.path.join(CSRC, "paged_attention_mfma.hip"),
+    os.path.join(CSRC, "paged_decode.hip"),
     os.path.join(CSRC, "mla_attention.hip"),
     os.path.join(CSRC, "mla_prefill.hip"),
     os.path.join(CSRC, "prefill_attention.hip"),

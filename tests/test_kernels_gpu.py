@@ -391,3 +391,44 @@ def test_sample_gumbel_kernel():
     c = ops.sample_tokens(torch.zeros(1, V, device="cuda"), [1.0], [1.0],
                           [-1], [0.0], generator=gen)
     assert len({int(a), int(b), int(c)}) > 1
+
+
+@pytest.mark.parametrize("D,BS,fp8,G,Hk", [
+    (128, 32, False, 4, 2), (128, 16, True, 1, 3), (64, 64, False, 7, 2),
+    (64, 16, True, 8, 2), (128, 64, False, 16, 1), (64, 32, True, 2, 8),
+])
+@pytest.mark.parametrize("lens,kw", [
+    ([1, 31, 32, 33, 64, 127, 128, 129, 255, 257, 512, 513, 1000], {}),
+    ([1025, 7, 3000, 128, 1, 2049, 64], {}),            # dealt to runs
+    ([1500] + [40, 0, 129] * 30, {"sliding_window": 1100}),
+    ([90, 300, 33, 1000], {"sliding_window": 77, "softcap": 20.0}),
+    ([5, 1900, 260, 31] * 24 + [1], {"sinks": True}),   # more than a wave's lanes
+])
+def test_paged_decode_units_runs_and_windows(D, BS, fp8, G, Hk, lens, kw):
+    """Lengths around the 32-token tiles and the units of 128 to 512, units dealt
+    to runs, windows that begin inside a tile; slots past a sequence's end hold
+    NaN. Weights and results are rounded to bf16 once each: an error of at most
+    2 * 2^-9 * max |v|, max |v| < 5.5 here."""
+    B, kw = len(lens), dict(kw)
+    kc, vc, bt = _make_paged_kv(B, Hk, D, BS, max(lens), seed=D + BS)
+    kc, vc = kc.clone(), vc.clone()
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+        kw.update(k_scale=0.75, v_scale=0.5)
+    full_k, full_v = kc.float(), vc.float()
+    for i, n in enumerate(lens):
+        if n % BS and not fp8:
+            page = int(bt[i, n // BS])
+            kc[page, :, n % BS:] = float("nan")
+            vc[page, :, :, n % BS:] = float("nan")
+    g = torch.Generator(device="cuda").manual_seed(B)
+    q = torch.randn(B, G * Hk, D, generator=g, device="cuda").bfloat16()
+    if kw.get("sinks"):
+        kw["sinks"] = torch.randn(G * Hk, generator=g, device="cuda")
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = ops.paged_attention_decode(q, kc, vc, bt, sl, D ** -0.5, **kw)
+    ks, vs = kw.pop("k_scale", 1.0), kw.pop("v_scale", 1.0)
+    some = [i for i in (set(range(13)) | {B - 2, B - 1}) if i < B and lens[i]]
+    want = ref.paged_attention_decode(
+        q[some].float(), full_k * ks, full_v * vs, bt[some], sl[some], D ** -0.5, **kw)
+    torch.testing.assert_close(out[some].float(), want.float(), atol=2.2e-2, rtol=0)
