@@ -380,8 +380,9 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
           }
       }
       mx = over_head(mx, [](float x, float y) { return fmaxf(x, y); });
-      // rescaled only when a maximum moved by more than 2^8
-      if (__any(mx > m + 8.f)) {
+      // rescaled when a maximum moved: its own weight is then 1, without rounding
+      // (only when it moved by 2^8: 5 to 10% more error)
+      if (__any(mx > m)) {
         const float m2 = fmaxf(m, mx);
         const float f = __builtin_amdgcn_exp2f(m - m2);
         m = m2;

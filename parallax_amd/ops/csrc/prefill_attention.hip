@@ -21,12 +21,11 @@
 // What bounds it: per tile and wave 1024 matrix-core cycles (D = 128), about
 // as many VALU cycles of softmax and as many LDS cycles for four waves; two
 // workgroups a CU overlap them. The accumulators are rescaled only when an
-// item's maximum moved by more than 2^8 (the weights are then at most 2^8 and
-// the sums fp32), the mask is applied only in tiles that the diagonal, the
+// item's maximum moved, the mask is applied only in tiles that the diagonal, the
 // window or the end of the sequence cuts.
 //
 // Measured (MI355X, bf16, 32 heads over 8 of 128, 8192 rows in two portions on
-// prefixes of up to 20,000): 3.37 ms = 907 TFLOP/s of what the mask leaves;
+// prefixes of up to 20,000): 3.59 ms = 851 TFLOP/s of what the mask leaves;
 // 16.6 ms with 32-row tiles of one head, P through LDS and six barriers a tile.
 
 #include "common.h"
@@ -339,7 +338,9 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[1][r]);
     mx = max_halves(mx) * c;
-    if (__any(mx > m + 8.f)) {
+    // rescaled when a maximum moved: its own weight is then 1, without rounding (only
+    // when it moved by 2^8: 2% more error)
+    if (__any(mx > m)) {
       const float m2 = fmaxf(m, mx);
       const float f = __builtin_amdgcn_exp2f(m - m2);
       m = m2;
