@@ -455,9 +455,9 @@ def gelu_and_mul(x: torch.Tensor) -> torch.Tensor:
 
 # -- dense linear (skinny-M fast path) ------------------------------------------
 
-# Rows of x up to which linear() and linear_fp8() try the weight-streaming kernel
-# (it has none above 32); 0 leaves every product to the library.
-SKINNY_GEMM_MAX_M = int(os.environ.get("PARALLAX_SKINNY_GEMM_MAX_M", "32"))
+# Rows of x up to which linear() and linear_fp8() try the weight-streaming kernels
+# (there are none above 128); 0 leaves every product to the library.
+SKINNY_GEMM_MAX_M = int(os.environ.get("PARALLAX_SKINNY_GEMM_MAX_M", "128"))
 LT_GEMM = os.environ.get("PARALLAX_LT_GEMM", "1") != "0"
 _LT_REFUSED = set()  # (N, K) shapes hipBLASLt had no algorithm for
 
@@ -465,7 +465,7 @@ _LT_REFUSED = set()  # (N, K) shapes hipBLASLt had no algorithm for
 def linear(
     x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None
 ) -> torch.Tensor:
-    """F.linear: a weight-streaming kernel for few rows (skinny_gemm.hip has the
+    """F.linear: weight-streaming kernels for few rows (skinny_gemm.hip has the
     sizes, with both sides measured), tuned hipBLASLt for the rest."""
     if (
         x.is_cuda
@@ -545,7 +545,7 @@ def fused_moe_forward(
 def linear_fp8(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor,
                bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """W8A8 dense GEMM: x quantized per-tensor on the fly (two launches, the
-    scale stays on the device), then the weight-streaming kernel for few rows
+    scale stays on the device), then the weight-streaming kernels for few rows
     or hipBLASLt fp8. CPU fallback dequantizes (plumbing tests)."""
     if not x.is_cuda:
         w = (w_q.float() * w_scale.float()).to(torch.float32)

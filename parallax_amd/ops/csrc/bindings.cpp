@@ -88,6 +88,10 @@ void launch_sample_gumbel(int64_t*, const float*, const float*,
 void launch_skinny_gemm(void*, const void*, const void*, const void*,
                         const float*, const float*, bool, int, int, int, int64_t,
                         int64_t, int, int64_t, int64_t, hipStream_t, bool*);
+int skinny_shared(int, int, int);
+void launch_skinny_split(void*, float*, int, const void*, const void*, const void*,
+                         const float*, const float*, bool, int, int, int, int64_t,
+                         int64_t, hipStream_t);
 void launch_mla_absorb(void*, const void*, const void*, int, int, int, int64_t,
                        int64_t, hipStream_t);
 int quantize_fp8_tensor_parts(int64_t);
@@ -727,13 +731,25 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
   if ((uintptr_t)x.data_ptr() % 16 || (uintptr_t)w.data_ptr() % 16 ||
       x.stride(0) * es % 16 || (uintptr_t)c.data_ptr() % 8 || c.stride(0) % 4)
     return false;
+  const int M = x.size(0), N = w.size(0), row_bytes = x.size(1) * es;
+  const void* b = bias.numel() ? bias.data_ptr() : nullptr;
+  const float* xs = fp8 ? x_scale.data_ptr<float>() : nullptr;
+  const float* ws = fp8 ? w_scale.data_ptr<float>() : nullptr;
+  const int splits = skinny_shared(M, N, row_bytes);
+  if (splits < 0) return false;
+  if (splits > 0) {
+    torch::Tensor part;
+    if (splits > 1)
+      part = torch::empty({splits, M, N}, x.options().dtype(at::kFloat));
+    launch_skinny_split(c.data_ptr(), splits > 1 ? part.data_ptr<float>() : nullptr,
+                        splits, x.data_ptr(), w.data_ptr(), b, xs, ws, fp8, M, N,
+                        row_bytes, x.stride(0) * es, c.stride(0), cur_stream());
+    return true;
+  }
   bool launched = false;
-  launch_skinny_gemm(c.data_ptr(), x.data_ptr(), w.data_ptr(),
-                     bias.numel() ? bias.data_ptr() : nullptr,
-                     fp8 ? x_scale.data_ptr<float>() : nullptr,
-                     fp8 ? w_scale.data_ptr<float>() : nullptr, fp8, x.size(0),
-                     w.size(0), x.size(1) * es, x.stride(0) * es, c.stride(0), 1,
-                     0, 0, cur_stream(), &launched);
+  launch_skinny_gemm(c.data_ptr(), x.data_ptr(), w.data_ptr(), b, xs, ws, fp8, M, N,
+                     row_bytes, x.stride(0) * es, c.stride(0), 1, 0, 0,
+                     cur_stream(), &launched);
   return launched;
 }
 

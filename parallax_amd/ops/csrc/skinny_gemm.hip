@@ -22,7 +22,8 @@
 
 typedef float f32x16v __attribute__((ext_vector_type(16)));
 typedef short s16x4v __attribute__((ext_vector_type(4)));
-typedef long longx2n __attribute__((ext_vector_type(2)));
+typedef int i32x4n __attribute__((ext_vector_type(4)));
+typedef int i32x8n __attribute__((ext_vector_type(8)));
 
 namespace {
 
@@ -30,6 +31,13 @@ DEVINL void copy16_to_lds(const void* src, void* dst) {
   __builtin_amdgcn_global_load_lds(
       (const __attribute__((address_space(1))) void*)src,
       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// 32 fp8 values of an operand; their order in K is that of the other operand's
+DEVINL i32x8n join(bf16x8v lo, bf16x8v hi) {
+  return __builtin_shufflevector(__builtin_bit_cast(i32x4n, lo),
+                                 __builtin_bit_cast(i32x4n, hi), 0, 1, 2, 3, 4, 5,
+                                 6, 7);
 }
 
 template <int N>
@@ -171,28 +179,26 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
     wait_copies<(STAGES - 2) * NI>();
     // into the place read in the turn before: its operands are in registers
     issue(i + STAGES - 1, next);
+    bf16x8v a[2][NT / 16], b[2][MT];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      bf16x8v a[NT / 16], b[MT];
-      read_operands((a_at + place * RING) ^ (ks * 64), (b_at + place * RING) ^ (ks * 64),
-                    a, b);
+    for (int ks = 0; ks < 2; ++ks)
+      read_operands((a_at + place * RING) ^ (ks * 64),
+                    (b_at + place * RING) ^ (ks * 64), a[ks], b[ks]);
 #pragma unroll
-      for (int t = 0; t < NT / 16; ++t)
+    for (int t = 0; t < NT / 16; ++t)
 #pragma unroll
-        for (int u = 0; u < MT; ++u) {
-          if constexpr (FP8) {
-            const auto p = __builtin_bit_cast(longx2n, a[t]);
-            const auto q = __builtin_bit_cast(longx2n, b[u]);
-            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-                p[0], q[0], acc[t][u], 0, 0, 0);
-            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-                p[1], q[1], acc[t][u], 0, 0, 0);
-          } else {
+      for (int u = 0; u < MT; ++u) {
+        if constexpr (FP8) {
+          acc[t][u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+              join(a[0][t], a[1][t]), join(b[0][u], b[1][u]), acc[t][u], 0, 0, 0,
+              0x7f7f7f7f, 0, 0x7f7f7f7f);
+        } else {
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
             acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                a[t], b[u], acc[t][u], 0, 0, 0);
-          }
+                a[ks][t], b[ks][u], acc[t][u], 0, 0, 0);
         }
-    }
+      }
     place = place + 1 == STAGES ? 0 : place + 1;
     next = next + 1 == STAGES ? 0 : next + 1;
   }
@@ -227,6 +233,225 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
   }
 }
 
+// ---- to 128 rows -------------------------------------------------------------------------
+// X is as large as W's part: the waves of a workgroup share its tile and take 32
+// rows of W each; one barrier a stage. Where W has few rows, K is split over
+// workgroups, whose fp32 parts a second kernel adds up. W's stream bounds it, 28672
+// x 4096 at 96 rows in 47 us or 5.0 TB/s, and for small weights the second launch.
+
+// Stage operands: 16 bytes of the wave's 32 rows of W, and of 32 XT rows of X
+template <int XT>
+DEVINL void read_stage(bf16x8v& a, bf16x8v (&b)[XT], uint32_t at, uint32_t x_at) {
+  static_assert(XT >= 1 && XT <= 4, "");
+  if constexpr (XT == 1)
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(a), "=&v"(b[0]) : "v"(at), "v"(x_at) : "memory");
+  if constexpr (XT == 2)
+    asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %4\n\t"
+                 "ds_read_b128 %2, %4 offset:4096\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a), "=&v"(b[0]), "=&v"(b[1])
+                 : "v"(at), "v"(x_at) : "memory");
+  if constexpr (XT == 3)
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+                 "ds_read_b128 %2, %5 offset:4096\n\t"
+                 "ds_read_b128 %3, %5 offset:8192\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a), "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2])
+                 : "v"(at), "v"(x_at) : "memory");
+  if constexpr (XT == 4)
+    asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %6\n\t"
+                 "ds_read_b128 %2, %6 offset:4096\n\t"
+                 "ds_read_b128 %3, %6 offset:8192\n\t"
+                 "ds_read_b128 %4, %6 offset:12288\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a), "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
+                 : "v"(at), "v"(x_at) : "memory");
+}
+
+template <bool FP8, int XT, int W, int STAGES>
+__global__ __launch_bounds__(W * 64) void skinny_split_kernel(
+    uint16_t* __restrict__ c, float* __restrict__ part,  // [splits, M, N] or null
+    const uint8_t* __restrict__ x, const uint8_t* __restrict__ w,
+    const uint16_t* __restrict__ bias, const float* __restrict__ x_scale,
+    const float* __restrict__ w_scale, const int M, const int N,
+    const int row_bytes, const int64_t x_stride, const int64_t c_stride) {
+  constexpr int NT = W * 32;
+  constexpr int ROWS = NT + XT * 32;
+  // copies a wave and stage: its rows of W, some of X
+  constexpr int NX = (XT * 4 + W - 1) / W;
+  constexpr int NI = 4 + NX;
+  constexpr int RING = ROWS * 128;
+  __shared__ __attribute__((aligned(128))) uint8_t S[STAGES * RING];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, l31 = lane & 31;
+  const int n0 = blockIdx.x * NT;
+
+  // this workgroup's columns of 128 bytes
+  const int cols = row_bytes / 128;
+  const int c0 = (int)((int64_t)cols * blockIdx.y / gridDim.y);
+  const int mine = (int)((int64_t)cols * (blockIdx.y + 1) / gridDim.y) - c0;
+  const uint8_t* wb = w + (size_t)n0 * row_bytes + (size_t)c0 * 128;
+  const uint8_t* xb = x + (size_t)c0 * 128;
+  uint32_t at[NI];
+  // eight rows of X: where the waves do not divide them, the last are copied twice
+  auto x_rows = [&](int i) { return min(wid + W * i, XT * 4 - 1) * 8; };
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = (i < 4 ? wid * 32 + i * 8 : x_rows(i - 4)) + (lane >> 3);
+    const int j = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    at[i] = i < 4 ? (uint32_t)min(r, N - 1 - n0) * row_bytes + j
+                  : (uint32_t)min(r, M - 1) * (uint32_t)x_stride + j;
+  }
+  // one head start a workgroup, see skinny_gemm_kernel
+  const int rot = (int)((blockIdx.x >> 3) * 3 % mine);
+  auto issue = [&](int i, int place) __attribute__((always_inline)) {
+    int t = min(i, mine - 1) + rot;
+    if (t >= mine) t -= mine;
+    uint8_t* dst = S + place * RING;
+#pragma unroll
+    for (int q = 0; q < NI; ++q)
+      copy16_to_lds((q < 4 ? wb : xb) + t * 128 + at[q],
+                    dst + (q < 4 ? wid * 32 + q * 8 : NT + x_rows(q - 4)) * 128);
+  };
+  f32x16v acc[XT] = {};
+  const uint32_t base =
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)S;
+  const uint32_t j0 = (half ^ ((l31 >> 1) & 7)) * 16;
+  const uint32_t a_at = base + (wid * 32 + l31) * 128 + j0;
+  const uint32_t b_at = base + (NT + l31) * 128 + j0;
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i) issue(i, i);
+  int place = 0, next = STAGES - 1;
+  for (int i = 0; i < mine; ++i) {
+    wait_copies<(STAGES - 2) * NI>();
+    // every wave's copies have landed, and every wave is done with the place
+    // that is filled next: its operands are in registers
+    __builtin_amdgcn_s_barrier();
+    issue(i + STAGES - 1, next);
+#pragma unroll
+    for (int ks = 0; ks < 4; ks += 2) {
+      bf16x8v a[2], b[2][XT];
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        read_stage<XT>(a[k], b[k], (a_at + place * RING) ^ ((ks + k) * 32),
+                       (b_at + place * RING) ^ ((ks + k) * 32));
+#pragma unroll
+      for (int t = 0; t < XT; ++t) {
+        if constexpr (FP8) {
+          acc[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+              join(a[0], a[1]), join(b[0][t], b[1][t]), acc[t], 0, 0, 0,
+              0x7f7f7f7f, 0, 0x7f7f7f7f);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], b[k][t], acc[t],
+                                                             0, 0, 0);
+        }
+      }
+    }
+    place = place + 1 == STAGES ? 0 : place + 1;
+    next = next + 1 == STAGES ? 0 : next + 1;
+  }
+  wait_copies<0>();
+  const float scale = FP8 ? x_scale[0] * w_scale[0] : 1.f;
+#pragma unroll
+  for (int t = 0; t < XT; ++t) {
+    const int m = t * 32 + l31;
+    if (m >= M) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = n0 + wid * 32 + 8 * q + 4 * half;
+      if (n >= N) continue;
+      f32x4v v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = acc[t][4 * q + r];
+      if (FP8) v *= scale;
+      if (part != nullptr) {
+        *reinterpret_cast<f32x4v*>(part + ((size_t)blockIdx.y * M + m) * N + n) = v;
+        continue;
+      }
+      uint16_t o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[r] = f32_to_bf16_bits(
+            v[r] + (bias != nullptr ? bf16_bits_to_f32(bias[n + r]) : 0.f));
+      *reinterpret_cast<uint2*>(c + (size_t)m * c_stride + n) =
+          make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void skinny_sum_kernel(
+    uint16_t* __restrict__ c, const float* __restrict__ part,
+    const uint16_t* __restrict__ bias, const int splits, const int M, const int N,
+    const int64_t c_stride) {
+  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const int64_t all = (int64_t)M * N;
+  if (e >= all) return;
+  f32x4v s = {};
+#pragma unroll 8
+  for (int k = 0; k < splits; ++k)
+    s += *reinterpret_cast<const f32x4v*>(part + k * all + e);
+  const int m = e / N, n = e % N;
+  uint16_t o[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    o[r] = f32_to_bf16_bits(
+        s[r] + (bias != nullptr ? bf16_bits_to_f32(bias[n + r]) : 0.f));
+  *reinterpret_cast<uint2*>(c + (size_t)m * c_stride + n) =
+      make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
+}
+
+// Waves a workgroup (32 rows of W each) and workgroups that share K: what keeps
+// most of the 256 CUs busy to the end. us of 40 rows with 3 / 4 / 5 waves: 28672 x
+// 4096 57 / 44 / 46, 24576 x 1536 17 / 19 / 20, 36864 x 7168 in fp8 58 / 67 / 51.
+static float busy(int tiles) {
+  return tiles < 256 ? tiles * (256 / tiles) / 256.f
+                     : tiles / (256.f * ceil_div(tiles, 256));
+}
+static int skinny_waves(int N) {
+  int best = 4;
+  for (int w : {3, 5})
+    if (busy(ceil_div(N, w * 32)) > busy(ceil_div(N, best * 32))) best = w;
+  return best;
+}
+static int skinny_splits(int N, int row_bytes) {
+  const int tiles = ceil_div(N, skinny_waves(N) * 32);
+  return max(1, min(256 / tiles, min(32, row_bytes / 512)));
+}
+
+extern "C" void launch_skinny_split(
+    void* c, float* part, int splits, const void* x, const void* w,
+    const void* bias, const float* x_scale, const float* w_scale, bool fp8, int M,
+    int N, int row_bytes, int64_t x_stride, int64_t c_stride, hipStream_t stream) {
+  const int waves = skinny_waves(N);
+  auto run = [&](auto kernel) {
+    kernel<<<dim3(ceil_div(N, waves * 32), splits), waves * 64, 0, stream>>>(
+        (uint16_t*)c, part, (const uint8_t*)x, (const uint8_t*)w,
+        (const uint16_t*)bias, x_scale, w_scale, M, N, row_bytes, x_stride,
+        c_stride);
+  };
+  auto pick = [&](auto f, auto wv) {
+    constexpr bool F = decltype(f)::value;
+    constexpr int W = decltype(wv)::value;
+    if (M <= 32) run(skinny_split_kernel<F, 1, W, 3>);
+    else if (M <= 64) run(skinny_split_kernel<F, 2, W, 3>);
+    else if (M <= 96) run(skinny_split_kernel<F, 3, W, W < 5 ? 4 : 3>);
+    else run(skinny_split_kernel<F, 4, W, 3>);
+  };
+  auto by = [&](auto f) {
+    if (waves == 3) pick(f, std::integral_constant<int, 3>{});
+    else if (waves == 4) pick(f, std::integral_constant<int, 4>{});
+    else pick(f, std::integral_constant<int, 5>{});
+  };
+  if (fp8) by(std::true_type{});
+  else by(std::false_type{});
+  if (splits > 1)
+    skinny_sum_kernel<<<ceil_div((int64_t)M * N, 1024), 256, 0, stream>>>(
+        (uint16_t*)c, part, (const uint16_t*)bias, splits, M, N, c_stride);
+}
+
 // Tiles, by rows of X and by how many tiles W gives. us of bf16 products, W from
 // memory (N x K; the library's tuned pick last):
 //   up to 8 rows, NT 16 of 4 waves, 5 stages / 3 stages (four workgroups a CU
@@ -236,9 +461,7 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
 //   that still gives 150 workgroups: 6144 x 4096 14.5 / 12.1 / 16.6 (15.7),
 //   28672 x 4096 48 / 45 / 42 (54), 4096 x 14336 26 / 32 / 49 (26)
 //   17 to 32, the same: 28672 x 4096 60 / 47 / 43 (56), 6144 x 4096 18 / 13.9 /
-//   19.5 (15.2), 4096 x 4096 10.7 / 13.4 / 19 (11.8); below 4800 rows of W and
-//   above 10 KB a row the library's split of K is better: 1536 x 7168 15 (12)
-// More rows of X than 32 need W's tiles shared: the library.
+//   19.5 (15.2), 4096 x 4096 10.7 / 13.4 / 19 (11.8)
 static int skinny_tile(int M, int64_t N, int row_bytes) {
   if (M <= 8) return 16;
   if (N >= 9600) return 64;
@@ -246,8 +469,32 @@ static int skinny_tile(int M, int64_t N, int row_bytes) {
   return M <= 16 || row_bytes <= 10240 ? 16 : 0;
 }
 
+// Workgroups that share K for M rows, 0: skinny_gemm_kernel (to 32 rows), -1: the
+// library. us of W alone / shared / the library: from 17 rows on where W is large
+// or long, 32 rows: 24576 x 1536 19.7 / 17.2 / 21, 4096 x 14336 34 / 25 / 36, 6144 x
+// 4096 13.8 / 14.8 / 16; from 9 rows on where the last tiles of 64 rows of W would
+// find the CUs empty, 36864 x 7168 in fp8, 12 rows: 64 / 51 / 50. From 33 rows on:
+// 28672 x 4096 at 96 rows - / 47 / 58, 4096 x 14336 - / 31 / 51; short K split, or
+// small weights under many rows, cost more in parts than they gain: 9728 x 896 at 96
+// rows 16 / 12, 576 x 7168 at 40 10.8 / 10.9, at 96 14 / 11. Above 128 rows: the
+// library.
+extern "C" int skinny_shared(int M, int N, int row_bytes) {
+  if (M > 128 || row_bytes % 128 || N % 4) return -1;
+  const int splits = skinny_splits(N, row_bytes);
+  const int64_t bytes = (int64_t)N * row_bytes;
+  if (M > 32)
+    return (splits == 1 || row_bytes >= 4096) && (M <= 64 || bytes >= 1 << 24)
+               ? splits : -1;
+  if (M <= 8) return 0;
+  const int nt = skinny_tile(M, N, row_bytes);
+  const int tiles = ceil_div(N, 64);
+  const bool ragged =
+      nt == 64 && tiles > 512 && tiles < 384 * ceil_div(tiles, 512);
+  return ragged || (M > 16 && (nt == 0 || bytes >= 1 << 26)) ? splits : 0;
+}
+
 // batch products of the same shape: x, w and c advance by x_batch bytes, N rows
-// and c_batch elements. A batch takes any number of rows of X, 32 at a time.
+// and c_batch elements. Any number of rows of X, 32 at a time.
 extern "C" void launch_skinny_gemm(
     void* c, const void* x, const void* w, const void* bias,
     const float* x_scale, const float* w_scale, bool fp8, int M, int N,
@@ -255,7 +502,7 @@ extern "C" void launch_skinny_gemm(
     int64_t x_batch, int64_t c_batch, hipStream_t stream, bool* launched) {
   *launched = false;
   const int nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes);
-  if (nt == 0 || (M > 32 && batch == 1) || row_bytes % 128 || N % 4) return;
+  if (nt == 0 || row_bytes % 128 || N % 4) return;
   *launched = true;
   auto run = [&](auto kernel, int xr, int waves) {
     kernel<<<dim3(ceil_div(N, nt), batch, ceil_div(M, xr)), waves * 64, 0,

@@ -13,12 +13,18 @@ def _rand(g, *s):
     return torch.randn(*s, generator=g, device="cuda")
 
 
-@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
-@pytest.mark.parametrize("N,K", [
-    (4, 64),        # one column of 128 bytes: waves without one
-    (900, 896),     # a tile cut by the last row
-    (4804, 2176),   # 32 rows a tile, deep rings
-    (9604, 320),    # 64 rows a tile
+@pytest.mark.parametrize("M,N,K", [
+    (M, N, K) for M in (1, 8, 9, 16, 17, 32) for N, K in (
+        (4, 64),        # one column of 128 bytes: waves without one
+        (900, 896),     # a tile cut by the last row
+        (4804, 2176),   # 32 rows a tile, deep rings
+        (9604, 320),    # 64 rows a tile
+    )
+] + [
+    (33, 576, 2112), (64, 100, 2048), (64, 5000, 3072),  # K shared, odd parts
+    (20, 1536, 7168), (32, 24576, 1408),                 # the same, fewer rows
+    (65, 4100, 4096), (96, 28672, 320), (128, 36864, 256),  # 3 to 5 waves
+    (127, 8192, 2112),
 ])
 def test_linear_few_rows(M, N, K):
     """fp32 sums of exact products: 2^-9 of the result for its rounding, and
@@ -40,7 +46,8 @@ def test_linear_few_rows(M, N, K):
 def test_linear_without_a_kernel():
     """Odd widths and misaligned rows take the library and agree."""
     g = torch.Generator(device="cuda").manual_seed(0)
-    for M, N, K in ((5, 8, 72), (3, 6, 64), (33, 64, 64), (20, 576, 7168)):
+    for M, N, K in ((5, 8, 72), (3, 6, 64), (33, 64, 64), (96, 576, 7168),
+                    (129, 4096, 512)):
         x, w = _rand(g, M, K).bfloat16(), _rand(g, N, K).bfloat16()
         torch.testing.assert_close(
             ops.linear(x, w).float(), x.float() @ w.float().t(), rtol=2 ** -8,
@@ -52,7 +59,9 @@ def test_linear_without_a_kernel():
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 64, 128), (7, 4800, 5120), (16, 64, 256),
-                                   (30, 9600, 384), (40, 256, 512)])
+                                   (30, 9600, 384), (40, 256, 512),
+                                   (12, 36864, 256), (50, 1000, 4224),
+                                   (96, 36864, 512), (128, 8192, 4096)])
 def test_linear_fp8_rows(M, N, K):
     g = torch.Generator(device="cuda").manual_seed(M)
     x = _rand(g, M, K).bfloat16()
