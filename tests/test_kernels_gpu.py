@@ -432,3 +432,47 @@ def test_paged_decode_units_runs_and_windows(D, BS, fp8, G, Hk, lens, kw):
     want = ref.paged_attention_decode(
         q[some].float(), full_k * ks, full_v * vs, bt[some], sl[some], D ** -0.5, **kw)
     torch.testing.assert_close(out[some].float(), want.float(), atol=2.2e-2, rtol=0)
+
+
+@pytest.mark.parametrize("neox", [True, False])
+@pytest.mark.parametrize("T,Hq,Hk,D,rot,BS,fp8,start", [
+    (1, 14, 2, 64, 64, 32, False, None),    # None: scattered slots, some absent
+    (97, 32, 8, 128, 128, 16, True, None),
+    (5, 3, 1, 128, 32, 64, False, None),    # dimensions passed through
+    (1031, 4, 2, 128, 64, 32, False, 0),    # slots in a row: 8 at a time,
+    (1024, 2, 3, 64, 64, 16, True, 4),      # from an offset of a page,
+    (1100, 2, 1, 128, 128, 64, False, 6),
+    (1030, 2, 2, 64, 32, 32, False, 3),     # an odd one
+    (1024, 2, 2, 64, 64, 32, True, None),
+    (1300, 2, 5, 64, 64, 16, False, -1),    # short runs with gaps
+])
+def test_rope_and_cache_pieces(T, Hq, Hk, D, rot, BS, fp8, start, neox):
+    """The same bytes as value by value, which rows that are not 16-byte aligned
+    still go."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    W = (Hq + 2 * Hk) * D
+    x = torch.randn(T, W, generator=g, device="cuda").bfloat16()
+    odd = torch.empty(T, W + 4, dtype=torch.bfloat16, device="cuda")[:, :W].copy_(x)
+    NB = (T + BS) // BS + 2
+    cs = torch.randn(4 * T + 8, rot, generator=g, device="cuda")
+    pos = torch.randint(0, 4 * T + 8, (T,), generator=g, device="cuda").int()
+    if start is None:
+        slots = torch.randperm(NB * BS, generator=g, device="cuda")[:T]
+        slots[T // 3 :: 7] = -1
+    elif start < 0:
+        i = torch.arange(T, device="cuda")
+        part = torch.randperm(T // 21 + 1, generator=g, device="cuda")
+        slots = part[i // 21] * 21 + i % 21
+        slots[5::100] = -1
+    else:
+        slots = torch.arange(T, device="cuda") + start
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    got = []
+    for buf in (x, odd):
+        q, k, v = (p.view(T, -1, D) for p in buf.split([Hq * D, Hk * D, Hk * D], 1))
+        kc = torch.zeros(NB, Hk, BS, D, device="cuda").to(dt)
+        vc = torch.zeros(NB, Hk, D, BS, device="cuda").to(dt)
+        ops.rope_and_cache(q, k, v, kc, vc, pos, cs, slots, neox, 0.5, 2.0)
+        got.append([t.contiguous().view(torch.uint8) for t in (q, kc, vc)])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
