@@ -154,7 +154,7 @@ class LlamaMLP(nn.Module):
         self.down_proj = RowParallelLinear(inter, cfg.hidden_size, bias=cfg.mlp_bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down_proj(ops.silu_and_mul(self.gate_up_proj(x)))
+        return self.down_proj(self.gate_up_proj.silu_and_mul(x))
 
 
 class LlamaDecoderLayer(nn.Module):

@@ -462,28 +462,39 @@ LT_GEMM = os.environ.get("PARALLAX_LT_GEMM", "1") != "0"
 _LT_REFUSED = set()  # (N, K) shapes hipBLASLt had no algorithm for
 
 
+def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
+    """x . weight^T (+ bias) by the kernels for few rows (with the scales: of fp8
+    values; gated: silu of the first half of the columns times the second), None
+    where they have none for it."""
+    fp8 = x_scale is not None
+    if not (
+        x.dim() == 2
+        and (fp8 or x.dtype == weight.dtype == torch.bfloat16)
+        and 0 < x.shape[0] <= SKINNY_GEMM_MAX_M
+        and weight.is_contiguous()
+        and x.stride(1) == 1
+        and (bias is None or bias.dtype == torch.bfloat16)
+    ):
+        return None
+    ext = _require_ext("skinny_gemm")
+    out = torch.empty(
+        x.shape[0], weight.shape[0] // (2 if gated else 1), dtype=torch.bfloat16,
+        device=x.device,
+    )
+    none = out.new_empty(0)
+    done = ext.skinny_gemm(out, x, weight, none if bias is None else bias,
+                           x_scale if fp8 else none, w_scale if fp8 else none, gated)
+    return out if done else None
+
+
 def linear(
     x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None
 ) -> torch.Tensor:
     """F.linear: weight-streaming kernels for few rows (skinny_gemm.hip has the
     sizes, with both sides measured), tuned hipBLASLt for the rest."""
-    if (
-        x.is_cuda
-        and x.dim() == 2
-        and x.dtype == torch.bfloat16
-        and 0 < x.shape[0] <= SKINNY_GEMM_MAX_M
-        and weight.dtype == torch.bfloat16
-        and weight.is_contiguous()
-        and x.stride(1) == 1
-        and (bias is None or bias.dtype == torch.bfloat16)
-    ):
-        ext = _require_ext("skinny_gemm")
-        out = torch.empty(
-            x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device
-        )
-        none = x.new_empty(0)
-        if ext.skinny_gemm(out, x, weight, none if bias is None else bias,
-                           none, none):
+    if x.is_cuda:
+        out = _few_rows(x, weight, bias)
+        if out is not None:
             return out
     if (
         LT_GEMM
@@ -552,20 +563,24 @@ def linear_fp8(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor,
         y = torch.nn.functional.linear(x.float(), w).to(x.dtype)
         return y if bias is None else y + bias
     ext = _require_ext("lt_linear_fp8")
-    M, _ = x.shape
+    _, _ = x.shape
     xq, xs = ext.quantize_fp8_tensor(
         (x if x.dtype == torch.bfloat16 else x.float()).contiguous())
-    if 0 < M <= SKINNY_GEMM_MAX_M and (
-        bias is None or bias.dtype == torch.bfloat16
-    ):
-        out = torch.empty(
-            M, w_q.shape[0], dtype=torch.bfloat16, device=x.device
-        )
-        if ext.skinny_gemm(out, xq, w_q, xs.new_empty(0, dtype=torch.bfloat16)
-                           if bias is None else bias, xs, w_scale):
-            return out
+    out = _few_rows(xq, w_q, bias, xs, w_scale)
+    if out is not None:
+        return out
     y = ext.lt_linear_fp8(xq, w_q, xs, w_scale)
     return y if bias is None else y + bias
+
+
+def linear_silu_and_mul(
+    x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None
+) -> torch.Tensor:
+    """silu_and_mul(linear(x, weight, bias)), in the product's own epilogue for
+    few rows: a launch of 3.5 us less. (Not of fp8: 40 rows of 36864 x 7168
+    take 5 us more that way, two streams of half as many rows each.)"""
+    out = _few_rows(x, weight, bias, gated=True) if x.is_cuda else None
+    return silu_and_mul(linear(x, weight, bias)) if out is None else out
 
 
 def mla_absorb(q_nope: torch.Tensor, w_uk: torch.Tensor) -> torch.Tensor:

@@ -87,11 +87,11 @@ void launch_sample_gumbel(int64_t*, const float*, const float*,
                           const uint8_t*, uint64_t, int, int, hipStream_t);
 void launch_skinny_gemm(void*, const void*, const void*, const void*,
                         const float*, const float*, bool, int, int, int, int64_t,
-                        int64_t, int, int64_t, int64_t, hipStream_t, bool*);
+                        int64_t, int, int64_t, int64_t, bool, hipStream_t, bool*);
 int skinny_shared(int, int, int);
 void launch_skinny_split(void*, float*, int, const void*, const void*, const void*,
                          const float*, const float*, bool, int, int, int, int64_t,
-                         int64_t, hipStream_t);
+                         int64_t, bool, hipStream_t);
 void launch_mla_absorb(void*, const void*, const void*, int, int, int, int64_t,
                        int64_t, hipStream_t);
 int quantize_fp8_tensor_parts(int64_t);
@@ -702,16 +702,17 @@ torch::Tensor sample_gumbel(torch::Tensor logits, torch::Tensor inv_temp,
   return out;
 }
 
-// c = x . w^T (+ bias): bf16, or fp8 with the two scales given. False where there
-// is no kernel.
+// c = x . w^T (+ bias): bf16, or fp8 with the two scales given; gated: c = silu(first
+// half of the columns) * second half. False where there is no kernel.
 bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
-                 torch::Tensor bias, torch::Tensor x_scale,
-                 torch::Tensor w_scale) {
+                 torch::Tensor bias, torch::Tensor x_scale, torch::Tensor w_scale,
+                 bool gated) {
   CHECK_GPU(x);
   const bool fp8 = x_scale.numel() > 0;
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) &&
               x.stride(1) == 1 && c.dim() == 2 && c.stride(1) == 1 &&
-              c.size(0) == x.size(0) && c.size(1) == w.size(0));
+              c.size(0) == x.size(0) &&
+              c.size(1) * (gated ? 2 : 1) == w.size(0));
   CHECK_CONTIG(w);
   CHECK_BF16(c);
   if (fp8) {
@@ -735,6 +736,8 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
   const void* b = bias.numel() ? bias.data_ptr() : nullptr;
   const float* xs = fp8 ? x_scale.data_ptr<float>() : nullptr;
   const float* ws = fp8 ? w_scale.data_ptr<float>() : nullptr;
+  // gated: halves as silu_and_mul takes them, offsets of 32 bits from row 0 on
+  if (gated && (N % 16 || (int64_t)N * row_bytes > UINT32_MAX)) return false;
   const int splits = skinny_shared(M, N, row_bytes);
   if (splits < 0) return false;
   if (splits > 0) {
@@ -743,12 +746,13 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
       part = torch::empty({splits, M, N}, x.options().dtype(at::kFloat));
     launch_skinny_split(c.data_ptr(), splits > 1 ? part.data_ptr<float>() : nullptr,
                         splits, x.data_ptr(), w.data_ptr(), b, xs, ws, fp8, M, N,
-                        row_bytes, x.stride(0) * es, c.stride(0), cur_stream());
+                        row_bytes, x.stride(0) * es, c.stride(0), gated,
+                        cur_stream());
     return true;
   }
   bool launched = false;
   launch_skinny_gemm(c.data_ptr(), x.data_ptr(), w.data_ptr(), b, xs, ws, fp8, M, N,
-                     row_bytes, x.stride(0) * es, c.stride(0), 1, 0, 0,
+                     row_bytes, x.stride(0) * es, c.stride(0), 1, 0, 0, gated,
                      cur_stream(), &launched);
   return launched;
 }
@@ -805,7 +809,8 @@ bool mla_project(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
   bool launched = false;
   launch_skinny_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), nullptr, nullptr,
                      nullptr, false, B, N, K * 2, x.stride(0) * 2, out.stride(0),
-                     H, x.stride(1) * 2, out.stride(1), cur_stream(), &launched);
+                     H, x.stride(1) * 2, out.stride(1), false, cur_stream(),
+                     &launched);
   return launched;
 }
 

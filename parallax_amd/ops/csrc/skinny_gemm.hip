@@ -112,6 +112,18 @@ DEVINL void read_operands(const uint32_t at, const uint32_t x_at, bf16x8v (&a)[A
 
 }  // namespace
 
+// Gated: W is [gate rows | up rows], N of both together; tiles take as many of
+// each, and the result is silu(gate) * up of the rounded products, [M, N / 2].
+DEVINL uint16_t silu_mul(float g, float u) {
+  g = bf16_bits_to_f32(f32_to_bf16_bits(g));
+  u = bf16_bits_to_f32(f32_to_bf16_bits(u));
+  return f32_to_bf16_bits(g / (1.f + __expf(-g)) * u);
+}
+
+DEVINL float biased(float v, const uint16_t* bias, int n) {
+  return bias != nullptr ? v + bf16_bits_to_f32(bias[n]) : v;
+}
+
 // XR: rows of X staged, a multiple of 8 that holds M.
 template <bool FP8, int NT, int XR, int WAVES, int STAGES>
 __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
@@ -121,7 +133,8 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
     const uint16_t* __restrict__ bias, // [N] or null
     const float* __restrict__ x_scale, const float* __restrict__ w_scale,
     const int M_all, const int N, const int row_bytes, const int64_t x_stride,
-    const int64_t c_stride, const int64_t x_batch, const int64_t c_batch) {
+    const int64_t c_stride, const int64_t x_batch, const int64_t c_batch,
+    const bool gated) {
   constexpr int ROWS = NT + XR;
   constexpr int NI = ROWS / 8;  // copies a stage: 8 rows of 128 bytes each
   constexpr int MT = (XR + 15) / 16;
@@ -133,7 +146,9 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
   const int lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, l4 = lane >> 4;
-  const int n0 = blockIdx.x * NT;
+  // rows of W that lie together in a tile, and in W
+  const int side = gated ? NT / 2 : NT, N1 = gated ? N / 2 : N;
+  const int n0 = blockIdx.x * side;
   const int M = min(XR, M_all - (int)blockIdx.z * XR);
   x += blockIdx.y * x_batch + blockIdx.z * XR * x_stride;
   c += blockIdx.y * c_batch + blockIdx.z * XR * c_stride;
@@ -145,7 +160,9 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
   for (int i = 0; i < NI; ++i) {
     const int r = i * 8 + (lane >> 3);
     const int j = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
-    at[i] = r < NT ? (uint32_t)min(r, N - 1 - n0) * row_bytes + j
+    const int up = r < side ? 0 : N1 - side;  // from a gate's row to an up row
+    at[i] = r < NT ? (uint32_t)(min(r, N1 - 1 - n0 + (r < side ? 0 : side)) + up) *
+                             row_bytes + j
                    : (uint32_t)min(r - NT, M - 1) * (uint32_t)x_stride + j;
   }
   const int cols = row_bytes / 128;
@@ -214,19 +231,24 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
           part + ((wid * MP + u * 16 + l15) * NT + t * 16 + l4 * 4)) = acc[t][u];
   __syncthreads();
   const float scale = FP8 ? x_scale[0] * w_scale[0] : 1.f;
-  for (int e = tid; e < M * (NT / 4); e += WAVES * 64) {
-    const int m = e / (NT / 4), n = e % (NT / 4) * 4;
-    if (n0 + n >= N) continue;
-    f32x4v s = {};
+  const int quads = side / 4;
+  for (int e = tid; e < M * quads; e += WAVES * 64) {
+    const int m = e / quads, n = e % quads * 4;
+    if (n0 + n >= N1) continue;
+    auto sum = [&](int n) {
+      f32x4v s = {};
 #pragma unroll
-    for (int v = 0; v < WAVES; ++v)
-      s += *reinterpret_cast<const f32x4v*>(part + ((v * MP + m) * NT + n));
+      for (int v = 0; v < WAVES; ++v)
+        s += *reinterpret_cast<const f32x4v*>(part + ((v * MP + m) * NT + n));
+      return FP8 ? s * scale : s;
+    };
+    const f32x4v s = sum(n), u = gated ? sum(n + side) : s;
     uint16_t o[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float f = FP8 ? s[r] * scale : s[r];
-      if (bias != nullptr) f += bf16_bits_to_f32(bias[n0 + n + r]);
-      o[r] = f32_to_bf16_bits(f);
+      const float f = biased(s[r], bias, n0 + n + r);
+      o[r] = gated ? silu_mul(f, biased(u[r], bias, N1 + n0 + n + r))
+                   : f32_to_bf16_bits(f);
     }
     *reinterpret_cast<uint2*>(c + (size_t)m * c_stride + n0 + n) =
         make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
@@ -273,7 +295,8 @@ __global__ __launch_bounds__(W * 64) void skinny_split_kernel(
     const uint8_t* __restrict__ x, const uint8_t* __restrict__ w,
     const uint16_t* __restrict__ bias, const float* __restrict__ x_scale,
     const float* __restrict__ w_scale, const int M, const int N,
-    const int row_bytes, const int64_t x_stride, const int64_t c_stride) {
+    const int row_bytes, const int64_t x_stride, const int64_t c_stride,
+    const bool gated) {
   constexpr int NT = W * 32;
   constexpr int ROWS = NT + XT * 32;
   // copies a wave and stage: its rows of W, some of X
@@ -285,7 +308,9 @@ __global__ __launch_bounds__(W * 64) void skinny_split_kernel(
   const int lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l31 = lane & 31;
-  const int n0 = blockIdx.x * NT;
+  // gated: a wave takes 16 rows of gate and 16 of up, which land in one lane
+  const int side = gated ? 16 : 32, N1 = gated ? N / 2 : N;
+  const int n0 = blockIdx.x * (W * side);
 
   // this workgroup's columns of 128 bytes
   const int cols = row_bytes / 128;
@@ -298,9 +323,10 @@ __global__ __launch_bounds__(W * 64) void skinny_split_kernel(
   auto x_rows = [&](int i) { return min(wid + W * i, XT * 4 - 1) * 8; };
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int r = (i < 4 ? wid * 32 + i * 8 : x_rows(i - 4)) + (lane >> 3);
+    const int r = (i < 4 ? i * 8 : x_rows(i - 4)) + (lane >> 3);
     const int j = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
-    at[i] = i < 4 ? (uint32_t)min(r, N - 1 - n0) * row_bytes + j
+    const int n = min(wid * side + r % side, N1 - 1 - n0) + r / side * N1;
+    at[i] = i < 4 ? (uint32_t)n * row_bytes + j
                   : (uint32_t)min(r, M - 1) * (uint32_t)x_stride + j;
   }
   // one head start a workgroup, see skinny_gemm_kernel
@@ -361,21 +387,30 @@ __global__ __launch_bounds__(W * 64) void skinny_split_kernel(
     if (m >= M) continue;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int n = n0 + wid * 32 + 8 * q + 4 * half;
-      if (n >= N) continue;
-      f32x4v v;
+      const int row = 8 * q + 4 * half;  // of the wave's 32
+      const int n = n0 + wid * side + row % side;
+      if (n >= N1) continue;
+      f32x4v v, u;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = acc[t][4 * q + r];
+      for (int r = 0; r < 4; ++r) {
+        v[r] = acc[t][4 * q + r];
+        u[r] = acc[t][(4 * q + 8 + r) & 15];
+      }
       if (FP8) v *= scale;
       if (part != nullptr) {
-        *reinterpret_cast<f32x4v*>(part + ((size_t)blockIdx.y * M + m) * N + n) = v;
+        *reinterpret_cast<f32x4v*>(part + ((size_t)blockIdx.y * M + m) * N + n +
+                                   row / side * N1) = v;
         continue;
       }
+      if (row >= side) continue;
+      if (FP8) u *= scale;
       uint16_t o[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        o[r] = f32_to_bf16_bits(
-            v[r] + (bias != nullptr ? bf16_bits_to_f32(bias[n + r]) : 0.f));
+      for (int r = 0; r < 4; ++r) {
+        const float f = biased(v[r], bias, n + r);
+        o[r] = gated ? silu_mul(f, biased(u[r], bias, N1 + n + r))
+                     : f32_to_bf16_bits(f);
+      }
       *reinterpret_cast<uint2*>(c + (size_t)m * c_stride + n) =
           make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
     }
@@ -385,20 +420,29 @@ __global__ __launch_bounds__(W * 64) void skinny_split_kernel(
 __global__ __launch_bounds__(256) void skinny_sum_kernel(
     uint16_t* __restrict__ c, const float* __restrict__ part,
     const uint16_t* __restrict__ bias, const int splits, const int M, const int N,
-    const int64_t c_stride) {
+    const int64_t c_stride, const bool gated) {
+  const int N1 = gated ? N / 2 : N;
   const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   const int64_t all = (int64_t)M * N;
-  if (e >= all) return;
-  f32x4v s = {};
+  const int m = (int)(e / N1), n = (int)(e % N1);
+  if (m >= M) return;
+  auto sum = [&](int n) {
+    const float* src = part + (int64_t)m * N + n;
+    f32x4v s = {};
 #pragma unroll 8
-  for (int k = 0; k < splits; ++k)
-    s += *reinterpret_cast<const f32x4v*>(part + k * all + e);
-  const int m = e / N, n = e % N;
+    for (int k = 0; k < splits; ++k)
+      s += *reinterpret_cast<const f32x4v*>(src + k * all);
+    return s;
+  };
+  const f32x4v s = sum(n);
+  f32x4v u = s;
+  if (gated) u = sum(N1 + n);
   uint16_t o[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    o[r] = f32_to_bf16_bits(
-        s[r] + (bias != nullptr ? bf16_bits_to_f32(bias[n + r]) : 0.f));
+  for (int r = 0; r < 4; ++r) {
+    const float f = biased(s[r], bias, n + r);
+    o[r] = gated ? silu_mul(f, biased(u[r], bias, N1 + n + r)) : f32_to_bf16_bits(f);
+  }
   *reinterpret_cast<uint2*>(c + (size_t)m * c_stride + n) =
       make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
 }
@@ -424,13 +468,16 @@ static int skinny_splits(int N, int row_bytes) {
 extern "C" void launch_skinny_split(
     void* c, float* part, int splits, const void* x, const void* w,
     const void* bias, const float* x_scale, const float* w_scale, bool fp8, int M,
-    int N, int row_bytes, int64_t x_stride, int64_t c_stride, hipStream_t stream) {
+    int N, int row_bytes, int64_t x_stride, int64_t c_stride, bool gated,
+    hipStream_t stream) {
   const int waves = skinny_waves(N);
   auto run = [&](auto kernel) {
-    kernel<<<dim3(ceil_div(N, waves * 32), splits), waves * 64, 0, stream>>>(
+    const int rows = waves * (gated ? 16 : 32);
+    kernel<<<dim3(ceil_div(gated ? N / 2 : N, rows), splits), waves * 64, 0,
+             stream>>>(
         (uint16_t*)c, part, (const uint8_t*)x, (const uint8_t*)w,
         (const uint16_t*)bias, x_scale, w_scale, M, N, row_bytes, x_stride,
-        c_stride);
+        c_stride, gated);
   };
   auto pick = [&](auto f, auto wv) {
     constexpr bool F = decltype(f)::value;
@@ -448,8 +495,8 @@ extern "C" void launch_skinny_split(
   if (fp8) by(std::true_type{});
   else by(std::false_type{});
   if (splits > 1)
-    skinny_sum_kernel<<<ceil_div((int64_t)M * N, 1024), 256, 0, stream>>>(
-        (uint16_t*)c, part, (const uint16_t*)bias, splits, M, N, c_stride);
+    skinny_sum_kernel<<<ceil_div(M * (gated ? N / 2 : N), 1024), 256, 0, stream>>>(
+        (uint16_t*)c, part, (const uint16_t*)bias, splits, M, N, c_stride, gated);
 }
 
 // Tiles, by rows of X and by how many tiles W gives. us of bf16 products, W from
@@ -499,17 +546,18 @@ extern "C" void launch_skinny_gemm(
     void* c, const void* x, const void* w, const void* bias,
     const float* x_scale, const float* w_scale, bool fp8, int M, int N,
     int row_bytes, int64_t x_stride, int64_t c_stride, int batch,
-    int64_t x_batch, int64_t c_batch, hipStream_t stream, bool* launched) {
+    int64_t x_batch, int64_t c_batch, bool gated, hipStream_t stream,
+    bool* launched) {
   *launched = false;
   const int nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes);
   if (nt == 0 || row_bytes % 128 || N % 4) return;
   *launched = true;
   auto run = [&](auto kernel, int xr, int waves) {
-    kernel<<<dim3(ceil_div(N, nt), batch, ceil_div(M, xr)), waves * 64, 0,
-             stream>>>(
+    const int tiles = gated ? ceil_div(N / 2, nt / 2) : ceil_div(N, nt);
+    kernel<<<dim3(tiles, batch, ceil_div(M, xr)), waves * 64, 0, stream>>>(
         (uint16_t*)c, (const uint8_t*)x, (const uint8_t*)w,
         (const uint16_t*)bias, x_scale, w_scale, M, N, row_bytes, x_stride,
-        c_stride, x_batch, c_batch);
+        c_stride, x_batch, c_batch, gated);
   };
   auto pick = [&](auto f) {
     constexpr bool F = decltype(f)::value;

@@ -137,6 +137,12 @@ class MergedColumnParallelLinear(nn.Module, _Fp8WeightMixin):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self._linear(x)
 
+    def silu_and_mul(self, x: torch.Tensor) -> torch.Tensor:
+        """silu(first part) * second part, of two equal ones."""
+        if self.fp8:
+            return ops.silu_and_mul(self._linear(x))
+        return ops.linear_silu_and_mul(x, self.weight, self.bias)
+
     def split_output(self, y: torch.Tensor) -> List[torch.Tensor]:
         return list(torch.split(y, self.shard_sizes, dim=-1))
 

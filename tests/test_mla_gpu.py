@@ -169,7 +169,7 @@ def test_mla_decode_listed_tokens(H, topk):
                                   # portion's first rows before it
 ])
 def test_mla_prefill(H, T, L, fp8):
-    """Against fp32 products. The result's rounding is 2^-9 of it; a logit is
+    """Against fp32 products. The result's rounding is 2^-8 of it at most; a logit is
     off by at most the lo parts' rounding, sum |q k| * scale * 2^-17 < 2e-4,
     a result by twice that of max |v| < 6."""
     g = torch.Generator(device="cuda").manual_seed(T)

@@ -27,7 +27,7 @@ def _rand(g, *s):
     (127, 8192, 2112),
 ])
 def test_linear_few_rows(M, N, K):
-    """fp32 sums of exact products: 2^-9 of the result for its rounding, and
+    """fp32 sums of exact products: 2^-8 of the result for its rounding, and
     K 2^-24 of the sum of magnitudes (< K here) for the sums."""
     g = torch.Generator(device="cuda").manual_seed(M + N)
     x = _rand(g, M, 2 * K).bfloat16()[:, K:]
@@ -36,7 +36,7 @@ def test_linear_few_rows(M, N, K):
     ext = ops._require_ext("skinny_gemm")
     out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
     none = x.new_empty(0)
-    assert ext.skinny_gemm(out, x, w, none, none, none)
+    assert ext.skinny_gemm(out, x, w, none, none, none, False)
     want = x.float() @ w.float().t()
     tol = dict(rtol=2 ** -8, atol=K * K * 2 ** -24)
     torch.testing.assert_close(out.float(), want, **tol)
@@ -118,3 +118,29 @@ def test_mla_products(B, H):
         ops.mla_absorb(q[..., :96], uk[:, :96]).float(),
         torch.einsum("bhd,hdr->bhr", q[..., :96].float(), uk[:, :96].float()),
         rtol=2 ** -8, atol=1e-2)
+
+
+@pytest.mark.parametrize("M,I,K", [
+    (1, 8, 128), (8, 456, 896), (9, 2408, 2176), (16, 4872, 384), (32, 4872, 384),
+    (20, 768, 11264), (33, 304, 4224), (64, 2408, 4224), (96, 14336, 256),
+    (128, 18432, 256), (3, 104, 72), (130, 64, 256),
+])
+def test_linear_silu_and_mul(M, I, K):
+    """Gate and up are rounded to bf16 (2^-8 of each at most), their function and the
+    result's rounding follow; |silu'| < 1.1."""
+    g = torch.Generator(device="cuda").manual_seed(M + I)
+    x = _rand(g, M, K).bfloat16()
+    w = (_rand(g, 2 * I, K) * K ** -0.5).bfloat16()
+    b = _rand(g, 2 * I).bfloat16()
+    out = ops.linear_silu_and_mul(x, w, b)
+    y = x.float() @ w.float().t() + b.float()
+    gate, up = y[:, :I], y[:, I:]
+    silu = torch.nn.functional.silu(gate)
+    want = silu * up
+    # where the library has the product, it is rounded before the bias as well:
+    # gate and up are off by 2^-8 of themselves and of what they were without it
+    p = y - b.float()
+    e = (y.abs() + p.abs()) * 2 ** -8
+    bound = (1.1 * e[:, :I] * up.abs() + silu.abs() * e[:, I:]
+             + want.abs() * 2 ** -8 + 1e-3)
+    assert ((out.float() - want).abs() <= bound).all()
