@@ -42,7 +42,13 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-constexpr float kHidden = -1e30f;  // score of a key that is not seen
+// Score of a key that is not seen, and where an item's maximum starts. A tile in
+// which an item sees nothing (a window, a split at the diagonal) leaves its m, l
+// and O alone: -inf raises no maximum and weighs exp2(-inf) = 0. A finite hidden
+// score would be rounded once in m and not in the weight's fma, whose exponent is
+// then the rounding error: +8e20 for 64-wide heads.
+constexpr float kHidden = -__builtin_inff();
+constexpr float kLowest = -1e30f;
 
 DEVINL float max_halves(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v),
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
       if (half == 0 && item_ok) {
         float* ml = tmp_ml +
             (((size_t)(q0 + row) * Hq + h) * gridDim.y + blockIdx.y) * 2;
-        ml[0] = kHidden;
+        ml[0] = kLowest;
         ml[1] = 0.f;
       }
       return;
@@ -205,11 +211,13 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
       qf[s] = __builtin_bit_cast(bf16x8v, v);
     }
   }
-  // scores in units of log2: exp2(c * s - m)
-  const float c = softcap > 0.f ? 1.f : fabsf(scale) * kLog2e;
+  // scores in units of log2: exp2(c * s - m); c > 0 also for a scale of 0, as
+  // hidden scores are multiplied by it too
+  const float c =
+      softcap > 0.f ? 1.f : fmaxf(fabsf(scale) * kLog2e, 1e-20f);
 
   f32x16v o[DT] = {};
-  float m = kHidden, l = 0.f;  // l: this half's tokens only
+  float m = kLowest, l = 0.f;  // l: this half's tokens only
 
   // ---- tile addresses -----------------------------------------------------------
   // 16 chunks (256 bytes) make a turn over the banks: a K row of 128 values,

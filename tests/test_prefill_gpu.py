@@ -142,3 +142,34 @@ def test_prefill_items_pages_and_splits(Hq, Hk, D, BS, fp8, kw):
             q.float().cpu(), ref_k.cpu(), ref_v.cpu(), bt.cpu(), slt.cpu(),
             qlt.cpu(), D ** -0.5, **kw)
         torch.testing.assert_close(out.float().cpu(), want, atol=2.1e-2, rtol=0)
+
+
+@pytest.mark.parametrize("D,Hq,Hk,ql,pre,window,scale", [
+    (64, 64, 8, 512, 0, 128, 0.125),       # rows 63 modulo 64: first tile unseen
+    (64, 14, 2, 512, 0, 128, 0.125),       # rows cut by a tile's edge
+    (64, 16, 16, 2300, 0, 2047, 0.125),
+    (64, 8, 1, 261, 0, 127, 0.1),
+    (64, 8, 8, 261, 30, 65, 80 ** -0.5),
+    (128, 8, 2, 300, 0, 100, 1 / 12),
+    (128, 8, 8, 200, 37, 65, 1 / 128),
+    (64, 14, 2, 40, 4607, -1, 0.125),      # the last split begins at the diagonal
+    (64, 14, 2, 40, 4607, 700, 0.125),
+    (64, 8, 2, 200, 50, 70, -0.125),
+    (64, 8, 2, 200, 50, 70, 0.0),
+    (128, 8, 2, 40, 2000, 70, 0.0),
+])
+@pytest.mark.parametrize("sinks", [False, True])
+def test_prefill_rows_whose_first_tile_is_hidden(D, Hq, Hk, ql, pre, window, scale,
+                                                 sinks):
+    """Items that see no key of the first tile their wave computes, by a window or
+    by a split of the keys, for scales whose product with a hidden score rounds
+    either way. Tolerance as above; sinks take weight away only."""
+    q, kc, vc, bt, sl, qlt = _setup([ql], [pre + ql], Hq, Hk, D, seed=ql)
+    sk = torch.linspace(-2, 2, Hq, device="cuda") if sinks else None
+    out = ops.prefill_attention(q, kc, vc, bt, sl, qlt, scale,
+                                sliding_window=window, sinks=sk)
+    assert bool(out.isfinite().all())
+    want = ref.prefill_attention(
+        q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt.cpu(), sl.cpu(),
+        qlt.cpu(), scale, sliding_window=window, sinks=sk.cpu() if sinks else None)
+    torch.testing.assert_close(out.float().cpu(), want, atol=2.1e-2, rtol=0)
