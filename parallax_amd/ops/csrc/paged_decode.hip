@@ -45,7 +45,8 @@ typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kHidden = -1e30f;
+constexpr float kHidden = -__builtin_inff();  // score of a key that is not seen
+constexpr float kLowest = -1e30f;              // where a maximum starts
 
 DEVINL uint32_t pack_bf16(float a, float b) {
   bf16x2n p;
@@ -323,13 +324,18 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
       const uint16_t* row = q + (size_t)seq * q_stride +
                             (size_t)(hk * G + min(l15, G - 1)) * D;
 #pragma unroll
-      for (int s = 0; s < KC; ++s)
-        qf[s] = *(const bf16x8v*)(row + (FP8 ? ((s >> 1) * 4 + l4) * 16 + (s & 1) * 8
-                                             : s * 32 + l4 * 8));
+      for (int s = 0; s < KC; ++s) {
+        u32x4v v = *(const u32x4v*)(row + (FP8 ? ((s >> 1) * 4 + l4) * 16 + (s & 1) * 8
+                                              : s * 32 + l4 * 8));
+        if (scale < 0.f) v ^= 0x80008000u;  // the sign goes with q: c takes maxima
+        qf[s] = __builtin_bit_cast(bf16x8v, v);
+      }
     }
     f32x4v o[MT] = {};
-    float m = kHidden, l = 0.f;
-    const float c = softcap > 0.f ? 1.f : scale * kLog2e;
+    float m = kLowest, l = 0.f;
+    // above 0 also for a scale of 0: hidden scores are multiplied by it too
+    const float c =
+        softcap > 0.f ? 1.f : fmaxf(fabsf(scale) * kLog2e, 1e-20f);
 
     // this wave's tiles: from first on, a unit apart
     int first = (unit0 + t0) * U + wid * PD_KT;
@@ -403,7 +409,7 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             s[e >> 2][e & 3] =
-                softcap * tanhf(s[e >> 2][e & 3] * scale / softcap) * kLog2e;
+                softcap * tanhf(s[e >> 2][e & 3] * fabsf(scale) / softcap) * kLog2e;
         }
         const bool cut = tok + PD_KT > L;
         if (cut || tok < lo) {
@@ -473,7 +479,7 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
       ls[wid][l15] = l;
     }
     __syncthreads();
-    float M = kHidden;
+    float M = kLowest;
 #pragma unroll
     for (int w = 0; w < W; ++w) M = fmaxf(M, ms[w][l15]);
     const float f = __builtin_amdgcn_exp2f(m - M) * v_scale;
@@ -488,7 +494,7 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
         whole ? seq : (size_t)blockIdx.y + seq;  // named by run + sequence
     for (int e = tid; e < G * (D / 4); e += W * 64) {
       const int g = e / (D / 4), d = e % (D / 4) * 4;
-      float Mg = kHidden, lg = 0.f;
+      float Mg = kLowest, lg = 0.f;
 #pragma unroll
       for (int w = 0; w < W; ++w) Mg = fmaxf(Mg, ms[w][g]);
 #pragma unroll
@@ -554,7 +560,7 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
   const int parts = r1 - r0 + 1;
   const size_t row0 = ((size_t)r0 + seq) * Hq + hk * G;
   for (int g = tid >> 6; g < G; g += 4) {  // a wave a head
-    float M = kHidden, l = 0.f;
+    float M = kLowest, l = 0.f;
     for (int r = lane; r < parts; r += 64)
       M = fmaxf(M, tmp_ml[(row0 + (size_t)r * Hq + g) * 2]);
     M = wave_reduce_max(M);

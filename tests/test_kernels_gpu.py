@@ -434,6 +434,30 @@ def test_paged_decode_units_runs_and_windows(D, BS, fp8, G, Hk, lens, kw):
     torch.testing.assert_close(out[some].float(), want.float(), atol=2.2e-2, rtol=0)
 
 
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 1e-25])
+@pytest.mark.parametrize("lens,kw", [
+    ([1, 31, 33, 100, 300], {}),                  # tiles cut by the end
+    ([90, 300, 33, 1000], {"sliding_window": 77}),
+    ([3000, 7, 1025], {}),                        # parts of several runs
+    ([90, 300], {"softcap": 20.0}),
+])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_paged_decode_scales_of_any_sign(scale, lens, kw, fp8):
+    """A scale below 0 or of 0 (a plain mean): hidden keys have no weight either
+    way. Tolerance as above."""
+    B, D = len(lens), 64
+    kc, vc, bt = _make_paged_kv(B, 2, D, 32, max(lens), seed=B)
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+    q = torch.randn(B, 8, D, device="cuda",
+                    generator=torch.Generator(device="cuda").manual_seed(B)).bfloat16()
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = ops.paged_attention_decode(q, kc, vc, bt, sl, scale, **kw)
+    want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl,
+                                      scale, **kw)
+    torch.testing.assert_close(out.float(), want.float(), atol=2.2e-2, rtol=0)
+
+
 @pytest.mark.parametrize("neox", [True, False])
 @pytest.mark.parametrize("T,Hq,Hk,D,rot,BS,fp8,start", [
     (1, 14, 2, 64, 64, 32, False, None),    # None: scattered slots, some absent
