@@ -41,7 +41,8 @@ typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kHidden = -1e30f;
+constexpr float kHidden = -__builtin_inff();  // score of a key that is not seen
+constexpr float kLowest = -1e30f;              // where a maximum starts
 
 DEVINL uint32_t pack_bf16(float a, float b) {
   bf16x2n p;
@@ -234,9 +235,15 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
     for (int s = 0; s < 12; ++s)
       qf[s] = s < 8 ? *(const bf16x8v*)(a + s * 16)
                     : *(const bf16x8v*)(b + (s - 8) * 16);
+    if (scale < 0.f) {  // the sign goes with q: c takes maxima
+#pragma unroll
+      for (int s = 0; s < 12; ++s)
+        qf[s] = __builtin_bit_cast(
+            bf16x8v, __builtin_bit_cast(u32x4v, qf[s]) ^ 0x80008000u);
+    }
   }
   f32x16v o[4] = {};
-  float m = kHidden, l = 0.f;  // l: this half's keys only
+  float m = kLowest, l = 0.f;  // l: this half's keys only
   float* st = state + ((size_t)row_c * H + h) * 130;
   if (!first) {
     m = st[128];
@@ -249,7 +256,8 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
         for (int r = 0; r < 4; ++r)
           o[t][4 * i + r] = st[t * 32 + 8 * i + 4 * half + r];
   }
-  const float c = scale * kLog2e;
+  // above 0 also for a scale of 0: hidden scores are multiplied by it too
+  const float c = fmaxf(fabsf(scale) * kLog2e, 1e-20f);
 
   // ---- copies: chunk numbers within a tile, LDS places XOR-swizzled by row ---------
   const uint16_t* kh = k_hi + (size_t)h * cap * MP_D;

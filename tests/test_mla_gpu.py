@@ -192,6 +192,29 @@ def test_mla_prefill(H, T, L, fp8):
             out[:, h].float(), p @ v, atol=2.4e-3, rtol=2 ** -8)
 
 
+@pytest.mark.parametrize("scale", [-0.07, 0.0])
+def test_mla_prefill_scales_of_any_sign(scale):
+    """Below 0 and 0 (a plain mean): hidden keys have no weight either way. 3 heads,
+    130 rows on 170, tolerance as above."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    H, T, L = 3, 130, 300
+    q_nope, q_pe = r(T, H, 128).bfloat16(), r(T, H, 64).bfloat16()
+    rows = r(L, 576).bfloat16()
+    uk, uv = ((r(H, 128, 512) * 512 ** -0.5).bfloat16() for _ in range(2))
+    out = torch.empty(T, H, 128, dtype=torch.bfloat16, device="cuda")
+    assert ops.mla_prefill_attention(out, q_nope, q_pe, rows, uk, uv, scale)
+    e = rows.float()
+    hidden = torch.arange(L, device="cuda")[None] > torch.arange(
+        L - T, L, device="cuda")[:, None]
+    for h in range(H):
+        k, v = e[:, :512] @ uk[h].float().t(), e[:, :512] @ uv[h].float().t()
+        s = q_nope[:, h].float() @ k.t() + q_pe[:, h].float() @ e[:, 512:].t()
+        p = (s * scale).masked_fill(hidden, float("-inf")).softmax(-1)
+        torch.testing.assert_close(
+            out[:, h].float(), p @ v, atol=2.4e-3, rtol=2 ** -8)
+
+
 def test_mla_prefill_left_to_the_caller():
     """Types, widths and few rows on a long context have no kernel."""
     def call(T, L, H=16, dtype=torch.bfloat16, dn=128, dr=64, dev="cuda"):
