@@ -407,14 +407,18 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
     compute(kt, Kl, Vl);
     if (KV_FP8 && more) widen8(Kn, Vn);
   };
-  pages(kt_begin);
-  if (KV_FP8) {
-    fetch8(kt_begin);
-    widen8(K0, V0);
-  } else {
-    issue(kt_begin, K0, V0);
+  // a portion longer than its context has rows that see nothing, and pages that
+  // must not be looked up
+  if (kt_begin < kt_end) {
+    pages(kt_begin);
+    if (KV_FP8) {
+      fetch8(kt_begin);
+      widen8(K0, V0);
+    } else {
+      issue(kt_begin, K0, V0);
+    }
+    pages(kt_begin + 1);
   }
-  pages(kt_begin + 1);
   for (int kt = kt_begin; kt < kt_end; kt += 2) {
     turn(kt, K0, V0, K1, V1);
     if (kt + 1 < kt_end) turn(kt + 1, K1, V1, K0, V0);

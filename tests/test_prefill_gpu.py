@@ -173,3 +173,20 @@ def test_prefill_rows_whose_first_tile_is_hidden(D, Hq, Hk, ql, pre, window, sca
         q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt.cpu(), sl.cpu(),
         qlt.cpu(), scale, sliding_window=window, sinks=sk.cpu() if sinks else None)
     torch.testing.assert_close(out.float().cpu(), want, atol=2.1e-2, rtol=0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_prefill_portion_without_context(fp8):
+    """A request whose context is shorter than its portion, or empty, reads no page
+    for the rows before it (its table row holds a page that is not there); the other
+    requests are right."""
+    q, kc, vc, bt, sl, ql = _setup([40, 70, 33], [64, 70, 33], 8, 2, 64, seed=11)
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+    bt[1], sl[1] = -1, 0
+    out = ops.prefill_attention(q, kc, vc, bt, sl, ql, 0.125)
+    keep = torch.cat([torch.arange(40), torch.arange(110, 143)]).cuda()
+    pick = torch.tensor([0, 2], device="cuda")
+    want = ref.prefill_attention(q[keep].float(), kc.float(), vc.float(), bt[pick],
+                                 sl[pick], ql[pick], 0.125)
+    torch.testing.assert_close(out[keep].float(), want, atol=2.1e-2, rtol=0)
