@@ -166,6 +166,12 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     at = 0;
     todo = (domain_of<SPARSE>(seq_lens, topk, max_topk, seq) + MLA_KT - 1) /
            MLA_KT;
+    if (todo == 0) {  // no tokens: zeros, of this workgroup's heads
+      const int h0 = blockIdx.y * (W * 8), n = min(W * 8, H - h0);
+      for (int e = tid; e < n * (MLA_R / 4); e += W * 64)
+        *reinterpret_cast<uint2*>(out + ((size_t)seq * H + h0) * MLA_R + e * 4) =
+            make_uint2(0, 0);
+    }
   } else {
     int first;
     const int total = find_tile<SPARSE>(seq_lens, topk, max_topk, B, 0, &seq,
@@ -533,7 +539,14 @@ __global__ __launch_bounds__(512) void mla_reduce_kernel(
   }
   const int tiles =
       (domain_of<SPARSE>(seq_lens, topk, max_topk, seq) + MLA_KT - 1) / MLA_KT;
-  if (tiles == 0) return;
+  if (tiles == 0) {  // no tokens: zeros
+    if (head < H)
+      for (int d = (BY_HEAD ? tid & 127 : tid) * 4; d < MLA_R;
+           d += (BY_HEAD ? 128 : 512) * 4)
+        *reinterpret_cast<uint2*>(out + ((size_t)seq * H + head) * MLA_R + d) =
+            make_uint2(0, 0);
+    return;
+  }
   const int per = run_length(total, runs);
   const int r0 = first / per, r1 = (first + tiles - 1) / per;
   if (r0 == r1) return;  // finished by its run

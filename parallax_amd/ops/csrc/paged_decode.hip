@@ -276,6 +276,10 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
     seq = blockIdx.y;
     at = 0;
     todo = units_of(seq_lens[seq], window, U);
+    if (todo == 0)  // no tokens: zeros
+      for (int e = tid; e < G * (D / 4); e += W * 64)
+        *reinterpret_cast<uint2*>(out + ((size_t)seq * Hq + hk * G) * D + e * 4) =
+            make_uint2(0, 0);
   } else {
     todo = find_run(seq_lens, window, U, B, blockIdx.y, gridDim.y, &seq, &at);
   }
@@ -549,7 +553,12 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
     first += __shfl_xor(first, o, WAVE_SIZE);
   }
   const int units = units_of(seq_lens[seq], window, u);
-  if (units == 0) return;
+  if (units == 0) {  // no tokens: zeros
+    for (int e = tid; e < G * (D / 4); e += 256)
+      *reinterpret_cast<uint2*>(out + ((size_t)seq * Hq + hk * G) * D + e * 4) =
+          make_uint2(0, 0);
+    return;
+  }
   const int per = run_length(total, runs);
   const int r0 = first / per, r1 = (first + units - 1) / per;
   if (r0 == r1) return;  // finished by its run

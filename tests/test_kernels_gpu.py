@@ -458,6 +458,26 @@ def test_paged_decode_scales_of_any_sign(scale, lens, kw, fp8):
     torch.testing.assert_close(out.float(), want.float(), atol=2.2e-2, rtol=0)
 
 
+@pytest.mark.parametrize("sinks", [False, True])
+@pytest.mark.parametrize("max_seq_len", [200, 4096])   # a workgroup each, runs
+def test_paged_decode_sequences_without_tokens(max_seq_len, sinks):
+    """Results of 0, whatever the memory held; the others as ever."""
+    lens = [0, 130, 0, 0, 7, 0]
+    kc, vc, bt = _make_paged_kv(6, 2, 64, 32, 130)
+    q = torch.randn(6, 14, 64, device="cuda").bfloat16()
+    sk = torch.zeros(14, device="cuda") if sinks else None
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    poison = [torch.full(q.shape, float("nan"), dtype=q.dtype, device="cuda")
+              for _ in range(8)]
+    del poison
+    out = ops.paged_attention_decode(q, kc, vc, bt, sl, 0.125, sinks=sk,
+                                     max_seq_len=max_seq_len)
+    want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl,
+                                      0.125, sinks=sk)
+    assert want[0].abs().sum() == 0
+    torch.testing.assert_close(out.float(), want.float(), atol=2.2e-2, rtol=0)
+
+
 @pytest.mark.parametrize("neox", [True, False])
 @pytest.mark.parametrize("T,Hq,Hk,D,rot,BS,fp8,start", [
     (1, 14, 2, 64, 64, 32, False, None),    # None: scattered slots, some absent

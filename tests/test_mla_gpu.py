@@ -138,6 +138,25 @@ def test_mla_decode_runs(H, BS, ctxs, fp8):
     torch.testing.assert_close(out.float().cpu(), want, atol=2.2e-2, rtol=0)
 
 
+@pytest.mark.parametrize("H", [16, 72, 128])
+@pytest.mark.parametrize("max_seq_len", [200, 4096, 10 ** 6])
+def test_mla_decode_sequences_without_tokens(H, max_seq_len):
+    """Results of 0, whatever the memory held; the others as ever."""
+    ctxs = [0, 130, 0, 0, 7, 0] * (4 if max_seq_len == 10 ** 6 else 1)
+    ql, qp, cache, bt, sl = _setup(len(ctxs), H, ctxs, seed=H)
+    poison = [torch.full_like(ql, float("nan")) for _ in range(8)]
+    del poison
+    scale = 192 ** -0.5
+    out = ops.mla_paged_attention_decode(ql, qp, cache, bt, sl, scale,
+                                         max_seq_len=max_seq_len)
+    want = torch.zeros(ql.shape)
+    some = [i for i, n in enumerate(ctxs) if n]
+    want[some] = ref.mla_paged_attention_decode(
+        ql[some].float().cpu(), qp[some].float().cpu(), cache.float().cpu(),
+        bt[some].cpu(), sl[some].cpu(), scale)
+    torch.testing.assert_close(out.float().cpu(), want, atol=2.2e-2, rtol=0)
+
+
 @pytest.mark.parametrize("H,topk", [(16, 40), (128, 512)])
 def test_mla_decode_listed_tokens(H, topk):
     """Rows restricted to listed positions (some entries stand for none), beside
