@@ -244,10 +244,11 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     auto slot_of = [&](int tok) INL -> int {
       return (btab[tok >> bs_shift] << bs_shift) + (tok & (BS - 1));
     };
-    // cache row (token slot) of tile row `lane`, listed
+    // cache row (token slot) of tile row `lane`, listed; a sequence without tokens
+    // has no page to look up
     auto listed_slot = [&](int t) INL {
       const int e = entry(t * MLA_KT + lane);
-      return slot_of(e >= 0 && e < L ? e : 0);
+      return L > 0 ? slot_of(e >= 0 && e < L ? e : 0) : 0;
     };
     constexpr int ESZ = KV_FP8 ? 1 : 2;
     // where the copies of tile t read: a base that all lanes share, and 32 bits.

@@ -179,6 +179,24 @@ def test_mla_decode_listed_tokens(H, topk):
     torch.testing.assert_close(out.float().cpu(), want, atol=2.2e-2, rtol=0)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+def test_mla_decode_list_without_tokens(fp8):
+    """A list beside an empty sequence, whose table row holds a page that is not
+    there: no page is read for it, its result is 0."""
+    ql, qp, cache, bt, sl = _setup(3, 16, [300, 300, 300], seed=3)
+    ql, idx = ql * 10, torch.full((3, 70), -1, dtype=torch.int32, device="cuda")
+    idx[:, :40] = torch.arange(0, 280, 7, dtype=torch.int32, device="cuda")
+    if fp8:
+        cache = cache.to(torch.float8_e4m3fn)
+    bt[1], sl[1] = -1, 0
+    out = ops.dsa_paged_attention_decode(ql, qp, cache, bt, sl, idx, 192 ** -0.5)
+    assert float(out[1].abs().max()) == 0
+    want = ref.dsa_paged_attention_decode(
+        ql[::2].float(), qp[::2].float(), cache.float(), bt[::2], sl[::2], idx[::2],
+        192 ** -0.5)
+    torch.testing.assert_close(out[::2].float(), want, atol=2.2e-2, rtol=0)
+
+
 @pytest.mark.parametrize("H,T,L,fp8", [
     (128, 1, 1, False),
     (8, 33, 33, False),           # past a wave's 32 rows and a tile's 32 keys
