@@ -459,14 +459,12 @@ bool mla_prefill_attention(torch::Tensor out, torch::Tensor q_nope,
     return false;
   if (q_nope.stride(2) != 1 || q_nope.stride(1) % 8 || q_nope.stride(0) % 8)
     return false;
-  CHECK_CONTIG(out);
-  CHECK_CONTIG(q_pe);
-  CHECK_CONTIG(rows);
-  CHECK_CONTIG(w_uk);
-  CHECK_CONTIG(w_uv);
+  if (L < T) return false;
+  for (const auto& t : {out, q_pe, rows, w_uk, w_uv})
+    if (!t.is_contiguous()) return false;
   TORCH_CHECK(q_pe.size(0) == T && q_pe.size(1) == H && out.size(0) == T &&
               out.size(1) == H && out.size(2) == 128 && w_uk.size(0) == H &&
-              w_uv.size(0) == H && w_uv.size(2) == 512 && L >= T);
+              w_uv.size(0) == H && w_uv.size(2) == 512);
   if (T == 0 || H == 0) return true;
   // 1 GB of expanded keys and values a run
   const int64_t run = std::max<int64_t>(128, ((1 << 20) / H) & ~127);
@@ -784,13 +782,14 @@ static bool rows16(const torch::Tensor& t) {
 bool mla_absorb(torch::Tensor out, torch::Tensor q, torch::Tensor w) {
   CHECK_GPU(q);
   const int64_t B = q.size(0), H = q.size(1), R = w.size(2);
-  if (!rows16(q) || !rows16(w) || q.size(2) != 128 || R % 128) return false;
-  CHECK_CONTIG(w);
+  if (!rows16(q) || !rows16(w) || !w.is_contiguous() || q.size(2) != 128 ||
+      R % 128)
+    return false;
   CHECK_CONTIG(out);
   CHECK_BF16(out);
   TORCH_CHECK(w.size(0) == H && w.size(1) == 128 && out.size(0) == B &&
               out.size(1) == H && out.size(2) == R);
-  if (B == 0) return true;
+  if (out.numel() == 0) return true;
   launch_mla_absorb(out.data_ptr(), q.data_ptr(), w.data_ptr(), B, H, R,
                     q.stride(0), q.stride(1), cur_stream());
   return true;
@@ -799,13 +798,13 @@ bool mla_absorb(torch::Tensor out, torch::Tensor q, torch::Tensor w) {
 bool mla_project(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
   CHECK_GPU(x);
   const int64_t B = x.size(0), H = x.size(1), N = w.size(1), K = w.size(2);
-  if (!rows16(x) || !rows16(w) || K % 64 || N % 64) return false;
-  CHECK_CONTIG(w);
+  if (!rows16(x) || !rows16(w) || !w.is_contiguous() || K % 64 || N % 64)
+    return false;
   CHECK_CONTIG(out);
   CHECK_BF16(out);
   TORCH_CHECK(w.size(0) == H && x.size(2) == K && out.size(0) == B &&
               out.size(1) == H && out.size(2) == N);
-  if (B == 0) return true;
+  if (out.numel() == 0) return true;
   bool launched = false;
   launch_skinny_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), nullptr, nullptr,
                      nullptr, false, B, N, K * 2, x.stride(0) * 2, out.stride(0),

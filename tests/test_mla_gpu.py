@@ -265,3 +265,18 @@ def test_mla_prefill_left_to_the_caller():
     assert not call(40, 40, dn=64)
     assert not call(40, 40, dr=32)
     assert not call(40, 40, dev="cpu")
+
+
+def test_mla_prefill_operands_in_other_orders_left_to_the_caller():
+    """Views of a fused weight, a result or a context that is not the kernel's."""
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device="cuda")
+    q, pe, rows, w = z(40, 16, 128), z(40, 16, 64), z(50, 576), z(16, 128, 512)
+    fused = z(16, 256, 512)
+    assert ops.mla_prefill_attention(z(40, 16, 128), q, pe, rows, w, w, 1.0)
+    for out, r, uk, uv in (
+        (z(40, 16, 128), rows, fused[:, :128], w),
+        (z(40, 16, 128), rows, w, fused[:, 128:]),
+        (z(40, 16, 256)[..., :128], rows, w, w),
+        (z(40, 16, 128), rows[:39], w, w),      # a portion longer than its context
+    ):
+        assert not ops.mla_prefill_attention(out, q, pe, r, uk, uv, 1.0)

@@ -120,6 +120,26 @@ def test_mla_products(B, H):
         rtol=2 ** -8, atol=1e-2)
 
 
+def test_mla_products_of_weights_in_other_orders():
+    """Views of a fused weight, rows apart or transposed, and a batch of none."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = _rand(g, 5, 3, 128).bfloat16()
+    lat = _rand(g, 5, 3, 512).bfloat16()
+    fused = _rand(g, 3, 256, 512).bfloat16()
+    turned = _rand(g, 3, 512, 128).bfloat16().transpose(1, 2)
+    for w in (fused[:, :128], fused[:, 128:], turned):
+        torch.testing.assert_close(
+            ops.mla_absorb(q, w).float(),
+            torch.einsum("bhd,hdr->bhr", q.float(), w.float()), rtol=2 ** -8,
+            atol=128 ** 2 * 2 ** -24)
+        torch.testing.assert_close(
+            ops.mla_project_out(lat, w).float(),
+            torch.einsum("bhr,hvr->bhv", lat.float(), w.float()), rtol=2 ** -8,
+            atol=512 ** 2 * 2 ** -24)
+    assert ops.mla_absorb(q[:, :0], fused[:0, :128]).shape == (5, 0, 512)
+    assert ops.mla_project_out(lat[:0], fused[:, :128]).shape == (0, 3, 128)
+
+
 @pytest.mark.parametrize("M,I,K", [
     (1, 8, 128), (8, 456, 896), (9, 2408, 2176), (16, 4872, 384), (32, 4872, 384),
     (20, 768, 11264), (33, 304, 4224), (64, 2408, 4224), (96, 14336, 256),
