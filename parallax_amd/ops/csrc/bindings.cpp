@@ -727,6 +727,8 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
                        !bias.is_contiguous()))
     return false;
   const int64_t es = x.element_size();
+  // the kernels place rows of x by 32-bit offsets
+  if ((x.size(0) - 1) * x.stride(0) * es + 128 > UINT32_MAX) return false;
   if ((uintptr_t)x.data_ptr() % 16 || (uintptr_t)w.data_ptr() % 16 ||
       x.stride(0) * es % 16 || (uintptr_t)c.data_ptr() % 8 || c.stride(0) % 4)
     return false;
@@ -800,6 +802,8 @@ bool mla_project(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
   const int64_t B = x.size(0), H = x.size(1), N = w.size(1), K = w.size(2);
   if (!rows16(x) || !rows16(w) || !w.is_contiguous() || K % 64 || N % 64)
     return false;
+  // rows go 32 at a time, placed by 32-bit offsets
+  if (31 * x.stride(0) * 2 + 128 > UINT32_MAX) return false;
   CHECK_CONTIG(out);
   CHECK_BF16(out);
   TORCH_CHECK(w.size(0) == H && x.size(2) == K && out.size(0) == B &&

@@ -58,6 +58,28 @@ def test_linear_without_a_kernel():
         ops.linear(x, w).float(), x.float() @ w.float().t(), rtol=2 ** -8, atol=1e-3)
 
 
+def test_linear_of_rows_far_apart():
+    """Rows whose places do not fit 32 bits (the last token of every long prompt,
+    say)."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    apart = 24 << 20
+    buf = torch.empty(100 * apart, dtype=torch.bfloat16, device="cuda")
+    for M in (100, 100, 24):
+        x = buf.as_strided((M, 512), (apart * (100 // M), 1))
+        x.copy_(_rand(g, M, 512))
+        w = _rand(g, 28672, 512).bfloat16()
+        torch.testing.assert_close(
+            ops.linear(x, w).float(), x.float() @ w.float().t(), rtol=2 ** -8,
+            atol=512 ** 2 * 2 ** -24)
+    lat = buf.as_strided((34, 2, 512), (apart * 2, 512, 1))
+    lat.copy_(_rand(g, 34, 2, 512))
+    uv = _rand(g, 2, 128, 512).bfloat16()
+    torch.testing.assert_close(
+        ops.mla_project_out(lat, uv).float(),
+        torch.einsum("bhr,hvr->bhv", lat.float(), uv.float()), rtol=2 ** -8,
+        atol=512 ** 2 * 2 ** -24)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 64, 128), (7, 4800, 5120), (16, 64, 256),
                                    (30, 9600, 384), (40, 256, 512),
                                    (12, 36864, 256), (50, 1000, 4224),
