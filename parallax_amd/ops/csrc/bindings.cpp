@@ -726,6 +726,7 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
   if (bias.numel() && (bias.dim() != 1 || bias.numel() != w.size(0) ||
                        !bias.is_contiguous()))
     return false;
+  if (w.numel() == 0) return false;
   const int64_t es = x.element_size();
   // the kernels place rows of x by 32-bit offsets
   if ((x.size(0) - 1) * x.stride(0) * es + 128 > UINT32_MAX) return false;

@@ -80,6 +80,14 @@ def test_linear_of_rows_far_apart():
         atol=512 ** 2 * 2 ** -24)
 
 
+def test_linear_of_no_columns():
+    """Refused by the kernels, whose deals of columns assume one."""
+    ext = ops._require_ext("skinny_gemm")
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device="cuda")
+    for M, N, K in ((4, 64, 0), (40, 64, 0), (4, 0, 64)):
+        assert not ext.skinny_gemm(z(M, N), z(M, K), z(N, K), z(0), z(0), z(0), False)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 64, 128), (7, 4800, 5120), (16, 64, 256),
                                    (30, 9600, 384), (40, 256, 512),
                                    (12, 36864, 256), (50, 1000, 4224),
