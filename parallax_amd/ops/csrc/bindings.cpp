@@ -67,10 +67,11 @@ void launch_moe_gate_up(void*, const void*, const float*, const void*,
                         bool, bool, bool, float, hipStream_t);
 void launch_moe_down(float*, const void*, const float*, const void*,
                      const float*, const int*, const void*, const int*,
-                     const float*, int, int, int, int, int, bool, bool,
-                     hipStream_t);
+                     const float*, int, int, int, int, int, int, int, bool,
+                     bool, hipStream_t);
 void launch_moe_combine(float*, const float*, const int64_t*, int, int, int,
-                        int, hipStream_t);
+                        int, int, int, hipStream_t);
+int moe_down_cols(int, int);
 void launch_dsa_indexer_scores(float*, const void*, const void*, const float*,
                                const int*, const int*, int, int, int, int,
                                int, int, hipStream_t, bool*);
@@ -565,15 +566,19 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
                              stream);
     hp = hq.data_ptr();
   }
-  torch::Tensor y = torch::empty({n, H}, fopts);
+  const int slab = moe_down_cols(n, H);
+  torch::Tensor y = torch::empty({n, slab}, fopts);
   torch::Tensor out = torch::empty({T, H}, fopts);
-  launch_moe_down(y.data_ptr<float>(), hp,
-                  fp8 ? hs.data_ptr<float>() : nullptr, w_down.data_ptr(),
-                  fp8 ? w_down_scale.data_ptr<float>() : nullptr, perm, tiles,
-                  n_tiles, wts, k, H, I, max_tiles, tm, fp8, weight_on_input,
-                  stream);
-  launch_moe_combine(out.data_ptr<float>(), y.data_ptr<float>(), ids, T, k, E,
-                     H, stream);
+  for (int first = 0; first < H; first += slab) {
+    const int cols = std::min(slab, H - first);
+    launch_moe_down(y.data_ptr<float>(), hp,
+                    fp8 ? hs.data_ptr<float>() : nullptr, w_down.data_ptr(),
+                    fp8 ? w_down_scale.data_ptr<float>() : nullptr, perm, tiles,
+                    n_tiles, wts, k, H, I, first, cols, max_tiles, tm, fp8,
+                    weight_on_input, stream);
+    launch_moe_combine(out.data_ptr<float>(), y.data_ptr<float>(), ids, T, k, E,
+                       H, first, cols, stream);
+  }
   return out;
 }
 

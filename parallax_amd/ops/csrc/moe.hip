@@ -204,8 +204,9 @@ struct MoeArgs {
   const int* n_tiles;
   const float* choice_w;   // [T, k] routing weights
   const uint16_t* bias;    // [E, 2I] or null (GATE)
-  void* out;               // GATE: h [n, N] bf16; else y [T * k, N] fp32
+  void* out;               // GATE: h [n, N] bf16; else y [T * k, cols] fp32
   int topk, N, kb, nb;     // N output features, kb bytes a row, nb column blocks
+  int first, cols;         // the features of this launch: all (GATE), or a slab
   int in_w, gelu;
   float limit;             // > 0: clamped activation
 };
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
   const int e = __builtin_amdgcn_readfirstlane(tile.x);
   const int row0 = __builtin_amdgcn_readfirstlane(tile.y);
   const int rows_end = __builtin_amdgcn_readfirstlane(tile.z);
-  const int n0 = (idx % p.nb) * (GATE ? TN / 2 : TN);
+  const int n0 = p.first + (idx % p.nb) * (GATE ? TN / 2 : TN);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -446,11 +447,11 @@ __global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
           *reinterpret_cast<uint2*>(h + f) = o;
         }
       } else {
-        float* y = (float*)p.out + (size_t)choice * p.N;
+        float* y = (float*)p.out + (size_t)choice * p.cols - p.first;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int f = n0 + wb + i * 32 + 8 * q + 4 * half;
-          if (f >= p.N) continue;
+          if (f >= p.first + p.cols) continue;
           f32x4v o;
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
@@ -466,22 +467,22 @@ __global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
 }
 
 // ---- combine --------------------------------------------------------------------
-// out[t] = sum over its choices; four features a thread.
+// out[t] = sum over its choices, of the features from first on; four a thread.
 
 __global__ __launch_bounds__(256) void moe_combine_kernel(
     float* __restrict__ out, const float* __restrict__ y,
     const int64_t* __restrict__ ids, const int T, const int k, const int E,
-    const int H) {
+    const int H, const int first, const int cols) {
   const int t = blockIdx.x;
-  for (int c = (blockIdx.y * 256 + threadIdx.x) * 4; c < H;
+  for (int c = (blockIdx.y * 256 + threadIdx.x) * 4; c < cols;
        c += gridDim.y * 1024) {
     f32x4v s = {0.f, 0.f, 0.f, 0.f};
     for (int j = 0; j < k; ++j) {
       const int64_t e = ids[(size_t)t * k + j];
       if (e >= 0 && e < E)
-        s += *reinterpret_cast<const f32x4v*>(y + ((size_t)t * k + j) * H + c);
+        s += *reinterpret_cast<const f32x4v*>(y + ((size_t)t * k + j) * cols + c);
     }
-    *reinterpret_cast<f32x4v*>(out + (size_t)t * H + c) = s;
+    *reinterpret_cast<f32x4v*>(out + (size_t)t * H + first + c) = s;
   }
 }
 
@@ -533,7 +534,7 @@ extern "C" void launch_quantize_fp8_rows(
 template <bool FP8, int TN, int TM, int STAGES>
 static void launch_gemm(bool gate, MoeArgs& p, int max_tiles,
                         hipStream_t stream) {
-  p.nb = ceil_div(p.N, gate ? TN / 2 : TN);
+  p.nb = ceil_div(p.cols, gate ? TN / 2 : TN);
   const int blocks = (max_tiles * p.nb + 7) / 8 * 8;
   if (gate)
     moe_gemm_kernel<FP8, TN, TM, true, STAGES>
@@ -573,6 +574,14 @@ extern "C" int moe_max_tiles(int n, int E, int tm) {
   return n / tm + (n < E ? n : E);
 }
 
+// Output features of a down product and combine: y takes at most MOE_Y_BYTES (of
+// 256 features, a tile's width, at least), however many tokens a step brings.
+#define MOE_Y_BYTES (256ll << 20)
+extern "C" int moe_down_cols(int n, int H) {
+  const int64_t cols = MOE_Y_BYTES / (4ll * n) & ~255ll;
+  return cols >= H ? H : cols < 256 ? (H < 256 ? H : 256) : (int)cols;
+}
+
 // ints of scratch that routing n choices takes besides perm and tiles
 extern "C" int64_t moe_route_scratch(int n, int E) {
   return n > 2 * ROUTE_PART ? (int64_t)ceil_div(n, ROUTE_PART) * E : 0;
@@ -597,7 +606,7 @@ extern "C" void launch_moe_gate_up(
     float limit, hipStream_t stream) {
   MoeArgs p{(const uint8_t*)w_gu, w_scale, (const uint8_t*)x, x_scale, perm,
             (const int4*)tiles, n_tiles, choice_w, (const uint16_t*)bias, h,
-            topk, I, fp8 ? H : 2 * H, 0, in_w, gelu,
+            topk, I, fp8 ? H : 2 * H, 0, 0, I, in_w, gelu,
             limit};
   if (fp8)
     launch_gemm_tm<true>(tm, true, p, max_tiles, stream);
@@ -609,10 +618,11 @@ extern "C" void launch_moe_down(
     float* y, const void* h, const float* h_scale, const void* w_down,
     const float* w_scale, const int* perm, const void* tiles,
     const int* n_tiles, const float* choice_w, int topk, int H, int I,
-    int max_tiles, int tm, bool fp8, bool in_w, hipStream_t stream) {
+    int first, int cols, int max_tiles, int tm, bool fp8, bool in_w,
+    hipStream_t stream) {
   MoeArgs p{(const uint8_t*)w_down, w_scale, (const uint8_t*)h, h_scale, perm,
             (const int4*)tiles, n_tiles, choice_w, nullptr, y, topk, H,
-            fp8 ? I : 2 * I, 0, in_w, 0, 0.f};
+            fp8 ? I : 2 * I, 0, first, cols, in_w, 0, 0.f};
   if (fp8)
     launch_gemm_tm<true>(tm, false, p, max_tiles, stream);
   else
@@ -621,7 +631,9 @@ extern "C" void launch_moe_down(
 
 extern "C" void launch_moe_combine(float* out, const float* y,
                                    const int64_t* ids, int T, int k, int E,
-                                   int H, hipStream_t stream) {
-  dim3 grid(T, T < 256 ? ceil_div(H, 1024) : 1, 1);
-  moe_combine_kernel<<<grid, 256, 0, stream>>>(out, y, ids, T, k, E, H);
+                                   int H, int first, int cols,
+                                   hipStream_t stream) {
+  dim3 grid(T, T < 256 ? ceil_div(cols, 1024) : 1, 1);
+  moe_combine_kernel<<<grid, 256, 0, stream>>>(out, y, ids, T, k, E, H, first,
+                                               cols);
 }
