@@ -518,7 +518,6 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
   TORCH_CHECK(H % 32 == 0 && I % (fp8 ? 64 : 32) == 0,
               "MoE dims must be multiples of 32, fp8 I of 64 (H=", H, " I=", I,
               ")");
-  TORCH_CHECK(E <= 16384, "more than 16384 experts");
   TORCH_CHECK(bias_gu.numel() == 0 ||
               (bias_gu.scalar_type() == at::kBFloat16 &&
                bias_gu.is_contiguous() &&

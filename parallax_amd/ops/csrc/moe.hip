@@ -54,8 +54,27 @@ DEVINL void copy16_to_lds(const void* src, void* dst) {
 
 #define ROUTE_THREADS 1024
 #define ROUTE_PART 4096
+#define ROUTE_LDS 8192  // experts whose counters fit the LDS
 
-// cnt[e] += this part's choices of expert e; cnt is in LDS
+// The counters of more experts lie in memory and belong to one workgroup, which
+// goes by atomic operations only: plain ones may meet its own cache.
+template <bool LDS>
+DEVINL int get_count(const int* p) {
+  return LDS ? *p
+             : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool LDS>
+DEVINL void set_count(int* p, int v) {
+  if (LDS) *p = v;
+  else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool LDS>
+DEVINL void route_sync() {
+  if (!LDS) __threadfence();
+  __syncthreads();
+}
+
+// cnt[e] += this part's choices of expert e
 DEVINL void count_choices(int* cnt, const int64_t* ids, int begin, int end,
                           int E) {
   // ids are fetched four ahead of the counters, which would wait for each
@@ -86,12 +105,13 @@ __global__ __launch_bounds__(ROUTE_THREADS) void moe_count_kernel(
     counts[(size_t)blockIdx.x * E + e] = lds[e];
 }
 
+template <bool LDS>
 __global__ __launch_bounds__(ROUTE_THREADS) void moe_route_kernel(
     int* __restrict__ perm, int4* __restrict__ tiles, int* __restrict__ n_tiles,
-    const int* __restrict__ counts, const int64_t* __restrict__ ids,
+    int* __restrict__ counts, const int64_t* __restrict__ ids,
     const int n, const int E, const int tm) {
   extern __shared__ int lds[];
-  int* cur = lds;  // counters, then the next place of every expert
+  int* cur = LDS ? lds : counts;  // counters, then every expert's next place
   __shared__ int wave_rows[16], wave_tiles[16];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wid = tid >> 6;
@@ -99,10 +119,10 @@ __global__ __launch_bounds__(ROUTE_THREADS) void moe_route_kernel(
   const int begin = parts > 1 ? blockIdx.x * ROUTE_PART : 0;
   const int end = parts > 1 ? min(n, begin + ROUTE_PART) : n;
   if (parts == 1) {
-    for (int e = tid; e < E; e += ROUTE_THREADS) cur[e] = 0;
-    __syncthreads();
+    for (int e = tid; e < E; e += ROUTE_THREADS) set_count<LDS>(cur + e, 0);
+    route_sync<LDS>();
     count_choices(cur, ids, begin, end, E);
-    __syncthreads();
+    route_sync<LDS>();
   }
   // exclusive sums of rows and tiles over the experts, 1024 at a time
   int rows0 = 0, tiles0 = 0;
@@ -111,7 +131,7 @@ __global__ __launch_bounds__(ROUTE_THREADS) void moe_route_kernel(
     int c = 0, before = 0;
     if (e < E) {
       if (parts == 1) {
-        c = cur[e];
+        c = get_count<LDS>(cur + e);
       } else {
         for (int q = 0; q < parts; ++q) {
           const int v = counts[(size_t)q * E + e];
@@ -149,14 +169,14 @@ __global__ __launch_bounds__(ROUTE_THREADS) void moe_route_kernel(
     if (e < E) {
       const int r0 = rb + rs - c;
       int at = tb + ts - t;
-      cur[e] = r0 + before;
+      set_count<LDS>(cur + e, r0 + before);
       if (blockIdx.x == 0)
         for (int r = r0; r < r0 + c; r += tm)
           tiles[at++] = make_int4(e, r, r0 + c, 0);
     }
     rows0 += rsum;
     tiles0 += tsum;
-    __syncthreads();
+    route_sync<LDS>();
   }
   if (tid == 0 && blockIdx.x == 0) *n_tiles = tiles0;
   constexpr int AHEAD = ROUTE_PART / ROUTE_THREADS;
@@ -583,18 +603,27 @@ extern "C" int moe_down_cols(int n, int H) {
 }
 
 // ints of scratch that routing n choices takes besides perm and tiles
+static int route_parts(int n, int E) {
+  return n > 2 * ROUTE_PART && E <= ROUTE_LDS ? ceil_div(n, ROUTE_PART) : 1;
+}
 extern "C" int64_t moe_route_scratch(int n, int E) {
-  return n > 2 * ROUTE_PART ? (int64_t)ceil_div(n, ROUTE_PART) * E : 0;
+  const int parts = route_parts(n, E);
+  return parts > 1 || E > ROUTE_LDS ? (int64_t)parts * E : 0;
 }
 
 extern "C" void launch_moe_route(int* perm, void* tiles, int* n_tiles,
                                  int* counts, const int64_t* ids, int n, int E,
                                  int tm, hipStream_t stream) {
-  const int parts = n > 2 * ROUTE_PART ? ceil_div(n, ROUTE_PART) : 1;
+  const int parts = route_parts(n, E);
+  if (E > ROUTE_LDS) {
+    moe_route_kernel<false><<<1, ROUTE_THREADS, 0, stream>>>(
+        perm, (int4*)tiles, n_tiles, counts, ids, n, E, tm);
+    return;
+  }
   if (parts > 1)
     moe_count_kernel<<<parts, ROUTE_THREADS, E * sizeof(int), stream>>>(
         counts, ids, n, E);
-  moe_route_kernel<<<parts, ROUTE_THREADS, E * sizeof(int), stream>>>(
+  moe_route_kernel<true><<<parts, ROUTE_THREADS, E * sizeof(int), stream>>>(
       perm, (int4*)tiles, n_tiles, counts, ids, n, E, tm);
 }
 

@@ -255,3 +255,26 @@ def test_moe_many_choices_within_a_fixed_workspace(fp8):
     assert torch.cuda.max_memory_allocated() - before < (
         (256 << 20) + out.numel() * 4 + (32 << 20))
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("E", [8192, 8193, 20000])
+@pytest.mark.parametrize("T", [3, 70])
+def test_moe_many_experts(E, T):
+    """More experts than their counters have room in LDS; most are chosen by none,
+    some by many, the first and the last by some."""
+    g = torch.Generator(device="cuda").manual_seed(E)
+    H, I, k = 64, 32, 4
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    w_gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * 0.1).bfloat16()
+    w_dn = (torch.randn(E, H, I, generator=g, device="cuda") * 0.2).bfloat16()
+    ids = torch.randint(0, E, (T, k), generator=g, device="cuda")
+    ids[:, 0] = torch.tensor([0, E - 1, 5000], device="cuda").repeat(24)[:T]
+    ids[1, 2] = E
+    wts = torch.rand(T, k, generator=g, device="cuda")
+    out = ops.fused_moe_forward(x, w_gu, w_dn, ids, wts)
+    wts[1, 2], ids[1, 2] = 0, 0
+    used, local = ids.cpu().unique(return_inverse=True)
+    want = _cpu_moe(x.cpu(), w_gu[used.cuda()].cpu(), w_dn[used.cuda()].cpu(), local,
+                    wts.cpu())
+    # h is rounded to bf16: 2^-9 of sums of |h w| < 4 weights * 32 * |h| 3 * |w| 0.9
+    torch.testing.assert_close(out.cpu(), want, atol=0.05, rtol=1e-2)
