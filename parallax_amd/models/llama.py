@@ -154,7 +154,9 @@ class LlamaMLP(nn.Module):
         self.down_proj = RowParallelLinear(inter, cfg.hidden_size, bias=cfg.mlp_bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down_proj(self.gate_up_proj.silu_and_mul(x))
+        proj = self.gate_up_proj
+        fused = getattr(proj, "silu_and_mul", None)  # another module may stand there
+        return self.down_proj(fused(x) if fused else ops.silu_and_mul(proj(x)))
 
 
 class LlamaDecoderLayer(nn.Module):

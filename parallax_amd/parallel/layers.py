@@ -47,6 +47,14 @@ class _Fp8WeightMixin:
         return ops.linear(x, self.weight, getattr(self, "bias", None))
 
 
+def _plain_call(m: nn.Module, forward) -> bool:
+    """Whether calling m runs this forward and nothing else."""
+    g = nn.modules.module
+    return getattr(m.forward, "__func__", None) is forward and not (
+        m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks
+        or g._global_forward_pre_hooks)
+
+
 def _shard(dim_size: int, tp_size: int, tp_rank: int) -> tuple:
     """(start, size) of this rank's shard; dims that do not divide evenly are
     REPLICATED (e.g. odd vocab sizes in the lm_head) — the layer then behaves
@@ -138,9 +146,10 @@ class MergedColumnParallelLinear(nn.Module, _Fp8WeightMixin):
         return self._linear(x)
 
     def silu_and_mul(self, x: torch.Tensor) -> torch.Tensor:
-        """silu(first part) * second part, of two equal ones."""
-        if self.fp8:
-            return ops.silu_and_mul(self._linear(x))
+        """silu(first part) * second part, of two equal ones. Hooks and forwards of
+        others see the product itself, which the fused epilogue never stores."""
+        if self.fp8 or not _plain_call(self, MergedColumnParallelLinear.forward):
+            return ops.silu_and_mul(self(x))
         return ops.linear_silu_and_mul(x, self.weight, self.bias)
 
     def split_output(self, y: torch.Tensor) -> List[torch.Tensor]:
