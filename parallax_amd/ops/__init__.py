@@ -487,16 +487,8 @@ def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
     return out if done else None
 
 
-def linear(
-    x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None
-) -> torch.Tensor:
-    """F.linear: weight-streaming kernels for few rows (skinny_gemm.hip has the
-    sizes, with both sides measured), tuned hipBLASLt for the rest."""
-    if x.is_cuda:
-        out = _few_rows(x, weight, bias)
-        if out is not None:
-            return out
-    if (
+def _library_takes(x, weight):
+    return (
         LT_GEMM
         and x.is_cuda
         and x.dim() == 2
@@ -507,7 +499,26 @@ def linear(
         and weight.shape[0] % 8 == 0
         and weight.shape[1] % 8 == 0
         and (weight.shape[0], weight.shape[1]) not in _LT_REFUSED
+    )
+
+
+def linear(
+    x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None
+) -> torch.Tensor:
+    """F.linear: weight-streaming kernels for few rows (skinny_gemm.hip has the
+    sizes, with both sides measured), tuned hipBLASLt for the rest. Neither takes
+    part in autograd; operands that only torch's product takes otherwise (rows
+    apart, odd widths) are left to it where a gradient is asked for."""
+    if x.is_cuda and not (
+        torch.is_grad_enabled()
+        and (x.requires_grad or weight.requires_grad
+             or (bias is not None and bias.requires_grad))
+        and not _library_takes(x, weight)
     ):
+        out = _few_rows(x, weight, bias)
+        if out is not None:
+            return out
+    if _library_takes(x, weight):
         # tuned hipBLASLt: the default heuristic's decode-shape tile picks
         # are ~2.5x off the weight-streaming roofline (profiles/README.md);
         # first call per shape times the heuristic candidates (engine warmup,

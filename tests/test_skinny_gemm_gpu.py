@@ -80,6 +80,27 @@ def test_linear_of_rows_far_apart():
         atol=512 ** 2 * 2 ** -24)
 
 
+def test_linear_gradients():
+    """Rows apart and odd widths, which torch's product takes, have gradients."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for M, N, K, cut in ((6, 64, 128, True), (6, 68, 128, False)):
+        base = _rand(g, M, 2 * K if cut else K).bfloat16().requires_grad_()
+        w = _rand(g, N, K).bfloat16().requires_grad_()
+        b = _rand(g, N).bfloat16().requires_grad_()
+        y = ops.linear(base[:, :K], w, b)
+        y.float().sum().backward()
+        torch.testing.assert_close(b.grad.float(), torch.full((N,), float(M), device="cuda"))
+        torch.testing.assert_close(
+            base.grad[:, :K].float(),
+            w.detach().float().sum(0).expand(M, K), rtol=2 ** -7, atol=2 ** -7)
+        torch.testing.assert_close(
+            w.grad.float(), base.detach()[:, :K].float().sum(0).expand(N, K),
+            rtol=2 ** -7, atol=2 ** -7)
+        with torch.no_grad():
+            torch.testing.assert_close(ops.linear(base[:, :K], w, b).float(), y.float(),
+                                       rtol=2 ** -7, atol=2 ** -7)
+
+
 def test_linear_of_no_columns():
     """Refused by the kernels, whose deals of columns assume one."""
     ext = ops._require_ext("skinny_gemm")
