@@ -476,15 +476,10 @@ def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
         and (bias is None or bias.dtype == torch.bfloat16)
     ):
         return None
-    ext = _require_ext("skinny_gemm")
-    out = torch.empty(
-        x.shape[0], weight.shape[0] // (2 if gated else 1), dtype=torch.bfloat16,
-        device=x.device,
-    )
-    none = out.new_empty(0)
-    done = ext.skinny_gemm(out, x, weight, none if bias is None else bias,
-                           x_scale if fp8 else none, w_scale if fp8 else none, gated)
-    return out if done else None
+    ext = _require_ext("few_rows")
+    none = weight.new_empty(0, dtype=torch.bfloat16)
+    return ext.few_rows(x, weight, none if bias is None else bias,
+                        x_scale if fp8 else none, w_scale if fp8 else none, gated)
 
 
 def _library_takes(x, weight):

@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <optional>
 
 #define CHECK_GPU(x) TORCH_CHECK(x.is_cuda(), #x " must be on GPU")
 #define CHECK_CONTIG(x) TORCH_CHECK(x.is_contiguous(), #x " must be contiguous")
@@ -705,18 +706,22 @@ torch::Tensor sample_gumbel(torch::Tensor logits, torch::Tensor inv_temp,
 }
 
 // c = x . w^T (+ bias): bf16, or fp8 with the two scales given; gated: c = silu(first
-// half of the columns) * second half. False where there is no kernel.
-bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
-                 torch::Tensor bias, torch::Tensor x_scale, torch::Tensor w_scale,
-                 bool gated) {
+// half of the columns) * second half. False where there is no kernel; c is allocated
+// where it is not given, once there is one.
+static bool skinny_run(torch::Tensor& c, torch::Tensor x, torch::Tensor w,
+                       torch::Tensor bias, torch::Tensor x_scale,
+                       torch::Tensor w_scale, bool gated) {
   CHECK_GPU(x);
   const bool fp8 = x_scale.numel() > 0;
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) &&
-              x.stride(1) == 1 && c.dim() == 2 && c.stride(1) == 1 &&
-              c.size(0) == x.size(0) &&
-              c.size(1) * (gated ? 2 : 1) == w.size(0));
+              x.stride(1) == 1);
   CHECK_CONTIG(w);
-  CHECK_BF16(c);
+  if (c.defined()) {
+    TORCH_CHECK(c.dim() == 2 && c.stride(1) == 1 && c.size(0) == x.size(0) &&
+                c.size(1) * (gated ? 2 : 1) == w.size(0));
+    CHECK_BF16(c);
+    if ((uintptr_t)c.data_ptr() % 8 || c.stride(0) % 4) return false;
+  }
   if (fp8) {
     TORCH_CHECK(is_fp8(x) && is_fp8(w) &&
                 x_scale.scalar_type() == at::kFloat &&
@@ -735,7 +740,7 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
   // the kernels place rows of x by 32-bit offsets
   if ((x.size(0) - 1) * x.stride(0) * es + 128 > UINT32_MAX) return false;
   if ((uintptr_t)x.data_ptr() % 16 || (uintptr_t)w.data_ptr() % 16 ||
-      x.stride(0) * es % 16 || (uintptr_t)c.data_ptr() % 8 || c.stride(0) % 4)
+      x.stride(0) * es % 16)
     return false;
   const int M = x.size(0), N = w.size(0), row_bytes = x.size(1) * es;
   const void* b = bias.numel() ? bias.data_ptr() : nullptr;
@@ -745,6 +750,8 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
   if (gated && (N % 16 || (int64_t)N * row_bytes > UINT32_MAX)) return false;
   const int splits = skinny_shared(M, N, row_bytes);
   if (splits < 0) return false;
+  if (!c.defined())
+    c = torch::empty({M, gated ? N / 2 : N}, x.options().dtype(at::kBFloat16));
   if (splits > 0) {
     torch::Tensor part;
     if (splits > 1)
@@ -760,6 +767,21 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
                      row_bytes, x.stride(0) * es, c.stride(0), 1, 0, 0, gated,
                      cur_stream(), &launched);
   return launched;
+}
+
+bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
+                 torch::Tensor bias, torch::Tensor x_scale, torch::Tensor w_scale,
+                 bool gated) {
+  return skinny_run(c, x, w, bias, x_scale, w_scale, gated);
+}
+
+// the same with the result allocated; None where there is no kernel
+std::optional<torch::Tensor> few_rows(torch::Tensor x, torch::Tensor w,
+                                      torch::Tensor bias, torch::Tensor x_scale,
+                                      torch::Tensor w_scale, bool gated) {
+  torch::Tensor c;
+  if (!skinny_run(c, x, w, bias, x_scale, w_scale, gated)) return std::nullopt;
+  return c;
 }
 
 // x quantised per tensor: (fp8 values, scale [1])
@@ -862,6 +884,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "tuned hipBLASLt y = x @ w^T (bf16, fp32 accum)");
   m.def("msa_paged_attention_decode", &msa_paged_attention_decode);
   m.def("skinny_gemm", &skinny_gemm);
+  m.def("few_rows", &few_rows);
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);
   m.def("mla_absorb", &mla_absorb);
   m.def("mla_project", &mla_project);

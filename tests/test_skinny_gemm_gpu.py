@@ -101,6 +101,18 @@ def test_linear_gradients():
                                        rtol=2 ** -7, atol=2 ** -7)
 
 
+def test_linear_allocates_its_result_once():
+    """Also where no kernel for few rows takes the product."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    for M, N, K in ((96, 576, 7168), (33, 64, 64), (8, 900, 896)):
+        x, w = _rand(g, M, K).bfloat16(), _rand(g, N, K).bfloat16()
+        ops.linear(x, w)
+        n = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+        before = n()
+        y = ops.linear(x, w)
+        assert n() - before == 1 and y.shape == (M, N)
+
+
 def test_linear_of_no_columns():
     """Refused by the kernels, whose deals of columns assume one."""
     ext = ops._require_ext("skinny_gemm")
