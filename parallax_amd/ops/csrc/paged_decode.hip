@@ -328,12 +328,9 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
       const uint16_t* row = q + (size_t)seq * q_stride +
                             (size_t)(hk * G + min(l15, G - 1)) * D;
 #pragma unroll
-      for (int s = 0; s < KC; ++s) {
-        u32x4v v = *(const u32x4v*)(row + (FP8 ? ((s >> 1) * 4 + l4) * 16 + (s & 1) * 8
-                                              : s * 32 + l4 * 8));
-        if (scale < 0.f) v ^= 0x80008000u;  // the sign goes with q: c takes maxima
-        qf[s] = __builtin_bit_cast(bf16x8v, v);
-      }
+      for (int s = 0; s < KC; ++s)
+        qf[s] = *(const bf16x8v*)(row + (FP8 ? ((s >> 1) * 4 + l4) * 16 + (s & 1) * 8
+                                             : s * 32 + l4 * 8));
     }
     f32x4v o[MT] = {};
     float m = kLowest, l = 0.f;
@@ -383,6 +380,12 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
       issue_k(first, nx);
       issue_v(first, nx);
       pages(first + U, nx);
+      if (scale < 0.f) {  // the sign goes with q, as c takes maxima; with copies on
+#pragma unroll           // their way, because it waits for q
+        for (int s = 0; s < KC; ++s)
+          qf[s] = __builtin_bit_cast(
+              bf16x8v, __builtin_bit_cast(u32x4v, qf[s]) ^ 0x80008000u);
+      }
       for (int tok = first; tok < end; tok += U) {
         wait_copies<NC>();
         u32x4v kr[KC * ES];  // [chunk group][t]
