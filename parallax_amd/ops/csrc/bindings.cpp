@@ -91,6 +91,7 @@ void launch_skinny_gemm(void*, const void*, const void*, const void*,
                         const float*, const float*, bool, int, int, int, int64_t,
                         int64_t, int, int64_t, int64_t, bool, hipStream_t, bool*);
 int skinny_shared(int, int, int);
+bool skinny_pays(int, int, int);
 void launch_skinny_split(void*, float*, int, const void*, const void*, const void*,
                          const float*, const float*, bool, int, int, int, int64_t,
                          int64_t, bool, hipStream_t);
@@ -775,11 +776,14 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
   return skinny_run(c, x, w, bias, x_scale, w_scale, gated);
 }
 
-// the same with the result allocated; None where there is no kernel
+// the same with the result allocated; None where there is no kernel, or the library
+// is faster
 std::optional<torch::Tensor> few_rows(torch::Tensor x, torch::Tensor w,
                                       torch::Tensor bias, torch::Tensor x_scale,
                                       torch::Tensor w_scale, bool gated) {
   torch::Tensor c;
+  if (!gated && !skinny_pays(x.size(0), w.size(0), x.size(1) * x.element_size()))
+    return std::nullopt;
   if (!skinny_run(c, x, w, bias, x_scale, w_scale, gated)) return std::nullopt;
   return c;
 }

@@ -540,6 +540,24 @@ extern "C" int skinny_shared(int M, int N, int row_bytes) {
   return ragged || (M > 16 && (nt == 0 || bytes >= 1 << 26)) ? splits : 0;
 }
 
+// Whether a kernel above beats the library's tuned product, us of both. Short rows of
+// a tall W are over before a workgroup has its copies under way; only up to 6 rows
+// and from 17 to 32 do its tiles gain: 151936 x 896 with 4 / 8 / 16 / 24 / 72 / 112
+// rows 52 / 55 / 59 / 57 / 73 / 85 (54 / 55 / 55 / 57 / 69 / 76), 100352 x 1024 with
+// 16 / 112 46 / 65 (42 / 51); 40960 x 1024 17.7 / 24 (20 / 26) and 65536 x 2048 50 /
+// 63 (67 / 77). A K split over workgroups must be long, or W large, for its parts,
+// longer above 64 rows: 5120 x 2560 with 40 / 96 rows 14 / 17 (13 / 15), 3584 x 3584
+// 14 / 17 (12.5 / 16), 2560 x 4096 14 / 16 (12.5 / 13), 7168 x 2048 12.5 / 15 (13 /
+// 14); 4096 x 4096 12.6 / 16 (14 / 19), 1536 x 7168 12 / 14 (18 / 19). Not of the gated
+// form, which saves the activation's launch besides.
+extern "C" bool skinny_pays(int M, int N, int row_bytes) {
+  const bool tall = N > 40960 && row_bytes < 4096;
+  if (M <= 32) return !tall || M <= 6 || M > 16;
+  if (skinny_splits(N, row_bytes) == 1) return !tall;
+  const bool large = (int64_t)N * row_bytes >= 28000000;
+  return (large || row_bytes >= 14336) && row_bytes >= (M > 64 ? 7168 : 4096);
+}
+
 // batch products of the same shape: x, w and c advance by x_batch bytes, N rows
 // and c_batch elements. Any number of rows of X, 32 at a time.
 extern "C" void launch_skinny_gemm(

@@ -80,6 +80,26 @@ def test_linear_of_rows_far_apart():
         atol=512 ** 2 * 2 ** -24)
 
 
+@pytest.mark.parametrize("M,N,K,own", [
+    (6, 40964, 64, True), (7, 40964, 64, False), (16, 40964, 64, False),
+    (17, 40964, 64, True), (16, 40960, 64, True), (16, 40964, 2048, True),
+    (33, 40964, 64, False), (100, 40964, 2048, True),
+    (33, 5120, 2560, False), (64, 8192, 2048, True), (65, 8192, 2048, False),
+    (65, 4096, 3584, True), (40, 256, 7168, True), (40, 256, 4096, False),
+])
+def test_linear_takes_the_faster_side(M, N, K, own):
+    """Both sides of the lines between the kernels and the library agree."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x, w = _rand(g, M, K).bfloat16(), _rand(g, N, K).bfloat16()
+    ext = ops._require_ext("few_rows")
+    none = x.new_empty(0)
+    got = ext.few_rows(x, w, none, none, none, False)
+    assert (got is not None) == own
+    torch.testing.assert_close(
+        ops.linear(x, w).float(), x.float() @ w.float().t(), rtol=2 ** -8,
+        atol=K * K * 2 ** -24)
+
+
 def test_linear_gradients():
     """Rows apart and odd widths, which torch's product takes, have gradients."""
     g = torch.Generator(device="cuda").manual_seed(3)
