@@ -187,15 +187,21 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
     const int per = (kt_end - kt_begin + gridDim.y - 1) / gridDim.y;
     kt_begin += blockIdx.y * per;
     kt_end = min(kt_end, kt_begin + per);
-    if (kt_begin >= kt_end) {
-      if (half == 0 && item_ok) {
-        float* ml = tmp_ml +
-            (((size_t)(q0 + row) * Hq + h) * gridDim.y + blockIdx.y) * 2;
+  }
+  if (kt_begin >= kt_end) {  // no keys: nothing is looked up or copied
+    if (half == 0 && item_ok) {
+      const size_t at = (size_t)(q0 + row) * Hq + h;
+      if (tmp_acc != nullptr) {
+        float* ml = tmp_ml + (at * gridDim.y + blockIdx.y) * 2;
         ml[0] = kLowest;
         ml[1] = 0.f;
+      } else {  // a portion longer than its context: 0 / 0, 0 beside a sink
+        const uint32_t v = sinks != nullptr ? 0u : 0x7fc07fc0u;
+        for (int d = 0; d < D; d += 4)
+          *reinterpret_cast<uint2*>(out + at * D + d) = make_uint2(v, v);
       }
-      return;
     }
+    return;
   }
 
   // ---- Q as B operands: item l31, d = 16 s + 8 half + (0..7) -------------------
@@ -407,18 +413,14 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
     compute(kt, Kl, Vl);
     if (KV_FP8 && more) widen8(Kn, Vn);
   };
-  // a portion longer than its context has rows that see nothing, and pages that
-  // must not be looked up
-  if (kt_begin < kt_end) {
-    pages(kt_begin);
-    if (KV_FP8) {
-      fetch8(kt_begin);
-      widen8(K0, V0);
-    } else {
-      issue(kt_begin, K0, V0);
-    }
-    pages(kt_begin + 1);
+  pages(kt_begin);
+  if (KV_FP8) {
+    fetch8(kt_begin);
+    widen8(K0, V0);
+  } else {
+    issue(kt_begin, K0, V0);
   }
+  pages(kt_begin + 1);
   for (int kt = kt_begin; kt < kt_end; kt += 2) {
     turn(kt, K0, V0, K1, V1);
     if (kt + 1 < kt_end) turn(kt + 1, K1, V1, K0, V0);
