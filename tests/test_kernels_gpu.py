@@ -428,10 +428,36 @@ def test_paged_decode_units_runs_and_windows(D, BS, fp8, G, Hk, lens, kw):
     sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
     out = ops.paged_attention_decode(q, kc, vc, bt, sl, D ** -0.5, **kw)
     ks, vs = kw.pop("k_scale", 1.0), kw.pop("v_scale", 1.0)
-    some = [i for i in (set(range(13)) | {B - 2, B - 1}) if i < B and lens[i]]
+    some = [i for i in range(B) if lens[i]]
     want = ref.paged_attention_decode(
         q[some].float(), full_k * ks, full_v * vs, bt[some], sl[some], D ** -0.5, **kw)
     torch.testing.assert_close(out[some].float(), want.float(), atol=2.2e-2, rtol=0)
+
+
+@pytest.mark.parametrize("B,Hk,longest,max_seq_len", [
+    (5, 2, 300, 32768),      # a captured step's bucket: most runs have no unit
+    (37, 8, 900, 131072),
+    (3, 1, 100, 1025),
+    (100, 8, 2000, 2000),    # short contexts of many: a workgroup each
+    (100, 8, 2000, 2049),    # and the same dealt to runs
+    (33, 8, 1024, 1024),
+])
+@pytest.mark.parametrize("D,fp8", [(128, False), (64, True)])
+def test_paged_decode_ways_by_bucket(B, Hk, longest, max_seq_len, D, fp8):
+    """max_seq_len, not the lengths, decides how the work is dealt. Tolerance as
+    above."""
+    g = torch.Generator().manual_seed(B)
+    lens = torch.randint(1, longest + 1, (B,), generator=g).tolist()
+    kc, vc, bt = _make_paged_kv(B, Hk, D, 32, max(lens), seed=B)
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+    q = torch.randn(B, 4 * Hk, D, generator=g).bfloat16().cuda()
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = ops.paged_attention_decode(q, kc, vc, bt, sl, D ** -0.5,
+                                     max_seq_len=max_seq_len)
+    want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl,
+                                      D ** -0.5)
+    torch.testing.assert_close(out.float(), want, atol=2.2e-2, rtol=0)
 
 
 @pytest.mark.parametrize("scale", [-0.125, 0.0, 1e-25])
