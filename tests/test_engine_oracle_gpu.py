@@ -186,6 +186,26 @@ def test_gpu_engine_matches_cpu_fp32_engine(family):
     assert all(len(v) == 4 for v in out_gpu.values())
 
 
+@pytest.mark.parametrize("family,window", [("gpt_oss", 32), ("gpt_oss", 128),
+                                           ("step3p5", 32)])
+def test_prompts_past_the_window(family, window):
+    """Windowed layers of 64-wide heads on prompts of several windows: rows that see
+    nothing of the first keys their wave looks at."""
+    d = dict(FAMILIES[family], sliding_window=window)
+    prompts = [[(7 * i + 3) % 500 for i in range(300)], [(i * i) % 487 for i in range(193)]]
+    sp = [SamplingParams(temperature=0.0, max_new_tokens=2, ignore_eos=True)] * 2
+    logits = []
+    for device_gpu in (False, True):
+        torch.manual_seed(0)
+        eng = _build(d, device_gpu)
+        with _LogitTap(eng.sampler) as tap:
+            eng.generate([list(p) for p in prompts], sp)
+        logits.append(tap.logits)
+    assert bool(logits[1].isfinite().all())
+    rel = (logits[0] - logits[1]).norm() / logits[0].norm()
+    assert rel < 0.10, f"{family}: prefill logits rel err {rel:.3f}"
+
+
 def test_kimi_k2_256k_prefix_reuse_smoke():
     """BASELINE config 5 at reduced depth: Kimi-K2 architecture class (MLA
     512/64, 384 routed experts, sigmoid routing) with ONE layer and 16 heads,
