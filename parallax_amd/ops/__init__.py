@@ -569,7 +569,8 @@ def linear_fp8(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor,
         y = torch.nn.functional.linear(x.float(), w).to(x.dtype)
         return y if bias is None else y + bias
     ext = _require_ext("lt_linear_fp8")
-    _, _ = x.shape
+    if x.dim() != 2:
+        raise ValueError(f"linear_fp8 takes rows [M, K], not {tuple(x.shape)}")
     xq, xs = ext.quantize_fp8_tensor(
         (x if x.dtype == torch.bfloat16 else x.float()).contiguous())
     out = _few_rows(xq, w_q, bias, xs, w_scale)

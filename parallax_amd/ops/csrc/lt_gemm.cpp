@@ -284,10 +284,11 @@ torch::Tensor lt_linear(torch::Tensor x, torch::Tensor w) {
   return y;
 }
 
-// fp8-E4M3 W8A8 GEMM (BASELINE DeepSeek-V3 "fp8 MFMA" dense route):
+// fp8-E4M3 W8A8 GEMM (the dense products of a DeepSeek-V3 in fp8):
 // y[M,N] bf16 = (x_q[M,K] * sx) . (w_q[N,K] * sw)^T with per-tensor DEVICE
-// scale pointers (hipblaslt reads them at kernel time, so graph capture
-// bakes only the persistent buffer addresses the caller guarantees).
+// scale pointers, read at kernel time. Under graph capture x_q, its scale and the
+// result live in the capturing graph's memory pool, which keeps their addresses
+// for every replay.
 torch::Tensor lt_linear_fp8(torch::Tensor x_q, torch::Tensor w_q,
                             torch::Tensor x_scale, torch::Tensor w_scale) {
   TORCH_CHECK(x_q.is_cuda() && w_q.is_cuda());

@@ -21,9 +21,9 @@
 // others the runs leave fp32 parts that a second kernel adds up. Short contexts
 // take a workgroup a sequence and head, of more waves where there are few.
 //
-// What bounds it: large batches the cache's stream, 128 x 8 heads x 128 of 4,096
-// tokens 251 us or 5.5 TB/s (before, barriers in every tile and fixed partitions:
-// 272); 64-wide fp8 heads the instructions of a tile beside its few bytes, 200 x 8
+// What bounds it: large batches the cache's stream, 128 x 8 heads x 128 of 1,024 to
+// 4,096 tokens (1.39 GB) 253 us or 5.5 TB/s (before, barriers in every tile and
+// fixed partitions: 272); 64-wide fp8 heads the instructions of a tile beside its few bytes, 200 x 8
 // of 3,001 87 us (196); one sequence two round trips and the launches, 8 heads of
 // 1,000 9.4 us (11.8), of 32,000 34 us (84).
 //

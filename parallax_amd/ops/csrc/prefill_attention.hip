@@ -25,7 +25,7 @@
 // window or the end of the sequence cuts.
 //
 // Measured (MI355X, bf16, 32 heads over 8 of 128, 8192 rows in two portions on
-// prefixes of up to 20,000): 3.59 ms = 851 TFLOP/s of what the mask leaves;
+// prefixes of up to 20,000): 3.5 ms = 870 TFLOP/s of what the mask leaves;
 // 16.6 ms with 32-row tiles of one head, P through LDS and six barriers a tile.
 
 #include "common.h"
