@@ -118,6 +118,12 @@ static bool is_fp8(const torch::Tensor& t) {
   return t.scalar_type() == at::kFloat8_e4m3fn;
 }
 
+// Kernels that copy memory to LDS directly take 16 bytes from multiples of 16. A
+// tensor that begins elsewhere (a view at an odd offset) is copied to one that does.
+static torch::Tensor from16(const torch::Tensor& t) {
+  return (uintptr_t)t.data_ptr() % 16 ? t.clone() : t;
+}
+
 static int64_t row_stride(const torch::Tensor& t, const char* name) {
   TORCH_CHECK(t.dim() == 3 && t.stride(2) == 1 && t.stride(1) == t.size(2),
               name, " must be [T, H, D] with dense inner dims");
@@ -284,6 +290,8 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   bool launched = false;
   if (!use_valu || kv_fp8) {
     if (B == 0) return;
+    k_cache = from16(k_cache);
+    v_cache = from16(v_cache);
     // every part of a sequence is named by (run + sequence); see the kernel
     const int runs = paged_decode_runs(B, Hk, D, (int)max_seq_len,
                                        (int)sliding_window);
@@ -358,6 +366,8 @@ void prefill_attention(torch::Tensor out, torch::Tensor q,
   const int max_blocks = block_tables.size(1);
   TORCH_CHECK(D == 128 || D == 64, "head_dim must be 64 or 128");
   if (T == 0 || B == 0) return;
+  k_cache = from16(k_cache);
+  v_cache = from16(v_cache);
 
   const float* sinks_ptr = nullptr;
   torch::Tensor sinks_f;
@@ -437,6 +447,7 @@ void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,
     ml_ptr = tmp_ml.data_ptr<float>();
   }
   if (B == 0) return;
+  cache = from16(cache);
   bool launched = false;
   launch_mla_paged_attention_decode(
       out.data_ptr(), q_latent.data_ptr(), q_pe.data_ptr(), cache.data_ptr(),
@@ -527,6 +538,9 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
   auto fopts = x.options().dtype(at::kFloat);
   auto bopts = x.options().dtype(at::kByte);
   if (n == 0) return torch::zeros({T, H}, fopts);
+  x = from16(x);
+  w_gu = from16(w_gu);
+  w_down = from16(w_down);
   auto stream = cur_stream();
 
   const int tm = moe_tile_rows(n, E, I, fp8);
