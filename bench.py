@@ -1,6 +1,6 @@
 """Flagship benchmark: continuous-batching decode throughput (output tokens/s)
 of DeepSeek-R1-Distill-Llama-8B (Llama-3.1-8B architecture), bf16, synthetic
-data, random-init weights — the BASELINE.json PP=1 headline config.
+data, random-init weights, one pipeline stage.
 
 Single GPU by default. With --gpus N (launched via torch.distributed.run, one
 rank per GPU) the model runs pipeline-parallel over N stages with the global
@@ -119,7 +119,7 @@ def deepseek_v3() -> dict:
 
 def kimi_k2() -> dict:
     """Kimi-K2 (1T MoE): DeepSeek-V3 architecture class with 384 routed
-    experts — the BASELINE prefix-reuse config (Kimi-K2 PP=8 @ 256k ctx)."""
+    experts — the prefix-reuse config (8 pipeline stages, 256k context)."""
     cfg = deepseek_v3()
     cfg.update({
         "architectures": ["KimiK2ForCausalLM"],
@@ -564,7 +564,7 @@ def main():
     ap.add_argument("--model", default="deepseek-r1-distill-llama-8b", choices=MODELS)
     ap.add_argument("--batch-per-gpu", type=int, default=1024,
                     help="decode batch per GPU (global batch = N * this). "
-                         "Measured sweep (profiles/README.md round 2): 128 -> "
+                         "Measured sweep (profiles/README.md): 128 -> "
                          "15.6k tok/s @ 574 ms TTFT, 512 -> 27.1k @ 1.7 s, "
                          "1024 -> 31.1k @ 3.2 s, 2048 -> 33.5k @ 6.3 s; 1024 "
                          "is the default throughput/latency point")
@@ -576,15 +576,15 @@ def main():
     ap.add_argument("--weight-dtype", default="auto",
                     choices=["auto", "bf16", "fp8"],
                     help="auto: fp8 W8A8 expert weights for the MoE configs "
-                         "whose BASELINE entry names fp8 (deepseek-v3, "
+                         "that are quoted in fp8 (deepseek-v3, "
                          "kimi-k2), bf16 otherwise")
     ap.add_argument("--parallelism", default="auto", choices=["auto", "dp", "pp"],
                     help="auto: DP replicas when the model fits one GPU "
                          "(288 GB HBM3E), PP layer split otherwise")
     ap.add_argument("--shared-prefix", type=int, default=0,
                     help="tokens of prompt shared across all requests "
-                         "(exercises block-radix prefix reuse; BASELINE "
-                         "Kimi-K2 config)")
+                         "(exercises block-radix prefix reuse, as the "
+                         "Kimi-K2 config does)")
     ap.add_argument("--layers", type=int, default=0,
                     help="override num_hidden_layers (reduced-layer single-GPU "
                          "runs of the PP=8 configs; headline runs use 0 = full)")
@@ -677,7 +677,7 @@ def main():
         wdtype = "fp8" if args.model in ("deepseek-v3", "kimi-k2") and use_gpu else "bf16"
     if wdtype == "fp8":
         eargs.moe_weight_dtype = "fp8"
-        eargs.linear_weight_dtype = "fp8"   # dense GEMM route too (BASELINE)
+        eargs.linear_weight_dtype = "fp8"   # dense GEMM route too
     engine = Engine(cfg, eargs, comm=comm, random_weights=True)
     if use_gpu:
         # pre-tune hipBLASLt algo picks for the Ms this run will see:

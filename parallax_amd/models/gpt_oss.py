@@ -26,7 +26,7 @@ class GptOssMoE(nn.Module):
 
     GPU path: the grouped-GEMM MoE kernel (deinterleaved [E, 2I, H] layout
     built at load time) with the gate/up BIAS folded into the kernel epilogue
-    and the down bias added as a capture-safe torch gather — the round-1
+    and the down bias added as a capture-safe torch gather — an earlier
     per-expert torch loop used torch.unique, which is illegal inside hipGraph
     capture and serialized experts on the host."""
 

@@ -180,7 +180,7 @@ class FusedMoE(nn.Module):
 
     def quantize_fp8(self) -> None:
         """Convert expert weights to fp8-E4M3 with per-output-channel dequant
-        scales — the BASELINE DeepSeek-V3 "fp8 MFMA" configuration. The GPU
+        scales, as DeepSeek-V3 runs in fp8. The GPU
         path then runs the fp8 grouped-GEMM kernels (ops.fused_moe_forward_fp8)
         with per-token activation quantization; the CPU fallback dequantizes.
         Quantization is chunked over experts to bound the fp32 temporary."""

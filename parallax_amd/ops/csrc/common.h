@@ -119,7 +119,7 @@ typedef float f32x2v __attribute__((ext_vector_type(2)));
 // 8 fp8-E4M3 bytes -> 8 bf16 (scaled): packed HW converts
 // (v_cvt_pk_f32_fp8 on dword halves) instead of 8 byte-extract + scalar
 // convert chains — the fp8-KV fragment-load path was VALU-bound on the
-// scalar version (profiles/README.md round 2 fp8-KV note).
+// scalar version.
 DEVINL void fp8x8_to_bf16x8(uint64_t raw, float scale, uint16_t* out8) {
   const uint32_t lo = (uint32_t)raw;
   const uint32_t hi = (uint32_t)(raw >> 32);

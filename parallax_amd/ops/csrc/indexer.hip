@@ -5,7 +5,7 @@
 // context tokens the sparse decode kernels attend to. At 256k context the
 // score pass streams the whole index/K cache, so these are written as real
 // CDNA4 kernels (MFMA for the DSA q.k scores, coalesced streaming reduction
-// for the MSA block pool) instead of the round-1 torch compositions.
+// for the MSA block pool) instead of torch compositions.
 //
 //   dsa_indexer_scores: score[t] = sum_h w[h] * relu(q[h] . k[t])  (shared
 //     keys across heads, DeepSeek-V3.2 geometry: Hi<=64, Di=128). One

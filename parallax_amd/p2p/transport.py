@@ -3,8 +3,7 @@
 Reference analogue: Lattica (libp2p RPC) in p2p/server.py. Fresh design with
 two implementations behind one interface:
 - LoopbackTransport: in-process queues — the reference's own test strategy
-  ("loopback in-process transport so N-stage pipelines are
-  testable in one process").
+  (N-stage pipelines are testable in one process).
 - TcpTransport: length-prefixed msgpack frames over TCP sockets between hosts
   (offline environment: no libp2p; NAT traversal is out of scope, peers
   address each other host:port as assigned by the scheduler service).

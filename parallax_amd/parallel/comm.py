@@ -1,7 +1,7 @@
 """Distributed communication context: RCCL over xGMI (single host), gloo for
 CPU tests.
 
-MI355X-first design (SURVEY.md §2.5): one process per GPU; the world is laid out
+MI355X-first design: one process per GPU; the world is laid out
 as pp_size x tp_size with rank = pp_rank * tp_size + tp_rank. Pipeline
 hidden-state transport is torch.distributed send/recv (RCCL point-to-point over
 xGMI; ~153 GB/s per link); the async variants (pp_irecv/pp_send_async) ride the

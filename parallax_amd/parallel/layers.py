@@ -5,7 +5,7 @@ Column-parallel: weight is split on the output dim, no communication on forward
 weight split on the input dim; forward ends with a TP all-reduce. At tp_size=1
 these are plain GEMMs through hipBLASLt (torch.nn.functional.linear).
 Mirrors the capability of the reference's shard_linear / SGLang TP layers
-(SURVEY.md §2.3 TP row) as a fresh design.
+as a fresh design.
 """
 
 from __future__ import annotations
@@ -22,7 +22,7 @@ from .. import ops
 
 class _Fp8WeightMixin:
     """Per-tensor fp8-E4M3 weight storage for the hipBLASLt W8A8 route
-    (BASELINE DeepSeek-V3 fp8 config). quantize_fp8() swaps the bf16 weight
+    (DeepSeek-V3 in fp8). quantize_fp8() swaps the bf16 weight
     parameter for an fp8 buffer + device scale; forward then dispatches
     ops.linear_fp8 (activations quantize per-call on device)."""
 

@@ -4,7 +4,7 @@ Design: SPMD replicated scheduling. Every pipeline stage runs an identical
 continuous-batching scheduler on identical request state; only hidden states
 move point-to-point (RCCL send/recv over xGMI) and sampled tokens are broadcast
 once per step. This removes the reference's per-hop serialize+RPC cost
-(SURVEY.md §3.3 — decode pays a Lattica RPC of (1, hidden) per token per hop)
+(decode pays a Lattica RPC of (1, hidden) per token per hop)
 for the in-host path; the packet-driven peer executor (p2p/) remains the
 multi-host path.
 

@@ -75,7 +75,7 @@ class EngineServer:
         self.step_ms_ewma: Optional[float] = None
         self.last_batch_tokens = 0
         self.tps_ewma: Optional[float] = None  # output tokens/s over steps
-        # on-demand tracing (SURVEY §5: the reference has no tracer; here a
+        # on-demand tracing (the reference has no tracer; here a
         # chrome trace of the live step loop is one POST /profile away)
         self._profile_req: Optional[tuple] = None  # (steps, path)
         self._profiler = None

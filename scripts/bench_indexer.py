@@ -1,5 +1,4 @@
-"""Microbench: DSA indexer score pass at long context (VERDICT item 5's
-128k-ctx datapoint). Compares the HIP MFMA kernel against the batched torch
+"""Microbench: DSA indexer score pass at long context (128k tokens). Compares the HIP MFMA kernel against the batched torch
 composition it replaced and reports effective index-cache stream bandwidth.
 
 Run on a GPU box:  python scripts/bench_indexer.py [--ctx 131072] [--batch 4]

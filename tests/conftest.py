@@ -4,7 +4,7 @@ import torch
 
 def pytest_configure(config):
     config.addinivalue_line(
-        "markers", "gpu: needs a ROCm GPU (run on an MI355X box via gpurun)"
+        "markers", "gpu: needs a ROCm GPU (run on an MI355X)"
     )
 
 

@@ -1,6 +1,6 @@
 """Allocator / radix prefix cache / cache-manager unit tests (CPU).
 
-Test strategy mirrors the reference's cache tests (SURVEY.md §4): pure
+Test strategy mirrors the reference's cache tests: pure
 bookkeeping, no tensors needed.
 """
 

@@ -1,5 +1,5 @@
 """json_schema constrained decoding: FSM unit tests + engine conformance on
-the synthetic tokenizer (VERDICT item 8; reference carries json_schema on
+the synthetic tokenizer (reference carries json_schema on
 SamplingParams, sampling/sampling_params.py:25)."""
 
 import json

@@ -108,7 +108,7 @@ def test_greedy_parity_chunked(tiny_dsv3):
 
 def test_mla_prefix_cache_reuse(tiny_dsv3):
     """Kimi-K2-style prefix reuse: shared-prefix requests hit the block-radix
-    cache over the compressed MLA latent cache (BASELINE config 5 behavior)."""
+    cache over the compressed MLA latent cache."""
     hf, cfg = tiny_dsv3
     eng = Engine(cfg, EngineArgs(block_size=8, num_kv_blocks=256,
                                  dtype=torch.float32))

@@ -8,8 +8,8 @@ async pipelining envelope must preserve the engine's resource invariants:
   disabled so retention is not expected);
 - no requests remain running/waiting and no deferred frees are stranded.
 
-(The reference relies on architecture for concurrency safety — SURVEY §5
-"race detection: none"; this fuzz is the equivalent safety net here.)
+(The reference relies on architecture for concurrency safety
+and has no race detection; this fuzz is the equivalent safety net here.)
 """
 
 import pytest

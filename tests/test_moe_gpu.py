@@ -103,7 +103,7 @@ def test_moe_forward_fp8(T, E, k, H, I):
 
 def test_moe_fp8_engine_decode():
     """DeepSeek-V3-class engine with fp8 expert weights decodes through the
-    graph-captured path (BASELINE fp8 MFMA config, reduced layer count)."""
+    graph-captured path (reduced layer count)."""
     from parallax_amd.models.config import ModelConfig
     from parallax_amd.server.engine import Engine, EngineArgs
     from parallax_amd.server.sampling_params import SamplingParams

@@ -253,7 +253,7 @@ def test_tcp_transport_many_frames_in_order():
 
 def test_tcp_auth_handshake():
     """Auth-token transports accept matching peers and drop mismatched or
-    unauthenticated connections (VERDICT weak #8)."""
+    unauthenticated connections."""
     import time as _time
 
     from parallax_amd.p2p.transport import TcpTransport

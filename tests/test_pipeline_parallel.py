@@ -152,7 +152,7 @@ def _pp4_counter_worker(rank, world, port, out_file):
 
 
 def test_pp4_decode_path_is_object_free(tmp_path):
-    """steady-state PP decode must not pickle host objects —
+    """Steady-state PP decode must not pickle host objects —
     the only payload broadcast is the one carrying the initial adds."""
     from parallax_amd.parallel import comm as comm_mod
     from parallax_amd.server.engine import Engine, EngineArgs

@@ -108,7 +108,7 @@ class FixedCapNode(Node):
 
 
 def test_dp_allocator_finds_interleaved_partition():
-    """a heterogeneous pool where greedy/round-robin grouping
+    """A heterogeneous pool where greedy/round-robin grouping
     cannot form two pipelines but the memoized dp(i, open_residuals, finished)
     search can. Capacities (40,35,30,30,25,20) over 90 layers: the only
     2-pipeline partition is {40,30,20} + {35,30,25}; round-robin over the

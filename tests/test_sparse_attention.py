@@ -1,5 +1,5 @@
 """DSA / MSA sparse attention: CPU reference semantics + GPU kernels vs
-reference (the reference's dsa/msa kernel test coverage, SURVEY.md §2.2)."""
+reference (the reference's dsa/msa kernel test coverage)."""
 
 import math
 
@@ -190,8 +190,7 @@ def test_msa_kernel_gpu_per_head_positions():
 
 @pytest.mark.gpu
 def test_dsa_indexer_scores_kernel_gpu():
-    """HIP MFMA indexer score pass vs the fp32 torch reference (VERDICT item
-    5; reference Metal analogue dsa_indexer.metal)."""
+    """HIP MFMA indexer score pass vs the fp32 torch reference (reference Metal analogue dsa_indexer.metal)."""
     torch.manual_seed(0)
     B, Hi, Di, bs = 3, 64, 128, 32
     seq_lens = torch.tensor([70, 128, 15], dtype=torch.int32, device="cuda")

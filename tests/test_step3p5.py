@@ -1,4 +1,4 @@
-"""Step-3.5 architecture coverage (VERDICT item 9). No offline HF oracle
+"""Step-3.5 architecture coverage. No offline HF oracle
 exists (transformers 5.15 has no step3p5), so coverage is: config derivation,
 determinism, head-gate effectiveness, sliding-window layer interleave, and
 chunked-prefill / decode consistency against the model's own full-prefill

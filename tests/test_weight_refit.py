@@ -117,7 +117,7 @@ def test_http_update_weights_endpoint(tmp_path):
         server.stop()
 
 
-# -- chunked refit distribution over the P2P transport (VERDICT item 7; reference
+# -- chunked refit distribution over the P2P transport (reference
 #    p2p/server.py:224-338 CID-checksummed block store + 3-version GC) -----------
 
 
