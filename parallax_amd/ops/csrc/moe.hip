@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #define MOE_BKB 128    // bytes of the contraction a stage
+#define MOE_UNIT (256 * MOE_BKB)
 
 typedef float f32x16v __attribute__((ext_vector_type(16)));
 typedef int i32x4v __attribute__((ext_vector_type(4)));
@@ -36,10 +37,22 @@ DEVINL uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, p);
 }
 
-DEVINL void copy16_to_lds(const void* src, void* dst) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void*)src,
-      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+// 16 bytes a lane from memory to LDS, at + 16 lane. In assembly, without a register
+// of its own: of the builtin the compiler knows that it writes LDS, and where the
+// places rotate it waits for every copy in flight once a loop's turn before it reads.
+DEVINL void copy16(const void* src, uint32_t at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               :: "v"(src), "s"(at) : "m0", "memory");
+}
+// The same from a uniform base: no address arithmetic a lane.
+DEVINL void copy16(const uint8_t* base, uint32_t off, uint32_t at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(base), "s"(at) : "m0", "memory");
+}
+
+DEVINL uint32_t lds_address(const void* p) {
+  return __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
 }
 
 }  // namespace
@@ -195,24 +208,18 @@ __global__ __launch_bounds__(ROUTE_THREADS) void moe_route_kernel(
 }
 
 // ---- grouped GEMM ----------------------------------------------------------------
-// A workgroup takes one tile of TM rows of one expert and TN of its weight
+// A workgroup takes one tile of TM rows of one expert and 128 of its weight
 // rows: D[feature x row] = W . A^T on 32x32 matrix instructions, so that a lane
 // ends with four neighbouring features of one row. Both operands go global ->
 // LDS directly (16 bytes a lane, STAGES - 1 stages of 128 bytes of every row in
 // flight), 16-byte chunks XOR-swizzled by row so that 16 rows of one chunk
 // column lie in 16 bank groups.
-//   TM 32, 64: the weights' stream is the work. 4 waves x 32 weight rows.
-//   TM 128:    matrix products, 256 weight rows: 4 x 2 waves of 64 x 64.
+// TM 32 or 64: the weights' stream is the work. 4 waves x 32 weight rows.
 // GATE: of 32 weight rows of a wave 16 are gate and 16 the up rows of the same
 // columns; the accumulator's upper registers are the lower ones' partners.
-// What bounds it: few rows, the weights' stream: 256 fp8 experts of 7168 x 2048,
-// 200 tokens x 8 choices, gate/up 0.99 ms and down 0.55 ms = 6.2 TB/s of the
-// experts touched (2.44 and 1.06 ms with fragments loaded straight to
-// registers). Many rows, the address unit: it moves 64 bytes a cycle and CU, so
-// a 128 x 256 tile takes 768 of its cycles for 1024 of the matrix cores (128 x
-// 128: 512 for 512), and copies asked for in one burst hold their wave up: they
-// are spread over the products. 128 bf16 experts of 2048 x 768, 8192 tokens x 8:
-// gate/up 585 us = 705 TFLOP/s, down 450 us in two slabs (2247 and 1530 us before).
+// What bounds it: the weights' stream. 128 bf16 experts of 2048 x 768, 24 tokens x 8
+// choices: a whole call 123 us, 126 where the compiler waited for every copy in flight
+// once in STAGES stages (see copy16).
 
 struct MoeArgs {
   const uint8_t* w;        // [E, w_rows, kb] bytes
@@ -231,9 +238,87 @@ struct MoeArgs {
   float limit;             // > 0: clamped activation
 };
 
-template <bool FP8, int TN, int TM, bool GATE, int STAGES>
-__global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
-  constexpr int WN = TM == 128 ? 2 : 1;  // 32-row weight tiles a wave
+// ---- results: column = row of the tile, registers = features ----------------------
+// A wave's 32 WN weight rows from wb on.
+template <bool FP8, bool GATE, int WN, int WM>
+DEVINL void store_results(const MoeArgs& p, const f32x16v (&acc)[WN][WM],
+                          const int e, const int row0, const int rows_end,
+                          const int n0, const int wb) {
+  const int half = (threadIdx.x >> 5) & 1, l31 = threadIdx.x & 31;
+#pragma unroll
+  for (int j = 0; j < WM; ++j) {
+    const int r = row0 + j * 32 + l31;
+    if (r >= rows_end) continue;
+    const int choice = p.perm[r];
+    const float w = p.choice_w[choice];
+    const float sa = FP8 ? p.a_scale[GATE ? choice / p.topk : r] : 1.f;
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+      if (GATE) {
+        uint16_t* h = (uint16_t*)p.out + (size_t)r * p.N;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int f = n0 + (wb >> 1) + i * 16 + 8 * q + 4 * half;
+          if (f >= p.N) continue;
+          float v[4];
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            float g = acc[i][j][4 * q + s], u = acc[i][j][8 + 4 * q + s];
+            if (FP8) {
+              const float* ws = p.w_scale + (size_t)e * 2 * p.N + f + s;
+              g *= sa * ws[0];
+              u *= sa * ws[p.N];
+            }
+            if (p.in_w) {
+              g *= w;
+              u *= w;
+            }
+            if (p.bias != nullptr) {
+              const uint16_t* b = p.bias + (size_t)e * 2 * p.N + f + s;
+              g += bf16_bits_to_f32(b[0]);
+              u += bf16_bits_to_f32(b[p.N]);
+            }
+            if (p.limit > 0.f) {  // gpt-oss clamped act
+              g = fminf(g, p.limit);
+              u = fminf(fmaxf(u, -p.limit), p.limit);
+              v[s] = (u + 1.f) * (g / (1.f + __expf(-g * 1.702f)));
+            } else if (p.gelu) {
+              const float c = 0.7978845608028654f;
+              v[s] =
+                  0.5f * g * (1.f + tanhf(c * (g + 0.044715f * g * g * g))) * u;
+            } else {
+              v[s] = g / (1.f + __expf(-g)) * u;
+            }
+          }
+          uint2 o;
+          o.x = pack_bf16(v[0], v[1]);
+          o.y = pack_bf16(v[2], v[3]);
+          *reinterpret_cast<uint2*>(h + f) = o;
+        }
+      } else {
+        float* y = (float*)p.out + (size_t)choice * p.cols - p.first;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int f = n0 + wb + i * 32 + 8 * q + 4 * half;
+          if (f >= p.first + p.cols) continue;
+          f32x4v o;
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            float c = p.in_w ? 1.f : w;
+            if (FP8) c *= sa * p.w_scale[(size_t)e * p.N + f + s];
+            o[s] = acc[i][j][4 * q + s] * c;
+          }
+          *reinterpret_cast<f32x4v*>(y + f) = o;
+        }
+      }
+    }
+  }
+}
+
+template <bool FP8, int TM, bool GATE, int STAGES>
+__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeArgs p) {
+  constexpr int TN = 128;
+  constexpr int WN = 1;                   // 32-row weight tiles a wave
   constexpr int WM = TM == 32 ? 1 : 2;   // 32-row activation tiles a wave
   constexpr int PASS = TN / 4;            // rows the threads copy at once
   constexpr int APASS = TM / PASS;
@@ -286,10 +371,10 @@ __global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
   // copy i of a stage: 4 passes over the weight rows, then the activation rows
   auto copy = [&](int i, int off, uint8_t* S) {
     if (i < 4)
-      copy16_to_lds(wp[i] + off, S + (i * PASS + wid * 8) * MOE_BKB);
+      copy16(wp[i] + off, lds_address(S + (i * PASS + wid * 8) * MOE_BKB));
     else
-      copy16_to_lds(ap[i - 4] + off,
-                    S + (TN + (i - 4) * PASS + wid * 8) * MOE_BKB);
+      copy16(ap[i - 4] + off,
+             lds_address(S + (TN + (i - 4) * PASS + wid * 8) * MOE_BKB));
   };
   auto offset = [&](int kt) {
     return min(kt * MOE_BKB + src * 16, p.kb - 16);
@@ -300,9 +385,7 @@ __global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
     for (int i = 0; i < LOADS; ++i) copy(i, off, S);
   };
 
-  // waves: TM 128: TN / 64 x 2 of 64 x 64; else TN / 32 x 1 of 32 x TM
-  const int wb = TM == 128 ? (wid & (TN / 64 - 1)) * 64 : wid * 32;
-  const int ab = TM == 128 ? wid / (TN / 64) * 64 : 0;
+  const int wb = wid * 32;  // a wave takes 32 weight rows and all TM rows
   const int swz_l = (l31 >> 1) & 7;
   using frag_t = std::conditional_t<FP8, i32x8v, bf16x8v>;
   f32x16v acc[WN][WM] = {};
@@ -312,7 +395,7 @@ __global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
     constexpr bool FULL = decltype(full)::value;
     constexpr int KS = FP8 ? 2 : 4;
     const uint8_t* Wl = S + (wb + l31) * MOE_BKB;
-    const uint8_t* Al = S + (TN + ab + l31) * MOE_BKB;
+    const uint8_t* Al = S + (TN + l31) * MOE_BKB;
     frag_t a[2][WN], b[2][WM];
     auto fetch = [&](int ks) {
 #pragma unroll
@@ -415,77 +498,408 @@ __global__ __launch_bounds__(2 * TN, 2) void moe_gemm_kernel(const MoeArgs p) {
           std::false_type{}, [](int) {});
   }
 
-  // ---- results: column = row of the tile, registers = features --------------------
+  store_results<FP8, GATE>(p, acc, e, row0, rows_end, n0, wb);
+}
+
+// ---- many rows -----------------------------------------------------------------
+// A workgroup takes up to 256 rows of one expert and 256 of its weight rows, 8 waves
+// of 64 weight rows (4 across) and every other block of 32 rows (2 across): WM blocks
+// of each, so that an expert's last tile costs what its rows do, in steps of 64.
+// Operands lie in a ring of five units of 32 KB, a stage's W or A each: of turn t
+// W is unit 2t, A unit 2t + 1, and W of turn t + 1 has had a turn longer to land.
+// What bounds it: the card's power, and where operands come from behind the L2 the
+// wait for them. 128 bf16 experts of 2048 x 768, 8192 tokens x 8: gate/up 443 us = 930
+// TFLOP/s, down 2 x 159 us (tiles of 128 x 256, 48 KB a stage for half the products:
+// 498 and 2 x 187); with operands from the L2 alone 1.27 PFLOP/s, where the matrix
+// cores work 88% of the cycles of a clock that sinks to 1.45 GHz: half the copies, or
+// reads of LDS left out, raise the clock, not the products a cycle. Copies asked for in
+// one burst hold their wave up, so they are spread over the products. Workgroups that
+// go on to another block by a queue, so that the last ones end together, were no faster
+// (870 us a call, 874 so), nor was a longer part of the chip busy.
+// ---- its results: rows through LDS, so that a wave stores long runs of each --------
+// Stored from the accumulators, 16 or 32 bytes of 32 rows an instruction: gate/up 351 /
+// 325 us, down 143 / 122 (65,536 rows of one expert).
+
+// one uniform branch for four features
+DEVINL void activate(const MoeArgs& p, f32x4v g, f32x4v u, float (&v)[4]) {
+  if (p.limit > 0.f) {  // gpt-oss clamped act
 #pragma unroll
-  for (int j = 0; j < WM; ++j) {
-    const int r = row0 + ab + j * 32 + l31;
-    if (r >= rows_end) continue;
-    const int choice = p.perm[r];
-    const float w = p.choice_w[choice];
-    const float sa = FP8 ? p.a_scale[GATE ? choice / p.topk : r] : 1.f;
+    for (int s = 0; s < 4; ++s) {
+      const float a = fminf(g[s], p.limit);
+      const float b = fminf(fmaxf(u[s], -p.limit), p.limit);
+      v[s] = (b + 1.f) * (a / (1.f + __expf(-a * 1.702f)));
+    }
+  } else if (p.gelu) {
+    const float c = 0.7978845608028654f;
 #pragma unroll
-    for (int i = 0; i < WN; ++i) {
-      if (GATE) {
-        uint16_t* h = (uint16_t*)p.out + (size_t)r * p.N;
+    for (int s = 0; s < 4; ++s)
+      v[s] = 0.5f * g[s] *
+             (1.f + tanhf(c * (g[s] + 0.044715f * g[s] * g[s] * g[s]))) * u[s];
+  } else {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) v[s] = g[s] / (1.f + __expf(-g[s])) * u[s];
+  }
+}
+
+// Row block j of a wave: rows ab + 64 j + l31 of the tile. rowc, roww, rows_a: the
+// choice, routing weight and activation scale of this thread's row (tid < 256).
+template <bool FP8, bool GATE, int WM>
+DEVINL void store_big(const MoeArgs& p, uint8_t* S, const f32x16v (&acc)[2][WM],
+                      const int e, const int row0, const int rows, const int n0,
+                      const int wb, const int ab, const int rowc,
+                      const float roww, const float rows_a) {
+  constexpr int PITCH = 272;  // bytes a row: 128 bf16 or 64 fp32, and 16
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, l31 = lane & 31, half = lane >> 5;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int* choices = reinterpret_cast<int*>(S + 8 * 64 * PITCH);
+  float* weights = reinterpret_cast<float*>(choices + 256);
+  float* scales = weights + 256;
+  __syncthreads();  // every wave is done with the ring
+  if (tid < 256) {
+    choices[tid] = rowc;
+    weights[tid] = roww;
+    if (FP8) scales[tid] = rows_a;
+  }
+  __syncthreads();
+  if constexpr (GATE) {
+#pragma unroll
+    for (int j = 0; j < WM; ++j) {
+      const int r = ab + j * 64 + l31;
+      const float w = weights[r];
+      const float sa = FP8 ? scales[r] : 1.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-          const int f = n0 + (wb >> 1) + i * 16 + 8 * q + 4 * half;
-          if (f >= p.N) continue;
+          const int f = (wb >> 1) + i * 16 + 8 * q + 4 * half;  // of the tile's 128
+          const int fn = min(n0 + f, p.N - 4);  // not stored from N on
+          f32x4v g, u;
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            g[s] = acc[i][j][4 * q + s];
+            u[s] = acc[i][j][8 + 4 * q + s];
+          }
+          if (FP8) {
+            const float* ws = p.w_scale + (size_t)e * 2 * p.N + fn;
+            g *= sa * *reinterpret_cast<const f32x4v*>(ws);
+            u *= sa * *reinterpret_cast<const f32x4v*>(ws + p.N);
+          }
+          if (p.in_w) {
+            g *= w;
+            u *= w;
+          }
+          if (p.bias != nullptr) {
+            const uint16_t* b = p.bias + (size_t)e * 2 * p.N + fn;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+              g[s] += bf16_bits_to_f32(b[s]);
+              u[s] += bf16_bits_to_f32(b[p.N + s]);
+            }
+          }
           float v[4];
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            float g = acc[i][j][4 * q + s], u = acc[i][j][8 + 4 * q + s];
-            if (FP8) {
-              const float* ws = p.w_scale + (size_t)e * 2 * p.N + f + s;
-              g *= sa * ws[0];
-              u *= sa * ws[p.N];
-            }
-            if (p.in_w) {
-              g *= w;
-              u *= w;
-            }
-            if (p.bias != nullptr) {
-              const uint16_t* b = p.bias + (size_t)e * 2 * p.N + f + s;
-              g += bf16_bits_to_f32(b[0]);
-              u += bf16_bits_to_f32(b[p.N]);
-            }
-            if (p.limit > 0.f) {  // gpt-oss clamped act
-              g = fminf(g, p.limit);
-              u = fminf(fmaxf(u, -p.limit), p.limit);
-              v[s] = (u + 1.f) * (g / (1.f + __expf(-g * 1.702f)));
-            } else if (p.gelu) {
-              const float c = 0.7978845608028654f;
-              v[s] =
-                  0.5f * g * (1.f + tanhf(c * (g + 0.044715f * g * g * g))) * u;
-            } else {
-              v[s] = g / (1.f + __expf(-g)) * u;
-            }
-          }
-          uint2 o;
-          o.x = pack_bf16(v[0], v[1]);
-          o.y = pack_bf16(v[2], v[3]);
-          *reinterpret_cast<uint2*>(h + f) = o;
+          activate(p, g, u, v);
+          *reinterpret_cast<uint2*>(S + r * PITCH + f * 2) =
+              make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
         }
-      } else {
-        float* y = (float*)p.out + (size_t)choice * p.cols - p.first;
+    }
+    __syncthreads();
+    const int f = (tid & 15) * 8;
+    uint16_t* h = (uint16_t*)p.out + (size_t)row0 * p.N + n0 + f;
+    if (n0 + f < p.N)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int f = n0 + wb + i * 32 + 8 * q + 4 * half;
-          if (f >= p.first + p.cols) continue;
-          f32x4v o;
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            float c = p.in_w ? 1.f : w;
-            if (FP8) c *= sa * p.w_scale[(size_t)e * p.N + f + s];
-            o[s] = acc[i][j][4 * q + s] * c;
-          }
-          *reinterpret_cast<f32x4v*>(y + f) = o;
-        }
+      for (int k = 0; k < 2 * WM; ++k) {
+        const int r = k * 32 + (tid >> 4);
+        if (r < rows)
+          *reinterpret_cast<int4*>(h + (size_t)r * p.N) =
+              *reinterpret_cast<const int4*>(S + r * PITCH + f * 2);
       }
+  } else {
+    // a wave's own 64 rows of 64 features, twice
+    uint8_t* T = S + wid * 64 * PITCH;
+    float* y = (float*)p.out + n0 + wb - p.first;
+    f32x4v ws[2][4];
+    if (FP8)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          ws[i][q] = *reinterpret_cast<const f32x4v*>(
+              p.w_scale + (size_t)e * p.N +
+              min(n0 + wb + i * 32 + 8 * q + 4 * half, p.N - 4));
+#pragma unroll
+    for (int j0 = 0; j0 < WM; j0 += 2) {
+#pragma unroll
+      for (int j = j0; j < WM && j < j0 + 2; ++j) {
+        const float w = weights[ab + j * 64 + l31];
+        const float sa = FP8 ? scales[ab + j * 64 + l31] : 1.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            f32x4v o;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) o[s] = acc[i][j][4 * q + s];
+            if (FP8) o *= w * (sa * ws[i][q]);
+            else o *= w;
+            *reinterpret_cast<f32x4v*>(T + ((j - j0) * 32 + l31) * PITCH +
+                                       (i * 32 + 8 * q + 4 * half) * 4) = o;
+          }
+      }
+      __builtin_amdgcn_wave_barrier();
+      const int f = (lane & 15) * 4;
+      if (n0 + wb + f < p.first + p.cols)
+#pragma unroll
+        for (int k = 0; k < (WM - j0 < 2 ? 8 : 16); ++k) {
+          const int t = k * 4 + (lane >> 4);
+          const int r = ab + (j0 + (t >> 5)) * 64 + (t & 31);
+          if (r < rows)
+            *reinterpret_cast<f32x4v*>(y + (size_t)choices[r] * p.cols + f) =
+                *reinterpret_cast<const f32x4v*>(T + t * PITCH + f * 4);
+        }
+      __builtin_amdgcn_wave_barrier();
     }
   }
 }
 
+template <bool FP8, bool GATE, int WM>
+DEVINL void big_tile(const MoeArgs& p, uint8_t* S, const int e, const int row0,
+                     const int rows_end, const int n0) {
+  constexpr int WN = 2;
+  constexpr int KS = FP8 ? 2 : 4;  // products along a stage
+  constexpr int NB = FP8 ? 1 : 2;  // fp8: two sets of operands do not fit 256 registers
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5;
+  const int l31 = lane & 31;
+
+  int rowc = 0;
+  float roww = 1.f, rows_a = 1.f;
+  if (tid < rows_end - row0 && tid < 256) {
+    rowc = p.perm[row0 + tid];
+    if (FP8) rows_a = p.a_scale[GATE ? rowc / p.topk : row0 + tid];
+    if (GATE ? p.in_w : !p.in_w) roww = p.choice_w[rowc];
+  }
+  // ---- what a thread copies: one chunk of rows tid / 8 + 64 i, those of a wave from a
+  // uniform row on (but the gathered rows of x)
+  const int src = ((tid & 7) ^ ((tid >> 4) & 7)) * 16;
+  const int r0 = wid * 8, lr = lane >> 3;
+  const uint8_t* wp[4];
+  uint32_t wo[4];
+  const uint8_t* ap[WM];
+  uint32_t ao[WM];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 64 + r0;
+    // rows past the last feature are read twice and never stored
+    const int n = GATE ? n0 + (r >> 5) * 16 + (r & 15) : n0 + r;
+    const int n1 = min(n, p.N - 1);
+    const int row = n1 + (GATE ? ((r >> 4) & 1) * p.N : 0);
+    wp[i] = p.w + ((size_t)e * (GATE ? 2 * p.N : p.N) + row) * p.kb;
+    wo[i] = (uint32_t)min(lr, p.N - 1 - n1) * (uint32_t)p.kb + src;
+  }
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    const int r = min(row0 + i * 64 + r0, rows_end - 1);
+    const int l = min(lr, rows_end - 1 - r);
+    ap[i] = p.a + (GATE ? (size_t)(p.perm[r + l] / p.topk) * p.kb + src
+                        : (size_t)r * p.kb);
+    ao[i] = (uint32_t)l * (uint32_t)p.kb + src;
+  }
+  const uint32_t s0 = lds_address(S) + r0 * MOE_BKB;
+  auto copy_w = [&](int i, int off, int u) {
+    copy16(wp[i] + off, wo[i], s0 + u * MOE_UNIT + i * 64 * MOE_BKB);
+  };
+  auto copy_a = [&](int i, int off, int u) {
+    const uint32_t at = s0 + u * MOE_UNIT + i * 64 * MOE_BKB;
+    if (GATE) copy16(ap[i] + off, at);
+    else copy16(ap[i] + off, ao[i], at);
+  };
+  auto issue_w = [&](int off, int u) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) copy_w(i, off, u);
+  };
+  auto issue_a = [&](int off, int u) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i) copy_a(i, off, u);
+  };
+  const int nk = p.kb / MOE_BKB;  // full stages
+  // Past the last full stage the copies go on, of that stage again, so that their
+  // number in flight is the same for every turn and the wait a constant.
+  auto offset = [&](int kt) { return min(kt, nk - 1) * MOE_BKB; };
+
+  const int wb = (wid & 3) * 64, ab = (wid >> 2) * 32;
+  const int swz_l = (l31 >> 1) & 7;
+  using frag_t = std::conditional_t<FP8, i32x8v, bf16x8v>;
+  f32x16v acc[WN][WM] = {};
+  frag_t a[NB][WN], b[NB][WM];
+  // of units u (W) and v (A); left: bytes of the contraction in the stage
+  auto fetch = [&](int u, int v, int ks, int left, auto full) {
+    constexpr bool FULL = decltype(full)::value;
+    const uint8_t* W = S + u * MOE_UNIT;
+    const uint8_t* A = S + v * MOE_UNIT;
+#pragma unroll
+    for (int i = 0; i < WN + WM; ++i) {
+      const uint8_t* r = i < WN ? W + (wb + i * 32 + l31) * MOE_BKB
+                                : A + (ab + (i - WN) * 64 + l31) * MOE_BKB;
+      frag_t& f = i < WN ? a[ks % NB][i] : b[ks % NB][i - WN];
+      if constexpr (FP8) {
+        const int c0 = ((4 * ks + 2 * half) ^ swz_l) * 16;
+        const int c1 = ((4 * ks + 2 * half + 1) ^ swz_l) * 16;
+        f = __builtin_shufflevector(*(const i32x4v*)(r + c0),
+                                    *(const i32x4v*)(r + c1), 0, 1, 2, 3, 4, 5,
+                                    6, 7);
+        // of a last step of 32 the upper half of the lanes has nothing, and of
+        // a step behind the end no lane has
+        if (!FULL && left - ks * 64 < (half ? 64 : 1)) f = 0;
+      } else {
+        f = *(const bf16x8v*)(r + ((2 * ks + half) ^ swz_l) * 16);
+        if (!FULL && ks * 32 >= left) f = 0;
+      }
+    }
+  };
+  auto products = [&](int ks, auto&& between) {
+#pragma unroll
+    for (int i = 0; i < WN; ++i)
+#pragma unroll
+      for (int j = 0; j < WM; ++j) {
+        if constexpr (FP8)
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+              a[ks % NB][i], b[ks % NB][j], acc[i][j], 0, 0, 0, 0x7f7f7f7f, 0,
+              0x7f7f7f7f);
+        else
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              a[ks % NB][i], b[ks % NB][j], acc[i][j], 0, 0, 0);
+        between(i * WM + j);
+      }
+  };
+  // lgkmcnt(0) before the next step's operands are asked for: this step's products
+  // need no further wait and run while those are under way
+  auto landed = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // a fence would wait for every copy: vmcnt(V) and lgkmcnt(0) by hand, and no LDS
+  // access moves over the barrier
+  auto meet = [](auto v) {
+    constexpr int V = decltype(v)::value;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (V & 15) | ((V >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // A copy between products: a wave that asks for several at once waits for the
+  // address unit, which takes 64 bytes a cycle.
+  auto spread = [](int m, int first, int step, int n, auto&& copy) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < n && m == first + i * step) {
+        __builtin_amdgcn_sched_barrier(0);
+        copy(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  };
+
+  // Turn kt: products of units u (W) and u + 1 (A); the copies of W two turns on go
+  // to u + 4. Before the last products every wave has its operands in registers:
+  // behind that barrier the next turn's units are there, and A two turns on goes to
+  // W's own place.
+  auto turn = [&](int kt, auto unit) {
+    constexpr int u = decltype(unit)::value;
+    const int off = offset(kt + 2);
+    constexpr int PRODUCTS = WN * WM;
+    constexpr int STEP = (KS - 1) * PRODUCTS / 4;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      auto next = [&] {
+        if (ks + 1 < KS) fetch(u, (u + 1) % 5, ks + 1, MOE_BKB, std::true_type{});
+        else fetch((u + 2) % 5, (u + 3) % 5, 0, MOE_BKB, std::true_type{});
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      landed();
+      if (ks + 1 == KS) meet(std::integral_constant<int, 4>{});
+      if (NB == 2) next();
+      products(ks, [&](int m) {
+        if (ks + 1 < KS)
+          spread(ks * PRODUCTS + m, 0, STEP, 4,
+                 [&](int i) { copy_w(i, off, (u + 4) % 5); });
+        else
+          spread(m, 0, PRODUCTS / WM, WM, [&](int i) { copy_a(i, off, u); });
+      });
+      if (NB == 1) next();
+    }
+  };
+  if (nk > 0) {
+    issue_w(0, 0);
+    issue_a(0, 1);
+    issue_w(offset(1), 2);
+    issue_a(offset(1), 3);
+    meet(std::integral_constant<int, 4 + WM>{});
+    fetch(0, 1, 0, MOE_BKB, std::true_type{});
+    for (int kt = 0; kt < nk;) {
+      turn(kt, std::integral_constant<int, 0>{});
+      if (++kt >= nk) break;
+      turn(kt, std::integral_constant<int, 2>{});
+      if (++kt >= nk) break;
+      turn(kt, std::integral_constant<int, 4>{});
+      if (++kt >= nk) break;
+      turn(kt, std::integral_constant<int, 1>{});
+      if (++kt >= nk) break;
+      turn(kt, std::integral_constant<int, 3>{});
+      ++kt;
+    }
+    // the last copies: no more may land in LDS once the workgroup has ended
+    __builtin_amdgcn_s_waitcnt(0x0070);
+  }
+  const int left = p.kb % MOE_BKB;
+  if (left) {
+    __syncthreads();
+    const int back = max(src - (left - 16), 0);  // within the row
+    const int at = nk * MOE_BKB;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      copy16(wp[i] + at, wo[i] - back, s0 + i * 64 * MOE_BKB);
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+      copy16(ap[i] + at + (GATE ? 0 : ao[i]) - back,
+             s0 + MOE_UNIT + i * 64 * MOE_BKB);
+    meet(std::integral_constant<int, 0>{});
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      fetch(0, 1, ks, left, std::false_type{});
+      products(ks, [](int) {});
+    }
+  }
+  store_big<FP8, GATE, WM>(p, S, acc, e, row0, rows_end - row0, n0, wb, ab, rowc,
+                           roww, rows_a);
+}
+
+template <bool FP8, bool GATE>
+__global__ __launch_bounds__(512, 2) void moe_big_kernel(const MoeArgs p) {
+  __shared__ __attribute__((aligned(128))) uint8_t S[5 * MOE_UNIT];
+  // an eighth of the list an XCD, see moe_gemm_kernel
+  const int total = *p.n_tiles * p.nb;
+  const int chunk = (total + 7) >> 3;
+  const int slot = blockIdx.x >> 3;
+  const int idx = (blockIdx.x & 7) * chunk + slot;
+  if (slot >= chunk || idx >= total) return;
+  const int4 tile = p.tiles[idx / p.nb];
+  const int e = __builtin_amdgcn_readfirstlane(tile.x);
+  const int row0 = __builtin_amdgcn_readfirstlane(tile.y);
+  const int rows_end = __builtin_amdgcn_readfirstlane(tile.z);
+  const int n0 = p.first + (idx % p.nb) * (GATE ? 128 : 256);
+  const int rows = rows_end - row0;
+  if (rows > 192)
+    big_tile<FP8, GATE, 4>(p, S, e, row0, rows_end, n0);
+  else if (rows > 128)
+    big_tile<FP8, GATE, 3>(p, S, e, row0, rows_end, n0);
+  else if (rows > 64)
+    big_tile<FP8, GATE, 2>(p, S, e, row0, rows_end, n0);
+  else
+    big_tile<FP8, GATE, 1>(p, S, e, row0, rows_end, n0);
+}
 // ---- combine --------------------------------------------------------------------
 // out[t] = sum over its choices, of the features from first on; four a thread.
 
@@ -551,43 +965,52 @@ extern "C" void launch_quantize_fp8_rows(
 
 // ---- the two products of a layer -----------------------------------------------
 
-template <bool FP8, int TN, int TM, int STAGES>
+template <bool FP8, int TM, int STAGES>
 static void launch_gemm(bool gate, MoeArgs& p, int max_tiles,
                         hipStream_t stream) {
-  p.nb = ceil_div(p.cols, gate ? TN / 2 : TN);
+  p.nb = ceil_div(p.cols, gate ? 64 : 128);
   const int blocks = (max_tiles * p.nb + 7) / 8 * 8;
   if (gate)
-    moe_gemm_kernel<FP8, TN, TM, true, STAGES>
-        <<<blocks, 2 * TN, 0, stream>>>(p);
+    moe_gemm_kernel<FP8, TM, true, STAGES><<<blocks, 256, 0, stream>>>(p);
   else
-    moe_gemm_kernel<FP8, TN, TM, false, STAGES>
-        <<<blocks, 2 * TN, 0, stream>>>(p);
+    moe_gemm_kernel<FP8, TM, false, STAGES><<<blocks, 256, 0, stream>>>(p);
 }
 
 template <bool FP8>
 static void launch_gemm_tm(int tm, bool gate, MoeArgs& p, int max_tiles,
                            hipStream_t stream) {
-  if (tm == 32)
-    launch_gemm<FP8, 128, 32, 4>(gate, p, max_tiles, stream);
-  else if (tm == 64)
-    launch_gemm<FP8, 128, 64, 3>(gate, p, max_tiles, stream);
-  else
-    launch_gemm<FP8, 256, 128, 3>(gate, p, max_tiles, stream);
+  if (tm == 32) {
+    launch_gemm<FP8, 32, 4>(gate, p, max_tiles, stream);
+  } else if (tm == 64) {
+    launch_gemm<FP8, 64, 3>(gate, p, max_tiles, stream);
+  } else {
+    p.nb = ceil_div(p.cols, gate ? 128 : 256);
+    const int blocks = (max_tiles * p.nb + 7) / 8 * 8;
+    if (gate) {
+      moe_big_kernel<FP8, true><<<blocks, 512, 0, stream>>>(p);
+    } else {
+      moe_big_kernel<FP8, false><<<blocks, 512, 0, stream>>>(p);
+    }
+  }
 }
 
-// Rows a tile, by the mean number of choices an expert. Measured (us, tiles of
-// 32 / 64 / 128 rows): bf16 128 experts of 2048 x 768, mean 6: 182 / 189 / 230,
-// 25: 251 / 246 / 247, 43: 326 / 284 / 311, 62: 390 / 338 / 319, 512: 1855 /
-// 1378 / 1089; 32 experts of 2048 x 1024, mean 25: 106 / 122 / 151, 62: 148 /
-// 123 / 156, 250: 353 / 252 / 223; fp8 256 experts of 7168 x 2048, mean 6: 1334 /
-// 1296 / 1360, 21: 2167 / 1926 / 1989, 46: 3178 / 2503 / 2306. Below, the
-// weights' stream is the work and few rows cost nothing; 128 rows pay earlier
-// where there are blocks enough for the chip (8 a CU).
+// Rows a tile, by the mean number of choices an expert and by how many blocks of 256
+// rows x 256 weight rows there are: fewer than CUs leave some of them idle, unless the
+// experts' last tiles are few beside the full ones. Measured (us, tiles of 32 / 64 /
+// 256 rows): bf16 128 experts of 2048 x 768, mean 6: 180 / 181 / 201, 25: 247 / 241 /
+// 241, 50: 319 / 289 / 284, 100: 456 / 379 / 340, 300: 1091 / 815 / 608; 32 experts of
+// 2048 x 1024, mean 50: 124 / 115 / 128, 125: 191 / 157 / 168 (240 blocks), 150: 231 /
+// 169 / 164 (280), 400: 504 / 360 / 280; 16 experts of 1024 x 512, mean 300: 58 / 57 /
+// 67 (104), 625: 104 / 87 / 78 (188); fp8 256 experts of 7168 x 2048, mean 2: 961 / 961
+// / 984, 6: 1432 / 1415 / 1389, 25: 2177 / 1881 / 1739, 47: 3228 / 2409 / 2028; 128 of
+// 2048 x 768, mean 12: 131 / 131 / 135, 25: 155 / 156 / 151, 200: 492 / 424 / 346.
 extern "C" int moe_tile_rows(int n, int E, int I, bool fp8) {
   const int mean = n / (E > 0 ? E : 1);
-  if (mean <= (fp8 ? 12 : 24)) return 32;
-  const int64_t blocks = ((int64_t)n / 128 + E / 2) * ceil_div(I, 128);
-  return mean > 96 || (mean > 40 && blocks >= 2048) ? 128 : 64;
+  const int64_t blocks = ((int64_t)n / 256 + E / 2) * ceil_div(I, 128);
+  if (mean > 450 || (blocks >= 256 && mean > (fp8 ? 16 : 40)) ||
+      (fp8 && blocks >= 2048 && mean > 4))
+    return 256;
+  return mean <= (fp8 ? 12 : 24) ? 32 : 64;
 }
 
 extern "C" int moe_max_tiles(int n, int E, int tm) {
@@ -596,8 +1019,8 @@ extern "C" int moe_max_tiles(int n, int E, int tm) {
 
 // Output features of a down product and combine: y takes at most MOE_Y_BYTES (of
 // 256 features, a tile's width, at least), however many tokens a step brings. 65,536
-// choices of 2048 features, a whole call: one slab of 537 MB 1.033 ms, two of 256
-// MB at most 1.030.
+// choices of 2048 features, a whole call with the tiles of 128 rows that there were:
+// one slab of 537 MB 1.033 ms, two of 256 MB at most 1.030.
 #define MOE_Y_BYTES (256ll << 20)
 extern "C" int moe_down_cols(int n, int H) {
   const int64_t cols = MOE_Y_BYTES / (4ll * n) & ~255ll;

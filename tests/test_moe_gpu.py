@@ -227,6 +227,49 @@ def test_moe_tiles(T, E, k, H, I, fp8):
     assert ops.fused_moe_forward(x[:0], gu, dn, ids[:0], w[:0]).shape == (0, H)
 
 
+@pytest.mark.parametrize("H,I,fp8", [
+    (96, 96, False),      # a stage and a half, then half a stage
+    (704, 544, False),    # 11 and 8.5 stages; 544 features: blocks cut by the end
+    (32, 32, False),      # less than a stage
+    (160, 192, True),
+    (896, 64, True),
+])
+def test_moe_rows_of_large_tiles(H, I, fp8):
+    """Tiles of 256 rows at the edges of their steps of 64: 1 .. 512 rows an expert.
+    Tolerances as in test_moe_tiles."""
+    rows = [1, 64, 65, 128, 0, 129, 192, 193, 256, 257, 511, 512, 3000]
+    E, n = len(rows) + 1, sum(rows)
+    g = torch.Generator(device="cuda").manual_seed(H)
+    owner = torch.repeat_interleave(torch.arange(len(rows)), torch.tensor(rows))
+    owner = owner[torch.randperm(n, generator=torch.Generator().manual_seed(1))]
+    owner = torch.cat([owner, owner.new_full((16384 - n,), E)])  # of another rank
+    ids = owner.view(-1, 2).cuda()
+    T = ids.shape[0]
+    assert 16384 // E > 450                     # tiles of 256 rows by the rule
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
+    w = torch.rand(T, 2, generator=g, device="cuda")
+    if fp8:
+        qg, sg = ops.quantize_fp8_weight(gu)
+        qd, sd = ops.quantize_fp8_weight(dn)
+        got = ops.fused_moe_forward_fp8(x, qg, sg, qd, sd, ids, w)
+        want = _experts64(x, qg.double() * sg[..., None], qd.double() * sd[..., None],
+                          ids, w, fp8=True)
+        assert (got - want).norm() < 2e-2 * want.norm()
+        return
+    bias = torch.randn(E, 2 * I, generator=g, device="cuda").bfloat16()
+    for kw in ({}, {"on_input": True}, {"limit": 7.0, "bias": bias}, {"gelu": True}):
+        got = ops.fused_moe_forward(
+            x, gu, dn, ids, w, activation="gelu" if kw.get("gelu") else "silu",
+            limit=kw.get("limit", 0.0), bias_gate_up=kw.get("bias"),
+            weight_on_input=kw.get("on_input", False))
+        want = _experts64(x, gu, dn, ids, w, **kw)
+        # every row on its own: a row that is wrong does not hide among the others
+        err = (got - want).norm(dim=1)
+        assert (err <= 2 ** -7 * want.norm(dim=1) + 1e-30).all()
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 def test_moe_many_choices_within_a_fixed_workspace(fp8):
     """The down product and its combine go over the output features in slabs once a
