@@ -139,6 +139,7 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
   constexpr int NI = ROWS / 8;  // copies a stage: 8 rows of 128 bytes each
   constexpr int MT = (XR + 15) / 16;
   constexpr int MP = MT * 16;
+  constexpr int AT = (NT + 15) / 16;  // NT 8: the operand's upper rows are the lower
   constexpr int RING = ROWS * 128;  // a wave's stage
   __shared__ __attribute__((aligned(128))) uint8_t S[WAVES * STAGES * RING];
 
@@ -180,14 +181,14 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
       copy16_to_lds((q * 8 < NT ? wb : x) + k + at[q], dst + q * 1024);
   };
 
-  f32x4v acc[NT / 16][MT] = {};
+  f32x4v acc[AT][MT] = {};
   const uint32_t ring_at =
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring;
-  const int j0 = (l4 ^ ((l15 >> 1) & 7)) * 16;
+  const int wr = l15 & (NT < 16 ? NT - 1 : 15);
   const int xr = l15 & (XR < 16 ? XR - 1 : 15);
-  const uint32_t a_at = ring_at + l15 * 128 + j0;
+  const uint32_t a_at = ring_at + wr * 128 + (l4 ^ ((wr >> 1) & 7)) * 16;
   const uint32_t b_at =
-      ring_at + (NT + xr) * 128 + (l4 ^ ((xr >> 1) & 7)) * 16;
+      ring_at + (NT + xr) * 128 + (l4 ^ (((NT + xr) >> 1) & 7)) * 16;
   int place = 0, next = STAGES - 1;
 #pragma unroll
   for (int i = 0; i < STAGES - 1; ++i)
@@ -196,13 +197,13 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
     wait_copies<(STAGES - 2) * NI>();
     // into the place read in the turn before: its operands are in registers
     issue(i + STAGES - 1, next);
-    bf16x8v a[2][NT / 16], b[2][MT];
+    bf16x8v a[2][AT], b[2][MT];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
       read_operands((a_at + place * RING) ^ (ks * 64),
                     (b_at + place * RING) ^ (ks * 64), a[ks], b[ks]);
 #pragma unroll
-    for (int t = 0; t < NT / 16; ++t)
+    for (int t = 0; t < AT; ++t)
 #pragma unroll
       for (int u = 0; u < MT; ++u) {
         if constexpr (FP8) {
@@ -224,11 +225,12 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(
   float* part = reinterpret_cast<float*>(S);
   static_assert(MP * NT * 4 <= STAGES * RING, "");
 #pragma unroll
-  for (int t = 0; t < NT / 16; ++t)
+  for (int t = 0; t < AT; ++t)
 #pragma unroll
     for (int u = 0; u < MT; ++u)
-      *reinterpret_cast<f32x4v*>(
-          part + ((wid * MP + u * 16 + l15) * NT + t * 16 + l4 * 4)) = acc[t][u];
+      if (NT >= 16 || l4 * 4 < NT)
+        *reinterpret_cast<f32x4v*>(
+            part + ((wid * MP + u * 16 + l15) * NT + t * 16 + l4 * 4)) = acc[t][u];
   __syncthreads();
   const float scale = FP8 ? x_scale[0] * w_scale[0] : 1.f;
   const int quads = side / 4;
@@ -501,6 +503,10 @@ extern "C" void launch_skinny_split(
 
 // Tiles, by rows of X and by how many tiles W gives. us of bf16 products, W from
 // memory (N x K; the library's tuned pick last):
+//   up to 8 rows, NT 8 of 8 waves / 16 of 4 where W has few rows, each CU's own rate
+//   being the bound: 896 x 4864 5.7 / 6.5, 2048 x 5632 7.2 / 8.4, 1536 x 8960 8.2 /
+//   11.7, 2048 x 2048 5.0 / 5.4 but 896 x 896 3.6 / 3.4, 4096 x 4096 9.2 / 8.6
+//   (8 rows 6.6 / 7.5, 7.7 / 8.8, 9.7 / 11.7)
 //   up to 8 rows, NT 16 of 4 waves, 5 stages / 3 stages (four workgroups a CU
 //   instead of two): 28672 x 4096 40 / 41 (50), 4096 x 14336 22 / 25 (25), 9728 x
 //   896 8.6 / 6.6 (12), 24576 x 1536 17 / 16 (21), 896 x 896 3.3 (5.5)
@@ -509,8 +515,8 @@ extern "C" void launch_skinny_split(
 //   28672 x 4096 48 / 45 / 42 (54), 4096 x 14336 26 / 32 / 49 (26)
 //   17 to 32, the same: 28672 x 4096 60 / 47 / 43 (56), 6144 x 4096 18 / 13.9 /
 //   19.5 (15.2), 4096 x 4096 10.7 / 13.4 / 19 (11.8)
-static int skinny_tile(int M, int64_t N, int row_bytes) {
-  if (M <= 8) return 16;
+static int skinny_tile(int M, int64_t N, int row_bytes, bool gated) {
+  if (M <= 8) return N <= 2048 && row_bytes >= 4096 && !gated ? 8 : 16;
   if (N >= 9600) return 64;
   if (N >= 4800) return 32;
   return M <= 16 || row_bytes <= 10240 ? 16 : 0;
@@ -533,7 +539,7 @@ extern "C" int skinny_shared(int M, int N, int row_bytes) {
     return (splits == 1 || row_bytes >= 4096) && (M <= 64 || bytes >= 1 << 24)
                ? splits : -1;
   if (M <= 8) return 0;
-  const int nt = skinny_tile(M, N, row_bytes);
+  const int nt = skinny_tile(M, N, row_bytes, false);
   const int tiles = ceil_div(N, 64);
   const bool ragged =
       nt == 64 && tiles > 512 && tiles < 384 * ceil_div(tiles, 512);
@@ -567,7 +573,7 @@ extern "C" void launch_skinny_gemm(
     int64_t x_batch, int64_t c_batch, bool gated, hipStream_t stream,
     bool* launched) {
   *launched = false;
-  const int nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes);
+  const int nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes, gated);
   if (nt == 0 || row_bytes % 128 || N % 4) return;
   *launched = true;
   auto run = [&](auto kernel, int xr, int waves) {
@@ -580,7 +586,8 @@ extern "C" void launch_skinny_gemm(
   auto pick = [&](auto f) {
     constexpr bool F = decltype(f)::value;
     if (M <= 8) {
-      if (row_bytes <= 4096) run(skinny_gemm_kernel<F, 16, 8, 4, 3>, 8, 4);
+      if (nt == 8) run(skinny_gemm_kernel<F, 8, 8, 8, 4>, 8, 8);
+      else if (row_bytes <= 4096) run(skinny_gemm_kernel<F, 16, 8, 4, 3>, 8, 4);
       else run(skinny_gemm_kernel<F, 16, 8, 4, 5>, 8, 4);
     } else if (M <= 16) {
       if (nt == 64) run(skinny_gemm_kernel<F, 64, 16, 2, 4>, 16, 2);

@@ -21,6 +21,7 @@ def _rand(g, *s):
         (9604, 320),    # 64 rows a tile
     )
 ] + [
+    (1, 2044, 2048), (5, 900, 4864), (8, 12, 2112),      # 8 rows a tile
     (33, 576, 2112), (64, 100, 2048), (64, 5000, 3072),  # K shared, odd parts
     (20, 1536, 7168), (32, 24576, 1408),                 # the same, fewer rows
     (65, 4100, 4096), (96, 28672, 320), (128, 36864, 256),  # 3 to 5 waves
