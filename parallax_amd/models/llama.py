@@ -23,6 +23,7 @@ from ..parallel.layers import (
     MergedColumnParallelLinear,
     RowParallelLinear,
     VocabEmbedding,
+    plain_call,
 )
 from .config import ModelConfig
 from .forward_meta import ForwardMeta
@@ -40,6 +41,19 @@ class RMSNorm(nn.Module):
         if residual is None:
             return ops.rmsnorm(x, self.weight, self.eps)
         return ops.fused_add_rmsnorm(x, residual, self.weight, self.eps)
+
+
+def norm_project(norm: nn.Module, proj: nn.Module, x: torch.Tensor,
+                 residual: Optional[torch.Tensor], gated: bool = False):
+    """(proj(norm(x, residual)), the residual then) of a few rows in one launch, gated:
+    silu of its first part times the second. None where there is no kernel for it, and
+    for modules that are more than these two: hooks and forwards of others see the
+    normed rows, which one launch never stores."""
+    if not (plain_call(norm, RMSNorm.forward)
+            and plain_call(proj, MergedColumnParallelLinear.forward)) or proj.fp8:
+        return None
+    return ops.norm_linear(x, residual, norm.weight, norm.eps, proj.weight, proj.bias,
+                           gated)
 
 
 class ResidualLayerNorm(nn.Module):
@@ -103,8 +117,12 @@ class LlamaAttention(nn.Module):
             )
 
     def forward(self, x: torch.Tensor, meta: ForwardMeta, rope_cache: torch.Tensor):
-        T = x.shape[0]
-        qkv = self.qkv_proj(x)
+        return self.attend(self.qkv_proj(x), x, meta, rope_cache)
+
+    def attend(self, qkv: torch.Tensor, x: torch.Tensor, meta: ForwardMeta,
+               rope_cache: torch.Tensor):
+        """The layer from its projection on; x only to be handed on."""
+        T = qkv.shape[0]
         q, k, v = self.qkv_proj.split_output(qkv)
         # strided views into the fused QKV buffer — no contiguous copies; the
         # HIP kernels take a row stride
@@ -168,15 +186,29 @@ class LlamaDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, x, residual, meta: ForwardMeta, rope_cache):
-        if residual is None:
-            residual = x
-            x = self.input_layernorm(x)
+        attn, mlp = self.self_attn, self.mlp
+        fused = None
+        if plain_call(attn, LlamaAttention.forward) and (
+                type(attn)._project_out is LlamaAttention._project_out):
+            fused = norm_project(self.input_layernorm, attn.qkv_proj, x, residual)
+        if fused is not None:
+            qkv, residual = fused
+            x = attn.attend(qkv, x, meta, rope_cache)
         else:
-            x, residual = self.input_layernorm(x, residual)
-        x = self.self_attn(x, meta, rope_cache)
+            if residual is None:
+                residual = x
+                x = self.input_layernorm(x)
+            else:
+                x, residual = self.input_layernorm(x, residual)
+            x = attn(x, meta, rope_cache)
+        if plain_call(mlp, LlamaMLP.forward):
+            fused = norm_project(self.post_attention_layernorm, mlp.gate_up_proj, x,
+                                 residual, gated=True)
+            if fused is not None:
+                x, residual = fused
+                return mlp.down_proj(x), residual
         x, residual = self.post_attention_layernorm(x, residual)
-        x = self.mlp(x)
-        return x, residual
+        return mlp(x), residual
 
 
 @register_model("LlamaForCausalLM", "Qwen2ForCausalLM", "MistralForCausalLM")

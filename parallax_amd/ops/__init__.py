@@ -482,6 +482,31 @@ def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
                         x_scale if fp8 else none, w_scale if fp8 else none, gated)
 
 
+def norm_linear(
+    x: torch.Tensor, residual: Optional[torch.Tensor], norm_weight: torch.Tensor,
+    eps: float, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+    gated: bool = False,
+) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """(rmsnorm(x + residual) . weight^T + bias, x + residual) of a few rows in one
+    launch, as fused_add_rmsnorm and linear give them, x and residual left as they
+    are; gated: silu of the first half of the columns times the second. None where
+    the kernel has nothing for it, or two launches are as fast (norm_linear.hip has
+    the sizes); no part of autograd."""
+    args = [x, norm_weight, weight] + [t for t in (residual, bias) if t is not None]
+    if not x.is_cuda or x.dim() != 2 or weight.dim() != 2 or any(
+            t.dtype != torch.bfloat16 for t in args):
+        return None
+    if torch.is_grad_enabled() and any(t.requires_grad for t in args):
+        return None
+    if x.shape[1] != weight.shape[1] or SKINNY_GEMM_MAX_M < x.shape[0]:
+        return None
+    ext = _require_ext("norm_linear")
+    none = x.new_empty(0)
+    return ext.norm_linear(
+        x, none if residual is None else residual, norm_weight, eps, weight,
+        none if bias is None else bias, gated)
+
+
 def _library_takes(x, weight):
     return (
         LT_GEMM

@@ -18,6 +18,10 @@ extern "C" {
 void launch_rmsnorm(void*, void*, const void*, float, int, int, hipStream_t);
 void launch_fused_add_rmsnorm(void*, void*, const void*, float, int, int,
                               hipStream_t);
+bool norm_linear_takes(int64_t, int64_t, int64_t, bool);
+void launch_norm_linear(void*, void*, const void*, const void*, const void*,
+                        const void*, const void*, float, int, int, int, int64_t,
+                        int64_t, bool, hipStream_t);
 void launch_rope(void*, void*, const int*, const float*, int, int, int, int,
                  int, bool, int64_t, int64_t, hipStream_t);
 void launch_rope_and_cache(void*, const void*, const void*, void*, void*,
@@ -790,12 +794,56 @@ bool skinny_gemm(torch::Tensor c, torch::Tensor x, torch::Tensor w,
   return skinny_run(c, x, w, bias, x_scale, w_scale, gated);
 }
 
-// the same with the result allocated; None where there is no kernel, or the library
+// (f(rms_norm(x + res)) . w^T + bias, x + res) of few rows: bf16; without a norm (empty)
+// or res (empty) neither is there. None where there is no kernel.
+std::optional<std::tuple<torch::Tensor, torch::Tensor>> norm_linear(
+    torch::Tensor x, torch::Tensor res, torch::Tensor norm, double eps,
+    torch::Tensor w, torch::Tensor bias, bool gated) {
+  CHECK_GPU(x);
+  CHECK_BF16(x);
+  CHECK_BF16(w);
+  CHECK_BF16(res);
+  CHECK_BF16(norm);
+  CHECK_BF16(bias);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1));
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  const bool has_norm = norm.numel() > 0, has_res = res.numel() > 0;
+  auto rows16 = [](const torch::Tensor& t) {
+    return (uintptr_t)t.data_ptr() % 16 == 0 && t.stride(1) == 1 &&
+           t.stride(0) % 8 == 0;
+  };
+  if (!norm_linear_takes(M, N, K, has_norm) || !rows16(x) || !rows16(w) ||
+      !w.is_contiguous() || (gated && N % 2))
+    return std::nullopt;
+  if (has_res && (!has_norm || res.dim() != 2 || res.size(0) != M ||
+                  res.size(1) != K || !rows16(res)))
+    return std::nullopt;
+  if (has_norm && (norm.dim() != 1 || norm.size(0) != K || !norm.is_contiguous() ||
+                   (uintptr_t)norm.data_ptr() % 16))
+    return std::nullopt;
+  if (bias.numel() && (bias.dim() != 1 || bias.size(0) != N || !bias.is_contiguous()))
+    return std::nullopt;
+  auto c = torch::empty({M, gated ? N / 2 : N}, x.options());
+  auto sum = has_res ? torch::empty({M, K}, x.options()) : x;
+  launch_norm_linear(c.data_ptr(), sum.data_ptr(), x.data_ptr(),
+                     has_res ? res.data_ptr() : nullptr,
+                     has_norm ? norm.data_ptr() : nullptr, w.data_ptr(),
+                     bias.numel() ? bias.data_ptr() : nullptr, (float)eps, M, N, K,
+                     x.stride(0), has_res ? res.stride(0) : 0, gated, cur_stream());
+  return std::make_tuple(c, sum);
+}
+
+// skinny_gemm with the result allocated; None where there is no kernel, or the library
 // is faster
 std::optional<torch::Tensor> few_rows(torch::Tensor x, torch::Tensor w,
                                       torch::Tensor bias, torch::Tensor x_scale,
                                       torch::Tensor w_scale, bool gated) {
   torch::Tensor c;
+  const auto none = w.new_empty({0});
+  if (x_scale.numel() == 0) {
+    auto r = norm_linear(x, none, none, 0., w, bias, gated);
+    if (r) return std::get<0>(*r);
+  }
   if (!gated && !skinny_pays(x.size(0), w.size(0), x.size(1) * x.element_size()))
     return std::nullopt;
   if (!skinny_run(c, x, w, bias, x_scale, w_scale, gated)) return std::nullopt;
@@ -903,6 +951,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("msa_paged_attention_decode", &msa_paged_attention_decode);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("few_rows", &few_rows);
+  m.def("norm_linear", &norm_linear);
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);
   m.def("mla_absorb", &mla_absorb);
   m.def("mla_project", &mla_project);

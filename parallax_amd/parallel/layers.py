@@ -47,7 +47,7 @@ class _Fp8WeightMixin:
         return ops.linear(x, self.weight, getattr(self, "bias", None))
 
 
-def _plain_call(m: nn.Module, forward) -> bool:
+def plain_call(m: nn.Module, forward) -> bool:
     """Whether calling m runs this forward and nothing else."""
     g = nn.modules.module
     return getattr(m.forward, "__func__", None) is forward and not (
@@ -148,7 +148,7 @@ class MergedColumnParallelLinear(nn.Module, _Fp8WeightMixin):
     def silu_and_mul(self, x: torch.Tensor) -> torch.Tensor:
         """silu(first part) * second part, of two equal ones. Hooks and forwards of
         others see the product itself, which the fused epilogue never stores."""
-        if self.fp8 or not _plain_call(self, MergedColumnParallelLinear.forward):
+        if self.fp8 or not plain_call(self, MergedColumnParallelLinear.forward):
             return ops.silu_and_mul(self(x))
         return ops.linear_silu_and_mul(x, self.weight, self.bias)
 

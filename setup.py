@@ -34,6 +34,7 @@ sources = [
     os.path.join(CSRC, "prefill_attention.hip"),
     os.path.join(CSRC, "moe.hip"),
     os.path.join(CSRC, "skinny_gemm.hip"),
+    os.path.join(CSRC, "norm_linear.hip"),
     os.path.join(CSRC, "indexer.hip"),
     os.path.join(CSRC, "sampler.hip"),
 ]
