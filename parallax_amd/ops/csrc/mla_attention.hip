@@ -2,8 +2,8 @@
 //
 //   S^T[64 tok x 16 heads] = C . Q^T     C = [latent | rope] rows, 576 values
 //   O^T[512 x 16 heads]   += C_v^T . P   C_v = the latent part of the same rows
-// All query heads share ONE cache row a token; a workgroup takes 64 heads (16 a
-// wave, Q and O^T in registers). With 128 heads two workgroups read a row, at
+// All query heads share ONE cache row a token; a workgroup takes 64 heads (16 a pair of
+// waves, Q and O^T in registers). With 128 heads two workgroups read a row, at
 // the same time and through one XCD's L2: 128 heads a workgroup need 512
 // registers a wave, which the compiler spilled.
 // Tiles of 64 tokens are copied global -> LDS directly, the next one while this
@@ -20,12 +20,12 @@
 // adds up. Short sequences (256 tokens at most) take a workgroup each and need
 // no second kernel.
 //
-// What bounds it: the waves of a workgroup go through a tile in step (operands out
-// of LDS, products, softmax), 37% of the matrix cores' time at 64 heads; with 16
-// heads the latent rows, 4.2 TB/s. Measured (before: single-buffered tiles
-// transposed value by value into LDS, fixed partitions of the context): 64 heads,
-// 4 x 100,000 tokens 111 us (613); 128 heads, 40 x 4,000 78 us (351); 16 heads, 64
-// x 6,000 69 us (230); 128 heads, one sequence of 1,000 22 us (57).
+// What bounds it: the latent rows' stream, 3.1 us a tile and CU at 6.1 TB/s where a
+// tile takes 3.7, and the start and end of a run, a quarter of the time of runs of 18
+// tiles. Copies go between S^T's products from uniform addresses; worked out a lane in
+// front of them, 250 instructions a wave, and S^T computed by both waves of a pair,
+// they left each other no room: 64 heads, 4 x 100,000 tokens 98 us, now 84; 128 heads,
+// 40 x 4,000 71 and 63; with the second kernel's 9 and 11.
 //
 // Reference analogue: parallax_extensions/kernels/mla/ (Metal, VALU); fresh
 // MFMA design. Layout: cache [NB, BS, R+DR], q_latent [B, H, R], q_pe [B, H, DR].
@@ -35,7 +35,8 @@
 #define MLA_R 512
 #define MLA_DR 64
 #define MLA_DK 576          // values a cache row
-#define MLA_CH 72           // 16-byte chunks a row
+#define MLA_ROW 1024        // bytes of a row's latent values in LDS
+#define MLA_PE 128          // and of its rotated ones
 #define MLA_KT 64           // tokens a tile
 #define MLA_DT 16           // 16-value tiles of O^T a wave
 #define MLA_MIN_TILES 2     // a run is at least this long
@@ -60,10 +61,16 @@ DEVINL uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, p);
 }
 
-DEVINL void copy16_to_lds(const void* src, void* dst) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void*)src,
-      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+// 16 bytes a lane from memory to LDS, at + 16 lane, from a uniform base or a pointer a
+// lane. In assembly: of the builtin the compiler knows that it writes LDS, and waits
+// for copies in flight before reads of other places.
+DEVINL void copy16(const uint8_t* base, uint32_t off, uint32_t at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(base), "s"(at) : "m0", "memory");
+}
+DEVINL void copy16(const uint8_t* src, uint32_t at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               :: "v"(src), "s"(at) : "m0", "memory");
 }
 
 // over the four lanes that hold one head (l, l + 16, l + 32, l + 48)
@@ -77,13 +84,15 @@ DEVINL float over_head(float v, F f) {
   return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-// Chunk c of row r lies at chunk_at(r, c). A row of 72 chunks is 8 modulo a turn
-// of 16 over the banks, so row bit 0 does its part; the other bits move pairs of
-// chunks, which spreads both kinds of read: transposing ones, where half a wave
-// takes two chunks of 8 rows, and 16-byte ones, which go by lanes {0-3, 12-15,
-// 20-23, 24-27} and so on: 8 rows of one chunk and 8 others of the next.
-DEVINL int row_xor(int r) { return ((r >> 1) & 3) << 1; }
-DEVINL int chunk_at(int r, int c) { return (c & ~7) | ((c & 7) ^ row_xor(r)); }
+// A tile in LDS: 64 rows of 64 chunks (the latent values), then 64 rows of 8 (the
+// rotated ones). Chunk c of row r lies at c ^ row_xor(r), or rope_xor(r), which are
+// linear over xor in the row's four bits. 16-byte reads go by lanes {0-3, 12-15,
+// 20-23, 24-27} and so on, rows of one chunk and other rows of its neighbour, that is
+// rows with bits 2 and 3 alike or not: they meet in no bank as no two such rows differ
+// by 1 in row_xor. Transposing reads take two neighbouring chunks of 8 rows of one bit
+// 3: those rows differ above bit 0.
+DEVINL constexpr int row_xor(int r) { return (r & 7) * 2 ^ (r & 8 ? 9 : 0); }
+DEVINL constexpr int rope_xor(int r) { return (r & 6) ^ (r & 8 ? 5 : 0); }
 
 // tiles of sequence b: its tokens, or its list of token positions
 template <bool SPARSE>
@@ -146,11 +155,12 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     const int* __restrict__ topk,           // [B, max_topk] (SPARSE)
     const int max_topk, const int B, const int max_blocks, const int H,
     const int bs_shift, const float scale, const float c_scale) {
-  constexpr int COPIES = MLA_KT * MLA_CH / 64;   // 72 of 64 chunks each
-  constexpr int CPW = COPIES / W;                // a wave
-  constexpr int BUF = MLA_KT * MLA_DK;
-  __shared__ __attribute__((aligned(16))) uint16_t S0[BUF];
-  __shared__ __attribute__((aligned(16))) uint16_t S1[BUF];
+  constexpr int RPW = MLA_KT / W;      // rows a wave copies
+  constexpr int CPW = RPW + RPW / 8;   // copies: a row's latent values, 8 rows' rope
+  constexpr int BUF = MLA_KT * (MLA_ROW + MLA_PE);
+  __shared__ __attribute__((aligned(1024))) uint8_t S[2 * BUF];
+  // scores on their way between the two waves of a pair
+  __shared__ __attribute__((aligned(16))) f32x4v X[W][MLA_KT / 32][64];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -187,24 +197,26 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
   at = __builtin_amdgcn_readfirstlane(at);
   todo = __builtin_amdgcn_readfirstlane(todo);
 
-  // two waves share 16 heads: both compute S^T, each half of the latent values
+  // two waves share 16 heads: each computes S^T of half of the tokens, and O^T of
+  // half of the latent values
   const int head0 = (blockIdx.y * (W / 2) + (wid >> 1)) * 16;
   const int head = head0 + l15;
   const int d0 = (wid & 1) * (MLA_R / 2);
 
-  // what a lane reads of a tile: S^T's operand has two places in a group of
-  // eight chunks, O^T's has four; the groups follow at 64 values
-  int qk_at[2], tr_at[4];
-  {
-    const int r = 4 * l4 + (l15 >> 2);  // token row of a transposing read
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      qk_at[i] = l15 * MLA_DK + chunk_at(l15, i * 4 + l4) * 8;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      tr_at[i] = r * MLA_DK + d0 + chunk_at(r, i * 2 + ((l15 & 3) >> 1)) * 8 +
-                 (l15 & 1) * 4;
-  }
+  // what a lane reads of a tile, in bytes: rows of S^T's operand (chunks l4 and
+  // those at multiples of 4 from it) and of O^T's (chunks at multiples of 2)
+  const int tr_row = 4 * l4 + (l15 >> 2);
+  const uint32_t s_at = (uint32_t)(uintptr_t)(
+      __attribute__((address_space(3))) const void*)S;
+  const int qk_at = (wid & 1) * 32 * MLA_ROW + l15 * MLA_ROW +
+                    (l4 ^ row_xor(l15)) * 16;
+  const int pe_at = MLA_KT * MLA_ROW + (wid & 1) * 32 * MLA_PE + l15 * MLA_PE +
+                    (l4 ^ rope_xor(l15)) * 16;
+  const int tr_at = tr_row * MLA_ROW + d0 * 2 +
+                    (((l15 & 3) >> 1) ^ row_xor(tr_row)) * 16 + (l15 & 1) * 8;
+  // what a lane copies, in values: of row 8 g + i of the wave's (g the row's bit 3)
+  // chunk (lane ^ row_xor), of the rope of 8 rows one chunk of row lane / 8
+  const int bit3 = RPW == 8 ? wid & 1 : 0;
 
   while (todo > 0) {
     const int* btab = block_tables + (size_t)seq * max_blocks;
@@ -251,63 +263,76 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
       return L > 0 ? slot_of(e >= 0 && e < L ? e : 0) : 0;
     };
     constexpr int ESZ = KV_FP8 ? 1 : 2;
-    // where the copies of tile t read: a base that all lanes share, and 32 bits.
-    // 16 rows lie in one page and are 18 copies; rows past the end read a page
-    // that is there.
-    auto each_copy = [&](int t, auto&& use) INL {
-      // worked out anew for every tile: nine more registers would spill
-      int ln = lane;
-      asm volatile("" : "+v"(ln));
-      int base[MLA_KT / 16], mine = 0;
-      if (listed) mine = listed_slot(t);
+    // Where tile t's rows of this wave lie: of every 8 the first one's slot (8 rows
+    // lie in one page; rows past the end read a page that is there), or listed each
+    // lane's row.
+    int slots[RPW / 8], mine = 0;
+    auto look_up = [&](int t) INL {
+      if (listed) {
+        mine = listed_slot(t);
+        return;
+      }
 #pragma unroll
-      for (int g = 0; g < MLA_KT / 16; ++g)
-        base[g] = listed ? 0
-                         : slot_of(min(t * MLA_KT + 16 * g, (L - 1) & ~15)) -
-                               16 * g;
-#pragma unroll
-      for (int i = 0; i < CPW; ++i) {
-        const int k = wid + W * i;
-        const int ch = k * 64 + ln;
-        const int row = ch / MLA_CH;
-        const int at = row * MLA_DK + chunk_at(row, ch % MLA_CH) * 8;
-        const uint8_t* src = (const uint8_t*)cache;
+      for (int g = 0; g < RPW / 8; ++g)
+        slots[g] = slot_of(min(t * MLA_KT + wid * RPW + g * 8, (L - 1) & ~7));
+    };
+    // copy i: use(i, place in the buffer, uniform base, values from there of a lane)
+    auto copy_of = [&](int i, auto&& use) INL {
+      const int g = i / 9, k = i % 9;      // k 0 .. 7: a row, 8: the rope of eight
+      const int r0 = wid * RPW + g * 8;
+      const int b3 = RPW == 8 ? bit3 : g;
+      if (k < 8) {
+        const int slot = SPARSE && listed
+                             ? __builtin_amdgcn_readlane(mine, r0 + k)
+                             : slots[g] + k;
+        use(i, (r0 + k) * MLA_ROW,
+            (const uint8_t*)cache + (int64_t)slot * (MLA_DK * ESZ),
+            (lane ^ (2 * k) ^ b3 * 9) * 8);
+      } else {
+        const int r = lane >> 3;
+        const int ch = (lane & 7) ^ (r & 6) ^ b3 * 5;
         if (SPARSE && listed) {
-          const int slot = __shfl(mine, row, WAVE_SIZE) - row;
-          src += ((int64_t)slot * MLA_DK + at) * ESZ;
+          const int slot = __shfl(mine, r0 + r, WAVE_SIZE);
+          use(i, MLA_KT * MLA_ROW + r0 * MLA_PE,
+              (const uint8_t*)cache + (int64_t)slot * (MLA_DK * ESZ),
+              MLA_R + ch * 8);
         } else {
-          const int b = k < 36 ? (k < 18 ? base[0] : base[1])
-                               : (k < 54 ? base[2] : base[3]);
-          src += (int64_t)b * (MLA_DK * ESZ);
-          src += (uint32_t)(at * ESZ);
+          use(i, MLA_KT * MLA_ROW + r0 * MLA_PE,
+              (const uint8_t*)cache + (int64_t)slots[g] * (MLA_DK * ESZ),
+              r * MLA_DK + MLA_R + ch * 8);
         }
-        use(i, k, src);
       }
     };
-    auto issue = [&](int t, uint16_t* S) INL {
-      each_copy(t, [&](int, int k, const uint8_t* src) INL {
-        copy16_to_lds(src, S + k * 512);
+    auto issue = [&](int i, int buf) INL {
+      copy_of(i, [&](int i, int place, const uint8_t* base, int off) INL {
+        const uint32_t at = s_at + buf * BUF + place;
+        if (SPARSE && listed && i % 9 == 8) copy16(base + off * ESZ, at);
+        else copy16(base, off * ESZ, at);
       });
     };
     uint64_t raw[KV_FP8 ? CPW : 1];
-    auto fetch8 = [&](int t) INL {
-      each_copy(t, [&](int i, int, const uint8_t* src) INL {
-        raw[KV_FP8 ? i : 0] = *(const uint64_t*)src;
-      });
-    };
-    auto widen8 = [&](uint16_t* S) INL {
-      int at = lane * 8;
-      asm volatile("" : "+v"(at));
+    auto fetch8 = [&] INL {
 #pragma unroll
-      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i) {
-        int4 v;
-        fp8x8_to_bf16x8(raw[i], c_scale, reinterpret_cast<uint16_t*>(&v));
-        *reinterpret_cast<int4*>(S + (wid + W * i) * 512 + at) = v;
-      }
+      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i)
+        copy_of(i, [&](int i, int, const uint8_t* base, int off) INL {
+          raw[KV_FP8 ? i : 0] = *(const uint64_t*)(base + (uint32_t)off);
+        });
+    };
+    auto widen8 = [&](int buf) INL {
+#pragma unroll
+      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i)
+        copy_of(i, [&](int i, int place, const uint8_t*, int) INL {
+          int4 v;
+          fp8x8_to_bf16x8(raw[KV_FP8 ? i : 0], c_scale,
+                          reinterpret_cast<uint16_t*>(&v));
+          *reinterpret_cast<int4*>(S + buf * BUF + place + lane * 16) = v;
+        });
     };
 
     // ---- one tile --------------------------------------------------------------------
-    auto compute = [&](int t, uint16_t* S) INL {
+    // copy(n): the copies of the next tile that go with batch n of S^T's products
+    auto compute = [&](int t, const int buf, auto&& copy) INL {
+      uint8_t* T = S + buf * BUF;
       // rows that stand for a token, one bit each
       uint64_t alive = ~0ull;
       if (listed) {
@@ -317,20 +342,17 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
         alive = (1ull << (dom - t * MLA_KT)) - 1;
       }
       if (alive != ~0ull) {  // the others may hold anything: weight 0 times it
-        int i0 = tid;
-        asm volatile("" : "+v"(i0));
-        for (int i = i0; i < MLA_KT * MLA_CH; i += W * 64)
-          if (!((alive >> (i / MLA_CH)) & 1))
-            *reinterpret_cast<int4*>(S + i * 8) = make_int4(0, 0, 0, 0);
+        constexpr int CH = (MLA_ROW + MLA_PE) / 16;
+        for (int i = tid; i < MLA_KT * CH; i += W * 64) {
+          const int row = i / CH, ch = i % CH;
+          if (!((alive >> row) & 1))
+            *reinterpret_cast<int4*>(
+                T + (ch < 64 ? row * MLA_ROW + ch * 16
+                             : MLA_KT * MLA_ROW + row * MLA_PE + (ch - 64) * 16)) =
+                make_int4(0, 0, 0, 0);
+        }
         __syncthreads();
       }
-      if (head0 >= H) return;  // copies only
-
-      // opaque, or the addresses of every buffer are kept in registers
-      int qk[2] = {qk_at[0], qk_at[1]};
-      int tr[4] = {tr_at[0], tr_at[1], tr_at[2], tr_at[3]};
-      asm volatile("" : "+v"(qk[0]), "+v"(qk[1]), "+v"(tr[0]), "+v"(tr[1]),
-                   "+v"(tr[2]), "+v"(tr[3]));
       // Operands come in batches, the next one under way while this one's
       // products run: one read at a time would wait out the LDS each time.
       auto landed = [] INL {
@@ -338,35 +360,76 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         __builtin_amdgcn_sched_barrier(0);
       };
-      constexpr int KB = KV_FP8 ? 1 : 2;  // of the 18 steps of S^T
+      constexpr int KB = KV_FP8 ? 1 : 3;  // of the 18 steps of S^T
+      constexpr int NB = MLA_DK / 32 / KB;
       constexpr int TU = MLA_KT / 16;
+      const bool on = head0 < H;  // a wave without heads copies only
       f32x4v s[TU] = {};
-      {
-        bf16x8v a[2][KB][TU];
+      if (on) {
+        bf16x8v a[2][KB][TU / 2];
         auto fetch = [&](int n) INL {
 #pragma unroll
           for (int i = 0; i < KB; ++i)
 #pragma unroll
-            for (int u = 0; u < TU; ++u) {
+            for (int u = 0; u < TU / 2; ++u) {
               const int ks = n * KB + i;
               a[n & 1][i][u] = *reinterpret_cast<const bf16x8v*>(
-                  S + qk[ks & 1] + (ks >> 1) * 64 + u * 16 * MLA_DK);
+                  T + (ks < 16 ? (qk_at ^ (ks & 3) * 64) + (ks >> 2) * 256 +
+                                     u * 16 * MLA_ROW
+                               : (pe_at ^ (ks & 1) * 64) + u * 16 * MLA_PE));
             }
         };
         fetch(0);
 #pragma unroll
-        for (int n = 0; n < MLA_DK / 32 / KB; ++n) {
+        for (int n = 0; n < NB; ++n) {
           landed();
-          if (n + 1 < MLA_DK / 32 / KB) fetch(n + 1);
+          if (n + 1 < NB) fetch(n + 1);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int i = 0; i < KB; ++i)
+          for (int i = 0; i < KB; ++i) {
 #pragma unroll
-            for (int u = 0; u < TU; ++u)
+            for (int u = 0; u < TU / 2; ++u)
               s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                   a[n & 1][i][u], qf[n * KB + i], s[u], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            copy(n * KB + i);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
+#pragma unroll
+        for (int u = 0; u < TU / 2; ++u) X[wid][u][lane] = s[u];
+      } else {
+#pragma unroll
+        for (int i = 0; i < NB * KB; ++i) copy(i);
       }
+      // the scores of every wave are there; copies stay in flight
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (!on) return;
+#pragma unroll
+      for (int u = 0; u < TU; ++u)
+        s[u] = X[(wid & ~1) + u / (TU / 2)][u % (TU / 2)][lane];
+      // O^T's first operands are on their way beside the softmax
+      constexpr int DB = 2;  // of a wave's latent tiles
+      bf16x8v va[2][DB][TU / 2];
+      auto fetch_v = [&](int n) INL {
+#pragma unroll
+        for (int i = 0; i < DB; ++i)
+#pragma unroll
+          for (int u = 0; u < TU / 2; ++u) {
+            const int d = n * DB + i;
+            uint8_t* src = T + (tr_at ^ (d & 7) * 32) + (d >> 3) * 256 +
+                           u * 32 * MLA_ROW;
+            const s16x4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4v*)src);
+            const s16x4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4v*)(src + 16 * MLA_ROW));
+            va[n & 1][i][u] =
+                __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          }
+      };
       float mx = kHidden;
       if (alive == ~0ull) {
 #pragma unroll
@@ -414,68 +477,57 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
 
       // O^T: rows = 16 latent values, contraction over tokens 4 l4 + (0..3) and
       // 16 more: what lane group l4 of S^T holds
-      constexpr int DB = 2;  // of a wave's latent tiles
-      {
-        bf16x8v a[2][DB][TU / 2];
-        auto fetch = [&](int n) INL {
+      fetch_v(0);
+#pragma unroll
+      for (int n = 0; n < MLA_DT / DB; ++n) {
+        landed();
+        if (n + 1 < MLA_DT / DB) fetch_v(n + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < TU / 2; ++u)
 #pragma unroll
           for (int i = 0; i < DB; ++i)
-#pragma unroll
-            for (int u = 0; u < TU / 2; ++u) {
-              const int d = n * DB + i;
-              uint16_t* src =
-                  S + tr[d & 3] + (d >> 2) * 64 + u * 32 * MLA_DK;
-              const s16x4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                  (__attribute__((address_space(3))) s16x4v*)src);
-              const s16x4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                  (__attribute__((address_space(3))) s16x4v*)(src +
-                                                              16 * MLA_DK));
-              a[n & 1][i][u] =
-                  __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            }
-        };
-        fetch(0);
-#pragma unroll
-        for (int n = 0; n < MLA_DT / DB; ++n) {
-          landed();
-          if (n + 1 < MLA_DT / DB) fetch(n + 1);
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int u = 0; u < TU / 2; ++u)
-#pragma unroll
-            for (int i = 0; i < DB; ++i)
-              acc[n * DB + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  a[n & 1][i][u], b[u], acc[n * DB + i], 0, 0, 0);
-        }
+            acc[n * DB + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                va[n & 1][i][u], b[u], acc[n * DB + i], 0, 0, 0);
       }
     };
 
-    // ---- the run, one barrier a tile -----------------------------------------------
-    // Behind it this tile is in LDS, and every wave has left the buffer that the
-    // next one goes to.
+    // ---- the run -----------------------------------------------------------------------
+    // Behind a turn's first barrier this tile is in LDS, and every wave has left the
+    // buffer that the next one goes to. Past the run's end nothing is copied.
     __syncthreads();  // the buffers may still be read for the last sequence
-    auto turn = [&](int t, uint16_t* S, uint16_t* Sn) INL {
+    auto turn = [&](int t, const int buf) INL {
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's copies
       __syncthreads();
       const bool more = t + 1 < t1;
       if (more) {
-        if constexpr (KV_FP8) fetch8(t + 1);
-        else issue(t + 1, Sn);
+        look_up(t + 1);
+        if constexpr (KV_FP8) fetch8();
       }
-      compute(t, S);
+      compute(t, buf, [&](int n) INL {
+        if constexpr (!KV_FP8) {
+          constexpr int N = MLA_DK / 32;
+          if (more)
+#pragma unroll
+            for (int i = 0; i < CPW; ++i)
+              if (i * N / CPW == n) issue(i, buf ^ 1);
+        }
+      });
       if constexpr (KV_FP8)
-        if (more) widen8(Sn);
+        if (more) widen8(buf ^ 1);
     };
+    look_up(t0);
     if constexpr (KV_FP8) {
-      fetch8(t0);
-      widen8(S0);
+      fetch8();
+      widen8(0);
     } else {
-      issue(t0, S0);
+#pragma unroll
+      for (int i = 0; i < CPW; ++i) issue(i, 0);
     }
     for (int t = t0; t < t1;) {
-      turn(t, S0, S1);
+      turn(t, 0);
       if (++t >= t1) break;
-      turn(t, S1, S0);
+      turn(t, 1);
       ++t;
     }
 
