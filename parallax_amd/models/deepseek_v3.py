@@ -20,7 +20,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..parallel.comm import get_comm
-from ..parallel.layers import ColumnParallelLinear, RowParallelLinear
+from ..parallel.layers import ColumnParallelLinear, RowParallelLinear, plain_call
 from .config import ModelConfig
 from .forward_meta import ForwardMeta
 from .llama import LlamaMLP, LlamaShardModel, RMSNorm
@@ -91,16 +91,21 @@ class MLAAttention(nn.Module):
         q_nope, q_pe = q[..., : self.dn], q[..., self.dn :]
 
         kv_a = ops.linear(x, self.kv_a_proj_with_mqa.weight)
-        latent = self.kv_a_layernorm(kv_a[:, : self.r])
-        k_pe = kv_a[:, self.r :].unsqueeze(1)  # [T, 1, dr]
-
-        q_pe = q_pe.contiguous()
-        k_pe = k_pe.contiguous()
-        ops.rope_inplace(q_pe, k_pe, meta.positions, rope_cache,
-                         is_neox=self.rope_neox)
-
         cache = meta.mla_cache.layer(self.local_layer_idx)
-        ops.mla_reshape_and_cache(latent, k_pe.squeeze(1), cache, meta.slot_mapping)
+        norm, pe = self.kv_a_layernorm, q_pe
+        q_pe = None
+        if plain_call(norm, RMSNorm.forward):  # a hook sees the latent rows
+            q_pe = ops.mla_rope_and_cache(
+                pe, kv_a, norm.weight, norm.eps, meta.positions, rope_cache, cache,
+                meta.slot_mapping, is_neox=self.rope_neox)
+        if q_pe is None:
+            latent = norm(kv_a[:, : self.r])
+            q_pe = pe.contiguous()
+            k_pe = kv_a[:, self.r :].unsqueeze(1).contiguous()  # [T, 1, dr]
+            ops.rope_inplace(q_pe, k_pe, meta.positions, rope_cache,
+                             is_neox=self.rope_neox)
+            ops.mla_reshape_and_cache(latent, k_pe.squeeze(1), cache,
+                                      meta.slot_mapping)
 
         if meta.is_prefill:
             attn = self._prefill_attention(q_nope, q_pe, meta, cache)

@@ -163,6 +163,28 @@ def mla_reshape_and_cache(
     ref.mla_reshape_and_cache(kv_latent, k_rope, cache, slot_mapping)
 
 
+def mla_rope_and_cache(
+    q_pe: torch.Tensor,        # [T, H, DR] (a view into q)
+    kv: torch.Tensor,          # [T, R + DR]
+    norm_weight: torch.Tensor,  # [R]
+    eps: float,
+    positions: torch.Tensor,
+    cos_sin: torch.Tensor,
+    cache: torch.Tensor,
+    slot_mapping: torch.Tensor,
+    is_neox: bool = True,
+) -> Optional[torch.Tensor]:
+    """q_pe rotated, as rows of its own; kv's latent, RMS-normed, and its rotated key
+    into the latent cache, in one launch. None where there is no kernel (CPU, other
+    types, layouts or a gradient to be taken)."""
+    if not q_pe.is_cuda or (torch.is_grad_enabled() and (
+            q_pe.requires_grad or kv.requires_grad or norm_weight.requires_grad)):
+        return None
+    return _require_ext("mla_rope_and_cache").mla_rope_and_cache(
+        q_pe, kv, norm_weight, eps, positions.to(torch.int32), cos_sin, cache,
+        slot_mapping.to(torch.int64), is_neox)
+
+
 # -- attention ---------------------------------------------------------------------
 
 

@@ -33,6 +33,10 @@ void launch_reshape_and_cache(const void*, const void*, void*, void*,
 void launch_mla_reshape_and_cache(const void*, const void*, void*,
                                   const int64_t*, int, int, int, int, bool,
                                   float, hipStream_t);
+void launch_mla_rope_and_cache(void*, const void*, const void*, const void*, void*,
+                               const int*, const float*, const int64_t*, int, int,
+                               int, int, int64_t, int64_t, int64_t, float, bool,
+                               bool, hipStream_t);
 void launch_act_and_mul(void*, const void*, int64_t, int, bool, hipStream_t);
 void launch_paged_attention_decode(void*, const void*, const void*, const void*,
                                    const int*, const int*, int, int, int, int,
@@ -233,6 +237,47 @@ void mla_reshape_and_cache(torch::Tensor latent, torch::Tensor k_rope,
                                cache.data_ptr(),
                                slot_mapping.data_ptr<int64_t>(), T, R, DR, BS,
                                is_fp8(cache), 1.0f, cur_stream());
+}
+
+// rotated q [T, H, DR]; kv's normed latent and rotated key go to the cache. None where
+// there is no kernel.
+std::optional<torch::Tensor> mla_rope_and_cache(
+    torch::Tensor q, torch::Tensor kv, torch::Tensor w, double eps,
+    torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor cache,
+    torch::Tensor slot_mapping, bool neox) {
+  CHECK_GPU(q);
+  if (q.dim() != 3 || kv.dim() != 2 || w.dim() != 1 || cache.dim() != 3 ||
+      cos_sin.dim() != 2 || positions.dim() != 1 || slot_mapping.dim() != 1)
+    return std::nullopt;
+  const int64_t T = q.size(0), H = q.size(1), DR = q.size(2), R = w.size(0);
+  auto at16 = [](const torch::Tensor& t) {
+    return (uintptr_t)t.data_ptr() % 16 == 0;
+  };
+  if (q.scalar_type() != at::kBFloat16 || kv.scalar_type() != at::kBFloat16 ||
+      w.scalar_type() != at::kBFloat16 ||
+      (cache.scalar_type() != at::kBFloat16 && !is_fp8(cache)) ||
+      cos_sin.scalar_type() != at::kFloat ||
+      positions.scalar_type() != at::kInt ||
+      slot_mapping.scalar_type() != at::kLong || kv.size(0) != T ||
+      kv.size(1) != R + DR || positions.size(0) != T || slot_mapping.size(0) != T ||
+      cos_sin.size(1) != DR || cache.size(2) != R + DR)
+    return std::nullopt;
+  // pieces of 16 rotated values, at most a wave of them; vectors of 16 bytes
+  if (T == 0 || T > INT_MAX || H == 0 || R % 8 || DR % 16 || DR > 1024 ||
+      H * DR > 1 << 24 ||
+      q.stride(2) != 1 || q.stride(1) % 8 || q.stride(0) % 8 || kv.stride(1) != 1 ||
+      kv.stride(0) % 8 || !at16(q) || !at16(kv) || !at16(w) || !at16(cos_sin) ||
+      !at16(cache) || !w.is_contiguous() || !cache.is_contiguous() ||
+      !cos_sin.is_contiguous() || !positions.is_contiguous() ||
+      !slot_mapping.is_contiguous())
+    return std::nullopt;
+  auto out = torch::empty({T, H, DR}, q.options());
+  launch_mla_rope_and_cache(
+      out.data_ptr(), q.data_ptr(), kv.data_ptr(), w.data_ptr(), cache.data_ptr(),
+      positions.data_ptr<int>(), cos_sin.data_ptr<float>(),
+      slot_mapping.data_ptr<int64_t>(), T, H, R, DR, q.stride(0), q.stride(1),
+      kv.stride(0), (float)eps, neox, is_fp8(cache), cur_stream());
+  return out;
 }
 
 void silu_and_mul(torch::Tensor out, torch::Tensor x) {
@@ -971,6 +1016,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_and_cache", &rope_and_cache);
   m.def("reshape_and_cache", &reshape_and_cache);
   m.def("mla_reshape_and_cache", &mla_reshape_and_cache);
+  m.def("mla_rope_and_cache", &mla_rope_and_cache);
   m.def("silu_and_mul", &silu_and_mul);
   m.def("gelu_and_mul", &gelu_and_mul);
   m.def("paged_attention_decode", &paged_attention_decode);

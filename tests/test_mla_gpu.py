@@ -280,3 +280,31 @@ def test_mla_prefill_operands_in_other_orders_left_to_the_caller():
         (z(40, 16, 128), rows[:39], w, w),      # a portion longer than its context
     ):
         assert not ops.mla_prefill_attention(out, q, pe, r, uk, uv, 1.0)
+
+
+@pytest.mark.parametrize("T,H,R,DR", [(1, 128, 512, 64), (5, 3, 64, 16), (70, 16, 512, 64),
+                                      (3, 33, 1032, 128)])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("neox", [False, True])
+def test_mla_rope_and_cache(T, H, R, DR, fp8, neox):
+    """The same bits as its five steps: sums of squares run in the same order."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    q, kv, w = rand(T, H, DR + 32)[..., 32:], rand(T, R + DR + 8)[:, :R + DR], rand(R)
+    table = torch.randn(90, DR, generator=g, device="cuda")
+    pos = torch.randint(0, 90, (T,), generator=g, device="cuda", dtype=torch.int32)
+    slots = torch.randperm(96, generator=g, device="cuda")[:T]
+    slots[T // 2] = -1
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    caches = [torch.zeros(6, 16, R + DR, device="cuda").to(dt) for _ in range(2)]
+    got = ops.mla_rope_and_cache(q, kv, w, 1e-6, pos, table, caches[0], slots, neox)
+    pe, k = q.contiguous(), kv[:, R:].unsqueeze(1).contiguous()
+    ops.rope_inplace(pe, k, pos, table, is_neox=neox)
+    ops.mla_reshape_and_cache(ops.rmsnorm(kv[:, :R], w, 1e-6), k.squeeze(1), caches[1],
+                              slots)
+    assert torch.equal(got, pe)
+    assert torch.equal(caches[0].view(torch.uint8), caches[1].view(torch.uint8))
+    args = (w, 1e-6, pos, table, caches[0], slots, neox)
+    assert ops.mla_rope_and_cache(q.float(), kv, *args) is None
+    assert ops.mla_rope_and_cache(q[..., :DR - 8], kv, *args) is None
+    assert ops.mla_rope_and_cache(q, kv[:, 1:], *args) is None
