@@ -139,7 +139,10 @@ class MLAAttention(nn.Module):
             q_nope.shape[0], H, dv, dtype=q_nope.dtype, device=q_nope.device
         )
         t0 = 0
-        lens = zip(meta.query_lens.tolist(), meta.seq_lens.tolist())
+        if meta.portions is not None:  # known here: no wait for the device
+            lens = [(n, first + n) for first, n in meta.portions]
+        else:
+            lens = list(zip(meta.query_lens.tolist(), meta.seq_lens.tolist()))
         for i, (QL, L) in enumerate(lens):
             nb = (L + bs - 1) // bs
             entries = cache[meta.block_tables[i, :nb].long()].reshape(nb * bs, -1)[:L]

@@ -79,23 +79,34 @@ class DecodeGraphRunner:
         B = self.buckets[-1]
 
         dev = device
-        self.input_ids = torch.zeros(B, dtype=torch.long, device=dev)
+        # What a step brings lies in one buffer, here (pinned) and on the device: one
+        # copy, or one of all but the input ids, which come last, where those are on
+        # the device already. A copy takes 4 us of a step however short it is.
+        self._step = torch.zeros(24 * B, dtype=torch.uint8, device=dev)
+        self._h_step = torch.zeros(24 * B, dtype=torch.uint8, pin_memory=True)
+        self._without_ids = 16 * B
+
+        def views(buf):
+            return (buf[: 8 * B].view(torch.int64), buf[8 * B : 12 * B].view(torch.int32),
+                    buf[12 * B : 16 * B].view(torch.int32),
+                    buf[16 * B :].view(torch.int64))
+
+        self.slot_mapping, self.positions, self.seq_lens, self.input_ids = \
+            views(self._step)
+        self.slot_mapping.fill_(-1)
+        self.seq_lens.fill_(1)
         # models whose embedding reads the (previous token, token) pair
         self.uses_prev = bool(getattr(model, "uses_prev_tokens", False))
         self.prev_ids = torch.full((B,), -1, dtype=torch.long, device=dev)
         self.h_prev_ids = torch.full((B,), -1, dtype=torch.long, pin_memory=True)
         self.hidden_in = torch.zeros(B, hidden_size, dtype=dtype, device=dev)
-        self.positions = torch.zeros(B, dtype=torch.int32, device=dev)
-        self.slot_mapping = torch.full((B,), -1, dtype=torch.int64, device=dev)
         self.block_tables = torch.zeros(B, self.max_blocks, dtype=torch.int32, device=dev)
-        self.seq_lens = torch.ones(B, dtype=torch.int32, device=dev)
-        # pinned host staging (one copy per step)
-        self.h_input_ids = torch.zeros(B, dtype=torch.long, pin_memory=True)
-        self.h_positions = torch.zeros(B, dtype=torch.int32, pin_memory=True)
-        self.h_slot_mapping = torch.full((B,), -1, dtype=torch.int64, pin_memory=True)
+        self.h_slot_mapping, self.h_positions, self.h_seq_lens, self.h_input_ids = \
+            views(self._h_step)
+        self.h_slot_mapping.fill_(-1)
+        self.h_seq_lens.fill_(1)
         self.h_block_tables = torch.zeros(B, self.max_blocks, dtype=torch.int32,
                                           pin_memory=True)
-        self.h_seq_lens = torch.ones(B, dtype=torch.int32, pin_memory=True)
         if linear_cache is not None:
             self.linear_slots = torch.full((B,), linear_scratch_slot,
                                            dtype=torch.int64, device=dev)
@@ -280,8 +291,7 @@ class DecodeGraphRunner:
                 # what that step was fed is this step's predecessor
                 self.prev_ids[:B].copy_(self.input_ids[:B])
         if input_ids_dev is None:
-            self.input_ids[:bucket].copy_(self.h_input_ids[:bucket],
-                                          non_blocking=True)
+            self._step.copy_(self._h_step, non_blocking=True)
         else:
             # async decode: previous step's sampled tokens feed this step's
             # input ids without a host round-trip (device-to-device, ordered
@@ -290,9 +300,8 @@ class DecodeGraphRunner:
             if bucket > B:
                 self.input_ids[B:bucket].copy_(self.h_input_ids[B:bucket],
                                                non_blocking=True)
-        self.positions[:bucket].copy_(self.h_positions[:bucket], non_blocking=True)
-        self.slot_mapping[:bucket].copy_(self.h_slot_mapping[:bucket], non_blocking=True)
-        self.seq_lens[:bucket].copy_(self.h_seq_lens[:bucket], non_blocking=True)
+            self._step[: self._without_ids].copy_(self._h_step[: self._without_ids],
+                                                  non_blocking=True)
         if self.linear_cache is not None:
             self.h_linear_slots[:B] = torch.tensor(
                 linear_slots or [self.linear_scratch_slot] * B, dtype=torch.int64
