@@ -13,20 +13,34 @@
 // of the second product. P never touches LDS and a wave's softmax needs no
 // other wave, which leaves one barrier a tile.
 //
-// bf16 tiles are copied global -> LDS directly (16 bytes a lane), the next
-// tile while this one is computed; an fp8 cache passes through registers, where
-// it is widened. 16-byte chunks are placed XOR-swizzled by row: a quarter wave
-// reads 16 rows of one chunk column from 16 different bank groups.
+// bf16 tiles are copied global -> LDS directly (16 bytes a lane), a turn before
+// their use; an fp8 cache passes through registers, where it is widened. 16-byte
+// chunks are placed XOR-swizzled by row: a quarter wave reads 16 rows of one chunk
+// column from 16 different bank groups.
 //
-// What bounds it: per tile and wave 1024 matrix-core cycles (D = 128), about
-// as many VALU cycles of softmax and as many LDS cycles for four waves; two
-// workgroups a CU overlap them. The accumulators are rescaled only when an
-// item's maximum moved, the mask is applied only in tiles that the diagonal, the
-// window or the end of the sequence cuts.
+// A turn takes the scores of one tile and the values of the tile before, whose
+// weights depend on nothing of this turn. For 128-wide heads the two are interleaved
+// by hand, matrix instruction by matrix instruction, where no mask cuts the tile: two
+// waves a SIMD (240 registers) keep the matrix cores busy for 52% of the cycles
+// instead of 40. For 64-wide heads, where softmax outweighs the products, a second
+// set of scores costs the third wave a SIMD, and the turn goes through the two one
+// after the other (interleaved 255 us for 4,500 rows of 64 heads over 8, apart 254;
+// 3,000 rows with a window of 128 35.5 and 30).
+//
+// What bounds it: power. Per tile and wave 1024 matrix-core cycles (D = 128), about
+// as many VALU cycles, half as many of the LDS for four waves; with operands of
+// zeros the same instructions run at 1,410 TFLOP/s, with normal values the clock
+// falls to 1.65 GHz. The accumulators are rescaled only when an item's maximum moved,
+// the mask is applied only in tiles that the diagonal, the window or the end of the
+// sequence cuts.
 //
 // Measured (MI355X, bf16, 32 heads over 8 of 128, 8192 rows in two portions on
-// prefixes of up to 20,000): 3.5 ms = 870 TFLOP/s of what the mask leaves;
-// 16.6 ms with 32-row tiles of one head, P through LDS and six barriers a tile.
+// prefixes of up to 20,000): 3.00 ms among other work and 2.62 again and again =
+// 890 and 1,015 TFLOP/s of what the mask leaves; scores and values of one tile in turn,
+// with a branch and a wait at every operand of V, 3.47 and 2.99 ms. 5,700 rows on an fp8 cache 425 to 338 us (conversions by the hardware's
+// rounding), 64-wide heads 340 to 274; 8,192 rows without a prefix 228 to 213.
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -71,6 +85,20 @@ DEVINL uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, p);
 }
 
+// 8 e4m3 values, scaled, to bf16
+DEVINL u32x4v widen(uint64_t raw, float scale) {
+  u32x4v r;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int b = (int)(uint32_t)(raw >> (32 * i));
+    const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(b, false);
+    const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(b, true);
+    r[2 * i] = pack_bf16(lo[0] * scale, lo[1] * scale);
+    r[2 * i + 1] = pack_bf16(hi[0] * scale, hi[1] * scale);
+  }
+  return r;
+}
+
 DEVINL void copy16_to_lds(const void* src, void* dst) {
   __builtin_amdgcn_global_load_lds(
       (const __attribute__((address_space(1))) void*)src,
@@ -79,10 +107,12 @@ DEVINL void copy16_to_lds(const void* src, void* dst) {
 
 }  // namespace
 
-// FIXED: the page size is 1 << bs_shift, of 16, 32 or 64 tokens; otherwise it is
-// bs_shift itself, a multiple of 8.
+// FIXED: the page size is 1 << bs_shift, of 16, 32 or 64 tokens, and a page of all
+// heads has less than 2^32 values; otherwise the page size is bs_shift itself, a
+// multiple of 8.
 template <int D, bool KV_FP8, bool FIXED>
-__global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
+__global__ __launch_bounds__(PF_THREADS, D == 64 ? 3 : 2)
+void prefill_attention_kernel(
     uint16_t* __restrict__ out,            // [T, Hq, D]
     float* __restrict__ tmp_acc,           // [T, Hq, splits, D] or null
     float* __restrict__ tmp_ml,            // [T, Hq, splits, 2]
@@ -230,7 +260,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
   // or two of 64; a V row has 64 tokens, so two as well
   auto k_swz = [](int r) { return D == 128 ? r & 15 : (r >> 1) & 7; };
   const int BS = FIXED ? 1 << bs_shift : bs_shift;
-  const size_t page_elems = (size_t)Hk * BS * D;
+  const uint32_t page_elems = (uint32_t)Hk * BS * D;  // FIXED only
   // chunk i of a thread: its row of the tile and the chunk that belongs there
   auto k_row = [&](int i) { return ((wid * KPER + i) * 64 + lane) / KCH; };
   auto k_src = [&](int i) { return (lane % KCH) ^ k_swz(k_row(i)); };
@@ -238,7 +268,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
   auto v_src = [&](int i) { return (lane & 7) ^ ((v_row(i) >> 1) & 7); };
   // FIXED: 16 K rows of a wave lie in one page, a V chunk column changes with
   // the parity of i only, and the place in a page is the same for every tile.
-  // Page numbers are fetched a tile ahead of the copies that need them.
+  // Page numbers are fetched a turn ahead of the copies that need them.
   // Tokens past the end are hidden later; their addresses stay inside a page
   // of the sequence.
   int koff[KPER], voff[VPER];
@@ -251,109 +281,99 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
       voff[i] = (hk * D + v_row(i)) * BS + ((v_src(i) * 8) & (BS - 1));
   }
   int kpage = 0, vpage[2] = {0, 0};
-  auto pages = [&](int kt) {
+  auto pages = [&](int kt, int vt) {  // of K's tile kt and V's tile vt
     if (!FIXED) return;
     kpage = btab[min(kt * PF_KT + wid * 16, L - 1) >> bs_shift];
-    vpage[0] = btab[min(kt * PF_KT + v_src(0) * 8, L - 1) >> bs_shift];
-    vpage[1] = btab[min(kt * PF_KT + v_src(1) * 8, L - 1) >> bs_shift];
+    vpage[0] = btab[min(vt * PF_KT + v_src(0) * 8, L - 1) >> bs_shift];
+    vpage[1] = btab[min(vt * PF_KT + v_src(1) * 8, L - 1) >> bs_shift];
   };
   auto k_elem = [&](int kt, int i) -> size_t {
-    if (FIXED) return kpage * page_elems + koff[i];
+    if (FIXED) return (uint64_t)(uint32_t)kpage * page_elems + (uint32_t)koff[i];
     const int tok = min(kt * PF_KT + k_row(i), L - 1);
-    return btab[tok / BS] * page_elems + (hk * BS + tok % BS) * D +
+    return (size_t)btab[tok / BS] * Hk * BS * D + (hk * BS + tok % BS) * D +
            k_src(i) * 8;
   };
-  auto v_elem = [&](int kt, int i) -> size_t {
-    if (FIXED) return vpage[i & 1] * page_elems + voff[i];
+  auto v_elem = [&](int vt, int i) -> size_t {
+    if (FIXED)
+      return (uint64_t)(uint32_t)vpage[i & 1] * page_elems + (uint32_t)voff[i];
     // eight tokens of one page: BS is a multiple of 8
-    const int tok = min(kt * PF_KT + v_src(i) * 8, (L - 1) & ~7);
-    return btab[tok / BS] * page_elems + (hk * D + v_row(i)) * BS + tok % BS;
+    const int tok = min(vt * PF_KT + v_src(i) * 8, (L - 1) & ~7);
+    return (size_t)btab[tok / BS] * Hk * BS * D + (hk * D + v_row(i)) * BS +
+           tok % BS;
   };
-  auto issue = [&](int kt, uint16_t* Kl, uint16_t* Vl) {
+  auto copy_k = [&](int kt, uint16_t* Kl, int i) {
+    copy16_to_lds((const uint16_t*)k_cache + k_elem(kt, i),
+                  Kl + (wid * KPER + i) * 512);
+  };
+  auto copy_v = [&](int vt, uint16_t* Vl, int i) {
+    copy16_to_lds((const uint16_t*)v_cache + v_elem(vt, i),
+                  Vl + (wid * VPER + i) * 512);
+  };
+  auto issue_k = [&](int kt, uint16_t* Kl) {
 #pragma unroll
-    for (int i = 0; i < KPER; ++i)
-      copy16_to_lds((const uint16_t*)k_cache + k_elem(kt, i),
-                    Kl + (wid * KPER + i) * 512);
+    for (int i = 0; i < KPER; ++i) copy_k(kt, Kl, i);
+  };
+  auto issue_v = [&](int vt, uint16_t* Vl) {
 #pragma unroll
-    for (int i = 0; i < VPER; ++i)
-      copy16_to_lds((const uint16_t*)v_cache + v_elem(kt, i),
-                    Vl + (wid * VPER + i) * 512);
+    for (int i = 0; i < VPER; ++i) copy_v(vt, Vl, i);
   };
   uint64_t kraw[KV_FP8 ? KPER : 1], vraw[KV_FP8 ? VPER : 1];
-  auto fetch8 = [&](int kt) {
+  auto fetch_k = [&](int kt) {
 #pragma unroll
     for (int i = 0; i < KPER; ++i)
       kraw[i] = *reinterpret_cast<const uint64_t*>((const uint8_t*)k_cache +
                                                    k_elem(kt, i));
+  };
+  auto fetch_v = [&](int vt) {
 #pragma unroll
     for (int i = 0; i < VPER; ++i)
       vraw[i] = *reinterpret_cast<const uint64_t*>((const uint8_t*)v_cache +
-                                                   v_elem(kt, i));
+                                                   v_elem(vt, i));
   };
-  auto widen8 = [&](uint16_t* Kl, uint16_t* Vl) {
+  auto widen_k = [&](uint16_t* Kl) {
 #pragma unroll
-    for (int i = 0; i < KPER; ++i) {
-      int4 w;
-      fp8x8_to_bf16x8(kraw[i], k_scale, reinterpret_cast<uint16_t*>(&w));
-      *reinterpret_cast<int4*>(Kl + ((wid * KPER + i) * 64 + lane) * 8) = w;
-    }
+    for (int i = 0; i < KPER; ++i)
+      *reinterpret_cast<u32x4v*>(Kl + ((wid * KPER + i) * 64 + lane) * 8) =
+          widen(kraw[i], k_scale);
+  };
+  auto widen_v = [&](uint16_t* Vl) {
 #pragma unroll
-    for (int i = 0; i < VPER; ++i) {
-      int4 w;
-      fp8x8_to_bf16x8(vraw[i], v_scale, reinterpret_cast<uint16_t*>(&w));
-      *reinterpret_cast<int4*>(Vl + ((wid * VPER + i) * 64 + lane) * 8) = w;
-    }
+    for (int i = 0; i < VPER; ++i)
+      *reinterpret_cast<u32x4v*>(Vl + ((wid * VPER + i) * 64 + lane) * 8) =
+          widen(vraw[i], v_scale);
   };
 
   // operand rows: K row with bits 2 and 3 swapped (see the top), V row d
   const int krow = (l31 & 0x13) | ((l31 & 4) << 1) | ((l31 & 8) >> 1);
+  auto k_frag = [&](const uint16_t* Kl, int ks, int t) {
+    const int pos = (2 * ks + half) ^ k_swz(krow);
+    return *reinterpret_cast<const bf16x8v*>(Kl + (t * 32 + krow) * D + pos * 8);
+  };
+  auto v_frag = [&](const uint16_t* Vl, int ks, int t) {
+    const int d = t * 32 + l31;
+    const int pos = (2 * ks + half) ^ ((d >> 1) & 7);
+    return *reinterpret_cast<const bf16x8v*>(Vl + d * PF_KT + pos * 8);
+  };
 
-  auto compute = [&](int kt, const uint16_t* Kl, const uint16_t* Vl) {
-    const int kbase = kt * PF_KT;
-    if (!wave_on || kbase > wpos_hi) return;
-    if (window > 0 && kbase + PF_KT - 1 <= wpos_lo - window) return;
-
-    f32x16v s[2] = {};
+  float lsum = 0.f;
+  float mx = kLowest;  // of the scores whose weights come next
+  // weights of two tokens, part j of a B operand of 16
+  auto weigh = [&](const f32x16v (&s)[2], int ks, int j) {
+    const int r = (ks & 1) * 8 + 2 * j;
+    const float a = __builtin_amdgcn_exp2f(fmaf(s[ks >> 1][r], c, -m));
+    const float b = __builtin_amdgcn_exp2f(fmaf(s[ks >> 1][r + 1], c, -m));
+    lsum += a;
+    lsum += b;
+    return pack_bf16(a, b);
+  };
+  auto larger = [&](float mx, const f32x16v& s) {
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      const int pos = (2 * ks + half) ^ k_swz(krow);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const bf16x8v a = *reinterpret_cast<const bf16x8v*>(
-            Kl + (t * 32 + krow) * D + pos * 8);
-        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], s[t], 0, 0,
-                                                       0);
-      }
-    }
-
-    if (softcap > 0.f) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s[t][r] = softcap * tanhf(s[t][r] * fabsf(scale) / softcap) * kLog2e;
-    }
-    const bool inside = kbase + PF_KT - 1 <= wpos_lo &&
-                        (window <= 0 || kbase > wpos_hi - window);
-    if (!inside) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int tok = kbase + 32 * t + 16 * (r >> 3) + 8 * half + (r & 7);
-          const bool seen = tok <= qpos && (window <= 0 || tok > qpos - window);
-          s[t][r] = seen ? s[t][r] : kHidden;
-        }
-    }
-
-    float mx = s[0][0];
-#pragma unroll
-    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[0][r]);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[1][r]);
-    mx = max_halves(mx) * c;
-    // rescaled when a maximum moved: its own weight is then 1, without rounding (only
-    // when it moved by 2^8: 2% more error)
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    return mx;
+  };
+  // rescaled when a maximum moved: its own weight is then 1, without rounding (only
+  // when it moved by 2^8: 2% more error)
+  auto raise = [&](float mx) {
     if (__any(mx > m)) {
       const float m2 = fmaxf(m, mx);
       const float f = __builtin_amdgcn_exp2f(m - m2);
@@ -364,66 +384,201 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attention_kernel(
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[t][r] *= f;
     }
+  };
 
-    const bool past = kbase + PF_KT > L;  // uniform
-    float lsum = 0.f;
+  // ---- the tiles ------------------------------------------------------------------
+  // The tiles that this wave's items see; the others are copied for the rest of the
+  // workgroup.
+  int on_begin = kt_begin, on_end = min(kt_end, (wpos_hi >> 6) + 1);
+  if (window > 0) on_begin = max(on_begin, (wpos_lo - window + 1) >> 6);
+  if (!wave_on) on_end = on_begin;
+
+  auto hide = [&](int kbase, f32x16v (&s)[2]) {  // what the mask leaves out
+    int last = qpos - kbase - 8 * half;  // the last token that is seen
+    asm volatile("" : "+v"(last));  // not computed where no mask is applied
+    const int first = window > 0 ? last - window : -1 << 30;  // and the one before all
 #pragma unroll
-    for (int ks = 0; ks < PF_KT / 16; ++ks) {
-      float p[8];
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        p[j] = __builtin_amdgcn_exp2f(
-            fmaf(s[ks >> 1][(ks & 1) * 8 + j], c, -m));
-        lsum += p[j];
+      for (int r = 0; r < 16; ++r) {
+        const int tok = 32 * t + 16 * (r >> 3) + (r & 7);
+        s[t][r] = tok <= last && tok > first ? s[t][r] : kHidden;
       }
-      u32x4v pk;
+  };
+
+  // tiles of [inner, outer) are seen whole
+  const int outer = (wpos_lo + 1) >> 6;
+  const int inner = window > 0 ? ((wpos_hi - window) >> 6) + 1 : 0;
+
+  // A turn takes the scores of tile kt and the weights and values of tile kt - 1.
+  // One barrier a turn: behind it K of tile kt and V of tile kt - 1 are in LDS, and
+  // every wave has left the buffers that the next ones go to.
+  auto meet = [&](auto left) {  // copies of this thread that may be under way
+    constexpr int n = decltype(left)::value;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070 | n);  // and lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  using none = std::integral_constant<int, 0>;
+  f32x16v s0[2] = {}, s1[2];
+
+  // Any turn: also the first and the last of this wave's tiles, a softcap, a mask.
+  auto cut_turn = [&](int kt, const uint16_t* Kl, uint16_t* Kn, const uint16_t* Vl,
+                      uint16_t* Vn) {
+    const int kbase = kt * PF_KT;
+    const bool more = kt < kt_end, first = kt == kt_begin;
+    if (first) meet(std::integral_constant<int, KV_FP8 ? 0 : KPER + VPER>{});
+    else meet(none{});
+    if (more) {  // past the last tile K's copy is the last again
+      if (first) {
+      } else if (KV_FP8) {
+        fetch_k(min(kt + 1, kt_end - 1));
+        fetch_v(kt);
+      } else {
+        issue_k(min(kt + 1, kt_end - 1), Kn);
+        issue_v(kt, Vn);
+      }
+      pages(min(kt + 2, kt_end - 1), kt + 1);
+    }
+    if (kt > on_begin && kt <= on_end) {
+      raise(mx);
+      const int n = L - kbase + PF_KT - 8 * half;  // tokens from this half's first
+      const bool past = kbase > L;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) pk[j] = pack_bf16(p[2 * j], p[2 * j + 1]);
-      const bf16x8v b = __builtin_bit_cast(bf16x8v, pk);
+      for (int ks = 0; ks < PF_KT / 16; ++ks) {
+        u32x4v w;
 #pragma unroll
-      for (int t = 0; t < DT; ++t) {
-        const int d = t * 32 + l31;
-        const int pos = (2 * ks + half) ^ ((d >> 1) & 7);
-        bf16x8v a =
-            *reinterpret_cast<const bf16x8v*>(Vl + d * PF_KT + pos * 8);
+        for (int j = 0; j < 4; ++j) w[j] = weigh(s0, ks, j);
+        bf16x8v a[DT];
+#pragma unroll
+        for (int t = 0; t < DT; ++t) a[t] = v_frag(Vl, ks, t);
         if (past) {  // a page's unused slots may hold anything
-          const int n = L - (kbase + 16 * ks + 8 * half);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) a[j] = j < n ? a[j] : (short)0;
+          for (int t = 0; t < DT; ++t)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              a[t][j] = 16 * ks + j < n ? a[t][j] : (short)0;
         }
-        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, o[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+          o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              a[t], __builtin_bit_cast(bf16x8v, w), o[t], 0, 0, 0);
       }
+      l += lsum;
+      lsum = 0.f;
     }
-    l += lsum;
+    if (kt >= on_begin && kt < on_end) {
+      s0[0] = s0[1] = f32x16v{};
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          s0[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k_frag(Kl, ks, t), qf[ks],
+                                                          s0[t], 0, 0, 0);
+      if (softcap > 0.f) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s0[t][r] =
+                softcap * tanhf(s0[t][r] * fabsf(scale) / softcap) * kLog2e;
+      }
+      if (kt < inner || kt >= outer) hide(kbase, s0);
+      mx = max_halves(larger(larger(s0[0][0], s0[0]), s0[1])) * c;
+    }
+    if (KV_FP8 && more) {
+      widen_k(Kn);
+      if (!first) widen_v(Vn);
+    }
   };
 
-  // ---- the tiles, two buffers in turn -------------------------------------------
-  // One barrier a tile: behind it this tile is in LDS and every wave has left
-  // the buffer that the next one goes to.
-  auto turn = [&](int kt, uint16_t* Kl, uint16_t* Vl, uint16_t* Kn,
-                  uint16_t* Vn) {
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's copies
-    __syncthreads();
-    const bool more = kt + 1 < kt_end;
-    if (more) {
-      if (KV_FP8) fetch8(kt + 1);
-      else issue(kt + 1, Kn, Vn);
-      pages(kt + 2);
+  // Tile kt seen whole, and tile kt - 1 one of this wave's. The order is the one that
+  // is written here, a matrix instruction and what fits beside it at a time, operands
+  // read AHEAD instructions early (2 to 8 measure the same); the compiler's own put
+  // every read right before its use.
+  auto whole_turn = [&](int kt, const uint16_t* Kl, uint16_t* Kn, const uint16_t* Vl,
+                        uint16_t* Vn, f32x16v (&sn)[2], const f32x16v (&sp)[2]) {
+    meet(none{});
+    raise(mx);
+    constexpr int S = 2 * KSTEPS, N = S + 4 * DT, AHEAD = 4;
+    const int k_next = min(kt + 1, kt_end - 1), k_page = min(kt + 2, kt_end - 1);
+    bf16x8v fr[AHEAD];
+    u32x4v w[4];
+    auto load = [&](int n) {
+      fr[n % AHEAD] = n < S ? k_frag(Kl, n % KSTEPS, n / KSTEPS)
+                            : v_frag(Vl, (n - S) / DT, (n - S) % DT);
+    };
+#pragma unroll
+    for (int n = 0; n < AHEAD; ++n) load(n);
+    if (KV_FP8) {
+      fetch_k(k_next);
+      fetch_v(kt);
+      pages(k_page, kt + 1);
     }
-    compute(kt, Kl, Vl);
-    if (KV_FP8 && more) widen8(Kn, Vn);
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (n < S) {
+        const int t = n / KSTEPS, ks = n % KSTEPS;
+        sn[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            fr[n % AHEAD], qf[ks], ks ? sn[t] : f32x16v{}, 0, 0, 0);
+      } else {
+        const int t = (n - S) % DT, ks = (n - S) / DT;
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            fr[n % AHEAD], __builtin_bit_cast(bf16x8v, w[ks]), o[t], 0, 0, 0);
+      }
+      if (n + AHEAD < N) load(n + AHEAD);
+      // 16 pairs of weights; each slice of four comes before its first product
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (u * (N - 4) / 16 == n) w[u / 4][u % 4] = weigh(sp, u / 4, u % 4);
+      if (!KV_FP8) {
+        if (n < KPER) copy_k(k_next, Kn, n);
+        else if (n - KPER < VPER) copy_v(kt, Vn, n - KPER);
+        else if (n == KPER + VPER) pages(k_page, kt + 1);
+      }
+      if (n == S) mx = larger(sn[0][0], sn[0]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    mx = max_halves(larger(mx, sn[1])) * c;
+    l += lsum;
+    lsum = 0.f;
+    if (KV_FP8) {
+      widen_k(Kn);
+      widen_v(Vn);
+    }
   };
-  pages(kt_begin);
+
+  const int whole = max(on_begin + 1, inner);
+  const int cut = softcap > 0.f ? 0 : min(on_end, outer);
+
+  // The first turn's K, and behind it what that turn would ask for: the buffers are
+  // free, and contexts of a few tiles are rows of such waits.
+  pages(kt_begin, kt_begin);
   if (KV_FP8) {
-    fetch8(kt_begin);
-    widen8(K0, V0);
+    fetch_k(kt_begin);
+    fetch_v(kt_begin);
+    pages(min(kt_begin + 1, kt_end - 1), kt_begin + 1);
+    widen_k(K0);
+    widen_v(V0);
+    fetch_k(min(kt_begin + 1, kt_end - 1));
   } else {
-    issue(kt_begin, K0, V0);
+    issue_k(kt_begin, K0);
+    pages(min(kt_begin + 1, kt_end - 1), kt_begin);
+    asm volatile("" ::: "memory");
+    issue_k(min(kt_begin + 1, kt_end - 1), K1);
+    issue_v(kt_begin, V0);
   }
-  pages(kt_begin + 1);
-  for (int kt = kt_begin; kt < kt_end; kt += 2) {
-    turn(kt, K0, V0, K1, V1);
-    if (kt + 1 < kt_end) turn(kt + 1, K1, V1, K0, V0);
+  for (int kt = kt_begin; kt <= kt_end; kt += 2) {
+    if constexpr (D == 128) {
+      for (; kt >= whole && kt + 1 < cut; kt += 2) {
+        whole_turn(kt, K0, K1, V1, V0, s1, s0);
+        whole_turn(kt + 1, K1, K0, V0, V1, s0, s1);
+      }
+    }
+    cut_turn(kt, K0, K1, V1, V0);
+    if (kt + 1 <= kt_end) cut_turn(kt + 1, K1, K0, V0, V1);
   }
 
   // ---- out: column = item, rows of O^T = d ---------------------------------------
@@ -476,7 +631,8 @@ extern "C" void launch_prefill_attention(
     bool* launched) {
   *launched = false;
   const int max_tiles = prefill_attention_tiles(T, B, Hq, Hk);
-  const bool fixed = BS == 16 || BS == 32 || BS == 64;
+  const bool fixed =
+      (BS == 16 || BS == 32 || BS == 64) && (int64_t)Hk * BS * D < 1ll << 32;
   const int bs = fixed ? __builtin_ctz(BS) : BS;
   dim3 grid(max_tiles * Hk, splits, 1);
 #define PF_LAUNCH(HD, FP8, P2)                                               \

@@ -190,3 +190,37 @@ def test_prefill_portion_without_context(fp8):
     want = ref.prefill_attention(q[keep].float(), kc.float(), vc.float(), bt[pick],
                                  sl[pick], ql[pick], 0.125)
     torch.testing.assert_close(out[keep].float(), want, atol=2.1e-2, rtol=0)
+
+
+@pytest.mark.parametrize("Hq,Hk,D,BS,fp8,window", [
+    (8, 2, 128, 32, False, -1),
+    (8, 2, 128, 16, False, 200),
+    (4, 4, 128, 64, False, 300),
+    (16, 2, 128, 24, False, -1),       # general page size
+    (16, 2, 128, 32, True, -1),
+    (8, 2, 128, 64, True, 200),
+    (16, 2, 64, 16, False, 200),
+    (16, 2, 64, 32, True, -1),
+])
+def test_prefill_contexts_of_few_tiles(Hq, Hk, D, BS, fp8, window):
+    """Contexts of every number of 64-key tiles from one to ten, ending at a tile's
+    edge and beside it: turns of pairs of tiles, the first and last turn alone, tiles
+    that the diagonal or the window cuts on either side of whole ones. Slots past the
+    end hold NaN. Tolerance as above."""
+    sl = sorted({64 * n + d for n in range(1, 11) for d in (-1, 0, 1, 32)})
+    ql = [min(n, 1 + 7 * i % 70) for i, n in enumerate(sl)]
+    q, kc, vc, bt, slt, qlt = _setup(ql, sl, Hq, Hk, D, BS=BS, seed=D + BS)
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+    ref_k, ref_v = kc.float(), vc.float()
+    for i, n in enumerate(sl):
+        if n % BS and not fp8:
+            page = int(bt[i, n // BS])
+            kc[page, :, n % BS:] = float("nan")
+            vc[page, :, :, n % BS:] = float("nan")
+    out = ops.prefill_attention(q, kc, vc, bt, slt, qlt, D ** -0.5,
+                                sliding_window=window)
+    want = ref.prefill_attention(
+        q.float().cpu(), ref_k.cpu(), ref_v.cpu(), bt.cpu(), slt.cpu(), qlt.cpu(),
+        D ** -0.5, sliding_window=window)
+    torch.testing.assert_close(out.float().cpu(), want, atol=2.1e-2, rtol=0)
