@@ -42,6 +42,10 @@ class ForwardMeta:
     # sequence's portion, for kernels whose workspace follows the context
     # (None: unknown, such kernels are not used)
     portions: Optional[List[Tuple[int, int]]] = None
+    # decode only: every row is the last token of a sequence that no other row reads,
+    # and slot_mapping that token's place (below 0 for rows that pad the batch), so
+    # that a layer may store it and attend in one launch
+    appends: bool = False
     # derived per-token tables for packed-sequence kernels (built on first
     # use, shared by every layer of the forward)
     _token_seq: Optional[torch.Tensor] = None

@@ -138,12 +138,20 @@ class LlamaAttention(nn.Module):
                 k = self.k_norm(k.contiguous())
             v = v.contiguous()
         k_cache, v_cache = meta.kv_cache.layer(self.local_layer_idx)
+        sinks = self.sinks.float() if self.sinks is not None else None
+        if meta.appends:
+            attn = ops.rope_cache_attention_decode(
+                q, k, v, k_cache, v_cache, meta.positions, rope_cache,
+                meta.slot_mapping, meta.block_tables, meta.seq_lens, self.scale,
+                self.sliding_window, sinks=sinks, max_seq_len=meta.max_seq_len or None,
+            )
+            if attn is not None:
+                return self._project_out(attn, x, T)
         ops.rope_and_cache(
             q, k, v, k_cache, v_cache, meta.positions, rope_cache,
             meta.slot_mapping,
         )
 
-        sinks = self.sinks.float() if self.sinks is not None else None
         if meta.is_prefill:
             attn = ops.prefill_attention(
                 q, k_cache, v_cache, meta.block_tables, meta.seq_lens,

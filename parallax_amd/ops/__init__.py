@@ -228,6 +228,36 @@ def paged_attention_decode(
     )
 
 
+def rope_cache_attention_decode(
+    q: torch.Tensor,             # [B, Hq, D] (rows may be strided, e.g. QKV views)
+    k: torch.Tensor,             # [B, Hk, D]
+    v: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    positions: torch.Tensor,
+    cos_sin: torch.Tensor,
+    slot_mapping: torch.Tensor,
+    block_tables: torch.Tensor,
+    seq_lens: torch.Tensor,
+    scale: float,
+    sliding_window: int = -1,
+    sinks: Optional[torch.Tensor] = None,
+    max_seq_len: Optional[int] = None,
+) -> Optional[torch.Tensor]:
+    """rope_and_cache and paged_attention_decode in one, q left unrotated, for steps in
+    which every row is the last token of a sequence that no other row reads, and
+    slot_mapping that token's place (below 0: all of the sequence is cached). None
+    where there is no kernel (CPU, other types and layouts, a gradient to be taken)."""
+    if not q.is_cuda or max_seq_len is None or (torch.is_grad_enabled() and any(
+            t.requires_grad for t in (q, k, v, k_cache, v_cache))):
+        return None
+    return _require_ext("rope_cache_attention_decode").rope_cache_attention_decode(
+        q, k, v, k_cache, v_cache, positions.to(torch.int32), cos_sin,
+        slot_mapping.to(torch.int64), block_tables.to(torch.int32),
+        seq_lens.to(torch.int32), scale, sliding_window,
+        q.new_empty(0) if sinks is None else sinks, max_seq_len)
+
+
 def prefill_attention(
     q: torch.Tensor,
     k_cache: torch.Tensor,

@@ -44,10 +44,11 @@ void launch_paged_attention_decode(void*, const void*, const void*, const void*,
                                    const float*, int, int, float*, float*,
                                    hipStream_t, bool*);
 int paged_decode_runs(int, int, int, int, int);
-void launch_paged_decode(void*, const void*, const void*, const void*, const int*,
-                         const int*, int, int, int, int, int, int, int64_t, float,
-                         int, float, const float*, int, float*, float*, bool,
-                         float, float, hipStream_t, bool*);
+void launch_paged_decode(void*, const void*, void*, void*, const int*, const int*,
+                         int, int, int, int, int, int, int64_t, float, int, float,
+                         const float*, int, float*, float*, bool, float, float,
+                         const void*, const void*, int64_t, int64_t, const int*,
+                         const float*, const int64_t*, hipStream_t, bool*);
 void launch_paged_attention_reduce(void*, const float*, const float*, int, int,
                                    int, int, const float*, hipStream_t);
 void launch_mla_paged_attention_decode(void*, const void*, const void*,
@@ -300,6 +301,11 @@ void gelu_and_mul(torch::Tensor out, torch::Tensor x) {
                      cur_stream());
 }
 
+static bool attention_by_valu() {
+  static const bool on = std::getenv("PARALLAX_ATTN_VALU") != nullptr;
+  return on;
+}
+
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
@@ -332,7 +338,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     sinks_ptr = sinks_f.data_ptr<float>();
   }
 
-  static const bool use_valu = std::getenv("PARALLAX_ATTN_VALU") != nullptr;
+  const bool use_valu = attention_by_valu();
   auto opts = q.options().dtype(at::kFloat);
   torch::Tensor tmp_acc, tmp_ml;
   float *acc_ptr = nullptr, *ml_ptr = nullptr;
@@ -355,7 +361,8 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
         block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, Hq, Hk, D,
         BS, max_blocks, row_stride(q, "q"), (float)scale, (int)sliding_window,
         (float)softcap, sinks_ptr, runs, acc_ptr, ml_ptr, kv_fp8, (float)k_scale,
-        (float)v_scale, cur_stream(), &launched);
+        (float)v_scale, nullptr, nullptr, 0, 0, nullptr, nullptr, nullptr,
+        cur_stream(), &launched);
     TORCH_CHECK(launched, "no kernel instantiation for D=", D, " BS=", BS,
                 " G=", G);
     return;
@@ -389,6 +396,68 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   if (num_parts > 1)
     launch_paged_attention_reduce(out.data_ptr(), acc_ptr, ml_ptr, B, Hq, D,
                                   num_parts, sinks_ptr, cur_stream());
+}
+
+// rope, the new token into the bf16 cache and decode attention over it; q, k and v are
+// left as they are. Every row is its sequence's last token, slot_mapping that token's
+// place (or below 0: nothing is stored). None where there is no kernel.
+std::optional<torch::Tensor> rope_cache_attention_decode(
+    torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
+    torch::Tensor v_cache, torch::Tensor positions, torch::Tensor cos_sin,
+    torch::Tensor slot_mapping, torch::Tensor block_tables, torch::Tensor seq_lens,
+    double scale, int64_t sliding_window, torch::Tensor sinks, int64_t max_seq_len) {
+  CHECK_GPU(q);
+  for (const auto* t : {&q, &k, &v})
+    if (t->dim() != 3 || t->scalar_type() != at::kBFloat16 || t->stride(2) != 1 ||
+        t->stride(1) != t->size(2) || t->stride(0) % 8 ||
+        (uintptr_t)t->data_ptr() % 16)
+      return std::nullopt;
+  if (k_cache.dim() != 4 || v_cache.dim() != 4 || block_tables.dim() != 2 ||
+      attention_by_valu())
+    return std::nullopt;
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(2), Hk = k.size(1),
+                BS = k_cache.size(2);
+  for (const auto* t : {&k_cache, &v_cache})
+    if (t->scalar_type() != at::kBFloat16 || !t->is_contiguous() ||
+        (uintptr_t)t->data_ptr() % 16 || t->size(0) != k_cache.size(0) ||
+        t->size(1) != Hk)
+      return std::nullopt;
+  for (const auto* t : {&positions, &slot_mapping, &seq_lens})
+    if (t->dim() != 1 || t->size(0) != B || !t->is_contiguous()) return std::nullopt;
+  if (B == 0 || B > 65535 || Hk == 0 || Hq % Hk || Hq / Hk > 15 ||
+      (D != 64 && D != 128) || (BS != 16 && BS != 32 && BS != 64) ||
+      k.size(0) != B || v.sizes() != k.sizes() || k.size(2) != D ||
+      k_cache.size(3) != D || v_cache.size(2) != D || v_cache.size(3) != BS ||
+      positions.scalar_type() != at::kInt || seq_lens.scalar_type() != at::kInt ||
+      slot_mapping.scalar_type() != at::kLong ||
+      block_tables.scalar_type() != at::kInt || block_tables.size(0) != B ||
+      !block_tables.is_contiguous() || cos_sin.dim() != 2 || cos_sin.size(1) != D ||
+      cos_sin.scalar_type() != at::kFloat || !cos_sin.is_contiguous() ||
+      (uintptr_t)cos_sin.data_ptr() % 16 ||
+      (sinks.numel() && (sinks.dim() != 1 || sinks.size(0) != Hq ||
+                         sinks.scalar_type() != at::kFloat || !sinks.is_contiguous())))
+    return std::nullopt;
+  auto out = torch::empty({B, Hq, D}, q.options());
+  const int runs = paged_decode_runs(B, Hk, D, (int)max_seq_len, (int)sliding_window);
+  torch::Tensor acc, ml;
+  if (runs > 0) {
+    const auto opts = q.options().dtype(at::kFloat);
+    acc = torch::empty({runs + B, Hq, D}, opts);
+    ml = torch::empty({runs + B, Hq, 2}, opts);
+  }
+  bool launched = false;
+  launch_paged_decode(
+      out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+      block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, Hq, Hk, D, BS,
+      block_tables.size(1), q.stride(0), (float)scale, (int)sliding_window, 0.f,
+      sinks.numel() ? sinks.data_ptr<float>() : nullptr, runs,
+      runs > 0 ? acc.data_ptr<float>() : nullptr,
+      runs > 0 ? ml.data_ptr<float>() : nullptr, false, 1.f, 1.f, k.data_ptr(),
+      v.data_ptr(), k.stride(0), v.stride(0), positions.data_ptr<int>(),
+      cos_sin.data_ptr<float>(), slot_mapping.data_ptr<int64_t>(), cur_stream(),
+      &launched);
+  TORCH_CHECK(launched, "no kernel instantiation for D=", D, " BS=", BS);
+  return out;
 }
 
 void prefill_attention(torch::Tensor out, torch::Tensor q,
@@ -1020,4 +1089,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_and_mul", &silu_and_mul);
   m.def("gelu_and_mul", &gelu_and_mul);
   m.def("paged_attention_decode", &paged_attention_decode);
+  m.def("rope_cache_attention_decode", &rope_cache_attention_decode);
 }

@@ -230,9 +230,53 @@ DEVINL int find_run(const int* seq_lens, int window, int u, int B, int run,
   return min(per, total - begin);
 }
 
+// 16 bytes, or 2, of a lane to LDS
+DEVINL void write16(uint32_t at, u32x4v v) {
+  asm volatile("ds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory");
+}
+DEVINL void write2(uint32_t at, uint32_t v) {
+  asm volatile("ds_write_b16 %0, %1" ::"v"(at), "v"(v) : "memory");
+}
+
+// Eight pairs of values turned, as rope_and_cache does it.
+DEVINL void rotate8(u32x4v& a, u32x4v& b, const f32x4v (&c)[2],
+                    const f32x4v (&s)[2]) {
+  float x[8], y[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const float u = bf16_bits_to_f32((uint16_t)(a[r >> 1] >> (16 * (r & 1))));
+    const float v = bf16_bits_to_f32((uint16_t)(b[r >> 1] >> (16 * (r & 1))));
+    x[r] = fmaf(u, c[r >> 2][r & 3], -v * s[r >> 2][r & 3]);
+    y[r] = fmaf(v, c[r >> 2][r & 3], u * s[r >> 2][r & 3]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
+    b[i] = pack_bf16(y[2 * i], y[2 * i + 1]);
+  }
+}
+
 }  // namespace
 
-template <int D, bool FP8, int W>
+// The step's token of every sequence, its last one, where it is not in the cache yet
+// and queries and keys are not rotated: the key goes with the queries as one more of
+// their 16 columns, whose sums nobody reads, and is turned with them; the wave whose
+// tile ends the sequence puts it and the value into the tile behind the copies, and
+// into the cache. No sequence may read another's. At most 15 query heads a
+// key/value head. us, in a row of such pairs: rope_and_cache and this kernel apart /
+// together: one sequence of 1,000, 14 heads over 2 x 64 9.8 / 8.9, 32 over 8 x 128 11.6 /
+// 10.8; 32 of up to 300 11.0 / 8.9; 96 of up to 1,900 109 / 104; 128 of up to 4,000 261
+// / 252. Nowhere slower.
+struct NewTokens {
+  const uint16_t *k, *v;  // [B, Hk, D] rows at strides
+  int64_t k_stride, v_stride;
+  const int* positions;    // [B]
+  const float* cos_sin;    // [.., D]
+  const int64_t* slots;    // [B], below 0: none, the sequence is all in the cache
+  uint16_t *k_out, *v_out;  // the cache
+};
+
+template <int D, bool FP8, int W, bool NEW>
 __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
     uint16_t* __restrict__ out,         // [B, Hq, D]
     float* __restrict__ tmp_acc,        // [parts, Hq, D]; null: a workgroup a
@@ -244,7 +288,8 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
     const int B, const int max_blocks, const int Hk, const int G,
     const int bs_shift, const int64_t q_stride, const float scale,
     const int window, const float softcap, const float* __restrict__ sinks,
-    const float v_scale) {
+    const float v_scale, const NewTokens nt) {
+  static_assert(!(NEW && FP8), "");
   constexpr int ES = FP8 ? 1 : 2;
   constexpr int RB = D * ES;             // bytes a K row
   constexpr int CPR = RB / 16;
@@ -309,6 +354,13 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
 
   while (todo > 0) {
     const int L = seq_lens[seq];
+    int pos = 0;
+    int64_t slot = -1;
+    if constexpr (NEW) {  // asked for with L: one wait of the scalar unit
+      pos = ((const __attribute__((address_space(4))) int*)nt.positions)[seq];
+      slot = ((const __attribute__((address_space(4))) int64_t*)nt.slots)[seq];
+      asm volatile("" ::"s"(L), "s"(pos), "s"(slot));
+    }
     const int lo = window > 0 ? max(0, L - window) : 0;
     const int units = units_of(L, window, U);
     if (at >= units) {  // a sequence without tokens
@@ -327,10 +379,27 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
     {
       const uint16_t* row = q + (size_t)seq * q_stride +
                             (size_t)(hk * G + min(l15, G - 1)) * D;
+      if (NEW && l15 == G) row = nt.k + (size_t)seq * nt.k_stride + hk * D;
 #pragma unroll
       for (int s = 0; s < KC; ++s)
         qf[s] = *(const bf16x8v*)(row + (FP8 ? ((s >> 1) * 4 + l4) * 16 + (s & 1) * 8
                                              : s * 32 + l4 * 8));
+    }
+    // NEW: what they are turned by, and the new value
+    f32x4v qc[KC / 2][2], qs[KC / 2][2];
+    uint32_t v_new[D / 64];
+    if constexpr (NEW) {
+      const float* turn = nt.cos_sin + (size_t)pos * D;
+      const uint16_t* vr = nt.v + (size_t)seq * nt.v_stride + hk * D;
+#pragma unroll
+      for (int i = 0; i < D / 64; ++i) v_new[i] = vr[i * 64 + lane];
+#pragma unroll
+      for (int s = 0; s < KC / 2; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          qc[s][i] = *(const f32x4v*)(turn + s * 32 + l4 * 8 + i * 4);
+          qs[s][i] = *(const f32x4v*)(turn + D / 2 + s * 32 + l4 * 8 + i * 4);
+        }
     }
     f32x4v o[MT] = {};
     float m = kLowest, l = 0.f;
@@ -374,20 +443,65 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
         copy16_to_lds(b + i * (1024 / VB) * BS * ES, Vt + i * 1024);
     };
 
+    // NEW: the tile of this wave that the new token is put into
+    const int fresh = NEW && slot >= 0 && last >= first && last < end &&
+                              (last - first) % U == 0
+                          ? last : -1;
     if (first < end) {
       int nx[2];
       pages(first, nx);
       issue_k(first, nx);
       issue_v(first, nx);
       pages(first + U, nx);
-      if (scale < 0.f) {  // the sign goes with q, as c takes maxima; with copies on
-#pragma unroll           // their way, because it waits for q
+      if constexpr (NEW) {
+        // What was asked for before K and V is here. Tied to it, or the compiler
+        // moves the arithmetic ahead and has it wait for every copy.
+        wait_copies<2 * NC>();
+#pragma unroll
+        for (int s = 0; s < KC; ++s) asm volatile("" : "+v"(qf[s]));
+#pragma unroll
+        for (int s = 0; s < KC / 2; ++s)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            asm volatile("" : "+v"(qc[s][i]), "+v"(qs[s][i]));
+#pragma unroll
+        for (int s = 0; s < KC / 2; ++s) {
+          u32x4v a = __builtin_bit_cast(u32x4v, qf[s]);
+          u32x4v b = __builtin_bit_cast(u32x4v, qf[s + KC / 2]);
+          rotate8(a, b, qc[s], qs[s]);
+          qf[s] = __builtin_bit_cast(bf16x8v, a);
+          qf[s + KC / 2] = __builtin_bit_cast(bf16x8v, b);
+        }
+      }
+      // here, not at the end: the barriers of the sums wait for stores
+      if (NEW && fresh >= 0) {
+        const int64_t row = (slot >> bs_shift) * Hk + hk;
+        const int in = (int)(slot & (BS - 1));
+        if (l15 == G) {
+          uint16_t* dst = nt.k_out + (row * BS + in) * D + l4 * 8;
+#pragma unroll
+          for (int s = 0; s < KC; ++s)
+            *reinterpret_cast<bf16x8v*>(dst + s * 32) = qf[s];
+        }
+#pragma unroll
+        for (int i = 0; i < D / 64; ++i)
+          nt.v_out[(row * D + i * 64 + lane) * BS + in] = (uint16_t)v_new[i];
+      }
+      if (scale < 0.f && (!NEW || l15 < G)) {  // the sign goes with q, as c takes
+#pragma unroll  // maxima; with copies on their way, because it waits for q
         for (int s = 0; s < KC; ++s)
           qf[s] = __builtin_bit_cast(
               bf16x8v, __builtin_bit_cast(u32x4v, qf[s]) ^ 0x80008000u);
       }
       for (int tok = first; tok < end; tok += U) {
         wait_copies<NC>();
+        if (NEW && tok == fresh && l15 == G) {
+          const int r = (L - 1) & (PD_KT - 1);
+#pragma unroll
+          for (int s = 0; s < KC; ++s)
+            write16(lds_at(Kt) + r * RB + ((s * 4 + l4) ^ swz_k<CPR>(r)) * 16,
+                    __builtin_bit_cast(u32x4v, qf[s]));
+        }
         u32x4v kr[KC * ES];  // [chunk group][t]
         if constexpr (CPR == 16)
           read8<4 * RB>(kr, k_at, k_at ^ 64, k_at ^ 128, k_at ^ 192);
@@ -450,6 +564,15 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
         }
 
         wait_copies<NC>();
+        if (NEW && tok == fresh) {
+          const int r = (L - 1) & (PD_KT - 1);
+#pragma unroll
+          for (int i = 0; i < D / 64; ++i) {
+            const int d = i * 64 + lane;
+            write2(lds_at(Vt) + d * VB + ((r >> 3) ^ swz_v<FP8>(d)) * 16 + (r & 7) * 2,
+                   v_new[i]);
+          }
+        }
         using VR = std::conditional_t<FP8, u32x2v, u32x4v>;
         VR vr[MT];
         read_rows(vr, v_at);
@@ -629,16 +752,19 @@ extern "C" int paged_decode_runs(int B, int Hk, int D, int max_len, int window) 
   return clamp_int((D == 128 ? 256 : 512) / Hk, 1, PD_MAX_RUNS);
 }
 
+// new_k null: every token is in the cache, q is rotated
 extern "C" void launch_paged_decode(
-    void* out, const void* q, const void* k_cache, const void* v_cache,
+    void* out, const void* q, void* k_cache, void* v_cache,
     const int* block_tables, const int* seq_lens, int B, int Hq, int Hk, int D,
     int BS, int max_blocks, int64_t q_stride, float scale, int window,
     float softcap, const float* sinks, int runs, float* tmp_acc, float* tmp_ml,
-    bool kv_fp8, float k_scale, float v_scale, hipStream_t stream,
-    bool* launched) {
+    bool kv_fp8, float k_scale, float v_scale, const void* new_k, const void* new_v,
+    int64_t k_stride, int64_t v_stride, const int* positions, const float* cos_sin,
+    const int64_t* slots, hipStream_t stream, bool* launched) {
   const int G = Hq / Hk;
   *launched = false;
-  if (G > 16 || (D != 64 && D != 128)) return;
+  if (G > 16 || (D != 64 && D != 128) || (new_k != nullptr && (kv_fp8 || G > 15)))
+    return;
   if (BS != 16 && BS != 32 && BS != 64) return;
   *launched = true;
   const int shift = __builtin_ctz(BS);
@@ -649,21 +775,30 @@ extern "C" void launch_paged_decode(
         (const uint8_t*)k_cache, (const uint8_t*)v_cache, block_tables, seq_lens,
         B, max_blocks, Hk, G, shift, q_stride,
         kv_fp8 ? scale * k_scale : scale, window, softcap, sinks,
-        kv_fp8 ? v_scale : 1.f);
+        kv_fp8 ? v_scale : 1.f,
+        NewTokens{(const uint16_t*)new_k, (const uint16_t*)new_v, k_stride, v_stride,
+                  positions, cos_sin, slots, (uint16_t*)k_cache, (uint16_t*)v_cache});
   };
   // few workgroups: more waves each (one sequence, 8 heads x 128, of 1,000: 4 waves
   // 10.1 us, 8 9.4; 512 workgroups of 200 tokens: 4 waves 12 us, 8 24)
   const bool wide = runs == 0 && B * Hk <= 256;
-  if (D == 128) {
-    if (kv_fp8) wide ? run(paged_decode_kernel<128, true, 16>, 16)
-                     : run(paged_decode_kernel<128, true, 4>, 4);
-    else wide ? run(paged_decode_kernel<128, false, 8>, 8)
-              : run(paged_decode_kernel<128, false, 4>, 4);
+  auto pick = [&](auto n) {
+    constexpr bool N = decltype(n)::value;
+    if (D == 128) wide ? run(paged_decode_kernel<128, false, 8, N>, 8)
+                       : run(paged_decode_kernel<128, false, 4, N>, 4);
+    else wide ? run(paged_decode_kernel<64, false, 16, N>, 16)
+              : run(paged_decode_kernel<64, false, 4, N>, 4);
+  };
+  if (new_k != nullptr) {
+    pick(std::true_type{});
+  } else if (!kv_fp8) {
+    pick(std::false_type{});
+  } else if (D == 128) {
+    wide ? run(paged_decode_kernel<128, true, 16, false>, 16)
+         : run(paged_decode_kernel<128, true, 4, false>, 4);
   } else {
-    if (kv_fp8) wide ? run(paged_decode_kernel<64, true, 16>, 16)
-                     : run(paged_decode_kernel<64, true, 4>, 4);
-    else wide ? run(paged_decode_kernel<64, false, 16>, 16)
-              : run(paged_decode_kernel<64, false, 4>, 4);
+    wide ? run(paged_decode_kernel<64, true, 16, false>, 16)
+         : run(paged_decode_kernel<64, true, 4, false>, 4);
   }
   if (runs > 0) {
     auto reduce = [&](auto kernel) {

@@ -856,6 +856,7 @@ class Engine:
             prev_ids=torch.tensor([r.decode_prev() for r in reqs],
                                   dtype=torch.long, device=dev)
             if self.uses_prev_tokens else None,
+            appends=True,
         )
         ids = torch.tensor(input_ids, dtype=torch.long, device=dev)
         return meta, ids

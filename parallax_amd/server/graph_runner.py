@@ -148,6 +148,7 @@ class DecodeGraphRunner:
             linear_slots=self.linear_slots[:bucket]
             if self.linear_cache is not None else None,
             prev_ids=self.prev_ids[:bucket] if self.uses_prev else None,
+            appends=True,
         )
 
     def _forward(self, bucket: int, ctx_bucket: Optional[int] = None) -> torch.Tensor:
