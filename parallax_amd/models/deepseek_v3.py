@@ -23,7 +23,7 @@ from ..parallel.comm import get_comm
 from ..parallel.layers import ColumnParallelLinear, RowParallelLinear, plain_call
 from .config import ModelConfig
 from .forward_meta import ForwardMeta
-from .llama import LlamaMLP, LlamaShardModel, RMSNorm
+from .llama import LlamaMLP, LlamaShardModel, RMSNorm, project_norm_mlp
 from .moe import MoEBlock
 from .registry import register_model
 
@@ -80,13 +80,26 @@ class MLAAttention(nn.Module):
         self.w_uv.copy_(w[:, self.dn :])
 
     def forward(self, x: torch.Tensor, meta: ForwardMeta, rope_cache: torch.Tensor):
+        return self.o_proj(self.attend(x, meta, rope_cache))
+
+    def _queries(self, x: torch.Tensor) -> torch.Tensor:
+        if not self.q_lora_rank:
+            return self.q_proj(x)
+        norm, proj = self.q_a_layernorm, self.q_b_proj
+        fused = None
+        if plain_call(norm, RMSNorm.forward) and plain_call(
+                proj, ColumnParallelLinear.forward) and not proj.gather_output:
+            fused = ops.linear_norm(x, self.q_a_proj.weight, None, None, norm.weight,
+                                    norm.eps, quantize=proj.fp8)
+        if fused is None:
+            return proj(norm(ops.linear(x, self.q_a_proj.weight)))
+        return proj._linear(fused[0], fused[1])
+
+    def attend(self, x: torch.Tensor, meta: ForwardMeta, rope_cache: torch.Tensor):
+        """The layer before its output projection."""
         T = x.shape[0]
         H = self.num_heads
-        if self.q_lora_rank:
-            q = self.q_b_proj(self.q_a_layernorm(
-                ops.linear(x, self.q_a_proj.weight)))
-        else:
-            q = self.q_proj(x)
+        q = self._queries(x)
         q = q.view(T, H, self.dn + self.dr)
         q_nope, q_pe = q[..., : self.dn], q[..., self.dn :]
 
@@ -118,7 +131,7 @@ class MLAAttention(nn.Module):
                 max_seq_len=meta.max_seq_len or None,
             )
             attn = ops.mla_project_out(out_latent, self.w_uv)
-        return self.o_proj(attn.reshape(T, H * self.dv))
+        return attn.reshape(T, H * self.dv)
 
     def _prefill_sparse_mask(self, i, t0, QL, L, meta):
         """Hook for sparse-attention subclasses (DSA): additive [QL, L] mask
@@ -221,7 +234,16 @@ class DeepseekV3DecoderLayer(nn.Module):
             x = self.input_layernorm(x)
         else:
             x, residual = self.input_layernorm(x, residual)
-        x = self.self_attn(x, meta, rope_cache)
+        attn = self.self_attn
+        if plain_call(attn, MLAAttention.forward):
+            y = attn.attend(x, meta, rope_cache)
+            fused = project_norm_mlp(attn.o_proj, y, residual,
+                                     self.post_attention_layernorm, self.mlp)
+            if fused is not None:
+                return fused
+            x = attn.o_proj(y)
+        else:
+            x = attn(x, meta, rope_cache)
         x, residual = self.post_attention_layernorm(x, residual)
         x = self.mlp(x)
         return x, residual

@@ -56,6 +56,28 @@ def norm_project(norm: nn.Module, proj: nn.Module, x: torch.Tensor,
                            gated)
 
 
+def project_norm_mlp(proj: nn.Module, y: torch.Tensor, residual: torch.Tensor,
+                     norm: nn.Module, mlp: nn.Module):
+    """(mlp(norm(proj(y), residual)), the residual then), the projection's parts added
+    up by the norm's launch, which also finds the scale of an fp8 MLP's input. None
+    where there is no kernel for it, and for modules that are more than these."""
+    if not (plain_call(norm, RMSNorm.forward) and isinstance(proj, RowParallelLinear)):
+        return None
+    quantize = mlp_takes_fp8(mlp)
+    fused = proj.then_norm(y, residual, norm.weight, norm.eps, quantize)
+    if fused is None:
+        return None
+    x, scale, residual = fused
+    return (mlp.from_fp8(x, scale) if quantize else mlp(x)), residual
+
+
+def mlp_takes_fp8(mlp: nn.Module) -> bool:
+    return plain_call(mlp, LlamaMLP.forward) and all(
+        plain_call(p, type_.forward) and p.fp8
+        for p, type_ in ((mlp.gate_up_proj, MergedColumnParallelLinear),
+                         (mlp.down_proj, RowParallelLinear)))
+
+
 class ResidualLayerNorm(nn.Module):
     """Layer norm (weight and bias) over an fp32 residual stream, fused with
     the scaled update that precedes it: resid += mult * scale * y, then
@@ -120,8 +142,9 @@ class LlamaAttention(nn.Module):
         return self.attend(self.qkv_proj(x), x, meta, rope_cache)
 
     def attend(self, qkv: torch.Tensor, x: torch.Tensor, meta: ForwardMeta,
-               rope_cache: torch.Tensor):
-        """The layer from its projection on; x only to be handed on."""
+               rope_cache: torch.Tensor, project: bool = True):
+        """The layer from its projection on, to its output projection or before it; x
+        only to be handed on."""
         T = qkv.shape[0]
         q, k, v = self.qkv_proj.split_output(qkv)
         # strided views into the fused QKV buffer — no contiguous copies; the
@@ -146,7 +169,7 @@ class LlamaAttention(nn.Module):
                 self.sliding_window, sinks=sinks, max_seq_len=meta.max_seq_len or None,
             )
             if attn is not None:
-                return self._project_out(attn, x, T)
+                return self._project_out(attn, x, T) if project else attn.reshape(T, -1)
         ops.rope_and_cache(
             q, k, v, k_cache, v_cache, meta.positions, rope_cache,
             meta.slot_mapping,
@@ -163,7 +186,7 @@ class LlamaAttention(nn.Module):
                 self.scale, self.sliding_window, sinks=sinks,
                 max_seq_len=meta.max_seq_len or None,
             )
-        return self._project_out(attn, x, T)
+        return self._project_out(attn, x, T) if project else attn.reshape(T, -1)
 
     def _project_out(self, attn: torch.Tensor, x: torch.Tensor, T: int):
         """Output projection; subclasses may gate `attn` first (step3p5)."""
@@ -184,6 +207,11 @@ class LlamaMLP(nn.Module):
         fused = getattr(proj, "silu_and_mul", None)  # another module may stand there
         return self.down_proj(fused(x) if fused else ops.silu_and_mul(proj(x)))
 
+    def from_fp8(self, x: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+        """forward() of rows that are fp8 values with one scale, by fp8 weights."""
+        return self.down_proj.from_fp8(
+            *ops.silu_and_mul_fp8(self.gate_up_proj._linear(x, scale)))
+
 
 class LlamaDecoderLayer(nn.Module):
     def __init__(self, cfg: ModelConfig, layer_idx: int, local_layer_idx: int):
@@ -196,18 +224,27 @@ class LlamaDecoderLayer(nn.Module):
     def forward(self, x, residual, meta: ForwardMeta, rope_cache):
         attn, mlp = self.self_attn, self.mlp
         fused = None
-        if plain_call(attn, LlamaAttention.forward) and (
-                type(attn)._project_out is LlamaAttention._project_out):
+        plain = plain_call(attn, LlamaAttention.forward) and (
+            type(attn)._project_out is LlamaAttention._project_out)
+        if plain:
             fused = norm_project(self.input_layernorm, attn.qkv_proj, x, residual)
         if fused is not None:
             qkv, residual = fused
-            x = attn.attend(qkv, x, meta, rope_cache)
         else:
             if residual is None:
                 residual = x
                 x = self.input_layernorm(x)
             else:
                 x, residual = self.input_layernorm(x, residual)
+            qkv = attn.qkv_proj(x) if plain else None
+        if plain:
+            y = attn.attend(qkv, x, meta, rope_cache, project=False)
+            fused = project_norm_mlp(attn.o_proj, y, residual,
+                                     self.post_attention_layernorm, mlp)
+            if fused is not None:
+                return fused
+            x = attn.o_proj(y)
+        else:
             x = attn(x, meta, rope_cache)
         if plain_call(mlp, LlamaMLP.forward):
             fused = norm_project(self.post_attention_layernorm, mlp.gate_up_proj, x,

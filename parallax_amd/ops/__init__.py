@@ -650,11 +650,48 @@ def linear_fp8(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor,
         raise ValueError(f"linear_fp8 takes rows [M, K], not {tuple(x.shape)}")
     xq, xs = ext.quantize_fp8_tensor(
         (x if x.dtype == torch.bfloat16 else x.float()).contiguous())
+    return linear_fp8_quantized(xq, xs, w_q, w_scale, bias)
+
+
+def linear_fp8_quantized(xq: torch.Tensor, xs: torch.Tensor, w_q: torch.Tensor,
+                         w_scale: torch.Tensor,
+                         bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """linear_fp8 of rows that are fp8 values with one scale already."""
+    ext = _require_ext("lt_linear_fp8")
     out = _few_rows(xq, w_q, bias, xs, w_scale)
     if out is not None:
         return out
     y = ext.lt_linear_fp8(xq, w_q, xs, w_scale)
     return y if bias is None else y + bias
+
+
+def silu_and_mul_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """silu_and_mul of bf16 rows as fp8 values with one scale, as linear_fp8 makes them
+    of its result; the largest magnitude is found on the way."""
+    return _require_ext("silu_and_mul_fp8").silu_and_mul_fp8(x.contiguous())
+
+
+def linear_norm(
+    x: torch.Tensor, weight: torch.Tensor, w_scale: Optional[torch.Tensor],
+    residual: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float,
+    quantize: bool = False,
+) -> Optional[Tuple[torch.Tensor, Optional[torch.Tensor], Optional[torch.Tensor]]]:
+    """(rmsnorm(linear(x, weight) + residual), its scale, linear(x, weight) + residual)
+    of few rows, x and residual left as they are: the launch that adds up a product's
+    parts normalises them too. quantize: the first as fp8 values with the scale, for
+    linear_fp8_quantized. weight is bf16, or fp8 with w_scale. None where the product has
+    no parts; no part of autograd."""
+    args = [t for t in (x, weight, residual, norm_weight) if t is not None]
+    if not x.is_cuda or x.dim() != 2 or SKINNY_GEMM_MAX_M < x.shape[0] or (
+            torch.is_grad_enabled() and any(t.requires_grad for t in args)):
+        return None
+    none = x.new_empty(0)
+    r = _require_ext("linear_norm").linear_norm(
+        x, weight, none if w_scale is None else w_scale,
+        none if residual is None else residual, norm_weight, eps, quantize)
+    if r is None:
+        return None
+    return r[0], r[1] if quantize else None, None if residual is None else r[2]
 
 
 def linear_silu_and_mul(

@@ -108,7 +108,12 @@ void launch_mla_absorb(void*, const void*, const void*, int, int, int, int64_t,
                        int64_t, hipStream_t);
 int quantize_fp8_tensor_parts(int64_t);
 void launch_quantize_fp8_tensor(void*, float*, uint32_t*, const void*, int64_t,
-                                bool, hipStream_t);
+                                bool, int, hipStream_t);
+void launch_skinny_norm(void*, void*, uint32_t*, const float*, const void*,
+                        const void*, float, int, int, int, int64_t, hipStream_t);
+int silu_and_mul_parts(int64_t, int);
+void launch_silu_and_mul_max(void*, uint32_t*, const void*, int64_t, int,
+                             hipStream_t);
 int prefill_attention_tiles(int, int, int, int);
 void launch_prefill_attention(void*, float*, float*, const void*, const void*,
                               const void*, const int*, const int*, const int*,
@@ -977,8 +982,90 @@ std::tuple<torch::Tensor, torch::Tensor> quantize_fp8_tensor(torch::Tensor x) {
                            x.options().dtype(at::kInt));
   launch_quantize_fp8_tensor(q.data_ptr(), scale.data_ptr<float>(),
                              (uint32_t*)part.data_ptr(), x.data_ptr(), n,
-                             x.scalar_type() == at::kBFloat16, cur_stream());
+                             x.scalar_type() == at::kBFloat16, 0, cur_stream());
   return {q, scale};
+}
+
+// fp8 values of bf16 x and their scale, from its parts' largest magnitudes
+static std::tuple<torch::Tensor, torch::Tensor> quantize_by_parts(
+    const torch::Tensor& x, const torch::Tensor& part) {
+  auto q = torch::empty(x.sizes(), x.options().dtype(at::kFloat8_e4m3fn));
+  auto scale = torch::empty({1}, x.options().dtype(at::kFloat));
+  launch_quantize_fp8_tensor(q.data_ptr(), scale.data_ptr<float>(),
+                             (uint32_t*)part.data_ptr(), x.data_ptr(), x.numel(), true,
+                             (int)part.numel(), cur_stream());
+  return {q, scale};
+}
+
+// silu(first half) * second half of bf16 rows, as fp8 values and their scale
+std::tuple<torch::Tensor, torch::Tensor> silu_and_mul_fp8(torch::Tensor x) {
+  CHECK_GPU(x);
+  CHECK_CONTIG(x);
+  CHECK_BF16(x);
+  TORCH_CHECK(x.dim() == 2 && x.numel() > 0 && x.size(1) % 16 == 0);
+  const int64_t T = x.size(0), I = x.size(1) / 2;
+  auto h = torch::empty({T, I}, x.options());
+  auto part = torch::empty({silu_and_mul_parts(T, I)}, x.options().dtype(at::kInt));
+  launch_silu_and_mul_max(h.data_ptr(), (uint32_t*)part.data_ptr(), x.data_ptr(), T, I,
+                          cur_stream());
+  return quantize_by_parts(h, part);
+}
+
+// rms_norm(x . w^T + residual) of few rows whose product is split over K: (the normed
+// rows, as fp8 values with their scale where quantize is set, else bf16 and an empty
+// scale; product + residual, empty without one). fp8 w takes bf16 x and its own scale.
+// None where there is no kernel or linear() has none.
+std::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> linear_norm(
+    torch::Tensor x, torch::Tensor w, torch::Tensor w_scale, torch::Tensor residual,
+    torch::Tensor norm, double eps, bool quantize) {
+  CHECK_GPU(x);
+  const bool fp8 = is_fp8(w), has_res = residual.numel() > 0;
+  auto rows16 = [](const torch::Tensor& t) {
+    return (uintptr_t)t.data_ptr() % 16 == 0 && t.stride(1) == 1;
+  };
+  if (x.dim() != 2 || w.dim() != 2 || norm.dim() != 1 || x.numel() == 0 ||
+      w.numel() == 0 || x.size(1) != w.size(1) || !w.is_contiguous() ||
+      x.scalar_type() != at::kBFloat16 || norm.scalar_type() != at::kBFloat16 ||
+      (!fp8 && w.scalar_type() != at::kBFloat16))
+    return std::nullopt;
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  if (M > 128 || N > 8192 || N % 8 || K > INT_MAX / 2 || norm.size(0) != N ||
+      !norm.is_contiguous() || (uintptr_t)norm.data_ptr() % 16 || !rows16(w))
+    return std::nullopt;
+  if (has_res && (residual.dim() != 2 || residual.size(0) != M ||
+                  residual.size(1) != N || !rows16(residual) ||
+                  residual.stride(0) % 8 ||
+                  residual.scalar_type() != at::kBFloat16))
+    return std::nullopt;
+  if (fp8 ? w_scale.numel() != 1 || w_scale.scalar_type() != at::kFloat ||
+                !x.is_contiguous()
+          : !rows16(x) || x.stride(0) % 8)
+    return std::nullopt;
+  const int64_t row_bytes = K * w.element_size();
+  if ((M - 1) * (fp8 ? K : x.stride(0) * 2) + 128 > UINT32_MAX) return std::nullopt;
+  if (!skinny_pays(M, N, row_bytes)) return std::nullopt;
+  const int splits = skinny_shared(M, N, row_bytes);
+  if (splits <= 1) return std::nullopt;
+  torch::Tensor x_scale, xq = x;
+  if (fp8) std::tie(xq, x_scale) = quantize_fp8_tensor(x);
+  auto part = torch::empty({splits, M, N}, x.options().dtype(at::kFloat));
+  launch_skinny_split(nullptr, part.data_ptr<float>(), splits, xq.data_ptr(),
+                      w.data_ptr(), nullptr, fp8 ? x_scale.data_ptr<float>() : nullptr,
+                      fp8 ? w_scale.data_ptr<float>() : nullptr, fp8, M, N, row_bytes,
+                      xq.stride(0) * xq.element_size(), 0, false, cur_stream());
+  auto out = torch::empty({M, N}, x.options());
+  auto sum = has_res ? torch::empty({M, N}, x.options()) : x.new_empty({0});
+  torch::Tensor top;
+  if (quantize) top = torch::empty({M}, x.options().dtype(at::kInt));
+  launch_skinny_norm(out.data_ptr(), has_res ? sum.data_ptr() : nullptr,
+                     quantize ? (uint32_t*)top.data_ptr() : nullptr,
+                     part.data_ptr<float>(), has_res ? residual.data_ptr() : nullptr,
+                     norm.data_ptr(), (float)eps, splits, M, N,
+                     has_res ? residual.stride(0) : 0, cur_stream());
+  if (!quantize)
+    return std::make_tuple(out, x.new_empty({0}, at::kFloat), sum);
+  auto [q, scale] = quantize_by_parts(out, top);
+  return std::make_tuple(q, scale, sum);
 }
 
 static bool rows16(const torch::Tensor& t) {
@@ -1067,6 +1154,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_rows", &few_rows);
   m.def("norm_linear", &norm_linear);
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);
+  m.def("silu_and_mul_fp8", &silu_and_mul_fp8);
+  m.def("linear_norm", &linear_norm);
   m.def("mla_absorb", &mla_absorb);
   m.def("mla_project", &mla_project);
   m.def("sample_gumbel", &sample_gumbel);

@@ -658,10 +658,14 @@ extern "C" void launch_mla_rope_and_cache(
 // ---- activations ----------------------------------------------------------------------
 // x: [T, 2I] (gate | up) -> out: [T, I];  grid-stride, vectorized.
 
-template <bool GELU>
+// MAX: part[block] is the largest magnitude among the block's results, as bits, for a
+// conversion to fp8 without a pass of its own to find it: 40 rows of 18432 8.0 to 6.7 us
+// with the conversion, one row 6.6 to 5.3
+template <bool GELU, bool MAX>
 __global__ void act_and_mul_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
-    const int64_t T, const int I) {
+    uint32_t* __restrict__ part, const int64_t T, const int I) {
+  uint32_t top = 0;
   const int64_t total = T * (I / 8);
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
        idx += (int64_t)gridDim.x * blockDim.x) {
@@ -683,8 +687,35 @@ __global__ void act_and_mul_kernel(
       }
       vals[j] = a * uv;
     }
-    store_bf16x8(out + t * I + i, vals);
+    bf16x8 o;
+    store_bf16x8(&o, vals);
+    *reinterpret_cast<int4*>(out + t * I + i) = o.raw;
+    if (MAX) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        top = max(top, __float_as_uint(bf16x8_get(o, j)) & 0x7fffffffu);
+    }
   }
+  if (MAX) {
+    __shared__ uint32_t tops[4];  // 256 threads
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+      top = max(top, (uint32_t)__shfl_xor((int)top, o, WAVE_SIZE));
+    if ((threadIdx.x & 63) == 0) tops[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      part[blockIdx.x] = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
+  }
+}
+
+// parts of silu_and_mul's results whose largest magnitudes launch_silu_and_mul_max gives
+extern "C" int silu_and_mul_parts(int64_t T, int I) {
+  return clamp_int((T * (I / 8) + 255) / 256, 1, 1024);
+}
+extern "C" void launch_silu_and_mul_max(void* out, uint32_t* part, const void* x,
+                                        int64_t T, int I, hipStream_t stream) {
+  act_and_mul_kernel<false, true><<<silu_and_mul_parts(T, I), 256, 0, stream>>>(
+      (uint16_t*)out, (const uint16_t*)x, part, T, I);
 }
 
 extern "C" void launch_act_and_mul(
@@ -692,9 +723,9 @@ extern "C" void launch_act_and_mul(
   long long total = (long long)T * (I / 8);
   int blocks = clamp_int((total + 255) / 256, 1, 2048);
   if (gelu)
-    act_and_mul_kernel<true><<<blocks, 256, 0, stream>>>(
-        (uint16_t*)out, (const uint16_t*)x, T, I);
+    act_and_mul_kernel<true, false><<<blocks, 256, 0, stream>>>(
+        (uint16_t*)out, (const uint16_t*)x, nullptr, T, I);
   else
-    act_and_mul_kernel<false><<<blocks, 256, 0, stream>>>(
-        (uint16_t*)out, (const uint16_t*)x, T, I);
+    act_and_mul_kernel<false, false><<<blocks, 256, 0, stream>>>(
+        (uint16_t*)out, (const uint16_t*)x, nullptr, T, I);
 }

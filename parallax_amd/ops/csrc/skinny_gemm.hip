@@ -449,6 +449,74 @@ __global__ __launch_bounds__(256) void skinny_sum_kernel(
       make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
 }
 
+// The sum with what follows a projection in a layer: the residual added, an RMS norm of
+// the row, and its largest magnitude for a conversion to fp8, as rmsnorm_kernel and
+// fp8_amax_kernel have them. A row is a workgroup's, eight values a thread's, N <= 8192.
+// The launches bound it, one or two less. us apart / in one, in brackets with the
+// conversion: 40 rows of 1536 x 7168 13.7 / 12.1 (18.4 / 15.2), of 7168 x 16384 in fp8
+// 37.9 / 35.8 (42.9 / 39.1), 96 rows of 4096 x 4096 19.4 / 17.1, 128 of 8192 x 8192 41.3
+// / 38.5; the slower side nowhere from 17 rows on.
+__global__ __launch_bounds__(1024) void skinny_norm_kernel(
+    uint16_t* __restrict__ out, uint16_t* __restrict__ sum_out,
+    uint32_t* __restrict__ largest,  // [M] or null
+    const float* __restrict__ part, const uint16_t* __restrict__ residual,
+    const uint16_t* __restrict__ w, const float eps, const int splits, const int M,
+    const int N, const int64_t res_stride) {
+  __shared__ float red[16];
+  __shared__ uint32_t tops[16];
+  const int row = blockIdx.x, n = threadIdx.x * 8;
+  const bool on = n < N;
+  float v[8], ss = 0.f;
+  bf16x8 x;
+  if (on) {
+    const float* src = part + (size_t)row * N + n;
+    const size_t all = (size_t)M * N;
+    f32x4v a = {}, b = {};
+#pragma unroll 8
+    for (int k = 0; k < splits; ++k) {
+      a += *reinterpret_cast<const f32x4v*>(src + k * all);
+      b += *reinterpret_cast<const f32x4v*>(src + k * all + 4);
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const float f = r < 4 ? a[r & 3] : b[r & 3];
+      v[r] = bf16_bits_to_f32(f32_to_bf16_bits(f));
+    }
+    if (residual != nullptr) {
+      const bf16x8 rv = load_bf16x8(residual + row * res_stride + n);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) v[r] += bf16x8_get(rv, r);
+    }
+    store_bf16x8(&x, v);
+    if (sum_out != nullptr)
+      *reinterpret_cast<int4*>(sum_out + (size_t)row * N + n) = x.raw;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) ss = fmaf(v[r], v[r], ss);
+  }
+  ss = block_reduce_sum(ss, red);
+  const float rstd = rsqrtf(ss / N + eps);
+  uint32_t top = 0;
+  if (on) {
+    const bf16x8 wv = load_bf16x8(w + n);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] = bf16x8_get(x, r) * rstd * bf16x8_get(wv, r);
+    store_bf16x8(&x, v);
+    *reinterpret_cast<int4*>(out + (size_t)row * N + n) = x.raw;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      top = max(top, __float_as_uint(bf16x8_get(x, r)) & 0x7fffffffu);
+  }
+  if (largest == nullptr) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    top = max(top, (uint32_t)__shfl_xor((int)top, o, WAVE_SIZE));
+  if ((threadIdx.x & 63) == 0) tops[threadIdx.x >> 6] = top;
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  for (int i = 1; i < (int)blockDim.x / 64; ++i) top = max(top, tops[i]);
+  largest[row] = top;
+}
+
 // Waves a workgroup (32 rows of W each) and workgroups that share K: what keeps
 // most of the 256 CUs busy to the end. us of 40 rows with 3 / 4 / 5 waves: 28672 x
 // 4096 57 / 44 / 46, 24576 x 1536 17 / 19 / 20, 36864 x 7168 in fp8 58 / 67 / 51.
@@ -467,6 +535,7 @@ static int skinny_splits(int N, int row_bytes) {
   return max(1, min(256 / tiles, min(32, row_bytes / 512)));
 }
 
+// c null: the parts alone
 extern "C" void launch_skinny_split(
     void* c, float* part, int splits, const void* x, const void* w,
     const void* bias, const float* x_scale, const float* w_scale, bool fp8, int M,
@@ -496,9 +565,18 @@ extern "C" void launch_skinny_split(
   };
   if (fp8) by(std::true_type{});
   else by(std::false_type{});
-  if (splits > 1)
+  if (splits > 1 && c != nullptr)
     skinny_sum_kernel<<<ceil_div(M * (gated ? N / 2 : N), 1024), 256, 0, stream>>>(
         (uint16_t*)c, part, (const uint16_t*)bias, splits, M, N, c_stride, gated);
+}
+
+extern "C" void launch_skinny_norm(void* out, void* sum_out, uint32_t* largest,
+                                   const float* part, const void* residual,
+                                   const void* w, float eps, int splits, int M, int N,
+                                   int64_t res_stride, hipStream_t stream) {
+  skinny_norm_kernel<<<M, ceil_div(N, 512) * 64, 0, stream>>>(
+      (uint16_t*)out, (uint16_t*)sum_out, largest, part, (const uint16_t*)residual,
+      (const uint16_t*)w, eps, splits, M, N, res_stride);
 }
 
 // Tiles, by rows of X and by how many tiles W gives. us of bf16 products, W from
@@ -727,9 +805,10 @@ template <typename T>
 __global__ __launch_bounds__(256) void fp8_convert_kernel(
     uint8_t* __restrict__ out, float* __restrict__ scale_out,
     const uint32_t* __restrict__ part, const T* __restrict__ x, const int64_t n,
-    const bool aligned) {
+    const bool aligned, const int parts) {
   __shared__ uint32_t lds[4];
-  const uint32_t m = threadIdx.x < gridDim.x ? part[threadIdx.x] : 0;
+  uint32_t m = 0;
+  for (int i = threadIdx.x; i < parts; i += 256) m = max(m, part[i]);
   float scale = __uint_as_float(block_max(m, lds)) * (1.f / 448.f);
   if (scale < 1e-8f) scale = 1e-8f;
   if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
@@ -750,16 +829,18 @@ extern "C" int quantize_fp8_tensor_parts(int64_t n) {
   return clamp_int((n + 2047) / 2048, 1, Q8_MAX_BLOCKS);
 }
 
+// parts > 0: the largest magnitudes of that many parts of x are in part already
 extern "C" void launch_quantize_fp8_tensor(void* out, float* scale,
                                            uint32_t* part, const void* x,
-                                           int64_t n, bool is_bf16,
+                                           int64_t n, bool is_bf16, int parts,
                                            hipStream_t stream) {
   const int blocks = quantize_fp8_tensor_parts(n);
   const bool aligned = (uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0;
   auto run = [&](auto* p) {
-    fp8_amax_kernel<<<blocks, 256, 0, stream>>>(part, p, n, aligned);
-    fp8_convert_kernel<<<blocks, 256, 0, stream>>>((uint8_t*)out, scale, part, p,
-                                                   n, aligned);
+    if (parts == 0)
+      fp8_amax_kernel<<<blocks, 256, 0, stream>>>(part, p, n, aligned);
+    fp8_convert_kernel<<<blocks, 256, 0, stream>>>(
+        (uint8_t*)out, scale, part, p, n, aligned, parts == 0 ? blocks : parts);
   };
   if (is_bf16) run((const uint16_t*)x);
   else run((const uint32_t*)x);

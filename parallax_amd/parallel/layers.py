@@ -40,7 +40,11 @@ class _Fp8WeightMixin:
         self.register_buffer("weight_scale", scale.to(w.device))
         self.fp8 = True
 
-    def _linear(self, x: torch.Tensor) -> torch.Tensor:
+    def _linear(self, x: torch.Tensor, scale: Optional[torch.Tensor] = None):
+        """scale: x is fp8 values with it."""
+        if scale is not None:
+            return ops.linear_fp8_quantized(x, scale, self.weight_fp8, self.weight_scale,
+                                            getattr(self, "bias", None))
         if self.fp8:
             return ops.linear_fp8(x, self.weight_fp8, self.weight_scale,
                                   getattr(self, "bias", None))
@@ -185,13 +189,30 @@ class RowParallelLinear(nn.Module, _Fp8WeightMixin):
             self.bias.data.copy_(b)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        comm = get_comm()
         if self.fp8:
-            y = ops.linear_fp8(x, self.weight_fp8, self.weight_scale)
-        else:
-            y = ops.linear(x, self.weight)
+            return self._reduce(ops.linear_fp8(x, self.weight_fp8, self.weight_scale))
+        return self._reduce(ops.linear(x, self.weight))
+
+    def from_fp8(self, x: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+        """forward() of rows that are fp8 values with one scale, by fp8 weights."""
+        return self._reduce(ops.linear_fp8_quantized(x, scale, self.weight_fp8,
+                                                     self.weight_scale))
+
+    def then_norm(self, x: torch.Tensor, residual: torch.Tensor,
+                  norm_weight: torch.Tensor, eps: float, quantize: bool):
+        """ops.linear_norm of this projection, where nothing else is done with its
+        result; None otherwise."""
+        if self.tp_size > 1 or self.bias is not None or not plain_call(
+                self, RowParallelLinear.forward):
+            return None
+        return ops.linear_norm(
+            x, self.weight_fp8 if self.fp8 else self.weight,
+            self.weight_scale if self.fp8 else None, residual, norm_weight, eps,
+            quantize)
+
+    def _reduce(self, y: torch.Tensor) -> torch.Tensor:
         if not self.replicated:
-            y = comm.tp_all_reduce(y)
+            y = get_comm().tp_all_reduce(y)
         # after the all-reduce every rank holds the full sum; bias is added once
         if self.bias is not None:
             y = y + self.bias

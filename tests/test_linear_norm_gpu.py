@@ -1,0 +1,153 @@
+"""Products of few rows whose parts are added up and normed in one launch: the same bits
+as product, residual, norm and conversion apart; layers that take it against the same
+layers with a hook, which do not."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from parallax_amd import ops
+from parallax_amd.models.forward_meta import ForwardMeta
+
+
+def _rand(g, *s):
+    return torch.randn(*s, generator=g, device="cuda").bfloat16()
+
+
+def _fp8(w):
+    scale = (w.float().abs().amax() / 448).reshape(1)
+    return (w.float() / scale).clamp(-448, 448).to(torch.float8_e4m3fn), scale
+
+
+@pytest.mark.parametrize("M,N,K,fp8", [
+    (40, 1536, 7168, False), (33, 4096, 4096, False), (64, 8192, 7168, False),
+    (17, 1032, 6144, False), (32, 4096, 14336, False), (128, 8192, 8192, False),
+    (9, 7168, 16384, True), (40, 7168, 16384, True), (97, 7168, 18432, True),
+    (34, 520, 7168, False),
+])
+@pytest.mark.parametrize("quantize", [False, True])
+def test_linear_norm_is_the_launches_apart(M, N, K, fp8, quantize):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w = _rand(g, M, K), _rand(g, N, K) * K ** -0.5
+    norm, res = 1 + 0.1 * _rand(g, N), (_rand(g, M, N + 8) * 3)[:, :N]
+    scale = None
+    if fp8:
+        w, scale = _fp8(w)
+    p = ops.linear_fp8(x, w, scale) if fp8 else ops.linear(x, w)
+    taken = 0
+    for residual in (None, res):
+        got = ops.linear_norm(x, w, scale, residual, norm, 1e-6, quantize)
+        if got is None:
+            continue
+        taken += 1
+        if residual is None:
+            want, sums = ops.rmsnorm(p, norm, 1e-6), None
+        else:
+            want, sums = ops.fused_add_rmsnorm(p.clone(), residual.contiguous().clone(),
+                                               norm, 1e-6)
+        if quantize:
+            q, s = ops._require_ext("t").quantize_fp8_tensor(want)
+            assert torch.equal(got[0].view(torch.uint8), q.view(torch.uint8))
+            assert torch.equal(got[1], s)
+        else:
+            assert got[1] is None and torch.equal(got[0], want)
+        assert sums is None and got[2] is None or torch.equal(got[2], sums)
+    # the smallest of these and 9 rows are one product each, without parts
+    assert taken == (0 if M == 9 else 2)  # 9 rows: a product without parts
+
+
+def test_linear_norm_without_a_kernel():
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, w, n = _rand(g, 40, 4096), _rand(g, 4096, 4096), _rand(g, 4096)
+    call = lambda x=x, w=w, r=None, n=n: ops.linear_norm(x, w, None, r, n, 1e-5)
+    assert call() is not None
+    assert call(x=x[:4]) is None and call(x=x[:0]) is None
+    assert call(x=x.float()) is None and call(w=w.float()) is None
+    assert call(x=_rand(g, 40, 4100)[:, 4:]) is None         # rows at odd places
+    assert call(n=n[:4088]) is None and call(r=_rand(g, 39, 4096)) is None
+    assert call(x=_rand(g, 129, 4096)) is None
+    assert call(w=w.clone().requires_grad_()) is None
+
+
+@pytest.mark.parametrize("T,I", [(1, 8), (3, 136), (40, 18432), (128, 1000)])
+def test_silu_and_mul_fp8(T, I):
+    g = torch.Generator(device="cuda").manual_seed(I)
+    x = _rand(g, T, 2 * I)
+    q, s = ops.silu_and_mul_fp8(x)
+    q2, s2 = ops._require_ext("t").quantize_fp8_tensor(ops.silu_and_mul(x))
+    assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8)) and torch.equal(s, s2)
+
+
+def _layer(kind, fp8):
+    from parallax_amd.models.config import ModelConfig
+    kw = dict(vocab_size=64, hidden_size=4096, num_layers=1, num_heads=32,
+              num_kv_heads=2, head_dim=128, intermediate_size=512,
+              max_position_embeddings=256, eos_token_ids=[])
+    if kind == "mla":
+        from parallax_amd.models.deepseek_v3 import DeepseekV3DecoderLayer as Layer
+        kw.update(q_lora_rank=1536, kv_lora_rank=512, qk_nope_head_dim=128,
+                  qk_rope_head_dim=64, v_head_dim=128, num_kv_heads=32)
+    else:
+        from parallax_amd.models.llama import LlamaDecoderLayer as Layer
+    cfg = ModelConfig(architecture="x", **kw)
+    with torch.device("cuda"):
+        layer = Layer(cfg, 0, 0).to(torch.bfloat16).eval()
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for name, p in layer.named_parameters():
+        p.data.copy_(1 + 0.1 * torch.randn(p.shape, generator=g, device="cuda")
+                     if p.dim() == 1 else
+                     torch.randn(p.shape, generator=g, device="cuda") * p.shape[1] ** -0.5)
+    if kind == "mla":
+        layer.self_attn.finalize_weights()
+    if fp8:
+        for m in list(layer.modules()):
+            if hasattr(m, "quantize_fp8"):
+                m.quantize_fp8()
+    return layer
+
+
+def _step(layer, kind, T):
+    from parallax_amd.server.kv_cache import KVCacheSpec, MLAKVCache, PagedKVCache
+    dev = torch.device("cuda")
+    g = torch.Generator(device="cuda").manual_seed(T)
+    if kind == "mla":
+        cache = MLAKVCache(1, 512, 64, 16, T, dev)
+        kept = cache.caches
+    else:
+        cache = PagedKVCache(KVCacheSpec(1, 2, 128, 16), T, dev)
+        kept = cache.k_caches + cache.v_caches
+    for c in kept:
+        c.copy_(torch.randn(c.shape, generator=g, device="cuda"))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    lens = [1 + i % 16 for i in range(T)]
+    meta = ForwardMeta(
+        is_prefill=False, positions=i32([n - 1 for n in lens]),
+        slot_mapping=torch.tensor([16 * i + n - 1 for i, n in enumerate(lens)],
+                                  device=dev),
+        block_tables=i32([[i] for i in range(T)]), seq_lens=i32(lens),
+        kv_cache=None if kind == "mla" else cache,
+        mla_cache=cache if kind == "mla" else None, max_seq_len=16, appends=True)
+    rope = torch.randn(32, 64 if kind == "mla" else 128, generator=g, device="cuda")
+    x, res = _rand(g, T, 4096), _rand(g, T, 4096)
+    with torch.inference_mode():
+        return list(layer(x, res, meta, rope)) + list(kept)
+
+
+@pytest.mark.parametrize("kind,fp8", [("llama", False), ("llama", True), ("mla", False),
+                                      ("mla", True)])
+@pytest.mark.parametrize("T", [1, 40, 128])
+def test_a_hook_sees_the_product_and_changes_nothing(kind, fp8, T):
+    layer = _layer(kind, fp8)
+    want = _step(layer, kind, T)
+    seen = []
+    layer.self_attn.o_proj.register_forward_hook(lambda m, a, out: seen.append(out.shape))
+    layer.post_attention_layernorm.register_forward_hook(
+        lambda m, a, out: seen.append(out[0].shape))
+    if kind == "mla":
+        layer.self_attn.q_a_layernorm.register_forward_hook(
+            lambda m, a, out: seen.append(out.shape))
+    got = _step(layer, kind, T)
+    assert len(seen) == (3 if kind == "mla" else 2)
+    if T > 4:  # one to four rows round on another way, see norm_linear
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
