@@ -281,9 +281,12 @@ void prefill_attention_kernel(
       voff[i] = (hk * D + v_row(i)) * BS + ((v_src(i) * 8) & (BS - 1));
   }
   int kpage = 0, vpage[2] = {0, 0};
+  auto page_of_k = [&](int kt) {
+    return FIXED ? btab[min(kt * PF_KT + wid * 16, L - 1) >> bs_shift] : 0;
+  };
   auto pages = [&](int kt, int vt) {  // of K's tile kt and V's tile vt
     if (!FIXED) return;
-    kpage = btab[min(kt * PF_KT + wid * 16, L - 1) >> bs_shift];
+    kpage = page_of_k(kt);
     vpage[0] = btab[min(vt * PF_KT + v_src(0) * 8, L - 1) >> bs_shift];
     vpage[1] = btab[min(vt * PF_KT + v_src(1) * 8, L - 1) >> bs_shift];
   };
@@ -556,17 +559,18 @@ void prefill_attention_kernel(
   // The first turn's K, and behind it what that turn would ask for: the buffers are
   // free, and contexts of a few tiles are rows of such waits.
   pages(kt_begin, kt_begin);
+  const int second = page_of_k(min(kt_begin + 1, kt_end - 1));
   if (KV_FP8) {
     fetch_k(kt_begin);
     fetch_v(kt_begin);
-    pages(min(kt_begin + 1, kt_end - 1), kt_begin + 1);
+    kpage = second;
     widen_k(K0);
     widen_v(V0);
     fetch_k(min(kt_begin + 1, kt_end - 1));
   } else {
     issue_k(kt_begin, K0);
-    pages(min(kt_begin + 1, kt_end - 1), kt_begin);
     asm volatile("" ::: "memory");
+    kpage = second;
     issue_k(min(kt_begin + 1, kt_end - 1), K1);
     issue_v(kt_begin, V0);
   }
