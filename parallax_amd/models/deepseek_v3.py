@@ -87,7 +87,8 @@ class MLAAttention(nn.Module):
             return self.q_proj(x)
         norm, proj = self.q_a_layernorm, self.q_b_proj
         fused = None
-        if plain_call(norm, RMSNorm.forward) and plain_call(
+        if ops.product_has_parts(x.shape[0], self.q_a_proj.weight) and plain_call(
+                norm, RMSNorm.forward) and plain_call(
                 proj, ColumnParallelLinear.forward) and not proj.gather_output:
             fused = ops.linear_norm(x, self.q_a_proj.weight, None, None, norm.weight,
                                     norm.eps, quantize=proj.fp8)
@@ -235,7 +236,8 @@ class DeepseekV3DecoderLayer(nn.Module):
         else:
             x, residual = self.input_layernorm(x, residual)
         attn = self.self_attn
-        if plain_call(attn, MLAAttention.forward):
+        if x.shape[0] <= ops.SKINNY_GEMM_MAX_M and plain_call(
+                attn, MLAAttention.forward):
             y = attn.attend(x, meta, rope_cache)
             fused = project_norm_mlp(attn.o_proj, y, residual,
                                      self.post_attention_layernorm, self.mlp)

@@ -49,7 +49,8 @@ def norm_project(norm: nn.Module, proj: nn.Module, x: torch.Tensor,
     silu of its first part times the second. None where there is no kernel for it, and
     for modules that are more than these two: hooks and forwards of others see the
     normed rows, which one launch never stores."""
-    if not (plain_call(norm, RMSNorm.forward)
+    if x.shape[0] > ops.NORM_LINEAR_MAX_M or not (
+            plain_call(norm, RMSNorm.forward)
             and plain_call(proj, MergedColumnParallelLinear.forward)) or proj.fp8:
         return None
     return ops.norm_linear(x, residual, norm.weight, norm.eps, proj.weight, proj.bias,
@@ -61,7 +62,7 @@ def project_norm_mlp(proj: nn.Module, y: torch.Tensor, residual: torch.Tensor,
     """(mlp(norm(proj(y), residual)), the residual then), the projection's parts added
     up by the norm's launch, which also finds the scale of an fp8 MLP's input. None
     where there is no kernel for it, and for modules that are more than these."""
-    if not (plain_call(norm, RMSNorm.forward) and isinstance(proj, RowParallelLinear)):
+    if not (parts_of(proj, y.shape[0]) and plain_call(norm, RMSNorm.forward)):
         return None
     quantize = mlp_takes_fp8(mlp)
     fused = proj.then_norm(y, residual, norm.weight, norm.eps, quantize)
@@ -69,6 +70,12 @@ def project_norm_mlp(proj: nn.Module, y: torch.Tensor, residual: torch.Tensor,
         return None
     x, scale, residual = fused
     return (mlp.from_fp8(x, scale) if quantize else mlp(x)), residual
+
+
+def parts_of(proj: nn.Module, rows: int) -> bool:
+    """Whether the projection of that many rows is a product with parts."""
+    return isinstance(proj, RowParallelLinear) and ops.product_has_parts(
+        rows, proj.weight_fp8 if proj.fp8 else proj.weight)
 
 
 def mlp_takes_fp8(mlp: nn.Module) -> bool:
@@ -222,6 +229,18 @@ class LlamaDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, x, residual, meta: ForwardMeta, rope_cache):
+        # sizes first: a prompt's layers wait for the host
+        rows = x.shape[0]
+        if rows > ops.SKINNY_GEMM_MAX_M or rows > ops.NORM_LINEAR_MAX_M and not parts_of(
+                getattr(self.self_attn, "o_proj", None), rows):
+            if residual is None:
+                residual = x
+                x = self.input_layernorm(x)
+            else:
+                x, residual = self.input_layernorm(x, residual)
+            x = self.self_attn(x, meta, rope_cache)
+            x, residual = self.post_attention_layernorm(x, residual)
+            return self.mlp(x), residual
         attn, mlp = self.self_attn, self.mlp
         fused = None
         plain = plain_call(attn, LlamaAttention.forward) and (

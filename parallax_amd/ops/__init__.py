@@ -510,7 +510,9 @@ def gelu_and_mul(x: torch.Tensor) -> torch.Tensor:
 # Rows of x up to which linear() and linear_fp8() try the weight-streaming kernels
 # (there are none above 128); 0 leaves every product to the library.
 SKINNY_GEMM_MAX_M = int(os.environ.get("PARALLAX_SKINNY_GEMM_MAX_M", "128"))
+NORM_LINEAR_MAX_M = 4  # rows of x up to which norm_linear() has kernels
 LT_GEMM = os.environ.get("PARALLAX_LT_GEMM", "1") != "0"
+_NONE = torch.empty(0, dtype=torch.bfloat16)  # an argument that is not there
 _LT_REFUSED = set()  # (N, K) shapes hipBLASLt had no algorithm for
 
 
@@ -529,9 +531,8 @@ def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
     ):
         return None
     ext = _require_ext("few_rows")
-    none = weight.new_empty(0, dtype=torch.bfloat16)
-    return ext.few_rows(x, weight, none if bias is None else bias,
-                        x_scale if fp8 else none, w_scale if fp8 else none, gated)
+    return ext.few_rows(x, weight, _NONE if bias is None else bias,
+                        x_scale if fp8 else _NONE, w_scale if fp8 else _NONE, gated)
 
 
 def norm_linear(
@@ -669,6 +670,14 @@ def silu_and_mul_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """silu_and_mul of bf16 rows as fp8 values with one scale, as linear_fp8 makes them
     of its result; the largest magnitude is found on the way."""
     return _require_ext("silu_and_mul_fp8").silu_and_mul_fp8(x.contiguous())
+
+
+def product_has_parts(rows: int, weight: torch.Tensor) -> bool:
+    """Whether the product of that many rows with weight is one that linear_norm() takes,
+    by its sizes: asked first, as a prompt's layers wait for the host."""
+    return 4 < rows <= SKINNY_GEMM_MAX_M and weight.is_cuda and _require_ext(
+        "product_parts").product_parts(rows, weight.shape[0],
+                                       weight.shape[1] * weight.element_size()) > 1
 
 
 def linear_norm(

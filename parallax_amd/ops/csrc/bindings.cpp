@@ -958,8 +958,9 @@ std::optional<torch::Tensor> few_rows(torch::Tensor x, torch::Tensor w,
                                       torch::Tensor bias, torch::Tensor x_scale,
                                       torch::Tensor w_scale, bool gated) {
   torch::Tensor c;
-  const auto none = w.new_empty({0});
-  if (x_scale.numel() == 0) {
+  if (x_scale.numel() == 0 && x.dim() == 2 && w.dim() == 2 &&
+      norm_linear_takes(x.size(0), w.size(0), x.size(1), false)) {
+    const auto none = w.new_empty({0});
     auto r = norm_linear(x, none, none, 0., w, bias, gated);
     if (r) return std::get<0>(*r);
   }
@@ -1011,6 +1012,15 @@ std::tuple<torch::Tensor, torch::Tensor> silu_and_mul_fp8(torch::Tensor x) {
   return quantize_by_parts(h, part);
 }
 
+// parts that linear() of few rows adds up in a launch of their own, 0: none
+int64_t product_parts(int64_t M, int64_t N, int64_t row_bytes) {
+  if (M < 1 || M > 128 || N < 1 || N > 8192 || row_bytes < 1 || row_bytes > INT_MAX ||
+      !skinny_pays(M, N, row_bytes))
+    return 0;
+  const int splits = skinny_shared(M, N, row_bytes);
+  return splits > 1 ? splits : 0;
+}
+
 // rms_norm(x . w^T + residual) of few rows whose product is split over K: (the normed
 // rows, as fp8 values with their scale where quantize is set, else bf16 and an empty
 // scale; product + residual, empty without one). fp8 w takes bf16 x and its own scale.
@@ -1043,8 +1053,7 @@ std::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> linear_no
     return std::nullopt;
   const int64_t row_bytes = K * w.element_size();
   if ((M - 1) * (fp8 ? K : x.stride(0) * 2) + 128 > UINT32_MAX) return std::nullopt;
-  if (!skinny_pays(M, N, row_bytes)) return std::nullopt;
-  const int splits = skinny_shared(M, N, row_bytes);
+  const int splits = product_parts(M, N, row_bytes);
   if (splits <= 1) return std::nullopt;
   torch::Tensor x_scale, xq = x;
   if (fp8) std::tie(xq, x_scale) = quantize_fp8_tensor(x);
@@ -1156,6 +1165,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);
   m.def("silu_and_mul_fp8", &silu_and_mul_fp8);
   m.def("linear_norm", &linear_norm);
+  m.def("product_parts", &product_parts);
   m.def("mla_absorb", &mla_absorb);
   m.def("mla_project", &mla_project);
   m.def("sample_gumbel", &sample_gumbel);
