@@ -176,7 +176,8 @@ class LlamaAttention(nn.Module):
                 self.sliding_window, sinks=sinks, max_seq_len=meta.max_seq_len or None,
             )
             if attn is not None:
-                return self._project_out(attn, x, T) if project else attn.reshape(T, -1)
+                return self._project_out(attn, x, T) if project else attn.reshape(
+                    T, self.num_heads * self.head_dim)
         ops.rope_and_cache(
             q, k, v, k_cache, v_cache, meta.positions, rope_cache,
             meta.slot_mapping,
@@ -193,7 +194,8 @@ class LlamaAttention(nn.Module):
                 self.scale, self.sliding_window, sinks=sinks,
                 max_seq_len=meta.max_seq_len or None,
             )
-        return self._project_out(attn, x, T) if project else attn.reshape(T, -1)
+        return self._project_out(attn, x, T) if project else attn.reshape(
+            T, self.num_heads * self.head_dim)
 
     def _project_out(self, attn: torch.Tensor, x: torch.Tensor, T: int):
         """Output projection; subclasses may gate `attn` first (step3p5)."""

@@ -2,10 +2,14 @@
 and the request-level timeout sweep (reference server/scheduler.py:314-330 +
 sglang_executor KV-OOM abort behavior)."""
 
+import pytest
 import torch
 
+from parallax_amd.models import get_model_class
 from parallax_amd.models.config import ModelConfig
+from parallax_amd.models.forward_meta import ForwardMeta
 from parallax_amd.server.engine import Engine, EngineArgs
+from parallax_amd.server.kv_cache import KVCacheSpec, PagedKVCache
 from parallax_amd.server.sampling_params import SamplingParams
 
 
@@ -81,3 +85,20 @@ def test_duplicate_rid_rejected():
     eng.submit([5, 6], sp, rid="dup")              # finished: rid reusable
     while eng.has_work:
         eng.step()
+
+
+@pytest.mark.parametrize("prefill", [True, False])
+def test_a_step_without_rows(prefill):
+    """No rows in, no rows out, and nothing stored."""
+    cfg = _cfg()
+    model = get_model_class(cfg.architecture)(cfg, 0, 1)
+    cache = PagedKVCache(KVCacheSpec(1, 2, 16, 16), 2, torch.device("cpu"))
+    none = torch.zeros(0, dtype=torch.int32)
+    meta = ForwardMeta(
+        is_prefill=prefill, positions=none, slot_mapping=none.long(),
+        block_tables=none.view(0, 1), seq_lens=none, query_lens=none, kv_cache=cache,
+        max_seq_len=16, appends=not prefill)
+    before = cache.k_caches[0].clone()
+    with torch.inference_mode():
+        out = model(model.embed(none.long()), meta)
+    assert out.shape == (0, 32) and torch.equal(cache.k_caches[0], before)
