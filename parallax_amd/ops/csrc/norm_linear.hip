@@ -19,6 +19,8 @@
 
 namespace {
 
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+
 // s_barrier behind this wave's LDS accesses; loads from memory stay in flight
 DEVINL void meet() {
   asm volatile("" ::: "memory");
@@ -56,8 +58,12 @@ struct NormLinearArgs {
 
 // The K-steps of 32 are dealt to the waves, S neighbouring ones each; a wave's part of X
 // stays in registers, and all of its part of a tile of 16 rows of W is asked for at
-// once, that of the next tile as soon as this one's is used.
-template <int WAVES, int S, bool NORM>
+// once, that of the next tile as soon as this one's is used. FULL: the steps fill the
+// waves. Else those past the end are the last one again with zeros for both operands, as
+// W may hold infinities; W's by a mask, which costs 0.5% where a branch around the
+// product kept the loads from running ahead (one row of 9000 x 1056 gated 7.05 us and
+// 8.3).
+template <int WAVES, int S, bool NORM, bool FULL>
 __global__ __launch_bounds__(WAVES * 64, 4) void norm_linear_kernel(
     const NormLinearArgs p) {
   __shared__ __attribute__((aligned(16))) float part[2][WAVES][16][16];  // [x row][W row]
@@ -69,7 +75,6 @@ __global__ __launch_bounds__(WAVES * 64, 4) void norm_linear_kernel(
   const int l15 = lane & 15, l4 = lane >> 4;
   const int steps = p.K / 32;
   const int m = min(l15, p.M - 1);  // a lane's row of X
-  // past the end of the contraction the last step again, times 0
   uint32_t off[S];
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -103,7 +108,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void norm_linear_kernel(
   {
     const uint16_t* r = row(blockIdx.x);
 #pragma unroll
-    for (int s = 0; s < S; ++s) load_w(r, s);
+    for (int s = 0; s < S; ++s) {
+      load_w(r, s);
+      asm volatile("" ::: "memory");  // asked for in the order of their use
+    }
   }
   if constexpr (NORM) {
     for_rows(p.M, [&](int r) {
@@ -142,9 +150,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void norm_linear_kernel(
     for (int s = 0; s < S; ++s)
       xf[s] = *reinterpret_cast<const bf16x8v*>(xs + m * (p.K + 32) + off[s]);
   }
+  if (!FULL)
 #pragma unroll
-  for (int s = 0; s < S; ++s)
-    if (wid * S + s >= steps) xf[s] = 0;
+    for (int s = 0; s < S; ++s)
+      if (wid * S + s >= steps) xf[s] = 0;
 
   int buf = 0;
   for (int tile = blockIdx.x; tile < p.tiles; tile += gridDim.x) {
@@ -153,7 +162,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void norm_linear_kernel(
     f32x4v acc = {};
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s], xf[s], acc, 0, 0, 0);
+      u32x4v w = __builtin_bit_cast(u32x4v, wf[s]);
+      if (!FULL) w &= wid * S + s < steps ? ~0u : 0u;
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, w),
+                                                    xf[s], acc, 0, 0, 0);
       if (more) load_w(r, s);
     }
     *reinterpret_cast<f32x4v*>(&part[buf][wid][l15][l4 * 4]) = acc;
@@ -208,13 +220,18 @@ extern "C" void launch_norm_linear(
     constexpr int W = decltype(wv)::value, S = decltype(sv)::value;
     const int slots = 4096 / W;  // workgroups that the chip holds: 4 waves a SIMD
     const int grid = min(p.tiles, slots);
-    if (norm == nullptr) {
-      if constexpr (W * S <= 48)
-        norm_linear_kernel<W, S, false><<<grid, W * 64, 0, stream>>>(p);
-    } else {
-      norm_linear_kernel<W, S, true>
-          <<<grid, W * 64, (size_t)M * (K + 32) * 2, stream>>>(p);
-    }
+    auto go = [&](auto full) {
+      constexpr bool F = decltype(full)::value;
+      if (norm == nullptr) {
+        if constexpr (W * S <= 48)
+          norm_linear_kernel<W, S, false, F><<<grid, W * 64, 0, stream>>>(p);
+      } else {
+        norm_linear_kernel<W, S, true, F>
+            <<<grid, W * 64, (size_t)M * (K + 32) * 2, stream>>>(p);
+      }
+    };
+    if (steps == W * S) go(std::true_type{});
+    else go(std::false_type{});
   };
 #define PICK(W, S) run(std::integral_constant<int, W>{}, std::integral_constant<int, S>{})
   if (steps <= 16) PICK(4, 4);

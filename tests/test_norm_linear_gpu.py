@@ -53,6 +53,27 @@ def test_norm_linear(M, N, K):
                                    atol=K * 2 ** -20)
 
 
+@pytest.mark.parametrize("K", [32, 480, 928, 1056, 1568, 2048, 2080, 3104, 3584])
+def test_norm_linear_infinities(K):
+    """An infinite weight of the last column or the first makes its row's results
+    infinite, with the sign of the value it meets, and no other's; also where the steps
+    along K leave waves of the last ones without any."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, norm, w = _rand(g, 2, K), torch.ones(K, device="cuda").bfloat16(), _rand(g, 70, K)
+    x[:, 0] = x[:, -1] = torch.tensor([1.0, -1.0])
+    for row, col in ((3, -1), (17, 0), (69, -1)):
+        w[row, col] = float("inf")
+    outs = [ops.norm_linear(x, None, norm, 1e-5, w)[0],
+            ops.norm_linear(x, x, norm, 1e-5, w)[0]]
+    if K <= 1536:
+        outs.append(ops.linear(x, w))
+    for out in outs:
+        for row in (3, 17, 69):
+            assert out[:, row].tolist() == [float("inf"), float("-inf")]
+        out[:, [3, 17, 69]] = 0
+        assert out.isfinite().all()
+
+
 def test_norm_linear_without_a_kernel():
     g = torch.Generator(device="cuda").manual_seed(0)
     x, w, n = _rand(g, 2, 64), _rand(g, 32, 64), _rand(g, 64)
