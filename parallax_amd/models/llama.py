@@ -46,12 +46,14 @@ class RMSNorm(nn.Module):
 def norm_project(norm: nn.Module, proj: nn.Module, x: torch.Tensor,
                  residual: Optional[torch.Tensor], gated: bool = False):
     """(proj(norm(x, residual)), the residual then) of a few rows in one launch, gated:
-    silu of its first part times the second. None where there is no kernel for it, and
-    for modules that are more than these two: hooks and forwards of others see the
-    normed rows, which one launch never stores."""
+    silu of its first part times the second. None where there is no kernel for it, for
+    parts that silu_and_mul refuses at any number of rows, and for modules that are more
+    than these two: hooks and forwards of others see the normed rows, which one launch
+    never stores."""
     if x.shape[0] > ops.NORM_LINEAR_MAX_M or not (
             plain_call(norm, RMSNorm.forward)
-            and plain_call(proj, MergedColumnParallelLinear.forward)) or proj.fp8:
+            and plain_call(proj, MergedColumnParallelLinear.forward)) or proj.fp8 or (
+            gated and proj.weight.shape[0] % 16):
         return None
     return ops.norm_linear(x, residual, norm.weight, norm.eps, proj.weight, proj.bias,
                            gated)

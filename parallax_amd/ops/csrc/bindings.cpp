@@ -958,7 +958,9 @@ std::optional<torch::Tensor> few_rows(torch::Tensor x, torch::Tensor w,
                                       torch::Tensor bias, torch::Tensor x_scale,
                                       torch::Tensor w_scale, bool gated) {
   torch::Tensor c;
+  // gated: halves as silu_and_mul takes them, for any number of rows
   if (x_scale.numel() == 0 && x.dim() == 2 && w.dim() == 2 &&
+      !(gated && w.size(0) % 16) &&
       norm_linear_takes(x.size(0), w.size(0), x.size(1), false)) {
     const auto none = w.new_empty({0});
     auto r = norm_linear(x, none, none, 0., w, bias, gated);

@@ -87,6 +87,25 @@ def test_norm_linear_without_a_kernel():
     assert ops.norm_linear(x, None, n, 1e-5, w.requires_grad_()) is None
 
 
+@pytest.mark.parametrize("T", [1, 4, 5])
+def test_gated_parts_of_odd_widths_are_refused(T):
+    """Of any number of rows alike: silu_and_mul takes parts of multiples of 8."""
+    from parallax_amd.models.llama import RMSNorm, norm_project
+    from parallax_amd.parallel.layers import MergedColumnParallelLinear
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, w = _rand(g, T, 64), _rand(g, 24, 64)
+    with pytest.raises(RuntimeError):
+        ops.linear_silu_and_mul(x, w)
+    with torch.device("cuda"):
+        norm = RMSNorm(64, 1e-5).bfloat16()
+        proj = MergedColumnParallelLinear(64, [12, 12]).bfloat16()
+        wide = MergedColumnParallelLinear(64, [16, 16]).bfloat16()
+    with torch.no_grad():
+        assert norm_project(norm, proj, x, None, gated=True) is None
+        assert (norm_project(norm, proj, x, None) is None) == (T > 4)
+        assert (norm_project(norm, wide, x, None, gated=True) is None) == (T > 4)
+
+
 def _shard(**kw):
     from parallax_amd.models import get_model_class
     from parallax_amd.models.config import ModelConfig
