@@ -47,13 +47,14 @@ def norm_project(norm: nn.Module, proj: nn.Module, x: torch.Tensor,
                  residual: Optional[torch.Tensor], gated: bool = False):
     """(proj(norm(x, residual)), the residual then) of a few rows in one launch, gated:
     silu of its first part times the second. None where there is no kernel for it, for
-    parts that silu_and_mul refuses at any number of rows, and for modules that are more
-    than these two: hooks and forwards of others see the normed rows, which one launch
-    never stores."""
+    rows apart and parts that the launches themselves refuse at any number of rows, and
+    for modules that are more than these two: hooks and forwards of others see the normed
+    rows, which one launch never stores."""
     if x.shape[0] > ops.NORM_LINEAR_MAX_M or not (
             plain_call(norm, RMSNorm.forward)
             and plain_call(proj, MergedColumnParallelLinear.forward)) or proj.fp8 or (
-            gated and proj.weight.shape[0] % 16):
+            gated and proj.weight.shape[0] % 16) or (
+            residual is not None and not (x.is_contiguous() and residual.is_contiguous())):
         return None
     return ops.norm_linear(x, residual, norm.weight, norm.eps, proj.weight, proj.bias,
                            gated)
@@ -63,8 +64,10 @@ def project_norm_mlp(proj: nn.Module, y: torch.Tensor, residual: torch.Tensor,
                      norm: nn.Module, mlp: nn.Module):
     """(mlp(norm(proj(y), residual)), the residual then), the projection's parts added
     up by the norm's launch, which also finds the scale of an fp8 MLP's input. None
-    where there is no kernel for it, and for modules that are more than these."""
-    if not (parts_of(proj, y.shape[0]) and plain_call(norm, RMSNorm.forward)):
+    where there is no kernel for it, for a residual of rows apart, which the norm refuses,
+    and for modules that are more than these."""
+    if not (parts_of(proj, y.shape[0]) and plain_call(norm, RMSNorm.forward)
+            and residual.is_contiguous()):
         return None
     quantize = mlp_takes_fp8(mlp)
     fused = proj.then_norm(y, residual, norm.weight, norm.eps, quantize)

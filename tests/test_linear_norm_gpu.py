@@ -107,7 +107,7 @@ def _layer(kind, fp8):
     return layer
 
 
-def _step(layer, kind, T):
+def _step(layer, kind, T, first=False, change=lambda t: t):
     from parallax_amd.server.kv_cache import KVCacheSpec, MLAKVCache, PagedKVCache
     dev = torch.device("cuda")
     g = torch.Generator(device="cuda").manual_seed(T)
@@ -129,9 +129,10 @@ def _step(layer, kind, T):
         kv_cache=None if kind == "mla" else cache,
         mla_cache=cache if kind == "mla" else None, max_seq_len=16, appends=True)
     rope = torch.randn(32, 64 if kind == "mla" else 128, generator=g, device="cuda")
-    x, res = _rand(g, T, 4096), _rand(g, T, 4096)
+    x, res = _rand(g, T, 4096), change(_rand(g, T, 4096))
     with torch.inference_mode():
-        return list(layer(x, res, meta, rope)) + list(kept)
+        out = layer(res, None, meta, rope) if first else layer(x, res, meta, rope)
+        return list(out) + list(kept)
 
 
 @pytest.mark.parametrize("kind,fp8", [("llama", False), ("llama", True), ("mla", False),
@@ -151,3 +152,14 @@ def test_a_hook_sees_the_product_and_changes_nothing(kind, fp8, T):
     assert len(seen) == (3 if kind == "mla" else 2)
     if T > 4:  # one to four rows round on another way, see norm_linear
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("kind", ["llama", "mla"])
+@pytest.mark.parametrize("T", [2, 4, 40, 130])
+@pytest.mark.parametrize("first", [False, True])
+def test_a_residual_of_rows_apart_is_refused(kind, T, first):
+    """As the norm that adds it refuses it, of any number of rows: it adds in place.
+    first: a stack's first layer, whose input is the residual."""
+    layer = _layer(kind, False)
+    with pytest.raises(RuntimeError, match="contiguous"):
+        _step(layer, kind, T, first, lambda t: torch.cat([t, t], 1)[:, :4096])
