@@ -185,13 +185,16 @@ def _experts64(x, gu, dn, ids, w, fp8=False, on_input=False, bias=None,
 
 
 @pytest.mark.parametrize("T,E,k,H,I,fp8", [
+    # tiles of 32 rows
     (1, 3, 1, 32, 32, False),       # less than a stage of the contraction
     (40, 5, 2, 96, 96, False),      # its last stage partly filled
+    # of 64
     (300, 2, 1, 160, 352, False),   # several tiles an expert, odd features
-    (450, 3, 2, 320, 288, False),   # 128-row tiles
-    (5000, 9, 2, 64, 32, False),    # choices counted in parts
+    (450, 3, 2, 320, 288, False),   # and remainders of every height
     (40, 5, 2, 96, 64, True),
     (700, 6, 2, 224, 192, True),
+    # of 256
+    (5000, 9, 2, 64, 32, False),    # choices counted in parts
 ])
 def test_moe_tiles(T, E, k, H, I, fp8):
     """Tile heights, remainders of rows, features and contraction, experts
@@ -236,7 +239,9 @@ def test_moe_tiles(T, E, k, H, I, fp8):
 ])
 def test_moe_rows_of_large_tiles(H, I, fp8):
     """Tiles of 256 rows at the edges of their steps of 64: 1 .. 512 rows an expert.
-    Tolerances as in test_moe_tiles."""
+    Every row on its own: a row that is wrong does not hide among the others. bf16 as in
+    test_moe_tiles, 2^-7 for a row's spread; fp8: were every value of a row's h moved by
+    one e4m3 step, 2^-3 of it, the row's result would move by as much of its norm."""
     rows = [1, 64, 65, 128, 0, 129, 192, 193, 256, 257, 511, 512, 3000]
     E, n = len(rows) + 1, sum(rows)
     g = torch.Generator(device="cuda").manual_seed(H)
@@ -249,14 +254,19 @@ def test_moe_rows_of_large_tiles(H, I, fp8):
     x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
     gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
     dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
-    w = torch.rand(T, 2, generator=g, device="cuda")
+    w = 0.5 + 0.5 * torch.rand(T, 2, generator=g, device="cuda")  # no choice is small
     if fp8:
         qg, sg = ops.quantize_fp8_weight(gu)
         qd, sd = ops.quantize_fp8_weight(dn)
-        got = ops.fused_moe_forward_fp8(x, qg, sg, qd, sd, ids, w)
-        want = _experts64(x, qg.double() * sg[..., None], qd.double() * sd[..., None],
-                          ids, w, fp8=True)
-        assert (got - want).norm() < 2e-2 * want.norm()
+        for kw in ({}, {"limit": 7.0}, {"gelu": True}):
+            got = ops.fused_moe_forward_fp8(
+                x, qg, sg, qd, sd, ids, w, limit=kw.get("limit", 0.0),
+                activation="gelu" if kw.get("gelu") else "silu")
+            want = _experts64(x, qg.double() * sg[..., None],
+                              qd.double() * sd[..., None], ids, w, fp8=True, **kw)
+            err = (got - want).norm(dim=1)
+            assert (err <= 2 ** -3 * want.norm(dim=1) + 1e-30).all()
+            assert (got - want).norm() < 2e-2 * want.norm()
         return
     bias = torch.randn(E, 2 * I, generator=g, device="cuda").bfloat16()
     for kw in ({}, {"on_input": True}, {"limit": 7.0, "bias": bias}, {"gelu": True}):
@@ -265,9 +275,32 @@ def test_moe_rows_of_large_tiles(H, I, fp8):
             limit=kw.get("limit", 0.0), bias_gate_up=kw.get("bias"),
             weight_on_input=kw.get("on_input", False))
         want = _experts64(x, gu, dn, ids, w, **kw)
-        # every row on its own: a row that is wrong does not hide among the others
         err = (got - want).norm(dim=1)
         assert (err <= 2 ** -7 * want.norm(dim=1) + 1e-30).all()
+
+
+@pytest.mark.parametrize("T", [40, 300, 5000])   # tiles of 32, 64 and 256 rows
+def test_moe_infinities(T):
+    """An infinite activation reaches its own row, an infinite weight the rows of its
+    expert; all others keep their bits. H and I end within a stage."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    E, H, I = 5, 96, 96
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
+    ids = torch.randint(0, E, (T, 1), generator=g, device="cuda")
+    ids[:2, 0] = 0
+    w = 0.5 + torch.rand(T, 1, generator=g, device="cuda")
+    want = ops.fused_moe_forward(x, gu, dn, ids, w)
+    x[1, H - 1] = gu[3, 7, H - 1] = dn[4, 5, I - 1] = float("inf")
+    got = ops.fused_moe_forward(x, gu, dn, ids, w)
+    e = ids[:, 0]
+    assert not got[1].isfinite().all() and not got[e == 3].isfinite().any()
+    assert not got[e == 4][:, 5].isfinite().any()
+    got[:, 5] = torch.where(e == 4, want[:, 5], got[:, 5])
+    same = e != 3
+    same[1] = False
+    assert torch.equal(got[same], want[same])
 
 
 @pytest.mark.parametrize("fp8", [False, True])
