@@ -66,6 +66,29 @@ def test_append_decode_is_store_and_attend(Hq, Hk, D, BS, lens, window, sinks, s
     assert torch.equal(kc, kc2) and torch.equal(vc, vc2) and torch.equal(q, before)
 
 
+@pytest.mark.parametrize("Hq,Hk,D,BS,lens", [
+    (14, 2, 64, 16, SHORT), (32, 8, 128, 32, SHORT), (32, 32, 128, 64, SHORT),
+    (32, 8, 128, 16, LONG), (16, 2, 64, 64, LONG),
+])
+def test_append_decode_over_stale_slots(Hq, Hk, D, BS, lens):
+    """The token's own place and those behind it hold NaN before."""
+    q, k, v, kc, vc, pos, cs, slots, bt, sl = _inputs(Hq, Hk, D, BS, lens, D + BS)
+    for i, n in enumerate(lens):
+        page, at = int(bt[i, (n - 1) // BS]), (n - 1) % BS
+        if i == 1:
+            slots[1], at = -1, at + 1  # this one's token is in the cache
+        kc[page, :, at:] = float("nan")
+        vc[page, :, :, at:] = float("nan")
+    kc2, vc2, q2 = kc.clone(), vc.clone(), q.clone()
+    ops.rope_and_cache(q2, k, v, kc2, vc2, pos, cs, slots)
+    want = ops.paged_attention_decode(q2, kc2, vc2, bt, sl, 0.1, max_seq_len=max(lens))
+    out = ops.rope_cache_attention_decode(q, k, v, kc, vc, pos, cs, slots, bt, sl, 0.1,
+                                          max_seq_len=max(lens))
+    assert out.isfinite().all() and torch.equal(out, want)
+    assert torch.equal(kc.view(torch.int16), kc2.view(torch.int16))
+    assert torch.equal(vc.view(torch.int16), vc2.view(torch.int16))
+
+
 def test_append_decode_in_a_graph():
     """Lengths, places and values of each replay are those in memory then."""
     q, k, v, kc, vc, pos, cs, slots, bt, sl = _inputs(32, 8, 128, 32, [700, 40, 512], 5)

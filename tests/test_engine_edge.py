@@ -102,3 +102,33 @@ def test_a_step_without_rows(prefill):
     with torch.inference_mode():
         out = model(model.embed(none.long()), meta)
     assert out.shape == (0, 32) and torch.equal(cache.k_caches[0], before)
+
+
+def test_decode_steps_store_each_sequences_last_token():
+    """What a decode step's `appends` promises: slot_mapping names the place of every
+    sequence's last token in its own table, and no other row reads that page."""
+    bs = 4
+    eng = Engine(_cfg(), EngineArgs(block_size=bs, num_kv_blocks=64,
+                                    dtype=torch.float32), random_weights=True)
+    build, steps = eng._build_decode_meta, []
+
+    def check(reqs):
+        meta, ids = build(reqs)
+        steps.append(len(reqs))
+        assert meta.appends and not meta.is_prefill
+        assert meta.positions.tolist() == [n - 1 for n in meta.seq_lens.tolist()]
+        pages = []
+        for row, slot, n in zip(meta.block_tables.tolist(), meta.slot_mapping.tolist(),
+                                meta.seq_lens.tolist()):
+            assert slot == row[(n - 1) // bs] * bs + (n - 1) % bs
+            pages.append(row[:(n + bs - 1) // bs])
+        for i, p in enumerate(pages):
+            assert not any(p[-1] in q for j, q in enumerate(pages) if j != i)
+        return meta, ids
+
+    eng._build_decode_meta = check
+    prompt = list(range(1, 13))  # three full pages, shared by the prefix cache
+    sp = SamplingParams(temperature=0.0, max_new_tokens=7, ignore_eos=True)
+    for prompts in ([prompt], [prompt, prompt, prompt[:8], prompt + [3], [5]]):
+        eng.generate(prompts, [sp] * len(prompts), max_steps=100)
+    assert max(steps) == 5

@@ -44,6 +44,21 @@ def test_linear_few_rows(M, N, K):
     torch.testing.assert_close(ops.linear(x, w, b).float(), want + b.float(), **tol)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 2044, 2048), (8, 12, 2112), (5, 4804, 2176),
+                                   (40, 1536, 7168)])
+def test_linear_infinities(M, N, K):
+    """An infinite weight reaches its own column, an infinite value its own row."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x, w = _rand(g, M, K).bfloat16(), _rand(g, N, K).bfloat16()
+    want = ops.linear(x, w)
+    w[3, K - 1] = w[N - 1, 0] = float("inf")
+    x[M - 1, K // 2] = float("inf")
+    got = ops.linear(x, w)
+    assert not got[:, [3, N - 1]].isfinite().any() and not got[M - 1].isfinite().any()
+    got[:, [3, N - 1]] = want[:, [3, N - 1]]
+    assert torch.equal(got[:M - 1], want[:M - 1])
+
+
 def test_linear_without_a_kernel():
     """Odd widths and misaligned rows take the library and agree."""
     g = torch.Generator(device="cuda").manual_seed(0)
