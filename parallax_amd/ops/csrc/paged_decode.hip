@@ -266,7 +266,10 @@ DEVINL void rotate8(u32x4v& a, u32x4v& b, const f32x4v (&c)[2],
 // key/value head. us, in a row of such pairs: rope_and_cache and this kernel apart /
 // together: one sequence of 1,000, 14 heads over 2 x 64 9.8 / 8.9, 32 over 8 x 128 11.6 /
 // 10.8; 32 of up to 300 11.0 / 8.9; 96 of up to 1,900 109 / 104; 128 of up to 4,000 261
-// / 252. Nowhere slower.
+// / 252; no pair of one to 128 sequences of up to 4,000 slower. The kernel alone, without
+// a token, takes what it took before it knew of them: one sequence of 600, 32 over 8 x
+// 128 7.15 and 7.15, 64 of 130, 64 over 8 x 128 6.79 and 6.74, one of 22,000, 64 over 8 x
+// 64 18.3 and 18.3.
 struct NewTokens {
   const uint16_t *k, *v;  // [B, Hk, D] rows at strides
   int64_t k_stride, v_stride;
@@ -275,6 +278,8 @@ struct NewTokens {
   const int64_t* slots;    // [B], below 0: none, the sequence is all in the cache
   uint16_t *k_out, *v_out;  // the cache
 };
+// nothing: 72 bytes less of arguments, 0.03 us of a launch on the host
+struct NoTokens {};
 
 template <int D, bool FP8, int W, bool NEW>
 __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
@@ -288,7 +293,7 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
     const int B, const int max_blocks, const int Hk, const int G,
     const int bs_shift, const int64_t q_stride, const float scale,
     const int window, const float softcap, const float* __restrict__ sinks,
-    const float v_scale, const NewTokens nt) {
+    const float v_scale, const std::conditional_t<NEW, NewTokens, NoTokens> nt) {
   static_assert(!(NEW && FP8), "");
   constexpr int ES = FP8 ? 1 : 2;
   constexpr int RB = D * ES;             // bytes a K row
@@ -379,7 +384,8 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
     {
       const uint16_t* row = q + (size_t)seq * q_stride +
                             (size_t)(hk * G + min(l15, G - 1)) * D;
-      if (NEW && l15 == G) row = nt.k + (size_t)seq * nt.k_stride + hk * D;
+      if constexpr (NEW)
+        if (l15 == G) row = nt.k + (size_t)seq * nt.k_stride + hk * D;
 #pragma unroll
       for (int s = 0; s < KC; ++s)
         qf[s] = *(const bf16x8v*)(row + (FP8 ? ((s >> 1) * 4 + l4) * 16 + (s & 1) * 8
@@ -474,18 +480,20 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
         }
       }
       // here, not at the end: the barriers of the sums wait for stores
-      if (NEW && fresh >= 0) {
-        const int64_t row = (slot >> bs_shift) * Hk + hk;
-        const int in = (int)(slot & (BS - 1));
-        if (l15 == G) {
-          uint16_t* dst = nt.k_out + (row * BS + in) * D + l4 * 8;
+      if constexpr (NEW) {
+        if (fresh >= 0) {
+          const int64_t row = (slot >> bs_shift) * Hk + hk;
+          const int in = (int)(slot & (BS - 1));
+          if (l15 == G) {
+            uint16_t* dst = nt.k_out + (row * BS + in) * D + l4 * 8;
 #pragma unroll
-          for (int s = 0; s < KC; ++s)
-            *reinterpret_cast<bf16x8v*>(dst + s * 32) = qf[s];
+            for (int s = 0; s < KC; ++s)
+              *reinterpret_cast<bf16x8v*>(dst + s * 32) = qf[s];
+          }
+#pragma unroll
+          for (int i = 0; i < D / 64; ++i)
+            nt.v_out[(row * D + i * 64 + lane) * BS + in] = (uint16_t)v_new[i];
         }
-#pragma unroll
-        for (int i = 0; i < D / 64; ++i)
-          nt.v_out[(row * D + i * 64 + lane) * BS + in] = (uint16_t)v_new[i];
       }
       if (scale < 0.f && (!NEW || l15 < G)) {  // the sign goes with q, as c takes
 #pragma unroll  // maxima; with copies on their way, because it waits for q
@@ -769,36 +777,37 @@ extern "C" void launch_paged_decode(
   *launched = true;
   const int shift = __builtin_ctz(BS);
   const dim3 grid(Hk, runs > 0 ? runs : B);
-  auto run = [&](auto kernel, int waves) {
+  auto run = [&](auto kernel, int waves, auto tokens) {
     kernel<<<grid, waves * 64, 0, stream>>>(
         (uint16_t*)out, tmp_acc, tmp_ml, (const uint16_t*)q,
         (const uint8_t*)k_cache, (const uint8_t*)v_cache, block_tables, seq_lens,
         B, max_blocks, Hk, G, shift, q_stride,
         kv_fp8 ? scale * k_scale : scale, window, softcap, sinks,
-        kv_fp8 ? v_scale : 1.f,
-        NewTokens{(const uint16_t*)new_k, (const uint16_t*)new_v, k_stride, v_stride,
-                  positions, cos_sin, slots, (uint16_t*)k_cache, (uint16_t*)v_cache});
+        kv_fp8 ? v_scale : 1.f, tokens);
   };
   // few workgroups: more waves each (one sequence, 8 heads x 128, of 1,000: 4 waves
   // 10.1 us, 8 9.4; 512 workgroups of 200 tokens: 4 waves 12 us, 8 24)
   const bool wide = runs == 0 && B * Hk <= 256;
-  auto pick = [&](auto n) {
-    constexpr bool N = decltype(n)::value;
-    if (D == 128) wide ? run(paged_decode_kernel<128, false, 8, N>, 8)
-                       : run(paged_decode_kernel<128, false, 4, N>, 4);
-    else wide ? run(paged_decode_kernel<64, false, 16, N>, 16)
-              : run(paged_decode_kernel<64, false, 4, N>, 4);
+  auto pick = [&](auto tokens) {
+    constexpr bool N = std::is_same_v<decltype(tokens), NewTokens>;
+    if (D == 128) wide ? run(paged_decode_kernel<128, false, 8, N>, 8, tokens)
+                       : run(paged_decode_kernel<128, false, 4, N>, 4, tokens);
+    else wide ? run(paged_decode_kernel<64, false, 16, N>, 16, tokens)
+              : run(paged_decode_kernel<64, false, 4, N>, 4, tokens);
   };
+  const NoTokens none{};
   if (new_k != nullptr) {
-    pick(std::true_type{});
+    pick(NewTokens{(const uint16_t*)new_k, (const uint16_t*)new_v, k_stride, v_stride,
+                   positions, cos_sin, slots, (uint16_t*)k_cache,
+                   (uint16_t*)v_cache});
   } else if (!kv_fp8) {
-    pick(std::false_type{});
+    pick(none);
   } else if (D == 128) {
-    wide ? run(paged_decode_kernel<128, true, 16, false>, 16)
-         : run(paged_decode_kernel<128, true, 4, false>, 4);
+    wide ? run(paged_decode_kernel<128, true, 16, false>, 16, none)
+         : run(paged_decode_kernel<128, true, 4, false>, 4, none);
   } else {
-    wide ? run(paged_decode_kernel<64, true, 16, false>, 16)
-         : run(paged_decode_kernel<64, true, 4, false>, 4);
+    wide ? run(paged_decode_kernel<64, true, 16, false>, 16, none)
+         : run(paged_decode_kernel<64, true, 4, false>, 4, none);
   }
   if (runs > 0) {
     auto reduce = [&](auto kernel) {
