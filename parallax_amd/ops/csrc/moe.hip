@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeArgs p) {
 // reads of LDS left out, raise the clock, not the products a cycle. Copies asked for in
 // one burst hold their wave up, so they are spread over the products. Workgroups that
 // go on to another block by a queue, so that the last ones end together, were no faster
-// (870 us a call, 874 so), nor was a longer part of the chip busy.
+// (of one run, a whole call: 870 us, 874 without), nor was a longer part of the chip busy.
 // ---- its results: rows through LDS, so that a wave stores long runs of each --------
 // Stored from the accumulators, 16 or 32 bytes of 32 rows an instruction: gate/up 351 /
 // 325 us, down 143 / 122 (65,536 rows of one expert).
