@@ -8,9 +8,10 @@
 //
 // What bounds it: one memory round trip and the launch, then the stream of W. Norm and
 // product of one row, us (norm_linear / fused_add_rmsnorm and a product of
-// skinny_gemm.hip, W from memory): 1152 x 896 3.3 / 5.7, 9728 x 896 gated 6.3 / 9.9,
-// 17920 x 1536 gated 14.6 / 19.0, 6144 x 4096 14.2 / 15.8, 28672 x 4096 gated 46 / 49;
-// of four rows 5.5 / 6.0, 9.2 / 10.2, 15.0 / 19.1, 16.7 / 16.4, 48 / 50.
+// skinny_gemm.hip, W from memory): 1152 x 896 3.1 / 5.5, 9728 x 896 gated 5.8 / 9.0,
+// 17920 x 1536 gated 13.2 / 15.8, 6144 x 4096 13.5 / 14.4, 28672 x 4096 gated 42.2 / 42.5;
+// of four rows the first three 5.2 / 5.6, 8.7 / 9.4, 13.5 / 15.6, of two rows the others
+// 14.0 / 14.5, 43.1 / 42.3.
 #include <type_traits>
 
 #include "common.h"
