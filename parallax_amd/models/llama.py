@@ -282,6 +282,56 @@ class LlamaDecoderLayer(nn.Module):
         return mlp(x), residual
 
 
+def stack_in_one(layers, hidden: torch.Tensor, meta: ForwardMeta,
+                 rope_cache: torch.Tensor):
+    """What the layers make of a decode step of a few rows, in one launch: (the last
+    one's branch, the residual stream). None where there is no kernel for it and for
+    layers that are more than LlamaDecoderLayer, of one width, without windows, sinks,
+    norms of heads and quantised weights."""
+    if not (meta.appends and meta.max_seq_len and hidden.is_cuda and layers) or (
+            hidden.shape[0] > ops.NORM_LINEAR_MAX_M
+            or not plain_call(layers[0], LlamaDecoderLayer.forward)):
+        return None
+    a0, eps = layers[0].self_attn, layers[0].input_layernorm.eps
+    if not (plain_call(a0, LlamaAttention.forward)
+            and plain_call(layers[0].mlp, LlamaMLP.forward)) or not ops.decode_stack_has(
+            *hidden.shape, a0.num_heads, a0.num_kv_heads, a0.head_dim,
+            getattr(layers[0].mlp.down_proj, "in_per_rank", 0), meta.max_seq_len):
+        return None
+    tensors = []
+    for layer in layers:
+        if not plain_call(layer, LlamaDecoderLayer.forward):
+            return None
+        attn, mlp = layer.self_attn, layer.mlp
+        if not (plain_call(attn, LlamaAttention.forward)
+                and getattr(attn.attend, "__func__", None) is LlamaAttention.attend
+                and getattr(attn._project_out, "__func__", None)
+                is LlamaAttention._project_out
+                and plain_call(mlp, LlamaMLP.forward)):
+            return None
+        norms = layer.input_layernorm, layer.post_attention_layernorm
+        up, down = (attn.qkv_proj, mlp.gate_up_proj), (attn.o_proj, mlp.down_proj)
+        if not (all(plain_call(n, RMSNorm.forward) and n.eps == eps for n in norms)
+                and all(plain_call(p, MergedColumnParallelLinear.forward)
+                        and not p.fp8 for p in up)
+                and all(plain_call(p, RowParallelLinear.forward) and not p.fp8
+                        and p.tp_size == 1 and p.bias is None for p in down)):
+            return None
+        if attn.qk_norm or attn.sinks is not None or attn.sliding_window > 0 or (
+                up[1].bias is not None or attn.scale != a0.scale
+                or (attn.num_heads, attn.num_kv_heads) != (a0.num_heads, a0.num_kv_heads)):
+            return None
+        w_qkv, b_qkv = up[0].weight, up[0].bias
+        tensors += [norms[0].weight, w_qkv,
+                    w_qkv.new_empty(0) if b_qkv is None else b_qkv, down[0].weight,
+                    norms[1].weight, up[1].weight, down[1].weight,
+                    *meta.kv_cache.layer(attn.local_layer_idx)]
+    return ops.decode_stack(
+        hidden, None, tensors, eps, a0.num_heads, a0.num_kv_heads, a0.scale,
+        meta.positions, rope_cache, meta.slot_mapping, meta.block_tables, meta.seq_lens,
+        meta.max_seq_len)
+
+
 @register_model("LlamaForCausalLM", "Qwen2ForCausalLM", "MistralForCausalLM")
 class LlamaShardModel(nn.Module):
     """A contiguous layer range [start_layer, end_layer) of a Llama-family model.
@@ -332,8 +382,12 @@ class LlamaShardModel(nn.Module):
         stage's output elsewhere. Returns [T, hidden] post final-norm on the
         last shard, pre-norm activations otherwise."""
         residual = None
-        for layer in self.layers:
-            hidden, residual = layer(hidden, residual, meta, self.rope_cache)
+        fused = stack_in_one(self.layers, hidden, meta, self.rope_cache)
+        if fused is not None:
+            hidden, residual = fused
+        else:
+            for layer in self.layers:
+                hidden, residual = layer(hidden, residual, meta, self.rope_cache)
         if self.is_last:
             if residual is None:  # post-norm families (minimax) fold residuals
                 hidden = self.norm(hidden)

@@ -258,6 +258,34 @@ def rope_cache_attention_decode(
         q.new_empty(0) if sinks is None else sinks, max_seq_len)
 
 
+def decode_stack_has(rows: int, hidden: int, num_heads: int, num_kv_heads: int,
+                     head_dim: int, intermediate: int, max_seq_len: int) -> bool:
+    """Whether decode_stack has a kernel for layers of these sizes."""
+    return _require_ext("decode_stack").decode_stack_has(
+        rows, hidden, num_heads, num_kv_heads, head_dim, intermediate, max_seq_len)
+
+
+def decode_stack(
+    x: torch.Tensor, residual: Optional[torch.Tensor], layers: List[torch.Tensor],
+    eps: float, num_heads: int, num_kv_heads: int, scale: float,
+    positions: torch.Tensor, cos_sin: torch.Tensor, slot_mapping: torch.Tensor,
+    block_tables: torch.Tensor, seq_lens: torch.Tensor, max_seq_len: int,
+) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """All layers of a Llama-type stack on a decode step of a few rows, in one launch:
+    (what the last layer adds, the residual stream it is added to). layers: norm weight,
+    q/k/v weight, its bias (empty: none), output weight, norm weight, gate/up weight,
+    down weight, K and V cache of each. Rows and slot_mapping as in
+    rope_cache_attention_decode. None where there is no kernel (decode_stack.hip has the
+    sizes); no part of autograd."""
+    if not x.is_cuda or x.dtype != torch.bfloat16 or (torch.is_grad_enabled() and any(
+            t.requires_grad for t in [x, *layers])):
+        return None
+    return _require_ext("decode_stack").decode_stack(
+        x, x.new_empty(0) if residual is None else residual, layers, eps, num_heads,
+        num_kv_heads, scale, positions, cos_sin, slot_mapping, block_tables, seq_lens,
+        max_seq_len)
+
+
 def prefill_attention(
     q: torch.Tensor,
     k_cache: torch.Tensor,

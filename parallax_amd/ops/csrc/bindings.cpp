@@ -43,6 +43,15 @@ void launch_paged_attention_decode(void*, const void*, const void*, const void*,
                                    int, int, int64_t, float, int, float,
                                    const float*, int, int, float*, float*,
                                    hipStream_t, bool*);
+struct StackSizes {
+  int M, H, Hq, Hk, D, F, max_len;
+};
+bool decode_stack_takes(const StackSizes*);
+int64_t decode_stack_words(const StackSizes*, int (*)[4]);
+void launch_decode_stack(const StackSizes*, const void* const*, int, const void*,
+                         const void*, void*, void*, void*, const int*, const int*,
+                         const int*, const int64_t*, const float*, int, int, float,
+                         float, hipStream_t);
 int paged_decode_runs(int, int, int, int, int);
 void launch_paged_decode(void*, const void*, void*, void*, const int*, const int*,
                          int, int, int, int, int, int, int64_t, float, int, float,
@@ -463,6 +472,83 @@ std::optional<torch::Tensor> rope_cache_attention_decode(
       &launched);
   TORCH_CHECK(launched, "no kernel instantiation for D=", D, " BS=", BS);
   return out;
+}
+
+// Whether decode_stack has a kernel for these sizes.
+bool decode_stack_has(int64_t M, int64_t H, int64_t Hq, int64_t Hk, int64_t D, int64_t F,
+                      int64_t max_seq_len) {
+  for (int64_t v : {M, H, Hq, Hk, D, F, max_seq_len})
+    if (v < 1 || v > 1 << 20) return false;
+  const StackSizes s{(int)M, (int)H, (int)Hq, (int)Hk, (int)D, (int)F, (int)max_seq_len};
+  return decode_stack_takes(&s);
+}
+
+// The layers of a Llama-type stack on a decode step of a few rows, in one launch. layers:
+// nine tensors each (norm, q/k/v weight, its bias or an empty one, output weight, norm,
+// gate and up weight, down weight, K and V cache); res: empty for none. Rows are the last
+// tokens of sequences of their own, as rope_cache_attention_decode takes them. Returns
+// what the last layer adds to the residual stream, and that. None where there is no
+// kernel.
+std::optional<std::tuple<torch::Tensor, torch::Tensor>> decode_stack(
+    torch::Tensor x, torch::Tensor res, const std::vector<torch::Tensor>& layers,
+    double eps, int64_t Hq, int64_t Hk, double scale, torch::Tensor positions,
+    torch::Tensor cos_sin, torch::Tensor slot_mapping, torch::Tensor block_tables,
+    torch::Tensor seq_lens, int64_t max_seq_len) {
+  CHECK_GPU(x);
+  constexpr size_t T = 9;  // tensors a layer
+  auto plain = [&](const torch::Tensor& t, at::ScalarType type) {
+    return t.scalar_type() == type && t.is_contiguous() &&
+           (uintptr_t)t.data_ptr() % (type == at::kInt || type == at::kLong ? 4 : 16) == 0 &&
+           t.device() == x.device();
+  };
+  if (layers.empty() || layers.size() % T || x.dim() != 2 ||
+      !plain(x, at::kBFloat16) || attention_by_valu())
+    return std::nullopt;
+  if (res.numel() && (!plain(res, at::kBFloat16) || res.sizes() != x.sizes()))
+    return std::nullopt;
+  for (const auto& t : layers)
+    if (!plain(t, at::kBFloat16)) return std::nullopt;
+  const int64_t M = x.size(0), H = x.size(1);
+  const auto& k0 = layers[7];
+  if (k0.dim() != 4 || layers[6].dim() != 2 || scale <= 0.) return std::nullopt;
+  const int64_t NB = k0.size(0), BS = k0.size(2), D = k0.size(3), F = layers[6].size(1),
+                N = (Hq + 2 * Hk) * D;
+  auto shape = [](const torch::Tensor& t, std::initializer_list<int64_t> s) {
+    return t.sizes() == at::IntArrayRef(s);
+  };
+  if (!decode_stack_has(M, H, Hq, Hk, D, F, max_seq_len)) return std::nullopt;
+  for (size_t i = 0; i < layers.size(); i += T) {
+    const torch::Tensor* t = &layers[i];
+    if (!shape(t[0], {H}) || !shape(t[1], {N, H}) ||
+        (t[2].numel() && !shape(t[2], {N})) || !shape(t[3], {H, Hq * D}) ||
+        !shape(t[4], {H}) || !shape(t[5], {2 * F, H}) || !shape(t[6], {H, F}) ||
+        !shape(t[7], {NB, Hk, BS, D}) || !shape(t[8], {NB, Hk, D, BS}))
+      return std::nullopt;
+  }
+  if ((BS != 16 && BS != 32 && BS != 64) || !plain(positions, at::kInt) ||
+      !plain(seq_lens, at::kInt) || !plain(block_tables, at::kInt) ||
+      !plain(slot_mapping, at::kLong) || !plain(cos_sin, at::kFloat) ||
+      !shape(positions, {M}) || !shape(seq_lens, {M}) || !shape(slot_mapping, {M}) ||
+      block_tables.dim() != 2 || block_tables.size(0) != M || cos_sin.dim() != 2 ||
+      cos_sin.size(1) != D)
+    return std::nullopt;
+  const StackSizes sizes{(int)M, (int)H, (int)Hq, (int)Hk, (int)D, (int)F,
+                         (int)max_seq_len};
+  const int n = (int)(layers.size() / T);
+  auto x_out = torch::empty_like(x), res_out = torch::empty_like(x);
+  auto work = torch::empty({decode_stack_words(&sizes, nullptr) + (n + 31) / 32 * 16},
+                           x.options().dtype(at::kLong));
+  std::vector<const void*> pointers(layers.size());
+  for (size_t i = 0; i < layers.size(); ++i)
+    pointers[i] = layers[i].numel() ? layers[i].data_ptr() : nullptr;
+  launch_decode_stack(&sizes, pointers.data(), n, x.data_ptr(),
+                      res.numel() ? res.data_ptr() : nullptr, x_out.data_ptr(),
+                      res_out.data_ptr(), work.data_ptr(), positions.data_ptr<int>(),
+                      seq_lens.data_ptr<int>(), block_tables.data_ptr<int>(),
+                      slot_mapping.data_ptr<int64_t>(), cos_sin.data_ptr<float>(),
+                      block_tables.size(1), __builtin_ctz((unsigned)BS), (float)eps,
+                      (float)scale, cur_stream());
+  return std::make_tuple(x_out, res_out);
 }
 
 void prefill_attention(torch::Tensor out, torch::Tensor q,
@@ -1164,6 +1250,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm);
   m.def("few_rows", &few_rows);
   m.def("norm_linear", &norm_linear);
+  m.def("decode_stack", &decode_stack);
+  m.def("decode_stack_has", &decode_stack_has);
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);
   m.def("silu_and_mul_fp8", &silu_and_mul_fp8);
   m.def("linear_norm", &linear_norm);

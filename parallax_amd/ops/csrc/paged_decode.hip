@@ -32,13 +32,13 @@
 #include <type_traits>
 
 #include "common.h"
+#include "decode_common.h"
 
 #define PD_KT 32           // tokens a tile
 #define PD_MAX_RUNS 512
 
 #define INL __attribute__((always_inline))
 
-typedef __bf16 bf16x2n __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x2v __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 
@@ -47,13 +47,6 @@ namespace {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kHidden = -__builtin_inff();  // score of a key that is not seen
 constexpr float kLowest = -1e30f;              // where a maximum starts
-
-DEVINL uint32_t pack_bf16(float a, float b) {
-  bf16x2n p;
-  p[0] = (__bf16)a;
-  p[1] = (__bf16)b;
-  return __builtin_bit_cast(uint32_t, p);
-}
 
 DEVINL void copy16_to_lds(const void* src, void* dst) {
   __builtin_amdgcn_global_load_lds(
@@ -143,17 +136,6 @@ DEVINL bf16x8v widen(uint32_t lo, uint32_t hi) {
   r[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, false));
   r[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, true));
   return __builtin_bit_cast(bf16x8v, r);
-}
-
-// over the four lanes that hold one query head (l, l + 16, l + 32, l + 48)
-template <class F>
-DEVINL float over_head(float v, F f) {
-  const auto a = __builtin_amdgcn_permlane16_swap(
-      __float_as_uint(v), __float_as_uint(v), false, false);
-  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(
-      __float_as_uint(v), __float_as_uint(v), false, false);
-  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 // Where chunk c of a row lies: at c ^ swz(row), linear over xor in the row's bits.

@@ -35,6 +35,7 @@ sources = [
     os.path.join(CSRC, "moe.hip"),
     os.path.join(CSRC, "skinny_gemm.hip"),
     os.path.join(CSRC, "norm_linear.hip"),
+    os.path.join(CSRC, "decode_stack.hip"),
     os.path.join(CSRC, "indexer.hip"),
     os.path.join(CSRC, "sampler.hip"),
 ]
