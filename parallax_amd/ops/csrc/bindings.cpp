@@ -75,6 +75,13 @@ void launch_msa_paged_attention_decode(void*, const void*, const void*,
                                        const int*, int, int, int, int, int,
                                        int, int, int, int64_t, float,
                                        hipStream_t, bool*);
+bool moe_few_takes(int, int, int, int, bool);
+void launch_moe_few_gate(void*, const void*, const float*, const void*, const float*,
+                         const int64_t*, const float*, const void*, int, int, int, int,
+                         int, bool, bool, bool, float, hipStream_t);
+void launch_moe_few_down(float*, const void*, const float*, const void*, const float*,
+                         const int64_t*, const float*, int, int, int, int, int, bool,
+                         bool, hipStream_t);
 int moe_tile_rows(int, int, int, bool);
 int64_t moe_route_scratch(int, int);
 int moe_max_tiles(int, int, int);
@@ -752,18 +759,22 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
   w_down = from16(w_down);
   auto stream = cur_stream();
 
+  const int64_t* ids = topk_ids.data_ptr<int64_t>();
+  const float* wts = topk_w.data_ptr<float>();
+  const bool few = moe_few_takes(n, E, H, I, fp8);
   const int tm = moe_tile_rows(n, E, I, fp8);
   const int max_tiles = moe_max_tiles(n, E, tm);
   // tiles (16 bytes each) first, then their number, the order, the counts
-  torch::Tensor ws = torch::empty(
-      {4 * (int64_t)max_tiles + 4 + n + moe_route_scratch(n, E)},
-      x.options().dtype(at::kInt));
-  int* tiles = ws.data_ptr<int>();
-  int* n_tiles = tiles + 4 * (int64_t)max_tiles;
-  int* perm = n_tiles + 4;
-  const int64_t* ids = topk_ids.data_ptr<int64_t>();
-  const float* wts = topk_w.data_ptr<float>();
-  launch_moe_route(perm, tiles, n_tiles, perm + n, ids, n, E, tm, stream);
+  torch::Tensor ws;
+  int *tiles = nullptr, *n_tiles = nullptr, *perm = nullptr;
+  if (!few) {
+    ws = torch::empty({4 * (int64_t)max_tiles + 4 + n + moe_route_scratch(n, E)},
+                      x.options().dtype(at::kInt));
+    tiles = ws.data_ptr<int>();
+    n_tiles = tiles + 4 * (int64_t)max_tiles;
+    perm = n_tiles + 4;
+    launch_moe_route(perm, tiles, n_tiles, perm + n, ids, n, E, tm, stream);
+  }
 
   torch::Tensor xq, xs, hq, hs;
   const void* xp = x.data_ptr();
@@ -775,13 +786,17 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
     xp = xq.data_ptr();
   }
   torch::Tensor h = torch::empty({n, I}, x.options());
-  launch_moe_gate_up(h.data_ptr(), xp, fp8 ? xs.data_ptr<float>() : nullptr,
-                     w_gu.data_ptr(),
-                     fp8 ? w_gu_scale.data_ptr<float>() : nullptr, perm, tiles,
-                     n_tiles, wts,
-                     bias_gu.numel() ? bias_gu.data_ptr() : nullptr, k, H, I,
-                     max_tiles, tm, fp8, weight_on_input, gelu, (float)limit,
-                     stream);
+  const float* gus = fp8 ? w_gu_scale.data_ptr<float>() : nullptr;
+  const float* ds = fp8 ? w_down_scale.data_ptr<float>() : nullptr;
+  const void* bias = bias_gu.numel() ? bias_gu.data_ptr() : nullptr;
+  if (few)
+    launch_moe_few_gate(h.data_ptr(), xp, fp8 ? xs.data_ptr<float>() : nullptr,
+                        w_gu.data_ptr(), gus, ids, wts, bias, n, k, E, H, I, fp8,
+                        weight_on_input, gelu, (float)limit, stream);
+  else
+    launch_moe_gate_up(h.data_ptr(), xp, fp8 ? xs.data_ptr<float>() : nullptr,
+                       w_gu.data_ptr(), gus, perm, tiles, n_tiles, wts, bias, k, H, I,
+                       max_tiles, tm, fp8, weight_on_input, gelu, (float)limit, stream);
   const void* hp = h.data_ptr();
   if (fp8) {
     hq = torch::empty({n, I}, bopts);
@@ -790,15 +805,20 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
                              stream);
     hp = hq.data_ptr();
   }
+  torch::Tensor out = torch::empty({T, H}, fopts);
+  if (few) {
+    launch_moe_few_down(out.data_ptr<float>(), hp, fp8 ? hs.data_ptr<float>() : nullptr,
+                        w_down.data_ptr(), ds, ids, wts, n, k, E, H, I, fp8,
+                        weight_on_input, stream);
+    return out;
+  }
   const int slab = moe_down_cols(n, H);
   torch::Tensor y = torch::empty({n, slab}, fopts);
-  torch::Tensor out = torch::empty({T, H}, fopts);
   for (int first = 0; first < H; first += slab) {
     const int cols = std::min(slab, H - first);
     launch_moe_down(y.data_ptr<float>(), hp,
-                    fp8 ? hs.data_ptr<float>() : nullptr, w_down.data_ptr(),
-                    fp8 ? w_down_scale.data_ptr<float>() : nullptr, perm, tiles,
-                    n_tiles, wts, k, H, I, first, cols, max_tiles, tm, fp8,
+                    fp8 ? hs.data_ptr<float>() : nullptr, w_down.data_ptr(), ds, perm,
+                    tiles, n_tiles, wts, k, H, I, first, cols, max_tiles, tm, fp8,
                     weight_on_input, stream);
     launch_moe_combine(out.data_ptr<float>(), y.data_ptr<float>(), ids, T, k, E,
                        H, first, cols, stream);

@@ -16,46 +16,14 @@
 // experts of another rank) are left out. Grids are upper bounds (blocks past
 // the live tiles exit), so a captured step replays with any routing.
 
-#include "common.h"
-
 #include <type_traits>
+
+#include "moe_common.h"
 
 #define MOE_BKB 128    // bytes of the contraction a stage
 #define MOE_UNIT (256 * MOE_BKB)
 
 typedef float f32x16v __attribute__((ext_vector_type(16)));
-typedef int i32x4v __attribute__((ext_vector_type(4)));
-typedef int i32x8v __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2n __attribute__((ext_vector_type(2)));
-
-namespace {
-
-DEVINL uint32_t pack_bf16(float a, float b) {
-  bf16x2n p;
-  p[0] = (__bf16)a;
-  p[1] = (__bf16)b;
-  return __builtin_bit_cast(uint32_t, p);
-}
-
-// 16 bytes a lane from memory to LDS, at + 16 lane. In assembly, without a register
-// of its own: of the builtin the compiler knows that it writes LDS, and where the
-// places rotate it waits for every copy in flight once a loop's turn before it reads.
-DEVINL void copy16(const void* src, uint32_t at) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               :: "v"(src), "s"(at) : "m0", "memory");
-}
-// The same from a uniform base: no address arithmetic a lane.
-DEVINL void copy16(const uint8_t* base, uint32_t off, uint32_t at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(off), "s"(base), "s"(at) : "m0", "memory");
-}
-
-DEVINL uint32_t lds_address(const void* p) {
-  return __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
-}
-
-}  // namespace
 
 // ---- routing ------------------------------------------------------------------
 // perm [n], tiles [max_tiles] as (expert, first row, end of the expert's rows,
@@ -520,27 +488,6 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeArgs p) {
 // Stored from the accumulators, 16 or 32 bytes of 32 rows an instruction: gate/up 351 /
 // 325 us, down 143 / 122 (65,536 rows of one expert).
 
-// one uniform branch for four features
-DEVINL void activate(const MoeArgs& p, f32x4v g, f32x4v u, float (&v)[4]) {
-  if (p.limit > 0.f) {  // gpt-oss clamped act
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const float a = fminf(g[s], p.limit);
-      const float b = fminf(fmaxf(u[s], -p.limit), p.limit);
-      v[s] = (b + 1.f) * (a / (1.f + __expf(-a * 1.702f)));
-    }
-  } else if (p.gelu) {
-    const float c = 0.7978845608028654f;
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      v[s] = 0.5f * g[s] *
-             (1.f + tanhf(c * (g[s] + 0.044715f * g[s] * g[s] * g[s]))) * u[s];
-  } else {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) v[s] = g[s] / (1.f + __expf(-g[s])) * u[s];
-  }
-}
-
 // Row block j of a wave: rows ab + 64 j + l31 of the tile. rowc, roww, rows_a: the
 // choice, routing weight and activation scale of this thread's row (tid < 256).
 template <bool FP8, bool GATE, int WM>
@@ -598,7 +545,7 @@ DEVINL void store_big(const MoeArgs& p, uint8_t* S, const f32x16v (&acc)[2][WM],
             }
           }
           float v[4];
-          activate(p, g, u, v);
+          activate(p.limit, p.gelu, g, u, v);
           *reinterpret_cast<uint2*>(S + r * PITCH + f * 2) =
               make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
         }

@@ -33,6 +33,7 @@ sources = [
     os.path.join(CSRC, "mla_prefill.hip"),
     os.path.join(CSRC, "prefill_attention.hip"),
     os.path.join(CSRC, "moe.hip"),
+    os.path.join(CSRC, "moe_few.hip"),
     os.path.join(CSRC, "skinny_gemm.hip"),
     os.path.join(CSRC, "norm_linear.hip"),
     os.path.join(CSRC, "decode_stack.hip"),

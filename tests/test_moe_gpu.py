@@ -354,3 +354,78 @@ def test_moe_many_experts(E, T):
                     wts.cpu())
     # h is rounded to bf16: 2^-9 of sums of |h w| < 4 weights * 32 * |h| 3 * |w| 0.9
     torch.testing.assert_close(out.cpu(), want, atol=0.05, rtol=1e-2)
+
+
+@pytest.mark.parametrize("T,E,k,H,I,fp8", [
+    (1, 3, 1, 64, 64, False),         # one stage along K, three waves without any
+    (32, 3, 1, 192, 128, False),      # experts of several times eight rows
+    (4, 6, 8, 320, 448, False),       # a token that chooses an expert twice
+    (8, 40, 4, 2112, 192, False),     # 16 features a workgroup
+    (2, 9, 8, 2048, 768, False),
+    (1, 2, 1, 128, 128, True),
+    (16, 3, 1, 384, 256, True),
+    (2, 30, 8, 2176, 640, True),
+])
+def test_moe_few(T, E, k, H, I, fp8):
+    """At most 32 choices (fp8: 16): every token on its own, bounds as in the tests of
+    tiles. Choices of other ranks' experts, a token without any other."""
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
+    ids = torch.randint(0, E, (T, k), generator=g, device="cuda")
+    if T > 2:
+        ids[1], ids[2, 0] = E, -1
+    if k > E:
+        ids[0, :2] = 4
+    w = 0.5 + 0.5 * torch.rand(T, k, generator=g, device="cuda")
+    bias = torch.randn(E, 2 * I, generator=g, device="cuda").bfloat16()
+    if fp8:
+        (qg, sg), (qd, sd) = ops.quantize_fp8_weight(gu), ops.quantize_fp8_weight(dn)
+        gu, dn = qg.double() * sg[..., None], qd.double() * sd[..., None]
+    for kw in ({}, {"limit": 7.0}, {"gelu": True}) + (
+            () if fp8 else ({"on_input": True}, {"bias": bias})):
+        act = "gelu" if kw.get("gelu") else "silu"
+        if fp8:
+            got = ops.fused_moe_forward_fp8(x, qg, sg, qd, sd, ids, w, activation=act,
+                                            limit=kw.get("limit", 0.0))
+        else:
+            got = ops.fused_moe_forward(
+                x, gu, dn, ids, w, activation=act, limit=kw.get("limit", 0.0),
+                bias_gate_up=kw.get("bias"), weight_on_input=kw.get("on_input", False))
+        want = _experts64(x, gu, dn, ids, w, fp8=fp8, **kw)
+        err = (got - want).norm(dim=1)
+        assert (err <= (2 ** -3 if fp8 else 2 ** -7) * want.norm(dim=1) + 1e-30).all()
+        assert (got - want).norm() < (2e-2 if fp8 else 2 ** -8) * want.norm()
+
+
+def test_moe_few_infinities_and_graph():
+    """An infinite weight reaches the results of its expert's rows alone; a replay takes
+    the choices of then."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    T, E, k, H, I = 6, 5, 2, 192, 192
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
+    ids = torch.tensor([[0, 1], [1, 2], [2, 3], [3, 0], [1, 0], [2, 0]], device="cuda")
+    w = 0.5 + torch.rand(T, k, generator=g, device="cuda")
+    want = ops.fused_moe_forward(x, gu, dn, ids, w)
+    gu[4, 3, H - 1] = dn[4, 5, I - 1] = dn[3, 7, 0] = float("inf")
+    got = ops.fused_moe_forward(x, gu, dn, ids, w)
+    hit = (ids == 3).any(1)
+    assert not got[hit, 7].isfinite().any()
+    got[hit, 7] = want[hit, 7]
+    assert torch.equal(got, want)
+    dn[3, 7, 0] = gu[4, 3, H - 1] = dn[4, 5, I - 1] = 0
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = ops.fused_moe_forward(x, gu, dn, ids, w)
+    for step in range(3):
+        ids.copy_((ids + 1) % E)
+        x.mul_(-0.5)
+        eager = ops.fused_moe_forward(x, gu, dn, ids, w)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
