@@ -140,6 +140,41 @@ DEVINL int run_length(int total, int runs) {
   return max((total + runs - 1) / runs, MLA_MIN_TILES);
 }
 
+// Run `run` of the list of all tiles: its length, the sequence of its first tile and
+// that tile's place there. Up to 64 sequences are looked at once, for the total too.
+template <bool SPARSE>
+DEVINL int find_run(const int* seq_lens, const int* topk, int max_topk, int B,
+                    int run, int runs, int* seq, int* at) {
+  int first;
+  if (B > 64) {
+    const int total = find_tile<SPARSE>(seq_lens, topk, max_topk, B, 0, seq, &first);
+    const int per = run_length(total, runs);
+    const int todo = min(per, total - run * per);
+    if (todo > 0)
+      find_tile<SPARSE>(seq_lens, topk, max_topk, B, run * per, seq, &first);
+    *at = run * per - first;
+    return todo;
+  }
+  const int lane = threadIdx.x & 63;
+  const int n = lane < B ? (domain_of<SPARSE>(seq_lens, topk, max_topk, lane) +
+                            MLA_KT - 1) / MLA_KT
+                         : 0;
+  int sum = n;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(sum, o, WAVE_SIZE);
+    if (lane >= o) sum += t;
+  }
+  const int total = __builtin_amdgcn_readlane(sum, 63);
+  const int per = run_length(total, runs);
+  const int begin = run * per;
+  const unsigned long long hit = __ballot(begin >= sum - n && begin < sum);
+  const int src = hit ? __ffsll(hit) - 1 : 0;
+  *seq = src;
+  *at = begin - (__builtin_amdgcn_readlane(sum, src) - __builtin_amdgcn_readlane(n, src));
+  return min(per, total - begin);
+}
+
 }  // namespace
 
 template <int W, bool KV_FP8, bool SPARSE>
@@ -183,15 +218,8 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
             make_uint2(0, 0);
     }
   } else {
-    int first;
-    const int total = find_tile<SPARSE>(seq_lens, topk, max_topk, B, 0, &seq,
-                                        &first);
-    const int per = run_length(total, gridDim.x);
-    const int begin = blockIdx.x * per;
-    todo = min(per, total - begin);
-    if (todo > 0)
-      find_tile<SPARSE>(seq_lens, topk, max_topk, B, begin, &seq, &first);
-    at = begin - first;
+    todo = find_run<SPARSE>(seq_lens, topk, max_topk, B, blockIdx.x, gridDim.x, &seq,
+                            &at);
   }
   seq = __builtin_amdgcn_readfirstlane(seq);
   at = __builtin_amdgcn_readfirstlane(at);
@@ -218,6 +246,7 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
   // chunk (lane ^ row_xor), of the rope of 8 rows one chunk of row lane / 8
   const int bit3 = RPW == 8 ? wid & 1 : 0;
 
+  bool first = true;
   while (todo > 0) {
     const int* btab = block_tables + (size_t)seq * max_blocks;
     const int L = seq_lens[seq];
@@ -234,18 +263,7 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     const int t0 = at;
     const int t1 = min(tiles, at + todo);
 
-    // ---- Q: B operands, head l15, values 32 ks + 8 l4 + (0..7) -------------------
-    bf16x8v qf[MLA_DK / 32];
-    {
-      const size_t row = (size_t)seq * H + min(head, H - 1);
-#pragma unroll
-      for (int ks = 0; ks < MLA_DK / 32; ++ks) {
-        const int k = ks * 32 + l4 * 8;
-        qf[ks] = ks < MLA_R / 32
-                     ? *(const bf16x8v*)(q_latent + row * MLA_R + k)
-                     : *(const bf16x8v*)(q_pe + row * MLA_DR + k - MLA_R);
-      }
-    }
+    bf16x8v qf[MLA_DK / 32];  // B operands: head l15, values 32 ks + 8 l4 + (0..7)
     f32x4v acc[MLA_DT] = {};
     float m = kHidden, l = 0.f;
     const float c = scale * kLog2e;
@@ -495,7 +513,8 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     // ---- the run -----------------------------------------------------------------------
     // Behind a turn's first barrier this tile is in LDS, and every wave has left the
     // buffer that the next one goes to. Past the run's end nothing is copied.
-    __syncthreads();  // the buffers may still be read for the last sequence
+    if (!first) __syncthreads();  // the buffers may still be read for the last sequence
+    first = false;
     auto turn = [&](int t, const int buf) INL {
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's copies
       __syncthreads();
@@ -523,6 +542,17 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     } else {
 #pragma unroll
       for (int i = 0; i < CPW; ++i) issue(i, 0);
+    }
+    // behind the first tile's copies, whose way is the longer one
+    {
+      const size_t row = (size_t)seq * H + min(head, H - 1);
+#pragma unroll
+      for (int ks = 0; ks < MLA_DK / 32; ++ks) {
+        const int k = ks * 32 + l4 * 8;
+        qf[ks] = ks < MLA_R / 32
+                     ? *(const bf16x8v*)(q_latent + row * MLA_R + k)
+                     : *(const bf16x8v*)(q_pe + row * MLA_DR + k - MLA_R);
+      }
     }
     for (int t = t0; t < t1;) {
       turn(t, 0);
@@ -609,6 +639,15 @@ __global__ __launch_bounds__(512) void mla_reduce_kernel(
   const int parts = r1 - r0 + 1;
   const bool on = head < H;
   const size_t first_part = ((size_t)r0 + seq) * H + (on ? head : 0);
+  // a thread's first parts, on their way beside the weights
+  constexpr int STEP = BY_HEAD ? 1 : 4, AHEAD = 8;
+  const int d = (tid & 127) * 4, mine = BY_HEAD ? 0 : grp;
+  const float* src = tmp_acc + first_part * MLA_R + d;
+  f32x4v v[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+    v[i] = *reinterpret_cast<const f32x4v*>(
+        src + (size_t)min(mine + i * STEP, parts - 1) * H * MLA_R);
   // the weights, worked out by each wave for itself, written by one of them
   float M = kHidden, l = 0.f;
   for (int r = lane; r < parts; r += 64)
@@ -622,18 +661,18 @@ __global__ __launch_bounds__(512) void mla_reduce_kernel(
   }
   l = wave_reduce_sum(l);
   __syncthreads();
-  const int d = (tid & 127) * 4;
   f32x4v s = {0.f, 0.f, 0.f, 0.f};
-  const float* src = tmp_acc + first_part * MLA_R + d;
-  constexpr int STEP = BY_HEAD ? 1 : 4;
-#pragma unroll 8
-  for (int r = BY_HEAD ? 0 : grp; r < parts; r += STEP) {
-    const f32x4v v =
-        *reinterpret_cast<const f32x4v*>(src + (size_t)r * H * MLA_R);
+  auto add = [&](f32x4v part, int r) {
     const float w = wt[BY_HEAD ? grp : 0][r];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s[i] = fmaf(v[i], w, s[i]);
-  }
+    for (int i = 0; i < 4; ++i) s[i] = fmaf(part[i], w, s[i]);
+  };
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+    if (mine + i * STEP < parts) add(v[i], mine + i * STEP);
+#pragma unroll 8
+  for (int r = mine + AHEAD * STEP; r < parts; r += STEP)
+    add(*reinterpret_cast<const f32x4v*>(src + (size_t)r * H * MLA_R), r);
   if (!BY_HEAD) {
     sums[grp][tid & 127] = s;
     __syncthreads();
@@ -642,10 +681,8 @@ __global__ __launch_bounds__(512) void mla_reduce_kernel(
   }
   if (!on) return;
   const float inv = 1.f / l;
-  uint2 v;
-  v.x = pack_bf16(s[0] * inv, s[1] * inv);
-  v.y = pack_bf16(s[2] * inv, s[3] * inv);
-  *reinterpret_cast<uint2*>(out + ((size_t)seq * H + head) * MLA_R + d) = v;
+  *reinterpret_cast<uint2*>(out + ((size_t)seq * H + head) * MLA_R + d) = make_uint2(
+      pack_bf16(s[0] * inv, s[1] * inv), pack_bf16(s[2] * inv, s[3] * inv));
 }
 
 // Runs the tiles are dealt to; 0: every sequence has a workgroup of its own.
