@@ -679,7 +679,7 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
   const int r0 = first / per, r1 = (first + units - 1) / per;
   if (r0 == r1) return;  // finished by its run
 
-  __shared__ float wt[16][PD_MAX_RUNS];
+  extern __shared__ float wt[];  // [G][runs]
   __shared__ float den[16];
   __shared__ f32x4v sums[256];
   const int parts = r1 - r0 + 1;
@@ -693,7 +693,7 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
       const float* ml = tmp_ml + (row0 + (size_t)r * Hq + g) * 2;
       const float w = __builtin_amdgcn_exp2f(ml[0] - M);
       l += ml[1] * w;
-      wt[g][r] = w;
+      wt[g * runs + r] = w;
     }
     l = wave_reduce_sum(l);
     if (lane == 0)
@@ -714,7 +714,7 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
       const float* src = tmp_acc + (row0 + g) * D + d;
 #pragma unroll 4
       for (int r = groups > 1 ? grp : 0; r < parts; r += groups)
-        s += *reinterpret_cast<const f32x4v*>(src + (size_t)r * Hq * D) * wt[g][r];
+        s += *reinterpret_cast<const f32x4v*>(src + (size_t)r * Hq * D) * wt[g * runs + r];
     }
     if (groups > 1) {
       sums[tid] = s;
@@ -793,9 +793,9 @@ extern "C" void launch_paged_decode(
   }
   if (runs > 0) {
     auto reduce = [&](auto kernel) {
-      kernel<<<dim3(Hk, B), 256, 0, stream>>>((uint16_t*)out, tmp_acc, tmp_ml,
-                                              seq_lens, sinks, B, Hk, G, window,
-                                              4 * PD_KT, runs);
+      kernel<<<dim3(Hk, B), 256, G * runs * sizeof(float), stream>>>(
+          (uint16_t*)out, tmp_acc, tmp_ml, seq_lens, sinks, B, Hk, G, window, 4 * PD_KT,
+          runs);
     };
     if (D == 128) reduce(paged_decode_reduce_kernel<128>);
     else reduce(paged_decode_reduce_kernel<64>);
