@@ -198,6 +198,20 @@ def test_quantize_fp8_tensor(dtype, n):
             assert torch.equal(a.nan_to_num(), b.nan_to_num())
 
 
+# both passes' grids at and past their ends: 1,024 and 2,048 workgroups of 2,048 values
+@pytest.mark.parametrize("n", [1024 * 2048, 1024 * 2048 + 1, 2048 * 2048 + 1, 9000003])
+@pytest.mark.parametrize("at", [0, -1])
+def test_quantize_fp8_tensor_large(n, at):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = _rand(g, n).bfloat16()
+    x[at] = 1000.0
+    q, s = ops._require_ext("quantize_fp8_tensor").quantize_fp8_tensor(x)
+    want_s = (x.float().abs().amax() / 448.0).reshape(1)
+    want = (x.float() / want_s).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+    assert torch.equal(s, want_s)
+    assert torch.equal(q.view(torch.uint8), want.view(torch.uint8))
+
+
 @pytest.mark.parametrize("B,H", [(1, 16), (8, 3), (16, 128), (33, 16), (70, 2)])
 def test_mla_products(B, H):
     g = torch.Generator(device="cuda").manual_seed(B)
