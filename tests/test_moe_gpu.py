@@ -429,3 +429,23 @@ def test_moe_few_infinities_and_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("k", [1, 7, 8, 9, 17])
+def test_moe_combine_leaves_out_rows_nobody_wrote(k):
+    """Choices are added up eight at a time. Those of no expert have rows that nothing
+    writes, here over memory that held NaN; a token of such choices only is zero."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    T, E, H, I = 40, 20, 320, 64
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
+    ids = torch.randint(-1, E + 1, (T, k), generator=g, device="cuda")
+    ids[3], ids[4], ids[4, -1] = -1, E, 0
+    w = 0.5 + 0.5 * torch.rand(T, k, generator=g, device="cuda")
+    want = _experts64(x, gu, dn, ids, w)
+    poison = [torch.full((T * k, H), float("nan"), device="cuda") for _ in range(4)]
+    del poison
+    got = ops.fused_moe_forward(x, gu, dn, ids, w)
+    assert not got[3].any() and not got[~((ids >= 0) & (ids < E)).any(1)].any()
+    assert ((got - want).norm(dim=1) <= 2 ** -7 * want.norm(dim=1) + 1e-30).all()
