@@ -104,11 +104,17 @@ class MLAAttention(nn.Module):
         q = q.view(T, H, self.dn + self.dr)
         q_nope, q_pe = q[..., : self.dn], q[..., self.dn :]
 
-        kv_a = ops.linear(x, self.kv_a_proj_with_mqa.weight)
+        weight = self.kv_a_proj_with_mqa.weight
         cache = meta.mla_cache.layer(self.local_layer_idx)
         norm, pe = self.kv_a_layernorm, q_pe
         q_pe = None
-        if plain_call(norm, RMSNorm.forward):  # a hook sees the latent rows
+        joins = plain_call(norm, RMSNorm.forward)  # a hook sees the latent rows
+        if joins and ops.product_has_parts(T, weight):
+            q_pe = ops.linear_mla_rope_and_cache(
+                x, weight, pe, norm.weight, norm.eps, meta.positions, rope_cache, cache,
+                meta.slot_mapping, is_neox=self.rope_neox)
+        kv_a = ops.linear(x, weight) if q_pe is None else None
+        if joins and q_pe is None:
             q_pe = ops.mla_rope_and_cache(
                 pe, kv_a, norm.weight, norm.eps, meta.positions, rope_cache, cache,
                 meta.slot_mapping, is_neox=self.rope_neox)

@@ -185,6 +185,24 @@ def mla_rope_and_cache(
         slot_mapping.to(torch.int64), is_neox)
 
 
+def linear_mla_rope_and_cache(
+    x: torch.Tensor, kv_weight: torch.Tensor, q_pe: torch.Tensor,
+    norm_weight: torch.Tensor, eps: float, positions: torch.Tensor,
+    cos_sin: torch.Tensor, cache: torch.Tensor, slot_mapping: torch.Tensor,
+    is_neox: bool = True,
+) -> Optional[torch.Tensor]:
+    """mla_rope_and_cache() of kv = linear(x, kv_weight) of few rows: the launch that
+    rotates and stores adds up the product's parts too. None where the product has no
+    parts (product_has_parts()) or there is no kernel; no part of autograd."""
+    if not x.is_cuda or SKINNY_GEMM_MAX_M < x.shape[0] or (
+            torch.is_grad_enabled() and any(
+                t.requires_grad for t in (x, kv_weight, q_pe, norm_weight))):
+        return None
+    return _require_ext("linear_mla_rope_and_cache").linear_mla_rope_and_cache(
+        x, kv_weight, q_pe, norm_weight, eps, positions.to(torch.int32), cos_sin, cache,
+        slot_mapping.to(torch.int64), is_neox)
+
+
 # -- attention ---------------------------------------------------------------------
 
 

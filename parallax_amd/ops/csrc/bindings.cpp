@@ -35,7 +35,7 @@ void launch_mla_reshape_and_cache(const void*, const void*, void*,
                                   float, hipStream_t);
 void launch_mla_rope_and_cache(void*, const void*, const void*, const void*, void*,
                                const int*, const float*, const int64_t*, int, int,
-                               int, int, int64_t, int64_t, int64_t, float, bool,
+                               int, int, int64_t, int64_t, int64_t, int, float, bool,
                                bool, hipStream_t);
 void launch_act_and_mul(void*, const void*, int64_t, int, bool, hipStream_t);
 void launch_paged_attention_decode(void*, const void*, const void*, const void*,
@@ -261,6 +261,52 @@ void mla_reshape_and_cache(torch::Tensor latent, torch::Tensor k_rope,
                                is_fp8(cache), 1.0f, cur_stream());
 }
 
+// What mla_rope_and_cache asks of all but kv
+static bool mla_rope_takes(const torch::Tensor& q, const torch::Tensor& w,
+                           const torch::Tensor& positions,
+                           const torch::Tensor& cos_sin, const torch::Tensor& cache,
+                           const torch::Tensor& slot_mapping) {
+  if (q.dim() != 3 || w.dim() != 1 || cache.dim() != 3 || cos_sin.dim() != 2 ||
+      positions.dim() != 1 || slot_mapping.dim() != 1)
+    return false;
+  const int64_t T = q.size(0), H = q.size(1), DR = q.size(2), R = w.size(0);
+  auto at16 = [](const torch::Tensor& t) {
+    return (uintptr_t)t.data_ptr() % 16 == 0;
+  };
+  if (q.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 ||
+      (cache.scalar_type() != at::kBFloat16 && !is_fp8(cache)) ||
+      cos_sin.scalar_type() != at::kFloat ||
+      positions.scalar_type() != at::kInt ||
+      slot_mapping.scalar_type() != at::kLong || positions.size(0) != T ||
+      slot_mapping.size(0) != T || cos_sin.size(1) != DR || cache.size(2) != R + DR)
+    return false;
+  // pieces of 16 rotated values, at most a wave of them; vectors of 16 bytes
+  return !(T == 0 || T > INT_MAX || H == 0 || R % 8 || DR % 16 || DR > 1024 ||
+           H * DR > 1 << 24 || q.stride(2) != 1 || q.stride(1) % 8 ||
+           q.stride(0) % 8 || !at16(q) || !at16(w) || !at16(cos_sin) ||
+           !at16(cache) || !w.is_contiguous() || !cache.is_contiguous() ||
+           !cos_sin.is_contiguous() || !positions.is_contiguous() ||
+           !slot_mapping.is_contiguous());
+}
+
+// kv: bf16 rows, or (splits > 0) the fp32 parts of their product
+static torch::Tensor mla_rope_run(const torch::Tensor& q, const torch::Tensor& kv,
+                                  int splits, const torch::Tensor& w, double eps,
+                                  const torch::Tensor& positions,
+                                  const torch::Tensor& cos_sin,
+                                  const torch::Tensor& cache,
+                                  const torch::Tensor& slot_mapping, bool neox) {
+  const int64_t T = q.size(0), H = q.size(1), DR = q.size(2), R = w.size(0);
+  auto out = torch::empty({T, H, DR}, q.options());
+  launch_mla_rope_and_cache(
+      out.data_ptr(), q.data_ptr(), kv.data_ptr(), w.data_ptr(), cache.data_ptr(),
+      positions.data_ptr<int>(), cos_sin.data_ptr<float>(),
+      slot_mapping.data_ptr<int64_t>(), T, H, R, DR, q.stride(0), q.stride(1),
+      splits > 0 ? 0 : kv.stride(0), splits, (float)eps, neox, is_fp8(cache),
+      cur_stream());
+  return out;
+}
+
 // rotated q [T, H, DR]; kv's normed latent and rotated key go to the cache. None where
 // there is no kernel.
 std::optional<torch::Tensor> mla_rope_and_cache(
@@ -268,38 +314,12 @@ std::optional<torch::Tensor> mla_rope_and_cache(
     torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor cache,
     torch::Tensor slot_mapping, bool neox) {
   CHECK_GPU(q);
-  if (q.dim() != 3 || kv.dim() != 2 || w.dim() != 1 || cache.dim() != 3 ||
-      cos_sin.dim() != 2 || positions.dim() != 1 || slot_mapping.dim() != 1)
+  if (!mla_rope_takes(q, w, positions, cos_sin, cache, slot_mapping) ||
+      kv.dim() != 2 || kv.scalar_type() != at::kBFloat16 ||
+      kv.size(0) != q.size(0) || kv.size(1) != cache.size(2) || kv.stride(1) != 1 ||
+      kv.stride(0) % 8 || (uintptr_t)kv.data_ptr() % 16)
     return std::nullopt;
-  const int64_t T = q.size(0), H = q.size(1), DR = q.size(2), R = w.size(0);
-  auto at16 = [](const torch::Tensor& t) {
-    return (uintptr_t)t.data_ptr() % 16 == 0;
-  };
-  if (q.scalar_type() != at::kBFloat16 || kv.scalar_type() != at::kBFloat16 ||
-      w.scalar_type() != at::kBFloat16 ||
-      (cache.scalar_type() != at::kBFloat16 && !is_fp8(cache)) ||
-      cos_sin.scalar_type() != at::kFloat ||
-      positions.scalar_type() != at::kInt ||
-      slot_mapping.scalar_type() != at::kLong || kv.size(0) != T ||
-      kv.size(1) != R + DR || positions.size(0) != T || slot_mapping.size(0) != T ||
-      cos_sin.size(1) != DR || cache.size(2) != R + DR)
-    return std::nullopt;
-  // pieces of 16 rotated values, at most a wave of them; vectors of 16 bytes
-  if (T == 0 || T > INT_MAX || H == 0 || R % 8 || DR % 16 || DR > 1024 ||
-      H * DR > 1 << 24 ||
-      q.stride(2) != 1 || q.stride(1) % 8 || q.stride(0) % 8 || kv.stride(1) != 1 ||
-      kv.stride(0) % 8 || !at16(q) || !at16(kv) || !at16(w) || !at16(cos_sin) ||
-      !at16(cache) || !w.is_contiguous() || !cache.is_contiguous() ||
-      !cos_sin.is_contiguous() || !positions.is_contiguous() ||
-      !slot_mapping.is_contiguous())
-    return std::nullopt;
-  auto out = torch::empty({T, H, DR}, q.options());
-  launch_mla_rope_and_cache(
-      out.data_ptr(), q.data_ptr(), kv.data_ptr(), w.data_ptr(), cache.data_ptr(),
-      positions.data_ptr<int>(), cos_sin.data_ptr<float>(),
-      slot_mapping.data_ptr<int64_t>(), T, H, R, DR, q.stride(0), q.stride(1),
-      kv.stride(0), (float)eps, neox, is_fp8(cache), cur_stream());
-  return out;
+  return mla_rope_run(q, kv, 0, w, eps, positions, cos_sin, cache, slot_mapping, neox);
 }
 
 void silu_and_mul(torch::Tensor out, torch::Tensor x) {
@@ -1185,6 +1205,34 @@ std::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> linear_no
   return std::make_tuple(q, scale, sum);
 }
 
+// mla_rope_and_cache of kv = x . kv_w^T, whose parts its launch adds up. None where
+// linear() has none for that product, and where mla_rope_and_cache has no kernel.
+std::optional<torch::Tensor> linear_mla_rope_and_cache(
+    torch::Tensor x, torch::Tensor kv_w, torch::Tensor q, torch::Tensor w, double eps,
+    torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor cache,
+    torch::Tensor slot_mapping, bool neox) {
+  CHECK_GPU(x);
+  if (!mla_rope_takes(q, w, positions, cos_sin, cache, slot_mapping) ||
+      x.dim() != 2 || kv_w.dim() != 2 || x.scalar_type() != at::kBFloat16 ||
+      kv_w.scalar_type() != at::kBFloat16 || x.size(0) != q.size(0) ||
+      x.size(1) != kv_w.size(1) || kv_w.size(0) != cache.size(2) ||
+      !kv_w.is_contiguous() || (uintptr_t)kv_w.data_ptr() % 16 ||
+      (uintptr_t)x.data_ptr() % 16 || x.stride(1) != 1 || x.stride(0) % 8)
+    return std::nullopt;
+  const int64_t M = x.size(0), K = x.size(1), N = kv_w.size(0);
+  if (M > 128 || K == 0 || K > INT_MAX / 2 ||
+      (M - 1) * x.stride(0) * 2 + 128 > UINT32_MAX)
+    return std::nullopt;
+  const int splits = product_parts(M, N, K * 2);
+  if (splits <= 1) return std::nullopt;
+  auto part = torch::empty({splits, M, N}, x.options().dtype(at::kFloat));
+  launch_skinny_split(nullptr, part.data_ptr<float>(), splits, x.data_ptr(),
+                      kv_w.data_ptr(), nullptr, nullptr, nullptr, false, M, N, K * 2,
+                      x.stride(0) * 2, 0, false, cur_stream());
+  return mla_rope_run(q, part, splits, w, eps, positions, cos_sin, cache, slot_mapping,
+                      neox);
+}
+
 static bool rows16(const torch::Tensor& t) {
   return t.scalar_type() == at::kBFloat16 && (uintptr_t)t.data_ptr() % 16 == 0 &&
          t.stride(2) == 1 && t.stride(1) % 8 == 0 && t.stride(0) % 8 == 0;
@@ -1295,6 +1343,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("reshape_and_cache", &reshape_and_cache);
   m.def("mla_reshape_and_cache", &mla_reshape_and_cache);
   m.def("mla_rope_and_cache", &mla_rope_and_cache);
+  m.def("linear_mla_rope_and_cache", &linear_mla_rope_and_cache);
   m.def("silu_and_mul", &silu_and_mul);
   m.def("gelu_and_mul", &gelu_and_mul);
   m.def("paged_attention_decode", &paged_attention_decode);

@@ -308,3 +308,37 @@ def test_mla_rope_and_cache(T, H, R, DR, fp8, neox):
     assert ops.mla_rope_and_cache(q.float(), kv, *args) is None
     assert ops.mla_rope_and_cache(q[..., :DR - 8], kv, *args) is None
     assert ops.mla_rope_and_cache(q, kv[:, 1:], *args) is None
+
+
+@pytest.mark.parametrize("M,K,R,DR", [(17, 7168, 512, 64), (40, 7168, 512, 64),
+                                      (64, 7168, 512, 64), (33, 8192, 64, 16),
+                                      (70, 7168, 1544, 128), (20, 16384, 512, 64)])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("neox", [False, True])
+def test_linear_mla_rope_and_cache(M, K, R, DR, fp8, neox):
+    """The same bits as the product and mla_rope_and_cache: parts are added in one
+    order. Infinities of x and a token without a slot included."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    x, kv_w = rand(M, K + 8)[:, :K], rand(R + DR, K) * K ** -0.5
+    q, w = rand(M, 3, DR + 32)[..., 32:], rand(R)
+    x[3, 5] = float("inf")
+    table = torch.randn(90, DR, generator=g, device="cuda")
+    pos = torch.randint(0, 90, (M,), generator=g, device="cuda", dtype=torch.int32)
+    slots = torch.randperm(96, generator=g, device="cuda")[:M]
+    slots[M // 2] = -1
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    caches = [torch.zeros(6, 16, R + DR, device="cuda").to(dt) for _ in range(2)]
+    args = lambda c: (w, 1e-6, pos, table, c, slots, neox)
+    assert ops.product_has_parts(M, kv_w)
+    got = ops.linear_mla_rope_and_cache(x, kv_w, q, *args(caches[0]))
+    want = ops.mla_rope_and_cache(q, ops.linear(x, kv_w), *args(caches[1]))
+    assert torch.equal(got, want)
+    assert torch.equal(caches[0].view(torch.uint8), caches[1].view(torch.uint8))
+    run = lambda x=x, kv_w=kv_w, q=q: ops.linear_mla_rope_and_cache(
+        x, kv_w, q, *args(caches[0]))
+    assert run(x=x[:4], q=q[:4]) is None and run(x=x[:-1]) is None
+    assert run(x=x.float()) is None and run(kv_w=kv_w.float()) is None
+    assert run(kv_w=kv_w[:-8]) is None and run(q=q.float()) is None
+    assert run(x=rand(M, K + 4)[:, 4:]) is None              # rows at odd places
+    assert run(kv_w=kv_w.clone().requires_grad_()) is None
