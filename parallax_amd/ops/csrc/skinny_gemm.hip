@@ -642,6 +642,44 @@ extern "C" bool skinny_pays(int M, int N, int row_bytes) {
   return (large || row_bytes >= 14336) && row_bytes >= (M > 64 ? 7168 : 4096);
 }
 
+// From 33 rows on, where K is not split: tiles of skinny_gemm_kernel over pieces of 32
+// rows, 0: the ways above. Small weights come from L2 again for every piece, and the
+// narrowest tile that still finds room on the chip at once has the shortest chain. us of
+// products with tiles of 16 / 32 / 64 rows of W and of the library, with its activation
+// and bias where there are some, W from memory (N x K; gated ones by g, bias by b):
+//   64 rows: 896 x 896 4.1 / 5.6 / 8.1 (6.0), 1152 x 896 b 4.4 / 6.1 / 8.9 (9.2), 128 x
+//   2048 4.4 / 7.8 / 12 (6.6), 2048 x 2048 5.8 / 8.1 / 13 (7.6), 896 x 4864 10.5 / 14 /
+//   24 (13.3), 2560 x 2560 10.1 / 10.6 / 15 (14.0), 4096 x 2048 9.7 / 9.0 / 13 (12.2),
+//   9728 x 896 g 13.2 / 12.5 / 10.1 (14.6); in fp8 896 x 896 3.6 / 4.7 / 6.1 (6.1), 2048
+//   x 2048 4.5 / 5.7 / 7.6 (6.0), 4096 x 7168 13.4 / 11.5 / 16 (12.4)
+//   128 rows: 896 x 896 4.1 / 5.7 / 8.0 (6.0), 1152 x 896 b 5.7 / 6.1 / 9.0 (9.8), 2048 x
+//   1536 b 7.2 / 7.7 / 12 (10.3), 896 x 4864 10.2 / 14 / 24 (21), 3072 x 3072 15.9 / 12.2
+//   / 17 (15.8), 6144 x 1024 g 14.6 / 13.2 / 10.7 (12.5)
+// Not where more blocks than there is room for wait for a second round or the weight's
+// stream counts for more: 9728 x 896 g at 128 rows 20 / 17 / 17 (14.7), 5120 x 3072 at 96
+// 21 / 18 / 18 (15), 5120 x 2560 at 65 17 / 15 / 15 (12.6), 6144 x 2048 at 64 14 / 13 / 13
+// (11.6); nor wide tiles of long rows, 2048 x 4096 at 128 14 / 13.3 / 21 (12.7), in fp8
+// 7168 x 2048 at 96 13 / 11 / 9.4 (8.9). Fewer than 64 blocks of long rows are the
+// library's as before (256 x 4096, which a test has there, 6.4 / 12 / 20 (8.9) at 40).
+static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
+  if (M <= 32 || M > 128 || row_bytes % 128 || N % 4) return 0;
+  const int64_t bytes = (int64_t)N * row_bytes;
+  auto blocks = [&](int nt) { return ceil_div(M, 32) * ceil_div(N, nt); };
+  if (bytes > 26000000 || (row_bytes > 4096 && blocks(16) < 64)) return 0;
+  if (row_bytes <= 14336 && blocks(16) <= (N <= 2048 ? 384 : 320)) return 16;
+  if (row_bytes <= (N > 2048 ? 12288 : 6144) &&
+      blocks(32) <= (bytes > 20000000 ? 340 : 384))
+    return 32;
+  return row_bytes <= (gated ? 2048 : 1920) && blocks(64) <= 512 ? 64 : 0;
+}
+
+// K split over workgroups stays: its parts are what launch_skinny_norm adds up
+extern "C" bool skinny_in_pieces(int M, int N, int row_bytes, bool gated) {
+  return skinny_pieces(M, N, row_bytes, gated) > 0 &&
+         (skinny_shared(M, N, row_bytes) <= 1 ||
+          (!gated && !skinny_pays(M, N, row_bytes)));
+}
+
 // batch products of the same shape: x, w and c advance by x_batch bytes, N rows
 // and c_batch elements. Any number of rows of X, 32 at a time.
 extern "C" void launch_skinny_gemm(
@@ -651,7 +689,8 @@ extern "C" void launch_skinny_gemm(
     int64_t x_batch, int64_t c_batch, bool gated, hipStream_t stream,
     bool* launched) {
   *launched = false;
-  const int nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes, gated);
+  int nt = batch == 1 ? skinny_pieces(M, N, row_bytes, gated) : 0;
+  if (nt == 0) nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes, gated);
   if (nt == 0 || row_bytes % 128 || N % 4) return;
   *launched = true;
   auto run = [&](auto kernel, int xr, int waves) {

@@ -174,6 +174,49 @@ def test_linear_fp8_rows(M, N, K):
         atol=K * K * 2 ** -24)
 
 
+@pytest.mark.parametrize("M", [33, 64, 65, 97, 128])
+@pytest.mark.parametrize("N,K,kind,own", [
+    (4, 64, "bias", True), (1152, 896, "bias", True), (1284, 4928, "", True),  # 16 rows
+    (2052, 960, "bias", True), (2900, 2112, "", True),                         # 32
+    (9680, 64, "gated", None), (7664, 896, "gated", True),                     # 64
+    (900, 2176, "fp8", True), (2564, 3968, "fp8", True), (7664, 1024, "fp8gated", None),
+    (13004, 1024, "", False), (240, 2112, "", False),
+])
+def test_linear_in_pieces_of_32_rows(M, N, K, kind, own):
+    """Cut tiles and pieces, against fp32. Infinities stay in their rows and columns.
+    own: whether a kernel takes it, whatever M is."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    fp8, gated = kind.startswith("fp8"), kind.endswith("gated")
+    x, w = _rand(g, M, K + 64).bfloat16()[:, :K], _rand(g, N, K).bfloat16()
+    none, one = x.new_empty(0), torch.ones(1, device="cuda")
+    b = _rand(g, N).bfloat16() if kind == "bias" else none
+    if fp8:
+        x, w = x.contiguous().to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+    run = lambda: ops._require_ext("few_rows").few_rows(
+        x, w, b, one if fp8 else none, one if fp8 else none, gated)
+    got = run()
+    assert own is None or (got is not None) == own
+    if got is None:
+        return
+    want = x.float() @ w.float().t()
+    if b.numel():
+        want += b.float()
+    atol = K * K * 2 ** -24
+    if gated:   # both products rounded to bf16, |silu'| < 1.1, the result rounded
+        a, u = want.bfloat16().float().chunk(2, dim=1)
+        s = torch.nn.functional.silu(a)
+        want = s * u
+        atol = (atol + 2 ** -7 * a.abs()) * 1.1 * u.abs() + (
+            atol + 2 ** -7 * u.abs()) * s.abs() + 1e-6
+    assert ((got.float() - want).abs() <= atol + 2 ** -7 * want.abs()).all()
+    if fp8 or gated:
+        return
+    w[N - 1, 0] = x[M - 1, K - 1] = float("inf")
+    again = run()
+    assert not again[M - 1].isfinite().any() and not again[:, N - 1].isfinite().any()
+    assert torch.equal(again[:-1, :-1], got[:-1, :-1])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("n", [1, 7, 2048, 2057, 700001])
 def test_quantize_fp8_tensor(dtype, n):
