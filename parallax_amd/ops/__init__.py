@@ -556,6 +556,7 @@ def gelu_and_mul(x: torch.Tensor) -> torch.Tensor:
 # Rows of x up to which linear() and linear_fp8() try the weight-streaming kernels
 # (there are none above 128); 0 leaves every product to the library.
 SKINNY_GEMM_MAX_M = int(os.environ.get("PARALLAX_SKINNY_GEMM_MAX_M", "128"))
+PIECES_MAX_BYTES = 26_000_000  # of weights with kernels for up to three times as many rows
 NORM_LINEAR_MAX_M = 4  # rows of x up to which norm_linear() has kernels
 LT_GEMM = os.environ.get("PARALLAX_LT_GEMM", "1") != "0"
 _NONE = torch.empty(0, dtype=torch.bfloat16)  # an argument that is not there
@@ -570,7 +571,9 @@ def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
     if not (
         x.dim() == 2
         and (fp8 or x.dtype == weight.dtype == torch.bfloat16)
-        and 0 < x.shape[0] <= SKINNY_GEMM_MAX_M
+        and (0 < x.shape[0] <= SKINNY_GEMM_MAX_M
+             or (SKINNY_GEMM_MAX_M < x.shape[0] <= 3 * SKINNY_GEMM_MAX_M
+                 and weight.numel() * weight.element_size() <= PIECES_MAX_BYTES))
         and weight.is_contiguous()
         and x.stride(1) == 1
         and (bias is None or bias.dtype == torch.bfloat16)

@@ -655,6 +655,11 @@ extern "C" bool skinny_pays(int M, int N, int row_bytes) {
 //   128 rows: 896 x 896 4.1 / 5.7 / 8.0 (6.0), 1152 x 896 b 5.7 / 6.1 / 9.0 (9.8), 2048 x
 //   1536 b 7.2 / 7.7 / 12 (10.3), 896 x 4864 10.2 / 14 / 24 (21), 3072 x 3072 15.9 / 12.2
 //   / 17 (15.8), 6144 x 1024 g 14.6 / 13.2 / 10.7 (12.5)
+//   192 rows: 896 x 896 5.5 / 5.7 / 8.1 (6.2), 1152 x 896 b 5.9 / 6.2 / 9.1 (10.0), 2048 x
+//   1536 b 9.7 / 8.2 / 12 (14.4), 896 x 4864 12.9 / 14 / 24 (22), 128 x 2048 4.9 / 7.8 /
+//   12 (6.4); 384 rows, the last: 7.4 / 6.5 / 8.2 (6.6), 9.3 / 7.1 / 9.1 (10.1), 16 / 14.3
+//   / 13 (15), 21 / 18 / 24 (18), 4.9 / 7.9 / 12 (7.6); 512: 896 x 896 8.9 / 6.6 / 8.3
+//   (7.3), 1536 x 1536 14.4 / 13.6 / 12.2 (9.2)
 // Not where more blocks than there is room for wait for a second round or the weight's
 // stream counts for more: 9728 x 896 g at 128 rows 20 / 17 / 17 (14.7), 5120 x 3072 at 96
 // 21 / 18 / 18 (15), 5120 x 2560 at 65 17 / 15 / 15 (12.6), 6144 x 2048 at 64 14 / 13 / 13
@@ -662,7 +667,7 @@ extern "C" bool skinny_pays(int M, int N, int row_bytes) {
 // 7168 x 2048 at 96 13 / 11 / 9.4 (8.9). Fewer than 64 blocks of long rows are the
 // library's as before (256 x 4096, which a test has there, 6.4 / 12 / 20 (8.9) at 40).
 static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
-  if (M <= 32 || M > 128 || row_bytes % 128 || N % 4) return 0;
+  if (M <= 32 || M > 384 || row_bytes % 128 || N % 4) return 0;
   const int64_t bytes = (int64_t)N * row_bytes;
   auto blocks = [&](int nt) { return ceil_div(M, 32) * ceil_div(N, nt); };
   if (bytes > 26000000 || (row_bytes > 4096 && blocks(16) < 64)) return 0;

@@ -174,14 +174,16 @@ def test_linear_fp8_rows(M, N, K):
         atol=K * K * 2 ** -24)
 
 
-@pytest.mark.parametrize("M", [33, 64, 65, 97, 128])
-@pytest.mark.parametrize("N,K,kind,own", [
+@pytest.mark.parametrize("M,N,K,kind,own", [(M, *c) for M in (33, 64, 65, 97, 128) for c in (
     (4, 64, "bias", True), (1152, 896, "bias", True), (1284, 4928, "", True),  # 16 rows
     (2052, 960, "bias", True), (2900, 2112, "", True),                         # 32
     (9680, 64, "gated", None), (7664, 896, "gated", True),                     # 64
     (900, 2176, "fp8", True), (2564, 3968, "fp8", True), (7664, 1024, "fp8gated", None),
     (13004, 1024, "", False), (240, 2112, "", False),
-])
+)] + [(M, *c) for M in (129, 300, 384) for c in (
+    (4, 64, "bias", True), (900, 896, "bias", True), (640, 1024, "gated", True),
+    (900, 2176, "fp8", True), (3076, 2048, "", False),
+)] + [(385, 896, 896, "", False)])
 def test_linear_in_pieces_of_32_rows(M, N, K, kind, own):
     """Cut tiles and pieces, against fp32. Infinities stay in their rows and columns.
     own: whether a kernel takes it, whatever M is."""
