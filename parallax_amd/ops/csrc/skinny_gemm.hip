@@ -644,34 +644,43 @@ extern "C" bool skinny_pays(int M, int N, int row_bytes) {
 
 // From 33 rows on, where K is not split: tiles of skinny_gemm_kernel over pieces of 32
 // rows, 0: the ways above. Small weights come from L2 again for every piece, and the
-// narrowest tile that still finds room on the chip at once has the shortest chain. us of
-// products with tiles of 16 / 32 / 64 rows of W and of the library, with its activation
-// and bias where there are some, W from memory (N x K; gated ones by g, bias by b):
-//   64 rows: 896 x 896 4.1 / 5.6 / 8.1 (6.0), 1152 x 896 b 4.4 / 6.1 / 8.9 (9.2), 128 x
-//   2048 4.4 / 7.8 / 12 (6.6), 2048 x 2048 5.8 / 8.1 / 13 (7.6), 896 x 4864 10.5 / 14 /
-//   24 (13.3), 2560 x 2560 10.1 / 10.6 / 15 (14.0), 4096 x 2048 9.7 / 9.0 / 13 (12.2),
-//   9728 x 896 g 13.2 / 12.5 / 10.1 (14.6); in fp8 896 x 896 3.6 / 4.7 / 6.1 (6.1), 2048
-//   x 2048 4.5 / 5.7 / 7.6 (6.0), 4096 x 7168 13.4 / 11.5 / 16 (12.4)
-//   128 rows: 896 x 896 4.1 / 5.7 / 8.0 (6.0), 1152 x 896 b 5.7 / 6.1 / 9.0 (9.8), 2048 x
-//   1536 b 7.2 / 7.7 / 12 (10.3), 896 x 4864 10.2 / 14 / 24 (21), 3072 x 3072 15.9 / 12.2
-//   / 17 (15.8), 6144 x 1024 g 14.6 / 13.2 / 10.7 (12.5)
-//   192 rows: 896 x 896 5.5 / 5.7 / 8.1 (6.2), 1152 x 896 b 5.9 / 6.2 / 9.1 (10.0), 2048 x
-//   1536 b 9.7 / 8.2 / 12 (14.4), 896 x 4864 12.9 / 14 / 24 (22), 128 x 2048 4.9 / 7.8 /
-//   12 (6.4); 384 rows, the last: 7.4 / 6.5 / 8.2 (6.6), 9.3 / 7.1 / 9.1 (10.1), 16 / 14.3
-//   / 13 (15), 21 / 18 / 24 (18), 4.9 / 7.9 / 12 (7.6); 512: 896 x 896 8.9 / 6.6 / 8.3
-//   (7.3), 1536 x 1536 14.4 / 13.6 / 12.2 (9.2)
-// Not where more blocks than there is room for wait for a second round or the weight's
-// stream counts for more: 9728 x 896 g at 128 rows 20 / 17 / 17 (14.7), 5120 x 3072 at 96
-// 21 / 18 / 18 (15), 5120 x 2560 at 65 17 / 15 / 15 (12.6), 6144 x 2048 at 64 14 / 13 / 13
-// (11.6); nor wide tiles of long rows, 2048 x 4096 at 128 14 / 13.3 / 21 (12.7), in fp8
-// 7168 x 2048 at 96 13 / 11 / 9.4 (8.9). Fewer than 64 blocks of long rows are the
-// library's as before (256 x 4096, which a test has there, 6.4 / 12 / 20 (8.9) at 40).
+// narrowest tile that still finds room on the chip at once has the shortest chain: 16
+// rows of W a block while every CU has one at most, then 32 by four waves (98 KB, one
+// block a CU) up to there, then 32 by two and 64 as far as two blocks a CU go. us of
+// products with tiles of 16 / 32 by four waves / 32 by two / 64 rows of W and of the
+// library, with its activation and bias where there are some, W from memory (N x K; gated
+// ones by g, bias by b):
+//   64 rows: 896 x 896 4.1 / 5.2 / 5.6 / 8.1 (6.0), 1152 x 896 b 4.4 / 5.4 / 6.1 / 9.0
+//   (9.2), 2048 x 1536 b 5.2 / 6.3 / 7.6 / 11 (11), 896 x 4864 10.5 / 14 / 14 / 24 (13.3),
+//   3072 x 2048 9.5 / 8.5 / 8.7 / 13 (9.8), 4096 x 2560 11.2 / 10.0 / 10.6 / 15 (11.4),
+//   9728 x 896 g 13 / 14 / 12.5 / 10.1 (14.6); in fp8 896 x 896 3.6 / - / 4.7 / 6.1 (6.1),
+//   2048 x 8192 7.1 / 8.8 / 10.9 / 16 (9.4), 4096 x 7168 13 / 9.2 / 11.1 / 16 (10.1)
+//   128 rows: 896 x 896 4.2 / 5.2 / 5.7 / 8.1 (6.1), 1152 x 896 b 5.6 / 5.6 / 6.1 / 9.0
+//   (9.1), 1536 x 1536 6.5 / 6.0 / 7.0 / 11 (7.1), 2048 x 2048 8.4 / 7.0 / 8.1 / 13 (8.2),
+//   896 x 4864 10.2 / 14 / 14 / 24 (13 to 21), 3072 x 3072 16 / 16 / 12.1 / 17 (14), 6144 x
+//   1024 g 15 / 14 / 13 / 10.6 (12.5 to 15); in fp8 2048 x 8192 12 / 9.0 / 11 / 16 (10.5)
+//   192 and 384 rows, the last: 896 x 896 5.5 / 5.3 / 5.6 / 8.1 (6.5) and 7.4 / 8.2 / 6.5 /
+//   8.2 (6.6 to 8.3), 1152 x 896 b 5.9 / 5.5 / 6.1 / 9.0 (9.6) and 9.2 / 8.7 / 7.0 / 9.1
+//   (12), 1024 x 2048 7.3 / 6.4 / 8.1 / 13 (7.4) and 10.2 / 10.4 / 8.8 / 13 (9.1); 512:
+//   1536 x 1536 14.4 / - / 13.6 / 12.2 (9.2)
+// Not where blocks wait for a second round or the weight's stream counts for more: 9728 x
+// 896 g at 128 rows 20 / 20 / 17 / 17 (14.7), 5120 x 3072 at 96 21 / - / 18 / 18 (15), 5120
+// x 2560 at 65 17 / - / 15 / 15 (12.6), 6144 x 2048 at 64 14 / - / 13 / 13 (11.6); nor wide
+// tiles of long rows: in fp8 7168 x 2048 at 96 13 / - / 11 / 9.4 (8.9). Fewer than 64 blocks
+// of long rows are the library's as before (256 x 4096, which a test has there, 6.4 / - /
+// 12 / 20 (8.9) at 40 rows).
+#define PIECES_ONE_A_CU 256
+static int piece_blocks(int M, int N, int nt) {
+  return ceil_div(M, 32) * ceil_div(N, nt);
+}
 static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
   if (M <= 32 || M > 384 || row_bytes % 128 || N % 4) return 0;
   const int64_t bytes = (int64_t)N * row_bytes;
-  auto blocks = [&](int nt) { return ceil_div(M, 32) * ceil_div(N, nt); };
+  auto blocks = [&](int nt) { return piece_blocks(M, N, nt); };
   if (bytes > 26000000 || (row_bytes > 4096 && blocks(16) < 64)) return 0;
-  if (row_bytes <= 14336 && blocks(16) <= (N <= 2048 ? 384 : 320)) return 16;
+  if (row_bytes <= 14336 && blocks(16) <= (row_bytes > 8192 ? 384 : PIECES_ONE_A_CU))
+    return 16;
+  if (row_bytes <= 12288 && blocks(32) <= PIECES_ONE_A_CU) return 32;
   if (row_bytes <= (N > 2048 ? 12288 : 6144) &&
       blocks(32) <= (bytes > 20000000 ? 340 : 384))
     return 32;
@@ -717,6 +726,9 @@ extern "C" void launch_skinny_gemm(
       else run(skinny_gemm_kernel<F, 16, 16, 4, 4>, 16, 4);
     } else {
       if (nt == 64) run(skinny_gemm_kernel<F, 64, 32, 2, 3>, 32, 2);
+      else if (nt == 32 && M > 32 && batch == 1 &&
+               piece_blocks(M, N, 32) <= PIECES_ONE_A_CU)
+        run(skinny_gemm_kernel<F, 32, 32, 4, 3>, 32, 4);
       else if (nt == 32) run(skinny_gemm_kernel<F, 32, 32, 2, 4>, 32, 2);
       else run(skinny_gemm_kernel<F, 16, 32, 4, 3>, 32, 4);
     }

@@ -176,7 +176,8 @@ def test_linear_fp8_rows(M, N, K):
 
 @pytest.mark.parametrize("M,N,K,kind,own", [(M, *c) for M in (33, 64, 65, 97, 128) for c in (
     (4, 64, "bias", True), (1152, 896, "bias", True), (1284, 4928, "", True),  # 16 rows
-    (2052, 960, "bias", True), (2900, 2112, "", True),                         # 32
+    (2052, 960, "bias", True), (2900, 2112, "", True), (4100, 64, "gated", None),  # 32
+    (2180, 5952, "", True),
     (9680, 64, "gated", None), (7664, 896, "gated", True),                     # 64
     (900, 2176, "fp8", True), (2564, 3968, "fp8", True), (7664, 1024, "fp8gated", None),
     (13004, 1024, "", False), (240, 2112, "", False),
