@@ -849,11 +849,13 @@ __global__ __launch_bounds__(512, 2) void moe_big_kernel(const MoeArgs p) {
 }
 // ---- combine --------------------------------------------------------------------
 // out[t] = sum over its choices, of the features from first on; four a thread. Memory
-// bounds it (5.2 TB/s of y), a round trip with few tokens: eight choices are loaded at
-// once, also those of no expert, whose rows are there and not added. A load and an
-// addition in turn / so, whole calls of 128 experts of 2048 x 768, 8 choices: 24 tokens
-// 144.2 / 142.5 us, 100 195.7 / 194.3, 8,192 896 / 892.
+// bounds it (5.2 TB/s of y), a round trip with few tokens: C choices are loaded at once,
+// also those of no expert, whose rows are there and not added. A load and an addition in
+// turn / so, whole calls of 128 experts of 2048 x 768, 8 choices: 24 tokens 144.2 / 142.5
+// us, 100 195.7 / 194.3, 8,192 896 / 892. C by k: eight for two choices loads three of
+// four twice, 16 experts of 1024 x 512, 575 tokens 26.4 / 27.0, with C two 27.1 / 27.0.
 
+template <int C>
 __global__ __launch_bounds__(256) void moe_combine_kernel(
     float* __restrict__ out, const float* __restrict__ y,
     const int64_t* __restrict__ ids, const int T, const int k, const int E,
@@ -862,14 +864,14 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
   for (int c = (blockIdx.y * 256 + threadIdx.x) * 4; c < cols;
        c += gridDim.y * 1024) {
     f32x4v s = {0.f, 0.f, 0.f, 0.f};
-    for (int j0 = 0; j0 < k; j0 += 8) {
-      f32x4v v[8];
+    for (int j0 = 0; j0 < k; j0 += C) {
+      f32x4v v[C];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
+      for (int j = 0; j < C; ++j)
         v[j] = *reinterpret_cast<const f32x4v*>(
             y + ((size_t)t * k + min(j0 + j, k - 1)) * cols + c);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < C; ++j) {
         const int64_t e = ids[(size_t)t * k + min(j0 + j, k - 1)];
         if (j0 + j < k && e >= 0 && e < E) s += v[j];
       }
@@ -1047,6 +1049,10 @@ extern "C" void launch_moe_combine(float* out, const float* y,
                                    int H, int first, int cols,
                                    hipStream_t stream) {
   dim3 grid(T, T < 256 ? ceil_div(cols, 1024) : 1, 1);
-  moe_combine_kernel<<<grid, 256, 0, stream>>>(out, y, ids, T, k, E, H, first,
-                                               cols);
+  auto run = [&](auto kernel) {
+    kernel<<<grid, 256, 0, stream>>>(out, y, ids, T, k, E, H, first, cols);
+  };
+  if (k <= 2) run(moe_combine_kernel<2>);
+  else if (k <= 4) run(moe_combine_kernel<4>);
+  else run(moe_combine_kernel<8>);
 }
