@@ -852,8 +852,8 @@ __global__ __launch_bounds__(512, 2) void moe_big_kernel(const MoeArgs p) {
 // bounds it (5.2 TB/s of y), a round trip with few tokens: C choices are loaded at once,
 // also those of no expert, whose rows are there and not added. A load and an addition in
 // turn / so, whole calls of 128 experts of 2048 x 768, 8 choices: 24 tokens 144.2 / 142.5
-// us, 100 195.7 / 194.3, 8,192 896 / 892. C by k: eight for two choices loads three of
-// four twice, 16 experts of 1024 x 512, 575 tokens 26.4 / 27.0, with C two 27.1 / 27.0.
+// us, 100 195.7 / 194.3, 8,192 896 / 892. C by k: of eight loads for two choices six are
+// of the last again, 16 experts of 1024 x 512, 575 tokens 26.4 / 27.0, with C two 27.1 / 27.0.
 
 template <int C>
 __global__ __launch_bounds__(256) void moe_combine_kernel(

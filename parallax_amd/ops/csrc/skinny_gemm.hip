@@ -668,13 +668,14 @@ extern "C" bool skinny_pays(int M, int N, int row_bytes) {
 // x 2560 at 65 17 / - / 15 / 15 (12.6), 6144 x 2048 at 64 14 / - / 13 / 13 (11.6); nor wide
 // tiles of long rows: in fp8 7168 x 2048 at 96 13 / - / 11 / 9.4 (8.9). Fewer than 64 blocks
 // of long rows are the library's as before (256 x 4096, which a test has there, 6.4 / - /
-// 12 / 20 (8.9) at 40 rows).
+// 12 / 20 (8.9) at 40 rows). Odd widths and rows apart (linear()'s callers see to that) are
+// torch's, whose product takes part in autograd and its transforms.
 #define PIECES_ONE_A_CU 256
 static int piece_blocks(int M, int N, int nt) {
   return ceil_div(M, 32) * ceil_div(N, nt);
 }
 static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
-  if (M <= 32 || M > 384 || row_bytes % 128 || N % 4) return 0;
+  if (M <= 32 || M > 384 || row_bytes % 128 || N % 8) return 0;
   const int64_t bytes = (int64_t)N * row_bytes;
   auto blocks = [&](int nt) { return piece_blocks(M, N, nt); };
   if (bytes > 26000000 || (row_bytes > 4096 && blocks(16) < 64)) return 0;

@@ -175,26 +175,29 @@ def test_linear_fp8_rows(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,kind,own", [(M, *c) for M in (33, 64, 65, 97, 128) for c in (
-    (4, 64, "bias", True), (1152, 896, "bias", True), (1284, 4928, "", True),  # 16 rows
-    (2052, 960, "bias", True), (2900, 2112, "", True), (4100, 64, "gated", None),  # 32
-    (2180, 5952, "", True),
+    (8, 64, "bias", True), (1152, 896, "bias", True), (1288, 4928, "", True),  # 16 rows
+    (2056, 960, "bias", True), (2904, 2112, "", True), (4104, 64, "gated", None),  # 32
+    (2184, 5952, "", True),
     (9680, 64, "gated", None), (7664, 896, "gated", True),                     # 64
-    (900, 2176, "fp8", True), (2564, 3968, "fp8", True), (7664, 1024, "fp8gated", None),
-    (13004, 1024, "", False), (240, 2112, "", False),
+    (904, 2176, "fp8", True), (2568, 3968, "fp8", True), (7664, 1024, "fp8gated", None),
+    (13008, 1024, "", False), (240, 2112, "", False),
+    (1156, 896, "", False), (1152, 896, "apart", False),  # torch's product as before
 )] + [(M, *c) for M in (129, 300, 384) for c in (
-    (4, 64, "bias", True), (900, 896, "bias", True), (640, 1024, "gated", True),
-    (900, 2176, "fp8", True), (3076, 2048, "", False),
+    (8, 64, "bias", True), (904, 896, "bias", True), (640, 1024, "gated", True),
+    (904, 2176, "fp8", True), (3080, 2048, "", False), (904, 896, "apart", False),
 )] + [(385, 896, 896, "", False)])
 def test_linear_in_pieces_of_32_rows(M, N, K, kind, own):
     """Cut tiles and pieces, against fp32. Infinities stay in their rows and columns.
     own: whether a kernel takes it, whatever M is."""
     g = torch.Generator(device="cuda").manual_seed(M + N)
     fp8, gated = kind.startswith("fp8"), kind.endswith("gated")
-    x, w = _rand(g, M, K + 64).bfloat16()[:, :K], _rand(g, N, K).bfloat16()
+    x, w = _rand(g, M, K).bfloat16(), _rand(g, N, K).bfloat16()
+    if kind == "apart":
+        x = torch.cat([x, x], 1)[:, :K]
     none, one = x.new_empty(0), torch.ones(1, device="cuda")
     b = _rand(g, N).bfloat16() if kind == "bias" else none
     if fp8:
-        x, w = x.contiguous().to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
     run = lambda: ops._require_ext("few_rows").few_rows(
         x, w, b, one if fp8 else none, one if fp8 else none, gated)
     got = run()
