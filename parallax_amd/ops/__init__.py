@@ -567,13 +567,17 @@ def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
     """x . weight^T (+ bias) by the kernels for few rows (with the scales: of fp8
     values; gated: silu of the first half of the columns times the second), None
     where they have none for it."""
+    if x.dim() != 2:
+        return None
+    rows = x.shape[0]  # sizes first: a prompt's layers wait for the host
+    if rows > SKINNY_GEMM_MAX_M and (
+            rows > 3 * SKINNY_GEMM_MAX_M
+            or weight.numel() * weight.element_size() > PIECES_MAX_BYTES):
+        return None
     fp8 = x_scale is not None
     if not (
-        x.dim() == 2
-        and (fp8 or x.dtype == weight.dtype == torch.bfloat16)
-        and (0 < x.shape[0] <= SKINNY_GEMM_MAX_M
-             or (SKINNY_GEMM_MAX_M < x.shape[0] <= 3 * SKINNY_GEMM_MAX_M
-                 and weight.numel() * weight.element_size() <= PIECES_MAX_BYTES))
+        (fp8 or x.dtype == weight.dtype == torch.bfloat16)
+        and rows > 0
         and weight.is_contiguous()
         and x.stride(1) == 1
         and (bias is None or bias.dtype == torch.bfloat16)
