@@ -17,7 +17,7 @@ def _model(H, Hq, Hk, D, F, layers, bias=True, seed=0):
     cfg = ModelConfig(
         architecture="Qwen2ForCausalLM" if bias else "LlamaForCausalLM", vocab_size=64,
         hidden_size=H, num_layers=layers + 1, num_heads=Hq, num_kv_heads=Hk, head_dim=D,
-        intermediate_size=F, max_position_embeddings=8192, attention_bias=bias,
+        intermediate_size=F, max_position_embeddings=10240, attention_bias=bias,
         eos_token_ids=[])
     model = get_model_class(cfg.architecture)(cfg, 0, layers).to(torch.bfloat16).cuda()
     g = torch.Generator(device="cuda").manual_seed(seed)
@@ -32,6 +32,7 @@ def _model(H, Hq, Hk, D, F, layers, bias=True, seed=0):
 
 def _step(cfg, layers, BS, lens, max_len=None, seed=1):
     """A step's input, its metadata on a cache of its own, and the cache."""
+    assert max(lens) <= cfg.max_position_embeddings  # the kernels read the rope table there
     g = torch.Generator(device="cuda").manual_seed(seed)
     counts = [(max(n, 1) + BS - 1) // BS for n in lens]
     ids = torch.randperm(sum(counts), generator=g, device="cuda").tolist()
