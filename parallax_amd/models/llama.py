@@ -292,12 +292,14 @@ def stack_in_one(layers, hidden: torch.Tensor, meta: ForwardMeta,
             hidden.shape[0] > ops.NORM_LINEAR_MAX_M
             or not plain_call(layers[0], LlamaDecoderLayer.forward)):
         return None
-    a0, eps = layers[0].self_attn, layers[0].input_layernorm.eps
+    a0, norm = layers[0].self_attn, layers[0].input_layernorm
     if not (plain_call(a0, LlamaAttention.forward)
-            and plain_call(layers[0].mlp, LlamaMLP.forward)) or not ops.decode_stack_has(
+            and plain_call(layers[0].mlp, LlamaMLP.forward)
+            and plain_call(norm, RMSNorm.forward)) or not ops.decode_stack_has(
             *hidden.shape, a0.num_heads, a0.num_kv_heads, a0.head_dim,
             getattr(layers[0].mlp.down_proj, "in_per_rank", 0), meta.max_seq_len):
         return None
+    eps = norm.eps
     tensors = []
     for layer in layers:
         if not plain_call(layer, LlamaDecoderLayer.forward):

@@ -248,3 +248,32 @@ def test_decode_stack_is_left(monkeypatch):
     assert not run(lambda m: m.layers[1].self_attn.o_proj.quantize_fp8())
     assert not run(lambda m: setattr(m.layers[1].self_attn, "sliding_window", 16))
     assert not run(lambda m: setattr(m.layers[1].post_attention_layernorm, "eps", 1e-3))
+
+
+class _Norm(torch.nn.Module):
+    """A norm of a caller's own: no RMSNorm, no eps."""
+
+    def __init__(self, norm):
+        super().__init__()
+        self.inner = norm
+
+    def forward(self, x, residual=None):
+        return self.inner(x, residual)
+
+
+@pytest.mark.parametrize("layer", [0, 1])
+@pytest.mark.parametrize("name", ["input_layernorm", "post_attention_layernorm"])
+def test_other_norms_run(layer, name):
+    """A step over modules that stand in a norm's place, as the layers themselves take
+    them, gives what it gives over the norms apart."""
+    model, cfg = _model(256, 4, 2, 64, 512, 2)
+    x, meta, _ = _step(cfg, 2, 32, [40, 9])
+    seen = []
+    with torch.inference_mode():
+        hooked = getattr(model.layers[layer], name)
+        handle = hooked.register_forward_hook(lambda *a: seen.append(1))
+        want = model(x.clone(), meta).clone()
+        handle.remove()
+        assert seen
+        setattr(model.layers[layer], name, _Norm(hooked))
+        assert torch.equal(model(x.clone(), meta), want)
