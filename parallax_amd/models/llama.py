@@ -289,7 +289,7 @@ def stack_in_one(layers, hidden: torch.Tensor, meta: ForwardMeta,
     layers that are more than LlamaDecoderLayer, of one width, without windows, sinks,
     norms of heads and quantised weights."""
     if not (meta.appends and meta.max_seq_len and hidden.is_cuda and layers) or (
-            hidden.shape[0] > ops.NORM_LINEAR_MAX_M
+            hidden.dim() != 2 or hidden.shape[0] > ops.NORM_LINEAR_MAX_M
             or not plain_call(layers[0], LlamaDecoderLayer.forward)):
         return None
     a0, norm = layers[0].self_attn, layers[0].input_layernorm

@@ -277,3 +277,15 @@ def test_other_norms_run(layer, name):
         assert seen
         setattr(model.layers[layer], name, _Norm(hooked))
         assert torch.equal(model(x.clone(), meta), want)
+
+
+def test_a_row_of_three_dimensions_runs():
+    """[1, 1, H] goes through the layers, whose results are bf16: 2^-6 of their norm is
+    four roundings of a value a layer."""
+    model, cfg = _model(256, 4, 2, 64, 512, 2)
+    x, meta, _ = _step(cfg, 2, 32, [40])
+    with torch.inference_mode():
+        want = model(x.clone(), meta).float()
+        got = model(x[None].clone(), meta)
+    assert got.shape == (1, 1, 256)
+    assert (got[0].float() - want).norm() <= 2 ** -6 * want.norm()
