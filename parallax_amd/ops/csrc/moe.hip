@@ -24,6 +24,7 @@
 #define MOE_UNIT (256 * MOE_BKB)
 
 typedef float f32x16v __attribute__((ext_vector_type(16)));
+typedef unsigned long long u64;
 
 // ---- routing ------------------------------------------------------------------
 // perm [n], tiles [max_tiles] as (expert, first row, end of the expert's rows,
@@ -849,34 +850,55 @@ __global__ __launch_bounds__(512, 2) void moe_big_kernel(const MoeArgs p) {
 }
 // ---- combine --------------------------------------------------------------------
 // out[t] = sum over its choices, of the features from first on; four a thread. Memory
-// bounds it (5.2 TB/s of y), a round trip with few tokens: C choices are loaded at once,
-// also those of no expert, whose rows are there and not added. A load and an addition in
-// turn / so, whole calls of 128 experts of 2048 x 768, 8 choices: 24 tokens 144.2 / 142.5
-// us, 100 195.7 / 194.3, 8,192 896 / 892. C by k: of eight loads for two choices six are
-// of the last again, 16 experts of 1024 x 512, 575 tokens 26.4 / 27.0, with C two 27.1 / 27.0.
+// bounds it (5.2 TB/s of y), a round trip or two with few tokens: a ballot tells which
+// choices have rows, those of experts of other ranks have none, and up to eight rows are
+// loaded at once, with fewer left four or two. us of the kernel, a load and an addition
+// in turn / all choices loaded, those without rows too / so: 8,192 tokens of 8 choices,
+// 2048 features, all experts here 106.8 / 102.4 / 103.2, one in eight 23.3 / 87.5 / 22.3;
+// 24 tokens 4.8 / 4.2 / 4.2; 8,192 of 2 choices, 1024 features, 15.6 / 15.0 / 15.9 and 8.0
+// / 10.3 / 8.7. The mask from scalar loads of the ids: one in eight 26.7, two choices
+// 15.6 and 8.4.
 
+// adds the rows of the first C choices of the mask and takes them off it
 template <int C>
+DEVINL void add_choices(f32x4v& s, const float* y, int cols, u64& mask) {
+  const int n = __popcll(mask);
+  uint32_t row = 0;
+  f32x4v v[C];
+  asm volatile("; up to %0" ::"n"(C) : "memory");  // no loads shared between the sizes
+#pragma unroll
+  for (int i = 0; i < C; ++i) {  // past the last one that one again
+    row = mask ? __ffsll(mask) - 1 : row;
+    mask &= mask - 1;
+    v[i] = *reinterpret_cast<const f32x4v*>(y + row * (uint32_t)cols);
+  }
+#pragma unroll
+  for (int i = 0; i < C; ++i)
+    if (i < n) s += v[i];
+}
+
 __global__ __launch_bounds__(256) void moe_combine_kernel(
     float* __restrict__ out, const float* __restrict__ y,
     const int64_t* __restrict__ ids, const int T, const int k, const int E,
     const int H, const int first, const int cols) {
-  const int t = blockIdx.x;
-  for (int c = (blockIdx.y * 256 + threadIdx.x) * 4; c < cols;
-       c += gridDim.y * 1024) {
+  const int t = blockIdx.x, lane = threadIdx.x & 63;
+  auto local = [&](int j0) {  // of choices j0 .. j0 + 63, those of experts that are here
+    const int64_t e = j0 + lane < k ? ids[(size_t)t * k + j0 + lane] : -1;
+    return (u64)__ballot(e >= 0 && e < E);
+  };
+  const u64 all = local(0);
+  for (int c0 = blockIdx.y * 1024; c0 < cols; c0 += gridDim.y * 1024) {
+    const int c = c0 + threadIdx.x * 4;
+    const float* row = y + (size_t)t * k * cols + min(c, cols - 4);
     f32x4v s = {0.f, 0.f, 0.f, 0.f};
-    for (int j0 = 0; j0 < k; j0 += C) {
-      f32x4v v[C];
-#pragma unroll
-      for (int j = 0; j < C; ++j)
-        v[j] = *reinterpret_cast<const f32x4v*>(
-            y + ((size_t)t * k + min(j0 + j, k - 1)) * cols + c);
-#pragma unroll
-      for (int j = 0; j < C; ++j) {
-        const int64_t e = ids[(size_t)t * k + min(j0 + j, k - 1)];
-        if (j0 + j < k && e >= 0 && e < E) s += v[j];
+    for (int j0 = 0; j0 < k; j0 += 64, row += (size_t)64 * cols)
+      for (u64 mask = j0 ? local(j0) : all; mask;) {
+        const int n = __popcll(mask);
+        if (n > 4) add_choices<8>(s, row, cols, mask);
+        else if (n > 2) add_choices<4>(s, row, cols, mask);
+        else add_choices<2>(s, row, cols, mask);
       }
-    }
-    *reinterpret_cast<f32x4v*>(out + (size_t)t * H + first + c) = s;
+    if (c < cols) *reinterpret_cast<f32x4v*>(out + (size_t)t * H + first + c) = s;
   }
 }
 
@@ -1049,10 +1071,5 @@ extern "C" void launch_moe_combine(float* out, const float* y,
                                    int H, int first, int cols,
                                    hipStream_t stream) {
   dim3 grid(T, T < 256 ? ceil_div(cols, 1024) : 1, 1);
-  auto run = [&](auto kernel) {
-    kernel<<<grid, 256, 0, stream>>>(out, y, ids, T, k, E, H, first, cols);
-  };
-  if (k <= 2) run(moe_combine_kernel<2>);
-  else if (k <= 4) run(moe_combine_kernel<4>);
-  else run(moe_combine_kernel<8>);
+  moe_combine_kernel<<<grid, 256, 0, stream>>>(out, y, ids, T, k, E, H, first, cols);
 }

@@ -431,10 +431,11 @@ def test_moe_few_infinities_and_graph():
         assert torch.equal(out, eager)
 
 
-@pytest.mark.parametrize("k", [1, 7, 8, 9, 17])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 7, 8, 9, 17, 70])
 def test_moe_combine_leaves_out_rows_nobody_wrote(k):
-    """Choices are added up eight at a time. Those of no expert have rows that nothing
-    writes, here over memory that held NaN; a token of such choices only is zero."""
+    """Choices are added up two, four or eight at a time, and looked at 64 at a time.
+    Those of no expert have rows that nothing writes, here over memory that held NaN; a
+    token of such choices only is zero."""
     g = torch.Generator(device="cuda").manual_seed(k)
     T, E, H, I = 40, 20, 320, 64
     x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
@@ -449,3 +450,25 @@ def test_moe_combine_leaves_out_rows_nobody_wrote(k):
     got = ops.fused_moe_forward(x, gu, dn, ids, w)
     assert not got[3].any() and not got[~((ids >= 0) & (ids < E)).any(1)].any()
     assert ((got - want).norm(dim=1) <= 2 ** -7 * want.norm(dim=1) + 1e-30).all()
+
+
+def test_moe_combine_reads_rows_of_local_experts_alone():
+    """With all experts on other ranks eight choices a token cost no more than what one
+    does but for their ids: 134 MB of zeros, where 1,074 MB of rows would be read."""
+    T, E, H, I = 16384, 4, 2048, 64
+    x = torch.zeros(T, H, dtype=torch.bfloat16, device="cuda")
+    gu = torch.zeros(E, 2 * I, H, dtype=torch.bfloat16, device="cuda")
+    dn = torch.zeros(E, H, I, dtype=torch.bfloat16, device="cuda")
+
+    def fastest(k):
+        ids = torch.full((T, k), E, device="cuda")
+        w = torch.ones(T, k, device="cuda")
+        at = [torch.cuda.Event(enable_timing=True) for _ in range(21)]
+        for e in at:
+            e.record()
+            assert e is at[-1] or ops.fused_moe_forward(x, gu, dn, ids, w).shape == (T, H)
+        torch.cuda.synchronize()
+        return min(a.elapsed_time(b) for a, b in zip(at, at[1:]))
+
+    fastest(1)
+    assert fastest(8) < 2.5 * fastest(1)
