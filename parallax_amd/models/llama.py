@@ -299,6 +299,12 @@ def stack_in_one(layers, hidden: torch.Tensor, meta: ForwardMeta,
             *hidden.shape, a0.num_heads, a0.num_kv_heads, a0.head_dim,
             getattr(layers[0].mlp.down_proj, "in_per_rank", 0), meta.max_seq_len):
         return None
+    # what an eager step can be refused for as a whole, before its layers are looked at
+    k_cache = meta.kv_cache.layer(a0.local_layer_idx)[0]
+    if not hidden.dtype == k_cache.dtype == torch.bfloat16 or (
+            rope_cache.shape[-1] != a0.head_dim
+            or torch.is_grad_enabled() and hidden.requires_grad):
+        return None
     eps = norm.eps
     tensors = []
     for layer in layers:

@@ -289,3 +289,23 @@ def test_a_row_of_three_dimensions_runs():
         got = model(x[None].clone(), meta)
     assert got.shape == (1, 1, 256)
     assert (got[0].float() - want).norm() <= 2 ** -6 * want.norm()
+
+
+def test_a_step_refused_as_a_whole_is_refused_early(monkeypatch):
+    """fp8 caches, rope of part of a head and a gradient to be taken are seen before the
+    layers are: the host pays for none of them."""
+    model, cfg = _model(256, 4, 2, 64, 512, 2)
+    monkeypatch.setattr(ops, "decode_stack", lambda *a: pytest.fail("asked"))
+    x, meta, cache = _step(cfg, 2, 32, [40, 9])
+    with torch.enable_grad():
+        model(x.clone().requires_grad_(), meta)
+    with torch.inference_mode():
+        with monkeypatch.context() as m:
+            m.setattr(model, "rope_cache", model.rope_cache[:, :32].contiguous())
+            model(x.clone(), meta)
+        meta.kv_cache = PagedKVCache(KVCacheSpec(2, 2, 64, 32, torch.float8_e4m3fn),
+                                     len(cache.k_caches[0]), torch.device("cuda"))
+        model(x.clone(), meta)
+        meta.kv_cache = cache
+        with pytest.raises(pytest.fail.Exception):
+            model(x.clone(), meta)
