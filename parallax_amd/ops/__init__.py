@@ -553,10 +553,12 @@ def gelu_and_mul(x: torch.Tensor) -> torch.Tensor:
 
 # -- dense linear (skinny-M fast path) ------------------------------------------
 
-# Rows of x up to which linear() and linear_fp8() try the weight-streaming kernels
-# (there are none above 128); 0 leaves every product to the library.
+# Rows of x up to which linear() and linear_fp8() try the weight-streaming kernels; 0
+# leaves every product to the library. Above 128 there are some for small weights alone,
+# which are tried where the limit is not below that.
 SKINNY_GEMM_MAX_M = int(os.environ.get("PARALLAX_SKINNY_GEMM_MAX_M", "128"))
-PIECES_MAX_BYTES = 26_000_000  # of weights with kernels for up to three times as many rows
+PIECES_MAX_M = 384  # rows, and bytes of a weight, up to which these are
+PIECES_MAX_BYTES = 26_000_000
 NORM_LINEAR_MAX_M = 4  # rows of x up to which norm_linear() has kernels
 LT_GEMM = os.environ.get("PARALLAX_LT_GEMM", "1") != "0"
 _NONE = torch.empty(0, dtype=torch.bfloat16)  # an argument that is not there
@@ -571,7 +573,7 @@ def _few_rows(x, weight, bias=None, x_scale=None, w_scale=None, gated=False):
         return None
     rows = x.shape[0]  # sizes first: a prompt's layers wait for the host
     if rows > SKINNY_GEMM_MAX_M and (
-            rows > 3 * SKINNY_GEMM_MAX_M
+            SKINNY_GEMM_MAX_M < 128 or rows > PIECES_MAX_M
             or weight.numel() * weight.element_size() > PIECES_MAX_BYTES):
         return None
     fp8 = x_scale is not None

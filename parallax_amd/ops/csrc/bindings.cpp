@@ -118,6 +118,7 @@ void launch_skinny_gemm(void*, const void*, const void*, const void*,
 int skinny_shared(int, int, int);
 bool skinny_pays(int, int, int);
 bool skinny_in_pieces(int, int, int, bool);
+void skinny_pieces_limits(int*, int64_t*);
 void launch_skinny_split(void*, float*, int, const void*, const void*, const void*,
                          const float*, const float*, bool, int, int, int, int64_t,
                          int64_t, bool, hipStream_t);
@@ -1323,6 +1324,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm);
   m.def("few_rows", &few_rows);
   m.def("norm_linear", &norm_linear);
+  m.def("skinny_pieces_limits", [] {
+    int rows;
+    int64_t bytes;
+    skinny_pieces_limits(&rows, &bytes);
+    return std::make_tuple(rows, bytes);
+  });
   m.def("decode_stack", &decode_stack);
   m.def("decode_stack_has", &decode_stack_has);
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);

@@ -608,7 +608,7 @@ static int skinny_tile(int M, int64_t N, int row_bytes, bool gated) {
 // 28672 x 4096 at 96 rows - / 47 / 58, 4096 x 14336 - / 31 / 51; short K split, or
 // small weights under many rows, cost more in parts than they gain: 9728 x 896 at 96
 // rows 16 / 12, 576 x 7168 at 40 10.8 / 10.9, at 96 14 / 11. Above 128 rows: the
-// library.
+// library, but for the pieces below.
 extern "C" int skinny_shared(int M, int N, int row_bytes) {
   if (M > 128 || row_bytes % 128 || N % 4) return -1;
   const int splits = skinny_splits(N, row_bytes);
@@ -671,14 +671,16 @@ extern "C" bool skinny_pays(int M, int N, int row_bytes) {
 // 12 / 20 (8.9) at 40 rows). Odd widths and rows apart (linear()'s callers see to that) are
 // torch's, whose product takes part in autograd and its transforms.
 #define PIECES_ONE_A_CU 256
+#define PIECES_MAX_M 384
+#define PIECES_MAX_BYTES 26000000
 static int piece_blocks(int M, int N, int nt) {
   return ceil_div(M, 32) * ceil_div(N, nt);
 }
 static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
-  if (M <= 32 || M > 384 || row_bytes % 128 || N % 8) return 0;
+  if (M <= 32 || M > PIECES_MAX_M || row_bytes % 128 || N % 8) return 0;
   const int64_t bytes = (int64_t)N * row_bytes;
   auto blocks = [&](int nt) { return piece_blocks(M, N, nt); };
-  if (bytes > 26000000 || (row_bytes > 4096 && blocks(16) < 64)) return 0;
+  if (bytes > PIECES_MAX_BYTES || (row_bytes > 4096 && blocks(16) < 64)) return 0;
   if (row_bytes <= 14336 && blocks(16) <= (row_bytes > 8192 ? 384 : PIECES_ONE_A_CU))
     return 16;
   if (row_bytes <= 12288 && blocks(32) <= PIECES_ONE_A_CU) return 32;
@@ -686,6 +688,13 @@ static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
       blocks(32) <= (bytes > 20000000 ? 340 : 384))
     return 32;
   return row_bytes <= (gated ? 2048 : 1920) && blocks(64) <= 512 ? 64 : 0;
+}
+
+// The rows and bytes of W above which there are none: callers that must not wait for the
+// rule ask these first.
+extern "C" void skinny_pieces_limits(int* rows, int64_t* bytes) {
+  *rows = PIECES_MAX_M;
+  *bytes = PIECES_MAX_BYTES;
 }
 
 // K split over workgroups stays: its parts are what launch_skinny_norm adds up
