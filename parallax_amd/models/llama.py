@@ -335,7 +335,7 @@ def stack_in_one(layers, hidden: torch.Tensor, meta: ForwardMeta,
                     norms[1].weight, up[1].weight, down[1].weight,
                     *meta.kv_cache.layer(attn.local_layer_idx)]
     return ops.decode_stack(
-        hidden, None, tensors, eps, a0.num_heads, a0.num_kv_heads, a0.scale,
+        hidden, tensors, eps, a0.num_heads, a0.num_kv_heads, a0.scale,
         meta.positions, rope_cache, meta.slot_mapping, meta.block_tables, meta.seq_lens,
         meta.max_seq_len)
 

@@ -284,10 +284,10 @@ def decode_stack_has(rows: int, hidden: int, num_heads: int, num_kv_heads: int,
 
 
 def decode_stack(
-    x: torch.Tensor, residual: Optional[torch.Tensor], layers: List[torch.Tensor],
-    eps: float, num_heads: int, num_kv_heads: int, scale: float,
-    positions: torch.Tensor, cos_sin: torch.Tensor, slot_mapping: torch.Tensor,
-    block_tables: torch.Tensor, seq_lens: torch.Tensor, max_seq_len: int,
+    x: torch.Tensor, layers: List[torch.Tensor], eps: float, num_heads: int,
+    num_kv_heads: int, scale: float, positions: torch.Tensor, cos_sin: torch.Tensor,
+    slot_mapping: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tensor,
+    max_seq_len: int,
 ) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
     """All layers of a Llama-type stack on a decode step of a few rows, in one launch:
     (what the last layer adds, the residual stream it is added to). layers: norm weight,
@@ -299,9 +299,8 @@ def decode_stack(
             t.requires_grad for t in [x, *layers])):
         return None
     return _require_ext("decode_stack").decode_stack(
-        x, x.new_empty(0) if residual is None else residual, layers, eps, num_heads,
-        num_kv_heads, scale, positions, cos_sin, slot_mapping, block_tables, seq_lens,
-        max_seq_len)
+        x, layers, eps, num_heads, num_kv_heads, scale, positions, cos_sin, slot_mapping,
+        block_tables, seq_lens, max_seq_len)
 
 
 def prefill_attention(

@@ -48,10 +48,10 @@ struct StackSizes {
 };
 bool decode_stack_takes(const StackSizes*);
 int64_t decode_stack_words(const StackSizes*, int (*)[4]);
-void launch_decode_stack(const StackSizes*, const void* const*, int, const void*,
-                         const void*, void*, void*, void*, const int*, const int*,
-                         const int*, const int64_t*, const float*, int, int, float,
-                         float, hipStream_t);
+void launch_decode_stack(const StackSizes*, const void* const*, int, const void*, void*,
+                         void*, void*, const int*, const int*, const int*,
+                         const int64_t*, const float*, int, int, float, float,
+                         hipStream_t);
 int paged_decode_runs(int, int, int, int, int);
 void launch_paged_decode(void*, const void*, void*, void*, const int*, const int*,
                          int, int, int, int, int, int, int64_t, float, int, float,
@@ -514,15 +514,14 @@ bool decode_stack_has(int64_t M, int64_t H, int64_t Hq, int64_t Hk, int64_t D, i
 
 // The layers of a Llama-type stack on a decode step of a few rows, in one launch. layers:
 // nine tensors each (norm, q/k/v weight, its bias or an empty one, output weight, norm,
-// gate and up weight, down weight, K and V cache); res: empty for none. Rows are the last
-// tokens of sequences of their own, as rope_cache_attention_decode takes them. Returns
-// what the last layer adds to the residual stream, and that. None where there is no
-// kernel.
+// gate and up weight, down weight, K and V cache). Rows are the last tokens of sequences
+// of their own, as rope_cache_attention_decode takes them. Returns what the last layer
+// adds to the residual stream, and that. None where there is no kernel.
 std::optional<std::tuple<torch::Tensor, torch::Tensor>> decode_stack(
-    torch::Tensor x, torch::Tensor res, const std::vector<torch::Tensor>& layers,
-    double eps, int64_t Hq, int64_t Hk, double scale, torch::Tensor positions,
-    torch::Tensor cos_sin, torch::Tensor slot_mapping, torch::Tensor block_tables,
-    torch::Tensor seq_lens, int64_t max_seq_len) {
+    torch::Tensor x, const std::vector<torch::Tensor>& layers, double eps, int64_t Hq,
+    int64_t Hk, double scale, torch::Tensor positions, torch::Tensor cos_sin,
+    torch::Tensor slot_mapping, torch::Tensor block_tables, torch::Tensor seq_lens,
+    int64_t max_seq_len) {
   CHECK_GPU(x);
   constexpr size_t T = 9;  // tensors a layer
   auto plain = [&](const torch::Tensor& t, at::ScalarType type) {
@@ -532,8 +531,6 @@ std::optional<std::tuple<torch::Tensor, torch::Tensor>> decode_stack(
   };
   if (layers.empty() || layers.size() % T || x.dim() != 2 ||
       !plain(x, at::kBFloat16) || attention_by_valu())
-    return std::nullopt;
-  if (res.numel() && (!plain(res, at::kBFloat16) || res.sizes() != x.sizes()))
     return std::nullopt;
   for (const auto& t : layers)
     if (!plain(t, at::kBFloat16)) return std::nullopt;
@@ -570,8 +567,7 @@ std::optional<std::tuple<torch::Tensor, torch::Tensor>> decode_stack(
   std::vector<const void*> pointers(layers.size());
   for (size_t i = 0; i < layers.size(); ++i)
     pointers[i] = layers[i].numel() ? layers[i].data_ptr() : nullptr;
-  launch_decode_stack(&sizes, pointers.data(), n, x.data_ptr(),
-                      res.numel() ? res.data_ptr() : nullptr, x_out.data_ptr(),
+  launch_decode_stack(&sizes, pointers.data(), n, x.data_ptr(), x_out.data_ptr(),
                       res_out.data_ptr(), work.data_ptr(), positions.data_ptr<int>(),
                       seq_lens.data_ptr<int>(), block_tables.data_ptr<int>(),
                       slot_mapping.data_ptr<int64_t>(), cos_sin.data_ptr<float>(),

@@ -44,7 +44,9 @@
 #define DS_WAVES 8
 #define DS_UNIT 256        // tokens of a sequence that a workgroup takes at a time
 #define DS_MAX_PARTS 8     // of the sequences together
-#define DS_STAGE 12288     // words of the attention's parts in LDS at a time
+#define DS_MAX_HEADS 1024  // values of all query heads, 64 or 128 each
+// words of the attention's parts in LDS: of a part D + 2 a head
+#define DS_STAGE (DS_MAX_PARTS * (DS_MAX_HEADS + DS_MAX_HEADS / 64 * 2))
 
 struct StackLayer {
   const uint16_t *norm1, *w_qkv, *b_qkv, *w_o, *norm2, *w_gu, *w_d;
@@ -53,7 +55,7 @@ struct StackLayer {
 
 struct StackArgs {
   StackLayer layer[DS_LAYERS];
-  const uint16_t *x, *res;    // [M, H]; res null: none (the first layer of all)
+  const uint16_t* x;          // [M, H]
   uint16_t *x_out, *res_out;  // [M, H] of the last layer
   unsigned long long* words;
   uint32_t* ticket;
@@ -314,16 +316,9 @@ __global__ __launch_bounds__(DS_THREADS, 4) void decode_stack_kernel(const Stack
       for (int n = 0; n < MB; ++n)
         if (n < M) {
           const uint32_t* x = reinterpret_cast<const uint32_t*>(p.x + (size_t)n * H);
-          const uint32_t* r = reinterpret_cast<const uint32_t*>(p.res + (size_t)n * H);
           for (int j = tid; j < pairs; j += DS_THREADS) {
-            uint32_t w = x[j];
-            float a = lo16(w), b = hi16(w);
-            if (p.res != nullptr) {
-              const uint32_t q = r[j];
-              a += lo16(q);
-              b += hi16(q);
-              w = pack(a, b);
-            }
+            const uint32_t w = x[j];
+            const float a = lo16(w), b = hi16(w);
             ss[n] += a * a + b * b;
             in[n * pairs + j] = w;
           }
@@ -613,10 +608,6 @@ __global__ __launch_bounds__(DS_THREADS, 4) void decode_stack_kernel(const Stack
       const int at = pm * (H / 2) + wg * 8 + pr;
       if (initial) {
         old = reinterpret_cast<const uint32_t*>(p.x)[at];
-        if (p.res != nullptr) {
-          const uint32_t r = reinterpret_cast<const uint32_t*>(p.res)[at];
-          old = pack(lo16(old) + lo16(r), hi16(old) + hi16(r));
-        }
       } else {
         uint32_t a[1] = {(uint32_t)(p.at_v5 + at)}, w[1];
         take(words, a, tag - 1, w);
@@ -625,53 +616,46 @@ __global__ __launch_bounds__(DS_THREADS, 4) void decode_stack_kernel(const Stack
     }
     if (wid == 0) until<4>(words + p.at_att + wg * 37 % (p.Hq * D), tag);
     meet();
-    // as many rows at a time as there is room for
     constexpr int W = D + 2;
     uint32_t* const xs = in + DS_STAGE;
-    for (int m0 = 0, m1; m0 < M; m0 = m1) {
-      int begin[MB + 1];
-      begin[0] = 0;
-      m1 = m0;
+    int begin[MB + 1];  // of the rows' parts in LDS
+    begin[0] = 0;
 #pragma unroll
-      for (int i = 0; i < MB; ++i) {
-        const int m = m0 + i;
-        int words = 0;
-        if (m < M) {
-          const int units = (p.seq_lens[m] + DS_UNIT - 1) / DS_UNIT;
-          words = max(1, min(p.parts, units)) * p.Hq * W;
-        }
-        const bool fits = m < M && m1 == m && begin[i] + words <= DS_STAGE;
-        begin[i + 1] = begin[i] + (fits ? words : 0);
-        if (fits) m1 = m + 1;
+    for (int m = 0; m < MB; ++m) {
+      int words = 0;
+      if (m < M) {
+        const int units = (p.seq_lens[m] + DS_UNIT - 1) / DS_UNIT;
+        words = max(1, min(p.parts, units)) * p.Hq * W;
       }
-      collect(begin[MB], in, tag, [&](int i) INL {
-        int row = 0, from = 0;
-#pragma unroll
-        for (int q = 1; q < MB; ++q)
-          if (i >= begin[q] && m0 + q < m1) row = q, from = begin[q];
-        return (uint32_t)(p.at_att + (m0 + row) * p.parts * p.Hq * W + i - from);
-      });
-      meet();
-      for (int j = tid; j < (m1 - m0) * (K / 2); j += DS_THREADS) {
-        const int row = j / (K / 2), k = j % (K / 2) * 2;
-        int from = 0, to = begin[1];
-#pragma unroll
-        for (int q = 1; q < MB; ++q)
-          if (row == q) from = begin[q], to = begin[q + 1];
-        const float* src = reinterpret_cast<const float*>(in) + k / D * W;
-        float mall = -1e30f, l = 0.f, a = 0.f, b = 0.f;
-        for (int o = from; o < to; o += p.Hq * W) mall = fmaxf(mall, src[o + D]);
-        for (int o = from; o < to; o += p.Hq * W) {
-          const float g = __builtin_amdgcn_exp2f(src[o + D] - mall);
-          l += src[o + D + 1] * g;
-          a += src[o + k % D] * g;
-          b += src[o + k % D + 1] * g;
-        }
-        const float inv = l > 0.f ? 1.f / l : 0.f;  // no tokens: zeros
-        xs[(m0 + row) * (K / 2) + k / 2] = pack_bf16(a * inv, b * inv);
-      }
-      meet();
+      begin[m + 1] = begin[m] + words;
     }
+    collect(begin[MB], in, tag, [&](int i) INL {
+      int row = 0, from = 0;
+#pragma unroll
+      for (int q = 1; q < MB; ++q)
+        if (i >= begin[q] && q < M) row = q, from = begin[q];
+      return (uint32_t)(p.at_att + row * p.parts * p.Hq * W + i - from);
+    });
+    meet();
+    for (int j = tid; j < M * (K / 2); j += DS_THREADS) {
+      const int row = j / (K / 2), k = j % (K / 2) * 2;
+      int from = 0, to = begin[1];
+#pragma unroll
+      for (int q = 1; q < MB; ++q)
+        if (row == q) from = begin[q], to = begin[q + 1];
+      const float* src = reinterpret_cast<const float*>(in) + k / D * W;
+      float mall = -1e30f, l = 0.f, a = 0.f, b = 0.f;
+      for (int o = from; o < to; o += p.Hq * W) mall = fmaxf(mall, src[o + D]);
+      for (int o = from; o < to; o += p.Hq * W) {
+        const float g = __builtin_amdgcn_exp2f(src[o + D] - mall);
+        l += src[o + D + 1] * g;
+        a += src[o + k % D] * g;
+        b += src[o + k % D + 1] * g;
+      }
+      const float inv = l > 0.f ? 1.f / l : 0.f;  // no tokens: zeros
+      xs[row * (K / 2) + k / 2] = pack_bf16(a * inv, b * inv);
+    }
+    meet();
     prod.x[0] = *reinterpret_cast<const u32x4v*>(xs + Out::x_row(M) * (K / 2) +
                                                  prod.at(0) / 2);
     prod.run(part, M);
@@ -769,7 +753,7 @@ int stack_lds(const StackSizes& s) {
 extern "C" bool decode_stack_takes(const StackSizes* s) {
   if (s->M < 1 || s->M > 4 || s->Hk < 1 || s->Hq % s->Hk || s->Hq / s->Hk > 15) return false;
   if (s->D != 64 && s->D != 128) return false;
-  if (s->H % 32 || s->H < 32 || s->H > 1024 || s->Hq * s->D > 1024) return false;
+  if (s->H % 32 || s->H < 32 || s->H > 1024 || s->Hq * s->D > DS_MAX_HEADS) return false;
   if (s->F % 32 || s->F < 32 || s->F > 5120) return false;
   return s->max_len >= 1 && (int64_t)s->M * s->max_len <= 16384;
 }
@@ -791,10 +775,9 @@ extern "C" int64_t decode_stack_words(const StackSizes* s, int (*at)[4]) {
 
 extern "C" void launch_decode_stack(
     const StackSizes* s, const void* const* pointers, int layers, const void* x,
-    const void* res, void* x_out, void* res_out, void* work, const int* positions,
-    const int* seq_lens, const int* block_tables, const int64_t* slots,
-    const float* cos_sin, int max_blocks, int bs_shift, float eps, float scale,
-    hipStream_t stream) {
+    void* x_out, void* res_out, void* work, const int* positions, const int* seq_lens,
+    const int* block_tables, const int64_t* slots, const float* cos_sin, int max_blocks,
+    int bs_shift, float eps, float scale, hipStream_t stream) {
   int at[4];
   const int64_t n = decode_stack_words(s, &at);
   const int launches = ceil_div(layers, DS_LAYERS);
@@ -805,7 +788,6 @@ extern "C" void launch_decode_stack(
   const int lds = stack_lds(*s);
   StackArgs p{};
   p.x = (const uint16_t*)x;
-  p.res = (const uint16_t*)res;
   p.x_out = (uint16_t*)x_out;
   p.res_out = (uint16_t*)res_out;
   p.words = words;
