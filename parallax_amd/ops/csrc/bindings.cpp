@@ -117,7 +117,7 @@ void launch_skinny_gemm(void*, const void*, const void*, const void*,
                         int64_t, int, int64_t, int64_t, bool, hipStream_t, bool*);
 int skinny_shared(int, int, int);
 bool skinny_pays(int, int, int);
-bool skinny_in_pieces(int, int, int, bool);
+bool skinny_in_pieces(int, int, int, bool, bool);
 void skinny_pieces_limits(int*, int64_t*);
 void launch_skinny_split(void*, float*, int, const void*, const void*, const void*,
                          const float*, const float*, bool, int, int, int, int64_t,
@@ -1010,7 +1010,7 @@ static bool skinny_run(torch::Tensor& c, torch::Tensor x, torch::Tensor w,
   const float* ws = fp8 ? w_scale.data_ptr<float>() : nullptr;
   // gated: halves as silu_and_mul takes them, offsets of 32 bits from row 0 on
   if (gated && (N % 16 || (int64_t)N * row_bytes > UINT32_MAX)) return false;
-  const int splits = x.is_contiguous() && skinny_in_pieces(M, N, row_bytes, gated)
+  const int splits = x.is_contiguous() && skinny_in_pieces(M, N, row_bytes, gated, b != nullptr)
                          ? 0 : skinny_shared(M, N, row_bytes);
   if (splits < 0) return false;
   if (!c.defined())
@@ -1094,7 +1094,7 @@ std::optional<torch::Tensor> few_rows(torch::Tensor x, torch::Tensor w,
   const int64_t row_bytes = x.size(1) * x.element_size();
   if (!gated && !skinny_pays(x.size(0), w.size(0), row_bytes) &&
       !(x.is_contiguous() &&
-        skinny_in_pieces(x.size(0), w.size(0), row_bytes, false)))
+        skinny_in_pieces(x.size(0), w.size(0), row_bytes, false, bias.numel() > 0)))
     return std::nullopt;
   if (!skinny_run(c, x, w, bias, x_scale, w_scale, gated)) return std::nullopt;
   return c;

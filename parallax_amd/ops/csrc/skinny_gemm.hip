@@ -652,31 +652,40 @@ extern "C" bool skinny_pays(int M, int N, int row_bytes) {
 // ones by g, bias by b):
 //   64 rows: 896 x 896 4.1 / 5.2 / 5.6 / 8.1 (6.0), 1152 x 896 b 4.4 / 5.4 / 6.1 / 9.0
 //   (9.2), 2048 x 1536 b 5.2 / 6.3 / 7.6 / 11 (11), 896 x 4864 10.5 / 14 / 14 / 24 (13.3),
-//   3072 x 2048 9.5 / 8.5 / 8.7 / 13 (9.8), 4096 x 2560 11.2 / 10.0 / 10.6 / 15 (11.4),
-//   9728 x 896 g 13 / 14 / 12.5 / 10.1 (14.6); in fp8 896 x 896 3.6 / - / 4.7 / 6.1 (6.1),
-//   2048 x 8192 7.1 / 8.8 / 10.9 / 16 (9.4), 4096 x 7168 13 / 9.2 / 11.1 / 16 (10.1)
+//   2048 x 2048 6.0 / 7.2 / 8.1 / 13 (16), and with a second round of blocks 2304 x 2048
+//   8.1 / 8.3 / 8.4 / 13 (12); 3072 x 2048 9.5 / 8.5 / 8.7 / 13 (9.8), 9728 x 896 g 13 / 14 /
+//   12.5 / 10.1 (14.6); in fp8 896 x 896 3.6 / - / 4.7 / 6.1 (6.1), 2048 x 8192 7.1 / 8.8 /
+//   10.9 / 16 (9.4), 4096 x 7168 13 / 9.2 / 11.1 / 16 (10.1)
 //   128 rows: 896 x 896 4.2 / 5.2 / 5.7 / 8.1 (6.1), 1152 x 896 b 5.6 / 5.6 / 6.1 / 9.0
-//   (9.1), 1536 x 1536 6.5 / 6.0 / 7.0 / 11 (7.1), 2048 x 2048 8.4 / 7.0 / 8.1 / 13 (8.2),
-//   896 x 4864 10.2 / 14 / 14 / 24 (13 to 21), 3072 x 3072 16 / 16 / 12.1 / 17 (14), 6144 x
+//   (9.1), 2048 x 2048 8.6 / 7.3 / 8.2 / 13 (10.9), 2304 x 2048 9.6 / 10.5 / 9.0 / 13 (12),
+//   896 x 4864 10.2 / 14 / 14 / 24 (13 to 21), 3072 x 3072 15 / 16 / 12.2 / 17 (16), 6144 x
 //   1024 g 15 / 14 / 13 / 10.6 (12.5 to 15); in fp8 2048 x 8192 12 / 9.0 / 11 / 16 (10.5)
 //   192 and 384 rows, the last: 896 x 896 5.5 / 5.3 / 5.6 / 8.1 (6.5) and 7.4 / 8.2 / 6.5 /
 //   8.2 (6.6 to 8.3), 1152 x 896 b 5.9 / 5.5 / 6.1 / 9.0 (9.6) and 9.2 / 8.7 / 7.0 / 9.1
-//   (12), 1024 x 2048 7.3 / 6.4 / 8.1 / 13 (7.4) and 10.2 / 10.4 / 8.8 / 13 (9.1); 512:
-//   1536 x 1536 14.4 / - / 13.6 / 12.2 (9.2)
-// Not where blocks wait for a second round or the weight's stream counts for more: 9728 x
-// 896 g at 128 rows 20 / 20 / 17 / 17 (14.7), 5120 x 3072 at 96 21 / - / 18 / 18 (15), 5120
-// x 2560 at 65 17 / - / 15 / 15 (12.6), 6144 x 2048 at 64 14 / - / 13 / 13 (11.6); nor wide
-// tiles of long rows: in fp8 7168 x 2048 at 96 13 / - / 11 / 9.4 (8.9). Fewer than 64 blocks
-// of long rows are the library's as before (256 x 4096, which a test has there, 6.4 / - /
-// 12 / 20 (8.9) at 40 rows). Odd widths and rows apart (linear()'s callers see to that) are
-// torch's, whose product takes part in autograd and its transforms.
+//   (12); 512: 1536 x 1536 14.4 / - / 13.6 / 12.2 (9.2)
+// The lines come from 1,900 sizes drawn over 33 to 384 rows, N of 256 to 16384, rows of 512
+// bytes to 16 KB, weights to 26 MB. Times as fast as the library there, in the mean and
+// without the outer quarters: 16 rows 1.57 (1.36 .. 1.86), in fp8 1.82, with a bias or
+// gated 1.73 to 2.00; 32 by four waves 1.31 (1.16 .. 1.44), fp8 1.44, with a bias or gated
+// 1.5 to 1.7; 32 by two waves with a bias or gated, a launch less, 1.34, by themselves 1.31
+// with rows of 3 KB and more, 1.15 with shorter ones, but for more than 320 blocks of up to
+// 128 rows, whose tall W the library likes, 0.80 to 1.3; 64 with a bias or gated 1.17 (of
+// more than 128 rows above 320 blocks 0.93 to 1.1), by themselves 0.85 (0.78 .. 0.94), in
+// fp8 0.90. 16 rows go on to 384 blocks where rows of more than 8 KB leave 32 their long
+// chain: 2048 x 5120 at 96 rows 14.6 / 14.4 (15.0), 2176 x 5120 16.9 / 14.8. Wide tiles have
+// no time for long rows: in fp8 7168 x 2048 at 96 13 / - / 11 / 9.4 (8.9). Fewer than 64
+// blocks of long rows are the library's (256 x 4096 at 40 rows 6.4 / 8.2 / 12 / 20, K split
+// 8.2, library 8.9 to 11.6: a line drawn before there were pieces, and on the safe side).
+// Odd widths and rows apart (linear()'s callers see to that) are torch's, whose product
+// takes part in autograd and its transforms.
 #define PIECES_ONE_A_CU 256
 #define PIECES_MAX_M 384
 #define PIECES_MAX_BYTES 26000000
 static int piece_blocks(int M, int N, int nt) {
   return ceil_div(M, 32) * ceil_div(N, nt);
 }
-static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
+// joined: gated, or with a bias: the library's product would be followed by a launch
+static int skinny_pieces(int M, int N, int row_bytes, bool gated, bool joined) {
   if (M <= 32 || M > PIECES_MAX_M || row_bytes % 128 || N % 8) return 0;
   const int64_t bytes = (int64_t)N * row_bytes;
   auto blocks = [&](int nt) { return piece_blocks(M, N, nt); };
@@ -684,10 +693,12 @@ static int skinny_pieces(int M, int N, int row_bytes, bool gated) {
   if (row_bytes <= 14336 && blocks(16) <= (row_bytes > 8192 ? 384 : PIECES_ONE_A_CU))
     return 16;
   if (row_bytes <= 12288 && blocks(32) <= PIECES_ONE_A_CU) return 32;
-  if (row_bytes <= (N > 2048 ? 12288 : 6144) &&
-      blocks(32) <= (bytes > 20000000 ? 340 : 384))
-    return 32;
-  return row_bytes <= (gated ? 2048 : 1920) && blocks(64) <= 512 ? 64 : 0;
+  const int most = !joined && row_bytes < 3072 && M <= 128 ? 320
+                   : bytes > 20000000 ? 340 : 384;
+  if (row_bytes <= (N > 2048 ? 12288 : 6144) && blocks(32) <= most) return 32;
+  return joined && row_bytes <= (gated ? 2048 : 1920) &&
+                 blocks(64) <= (M > 128 ? 320 : 512)
+             ? 64 : 0;
 }
 
 // The rows and bytes of W above which there are none: callers that must not wait for the
@@ -698,8 +709,8 @@ extern "C" void skinny_pieces_limits(int* rows, int64_t* bytes) {
 }
 
 // K split over workgroups stays: its parts are what launch_skinny_norm adds up
-extern "C" bool skinny_in_pieces(int M, int N, int row_bytes, bool gated) {
-  return skinny_pieces(M, N, row_bytes, gated) > 0 &&
+extern "C" bool skinny_in_pieces(int M, int N, int row_bytes, bool gated, bool bias) {
+  return skinny_pieces(M, N, row_bytes, gated, gated || bias) > 0 &&
          (skinny_shared(M, N, row_bytes) <= 1 ||
           (!gated && !skinny_pays(M, N, row_bytes)));
 }
@@ -713,7 +724,8 @@ extern "C" void launch_skinny_gemm(
     int64_t x_batch, int64_t c_batch, bool gated, hipStream_t stream,
     bool* launched) {
   *launched = false;
-  int nt = batch == 1 ? skinny_pieces(M, N, row_bytes, gated) : 0;
+  int nt = batch == 1 ? skinny_pieces(M, N, row_bytes, gated, gated || bias != nullptr)
+                      : 0;
   if (nt == 0) nt = skinny_tile(min(M, 32), (int64_t)N * batch, row_bytes, gated);
   if (nt == 0 || row_bytes % 128 || N % 4) return;
   *launched = true;

@@ -223,6 +223,45 @@ def test_linear_in_pieces_of_32_rows(M, N, K, kind, own):
     assert torch.equal(again[:-1, :-1], got[:-1, :-1])
 
 
+@pytest.mark.parametrize("M,N,K,kind,own", [
+    (128, 5056, 640, "", False), (128, 5056, 640, "bias", True),      # 64 rows a tile
+    (40, 9344, 512, "", False), (40, 9344, 512, "gated", True),
+    (192, 5184, 768, "", False), (256, 2240, 896, "", False),
+    (96, 7296, 512, "fp8", False), (80, 8640, 1792, "fp8", False),
+    (160, 4096, 960, "gated", True), (161, 4096, 960, "gated", False),
+    (97, 2880, 2560, "fp8", False), (97, 2560, 2560, "fp8", True),    # 32
+    (128, 2584, 1472, "", False), (128, 2560, 1472, "", True),
+    (128, 2584, 1472, "bias", True), (129, 2432, 1472, "", True), (128, 3072, 1536, "", True), (128, 3080, 1536, "", False),
+])
+def test_pieces_leave_the_library_what_it_does_faster(M, N, K, kind, own):
+    """Wide tiles that save no launch, and short rows in more blocks than the chip takes at
+    once, are the library's; both sides of these lines agree with fp32."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    fp8, gated = kind == "fp8", kind == "gated"
+    x, w = _rand(g, M, K).bfloat16(), _rand(g, N, K).bfloat16()
+    none, one = x.new_empty(0), torch.ones(1, device="cuda")
+    b = _rand(g, N).bfloat16() if kind == "bias" else None
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+    got = ops._require_ext("few_rows").few_rows(
+        x, w, none if b is None else b, one if fp8 else none, one if fp8 else none, gated)
+    assert (got is not None) == own
+    y = (ops.linear_fp8_quantized(x, one, w, one) if fp8 else
+         ops.linear_silu_and_mul(x, w) if gated else ops.linear(x, w, b)).float()
+    want = x.float() @ w.float().t()
+    if b is not None:
+        want += b.float()
+    # the library's bias comes behind a rounding of its own
+    atol = K * K * 2 ** -24 + (0 if b is None else 2 ** -8 * (want - b.float()).abs())
+    if gated:   # both products rounded to bf16, |silu'| < 1.1, the result rounded
+        a, u = want.bfloat16().float().chunk(2, dim=1)
+        s = torch.nn.functional.silu(a)
+        want = s * u
+        atol = (atol + 2 ** -7 * a.abs()) * 1.1 * u.abs() + (
+            atol + 2 ** -7 * u.abs()) * s.abs() + 1e-6
+    assert ((y - want).abs() <= atol + 2 ** -7 * want.abs()).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("n", [1, 7, 2048, 2057, 700001])
 def test_quantize_fp8_tensor(dtype, n):
