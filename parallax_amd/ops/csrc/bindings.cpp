@@ -1326,6 +1326,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     skinny_pieces_limits(&rows, &bytes);
     return std::make_tuple(rows, bytes);
   });
+  m.def("moe_few_takes", &moe_few_takes);
   m.def("decode_stack", &decode_stack);
   m.def("decode_stack_has", &decode_stack_has);
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);

@@ -1,5 +1,5 @@
 // Routed experts of at most 32 choices, in two launches: the decode step of one or a few
-// requests.
+// requests (moe_few_takes has the sizes).
 //
 //   moe_few_gate   h[choice] = act(x[token] . W_gu[e]^T), 16 features of one expert a
 //                  workgroup, whose waves share K
@@ -19,6 +19,7 @@
 // / 22.5, 36.4 / 36.7, 65.4 / 60.9, in fp8 29.7 / 22.8, 32.1 / 30.8, 43.3 / 44.1; 16 of
 // 1024 x 512, 2 a token, 20.5 / 12.7 of 1 token, 20.2 / 14.5 of 8, 20.3 / 17.6 of 16; fp8,
 // 256 of 7168 x 2048, 8 a token, 81.4 / 79.2, 137 / 133, 236 / 236.
+#include <cmath>
 #include <type_traits>
 
 #include "moe_common.h"
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(FEW_GATE_WAVES * 64, 2) void moe_few_gate_kernel(
   }
 }
 
-// Workgroup: eight features, all experts. A unit is up to eight choices of one expert;
+// Workgroup: NT features, all experts. A unit is up to eight choices of one expert;
 // the stages of all units form one list, of which every wave takes an equal run. A
 // wave's sums go to its own table of tokens where a unit ends.
 template <bool FP8, int NT, int STAGES>
@@ -364,11 +365,32 @@ __global__ __launch_bounds__(512, 2) void moe_few_down_kernel(const FewArgs p) {
   }
 }
 
-// Up to 32 choices, in fp8, whose weights are half as much, 16 (see above).
+// Features of a workgroup of the second launch. Eight give the chip's 256 workgroups where
+// H is 2048, and a workgroup's start is not paid twice: 7168 with 8 / 16 features 91 / 79 us,
+// 2048 (32 choices) 48.6 / 52.1.
+static int few_features(int H) { return H <= 2048 ? 8 : 16; }
+
+// Up to 32 choices, in fp8, whose weights are half as much, 16 (see above; with room for
+// 64, 40 / 48 / 64 choices took, general / these: 128 experts of 2048 x 768 76.1 / 77.2,
+// 95.3 / 93.6, 107.8 / 111.5; fp8 24 / 32: 43.6 / 43.2, 45.0 / 50.1).
+//
+// Of these the ones where two launches less, some 9 us, are worth more than what the
+// small tiles cost: 0.3 to 0.4 us for each expert that is met, the choices being alike,
+// and the time in which only a part of the chip reads the second launch's weights: where H
+// gives few workgroups, or a few beyond a round. General / these: 32 of 128 experts of 256
+// x 768 23.2 / 37.6 (32 workgroups), of 512 x 128 16.6 / 21.8; 24 of 64 of 4480 x 1280 147 /
+// 160 (280 workgroups); 30 of 64 of 768 x 1024 32.4 / 44.4. Over 510 drawn sizes the line
+// below leaves eight slower by 4 to 12% of 70 that were, by up to 48%, and keeps 1.35 times
+// the speed in the mean of those it takes.
 extern "C" bool moe_few_takes(int n, int E, int H, int I, bool fp8) {
   const int size = fp8 ? 1 : 2;
-  return n >= 1 && n <= (fp8 ? FEW_N / 2 : FEW_N) && H * size % FEW_SPAN == 0 &&
-         I * size % FEW_SPAN == 0 && 2ll * I * H * size < 1ll << 32;
+  if (n < 1 || n > (fp8 ? FEW_N / 2 : FEW_N) || E < 1 || H * size % FEW_SPAN ||
+      I * size % FEW_SPAN || 2ll * I * H * size >= 1ll << 32)
+    return false;
+  const double met = E * (1. - std::pow(1. - 1. / E, n));
+  const int nt = few_features(H), rounds = ceil_div(ceil_div(H, nt), 256);
+  const double idle = (rounds * nt - H / 256.) * I * size * met;  // bytes a CU
+  return met + idle / 5000. <= 28.5;
 }
 
 extern "C" void launch_moe_few_gate(void* h, const void* x, const float* x_scale,
@@ -393,11 +415,8 @@ extern "C" void launch_moe_few_down(float* out, const void* h, const float* h_sc
                                     hipStream_t stream) {
   const FewArgs p{(const uint8_t*)w, w_scale, (const uint8_t*)h, h_scale, ids, choice_w,
                   nullptr, out, n, topk, E, H, fp8 ? I : 2 * I, in_w, 0, 0.f};
-  // Eight features give the chip's 256 workgroups where H is 2048, and a workgroup's
-  // start is not paid twice: 7168 with 8 / 16 features 91 / 79 us, 2048 (32 choices) 48.6
-  // / 52.1.
   auto run = [&](auto kernel, int nt) { kernel<<<ceil_div(H, nt), 512, 0, stream>>>(p); };
-  if (H <= 2048) {
+  if (few_features(H) == 8) {
     if (fp8) run(moe_few_down_kernel<true, 8, 6>, 8);
     else run(moe_few_down_kernel<false, 8, 6>, 8);
   } else {

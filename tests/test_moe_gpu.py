@@ -360,7 +360,9 @@ def test_moe_many_experts(E, T):
     (1, 3, 1, 64, 64, False),         # one stage along K, three waves without any
     (32, 3, 1, 192, 128, False),      # experts of several times eight rows
     (4, 6, 8, 320, 448, False),       # a token that chooses an expert twice
-    (8, 40, 4, 2112, 192, False),     # 16 features a workgroup
+    (8, 40, 4, 2112, 192, False),     # 16 features a workgroup, few of them
+    (5, 20, 4, 4032, 192, False),     # and as many as the chip takes
+    (4, 128, 8, 2048, 128, False),    # most experts met once
     (2, 9, 8, 2048, 768, False),
     (1, 2, 1, 128, 128, True),
     (16, 3, 1, 384, 256, True),
@@ -397,6 +399,22 @@ def test_moe_few(T, E, k, H, I, fp8):
         err = (got - want).norm(dim=1)
         assert (err <= (2 ** -3 if fp8 else 2 ** -7) * want.norm(dim=1) + 1e-30).all()
         assert (got - want).norm() < (2e-2 if fp8 else 2 ** -8) * want.norm()
+
+
+@pytest.mark.parametrize("n,E,H,I,fp8,takes", [
+    (32, 128, 2048, 768, False, True),    # an expert a choice, a workgroup a CU
+    (32, 32, 2048, 1024, False, True), (16, 16, 1024, 512, False, True),
+    (8, 256, 7168, 2048, True, True), (16, 256, 7168, 2048, True, False),
+    (32, 128, 256, 768, False, False),    # 32 workgroups for all of the second launch
+    (32, 3, 256, 768, False, True),       # of three experts
+    (24, 64, 4480, 1280, False, False),   # 24 workgroups beyond a round
+    (24, 64, 4096, 1280, False, True),
+    (33, 3, 2048, 768, False, False), (17, 3, 2048, 768, True, False),
+    (8, 8, 2048, 160, True, False), (8, 8, 96, 128, False, False),  # K in no whole stages
+    (1, 1, 64, 64, False, True),
+])
+def test_moe_few_is_taken_where_it_is_faster(n, E, H, I, fp8, takes):
+    assert ops._require_ext("moe_few_takes").moe_few_takes(n, E, H, I, fp8) == takes
 
 
 def test_moe_few_infinities_and_graph():
