@@ -238,6 +238,16 @@ def test_decode_stack_in_a_graph():
         assert all(torch.equal(a, b) for a, b in zip(kv, cache.k_caches + cache.v_caches))
 
 
+@pytest.mark.parametrize("M,D,last", [
+    (1, 64, 16384), (2, 64, 8192), (3, 64, 4096), (4, 64, 4096),
+    (1, 128, 8192), (2, 128, 4096), (3, 128, 2048), (4, 128, 2048),
+])
+def test_contexts_up_to_what_a_workgroup_takes_in_turn(M, D, last):
+    """Eight units of 256 tokens a part of 64-wide heads, four of 128-wide ones."""
+    for n, has in ((1, True), (last, True), (last + 1, False)):
+        assert ops.decode_stack_has(M, 896, 512 // D, 2, D, 4864, n) == has
+
+
 def test_decode_stack_is_left(monkeypatch):
     """What is more than plain layers, or beyond the kernel's sizes, goes the other way."""
     took = []
