@@ -374,14 +374,14 @@ static int few_features(int H) { return H <= 2048 ? 8 : 16; }
 // 64, 40 / 48 / 64 choices took, general / these: 128 experts of 2048 x 768 76.1 / 77.2,
 // 95.3 / 93.6, 107.8 / 111.5; fp8 24 / 32: 43.6 / 43.2, 45.0 / 50.1).
 //
-// Of these the ones where two launches less, some 9 us, are worth more than what the
-// small tiles cost: 0.3 to 0.4 us for each expert that is met, the choices being alike,
-// and the time in which only a part of the chip reads the second launch's weights: where H
-// gives few workgroups, or a few beyond a round. General / these: 32 of 128 experts of 256
-// x 768 23.2 / 37.6 (32 workgroups), of 512 x 128 16.6 / 21.8; 24 of 64 of 4480 x 1280 147 /
-// 160 (280 workgroups); 30 of 64 of 768 x 1024 32.4 / 44.4. Over 510 drawn sizes the line
-// below leaves eight slower by 4 to 12% of 70 that were, by up to 48%, and keeps 1.35 times
-// the speed in the mean of those it takes.
+// Of these up to eight, and beyond the ones where two launches less, some 9 us, are worth
+// more than what the small tiles cost: 0.3 to 0.4 us for each expert that is met, the
+// choices being alike, and the time in which only a part of the chip reads the second
+// launch's weights: where H gives few workgroups, or a few beyond a round. General / these:
+// 32 of 128 experts of 256 x 768 23.2 / 37.6 (32 workgroups), of 512 x 128 16.6 / 21.8; 24
+// of 64 of 4480 x 1280 147 / 160 (280 workgroups); 30 of 64 of 768 x 1024 32.4 / 44.4. Of
+// 810 drawn sizes 130 were slower here, by up to 48%; of the 550 on this side of the line
+// 14 are, by 3 to 12%, and they are 1.34 times as fast in the mean.
 extern "C" bool moe_few_takes(int n, int E, int H, int I, bool fp8) {
   const int size = fp8 ? 1 : 2;
   if (n < 1 || n > (fp8 ? FEW_N / 2 : FEW_N) || E < 1 || H * size % FEW_SPAN ||
@@ -390,7 +390,7 @@ extern "C" bool moe_few_takes(int n, int E, int H, int I, bool fp8) {
   const double met = E * (1. - std::pow(1. - 1. / E, n));
   const int nt = few_features(H), rounds = ceil_div(ceil_div(H, nt), 256);
   const double idle = (rounds * nt - H / 256.) * I * size * met;  // bytes a CU
-  return met + idle / 5000. <= 28.5;
+  return n <= 8 || met + idle / 5000. <= 28.5;
 }
 
 extern "C" void launch_moe_few_gate(void* h, const void* x, const float* x_scale,

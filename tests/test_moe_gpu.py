@@ -409,6 +409,7 @@ def test_moe_few(T, E, k, H, I, fp8):
     (32, 3, 256, 768, False, True),       # of three experts
     (24, 64, 4480, 1280, False, False),   # 24 workgroups beyond a round
     (24, 64, 4096, 1280, False, True),
+    (8, 128, 256, 3072, False, True), (9, 128, 256, 3072, False, False),  # but up to eight
     (33, 3, 2048, 768, False, False), (17, 3, 2048, 768, True, False),
     (8, 8, 2048, 160, True, False), (8, 8, 96, 128, False, False),  # K in no whole stages
     (1, 1, 64, 64, False, True),
