@@ -18,7 +18,7 @@
 // fp8 30.3 / 21.8, 30.1 / 22.6, 30.4 / 27.5, 35.1 / 35.4; 128 of 2048 x 768, 8 a token, 26.7
 // / 22.5, 36.4 / 36.7, 65.4 / 60.9, in fp8 29.7 / 22.8, 32.1 / 30.8, 43.3 / 44.1; 16 of
 // 1024 x 512, 2 a token, 20.5 / 12.7 of 1 token, 20.2 / 14.5 of 8, 20.3 / 17.6 of 16; fp8,
-// 256 of 7168 x 2048, 8 a token, 81.4 / 79.2, 137 / 133, 236 / 236.
+// 256 of 7168 x 2048, 8 a token, 82 / 81, of 2 tokens 140 / 143.
 #include <cmath>
 #include <type_traits>
 

@@ -21,24 +21,25 @@
 // A turn takes the scores of one tile and the values of the tile before, whose
 // weights depend on nothing of this turn. For 128-wide heads the two are interleaved
 // by hand, matrix instruction by matrix instruction, where no mask cuts the tile: two
-// waves a SIMD (240 registers) keep the matrix cores busy for 52% of the cycles
+// waves a SIMD (240 registers) keep the matrix cores busy for 53% of the cycles
 // instead of 40. For 64-wide heads, where softmax outweighs the products, a second
 // set of scores costs the third wave a SIMD, and the turn goes through the two one
 // after the other (interleaved 255 us for 4,500 rows of 64 heads over 8, apart 254;
 // 3,000 rows with a window of 128 35.5 and 30).
 //
-// What bounds it: power. Per tile and wave 1024 matrix-core cycles (D = 128), about
-// as many VALU cycles, half as many of the LDS for four waves; with operands of
-// zeros the same instructions run at 1,410 TFLOP/s, with normal values the clock
-// falls to 1.65 GHz. The accumulators are rescaled only when an item's maximum moved,
-// the mask is applied only in tiles that the diagonal, the window or the end of the
-// sequence cuts.
+// What bounds it: the card's power, and within a cycle how little the units overlap. The
+// case below takes 5.53 M cycles of a CU, of which the matrix cores are busy for 53% and
+// VALU instructions, four cycles each, would take 37. With operands of zeros the same
+// products take 5.17 M (the accumulators are not rescaled), but at 2.38 GHz instead of
+// 1.55 to 1.84: 2.17 ms for 3.0 to 3.5 (profiles/rocprof/prefill_attention_power.txt). The
+// accumulators are rescaled only when an item's maximum moved, the mask is applied only in
+// tiles that the diagonal, the window or the end of the sequence cuts.
 //
 // Measured (MI355X, bf16, 32 heads over 8 of 128, 8192 rows in two portions on
-// prefixes of up to 20,000): 3.00 ms among other work and 2.62 again and again =
-// 890 and 1,015 TFLOP/s of what the mask leaves; scores and values of one tile in turn,
-// with a branch and a wait at every operand of V, 3.47 and 2.99 ms. 5,700 rows on an fp8 cache 425 to 338 us (conversions by the hardware's
-// rounding), 64-wide heads 340 to 274; 8,192 rows without a prefix 228 to 213.
+// prefixes of up to 20,000): 3.00 ms = 890 TFLOP/s of what the mask leaves; scores and
+// values of one tile in turn, with a branch and a wait at every operand of V, 3.47. 5,700
+// rows on an fp8 cache 425 to 338 us (conversions by the hardware's rounding), 64-wide
+// heads 340 to 274; 8,192 rows without a prefix 228 to 213.
 
 #include <type_traits>
 

@@ -360,8 +360,8 @@ def test_moe_many_experts(E, T):
     (1, 3, 1, 64, 64, False),         # one stage along K, three waves without any
     (32, 3, 1, 192, 128, False),      # experts of several times eight rows
     (4, 6, 8, 320, 448, False),       # a token that chooses an expert twice
-    (8, 40, 4, 2112, 192, False),     # 16 features a workgroup, few of them
-    (5, 20, 4, 4032, 192, False),     # and as many as the chip takes
+    (8, 40, 4, 2112, 192, False),     # a size that the kernels for more choices take
+    (5, 20, 4, 4032, 192, False),     # 16 features a workgroup
     (4, 128, 8, 2048, 128, False),    # most experts met once
     (2, 9, 8, 2048, 768, False),
     (1, 2, 1, 128, 128, True),
