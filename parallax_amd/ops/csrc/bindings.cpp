@@ -64,7 +64,7 @@ void launch_mla_paged_attention_decode(void*, const void*, const void*,
                                        const void*, const int*, const int*,
                                        int, int, int, int, int, int, float,
                                        int, float*, float*, const int*, int,
-                                       bool, float, hipStream_t, bool*);
+                                       bool, hipStream_t, bool*);
 int mla_decode_runs(int, int, int);
 void launch_mla_prefill_run(void*, float*, const void*, const void*, void*, void*,
                             void*, void*, const void*, const void*, const void*,
@@ -676,7 +676,8 @@ void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,
   if (runs > 0) {
     auto opts = q_latent.options().dtype(at::kFloat);
     tmp_acc = torch::empty({(int64_t)runs + B, H, R}, opts);
-    tmp_ml = torch::empty({(int64_t)runs + B, H, 2}, opts);
+    // of a part each head's maximum and sum; of a sequence its first and last run
+    tmp_ml = torch::empty({((int64_t)runs + B) * H * 2 + 2 * B}, opts);
     acc_ptr = tmp_acc.data_ptr<float>();
     ml_ptr = tmp_ml.data_ptr<float>();
   }
@@ -687,7 +688,7 @@ void mla_paged_attention_decode(torch::Tensor out, torch::Tensor q_latent,
       out.data_ptr(), q_latent.data_ptr(), q_pe.data_ptr(), cache.data_ptr(),
       block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), B, H, R, DR, BS,
       max_blocks, (float)scale, runs, acc_ptr, ml_ptr, idx_ptr, max_topk,
-      is_fp8(cache), 1.0f, cur_stream(), &launched);
+      is_fp8(cache), cur_stream(), &launched);
   TORCH_CHECK(launched, "no MLA kernel for R=", R, " DR=", DR, " BS=", BS);
 }
 

@@ -2,33 +2,29 @@
 //
 //   S^T[64 tok x 16 heads] = C . Q^T     C = [latent | rope] rows, 576 values
 //   O^T[512 x 16 heads]   += C_v^T . P   C_v = the latent part of the same rows
-// All query heads share ONE cache row a token; a workgroup takes 64 heads (16 a pair of
-// waves, Q and O^T in registers). With 128 heads two workgroups read a row, at
-// the same time and through one XCD's L2: 128 heads a workgroup need 512
-// registers a wave, which the compiler spilled.
-// Tiles of 64 tokens are copied global -> LDS directly, the next one while this
-// one is computed. Both products read the one copy: S^T's operand rows are token rows; O^T's operand
-// is transposed on the way out of LDS (ds_read_b64_tr_b16), and in the order in
-// which the accumulators of S^T hold their tokens, so P stays in registers.
-// 16-byte chunks are XOR-swizzled so that both kinds of read spread over the
-// banks. An fp8 cache is widened on its way through registers.
+// All query heads share ONE cache row a token; a workgroup takes 64 heads, of whose Q and
+// O^T its waves' registers hold all. With 128 heads two workgroups read a row, at the
+// same time and through one XCD's L2. Both products read the one copy of a tile in LDS:
+// S^T's operand rows are token rows; O^T's operand is transposed on the way out
+// (ds_read_b64_tr_b16), and in the order in which the accumulators of S^T hold their
+// tokens, so P stays in registers. 16-byte chunks are XOR-swizzled so that both kinds of
+// read spread over the banks. An fp8 cache is widened on its way through registers.
 //
-// Work is split by tiles, not by sequences: the tiles of all sequences form one
-// list, of which every workgroup takes an equal run. Lengths are read on the
-// device, so a captured step balances for any lengths. A sequence that lies in
-// one run is finished there; the others leave fp32 parts that a second kernel
-// adds up. Short sequences (256 tokens at most) take a workgroup each and need
-// no second kernel.
+// Every workgroup takes a run of tiles (find_run). Lengths are read on the device, so a
+// captured step balances for any lengths. A sequence that lies in one run is finished
+// there; the others leave fp32 parts that a second kernel adds up. Short sequences (256
+// tokens at most) take a workgroup each and need no second kernel.
 //
-// What bounds it: the latent rows' stream, 3.1 us a tile and CU at 6.1 TB/s where a
-// tile takes 3.7, and the start and end of a run, a quarter of the time of runs of 18
-// tiles. Copies go between S^T's products from uniform addresses; worked out a lane in
-// front of them, 250 instructions a wave, and S^T computed by both waves of a pair,
-// they left each other no room: 64 heads, 4 x 100,000 tokens 98 us, now 84; 128 heads,
-// 40 x 4,000 71 and 63; with the second kernel's 9 and 11.
+// Two kernels: mla_decode_wide_kernel for more than 32 heads, mla_decode_kernel for up to
+// 32 and for lists of token positions. What bounds them: with 64 heads the latent rows'
+// stream (6 TB/s), with 128 what a tile issues, 290 vector instructions and 34 products a
+// wave that hardly overlap, LDS reads; and the start and end of a run, 9 us of looking up,
+// first rows and parts, then 8 of the second kernel.
 //
 // Reference analogue: parallax_extensions/kernels/mla/ (Metal, VALU); fresh
 // MFMA design. Layout: cache [NB, BS, R+DR], q_latent [B, H, R], q_pe [B, H, DR].
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -37,9 +33,10 @@
 #define MLA_DK 576          // values a cache row
 #define MLA_ROW 1024        // bytes of a row's latent values in LDS
 #define MLA_PE 128          // and of its rotated ones
-#define MLA_KT 64           // tokens a tile
+#define MLA_KT 64           // tokens a tile,
 #define MLA_DT 16           // 16-value tiles of O^T a wave
-#define MLA_MIN_TILES 2     // a run is at least this long
+#define MLA_WT 32           // of the wide kernel
+#define MLA_MIN_TOKENS 128  // a run is at least this long
 #define MLA_MAX_RUNS 256    // one a CU
 
 // the lambdas below are called once a buffer: left out of line, their captures
@@ -47,12 +44,18 @@
 #define INL __attribute__((always_inline))
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
+typedef float f32x16v __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8n __attribute__((ext_vector_type(8)));
+typedef short bf16x2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2n __attribute__((ext_vector_type(2)));
 
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kHidden = -1e30f;
+
+template <int V> using Int = std::integral_constant<int, V>;
 
 DEVINL uint32_t pack_bf16(float a, float b) {
   bf16x2n p;
@@ -102,77 +105,87 @@ DEVINL int domain_of(const int* seq_lens, const int* topk, int max_topk,
   return max(seq_lens[b], 0);
 }
 
-// A sequence and its place in the list of all tiles, found by one wave: the
-// sequence with first <= tile < first + tiles. Returns the total of tiles.
-template <bool SPARSE>
-DEVINL int find_tile(const int* seq_lens, const int* topk, int max_topk, int B,
-                     int tile, int* seq, int* first) {
-  const int lane = threadIdx.x & 63;
-  int before = 0;
-  *seq = -1;
-  *first = 0;
-  for (int b0 = 0; b0 < B; b0 += 64) {
-    const int b = b0 + lane;
-    const int n =
-        b < B ? (domain_of<SPARSE>(seq_lens, topk, max_topk, b) + MLA_KT - 1) /
-                    MLA_KT
-              : 0;
-    int sum = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_up(sum, o, WAVE_SIZE);
-      if (lane >= o) sum += t;
-    }
-    const int t = tile - before;
-    const unsigned long long hit = __ballot(t >= sum - n && t < sum);
-    if (hit) {
-      const int src = __ffsll(hit) - 1;
-      *seq = b0 + src;
-      *first = before + __shfl(sum, src, WAVE_SIZE) -
-               __shfl(n, src, WAVE_SIZE);
-    }
-    before += __shfl(sum, 63, WAVE_SIZE);
-  }
-  return before;
+template <int CTRL>
+DEVINL int moved(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
 }
-
-DEVINL int run_length(int total, int runs) {
-  return max((total + runs - 1) / runs, MLA_MIN_TILES);
+DEVINL int wave_sum(int v) {
+  v += moved<0xb1>(v);   // lanes 1, 0, 3, 2
+  v += moved<0x4e>(v);   // lanes 2, 3, 0, 1
+  v += moved<0x141>(v);  // half rows mirrored
+  v += moved<0x140>(v);  // rows mirrored
+  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) +
+         __builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48);
 }
-
-// Run `run` of the list of all tiles: its length, the sequence of its first tile and
-// that tile's place there. Up to 64 sequences are looked at once, for the total too.
-template <bool SPARSE>
-DEVINL int find_run(const int* seq_lens, const int* topk, int max_topk, int B,
-                    int run, int runs, int* seq, int* at) {
-  int first;
-  if (B > 64) {
-    const int total = find_tile<SPARSE>(seq_lens, topk, max_topk, B, 0, seq, &first);
-    const int per = run_length(total, runs);
-    const int todo = min(per, total - run * per);
-    if (todo > 0)
-      find_tile<SPARSE>(seq_lens, topk, max_topk, B, run * per, seq, &first);
-    *at = run * per - first;
-    return todo;
-  }
-  const int lane = threadIdx.x & 63;
-  const int n = lane < B ? (domain_of<SPARSE>(seq_lens, topk, max_topk, lane) +
-                            MLA_KT - 1) / MLA_KT
-                         : 0;
-  int sum = n;
+DEVINL int sum_before(int v) {  // of lanes up to this one
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(sum, o, WAVE_SIZE);
-    if (lane >= o) sum += t;
+    const int t = __shfl_up(v, o, WAVE_SIZE);
+    if ((int)(threadIdx.x & 63) >= o) v += t;
   }
-  const int total = __builtin_amdgcn_readlane(sum, 63);
-  const int per = run_length(total, runs);
-  const int begin = run * per;
-  const unsigned long long hit = __ballot(begin >= sum - n && begin < sum);
-  const int src = hit ? __ffsll(hit) - 1 : 0;
-  *seq = src;
-  *at = begin - (__builtin_amdgcn_readlane(sum, src) - __builtin_amdgcn_readlane(n, src));
-  return min(per, total - begin);
+  return v;
+}
+// n / d rounded up, d > 0; exact to 2^21, and the same wherever it is asked
+DEVINL int div_up(int n, int d) {
+  return n > 0 ? (int)(((float)n - 0.5f) * __builtin_amdgcn_rcpf((float)d)) + 1 : 0;
+}
+
+// A workgroup's run: its sequence, the first tile there, and its tiles; how many there are
+// to a run of this sequence.
+struct Run {
+  int seq, at, todo, per;
+};
+
+// the first and the last run of each sequence, behind the parts' maxima and sums
+DEVINL int2* part_runs(float* tmp_ml, int runs, int B, int H) {
+  return reinterpret_cast<int2*>(tmp_ml + ((size_t)runs + B) * H * 2);
+}
+
+// How the tiles are dealt, found by one wave; tiles_of(b): of sequence b, 0 from B on.
+// Each run lies in one sequence, which has as many of equal length as it takes for none
+// to be longer than `per`, the least that `runs` suffice for. Or, where that is 256 tokens
+// more than even, runs go through the list of all tiles: a run that meets the next
+// sequence pays the start and the end of a run twice, which costs about as much. us of a
+// call, 64 heads, even / so: 4 sequences of 5,300 tokens 33.8 / 28.2, of 66,000 79.4 /
+// 73.8.
+template <int KT, class F>
+DEVINL Run find_run(int B, int run, int runs, F tiles_of) {
+  const int lane = threadIdx.x & 63;
+  const int n0 = tiles_of(lane);
+  int total = n0;
+  for (int b = lane + 64; b < B; b += 64) total += tiles_of(b);
+  total = wave_sum(total);
+  const int even = max(div_up(total, runs), MLA_MIN_TOKENS / KT);
+  int per = even;
+  bool whole = false;
+  while (!whole && per <= even + 256 / KT) {
+    int k = div_up(n0, per);
+    for (int b = lane + 64; b < B; b += 64) k += div_up(tiles_of(b), per);
+    k = wave_sum(k);
+    whole = k <= runs;
+    // as many runs as now go to rounding up
+    if (!whole) per = max(per + 1, div_up(total, max(runs - k + div_up(total, per), 1)));
+  }
+  if (!whole) per = even;
+  const int begin = whole ? run : run * per;  // in runs, or in tiles
+  int before = 0;
+  for (int b0 = 0; b0 < B; b0 += 64) {
+    const int tiles = b0 == 0 ? n0 : tiles_of(b0 + lane);
+    const int n = whole ? div_up(tiles, per) : tiles;
+    const int sum = before + sum_before(n);
+    const unsigned long long hit = __ballot(begin >= sum - n && begin < sum);
+    if (hit) {
+      const int src = __ffsll(hit) - 1;
+      const int t = __builtin_amdgcn_readlane(tiles, src);
+      const int k = __builtin_amdgcn_readlane(n, src);
+      const int first = __builtin_amdgcn_readlane(sum, src) - k;
+      if (!whole) return {b0 + src, begin - first, min(per, total - begin), per};
+      const int len = div_up(t, k), at = (run - first) * len;
+      return {b0 + src, at, min(len, t - at), len};
+    }
+    before = __builtin_amdgcn_readlane(sum, 63);
+  }
+  return {0, 0, 0, 1};
 }
 
 }  // namespace
@@ -189,7 +202,7 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     const int* __restrict__ seq_lens,
     const int* __restrict__ topk,           // [B, max_topk] (SPARSE)
     const int max_topk, const int B, const int max_blocks, const int H,
-    const int bs_shift, const float scale, const float c_scale) {
+    const int bs_shift, const float scale) {
   constexpr int RPW = MLA_KT / W;      // rows a wave copies
   constexpr int CPW = RPW + RPW / 8;   // copies: a row's latent values, 8 rows' rope
   constexpr int BUF = MLA_KT * (MLA_ROW + MLA_PE);
@@ -205,25 +218,28 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
   const int BS = 1 << bs_shift;
 
   // ---- this workgroup's run of tiles --------------------------------------------
-  int seq, at, todo;  // sequence, tile of it, tiles left
+  Run run = {(int)blockIdx.x, 0, 0, 1};
   if (tmp_acc == nullptr) {
-    seq = blockIdx.x;
-    at = 0;
-    todo = (domain_of<SPARSE>(seq_lens, topk, max_topk, seq) + MLA_KT - 1) /
-           MLA_KT;
-    if (todo == 0) {  // no tokens: zeros, of this workgroup's heads
+    run.todo = (domain_of<SPARSE>(seq_lens, topk, max_topk, run.seq) + MLA_KT - 1) /
+               MLA_KT;
+    if (run.todo == 0) {  // no tokens: zeros, of this workgroup's heads
       const int h0 = blockIdx.y * (W * 8), n = min(W * 8, H - h0);
       for (int e = tid; e < n * (MLA_R / 4); e += W * 64)
-        *reinterpret_cast<uint2*>(out + ((size_t)seq * H + h0) * MLA_R + e * 4) =
+        *reinterpret_cast<uint2*>(out + ((size_t)run.seq * H + h0) * MLA_R + e * 4) =
             make_uint2(0, 0);
     }
   } else {
-    todo = find_run<SPARSE>(seq_lens, topk, max_topk, B, blockIdx.x, gridDim.x, &seq,
-                            &at);
+    auto tiles_of = [&](int b) INL {
+      return b < B ? (domain_of<SPARSE>(seq_lens, topk, max_topk, b) + MLA_KT - 1) / MLA_KT
+                   : 0;
+    };
+    run = find_run<MLA_KT>(B, blockIdx.x, gridDim.x, tiles_of);
   }
-  seq = __builtin_amdgcn_readfirstlane(seq);
-  at = __builtin_amdgcn_readfirstlane(at);
-  todo = __builtin_amdgcn_readfirstlane(todo);
+  int seq = __builtin_amdgcn_readfirstlane(run.seq);
+  int at = __builtin_amdgcn_readfirstlane(run.at);    // tile of the sequence
+  int todo = __builtin_amdgcn_readfirstlane(run.todo);
+  int done = 0;  // tiles of the run so far
+  const int per = __builtin_amdgcn_readfirstlane(run.per);
 
   // two waves share 16 heads: each computes S^T of half of the tokens, and O^T of
   // half of the latent values
@@ -262,6 +278,9 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     }
     const int t0 = at;
     const int t1 = min(tiles, at + todo);
+    if (tmp_acc != nullptr && t0 == 0 && tid == 0 && blockIdx.y == 0)
+      part_runs(tmp_ml, gridDim.x, B, H)[seq] =
+          make_int2(blockIdx.x, blockIdx.x + (done + tiles - 1) / per);
 
     bf16x8v qf[MLA_DK / 32];  // B operands: head l15, values 32 ks + 8 l4 + (0..7)
     f32x4v acc[MLA_DT] = {};
@@ -341,7 +360,7 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
       for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i)
         copy_of(i, [&](int i, int place, const uint8_t*, int) INL {
           int4 v;
-          fp8x8_to_bf16x8(raw[KV_FP8 ? i : 0], c_scale,
+          fp8x8_to_bf16x8(raw[KV_FP8 ? i : 0], 1.f,
                           reinterpret_cast<uint16_t*>(&v));
           *reinterpret_cast<int4*>(S + buf * BUF + place + lane * 16) = v;
         });
@@ -575,7 +594,8 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
           *reinterpret_cast<uint2*>(o + d * 16) = v;
         }
       } else {
-        // runs and sequences both advance: their sum names a part
+        // a run has one part of a sequence, and one of each more sequence that it meets:
+        // runs and sequences both advance, so their sum names a part
         const size_t part = ((size_t)blockIdx.x + seq) * H + head;
         float* o = tmp_acc + part * MLA_R + d0 + l4 * 4;
 #pragma unroll
@@ -588,6 +608,418 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
       }
     }
     todo -= t1 - t0;
+    done += t1 - t0;
+    ++seq;
+    at = 0;
+  }
+}
+
+// ---- more than 32 heads ----------------------------------------------------------
+// Four waves, 64 heads: 32 a pair of waves, on 32x32 matrix instructions, so that an
+// operand row read from LDS serves 32 heads instead of 16. A wave computes S^T over
+// half of the 576 values, for which it holds the heads' Q, adds the other wave's half,
+// and takes half of the latent values of O^T: 200 registers of state, so one wave a
+// SIMD. Tiles of 32 tokens in a ring of four, three of them on their way. In turn t
+// the products of S^T of tile t + 1 stand beside tile t's softmax.
+// us of a call with the second kernel, mla_decode_kernel of eight waves (16 heads a pair,
+// tiles of 64) and an even deal / so: 64 heads, 4 sequences of 66,000 tokens 82 / 72, of
+// 5,300 34.3 / 26.7; 128 heads, 40 of 2,400 61.5 / 58.5, 99 of 233 54 / 33, fp8 4 of 66,000
+// 139 / 124. The maximum followed only when it has moved by 2^8 takes 128 of the 290
+// instructions away and 10% of the time with 128 heads, and adds 2 to 13% to the error.
+template <bool KV_FP8>
+__global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
+    uint16_t* __restrict__ out,             // [B, H, R]
+    float* __restrict__ tmp_acc,            // [parts, H, R]; null: a workgroup
+    float* __restrict__ tmp_ml,             // [parts, H, 2]      a sequence
+    const uint16_t* __restrict__ q_latent,  // [B, H, R]
+    const uint16_t* __restrict__ q_pe,      // [B, H, DR]
+    const void* __restrict__ cache,         // [NB, BS, R+DR] bf16 | fp8(e4m3)
+    const int* __restrict__ block_tables,   // [B, max_blocks]
+    const int* __restrict__ seq_lens, const int B, const int max_blocks,
+    const int H, const int bs_shift, const float scale) {
+  constexpr int BUF = MLA_WT * (MLA_ROW + MLA_PE);
+  constexpr int PE = MLA_WT * MLA_ROW;  // of a buffer's rotated values
+  constexpr int RING = 4;
+  constexpr int CPW = 9;                // copies a wave: 8 rows, their rotated values
+  constexpr int QS = 18;                // steps of 16 values of S^T a wave
+  constexpr int DT = 8;                 // tiles of 32 latent values of O^T a wave
+  constexpr int ESZ = KV_FP8 ? 1 : 2;
+  __shared__ __attribute__((aligned(1024))) uint8_t S[RING * BUF];
+  // sums over half of the values on their way to the other wave of a pair
+  __shared__ __attribute__((aligned(16))) f32x4v X[4][4][64];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, l31 = lane & 31, half = lane >> 5;
+  const int BS = 1 << bs_shift;
+
+  Run run = {(int)blockIdx.x, 0, 0, 1};
+  if (tmp_acc == nullptr) {
+    run.todo = (max(seq_lens[run.seq], 0) + MLA_WT - 1) / MLA_WT;
+    if (run.todo == 0) {  // no tokens: zeros, of this workgroup's heads
+      const int h0 = blockIdx.y * 64, n = min(64, H - h0);
+      for (int e = tid; e < n * (MLA_R / 4); e += 256)
+        *reinterpret_cast<uint2*>(out + ((size_t)run.seq * H + h0) * MLA_R + e * 4) =
+            make_uint2(0, 0);
+    }
+  } else {
+    auto tiles_of = [&](int b) INL {
+      return b < B ? (max(seq_lens[b], 0) + MLA_WT - 1) / MLA_WT : 0;
+    };
+    run = find_run<MLA_WT>(B, blockIdx.x, gridDim.x, tiles_of);
+  }
+  int seq = __builtin_amdgcn_readfirstlane(run.seq);
+  int at = __builtin_amdgcn_readfirstlane(run.at);    // tile of the sequence
+  int todo = __builtin_amdgcn_readfirstlane(run.todo);
+  int done = 0;  // tiles of the run so far
+  const int per = __builtin_amdgcn_readfirstlane(run.per);
+
+  const int h = wid & 1;  // which half of the values
+  const int head = (blockIdx.y * 2 + (wid >> 1)) * 32 + l31;
+
+  // Chunk c of row r of a tile lies at c ^ wide_xor(r), of its rotated values at c ^
+  // ((r >> 1) & 7). 16-byte reads of one chunk go by rows {0-3, 12-15, 20-23, 24-27}
+  // and the others, which differ in both; transposing reads take four neighbouring
+  // chunks of four rows, which differ in bits 2 and 3 of wide_xor.
+  auto wide_xor = [](int r) INL { return (r & 3) * 4 + (r >> 2 & 3); };
+  const uint32_t s_at = (uint32_t)(uintptr_t)(
+      __attribute__((address_space(3))) const void*)S;
+  const int qk_at = l31 * MLA_ROW + h * 512 + (half ^ wide_xor(l31)) * 16;
+  const int pe_at = PE + l31 * MLA_PE + ((4 * h + half) ^ (l31 >> 1 & 7)) * 16;
+  const int tr_row = 4 * half + (l15 >> 2);
+  const int tr_at = tr_row * MLA_ROW + h * 512 +
+                    ((2 * (lane >> 4 & 1) + (l15 >> 1 & 1)) ^ wide_xor(tr_row)) * 16 +
+                    (l15 & 1) * 8;
+  // copy i of a wave: row 8 wid + i's latent values, or of its 8 rows the rotated ones
+  uint32_t from[CPW];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    from[i] = (i * MLA_DK + (lane ^ wide_xor(wid * 8 + i)) * 8) * ESZ;
+  from[8] = ((lane >> 3) * MLA_DK + MLA_R +
+             ((lane & 7) ^ ((wid * 8 + (lane >> 3)) >> 1 & 7)) * 8) * ESZ;
+  auto place = [&](int i) INL {
+    return i < 8 ? (wid * 8 + i) * MLA_ROW : PE + wid * 8 * MLA_PE;
+  };
+
+  bool first = true;
+  while (todo > 0) {
+    // Q first: its many rows are on their way while length and pages are looked up
+    bf16x8v qf[QS];  // head l31, values 16 i + 8 half of this wave's
+    {
+      const size_t row = (size_t)seq * H + min(head, H - 1);
+#pragma unroll
+      for (int i = 0; i < QS; ++i)
+        qf[i] = i < 16
+                    ? *(const bf16x8v*)(q_latent + row * MLA_R + h * 256 + i * 16 + half * 8)
+                    : *(const bf16x8v*)(q_pe + row * MLA_DR + h * 32 + (i - 16) * 16 +
+                                        half * 8);
+    }
+    const int L = seq_lens[seq];
+    const int tiles = (max(L, 0) + MLA_WT - 1) / MLA_WT;
+    if (at >= tiles) {  // a sequence without tokens
+      ++seq;
+      at = 0;
+      continue;
+    }
+    const auto* btab = (const __attribute__((address_space(4))) int*)(
+        block_tables + (size_t)seq * max_blocks);
+    const int t0 = at;
+    const int t1 = min(tiles, at + todo);
+    if (tmp_acc != nullptr && t0 == 0 && tid == 0 && blockIdx.y == 0)
+      part_runs(tmp_ml, gridDim.x, B, H)[seq] =
+          make_int2(blockIdx.x, blockIdx.x + (done + tiles - 1) / per);
+
+    // ---- copies: tile t goes to place t - t0 of the ring -------------------------------
+    // 8 rows lie in one page; rows past the end read a page that is there
+    auto token_of = [&](int t) INL { return min(t * MLA_WT + wid * 8, (L - 1) & ~7); };
+    auto page_of = [&](int t) INL { return btab[token_of(t) >> bs_shift]; };
+    auto base_of = [&](int t, int page) INL {
+      const int slot = (page << bs_shift) + (token_of(t) & (BS - 1));
+      return (const uint8_t*)cache + (int64_t)slot * (MLA_DK * ESZ);
+    };
+    auto issue = [&](int i, const uint8_t* base, int t) INL {
+      copy16(base, from[i], s_at + ((t - t0) & (RING - 1)) * BUF + place(i));
+    };
+    uint64_t raw[2][KV_FP8 ? CPW : 1];  // an fp8 cache: two tiles on their way
+    auto fetch8 = [&](uint64_t (&r)[KV_FP8 ? CPW : 1], int t, int page) INL {
+      const uint8_t* base = base_of(t, page);
+#pragma unroll
+      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i)
+        r[i] = *(const uint64_t*)(base + from[i]);
+    };
+    auto widen8 = [&](const uint64_t (&r)[KV_FP8 ? CPW : 1], int t) INL {
+      uint8_t* T = S + ((t - t0) & (RING - 1)) * BUF + lane * 16;
+#pragma unroll
+      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i) {
+        bf16x8n v;  // every e4m3 number is one of bf16
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const auto two = j & 1
+              ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)(r[i] >> 32 * (j >> 1)),
+                                                          1.f, true)
+              : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)(r[i] >> 32 * (j >> 1)),
+                                                          1.f, false);
+          v[2 * j] = two[0];
+          v[2 * j + 1] = two[1];
+        }
+        *reinterpret_cast<bf16x8n*>(T + place(i)) = v;
+      }
+    };
+
+    f32x16v acc[DT] = {};
+    f32x16v sc[2];  // scores of a tile and of the next one
+    float m = kHidden, l = 0.f;
+    const float c = fmaxf(fabsf(scale) * kLog2e, 1e-30f);  // the sign: Q's
+    bf16x8v b[2];   // the weights, operands of O^T
+    float f = 1.f;  // of O^T so far
+
+    auto meet = [] INL {  // copies stay in flight
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    // rows of the last tile that stand for no token may hold anything: weight 0 times it
+    auto clear_rest = [&](int t) INL {
+      const int n = L - t * MLA_WT;
+      if (n >= MLA_WT || n <= 0) return;
+      constexpr int CH = (MLA_ROW + MLA_PE) / 16;
+      uint8_t* T = S + ((t - t0) & (RING - 1)) * BUF;
+      for (int i = n * CH + tid; i < MLA_WT * CH; i += 256) {
+        const int row = i / CH, ch = i % CH;
+        *reinterpret_cast<int4*>(
+            T + (ch < 64 ? row * MLA_ROW + ch * 16
+                         : PE + row * MLA_PE + (ch - 64) * 16)) = make_int4(0, 0, 0, 0);
+      }
+      __syncthreads();
+    };
+
+    // S^T over this wave's values; between(i): what goes with product i. One wave a
+    // SIMD: operands are asked for two batches ahead.
+    auto scores = [&](int t, f32x16v& r, auto&& between) INL {
+      const uint8_t* T = S + ((t - t0) & (RING - 1)) * BUF;
+      constexpr int KB = 3;
+      bf16x8v a[3][KB];
+      auto fetch = [&](int n) INL {
+#pragma unroll
+        for (int i = 0; i < KB; ++i) {
+          const int ks = n * KB + i;
+          a[n % 3][i] = *reinterpret_cast<const bf16x8v*>(
+              T + (ks < 16 ? (qk_at ^ (ks & 7) * 32) + (ks >> 3) * 256
+                           : pe_at ^ (ks & 1) * 32));
+        }
+      };
+      r = f32x16v{};
+      fetch(0);
+      fetch(1);
+#pragma unroll
+      for (int n = 0; n < QS / KB; ++n) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (n + 2 < QS / KB) fetch(n + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < KB; ++i) {
+          r = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[n % 3][i], qf[n * KB + i], r, 0, 0,
+                                                      0);
+          __builtin_amdgcn_sched_barrier(0);
+          between(n * KB + i);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    auto publish = [&](const f32x16v& r) INL {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        X[wid][q][lane] = f32x4v{r[4 * q], r[4 * q + 1], r[4 * q + 2], r[4 * q + 3]};
+    };
+
+    // ---- the softmax of a tile, in 18 pieces ---------------------------------------------
+    // token 8 q + 4 half + r of the tile in s[4 q + r]
+    float mx;
+    auto soften = [&](int i, f32x16v& s, const f32x4v (&x)[4]) INL {
+      if (i < 4) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[4 * i + r] += x[i][r];
+        const float a = fmaxf(fmaxf(s[4 * i], s[4 * i + 1]), s[4 * i + 2]);
+        mx = i == 0 ? fmaxf(a, s[3]) : fmaxf(fmaxf(mx, a), s[4 * i + 3]);
+      } else if (i == 4) {
+        const auto o = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = fmaxf(__uint_as_float(o[0]), __uint_as_float(o[1])) * c;
+        // a new maximum's own weight is 1, without rounding (m moved only by 2^8 and
+        // more: 2 to 13% more error)
+        const float m2 = fmaxf(m, mx);
+        f = __builtin_amdgcn_exp2f(m - m2);
+        m = m2;
+        l *= f;
+      } else if (i < 13) {
+        const int e = (i - 5) * 2;
+        uint32_t pk = pack_bf16(__builtin_amdgcn_exp2f(fmaf(s[e], c, -m)),
+                                __builtin_amdgcn_exp2f(fmaf(s[e + 1], c, -m)));
+        // of the rounded weights: what their rounding adds to O^T it adds to both
+        l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2v, pk),
+                                            __builtin_bit_cast(bf16x2v, 0x3f803f80u), l,
+                                            false);
+        auto w = __builtin_bit_cast(u32x4v, b[e >> 3]);
+        w[e >> 1 & 3] = pk;
+        b[e >> 3] = __builtin_bit_cast(bf16x8v, w);
+      }
+    };
+
+    // O^T: rows = 32 latent values, contraction over tokens 16 u + 4 half + (0..3) and
+    // 8 more: what this half of S^T's lanes holds
+    bf16x8v va[3][2];
+    auto fetch_v = [&](int t, int d) INL {
+      uint8_t* T = S + ((t - t0) & (RING - 1)) * BUF;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        uint8_t* src = T + (d >> 2) * 256 + u * 16 * MLA_ROW;
+        const s16x4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4v*)(src + (tr_at ^ (d & 3) * 64)));
+        const s16x4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4v*)(
+                src + 8 * MLA_ROW + (tr_at ^ ((d & 3) * 64 + 32))));
+        va[d % 3][u] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+    };
+    auto weigh = [&](int t) INL {  // behind fetch_v of 0 and 1
+      acc[0] *= f;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (d + 2 < DT) fetch_v(t, d + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[d] =
+            __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[d % 3][0], b[0], acc[d], 0, 0, 0);
+        if (d + 1 < DT) acc[d + 1] *= f;
+        acc[d] =
+            __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[d % 3][1], b[1], acc[d], 0, 0, 0);
+      }
+    };
+
+    // ---- the run -----------------------------------------------------------------------
+    if (scale < 0.f)
+#pragma unroll
+      for (int i = 0; i < QS; ++i) qf[i] ^= (short)0x8000;
+    // Q is read by products alone: in the registers that only those take as operands. It
+    // is there before the copies are asked for, as a wait for it would be one for them
+#pragma unroll
+    for (int i = 0; i < QS; ++i) asm volatile("" : "+a"(qf[i]));
+    if (!first) __syncthreads();  // the buffers may still be read for the last sequence
+    first = false;
+    if constexpr (KV_FP8) {
+      fetch8(raw[0], t0, page_of(t0));
+      fetch8(raw[1], min(t0 + 1, t1 - 1), page_of(min(t0 + 1, t1 - 1)));
+    } else {
+#pragma unroll
+      for (int k = 0; k < RING - 1; ++k) {
+        const int tk = min(t0 + k, t1 - 1);
+        const uint8_t* base = base_of(tk, page_of(tk));
+#pragma unroll
+        for (int i = 0; i < CPW; ++i) issue(i, base, t0 + k);
+      }
+    }
+    // the first tile's scores
+    if constexpr (KV_FP8) {
+      widen8(raw[0], t0);
+      const int t2 = min(t0 + 2, t1 - 1);
+      fetch8(raw[0], t2, page_of(t2));
+      widen8(raw[1], t0 + 1);
+    } else {
+      __builtin_amdgcn_s_waitcnt(0x4f72);  // vmcnt(18): those of two tiles in flight
+    }
+    meet();
+    clear_rest(t0);
+    scores(t0, sc[0], [](int) {});
+    publish(sc[0]);
+
+    // Turn t. Behind its first barrier tile t + 1 is in LDS, both halves of S^T of tile
+    // t are there, and every wave has left the place that tile t + 3 goes to. Past the
+    // run's end copies and products go on with its last tile: one loop for all turns, as
+    // instructions that are not in the cache yet cost a run of few tiles 1 us and more.
+    int page = page_of(min(t0 + 3, t1 - 1));  // of the tile that the next turn copies
+    auto turn = [&](int t, auto even) INL {
+      constexpr int P = decltype(even)::value;
+      const int ahead = min(t + 3, t1 - 1);
+      // this thread's copies of tile t + 1: those of t + 2 stay in flight
+      if constexpr (!KV_FP8) __builtin_amdgcn_s_waitcnt(0x0f70 | CPW);
+      meet();
+      f32x4v x[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[q] = X[wid ^ 1][q][lane];
+      const int rest = L - t * MLA_WT;
+      if (rest < MLA_WT)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            x[q][r] = 8 * q + 4 * half + r < rest ? x[q][r] : -3e38f;
+      const uint8_t* base = nullptr;
+      if constexpr (KV_FP8) fetch8(raw[P ^ 1], ahead, page);
+      else base = base_of(ahead, page);
+      clear_rest(t + 1);
+      scores(t + 1, sc[P ^ 1], [&](int i) INL {
+        if (!KV_FP8 && (i & 1) == 0) issue(i >> 1, base, t + 3);
+        soften(i, sc[P], x);
+        // on their way to behind the barrier
+        if (i == 15) fetch_v(t, 0);
+        if (i == 16) fetch_v(t, 1);
+        if (i == 17) page = page_of(min(t + 4, t1 - 1));
+      });
+      meet();  // every wave has the other's half of tile t
+      publish(sc[P ^ 1]);
+      weigh(t);
+      if constexpr (KV_FP8) widen8(raw[P], t + 2);
+    };
+    for (int t = t0;;) {
+      turn(t, Int<0>{});
+      if (++t >= t1) break;
+      turn(t, Int<1>{});
+      if (++t >= t1) break;
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // the last copies
+
+    // ---- results: column = head, rows = latent values --------------------------------
+    {
+      const auto o = __builtin_amdgcn_permlane32_swap(
+          __float_as_uint(l), __float_as_uint(l), false, false);
+      l = __uint_as_float(o[0]) + __uint_as_float(o[1]);
+    }
+    if (head < H) {
+      const int d0 = h * 256 + half * 4;
+      if (t0 == 0 && t1 == tiles) {
+        const float inv = 1.f / l;
+        uint16_t* o = out + ((size_t)seq * H + head) * MLA_R + d0;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            uint2 v;
+            v.x = pack_bf16(acc[d][4 * q] * inv, acc[d][4 * q + 1] * inv);
+            v.y = pack_bf16(acc[d][4 * q + 2] * inv, acc[d][4 * q + 3] * inv);
+            *reinterpret_cast<uint2*>(o + d * 32 + q * 8) = v;
+          }
+      } else {
+        // a run has one part of a sequence, and one of each more sequence that it meets:
+        // runs and sequences both advance, so their sum names a part
+        const size_t part = ((size_t)blockIdx.x + seq) * H + head;
+        float* o = tmp_acc + part * MLA_R + d0;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4v*>(o + d * 32 + q * 8) =
+                f32x4v{acc[d][4 * q], acc[d][4 * q + 1], acc[d][4 * q + 2],
+                       acc[d][4 * q + 3]};
+        if (half == 0 && h == 0) {
+          tmp_ml[part * 2] = m;  // in units of log2
+          tmp_ml[part * 2 + 1] = l;
+        }
+      }
+    }
+    todo -= t1 - t0;
+    done += t1 - t0;
     ++seq;
     at = 0;
   }
@@ -608,21 +1040,8 @@ __global__ __launch_bounds__(512) void mla_reduce_kernel(
   const int tid = threadIdx.x;
   const int lane = tid & 63, grp = tid >> 7;
   const int head = BY_HEAD ? blockIdx.x * 4 + grp : blockIdx.x;
-  int total = 0, first = 0;  // tiles of all sequences, of those before this one
-  for (int b = lane; b < B; b += 64) {
-    const int n =
-        (domain_of<SPARSE>(seq_lens, topk, max_topk, b) + MLA_KT - 1) / MLA_KT;
-    total += n;
-    first += b < seq ? n : 0;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    total += __shfl_xor(total, o, WAVE_SIZE);
-    first += __shfl_xor(first, o, WAVE_SIZE);
-  }
-  const int tiles =
-      (domain_of<SPARSE>(seq_lens, topk, max_topk, seq) + MLA_KT - 1) / MLA_KT;
-  if (tiles == 0) {  // no tokens: zeros
+  const int2 range = part_runs(const_cast<float*>(tmp_ml), runs, B, H)[seq];
+  if (domain_of<SPARSE>(seq_lens, topk, max_topk, seq) == 0) {  // no tokens: zeros
     if (head < H)
       for (int d = (BY_HEAD ? tid & 127 : tid) * 4; d < MLA_R;
            d += (BY_HEAD ? 128 : 512) * 4)
@@ -630,8 +1049,7 @@ __global__ __launch_bounds__(512) void mla_reduce_kernel(
             make_uint2(0, 0);
     return;
   }
-  const int per = run_length(total, runs);
-  const int r0 = first / per, r1 = (first + tiles - 1) / per;
+  const int r0 = range.x, r1 = range.y;
   if (r0 == r1) return;  // finished by its run
 
   __shared__ f32x4v sums[4][128];
@@ -686,7 +1104,7 @@ __global__ __launch_bounds__(512) void mla_reduce_kernel(
 }
 
 // Runs the tiles are dealt to; 0: every sequence has a workgroup of its own.
-// One workgroup a CU: its two tiles (144 KB) fill the LDS.
+// One workgroup a CU: its tiles (144 KB) fill the LDS.
 extern "C" int mla_decode_runs(int B, int H, int max_domain) {
   const int blocks = ceil_div(H, 64);
   if (max_domain <= 256) return 0;
@@ -698,7 +1116,7 @@ extern "C" void launch_mla_paged_attention_decode(
     const int* block_tables, const int* seq_lens, int B, int H, int R, int DR,
     int BS, int max_blocks, float scale, int runs, float* tmp_acc,
     float* tmp_ml, const int* topk_indices, int max_topk, bool kv_fp8,
-    float c_scale, hipStream_t stream, bool* launched) {
+    hipStream_t stream, bool* launched) {
   *launched = false;
   if (R != MLA_R || DR != MLA_DR) return;  // DeepSeek V2/V3/R1/K2 geometry
   if (BS != 16 && BS != 32 && BS != 64) return;
@@ -706,29 +1124,45 @@ extern "C" void launch_mla_paged_attention_decode(
   const int waves = H > 32 ? 8 : 4;
   dim3 grid(runs > 0 ? runs : B, ceil_div(H, waves * 8), 1);
 
-#define MLA_LAUNCH(WV, FP8, SP)                                               \
-  mla_decode_kernel<WV, FP8, SP><<<grid, WV * 64, 0, stream>>>(               \
-      (uint16_t*)out, tmp_acc, tmp_ml, (const uint16_t*)q_latent,             \
-      (const uint16_t*)q_pe, cache, block_tables, seq_lens, topk_indices,     \
-      max_topk, B, max_blocks, H, shift, scale, c_scale);
-#define MLA_LAUNCH2(FP8, SP)                 \
-  if (waves == 8) { MLA_LAUNCH(8, FP8, SP) } \
-  else { MLA_LAUNCH(4, FP8, SP) }
-#define MLA_REDUCE(SP, BY_HEAD, GRID)                                         \
-  mla_reduce_kernel<SP, BY_HEAD><<<dim3(GRID, B, 1), 512, 0, stream>>>(       \
-      (uint16_t*)out, tmp_acc, tmp_ml, seq_lens, topk_indices, max_topk, B, H, \
-      runs);
-#define MLA_LAUNCH3(SP)                                       \
-  if (kv_fp8) { MLA_LAUNCH2(true, SP) }                       \
-  else { MLA_LAUNCH2(false, SP) }                             \
-  if (runs > 0 && runs >= 16 * B) { MLA_REDUCE(SP, false, H) } \
-  else if (runs > 0) { MLA_REDUCE(SP, true, ceil_div(H, 4)) }
-
-  if (topk_indices != nullptr) { MLA_LAUNCH3(true) }
-  else { MLA_LAUNCH3(false) }
-#undef MLA_LAUNCH
-#undef MLA_LAUNCH2
-#undef MLA_LAUNCH3
-#undef MLA_REDUCE
+#define MLA_ARGS                                                               \
+  (uint16_t*)out, tmp_acc, tmp_ml, (const uint16_t*)q_latent,                  \
+      (const uint16_t*)q_pe, cache, block_tables, seq_lens
+  auto decode = [&](auto w, auto fp8, auto sparse) {
+    mla_decode_kernel<decltype(w)::value, decltype(fp8)::value, decltype(sparse)::value>
+        <<<grid, decltype(w)::value * 64, 0, stream>>>(
+            MLA_ARGS, topk_indices, max_topk, B, max_blocks, H, shift, scale);
+  };
+  auto reduce = [&](auto sparse) {
+    constexpr bool SP = decltype(sparse)::value;
+    if (runs <= 0) return;
+    if (runs >= 16 * B)
+      mla_reduce_kernel<SP, false><<<dim3(H, B, 1), 512, 0, stream>>>(
+          (uint16_t*)out, tmp_acc, tmp_ml, seq_lens, topk_indices, max_topk, B, H, runs);
+    else
+      mla_reduce_kernel<SP, true><<<dim3(ceil_div(H, 4), B, 1), 512, 0, stream>>>(
+          (uint16_t*)out, tmp_acc, tmp_ml, seq_lens, topk_indices, max_topk, B, H, runs);
+  };
+  using True = std::true_type;
+  using False = std::false_type;
+  if (topk_indices != nullptr) {
+    if (waves == 8 && kv_fp8) decode(Int<8>{}, True{}, True{});
+    else if (waves == 8) decode(Int<8>{}, False{}, True{});
+    else if (kv_fp8) decode(Int<4>{}, True{}, True{});
+    else decode(Int<4>{}, False{}, True{});
+    reduce(True{});
+  } else if (H > 32) {
+    if (kv_fp8)
+      mla_decode_wide_kernel<true><<<grid, 256, 0, stream>>>(MLA_ARGS, B, max_blocks, H,
+                                                             shift, scale);
+    else
+      mla_decode_wide_kernel<false><<<grid, 256, 0, stream>>>(MLA_ARGS, B, max_blocks, H,
+                                                              shift, scale);
+    reduce(False{});
+  } else {
+    if (kv_fp8) decode(Int<4>{}, True{}, False{});
+    else decode(Int<4>{}, False{}, False{});
+    reduce(False{});
+  }
+#undef MLA_ARGS
   *launched = true;
 }

@@ -342,3 +342,40 @@ def test_linear_mla_rope_and_cache(M, K, R, DR, fp8, neox):
     assert run(kv_w=kv_w[:-8]) is None and run(q=q.float()) is None
     assert run(x=rand(M, K + 4)[:, 4:]) is None              # rows at odd places
     assert run(kv_w=kv_w.clone().requires_grad_()) is None
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+@pytest.mark.parametrize("H,BS,ctxs", [
+    (64, 32, [257, 31, 32, 33, 1, 64, 65, 0, 96]),  # ends of tiles of 32, none
+    (33, 16, [1000]),                               # heads past the last one
+    (100, 64, [300, 129, 4000]),                    # two workgroups, one part full
+    (128, 32, [9000, 1, 290]),                      # many runs of one sequence
+    (128, 16, [260] + [90, 13, 200] * 50),          # runs that meet sequences
+    (64, 32, [20, 255]),                            # a workgroup a sequence
+    (16, 32, [3000, 0, 65]),                        # tiles of 64: the same deal
+])
+def test_mla_decode_tiles_and_runs(H, BS, ctxs, kv):
+    """Edges of tiles, runs and sequences; slots past a sequence's end hold NaN."""
+    B, scale = len(ctxs), 192 ** -0.5
+    ql, qp, cache, bt, sl = _setup(B, H, ctxs, BS=BS, seed=7)
+    ql, qp = ql * 10, qp * 10  # unit normal: weights of unequal size
+    dt = torch.float8_e4m3fn if kv == "fp8" else torch.bfloat16
+    cache = cache.to(dt)
+    for i, n in enumerate(ctxs):  # what a sequence has not filled
+        if n % BS:
+            cache[int(bt[i, n // BS]), n % BS:] = float("nan")
+    out = ops.mla_paged_attention_decode(ql, qp, cache, bt, sl, scale)
+    again = ops.mla_paged_attention_decode(ql, qp, cache, bt, sl, scale)
+    assert torch.equal(out, again)
+    for i, n in enumerate(ctxs):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        pages = bt[i, :(n + BS - 1) // BS].long()
+        e = cache[pages].double().flatten(0, 1)[:n]
+        p = ((ql[i].double() @ e[:, :512].T + qp[i].double() @ e[:, 512:].T)
+             * scale).softmax(-1)
+        want = p @ e[:, :512]
+        err = (out[i].double() - want).norm() / want.norm()
+        # weights and results are rounded to bf16: 2^-9 at most each
+        assert err < 2 * 2 ** -9, (i, n, float(err))
