@@ -85,6 +85,9 @@ DEVINL float sum_halves(float v) {
 // [head, row, feature] and values as [head, feature, row]: the operand order is
 // swapped between the two, so that a lane's four neighbouring registers are
 // neighbours in memory either way. Rows past the run are written as zeros.
+// What bounds it: LDS reads, as long as products and stages that it waits for beside
+// them. 1,900 rows, 128 heads: 128 us; stored from the accumulators, 16 bytes of 32 rows
+// an instruction, 155; five stages of 64 bytes in a ring 141.
 
 __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
     uint16_t* __restrict__ k_hi, uint16_t* __restrict__ k_lo,  // [H, cap, 128]
@@ -158,8 +161,9 @@ __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
     stage(S1);
   }
 
-  uint16_t* hi = (val ? v_hi : k_hi) + (size_t)h * cap * MP_D;
-  uint16_t* lo = (val ? v_lo : k_lo) + (size_t)h * cap * MP_D;
+  // Through LDS, so that a wave stores whole lines: rows of 128 (of a key's features, or
+  // of one feature's context rows), 16-byte chunk c of row r at c ^ (r & 15).
+  __syncthreads();  // every wave is done with the stages
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int col = (rb & 127) + j * 32 + l31;
@@ -177,11 +181,24 @@ __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
         }
         split2(x[0], x[1], a.x, b.x);
         split2(x[2], x[3], a.y, b.y);
-        const size_t at = val ? (size_t)col * cap + r0 + row
-                              : (size_t)(r0 + col) * MP_D + row;
-        *reinterpret_cast<uint2*>(hi + at) = a;
-        *reinterpret_cast<uint2*>(lo + at) = b;
+        const int at = col * 256 + ((row >> 3) ^ (col & 15)) * 16 + half * 8;
+        *reinterpret_cast<uint2*>(S0 + at) = a;
+        *reinterpret_cast<uint2*>(S1 + at) = b;
       }
+  }
+  __syncthreads();
+  const size_t base = (size_t)h * cap * MP_D + (val ? (size_t)r0 : (size_t)r0 * MP_D);
+  const size_t pitch = val ? cap : MP_D;
+  uint16_t* hi = (val ? v_hi : k_hi) + base;
+  uint16_t* lo = (val ? v_lo : k_lo) + base;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int row = i * 16 + (tid >> 4), ch = tid & 15;
+    const int at = row * 256 + (ch ^ (row & 15)) * 16;
+    *reinterpret_cast<u32x4v*>(hi + row * pitch + ch * 8) =
+        *reinterpret_cast<const u32x4v*>(S0 + at);
+    *reinterpret_cast<u32x4v*>(lo + row * pitch + ch * 8) =
+        *reinterpret_cast<const u32x4v*>(S1 + at);
   }
 }
 
