@@ -395,7 +395,8 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                                        (int)sliding_window);
     if (runs > 0) {
       tmp_acc = torch::empty({(int64_t)runs + B, Hq, D}, opts);
-      tmp_ml = torch::empty({(int64_t)runs + B, Hq, 2}, opts);
+      // of a part each head's maximum and sum; of a sequence its first and last run
+      tmp_ml = torch::empty({((int64_t)runs + B) * Hq * 2 + 2 * B}, opts);
       acc_ptr = tmp_acc.data_ptr<float>();
       ml_ptr = tmp_ml.data_ptr<float>();
     }
@@ -486,7 +487,7 @@ std::optional<torch::Tensor> rope_cache_attention_decode(
   if (runs > 0) {
     const auto opts = q.options().dtype(at::kFloat);
     acc = torch::empty({runs + B, Hq, D}, opts);
-    ml = torch::empty({runs + B, Hq, 2}, opts);
+    ml = torch::empty({(runs + B) * Hq * 2 + 2 * B}, opts);
   }
   bool launched = false;
   launch_paged_decode(

@@ -174,11 +174,16 @@ DEVINL int run_length(int total, int runs) {
   return max((total + runs - 1) / runs, 1);
 }
 
+// the first and the last run of each sequence, behind the parts' maxima and sums
+DEVINL int2* part_runs(float* tmp_ml, int runs, int B, int Hq) {
+  return reinterpret_cast<int2*>(tmp_ml + ((size_t)runs + B) * Hq * 2);
+}
+
 // Run `run` of the list of all sequences' units: its length, the sequence that
-// holds its first unit, and that unit's place there. Found by one wave: lanes sum
-// equal groups of sequences, the group's sequences are then looked at.
+// holds its first unit, that unit's place there, and the length of a full run. Found by
+// one wave: lanes sum equal groups of sequences, the group's sequences are then looked at.
 DEVINL int find_run(const int* seq_lens, int window, int u, int B, int run,
-                    int runs, int* seq, int* at) {
+                    int runs, int* seq, int* at, int* per_run) {
   const int lane = threadIdx.x & 63;
   const int per_lane = (B + 63) / 64;
   int n = 0;
@@ -189,6 +194,7 @@ DEVINL int find_run(const int* seq_lens, int window, int u, int B, int run,
   const int sum = scan64(n);
   const int total = __shfl(sum, 63, WAVE_SIZE);
   const int per = run_length(total, runs);
+  *per_run = per;
   const int begin = run * per;
   *seq = 0;
   *at = 0;
@@ -303,7 +309,7 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
   const int BS = 1 << bs_shift;
 
   // ---- this workgroup's run of units ---------------------------------------------
-  int seq, at, todo;  // sequence, unit of it, units left
+  int seq, at, todo, per = 1;  // sequence, unit of it, units left; of a full run
   if (tmp_acc == nullptr) {
     seq = blockIdx.y;
     at = 0;
@@ -313,8 +319,9 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
         *reinterpret_cast<uint2*>(out + ((size_t)seq * Hq + hk * G) * D + e * 4) =
             make_uint2(0, 0);
   } else {
-    todo = find_run(seq_lens, window, U, B, blockIdx.y, gridDim.y, &seq, &at);
+    todo = find_run(seq_lens, window, U, B, blockIdx.y, gridDim.y, &seq, &at, &per);
   }
+  int done = 0;  // units of the run so far
   seq = __builtin_amdgcn_readfirstlane(seq);
   at = __builtin_amdgcn_readfirstlane(at);
   todo = __builtin_amdgcn_readfirstlane(todo);
@@ -356,6 +363,9 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
       continue;
     }
     const int t0 = at, t1 = min(units, at + todo);
+    if (tmp_acc != nullptr && t0 == 0 && hk == 0 && tid == 0)
+      part_runs(tmp_ml, gridDim.y, B, Hq)[seq] =
+          make_int2(blockIdx.y, blockIdx.y + (done + units - 1) / per);
     const int unit0 = lo / U;
     // constant memory: read by the scalar unit, no vector load among the copies
     const auto* btab = (const __attribute__((address_space(4))) int*)(
@@ -641,13 +651,20 @@ __global__ __launch_bounds__(W * 64, W > 4 ? 1 : 2) void paged_decode_kernel(
     }
     __syncthreads();
     todo -= t1 - t0;
+    done += t1 - t0;
     ++seq;
     at = 0;
   }
 }
 
 // Adds up the parts of the sequences that several runs share: a workgroup a
-// sequence and key/value head, groups of G D / 4 threads share the parts.
+// sequence and key/value head, groups of G D / 4 threads share the parts. What bounds it:
+// one round trip after the other, for the sequence's runs, which its first run has left,
+// for the maxima and sums, beside which a thread's first parts are on their way. us of it,
+// the runs found from the lengths again and a round trip for each / so: 128 sequences of
+// up to 4,096, 32 heads over 8 of 128 7.0 / 5.6; 200 of up to 3,001, 64 over 8 of 64 8.7 /
+// 5.8; one of 32,000, 64 over 8 of 128 7.7 / 7.2. Eight parts ahead 6.2 for the two that
+// most sequences have.
 template <int D>
 __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
     uint16_t* __restrict__ out, const float* __restrict__ tmp_acc,
@@ -657,26 +674,14 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
   const int seq = blockIdx.y, hk = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int Hq = Hk * G;
-  int total = 0, first = 0;  // units of all sequences, of those before this one
-  for (int b = lane; b < B; b += 64) {
-    const int n = units_of(seq_lens[b], window, u);
-    total += n;
-    first += b < seq ? n : 0;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    total += __shfl_xor(total, o, WAVE_SIZE);
-    first += __shfl_xor(first, o, WAVE_SIZE);
-  }
-  const int units = units_of(seq_lens[seq], window, u);
-  if (units == 0) {  // no tokens: zeros
+  const int2 range = part_runs(const_cast<float*>(tmp_ml), runs, B, Hq)[seq];
+  if (units_of(seq_lens[seq], window, u) == 0) {  // no tokens: zeros
     for (int e = tid; e < G * (D / 4); e += 256)
       *reinterpret_cast<uint2*>(out + ((size_t)seq * Hq + hk * G) * D + e * 4) =
           make_uint2(0, 0);
     return;
   }
-  const int per = run_length(total, runs);
-  const int r0 = first / per, r1 = (first + units - 1) / per;
+  const int r0 = range.x, r1 = range.y;
   if (r0 == r1) return;  // finished by its run
 
   extern __shared__ float wt[];  // [G][runs]
@@ -684,15 +689,30 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
   __shared__ f32x4v sums[256];
   const int parts = r1 - r0 + 1;
   const size_t row0 = ((size_t)r0 + seq) * Hq + hk * G;
+  const int per_part = G * (D / 4);
+  const int groups = max(1, 256 / per_part);
+  const int grp = tid / per_part;
+  const int mine = groups > 1 ? grp : 0;
+  constexpr int AHEAD = 4;
+  f32x4v ahead[AHEAD];
+  {
+    const int e = min(groups > 1 ? tid % per_part : tid, per_part - 1);
+    const float* src = tmp_acc + (row0 + e / (D / 4)) * D + e % (D / 4) * 4;
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)  // past the last one that one again
+      ahead[i] = *reinterpret_cast<const f32x4v*>(
+          src + (size_t)min(mine + i * groups, parts - 1) * Hq * D);
+  }
   for (int g = tid >> 6; g < G; g += 4) {  // a wave a head
-    float M = kLowest, l = 0.f;
-    for (int r = lane; r < parts; r += 64)
-      M = fmaxf(M, tmp_ml[(row0 + (size_t)r * Hq + g) * 2]);
+    const f32x2v* ml = reinterpret_cast<const f32x2v*>(tmp_ml) + row0 + g;
+    const f32x2v first = ml[(size_t)min(lane, parts - 1) * Hq];
+    float M = first[0], l = 0.f;
+    for (int r = lane + 64; r < parts; r += 64) M = fmaxf(M, ml[(size_t)r * Hq][0]);
     M = wave_reduce_max(M);
     for (int r = lane; r < parts; r += 64) {
-      const float* ml = tmp_ml + (row0 + (size_t)r * Hq + g) * 2;
-      const float w = __builtin_amdgcn_exp2f(ml[0] - M);
-      l += ml[1] * w;
+      const f32x2v v = r < 64 ? first : ml[(size_t)r * Hq];
+      const float w = __builtin_amdgcn_exp2f(v[0] - M);
+      l += v[1] * w;
       wt[g * runs + r] = w;
     }
     l = wave_reduce_sum(l);
@@ -702,9 +722,6 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
                                      : 0.f);
   }
   __syncthreads();
-  const int per_part = G * (D / 4);
-  const int groups = max(1, 256 / per_part);
-  const int grp = tid / per_part;
   for (int e0 = 0; e0 < per_part; e0 += 256) {
     const int e = groups > 1 ? tid % per_part : e0 + tid;
     const bool on = e < per_part && grp < groups;
@@ -712,8 +729,13 @@ __global__ __launch_bounds__(256) void paged_decode_reduce_kernel(
     f32x4v s = {};
     if (on) {
       const float* src = tmp_acc + (row0 + g) * D + d;
-#pragma unroll 4
-      for (int r = groups > 1 ? grp : 0; r < parts; r += groups)
+      int r = mine;
+      if (e0 == 0)
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i, r += groups)
+          if (r < parts) s += ahead[i] * wt[g * runs + r];
+#pragma unroll 8
+      for (; r < parts; r += groups)
         s += *reinterpret_cast<const f32x4v*>(src + (size_t)r * Hq * D) * wt[g * runs + r];
     }
     if (groups > 1) {

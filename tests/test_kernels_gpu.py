@@ -546,3 +546,42 @@ def test_rope_and_cache_pieces(T, Hq, Hk, D, rot, BS, fp8, start, neox):
         got.append([t.contiguous().view(torch.uint8) for t in (q, kc, vc)])
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hk,d,lens", [
+    (7, 1, 64, [40000]),                   # more parts than lanes
+    (16, 1, 128, [5000, 0, 3000, 33]),     # more threads a part than there are
+    (8, 8, 128, [2100] * 5),               # one head a group, parts shared by groups
+    (64, 8, 64, [1, 3001, 2048, 129, 900] * 13),  # runs that meet sequences
+])
+def test_decode_attention_parts(hq, hk, d, lens):
+    """The sums of sequences that several workgroups share, each found once."""
+    from parallax_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(5)
+    bs, pages = 32, [(n + 31) // 32 for n in lens]
+    ids = torch.randperm(sum(pages), generator=g, device="cuda").int()
+    bt = torch.zeros(len(lens), max(pages), dtype=torch.int32, device="cuda")
+    at = 0
+    for i, c in enumerate(pages):
+        bt[i, :c] = ids[at:at + c]
+        at += c
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    q, k, v = mk(len(lens), hq, d), mk(at, hk, bs, d), mk(at, hk, d, bs)
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = ops.paged_attention_decode(q, k, v, bt, sl, d ** -0.5, max_seq_len=max(lens))
+    again = ops.paged_attention_decode(q, k, v, bt, sl, d ** -0.5, max_seq_len=max(lens))
+    assert torch.equal(out, again)
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        p = bt[i, :pages[i]].long()
+        kk = k[p].transpose(1, 2).flatten(0, 1)[:n].double()
+        vv = v[p].permute(0, 3, 1, 2).flatten(0, 1)[:n].double()
+        qq = q[i].double().view(hk, hq // hk, d)
+        w = (torch.bmm(qq, kk.permute(1, 2, 0).contiguous()) * d ** -0.5).softmax(-1)
+        want = torch.bmm(w, vv.transpose(0, 1).contiguous()).view(hq, d)
+        err = (out[i].double() - want).norm() / want.norm()
+        # weights and results are rounded to bf16: 2^-9 at most each
+        assert err < 2 * 2 ** -9, (i, n, float(err))
