@@ -85,8 +85,8 @@ void launch_moe_few_down(float*, const void*, const float*, const void*, const f
 int moe_tile_rows(int, int, int, bool);
 int64_t moe_route_scratch(int, int);
 int moe_max_tiles(int, int, int);
-void launch_moe_route(int*, void*, int*, int*, const int64_t*, int, int, int,
-                      hipStream_t);
+void launch_moe_route(int*, void*, int*, int*, const int64_t*, int, int, int, void*,
+                      float*, const void*, int, int, hipStream_t);
 void launch_moe_gate_up(void*, const void*, const float*, const void*,
                         const float*, const int*, const void*, const int*,
                         const float*, const void*, int, int, int, int, int,
@@ -793,7 +793,6 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
     tiles = ws.data_ptr<int>();
     n_tiles = tiles + 4 * (int64_t)max_tiles;
     perm = n_tiles + 4;
-    launch_moe_route(perm, tiles, n_tiles, perm + n, ids, n, E, tm, stream);
   }
 
   torch::Tensor xq, xs, hq, hs;
@@ -801,10 +800,15 @@ static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
   if (fp8) {
     xq = torch::empty({T, H}, bopts);
     xs = torch::empty({T}, fopts);
-    launch_quantize_fp8_rows(xq.data_ptr(), xs.data_ptr<float>(), xp, T, H,
-                             stream);
-    xp = xq.data_ptr();
+    if (few)
+      launch_quantize_fp8_rows(xq.data_ptr(), xs.data_ptr<float>(), xp, T, H,
+                               stream);
   }
+  if (!few)
+    launch_moe_route(perm, tiles, n_tiles, perm + n, ids, n, E, tm,
+                     fp8 ? xq.data_ptr() : nullptr, fp8 ? xs.data_ptr<float>() : nullptr,
+                     xp, T, H, stream);
+  if (fp8) xp = xq.data_ptr();
   torch::Tensor h = torch::empty({n, I}, x.options());
   const float* gus = fp8 ? w_gu_scale.data_ptr<float>() : nullptr;
   const float* ds = fp8 ? w_down_scale.data_ptr<float>() : nullptr;

@@ -26,6 +26,48 @@
 typedef float f32x16v __attribute__((ext_vector_type(16)));
 typedef unsigned long long u64;
 
+// ---- activations to fp8 (OCP e4m3), one scale a row --------------------------------
+
+#define FP8_MAX 448.f
+
+// Row `row` by 256 threads, tid of them; lds: four floats of theirs. The whole
+// workgroup calls it, on: whether there is such a row.
+DEVINL void quantize_row(uint8_t* out, float* scales, const uint16_t* x, int row,
+                         int C, int tid, float* lds, bool on) {
+  const uint16_t* xr = x + (size_t)row * C;
+  uint8_t* orow = out + (size_t)row * C;
+  const int end = on ? C : 0;
+  float amax = 1e-8f;
+  for (int c = tid * 8; c < end; c += 2048) {
+    bf16x8 v = load_bf16x8(xr + c);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(bf16x8_get(v, i)));
+  }
+  amax = wave_reduce_max(amax);
+  if ((tid & 63) == 0) lds[tid >> 6] = amax;
+  __syncthreads();
+  amax = fmaxf(fmaxf(lds[0], lds[1]), fmaxf(lds[2], lds[3]));
+  if (on && tid == 0) scales[row] = amax / FP8_MAX;
+  const float inv = FP8_MAX / amax;
+  for (int c = tid * 8; c < end; c += 2048) {
+    bf16x8 v = load_bf16x8(xr + c);
+    uint64_t qv = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      qv |= (uint64_t)f32_to_fp8_e4m3(bf16x8_get(v, i) * inv) << (8 * i);
+    *reinterpret_cast<uint64_t*>(orow + c) = qv;
+  }
+}
+
+__global__ __launch_bounds__(256) void quantize_fp8_rows_kernel(
+    uint8_t* __restrict__ out,      // [R, C]
+    float* __restrict__ scales,     // [R] dequant scale (amax/448)
+    const uint16_t* __restrict__ x, // [R, C] bf16
+    const int C) {
+  __shared__ float lds[4];
+  quantize_row(out, scales, x, blockIdx.x, C, threadIdx.x, lds, true);
+}
+
 // ---- routing ------------------------------------------------------------------
 // perm [n], tiles [max_tiles] as (expert, first row, end of the expert's rows,
 // -), n_tiles [1]. A decode step has a few hundred choices: one workgroup and
@@ -87,17 +129,36 @@ __global__ __launch_bounds__(ROUTE_THREADS) void moe_count_kernel(
     counts[(size_t)blockIdx.x * E + e] = lds[e];
 }
 
+// Rows that are quantised for the experts, four a workgroup behind those that route:
+// neither needs the other, and a decode step's launch costs more than either. us of a
+// call, a launch each / in one: 16 experts of 1024 x 512, 120 tokens 26.0 / 23.6, 849
+// tokens 37.2 / 34.2; 32 of 2048 x 1024, 71 tokens 45.3 / 42.9, 294 65.5 / 63.0; 128 of
+// 2048 x 768, 6,000 tokens 487 / 485; 256 of 7168 x 2048, 10 tokens 382 / 380.
+struct QuantizeRows {
+  uint8_t* out;        // [T, C], null: none
+  float* scales;       // [T]
+  const uint16_t* x;   // [T, C]
+  int T, C;
+};
+
 template <bool LDS>
 __global__ __launch_bounds__(ROUTE_THREADS) void moe_route_kernel(
     int* __restrict__ perm, int4* __restrict__ tiles, int* __restrict__ n_tiles,
     int* __restrict__ counts, const int64_t* __restrict__ ids,
-    const int n, const int E, const int tm) {
+    const int n, const int E, const int tm, const int parts, const QuantizeRows rows) {
   extern __shared__ int lds[];
+  if ((int)blockIdx.x >= parts) {
+    __shared__ float largest[ROUTE_THREADS / 64];
+    const int grp = threadIdx.x >> 8;
+    const int row = ((int)blockIdx.x - parts) * (ROUTE_THREADS / 256) + grp;
+    quantize_row(rows.out, rows.scales, rows.x, row, rows.C, threadIdx.x & 255,
+                 largest + grp * 4, row < rows.T);
+    return;
+  }
   int* cur = LDS ? lds : counts;  // counters, then every expert's next place
   __shared__ int wave_rows[16], wave_tiles[16];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wid = tid >> 6;
-  const int parts = gridDim.x;
   const int begin = parts > 1 ? blockIdx.x * ROUTE_PART : 0;
   const int end = parts > 1 ? min(n, begin + ROUTE_PART) : n;
   if (parts == 1) {
@@ -902,42 +963,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
   }
 }
 
-// ---- activations to fp8 (OCP e4m3), one scale a row --------------------------------
-
-#define FP8_MAX 448.f
-
-__global__ __launch_bounds__(256) void quantize_fp8_rows_kernel(
-    uint8_t* __restrict__ out,      // [R, C]
-    float* __restrict__ scales,     // [R] dequant scale (amax/448)
-    const uint16_t* __restrict__ x, // [R, C] bf16
-    const int C) {
-  const int row = blockIdx.x;
-  const uint16_t* xr = x + (size_t)row * C;
-  uint8_t* orow = out + (size_t)row * C;
-  float amax = 1e-8f;
-  for (int c = threadIdx.x * 8; c < C; c += blockDim.x * 8) {
-    bf16x8 v = load_bf16x8(xr + c);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(bf16x8_get(v, i)));
-  }
-  __shared__ float lds[8];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  amax = wave_reduce_max(amax);
-  if (lane == 0) lds[wid] = amax;
-  __syncthreads();
-  amax = fmaxf(fmaxf(lds[0], lds[1]), fmaxf(lds[2], lds[3]));
-  if (threadIdx.x == 0) scales[row] = amax / FP8_MAX;
-  const float inv = FP8_MAX / amax;
-  for (int c = threadIdx.x * 8; c < C; c += blockDim.x * 8) {
-    bf16x8 v = load_bf16x8(xr + c);
-    uint64_t qv = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      qv |= (uint64_t)f32_to_fp8_e4m3(bf16x8_get(v, i) * inv) << (8 * i);
-    *reinterpret_cast<uint64_t*>(orow + c) = qv;
-  }
-}
-
 extern "C" void launch_quantize_fp8_rows(
     void* out, float* scales, const void* x, int R, int C,
     hipStream_t stream) {
@@ -1019,20 +1044,24 @@ extern "C" int64_t moe_route_scratch(int n, int E) {
   return parts > 1 || E > ROUTE_LDS ? (int64_t)parts * E : 0;
 }
 
+// xq not null: x's rows are quantised too
 extern "C" void launch_moe_route(int* perm, void* tiles, int* n_tiles,
                                  int* counts, const int64_t* ids, int n, int E,
-                                 int tm, hipStream_t stream) {
+                                 int tm, void* xq, float* xs, const void* x, int T,
+                                 int H, hipStream_t stream) {
   const int parts = route_parts(n, E);
+  const QuantizeRows rows{(uint8_t*)xq, xs, (const uint16_t*)x, T, H};
+  const int more = xq != nullptr ? ceil_div(T, ROUTE_THREADS / 256) : 0;
   if (E > ROUTE_LDS) {
-    moe_route_kernel<false><<<1, ROUTE_THREADS, 0, stream>>>(
-        perm, (int4*)tiles, n_tiles, counts, ids, n, E, tm);
+    moe_route_kernel<false><<<1 + more, ROUTE_THREADS, 0, stream>>>(
+        perm, (int4*)tiles, n_tiles, counts, ids, n, E, tm, 1, rows);
     return;
   }
   if (parts > 1)
     moe_count_kernel<<<parts, ROUTE_THREADS, E * sizeof(int), stream>>>(
         counts, ids, n, E);
-  moe_route_kernel<true><<<parts, ROUTE_THREADS, E * sizeof(int), stream>>>(
-      perm, (int4*)tiles, n_tiles, counts, ids, n, E, tm);
+  moe_route_kernel<true><<<parts + more, ROUTE_THREADS, E * sizeof(int), stream>>>(
+      perm, (int4*)tiles, n_tiles, counts, ids, n, E, tm, parts, rows);
 }
 
 extern "C" void launch_moe_gate_up(

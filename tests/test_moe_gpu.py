@@ -230,6 +230,33 @@ def test_moe_tiles(T, E, k, H, I, fp8):
     assert ops.fused_moe_forward(x[:0], gu, dn, ids[:0], w[:0]).shape == (0, H)
 
 
+@pytest.mark.parametrize("T,E,k,H", [
+    (41, 5, 2, 96),         # rows that do not fill the last workgroup
+    (47, 5, 2, 2080),       # longer than its threads' first pass
+    (5001, 5, 2, 96),       # beside choices that are counted in parts
+    (47, 8200, 2, 32),      # counters of experts that do not fit the LDS
+])
+def test_moe_rows_quantised_beside_the_routing(T, E, k, H):
+    """Rows of other magnitudes and one of zeros: were every value of a row's h moved by
+    one e4m3 step, its result would move by 2^-3 at most."""
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    x = torch.randn(T, H, generator=g, device="cuda")
+    x = (x * 2.0 ** (torch.arange(T, device="cuda") % 13 - 6)[:, None]).bfloat16()
+    x[3] = 0
+    gu = (torch.randn(E, 128, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, 64, generator=g, device="cuda") / 8).bfloat16()
+    ids = torch.rand(T, min(E, 40), generator=g, device="cuda").topk(k, dim=-1).indices
+    ids = ids + (E - min(E, 40))
+    w = torch.rand(T, k, generator=g, device="cuda")
+    qg, sg = ops.quantize_fp8_weight(gu)
+    qd, sd = ops.quantize_fp8_weight(dn)
+    got = ops.fused_moe_forward_fp8(x, qg, sg, qd, sd, ids, w)
+    first = E - min(E, 40)  # the oracle goes through the experts that are chosen
+    want = _experts64(x, (qg[first:].double() * sg[first:, :, None]),
+                      qd[first:].double() * sd[first:, :, None], ids - first, w, fp8=True)
+    assert ((got - want).norm(dim=1) <= 2 ** -3 * want.norm(dim=1)).all()
+
+
 @pytest.mark.parametrize("H,I,fp8", [
     (96, 96, False),      # a stage and a half, then half a stage
     (704, 544, False),    # 11 and 8.5 stages; 544 features: blocks cut by the end
