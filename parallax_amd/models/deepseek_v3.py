@@ -236,25 +236,31 @@ class DeepseekV3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, x, residual, meta, rope_cache):
+        return self.run(x, residual, meta, rope_cache)
+
+    forward.is_run = True
+
+    def run(self, x, residual, meta, rope_cache, normed: bool = False,
+            opens: bool = False):
+        """As LlamaDecoderLayer.run."""
         if residual is None:
             residual = x
             x = self.input_layernorm(x)
-        else:
+        elif not normed:
             x, residual = self.input_layernorm(x, residual)
         attn = self.self_attn
         if x.shape[0] <= ops.SKINNY_GEMM_MAX_M and plain_call(
                 attn, MLAAttention.forward):
             y = attn.attend(x, meta, rope_cache)
             fused = project_norm_mlp(attn.o_proj, y, residual,
-                                     self.post_attention_layernorm, self.mlp)
+                                     self.post_attention_layernorm, self.mlp, opens)
             if fused is not None:
                 return fused
             x = attn.o_proj(y)
         else:
             x = attn(x, meta, rope_cache)
         x, residual = self.post_attention_layernorm(x, residual)
-        x = self.mlp(x)
-        return x, residual
+        return (self.mlp.open_rows(x) if opens else self.mlp(x)), residual
 
 
 @register_model("DeepseekV3ForCausalLM", "DeepseekV2ForCausalLM", "KimiK2ForCausalLM")

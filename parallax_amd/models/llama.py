@@ -61,11 +61,11 @@ def norm_project(norm: nn.Module, proj: nn.Module, x: torch.Tensor,
 
 
 def project_norm_mlp(proj: nn.Module, y: torch.Tensor, residual: torch.Tensor,
-                     norm: nn.Module, mlp: nn.Module):
+                     norm: nn.Module, mlp: nn.Module, opens: bool = False):
     """(mlp(norm(proj(y), residual)), the residual then), the projection's parts added
-    up by the norm's launch, which also finds the scale of an fp8 MLP's input. None
-    where there is no kernel for it, for a residual of rows apart, which the norm refuses,
-    and for modules that are more than these."""
+    up by the norm's launch, which also finds the scale of an fp8 MLP's input; opens: of
+    the MLP what open_rows() gives. None where there is no kernel for it, for a residual
+    of rows apart, which the norm refuses, and for modules that are more than these."""
     if not (parts_of(proj, y.shape[0]) and plain_call(norm, RMSNorm.forward)
             and residual.is_contiguous()):
         return None
@@ -74,7 +74,22 @@ def project_norm_mlp(proj: nn.Module, y: torch.Tensor, residual: torch.Tensor,
     if fused is None:
         return None
     x, scale, residual = fused
+    if opens:
+        return mlp.open_rows(x, scale), residual
     return (mlp.from_fp8(x, scale) if quantize else mlp(x)), residual
+
+
+def runs_as_written(layer: nn.Module) -> bool:
+    """Whether calling the layer is its run(), whose result nothing else sees."""
+    forward = type(layer).forward
+    return getattr(forward, "is_run", False) and plain_call(layer, forward)
+
+
+def opens_mlp(layer: nn.Module, rows: int) -> bool:
+    """Whether the launch behind the layer can add up its MLP's last product."""
+    down = getattr(layer.mlp, "down_proj", None)
+    return plain_call(layer.mlp, LlamaMLP.forward) and parts_of(
+        down, rows) and down.product_alone()
 
 
 def parts_of(proj: nn.Module, rows: int) -> bool:
@@ -221,6 +236,15 @@ class LlamaMLP(nn.Module):
         fused = getattr(proj, "silu_and_mul", None)  # another module may stand there
         return self.down_proj(fused(x) if fused else ops.silu_and_mul(proj(x)))
 
+    def open_rows(self, x: torch.Tensor, scale: Optional[torch.Tensor] = None):
+        """forward() up to its last product: (rows, their scale or None). scale: x is fp8
+        values with it."""
+        proj = self.gate_up_proj
+        if scale is not None:
+            return ops.silu_and_mul_fp8(proj._linear(x, scale))
+        fused = getattr(proj, "silu_and_mul", None)
+        return fused(x) if fused else ops.silu_and_mul(proj(x)), None
+
     def from_fp8(self, x: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
         """forward() of rows that are fp8 values with one scale, by fp8 weights."""
         return self.down_proj.from_fp8(
@@ -236,10 +260,19 @@ class LlamaDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, x, residual, meta: ForwardMeta, rope_cache):
+        return self.run(x, residual, meta, rope_cache)
+
+    forward.is_run = True
+
+    def run(self, x, residual, meta: ForwardMeta, rope_cache, normed: bool = False,
+            opens: bool = False):
+        """normed: x is the input norm's result and residual what it added up. opens: of
+        the MLP what open_rows() gives, in place of its result."""
         # sizes first: a prompt's layers wait for the host
         rows = x.shape[0]
-        if rows > ops.SKINNY_GEMM_MAX_M or rows > ops.NORM_LINEAR_MAX_M and not parts_of(
-                getattr(self.self_attn, "o_proj", None), rows):
+        if not (normed or opens) and (
+                rows > ops.SKINNY_GEMM_MAX_M or rows > ops.NORM_LINEAR_MAX_M
+                and not parts_of(getattr(self.self_attn, "o_proj", None), rows)):
             if residual is None:
                 residual = x
                 x = self.input_layernorm(x)
@@ -252,34 +285,36 @@ class LlamaDecoderLayer(nn.Module):
         fused = None
         plain = plain_call(attn, LlamaAttention.forward) and (
             type(attn)._project_out is LlamaAttention._project_out)
-        if plain:
+        if plain and not normed:
             fused = norm_project(self.input_layernorm, attn.qkv_proj, x, residual)
         if fused is not None:
             qkv, residual = fused
         else:
-            if residual is None:
-                residual = x
-                x = self.input_layernorm(x)
-            else:
-                x, residual = self.input_layernorm(x, residual)
+            if not normed:
+                x, residual = self._input_norm(x, residual)
             qkv = attn.qkv_proj(x) if plain else None
         if plain:
             y = attn.attend(qkv, x, meta, rope_cache, project=False)
             fused = project_norm_mlp(attn.o_proj, y, residual,
-                                     self.post_attention_layernorm, mlp)
+                                     self.post_attention_layernorm, mlp, opens)
             if fused is not None:
                 return fused
             x = attn.o_proj(y)
         else:
             x = attn(x, meta, rope_cache)
-        if plain_call(mlp, LlamaMLP.forward):
+        if not opens and plain_call(mlp, LlamaMLP.forward):
             fused = norm_project(self.post_attention_layernorm, mlp.gate_up_proj, x,
                                  residual, gated=True)
             if fused is not None:
                 x, residual = fused
                 return mlp.down_proj(x), residual
         x, residual = self.post_attention_layernorm(x, residual)
-        return mlp(x), residual
+        return (mlp.open_rows(x) if opens else mlp(x)), residual
+
+    def _input_norm(self, x, residual):
+        if residual is None:
+            return self.input_layernorm(x), x
+        return self.input_layernorm(x, residual)
 
 
 def stack_in_one(layers, hidden: torch.Tensor, meta: ForwardMeta,
@@ -393,6 +428,11 @@ class LlamaShardModel(nn.Module):
         fused = stack_in_one(self.layers, hidden, meta, self.rope_cache)
         if fused is not None:
             hidden, residual = fused
+        elif hidden.dim() == 2 and (
+                ops.NORM_LINEAR_MAX_M < hidden.shape[0] <= ops.SKINNY_GEMM_MAX_M):
+            hidden, residual, done = self._few_rows(hidden, meta)
+            if done:
+                return hidden
         else:
             for layer in self.layers:
                 hidden, residual = layer(hidden, residual, meta, self.rope_cache)
@@ -404,6 +444,46 @@ class LlamaShardModel(nn.Module):
         elif residual is not None:
             hidden = hidden + residual
         return hidden
+
+    def _few_rows(self, hidden: torch.Tensor, meta: ForwardMeta):
+        """The layers of a few rows: (hidden, residual, whether hidden is what the forward
+        returns). The parts of an MLP's last product are added up by the launch of the
+        norm that follows, or of the sum behind the last layer, where both modules are
+        what they are here and nothing looks on."""
+        rows, residual, normed = hidden.shape[0], None, False
+        runs = [hidden.is_cuda and runs_as_written(x) for x in self.layers]
+        for i, layer in enumerate(self.layers):
+            last = i + 1 == len(self.layers)
+            if last:
+                norm = self.norm if self.is_last else None
+            else:
+                norm = self.layers[i + 1].input_layernorm if runs[i + 1] else None
+            follows = last and not self.is_last or (
+                norm is not None and plain_call(norm, RMSNorm.forward))
+            opens = runs[i] and follows and opens_mlp(layer, rows)
+            if not (normed or opens):
+                hidden, residual = layer(hidden, residual, meta, self.rope_cache)
+                continue
+            hidden, residual = layer.run(hidden, residual, meta, self.rope_cache, normed,
+                                         opens)
+            normed = False
+            if not opens:
+                continue
+            (rows_in, scale), down = hidden, layer.mlp.down_proj
+            weight = down.weight_fp8 if down.fp8 else down.weight
+            w_scale = down.weight_scale if down.fp8 else None
+            if norm is not None:
+                fused = ops.linear_norm(rows_in, weight, w_scale, residual, norm.weight,
+                                        norm.eps, x_scale=scale)
+                if fused is not None:
+                    hidden, residual, normed = fused[0], fused[2], True
+            else:
+                fused = ops.linear_add(rows_in, weight, w_scale, residual, x_scale=scale)
+                if fused is not None:
+                    hidden, normed = fused, True
+            if fused is None:
+                hidden = down(rows_in) if scale is None else down.from_fp8(rows_in, scale)
+        return hidden, residual, normed
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         assert self.is_last, "only the last shard computes logits"

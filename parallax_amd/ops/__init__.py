@@ -737,24 +737,43 @@ def product_has_parts(rows: int, weight: torch.Tensor) -> bool:
 def linear_norm(
     x: torch.Tensor, weight: torch.Tensor, w_scale: Optional[torch.Tensor],
     residual: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float,
-    quantize: bool = False,
+    quantize: bool = False, x_scale: Optional[torch.Tensor] = None,
 ) -> Optional[Tuple[torch.Tensor, Optional[torch.Tensor], Optional[torch.Tensor]]]:
     """(rmsnorm(linear(x, weight) + residual), its scale, linear(x, weight) + residual)
     of few rows, x and residual left as they are: the launch that adds up a product's
     parts normalises them too. quantize: the first as fp8 values with the scale, for
-    linear_fp8_quantized. weight is bf16, or fp8 with w_scale. None where the product has
-    no parts; no part of autograd."""
-    args = [t for t in (x, weight, residual, norm_weight) if t is not None]
-    if not x.is_cuda or x.dim() != 2 or SKINNY_GEMM_MAX_M < x.shape[0] or (
-            torch.is_grad_enabled() and any(t.requires_grad for t in args)):
+    linear_fp8_quantized. weight is bf16, or fp8 with w_scale; x_scale: x is fp8 values
+    with it. None where the product has no parts; no part of autograd."""
+    if not _adds_parts(x, weight, residual, norm_weight):
         return None
     none = x.new_empty(0)
     r = _require_ext("linear_norm").linear_norm(
-        x, weight, none if w_scale is None else w_scale,
+        x, none if x_scale is None else x_scale, weight,
+        none if w_scale is None else w_scale,
         none if residual is None else residual, norm_weight, eps, quantize)
     if r is None:
         return None
     return r[0], r[1] if quantize else None, None if residual is None else r[2]
+
+
+def _adds_parts(x: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
+    return x.is_cuda and x.dim() == 2 and x.shape[0] <= SKINNY_GEMM_MAX_M and not (
+        torch.is_grad_enabled() and any(
+            t.requires_grad for t in (x, *others) if t is not None))
+
+
+def linear_add(
+    x: torch.Tensor, weight: torch.Tensor, w_scale: Optional[torch.Tensor],
+    residual: torch.Tensor, x_scale: Optional[torch.Tensor] = None,
+) -> Optional[torch.Tensor]:
+    """linear(x, weight) + residual of few rows, the sum by the launch that adds up the
+    product's parts. Operands and None as linear_norm()."""
+    if not _adds_parts(x, weight, residual):
+        return None
+    none = x.new_empty(0)
+    return _require_ext("linear_add").linear_add(
+        x, none if x_scale is None else x_scale, weight,
+        none if w_scale is None else w_scale, residual)
 
 
 def linear_silu_and_mul(

@@ -129,6 +129,8 @@ void launch_quantize_fp8_tensor(void*, float*, uint32_t*, const void*, int64_t,
                                 bool, int, hipStream_t);
 void launch_skinny_norm(void*, void*, uint32_t*, const float*, const void*,
                         const void*, float, int, int, int, int64_t, hipStream_t);
+void launch_skinny_add(void*, const float*, const void*, int, int, int, int64_t,
+                       hipStream_t);
 int silu_and_mul_parts(int64_t, int);
 void launch_silu_and_mul_max(void*, uint32_t*, const void*, int64_t, int,
                              hipStream_t);
@@ -1157,27 +1159,25 @@ int64_t product_parts(int64_t M, int64_t N, int64_t row_bytes) {
   return splits > 1 ? splits : 0;
 }
 
-// rms_norm(x . w^T + residual) of few rows whose product is split over K: (the normed
-// rows, as fp8 values with their scale where quantize is set, else bf16 and an empty
-// scale; product + residual, empty without one). fp8 w takes bf16 x and its own scale.
-// None where there is no kernel or linear() has none.
-std::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> linear_norm(
-    torch::Tensor x, torch::Tensor w, torch::Tensor w_scale, torch::Tensor residual,
-    torch::Tensor norm, double eps, bool quantize) {
-  CHECK_GPU(x);
-  const bool fp8 = is_fp8(w), has_res = residual.numel() > 0;
+// The parts [splits, M, N] of x . w^T of few rows, for a launch that adds them up to rows
+// beside those of residual. fp8 w takes its own scale, and bf16 x or fp8 x with x_scale.
+// None where linear() has no parts, and for operands that no such launch takes.
+static std::optional<torch::Tensor> product_in_parts(
+    const torch::Tensor& x, const torch::Tensor& x_scale, const torch::Tensor& w,
+    const torch::Tensor& w_scale, const torch::Tensor& residual) {
+  const bool fp8 = is_fp8(w), has_res = residual.numel() > 0, ready = x_scale.numel() > 0;
   auto rows16 = [](const torch::Tensor& t) {
     return (uintptr_t)t.data_ptr() % 16 == 0 && t.stride(1) == 1;
   };
-  if (x.dim() != 2 || w.dim() != 2 || norm.dim() != 1 || x.numel() == 0 ||
-      w.numel() == 0 || x.size(1) != w.size(1) || !w.is_contiguous() ||
-      x.scalar_type() != at::kBFloat16 || norm.scalar_type() != at::kBFloat16 ||
-      (!fp8 && w.scalar_type() != at::kBFloat16))
+  if (x.dim() != 2 || w.dim() != 2 || x.numel() == 0 || w.numel() == 0 ||
+      x.size(1) != w.size(1) || !w.is_contiguous() ||
+      (!fp8 && w.scalar_type() != at::kBFloat16) ||
+      (ready ? !fp8 || !is_fp8(x) || x_scale.numel() != 1 ||
+                   x_scale.scalar_type() != at::kFloat || !rows16(x)
+             : x.scalar_type() != at::kBFloat16))
     return std::nullopt;
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  if (M > 128 || N > 8192 || N % 8 || K > INT_MAX / 2 || norm.size(0) != N ||
-      !norm.is_contiguous() || (uintptr_t)norm.data_ptr() % 16 || !rows16(w))
-    return std::nullopt;
+  if (M > 128 || N > 8192 || N % 8 || K > INT_MAX / 2 || !rows16(w)) return std::nullopt;
   if (has_res && (residual.dim() != 2 || residual.size(0) != M ||
                   residual.size(1) != N || !rows16(residual) ||
                   residual.stride(0) % 8 ||
@@ -1191,26 +1191,61 @@ std::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> linear_no
   if ((M - 1) * (fp8 ? K : x.stride(0) * 2) + 128 > UINT32_MAX) return std::nullopt;
   const int splits = product_parts(M, N, row_bytes);
   if (splits <= 1) return std::nullopt;
-  torch::Tensor x_scale, xq = x;
-  if (fp8) std::tie(xq, x_scale) = quantize_fp8_tensor(x);
+  torch::Tensor scale = x_scale, xq = x;
+  if (fp8 && !ready) std::tie(xq, scale) = quantize_fp8_tensor(x);
   auto part = torch::empty({splits, M, N}, x.options().dtype(at::kFloat));
   launch_skinny_split(nullptr, part.data_ptr<float>(), splits, xq.data_ptr(),
-                      w.data_ptr(), nullptr, fp8 ? x_scale.data_ptr<float>() : nullptr,
+                      w.data_ptr(), nullptr, fp8 ? scale.data_ptr<float>() : nullptr,
                       fp8 ? w_scale.data_ptr<float>() : nullptr, fp8, M, N, row_bytes,
                       xq.stride(0) * xq.element_size(), 0, false, cur_stream());
-  auto out = torch::empty({M, N}, x.options());
-  auto sum = has_res ? torch::empty({M, N}, x.options()) : x.new_empty({0});
+  return part;
+}
+
+// rms_norm(x . w^T + residual) of few rows whose product is split over K: (the normed
+// rows, as fp8 values with their scale where quantize is set, else bf16 and an empty
+// scale; product + residual, empty without one). None where there is no kernel or
+// linear() has none.
+std::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> linear_norm(
+    torch::Tensor x, torch::Tensor x_scale, torch::Tensor w, torch::Tensor w_scale,
+    torch::Tensor residual, torch::Tensor norm, double eps, bool quantize) {
+  CHECK_GPU(x);
+  if (w.dim() != 2 || norm.dim() != 1 || norm.scalar_type() != at::kBFloat16 ||
+      norm.size(0) != w.size(0) || !norm.is_contiguous() ||
+      (uintptr_t)norm.data_ptr() % 16)
+    return std::nullopt;
+  const auto part = product_in_parts(x, x_scale, w, w_scale, residual);
+  if (!part) return std::nullopt;
+  const bool has_res = residual.numel() > 0;
+  const int splits = part->size(0), M = part->size(1), N = part->size(2);
+  const auto bf16 = x.options().dtype(at::kBFloat16);
+  auto out = torch::empty({M, N}, bf16);
+  auto sum = torch::empty({has_res ? M : 0, N}, bf16);
   torch::Tensor top;
   if (quantize) top = torch::empty({M}, x.options().dtype(at::kInt));
   launch_skinny_norm(out.data_ptr(), has_res ? sum.data_ptr() : nullptr,
                      quantize ? (uint32_t*)top.data_ptr() : nullptr,
-                     part.data_ptr<float>(), has_res ? residual.data_ptr() : nullptr,
+                     part->data_ptr<float>(), has_res ? residual.data_ptr() : nullptr,
                      norm.data_ptr(), (float)eps, splits, M, N,
                      has_res ? residual.stride(0) : 0, cur_stream());
   if (!quantize)
     return std::make_tuple(out, x.new_empty({0}, at::kFloat), sum);
   auto [q, scale] = quantize_by_parts(out, top);
   return std::make_tuple(q, scale, sum);
+}
+
+// x . w^T + residual of few rows whose product is split over K; None as linear_norm.
+std::optional<torch::Tensor> linear_add(torch::Tensor x, torch::Tensor x_scale,
+                                        torch::Tensor w, torch::Tensor w_scale,
+                                        torch::Tensor residual) {
+  CHECK_GPU(x);
+  if (residual.numel() == 0) return std::nullopt;
+  const auto part = product_in_parts(x, x_scale, w, w_scale, residual);
+  if (!part) return std::nullopt;
+  const int splits = part->size(0), M = part->size(1), N = part->size(2);
+  auto out = torch::empty({M, N}, residual.options());
+  launch_skinny_add(out.data_ptr(), part->data_ptr<float>(), residual.data_ptr(), splits,
+                    M, N, residual.stride(0), cur_stream());
+  return out;
 }
 
 // mla_rope_and_cache of kv = x . kv_w^T, whose parts its launch adds up. None where
@@ -1337,6 +1372,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_stack_has", &decode_stack_has);
   m.def("quantize_fp8_tensor", &quantize_fp8_tensor);
   m.def("silu_and_mul_fp8", &silu_and_mul_fp8);
+  m.def("linear_add", &linear_add);
   m.def("linear_norm", &linear_norm);
   m.def("product_parts", &product_parts);
   m.def("mla_absorb", &mla_absorb);

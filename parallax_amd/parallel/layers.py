@@ -198,12 +198,16 @@ class RowParallelLinear(nn.Module, _Fp8WeightMixin):
         return self._reduce(ops.linear_fp8_quantized(x, scale, self.weight_fp8,
                                                      self.weight_scale))
 
+    def product_alone(self) -> bool:
+        """Whether the forward is a product and nothing more is done with it."""
+        return self.tp_size == 1 and self.bias is None and plain_call(
+            self, RowParallelLinear.forward)
+
     def then_norm(self, x: torch.Tensor, residual: torch.Tensor,
                   norm_weight: torch.Tensor, eps: float, quantize: bool):
         """ops.linear_norm of this projection, where nothing else is done with its
         result; None otherwise."""
-        if self.tp_size > 1 or self.bias is not None or not plain_call(
-                self, RowParallelLinear.forward):
+        if not self.product_alone():
             return None
         return ops.linear_norm(
             x, self.weight_fp8 if self.fp8 else self.weight,

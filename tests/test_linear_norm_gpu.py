@@ -192,3 +192,114 @@ def test_a_residual_of_rows_apart_is_refused(kind, T, first):
     layer = _layer(kind, False)
     with pytest.raises(RuntimeError, match="contiguous"):
         _step(layer, kind, T, first, lambda t: torch.cat([t, t], 1)[:, :WIDTH])
+
+
+def _shard(kind, fp8, last):
+    from parallax_amd.models import get_model_class
+    from parallax_amd.models.config import ModelConfig
+    kw = dict(vocab_size=64, hidden_size=WIDTH, num_layers=3, num_heads=56,
+              num_kv_heads=4, head_dim=128, intermediate_size=4096,
+              max_position_embeddings=256, eos_token_ids=[])
+    if kind == "mla":
+        kw.update(q_lora_rank=1536, kv_lora_rank=512, qk_nope_head_dim=128,
+                  qk_rope_head_dim=64, v_head_dim=128, num_kv_heads=56)
+    name = "DeepseekV3ForCausalLM" if kind == "mla" else "LlamaForCausalLM"
+    with torch.device("cuda"):
+        model = get_model_class(name)(ModelConfig(architecture=name, **kw), 0,
+                                      3 if last else 2).to(torch.bfloat16).eval()
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for p in model.parameters():
+        p.data.copy_(1 + 0.1 * torch.randn(p.shape, generator=g, device="cuda")
+                     if p.dim() == 1 else
+                     torch.randn(p.shape, generator=g, device="cuda") * p.shape[1] ** -0.5)
+    model.rope_cache = model.rope_cache.float()
+    if kind == "mla":
+        model.finalize_weights()
+    if fp8:
+        for layer in model.layers:
+            for m in list(layer.modules()):
+                if hasattr(m, "quantize_fp8"):
+                    m.quantize_fp8()
+    return model
+
+
+@pytest.mark.parametrize("kind,fp8", [("llama", False), ("llama", True), ("mla", False),
+                                      ("mla", True)])
+@pytest.mark.parametrize("last", [False, True])
+def test_layers_that_end_in_the_next_norm(kind, fp8, last, monkeypatch):
+    """The parts of an MLP's last product are added up by the next layer's norm, the
+    shard's norm or its last sum, and by a launch of their own where a hook looks on: the
+    same bits either way."""
+    from parallax_amd.server.kv_cache import KVCacheSpec, MLAKVCache, PagedKVCache
+    dev = torch.device("cuda")
+    model = _shard(kind, fp8, last)
+    n = len(model.layers)
+
+    def step(T):
+        g = torch.Generator(device="cuda").manual_seed(T)
+        if kind == "mla":
+            cache = MLAKVCache(n, 512, 64, 16, T, dev)
+            kept = cache.caches
+        else:
+            cache = PagedKVCache(KVCacheSpec(n, 4, 128, 16), T, dev)
+            kept = cache.k_caches + cache.v_caches
+        for c in kept:
+            c.copy_(torch.randn(c.shape, generator=g, device="cuda"))
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+        lens = [1 + i % 16 for i in range(T)]
+        meta = ForwardMeta(
+            is_prefill=False, positions=i32([n - 1 for n in lens]),
+            slot_mapping=torch.tensor([16 * i + n - 1 for i, n in enumerate(lens)],
+                                      device=dev),
+            block_tables=i32([[i] for i in range(T)]), seq_lens=i32(lens),
+            kv_cache=None if kind == "mla" else cache,
+            mla_cache=cache if kind == "mla" else None, max_seq_len=16, appends=True)
+        with torch.inference_mode():
+            return [model(_rand(g, T, WIDTH), meta)] + list(kept)
+
+    calls = []
+    for name in ("linear_norm", "linear_add"):
+        def spy(x, w, *args, of=getattr(ops, name), name=name, **kw):
+            out = of(x, w, *args, **kw)
+            if w.shape[1] == 4096 and out is not None:  # a down projection
+                calls.append(name)
+            return out
+        monkeypatch.setattr(ops, name, spy)
+    rows = (4, 5, 33, 128, 130)
+    want = [step(T) for T in rows]
+    # five rows' products have no parts, of more than 128 none has
+    few = [T for T in rows if ops.product_has_parts(
+        T, next(iter(model.layers)).mlp.down_proj.weight_fp8 if fp8
+        else next(iter(model.layers)).mlp.down_proj.weight)]
+    assert 33 in few and 4 not in few and 130 not in few
+    assert calls == (["linear_norm"] * (n - 1) + ["linear_norm" if last else "linear_add"]
+                     ) * len(few)
+    calls.clear()
+    for layer in model.layers:
+        layer.register_forward_hook(lambda m, a, out: None)
+    for T, w in zip(rows, want):
+        assert all(torch.equal(a, b) for a, b in zip(w, step(T))), T
+    assert not calls
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 7168, 16384), (33, 4096, 4096), (128, 8192, 8192)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_linear_add(M, N, K, fp8):
+    """The bits of the product and the sum apart; rows of a residual that lie apart."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w = _rand(g, M, K), _rand(g, N, K) * K ** -0.5
+    res = _rand(g, M, N + 8)[:, :N]
+    scale = None
+    if fp8:
+        scale = (w.float().abs().amax() / 448).reshape(1)
+        w = (w.float() / scale).to(torch.float8_e4m3fn)
+    if not ops.product_has_parts(M, w):
+        assert ops.linear_add(x, w, scale, res) is None
+        return
+    want = (ops.linear_fp8(x, w, scale) if fp8 else ops.linear(x, w)) + res
+    assert torch.equal(ops.linear_add(x, w, scale, res), want)
+    if fp8:
+        xq, xs = ops._require_ext("t").quantize_fp8_tensor(x)
+        assert torch.equal(ops.linear_add(xq, w, scale, res, x_scale=xs), want)
+        assert ops.linear_add(xq, w, scale, res) is None
+    assert ops.linear_add(x, w, scale, res[:, :8]) is None
