@@ -163,6 +163,12 @@ class MLAAttention(nn.Module):
             lens = [(n, first + n) for first, n in meta.portions]
         else:
             lens = list(zip(meta.query_lens.tolist(), meta.seq_lens.tolist()))
+        dense = getattr(self._prefill_sparse_mask, "__func__", None) is (
+            MLAAttention._prefill_sparse_mask)
+        if dense and ops.mla_prefill_paged(
+                out, q_nope, q_pe, cache, meta.block_tables, lens, self.w_uk, self.w_uv,
+                self.scale):
+            return out
         for i, (QL, L) in enumerate(lens):
             nb = (L + bs - 1) // bs
             entries = cache[meta.block_tables[i, :nb].long()].reshape(nb * bs, -1)[:L]

@@ -10,7 +10,7 @@ never "pass" on a Python fallback. On CPU the fp32 reference implementations run
 from __future__ import annotations
 
 import os
-from typing import List, Optional, Tuple
+from typing import List, Optional, Sequence, Tuple
 
 import torch
 
@@ -388,14 +388,38 @@ def mla_prefill_attention(
     whatever is idle, 64 on 40,000 2.1 / 1.5 and 128 on 40,000 2.2 / 2.7."""
     if not q_nope.is_cuda:
         return False
-    T, H = q_nope.shape[:2]
-    if T * min(H, 40) < 2048 and rows.shape[0] * max(H, 40) > 1 << 18:
+    if not _expansion_pays(*q_nope.shape[:2], rows.shape[0]):
         return False
     ext = _require_ext("mla_prefill_attention")
     return ext.mla_prefill_attention(
         out, q_nope, q_pe.contiguous(), rows.to(q_nope.dtype).contiguous(),
         w_uk, w_uv, scale,
     )
+
+
+def _expansion_pays(rows: int, heads: int, context: int) -> bool:
+    return rows * min(heads, 40) >= 2048 or context * max(heads, 40) <= 1 << 18
+
+
+def mla_prefill_paged(
+    out: torch.Tensor,           # [T, H, dv], written
+    q_nope: torch.Tensor,        # [T, H, dn]
+    q_pe: torch.Tensor,          # [T, H, dr]
+    cache: torch.Tensor,         # [NB, BS, r + dr]
+    block_tables: torch.Tensor,  # [B, max_blocks] int32
+    lens: Sequence[Tuple[int, int]],
+    w_uk: torch.Tensor,          # [H, dn, r]
+    w_uv: torch.Tensor,          # [H, dv, r]
+    scale: float,
+) -> bool:
+    """mla_prefill_attention of all requests at once, lens their (portion's rows, context
+    rows with them), read from the cache's pages. False: the caller goes through them one
+    by one, as for a cache or a length that this does not take."""
+    if not q_nope.is_cuda or not all(
+            _expansion_pays(n, q_nope.shape[1], context) for n, context in lens if n):
+        return False
+    return _require_ext("mla_prefill_paged").mla_prefill_paged(
+        out, q_nope, q_pe.contiguous(), cache, block_tables, lens, w_uk, w_uv, scale)
 
 
 def dsa_paged_attention_decode(

@@ -8,6 +8,8 @@
 #include <algorithm>
 #include <cstdlib>
 #include <optional>
+#include <utility>
+#include <vector>
 
 #define CHECK_GPU(x) TORCH_CHECK(x.is_cuda(), #x " must be on GPU")
 #define CHECK_CONTIG(x) TORCH_CHECK(x.is_contiguous(), #x " must be contiguous")
@@ -66,6 +68,11 @@ void launch_mla_paged_attention_decode(void*, const void*, const void*,
                                        int, float*, float*, const int*, int,
                                        bool, hipStream_t, bool*);
 int mla_decode_runs(int, int, int);
+int mla_prefill_max_portions();
+void launch_mla_prefill_paged(void*, const void*, const void*, void*, void*, void*, void*,
+                              void*, const void*, const int*, int, int, const void*,
+                              const void*, const int*, const int*, int, int, int, int64_t,
+                              int64_t, float, hipStream_t);
 void launch_mla_prefill_run(void*, float*, const void*, const void*, void*, void*,
                             void*, void*, const void*, const void*, const void*,
                             int, int, int, int, int, int, int64_t, int64_t, float,
@@ -740,6 +747,80 @@ bool mla_prefill_attention(torch::Tensor out, torch::Tensor q_nope,
   return true;
 }
 
+// Portions of requests over their contexts in cache [NB, BS, 576]: lens (rows, context
+// rows with them) of each, whose rows lie one behind the other in q and out and whose
+// pages are the rows of block_tables. False where there is no kernel.
+bool mla_prefill_paged(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
+                       torch::Tensor cache, torch::Tensor block_tables,
+                       std::vector<std::pair<int64_t, int64_t>> lens, torch::Tensor w_uk,
+                       torch::Tensor w_uv, double scale) {
+  CHECK_GPU(q_nope);
+  const int64_t T = q_nope.size(0), H = q_nope.size(1);
+  for (const auto& t : {out, q_nope, q_pe, cache, w_uk, w_uv}) {
+    if (t.dim() != 3 || t.scalar_type() != at::kBFloat16 ||
+        (uintptr_t)t.data_ptr() % 16 || t.device() != q_nope.device())
+      return false;
+  }
+  const int64_t BS = cache.size(1);
+  if (q_nope.size(2) != 128 || q_pe.size(2) != 64 || w_uk.size(1) != 128 ||
+      w_uv.size(1) != 128 || w_uk.size(2) != 512 || cache.size(2) != 576 || BS < 1 ||
+      BS > 1 << 20 || (BS & (BS - 1)))
+    return false;
+  if (q_nope.stride(2) != 1 || q_nope.stride(1) % 8 || q_nope.stride(0) % 8)
+    return false;
+  for (const auto& t : {out, q_pe, cache, w_uk, w_uv, block_tables})
+    if (!t.is_contiguous()) return false;
+  if (block_tables.dim() != 2 || block_tables.scalar_type() != at::kInt ||
+      block_tables.device() != q_nope.device() ||
+      (int64_t)lens.size() > block_tables.size(0))
+    return false;
+  TORCH_CHECK(q_pe.size(0) == T && q_pe.size(1) == H && out.size(0) == T &&
+              out.size(1) == H && out.size(2) == 128 && w_uk.size(0) == H &&
+              w_uv.size(0) == H && w_uv.size(2) == 512);
+  if (H == 0) return true;
+  // 1 GB of expanded keys and values a pair of launches; a longer context goes by runs
+  const int64_t run = std::max<int64_t>(128, ((1 << 20) / H) & ~127);
+  struct Request { int64_t rows, context, first, seq; };
+  std::vector<Request> all;
+  int64_t at = 0;
+  for (size_t i = 0; i < lens.size(); ++i) {
+    const auto [rows, context] = lens[i];
+    if (rows < 0 || context < rows || context > run ||
+        (context + BS - 1) / BS > block_tables.size(1))
+      return false;
+    if (rows > 0) all.push_back({rows, context, at, (int64_t)i});
+    at += rows;
+  }
+  if (at > T) return false;
+  std::stable_sort(all.begin(), all.end(), [](const Request& a, const Request& b) {
+    return a.context < b.context;
+  });
+  const size_t most = mla_prefill_max_portions();
+  for (size_t i = 0; i < all.size();) {
+    std::vector<int> sizes, starts;
+    int64_t cap = 0;
+    size_t j = i;
+    for (; j < all.size() && j - i < most; ++j) {
+      const int64_t more = (all[j].context + 127) & ~127;
+      if (j > i && cap + more > run) break;
+      cap += more;
+      sizes.insert(sizes.end(), {(int)all[j].rows, (int)all[j].context});
+      starts.insert(starts.end(), {(int)all[j].first, (int)all[j].seq});
+    }
+    const int64_t part = H * cap * 128;
+    auto kv = torch::empty({4 * part + cap * 64}, q_nope.options());
+    uint16_t* p = (uint16_t*)kv.data_ptr();
+    launch_mla_prefill_paged(
+        out.data_ptr(), q_nope.data_ptr(), q_pe.data_ptr(), p, p + part, p + 2 * part,
+        p + 3 * part, p + 4 * part, cache.data_ptr(), block_tables.data_ptr<int>(),
+        block_tables.size(1), __builtin_ctzll(BS), w_uk.data_ptr(), w_uv.data_ptr(),
+        sizes.data(), starts.data(), (int)(j - i), H, cap, q_nope.stride(0),
+        q_nope.stride(1), (float)scale, cur_stream());
+    i = j;
+  }
+  return true;
+}
+
 // Routed experts of x [T, H]: bf16, or fp8 (W8A8) with w_gu_scale / w_down_scale
 // given. Returns fp32 [T, H].
 static torch::Tensor moe_layer(torch::Tensor x, torch::Tensor w_gu,
@@ -1386,6 +1467,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("msa_topk_tokens", &msa_topk_tokens);
   m.def("mla_paged_attention_decode", &mla_paged_attention_decode);
   m.def("mla_prefill_attention", &mla_prefill_attention);
+  m.def("mla_prefill_paged", &mla_prefill_paged);
   m.def("prefill_attention", &prefill_attention);
   m.def("rmsnorm", &rmsnorm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);

@@ -1,4 +1,4 @@
-// MLA prefill for gfx950: a request's prompt portion against its context.
+// MLA prefill for gfx950: prompt portions of requests against their contexts.
 //
 //   mla_expand   keys k = latent . W_uk[h]^T and values v = latent . W_uv[h]^T of
 //                a run of context rows, for every head, to bf16 pairs (below)
@@ -25,6 +25,8 @@
 // 2,500 rows at 128 heads: expansion 230 us, attention 500 us; the fp32 torch
 // operations in latent space that this replaced 25 ms. 512 rows on a context of
 // 40,000: 8.2 ms, before 71 ms.
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -79,6 +81,31 @@ DEVINL float sum_halves(float v) {
 
 }  // namespace
 
+// Portions of several requests in one pair of launches, whose contexts are read from the
+// cache's pages: a launch more for each, a copy of its rows and a conversion of its pages'
+// numbers cost more than a short portion's work, and leave most of the chip idle. us of
+// whole layers of 128 heads, a request at a time / so: three of 572 rows together 886 / 842,
+// in fp8 of 200 together 413 / 373, two of 2,500 together 2,957 / 2,903, one of 1,365
+// 1,679 / 1,664.
+#define MP_MAX_PORTIONS 16
+struct Portion {
+  int q0, T;     // query rows
+  int n, base;   // context rows, and where theirs begin among the expanded ones
+  int tile;      // first tile of MP_ROWS query rows
+  int seq;       // row of the block tables
+};
+struct Portions {
+  Portion p[MP_MAX_PORTIONS];
+  int count;
+};
+struct Pages {
+  const uint16_t* cache;  // [NB, 1 << shift, 576]
+  const int* tables;      // [B, max_blocks]
+  int max_blocks, shift;
+  uint16_t* pe;           // rotated parts of the expanded rows [.., 64], written
+};
+struct NoPages {};
+
 // ---- keys and values of a run ------------------------------------------------------
 // 128 context rows x 128 features a workgroup, 4 waves of 64 x 64, both operands
 // global -> LDS directly, 128 bytes of every row a stage. Keys come out as
@@ -89,12 +116,15 @@ DEVINL float sum_halves(float v) {
 // them. 1,900 rows, 128 heads: 128 us; stored from the accumulators, 16 bytes of 32 rows
 // an instruction, 155; five stages of 64 bytes in a ring 141.
 
+template <bool PAGED>
 __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
     uint16_t* __restrict__ k_hi, uint16_t* __restrict__ k_lo,  // [H, cap, 128]
     uint16_t* __restrict__ v_hi, uint16_t* __restrict__ v_lo,  // [H, 128, cap]
-    const uint16_t* __restrict__ rows,  // [n, 576]
+    const uint16_t* __restrict__ rows,  // [n, 576], not PAGED
     const uint16_t* __restrict__ w_uk,  // [H, 128, 512]
-    const uint16_t* __restrict__ w_uv, const int n, const int cap) {
+    const uint16_t* __restrict__ w_uv, int n, const int cap,
+    const std::conditional_t<PAGED, Portions, NoPages> portions,
+    const std::conditional_t<PAGED, Pages, NoPages> pages) {
   constexpr int BKB = 128;
   __shared__ __attribute__((aligned(16))) uint8_t S0[256 * BKB];
   __shared__ __attribute__((aligned(16))) uint8_t S1[256 * BKB];
@@ -102,9 +132,27 @@ __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
   const int lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l31 = lane & 31;
-  const int r0 = blockIdx.y * 128;
+  int r0 = blockIdx.y * 128;  // of the context; at0: of the expanded rows
+  const int at0 = r0;
   const int h = blockIdx.x >> 1;
   const bool val = blockIdx.x & 1;
+  const int* btab = nullptr;
+  if constexpr (PAGED) {
+    int i = portions.count - 1;
+    while (i > 0 && portions.p[i].base > at0) --i;
+    n = portions.p[i].n;
+    r0 = at0 - portions.p[i].base;
+    btab = pages.tables + (size_t)portions.p[i].seq * pages.max_blocks;
+  }
+  auto context_row = [&](int r) {
+    if constexpr (PAGED) {
+      const int slot = r & ((1 << pages.shift) - 1);
+      return pages.cache +
+             (((size_t)btab[r >> pages.shift] << pages.shift) + slot) * MP_DK;
+    } else {
+      return rows + (size_t)r * MP_DK;
+    }
+  };
   const uint8_t* w =
       (const uint8_t*)((val ? w_uv : w_uk) + (size_t)h * MP_D * MP_R);
 
@@ -115,7 +163,16 @@ __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
   for (int i = 0; i < 4; ++i) {
     const int r = i * 32 + (tid >> 3);
     wp[i] = w + (size_t)r * (MP_R * 2) + src;
-    rp[i] = (const uint8_t*)(rows + (size_t)min(r0 + r, n - 1) * MP_DK) + src;
+    rp[i] = (const uint8_t*)context_row(min(r0 + r, n - 1)) + src;
+  }
+  if constexpr (PAGED) {  // eight threads a row
+    if (blockIdx.x == 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<u32x4v*>(pages.pe + (size_t)(at0 + i * 32 + (tid >> 3)) * MP_DR +
+                                   (tid & 7) * 8) =
+            *reinterpret_cast<const u32x4v*>((const uint16_t*)(rp[i] - src) + MP_R +
+                                             (tid & 7) * 8);
   }
   auto issue = [&](int kt, uint8_t* S) {
 #pragma unroll
@@ -187,7 +244,7 @@ __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
       }
   }
   __syncthreads();
-  const size_t base = (size_t)h * cap * MP_D + (val ? (size_t)r0 : (size_t)r0 * MP_D);
+  const size_t base = (size_t)h * cap * MP_D + (val ? (size_t)at0 : (size_t)at0 * MP_D);
   const size_t pitch = val ? cap : MP_D;
   uint16_t* hi = (val ? v_hi : k_hi) + base;
   uint16_t* lo = (val ? v_lo : k_lo) + base;
@@ -206,6 +263,7 @@ __global__ __launch_bounds__(256, 2) void mla_expand_kernel(
 // 128 query rows of one head a workgroup, 32 a wave; see prefill_attention for
 // the operand orders (S^T = K Q^T, O^T = V^T P, P from the accumulators).
 
+template <bool PAGED>
 __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
     uint16_t* __restrict__ out,           // [T, H, 128]
     float* __restrict__ state,            // [T, H, 130] or null
@@ -213,10 +271,11 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
     const uint16_t* __restrict__ q_pe,    // [T, H, 64]
     const uint16_t* __restrict__ k_hi, const uint16_t* __restrict__ k_lo,
     const uint16_t* __restrict__ v_hi, const uint16_t* __restrict__ v_lo,
-    const uint16_t* __restrict__ rows,    // [n, 576]
-    const int T, const int H, const int n, const int cap, const int prefix,
+    const uint16_t* __restrict__ rows,    // [n, 576]; PAGED: rotated parts [cap, 64]
+    int T, const int H, int n, const int cap, int prefix,
     const int first_key, const int64_t q_row, const int64_t q_head,
-    const float scale, const int first, const int last) {
+    const float scale, const int first, const int last,
+    const std::conditional_t<PAGED, Portions, NoPages> portions) {
   __shared__ __attribute__((aligned(16))) uint16_t Kh0[MP_KT * 128], Kl0[MP_KT * 128];
   __shared__ __attribute__((aligned(16))) uint16_t Kh1[MP_KT * 128], Kl1[MP_KT * 128];
   __shared__ __attribute__((aligned(16))) uint16_t R0[MP_KT * 64], R1[MP_KT * 64];
@@ -230,7 +289,22 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
   // heads fastest: with 8 | H a head's blocks share an XCD's L2; the last rows
   // see the most keys and come first
   const int h = blockIdx.x % H;
-  const int tile = gridDim.x / H - 1 - blockIdx.x / H;
+  int tile = gridDim.x / H - 1 - blockIdx.x / H;
+  int base = 0;
+  if constexpr (PAGED) {
+    int i = portions.count - 1;
+    while (i > 0 && portions.p[i].tile > tile) --i;
+    const Portion p = portions.p[i];
+    tile -= p.tile;
+    T = p.T;
+    n = p.n;
+    prefix = n - T;
+    base = p.base;
+    out += (size_t)p.q0 * H * MP_D;
+    q_nope += p.q0 * q_row;
+    q_pe += (size_t)p.q0 * H * MP_DR;
+    rows += (size_t)base * MP_DR;
+  }
   const int w0 = tile * MP_ROWS + wid * 32;
   const int row = w0 + l31;
   const bool row_ok = row < T;
@@ -278,10 +352,10 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
   const float c = fmaxf(fabsf(scale) * kLog2e, 1e-20f);
 
   // ---- copies: chunk numbers within a tile, LDS places XOR-swizzled by row ---------
-  const uint16_t* kh = k_hi + (size_t)h * cap * MP_D;
-  const uint16_t* kl = k_lo + (size_t)h * cap * MP_D;
-  const uint16_t* vh = v_hi + (size_t)h * cap * MP_D;
-  const uint16_t* vl = v_lo + (size_t)h * cap * MP_D;
+  const uint16_t* kh = k_hi + ((size_t)h * cap + base) * MP_D;
+  const uint16_t* kl = k_lo + ((size_t)h * cap + base) * MP_D;
+  const uint16_t* vh = v_hi + (size_t)h * cap * MP_D + base;
+  const uint16_t* vl = v_lo + (size_t)h * cap * MP_D + base;
   int k_at[2], v_at[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -291,7 +365,8 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
     v_at[i] = vr * cap + ((ch & 3) ^ ((vr >> 2) & 3)) * 8;
   }
   const int pe_row = tid >> 3;
-  const int pe_at = MP_R + ((tid & 7) ^ ((pe_row >> 1) & 7)) * 8;
+  constexpr int PE_ROW = PAGED ? MP_DR : MP_DK;
+  const int pe_at = (PAGED ? 0 : MP_R) + ((tid & 7) ^ ((pe_row >> 1) & 7)) * 8;
   auto issue = [&](int kt, uint16_t* Kh, uint16_t* Kl, uint16_t* R,
                    uint16_t* Vh, uint16_t* Vl) {
 #pragma unroll
@@ -303,7 +378,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
       copy16_to_lds(vl + (size_t)kt * MP_KT + v_at[i], Vl + dst);
     }
     copy16_to_lds(
-        rows + (size_t)min(kt * MP_KT + pe_row, n - 1) * MP_DK + pe_at,
+        rows + (size_t)min(kt * MP_KT + pe_row, n - 1) * PE_ROW + pe_at,
         R + wid * 512);
   };
 
@@ -431,13 +506,44 @@ extern "C" void launch_mla_prefill_run(
     const void* w_uv, int T, int H, int n, int cap, int prefix, int first_key,
     int64_t q_row, int64_t q_head, float scale, bool first, bool last,
     hipStream_t stream) {
-  mla_expand_kernel<<<dim3(2 * H, ceil_div(n, 128), 1), 256, 0, stream>>>(
+  mla_expand_kernel<false><<<dim3(2 * H, ceil_div(n, 128), 1), 256, 0, stream>>>(
       (uint16_t*)k_hi, (uint16_t*)k_lo, (uint16_t*)v_hi, (uint16_t*)v_lo,
       (const uint16_t*)rows, (const uint16_t*)w_uk, (const uint16_t*)w_uv, n,
-      cap);
-  mla_prefill_kernel<<<ceil_div(T, MP_ROWS) * H, 256, 0, stream>>>(
+      cap, NoPages{}, NoPages{});
+  mla_prefill_kernel<false><<<ceil_div(T, MP_ROWS) * H, 256, 0, stream>>>(
       (uint16_t*)out, state, (const uint16_t*)q_nope, (const uint16_t*)q_pe,
       (const uint16_t*)k_hi, (const uint16_t*)k_lo, (const uint16_t*)v_hi,
       (const uint16_t*)v_lo, (const uint16_t*)rows, T, H, n, cap, prefix,
-      first_key, q_row, q_head, scale, first, last);
+      first_key, q_row, q_head, scale, first, last, NoPages{});
+}
+
+extern "C" int mla_prefill_max_portions() { return MP_MAX_PORTIONS; }
+
+// lens: rows and context rows of each of count portions, starts: their first query row
+// and their row of the block tables, in the order of their context rows, so that the
+// longest tiles, which are dealt from the end, come first. cap: the sum of the contexts,
+// each in multiples of 128.
+extern "C" void launch_mla_prefill_paged(
+    void* out, const void* q_nope, const void* q_pe, void* k_hi, void* k_lo, void* v_hi,
+    void* v_lo, void* pe, const void* cache, const int* tables, int max_blocks, int shift,
+    const void* w_uk, const void* w_uv, const int* lens, const int* starts, int count,
+    int H, int cap, int64_t q_row, int64_t q_head, float scale, hipStream_t stream) {
+  Portions ps{};
+  ps.count = count;
+  int base = 0, tiles = 0;
+  for (int i = 0; i < count; ++i) {
+    ps.p[i] = {starts[2 * i], lens[2 * i], lens[2 * i + 1], base, tiles,
+               starts[2 * i + 1]};
+    base += ceil_div(lens[2 * i + 1], 128) * 128;
+    tiles += ceil_div(lens[2 * i], MP_ROWS);
+  }
+  mla_expand_kernel<true><<<dim3(2 * H, cap / 128, 1), 256, 0, stream>>>(
+      (uint16_t*)k_hi, (uint16_t*)k_lo, (uint16_t*)v_hi, (uint16_t*)v_lo, nullptr,
+      (const uint16_t*)w_uk, (const uint16_t*)w_uv, 0, cap, ps,
+      Pages{(const uint16_t*)cache, tables, max_blocks, shift, (uint16_t*)pe});
+  mla_prefill_kernel<true><<<tiles * H, 256, 0, stream>>>(
+      (uint16_t*)out, nullptr, (const uint16_t*)q_nope, (const uint16_t*)q_pe,
+      (const uint16_t*)k_hi, (const uint16_t*)k_lo, (const uint16_t*)v_hi,
+      (const uint16_t*)v_lo, (const uint16_t*)pe, 0, H, 0, cap, 0, 0, q_row, q_head,
+      scale, 1, 1, ps);
 }

@@ -252,6 +252,54 @@ def test_mla_prefill_scales_of_any_sign(scale):
             out[:, h].float(), p @ v, atol=2.4e-3, rtol=2 ** -8)
 
 
+@pytest.mark.parametrize("H,page,lens", [
+    (128, 64, [(1, 1)]),
+    (16, 16, [(33, 33), (0, 40), (129, 1000), (127, 127)]),  # out of order, one without rows
+    (3, 32, [(130, 300), (256, 256), (1, 129)]),             # heads that XCDs do not share
+    (16, 16, [(5 + 13 * i, 5 + 17 * i) for i in range(19)]), # more than a launch takes
+    (128, 128, [(60, 5000), (300, 3500), (7, 20)]),          # more rows than it expands
+])
+def test_mla_prefill_of_all_requests(H, page, lens):
+    """The bits of a request at a time, from shuffled pages whose unused slots hold NaN."""
+    g = torch.Generator(device="cuda").manual_seed(H + len(lens))
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    T = sum(n for n, _ in lens)
+    q = r(T, H, 192).bfloat16()
+    q_nope, q_pe = q[..., :128], q[..., 128:].contiguous()
+    uk, uv = ((r(H, 128, 512) * 512 ** -0.5).bfloat16() for _ in range(2))
+    counts = [-(-n // page) for _, n in lens]
+    cache = torch.full((sum(counts) + 3, page, 576), float("nan"), device="cuda").bfloat16()
+    ids = torch.randperm(sum(counts), generator=g, device="cuda").int()
+    tables = torch.full((len(lens), max(counts) + 2), 1 << 30, dtype=torch.int32,
+                        device="cuda")
+    out = torch.empty(T, H, 128, dtype=torch.bfloat16, device="cuda")
+    want, at, row = torch.empty_like(out), 0, 0
+    for i, (n, context) in enumerate(lens):
+        mine = ids[at:at + counts[i]]
+        at += counts[i]
+        tables[i, :counts[i]] = mine
+        rows = r(context, 576).bfloat16()
+        for j in range(counts[i]):
+            part = rows[j * page:(j + 1) * page]
+            cache[mine[j].item(), :len(part)] = part
+        part = slice(row, row + n)
+        row += n
+        if n:
+            assert ops.mla_prefill_attention(want[part], q_nope[part], q_pe[part], rows,
+                                             uk, uv, 192 ** -0.5)
+    assert ops.mla_prefill_paged(out, q_nope, q_pe, cache, tables, lens, uk, uv,
+                                 192 ** -0.5)
+    assert torch.equal(out, want)
+    for lens, cache, tables in (
+        (lens, cache.float(), tables), (lens, cache.to(torch.float8_e4m3fn), tables),
+        (lens, cache[..., :512], tables), (lens, cache[:, :page - 1], tables),
+        (lens, cache, tables.long()), (lens, cache, tables[:, :max(counts) - 1]),
+        ([(lens[0][0], (1 << 20) // H + 128)] + lens[1:], cache, tables),  # by runs
+        (lens + [(1, 1)], cache, tables),
+    ):
+        assert not ops.mla_prefill_paged(out, q_nope, q_pe, cache, tables, lens, uk, uv, 1.0)
+
+
 def test_mla_prefill_left_to_the_caller():
     """Types, widths and few rows on a long context have no kernel."""
     def call(T, L, H=16, dtype=torch.bfloat16, dn=128, dr=64, dev="cuda"):
