@@ -46,7 +46,6 @@
 typedef short s16x4v __attribute__((ext_vector_type(4)));
 typedef float f32x16v __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8n __attribute__((ext_vector_type(8)));
-typedef short bf16x2v __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2n __attribute__((ext_vector_type(2)));
 
@@ -855,12 +854,11 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
         l *= f;
       } else if (i < 13) {
         const int e = (i - 5) * 2;
-        uint32_t pk = pack_bf16(__builtin_amdgcn_exp2f(fmaf(s[e], c, -m)),
-                                __builtin_amdgcn_exp2f(fmaf(s[e + 1], c, -m)));
-        // of the rounded weights: what their rounding adds to O^T it adds to both
-        l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2v, pk),
-                                            __builtin_bit_cast(bf16x2v, 0x3f803f80u), l,
-                                            false);
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[e], c, -m));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[e + 1], c, -m));
+        l += p0;  // in fp32: only the products' operands are rounded
+        l += p1;
+        const uint32_t pk = pack_bf16(p0, p1);
         auto w = __builtin_bit_cast(u32x4v, b[e >> 3]);
         w[e >> 1 & 3] = pk;
         b[e >> 3] = __builtin_bit_cast(bf16x8v, w);

@@ -427,3 +427,34 @@ def test_mla_decode_tiles_and_runs(H, BS, ctxs, kv):
         err = (out[i].double() - want).norm() / want.norm()
         # weights and results are rounded to bf16: 2^-9 at most each
         assert err < 2 * 2 ** -9, (i, n, float(err))
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+@pytest.mark.parametrize("H,ctxs", [
+    (16, [3200, 64, 200]),      # tiles of 64
+    (64, [3200, 64, 200]),      # tiles of 32, several runs
+    (128, [224, 32, 200]),      # a workgroup a sequence
+])
+def test_mla_decode_sums_weights_unrounded(H, ctxs, kv):
+    """Every 32nd token weighs 1, the others 2^-3 (1 + 0.45 * 2^-7), which is 2^-3 in
+    bf16, and only the former have values: their sum is exact, and a sum of rounded
+    weights would be 0.0028 short."""
+    ql, qp, cache, bt, sl = _setup(len(ctxs), H, ctxs, seed=11)
+    one = torch.arange(32, device="cuda") == 5
+    cache[..., 512:] = 0
+    cache[..., 512] = torch.where(one, 0.0, -1.0)
+    cache[:, ~one, :512] = 0
+    ql.zero_(), qp.zero_()
+    qp[..., 0] = 1
+    if kv == "fp8":
+        cache = cache.to(torch.float8_e4m3fn)
+    p = 2 ** -3 * (1 + 0.45 * 2 ** -7)
+    out = ops.mla_paged_attention_decode(ql, qp, cache, bt, sl, -math.log(p)).double()
+    for i, n in enumerate(ctxs):
+        e = cache[bt[i, :-(-n // 32)].long()].double().flatten(0, 1)[:n]
+        w = torch.where(e[:, 512] == 0, 1.0, p).double()
+        want = (w @ e[:, :512]) / w.sum()
+        # against the rounded result: fp32's own rounding, 1e-6, moves few of a head's 512
+        # values over the middle of two bf16 numbers, each by 2^-7, 2e-5 of all
+        off = ((out[i] - want.bfloat16().double()) @ want) / (want @ want)
+        assert off.abs().max() < 2e-4, (n, off.abs().max().item())
