@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "mla_deal.h"
 
 #define MLA_R 512
 #define MLA_DR 64
@@ -129,12 +130,6 @@ DEVINL int div_up(int n, int d) {
   return n > 0 ? (int)(((float)n - 0.5f) * __builtin_amdgcn_rcpf((float)d)) + 1 : 0;
 }
 
-// A workgroup's run: its sequence, the first tile there, and its tiles; how many there are
-// to a run of this sequence.
-struct Run {
-  int seq, at, todo, per;
-};
-
 // the first and the last run of each sequence, behind the parts' maxima and sums
 DEVINL int2* part_runs(float* tmp_ml, int runs, int B, int H) {
   return reinterpret_cast<int2*>(tmp_ml + ((size_t)runs + B) * H * 2);
@@ -142,45 +137,70 @@ DEVINL int2* part_runs(float* tmp_ml, int runs, int B, int H) {
 
 // How the tiles are dealt, found by one wave; tiles_of(b): of sequence b, 0 from B on.
 // Each run lies in one sequence, which has as many of equal length as it takes for none
-// to be longer than `per`, the least that `runs` suffice for. Or, where that is 256 tokens
-// more than even, runs go through the list of all tiles: a run that meets the next
-// sequence pays the start and the end of a run twice, which costs about as much. us of a
-// call, 64 heads, even / so: 4 sequences of 5,300 tokens 33.8 / 28.2, of 66,000 79.4 /
-// 73.8.
-template <int KT, class F>
+// to be longer than `per`, the least that `runs` suffice for. Or, where that is more than
+// MORE tokens longer than even, runs go through the list of all tiles: a run that meets the
+// next sequence pays the start and the end of a run twice, and leaves parts of both.
+// What that is worth is measured by kernel and cache (us of a call, through the list / in
+// one sequence, + how many tokens longer):
+// - more than 32 heads, 512: 64 heads 24 x 4,073 +32 46.8 / 41.6, 237 of up to 1,427 +512
+//   90.4 / 76.8, 132 x 1,410 +672 70.3 / 74.1; 128 heads 105 of up to 571 +352 49.7 / 41.9,
+//   112 of up to 1,021 +640 57.3 / 59.2.
+// - the same, fp8, whose tiles take longer, 288: 128 heads 33 x 1,081 +96 46 / 42, 110 of up
+//   to 429 +288 50.9 / 42.2, 46 x 2,311 +320 74.8 / 80.4; 64 heads 93 x 2,749 +352 82.9 /
+//   91.4.
+// - up to 32 heads, 192: 16 heads 225 x 1,352 +128 84.4 / 77.0, 70 x 3,000 +192 49.2 / 46.3,
+//   219 of up to 1,459 +448 48.4 / 55.9. fp8, 64: 165 of up to 1,388 +64 42.5 / 38.0, 107 of
+//   up to 2,274 +128 48.0 / 53.1.
+// - lists of 2,048 positions, more than 32 heads 192: 64 heads, 100 of them +192 91 / 86; 128
+//   heads in fp8, 47 of them +256 82 / 87. Up to 32, 64: 40 of them +64 34.2 / 33.2, 100 of
+//   them +192 64 / 68; in fp8 none longer: 40 of them +64 35 / 37.
+template <int KT, int MORE, class F>
 DEVINL Run find_run(int B, int run, int runs, F tiles_of) {
   const int lane = threadIdx.x & 63;
-  const int n0 = tiles_of(lane);
-  int total = n0;
-  for (int b = lane + 64; b < B; b += 64) total += tiles_of(b);
+  // a lane's sequences: 256 in registers, as each pass would wait for their lengths again
+  constexpr int KEPT = 4;
+  int kept[KEPT] = {tiles_of(lane)};
+  if (B > 64)
+#pragma unroll
+    for (int j = 1; j < KEPT; ++j) kept[j] = tiles_of(j * 64 + lane);
+  auto each = [&](auto&& use) INL {
+    use(kept[0]);
+    if (B <= 64) return;
+#pragma unroll
+    for (int j = 1; j < KEPT; ++j) use(kept[j]);
+    for (int b = KEPT * 64 + lane; b < B; b += 64) use(tiles_of(b));
+  };
+  int total = 0;
+  each([&](int tiles) INL { total += tiles; });
   total = wave_sum(total);
   const int even = max(div_up(total, runs), MLA_MIN_TOKENS / KT);
-  int per = even;
-  bool whole = false;
-  while (!whole && per <= even + 256 / KT) {
-    int k = div_up(n0, per);
-    for (int b = lane + 64; b < B; b += 64) k += div_up(tiles_of(b), per);
-    k = wave_sum(k);
-    whole = k <= runs;
-    // as many runs as now go to rounding up
-    if (!whole) per = max(per + 1, div_up(total, max(runs - k + div_up(total, per), 1)));
-  }
-  if (!whole) per = even;
+  const int most = even + MORE / KT;
+  const int least = least_length(even, most, runs, [&](int length) INL {
+    int n = 0;
+    each([&](int tiles) INL { n += div_up(tiles, length); });
+    return wave_sum(n);
+  });
+  const bool whole = least <= most;
+  const int per = whole ? least : even;
   const int begin = whole ? run : run * per;  // in runs, or in tiles
   int before = 0;
   for (int b0 = 0; b0 < B; b0 += 64) {
-    const int tiles = b0 == 0 ? n0 : tiles_of(b0 + lane);
+    int tiles = kept[0];
+    if (b0 > 0) {
+#pragma unroll
+      for (int j = 1; j < KEPT; ++j) tiles = b0 == j * 64 ? kept[j] : tiles;
+      if (b0 >= KEPT * 64) tiles = tiles_of(b0 + lane);
+    }
     const int n = whole ? div_up(tiles, per) : tiles;
     const int sum = before + sum_before(n);
     const unsigned long long hit = __ballot(begin >= sum - n && begin < sum);
     if (hit) {
       const int src = __ffsll(hit) - 1;
-      const int t = __builtin_amdgcn_readlane(tiles, src);
       const int k = __builtin_amdgcn_readlane(n, src);
       const int first = __builtin_amdgcn_readlane(sum, src) - k;
-      if (!whole) return {b0 + src, begin - first, min(per, total - begin), per};
-      const int len = div_up(t, k), at = (run - first) * len;
-      return {b0 + src, at, min(len, t - at), len};
+      if (!whole) return run_of_list(b0 + src, begin, first, per, total);
+      return run_of_sequence(b0 + src, run - first, __builtin_amdgcn_readlane(tiles, src), k,
+                             div_up);
     }
     before = __builtin_amdgcn_readlane(sum, 63);
   }
@@ -202,6 +222,8 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     const int* __restrict__ topk,           // [B, max_topk] (SPARSE)
     const int max_topk, const int B, const int max_blocks, const int H,
     const int bs_shift, const float scale) {
+  // see find_run
+  constexpr int MORE = W == 8 ? 192 : KV_FP8 ? (SPARSE ? 0 : 64) : SPARSE ? 64 : 192;
   constexpr int RPW = MLA_KT / W;      // rows a wave copies
   constexpr int CPW = RPW + RPW / 8;   // copies: a row's latent values, 8 rows' rope
   constexpr int BUF = MLA_KT * (MLA_ROW + MLA_PE);
@@ -232,7 +254,7 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
       return b < B ? (domain_of<SPARSE>(seq_lens, topk, max_topk, b) + MLA_KT - 1) / MLA_KT
                    : 0;
     };
-    run = find_run<MLA_KT>(B, blockIdx.x, gridDim.x, tiles_of);
+    run = find_run<MLA_KT, MORE>(B, blockIdx.x, gridDim.x, tiles_of);
   }
   int seq = __builtin_amdgcn_readfirstlane(run.seq);
   int at = __builtin_amdgcn_readfirstlane(run.at);    // tile of the sequence
@@ -636,6 +658,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
     const int* __restrict__ block_tables,   // [B, max_blocks]
     const int* __restrict__ seq_lens, const int B, const int max_blocks,
     const int H, const int bs_shift, const float scale) {
+  constexpr int MORE = KV_FP8 ? 288 : 512;  // see find_run
   constexpr int BUF = MLA_WT * (MLA_ROW + MLA_PE);
   constexpr int PE = MLA_WT * MLA_ROW;  // of a buffer's rotated values
   constexpr int RING = 4;
@@ -666,7 +689,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
     auto tiles_of = [&](int b) INL {
       return b < B ? (max(seq_lens[b], 0) + MLA_WT - 1) / MLA_WT : 0;
     };
-    run = find_run<MLA_WT>(B, blockIdx.x, gridDim.x, tiles_of);
+    run = find_run<MLA_WT, MORE>(B, blockIdx.x, gridDim.x, tiles_of);
   }
   int seq = __builtin_amdgcn_readfirstlane(run.seq);
   int at = __builtin_amdgcn_readfirstlane(run.at);    // tile of the sequence
