@@ -15,8 +15,8 @@
 // there; the others leave fp32 parts that a second kernel adds up. Short sequences (256
 // tokens at most) take a workgroup each and need no second kernel.
 //
-// Two kernels: mla_decode_wide_kernel for more than 32 heads, mla_decode_kernel for up to
-// 32 and for lists of token positions. What bounds them: with 64 heads the latent rows'
+// Two kernels: mla_decode_wide_kernel for more than 32 heads on an fp8 cache,
+// mla_decode_kernel for the others. What bounds them: with 64 heads the latent rows'
 // stream (6 TB/s), with 128 what a tile issues, 290 vector instructions and 34 products a
 // wave that hardly overlap, LDS reads; and the start and end of a run, 9 us of looking up,
 // first rows and parts, then 8 of the second kernel.
@@ -142,12 +142,12 @@ DEVINL int2* part_runs(float* tmp_ml, int runs, int B, int H) {
 // next sequence pays the start and the end of a run twice, and leaves parts of both.
 // What that is worth is measured by kernel and cache (us of a call, through the list / in
 // one sequence, + how many tokens longer):
-// - more than 32 heads, 512: 64 heads 24 x 4,073 +32 46.8 / 41.6, 237 of up to 1,427 +512
-//   90.4 / 76.8, 132 x 1,410 +672 70.3 / 74.1; 128 heads 105 of up to 571 +352 49.7 / 41.9,
-//   112 of up to 1,021 +640 57.3 / 59.2.
-// - the same, fp8, whose tiles take longer, 288: 128 heads 33 x 1,081 +96 46 / 42, 110 of up
-//   to 429 +288 50.9 / 42.2, 46 x 2,311 +320 74.8 / 80.4; 64 heads 93 x 2,749 +352 82.9 /
-//   91.4.
+// - more than 32 heads, 384: 64 heads 24 x 5,158 +64 51.1 / 45.9, 238 of up to 1,077 +384
+//   79 / 63; 128 heads 98 of up to 1,650 +320 66 / 54, 44 x 2,682 +384 70 / 73, 44 x 3,202 +512
+//   77 / 84.
+// - the same with an fp8 cache, in the wide kernel, 288: 128 heads 33 x 1,081 +96 46 / 42,
+//   110 of up to 429 +288 50.9 / 42.2, 46 x 2,311 +320 74.8 / 80.4; 64 heads 93 x 2,749 +352
+//   82.9 / 91.4.
 // - up to 32 heads, 192: 16 heads 225 x 1,352 +128 84.4 / 77.0, 70 x 3,000 +192 49.2 / 46.3,
 //   219 of up to 1,459 +448 48.4 / 55.9. fp8, 64: 165 of up to 1,388 +64 42.5 / 38.0, 107 of
 //   up to 2,274 +128 48.0 / 53.1.
@@ -223,7 +223,8 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
     const int max_topk, const int B, const int max_blocks, const int H,
     const int bs_shift, const float scale) {
   // see find_run
-  constexpr int MORE = W == 8 ? 192 : KV_FP8 ? (SPARSE ? 0 : 64) : SPARSE ? 64 : 192;
+  constexpr int MORE =
+      W == 8 ? (SPARSE ? 192 : 384) : KV_FP8 ? (SPARSE ? 0 : 64) : SPARSE ? 64 : 192;
   constexpr int RPW = MLA_KT / W;      // rows a wave copies
   constexpr int CPW = RPW + RPW / 8;   // copies: a row's latent values, 8 rows' rope
   constexpr int BUF = MLA_KT * (MLA_ROW + MLA_PE);
@@ -635,37 +636,35 @@ __global__ __launch_bounds__(W * 64, 2) void mla_decode_kernel(
   }
 }
 
-// ---- more than 32 heads ----------------------------------------------------------
+// ---- an fp8 cache, more than 32 heads ---------------------------------------------
 // Four waves, 64 heads: 32 a pair of waves, on 32x32 matrix instructions, so that an
 // operand row read from LDS serves 32 heads instead of 16. A wave computes S^T over
 // half of the 576 values, for which it holds the heads' Q, adds the other wave's half,
 // and takes half of the latent values of O^T: 200 registers of state, so one wave a
 // SIMD. Tiles of 32 tokens in a ring of four, three of them on their way. In turn t
 // the products of S^T of tile t + 1 stand beside tile t's softmax.
-// us of a call with the second kernel, mla_decode_kernel of eight waves (16 heads a pair,
-// tiles of 64) and an even deal / so: 64 heads, 4 sequences of 66,000 tokens 82 / 72, of
-// 5,300 34.3 / 26.7; 128 heads, 40 of 2,400 61.5 / 58.5, 99 of 233 54 / 33, fp8 4 of 66,000
-// 139 / 124. The maximum followed only when it has moved by 2^8 takes 128 of the 290
-// instructions away and 10% of the time with 128 heads, and adds 2 to 13% to the error.
-template <bool KV_FP8>
+// us of a call, mla_decode_kernel of eight waves (16 heads a pair, tiles of 64) / so: 64
+// heads, 4 x 21,111 tokens 42.7 / 41.4, 2 x 100,000 66.1 / 63.9; 128 heads, 20 x 9,000 100.5 /
+// 97.3, 70 x 3,000 121 / 118. With a bf16 cache the eight waves are as fast or faster: 64
+// heads, 20 x 9,000 54.4 / 56.1, 2 x 18,786 30.9 / 31.8; 128 heads, 16 x 16,384 119 / 122, 40
+// x 4,000 77 / 80.
 __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
     uint16_t* __restrict__ out,             // [B, H, R]
     float* __restrict__ tmp_acc,            // [parts, H, R]; null: a workgroup
     float* __restrict__ tmp_ml,             // [parts, H, 2]      a sequence
     const uint16_t* __restrict__ q_latent,  // [B, H, R]
     const uint16_t* __restrict__ q_pe,      // [B, H, DR]
-    const void* __restrict__ cache,         // [NB, BS, R+DR] bf16 | fp8(e4m3)
+    const void* __restrict__ cache,         // [NB, BS, R+DR] fp8(e4m3)
     const int* __restrict__ block_tables,   // [B, max_blocks]
     const int* __restrict__ seq_lens, const int B, const int max_blocks,
     const int H, const int bs_shift, const float scale) {
-  constexpr int MORE = KV_FP8 ? 288 : 512;  // see find_run
+  constexpr int MORE = 288;  // see find_run
   constexpr int BUF = MLA_WT * (MLA_ROW + MLA_PE);
   constexpr int PE = MLA_WT * MLA_ROW;  // of a buffer's rotated values
   constexpr int RING = 4;
   constexpr int CPW = 9;                // copies a wave: 8 rows, their rotated values
   constexpr int QS = 18;                // steps of 16 values of S^T a wave
   constexpr int DT = 8;                 // tiles of 32 latent values of O^T a wave
-  constexpr int ESZ = KV_FP8 ? 1 : 2;
   __shared__ __attribute__((aligned(1024))) uint8_t S[RING * BUF];
   // sums over half of the values on their way to the other wave of a pair
   __shared__ __attribute__((aligned(16))) f32x4v X[4][4][64];
@@ -705,8 +704,6 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
   // and the others, which differ in both; transposing reads take four neighbouring
   // chunks of four rows, which differ in bits 2 and 3 of wide_xor.
   auto wide_xor = [](int r) INL { return (r & 3) * 4 + (r >> 2 & 3); };
-  const uint32_t s_at = (uint32_t)(uintptr_t)(
-      __attribute__((address_space(3))) const void*)S;
   const int qk_at = l31 * MLA_ROW + h * 512 + (half ^ wide_xor(l31)) * 16;
   const int pe_at = PE + l31 * MLA_PE + ((4 * h + half) ^ (l31 >> 1 & 7)) * 16;
   const int tr_row = 4 * half + (l15 >> 2);
@@ -717,9 +714,9 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
   uint32_t from[CPW];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    from[i] = (i * MLA_DK + (lane ^ wide_xor(wid * 8 + i)) * 8) * ESZ;
-  from[8] = ((lane >> 3) * MLA_DK + MLA_R +
-             ((lane & 7) ^ ((wid * 8 + (lane >> 3)) >> 1 & 7)) * 8) * ESZ;
+    from[i] = i * MLA_DK + (lane ^ wide_xor(wid * 8 + i)) * 8;
+  from[8] = (lane >> 3) * MLA_DK + MLA_R +
+            ((lane & 7) ^ ((wid * 8 + (lane >> 3)) >> 1 & 7)) * 8;
   auto place = [&](int i) INL {
     return i < 8 ? (wid * 8 + i) * MLA_ROW : PE + wid * 8 * MLA_PE;
   };
@@ -758,22 +755,19 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
     auto page_of = [&](int t) INL { return btab[token_of(t) >> bs_shift]; };
     auto base_of = [&](int t, int page) INL {
       const int slot = (page << bs_shift) + (token_of(t) & (BS - 1));
-      return (const uint8_t*)cache + (int64_t)slot * (MLA_DK * ESZ);
+      return (const uint8_t*)cache + (int64_t)slot * MLA_DK;
     };
-    auto issue = [&](int i, const uint8_t* base, int t) INL {
-      copy16(base, from[i], s_at + ((t - t0) & (RING - 1)) * BUF + place(i));
-    };
-    uint64_t raw[2][KV_FP8 ? CPW : 1];  // an fp8 cache: two tiles on their way
-    auto fetch8 = [&](uint64_t (&r)[KV_FP8 ? CPW : 1], int t, int page) INL {
+    uint64_t raw[2][CPW];  // two tiles on their way
+    auto fetch8 = [&](uint64_t (&r)[CPW], int t, int page) INL {
       const uint8_t* base = base_of(t, page);
 #pragma unroll
-      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i)
+      for (int i = 0; i < CPW; ++i)
         r[i] = *(const uint64_t*)(base + from[i]);
     };
-    auto widen8 = [&](const uint64_t (&r)[KV_FP8 ? CPW : 1], int t) INL {
+    auto widen8 = [&](const uint64_t (&r)[CPW], int t) INL {
       uint8_t* T = S + ((t - t0) & (RING - 1)) * BUF + lane * 16;
 #pragma unroll
-      for (int i = 0; i < (KV_FP8 ? CPW : 1); ++i) {
+      for (int i = 0; i < CPW; ++i) {
         bf16x8n v;  // every e4m3 number is one of bf16
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -929,27 +923,13 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
     for (int i = 0; i < QS; ++i) asm volatile("" : "+a"(qf[i]));
     if (!first) __syncthreads();  // the buffers may still be read for the last sequence
     first = false;
-    if constexpr (KV_FP8) {
-      fetch8(raw[0], t0, page_of(t0));
-      fetch8(raw[1], min(t0 + 1, t1 - 1), page_of(min(t0 + 1, t1 - 1)));
-    } else {
-#pragma unroll
-      for (int k = 0; k < RING - 1; ++k) {
-        const int tk = min(t0 + k, t1 - 1);
-        const uint8_t* base = base_of(tk, page_of(tk));
-#pragma unroll
-        for (int i = 0; i < CPW; ++i) issue(i, base, t0 + k);
-      }
-    }
+    fetch8(raw[0], t0, page_of(t0));
+    fetch8(raw[1], min(t0 + 1, t1 - 1), page_of(min(t0 + 1, t1 - 1)));
     // the first tile's scores
-    if constexpr (KV_FP8) {
-      widen8(raw[0], t0);
-      const int t2 = min(t0 + 2, t1 - 1);
-      fetch8(raw[0], t2, page_of(t2));
-      widen8(raw[1], t0 + 1);
-    } else {
-      __builtin_amdgcn_s_waitcnt(0x4f72);  // vmcnt(18): those of two tiles in flight
-    }
+    widen8(raw[0], t0);
+    const int t2 = min(t0 + 2, t1 - 1);
+    fetch8(raw[0], t2, page_of(t2));
+    widen8(raw[1], t0 + 1);
     meet();
     clear_rest(t0);
     scores(t0, sc[0], [](int) {});
@@ -962,9 +942,6 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
     int page = page_of(min(t0 + 3, t1 - 1));  // of the tile that the next turn copies
     auto turn = [&](int t, auto even) INL {
       constexpr int P = decltype(even)::value;
-      const int ahead = min(t + 3, t1 - 1);
-      // this thread's copies of tile t + 1: those of t + 2 stay in flight
-      if constexpr (!KV_FP8) __builtin_amdgcn_s_waitcnt(0x0f70 | CPW);
       meet();
       f32x4v x[4];
 #pragma unroll
@@ -976,12 +953,9 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             x[q][r] = 8 * q + 4 * half + r < rest ? x[q][r] : -3e38f;
-      const uint8_t* base = nullptr;
-      if constexpr (KV_FP8) fetch8(raw[P ^ 1], ahead, page);
-      else base = base_of(ahead, page);
+      fetch8(raw[P ^ 1], min(t + 3, t1 - 1), page);
       clear_rest(t + 1);
       scores(t + 1, sc[P ^ 1], [&](int i) INL {
-        if (!KV_FP8 && (i & 1) == 0) issue(i >> 1, base, t + 3);
         soften(i, sc[P], x);
         // on their way to behind the barrier
         if (i == 15) fetch_v(t, 0);
@@ -991,7 +965,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
       meet();  // every wave has the other's half of tile t
       publish(sc[P ^ 1]);
       weigh(t);
-      if constexpr (KV_FP8) widen8(raw[P], t + 2);
+      widen8(raw[P], t + 2);
     };
     for (int t = t0;;) {
       turn(t, Int<0>{});
@@ -999,7 +973,6 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
       turn(t, Int<1>{});
       if (++t >= t1) break;
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // the last copies
 
     // ---- results: column = head, rows = latent values --------------------------------
     {
@@ -1173,11 +1146,10 @@ extern "C" void launch_mla_paged_attention_decode(
     reduce(True{});
   } else if (H > 32) {
     if (kv_fp8)
-      mla_decode_wide_kernel<true><<<grid, 256, 0, stream>>>(MLA_ARGS, B, max_blocks, H,
-                                                             shift, scale);
+      mla_decode_wide_kernel<<<grid, 256, 0, stream>>>(MLA_ARGS, B, max_blocks, H, shift,
+                                                       scale);
     else
-      mla_decode_wide_kernel<false><<<grid, 256, 0, stream>>>(MLA_ARGS, B, max_blocks, H,
-                                                              shift, scale);
+      decode(Int<8>{}, False{}, False{});
     reduce(False{});
   } else {
     if (kv_fp8) decode(Int<4>{}, True{}, False{});
