@@ -194,7 +194,7 @@ def test_a_residual_of_rows_apart_is_refused(kind, T, first):
         _step(layer, kind, T, first, lambda t: torch.cat([t, t], 1)[:, :WIDTH])
 
 
-def _shard(kind, fp8, last):
+def _shard(kind, fp8, last, experts=0):
     from parallax_amd.models import get_model_class
     from parallax_amd.models.config import ModelConfig
     kw = dict(vocab_size=64, hidden_size=WIDTH, num_layers=3, num_heads=56,
@@ -203,6 +203,9 @@ def _shard(kind, fp8, last):
     if kind == "mla":
         kw.update(q_lora_rank=1536, kv_lora_rank=512, qk_nope_head_dim=128,
                   qk_rope_head_dim=64, v_head_dim=128, num_kv_heads=56)
+    if experts:  # but for the first layer
+        kw.update(num_experts=experts, num_experts_per_tok=2, moe_intermediate_size=64,
+                  first_k_dense_layers=1)
     name = "DeepseekV3ForCausalLM" if kind == "mla" else "LlamaForCausalLM"
     with torch.device("cuda"):
         model = get_model_class(name)(ModelConfig(architecture=name, **kw), 0,
@@ -223,6 +226,33 @@ def _shard(kind, fp8, last):
     return model
 
 
+def _shard_step(model, kind, T):
+    """One decode step of T requests: what the model returns, and its caches."""
+    from parallax_amd.server.kv_cache import KVCacheSpec, MLAKVCache, PagedKVCache
+    dev = torch.device("cuda")
+    n = len(model.layers)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    if kind == "mla":
+        cache = MLAKVCache(n, 512, 64, 16, T, dev)
+        kept = cache.caches
+    else:
+        cache = PagedKVCache(KVCacheSpec(n, 4, 128, 16), T, dev)
+        kept = cache.k_caches + cache.v_caches
+    for c in kept:
+        c.copy_(torch.randn(c.shape, generator=g, device="cuda"))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    lens = [1 + i % 16 for i in range(T)]
+    meta = ForwardMeta(
+        is_prefill=False, positions=i32([n - 1 for n in lens]),
+        slot_mapping=torch.tensor([16 * i + n - 1 for i, n in enumerate(lens)],
+                                  device=dev),
+        block_tables=i32([[i] for i in range(T)]), seq_lens=i32(lens),
+        kv_cache=None if kind == "mla" else cache,
+        mla_cache=cache if kind == "mla" else None, max_seq_len=16, appends=True)
+    with torch.inference_mode():
+        return [model(_rand(g, T, WIDTH), meta)] + list(kept)
+
+
 @pytest.mark.parametrize("kind,fp8", [("llama", False), ("llama", True), ("mla", False),
                                       ("mla", True)])
 @pytest.mark.parametrize("last", [False, True])
@@ -230,33 +260,9 @@ def test_layers_that_end_in_the_next_norm(kind, fp8, last, monkeypatch):
     """The parts of an MLP's last product are added up by the next layer's norm, the
     shard's norm or its last sum, and by a launch of their own where a hook looks on: the
     same bits either way."""
-    from parallax_amd.server.kv_cache import KVCacheSpec, MLAKVCache, PagedKVCache
-    dev = torch.device("cuda")
     model = _shard(kind, fp8, last)
     n = len(model.layers)
-
-    def step(T):
-        g = torch.Generator(device="cuda").manual_seed(T)
-        if kind == "mla":
-            cache = MLAKVCache(n, 512, 64, 16, T, dev)
-            kept = cache.caches
-        else:
-            cache = PagedKVCache(KVCacheSpec(n, 4, 128, 16), T, dev)
-            kept = cache.k_caches + cache.v_caches
-        for c in kept:
-            c.copy_(torch.randn(c.shape, generator=g, device="cuda"))
-        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
-        lens = [1 + i % 16 for i in range(T)]
-        meta = ForwardMeta(
-            is_prefill=False, positions=i32([n - 1 for n in lens]),
-            slot_mapping=torch.tensor([16 * i + n - 1 for i, n in enumerate(lens)],
-                                      device=dev),
-            block_tables=i32([[i] for i in range(T)]), seq_lens=i32(lens),
-            kv_cache=None if kind == "mla" else cache,
-            mla_cache=cache if kind == "mla" else None, max_seq_len=16, appends=True)
-        with torch.inference_mode():
-            return [model(_rand(g, T, WIDTH), meta)] + list(kept)
-
+    step = lambda T: _shard_step(model, kind, T)
     calls = []
     for name in ("linear_norm", "linear_add"):
         def spy(x, w, *args, of=getattr(ops, name), name=name, **kw):
@@ -280,6 +286,45 @@ def test_layers_that_end_in_the_next_norm(kind, fp8, last, monkeypatch):
     for T, w in zip(rows, want):
         assert all(torch.equal(a, b) for a, b in zip(w, step(T))), T
     assert not calls
+
+
+@pytest.mark.parametrize("kind,where", [
+    (kind, where) for kind in ("llama", "mla")
+    for where in ("mlp", "layer", "input_layernorm", "experts", "no kernel")
+    if kind == "mla" or where != "experts"])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("last", [False, True])
+def test_layers_of_which_one_does_not_end_so(kind, fp8, where, last, monkeypatch):
+    """A layer that gets its input normed and does not end in the next norm, one behind a
+    layer that may not, and products left to the caller behind an opened MLP: the bits of
+    the layers one by one."""
+    T = 33
+    model = _shard(kind, fp8, last, experts=4 if where == "experts" else 0)
+    joined = []
+    for name in ("linear_norm", "linear_add"):
+        def spy(x, w, *args, of=getattr(ops, name), name=name, **kw):
+            if w.shape[1] != 4096:
+                return of(x, w, *args, **kw)
+            joined.append(name)
+            return None if where == "no kernel" else of(x, w, *args, **kw)
+        monkeypatch.setattr(ops, name, spy)
+    if where in ("mlp", "layer", "input_layernorm"):
+        at = model.layers[1]
+        (at if where == "layer" else getattr(at, where)).register_forward_hook(
+            lambda m, a, out: None)
+    got = _shard_step(model, kind, T)
+    norm, add = "linear_norm", "linear_add"
+    assert joined == (  # of three layers and the last norm, or of two and a sum
+        {"mlp": [norm, norm], "layer": [norm], "input_layernorm": [norm, norm],
+         "experts": [norm], "no kernel": [norm, norm, norm]} if last else
+        {"mlp": [norm], "layer": [], "input_layernorm": [add], "experts": [norm],
+         "no kernel": [norm, add]})[where]
+    joined.clear()
+    for layer in model.layers:
+        layer.register_forward_hook(lambda m, a, out: None)
+    want = _shard_step(model, kind, T)
+    assert not joined and all(torch.equal(a, b) for a, b in zip(got, want))
+    assert got[0].isfinite().all()
 
 
 @pytest.mark.parametrize("M,N,K", [(9, 7168, 16384), (33, 4096, 4096), (128, 8192, 8192)])
