@@ -540,7 +540,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(const MoeArgs p) {
 // What bounds it: the card's power, and where operands come from behind the L2 the
 // wait for them. 128 bf16 experts of 2048 x 768, 8192 tokens x 8: gate/up 443 us = 930
 // TFLOP/s, down 2 x 159 us (tiles of 128 x 256, 48 KB a stage for half the products:
-// 498 and 2 x 187); with operands from the L2 alone 1.27 PFLOP/s, where the matrix
+// 498 and 2 x 187), on other cards up to 498 and 2 x 168; with operands from the L2 alone 1.27 PFLOP/s, where the matrix
 // cores work 88% of the cycles of a clock that sinks to 1.45 GHz: half the copies, or
 // reads of LDS left out, raise the clock, not the products a cycle. Copies asked for in
 // one burst hold their wave up, so they are spread over the products. Workgroups that
