@@ -938,7 +938,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_wide_kernel(
     publish(sc[0]);
 
     // Turn t. Behind its first barrier tile t + 1 is in LDS, both halves of S^T of tile
-    // t are there, and every wave has left the place that tile t + 3 goes to. Past the
+    // t are there, and every wave has left the place that tile t + 2 goes to. Past the
     // run's end copies and products go on with its last tile: one loop for all turns, as
     // instructions that are not in the cache yet cost a run of few tiles 1 us and more.
     int page = page_of(min(t0 + 3, t1 - 1));  // of the tile that the next turn copies

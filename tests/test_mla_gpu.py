@@ -511,3 +511,25 @@ def test_mla_decode_infinities(H, first, kv):
                 continue
             err = (out[i].double() - want).norm() / want.norm()
             assert err < 2 * 2 ** -9, (i, scale, float(err))  # as above
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+@pytest.mark.parametrize("H", [16, 64, 128])
+@pytest.mark.parametrize("B", [64, 65, 256, 257, 321])
+def test_mla_decode_many_sequences(B, H, kv):
+    """A lane deals one, four or more sequences' tiles; the last ones as the first."""
+    ctxs = [(0, 270, 40, 129, 31)[i * i % 5] + i % 3 for i in range(B)]
+    ctxs[-1] = 300
+    ql, qp, cache, bt, sl = _setup(B, H, ctxs, seed=B)
+    if kv == "fp8":
+        cache = cache.to(torch.float8_e4m3fn)
+    out = ops.mla_paged_attention_decode(ql, qp, cache, bt, sl, 192 ** -0.5)
+    for i, n in enumerate(ctxs):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        e = cache[bt[i, :-(-n // 32)].long()].double().flatten(0, 1)[:n]
+        s = (ql[i].double() @ e[:, :512].T + qp[i].double() @ e[:, 512:].T) * 192 ** -0.5
+        want = s.softmax(-1) @ e[:, :512]
+        err = (out[i].double() - want).norm() / want.norm()
+        assert err < 2 * 2 ** -9, (i, n, float(err))  # as above
